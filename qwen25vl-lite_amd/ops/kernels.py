@@ -32,13 +32,13 @@ class KernelError(RuntimeError):
 _functions: Dict[Tuple[str, str, Tuple], ctypes._CFuncPtr] = {}
 
 
-def _fn(stem: str, name: str, argtypes, defines=None):
+def _fn(stem: str, name: str, argtypes, defines=None, restype=_c_int):
     key = (stem, name, tuple(sorted((defines or {}).items())))
     fn = _functions.get(key)
     if fn is None:
         fn = getattr(load_library(stem, defines), name)
         fn.argtypes = list(argtypes)
-        fn.restype = _c_int
+        fn.restype = restype
         _functions[key] = fn
     return fn
 

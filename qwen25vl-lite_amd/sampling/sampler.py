@@ -2,8 +2,9 @@
 
 The reference samples on the host, one request at a time (reference
 src/qwen25vl_lite/sampling.py:67-121, engine.py:802-829).  Here a step's rows are sampled
-together on the GPU; the only host work is the uniform random number of each row, which comes
-from the reference's per-token generator rule (seed + number of tokens generated so far).
+together on the GPU.  A row's uniform random number comes from the reference's per-token generator
+rule (seed + number of tokens generated so far); the kernel draws it from the seed, and only rows
+without a seed draw theirs here, from the global generator.
 """
 
 from __future__ import annotations
@@ -21,7 +22,7 @@ __all__ = ["sample_rows", "sample_rows_begin", "sample_slots_begin", "PendingSam
 
 _ROW = np.dtype([("temperature", "<f4"), ("top_p", "<f4"), ("min_p", "<f4"), ("u", "<f4"),
                  ("repetition", "<f4"), ("presence", "<f4"), ("frequency", "<f4"), ("top_k", "<i4"),
-                 ("prev_begin", "<i4"), ("prev_end", "<i4")])
+                 ("prev_begin", "<i4"), ("prev_end", "<i4"), ("seed", "<u4"), ("seeded", "<i4")])
 
 
 def uniform_from(seed: Optional[int], step: int) -> float:
@@ -38,6 +39,11 @@ def uniform_from(seed: Optional[int], step: int) -> float:
 def uniform_for(params: SamplingParams, step: int) -> float:
     """The uniform number in [0, 1) for a request's output token number ``step``."""
     return 0.0 if params.temperature <= 0 else uniform_from(params.seed, step)
+
+
+def _seed_words(seeds: np.ndarray, steps: np.ndarray) -> np.ndarray:
+    """What :func:`uniform_from`'s generators start from: the lower 32 bits of ``seed + step`` (int64 arrays)."""
+    return (seeds.astype(np.uint64) + steps.astype(np.uint64)).astype(np.uint32)
 
 
 class _Staging:
@@ -124,22 +130,27 @@ def sample_rows_begin(logits: torch.Tensor, params: Sequence[SamplingParams], pr
     if (uniforms is None and first.temperature <= 0 and first.repetition_penalty == 1.0 and first.presence_penalty == 0.0
             and first.frequency_penalty == 0.0 and all(p is first or p == first for p in params)):
         # one greedy setting for the whole batch (the usual decode step): fill the rows at once
-        rows[:] = (first.temperature, first.top_p, first.min_p, 0.0, 1.0, 0.0, 0.0, first.top_k if first.top_k else -1, 0, 0)
-        params_iter = ()
-    else:
-        params_iter = enumerate(params)
-    for i, p in params_iter:
+        rows[:] = (first.temperature, first.top_p, first.min_p, 0.0, 1.0, 0.0, 0.0, first.top_k if first.top_k else -1, 0, 0, 0, 0)
+        return _launch(logits, rows, flat)
+    filled = []
+    for i, p in enumerate(params):
         need_prev = p.repetition_penalty != 1.0 or p.presence_penalty != 0.0 or p.frequency_penalty != 0.0
         begin = len(flat)
         if need_prev:
-            flat.extend(int(t) for t in prev_ids[i])
-        u = uniforms[i] if uniforms is not None else uniform_for(p, steps[i])
-        rows[i] = (p.temperature, p.top_p, p.min_p, u, p.repetition_penalty, p.presence_penalty,
-                   p.frequency_penalty, p.top_k if p.top_k else -1, begin, len(flat))
-    need_scores = any(p.temperature > 0 or len(flat) for p in params)
-    plain = any(p.temperature <= 0 and p.repetition_penalty == 1.0 and p.presence_penalty == 0.0
-                and p.frequency_penalty == 0.0 for p in params)
-    return _launch(logits, rows, flat, need_scores, plain)
+            flat.extend(prev_ids[i])
+        u, word, seeded = 0.0, 0, 0
+        if uniforms is not None:
+            u = uniforms[i]
+        elif p.temperature > 0:
+            start = None if p.seed is None else int(p.seed) + int(steps[i])
+            if start is not None and -(1 << 63) <= start < 1 << 64:
+                word, seeded = start & 0xffffffff, 1
+            else:
+                u = uniform_from(p.seed, steps[i])      # the global generator; a seed no generator takes raises
+        filled.append((p.temperature, p.top_p, p.min_p, u, p.repetition_penalty, p.presence_penalty, p.frequency_penalty,
+                       p.top_k if p.top_k else -1, begin, len(flat), word, seeded))
+    rows[:] = filled
+    return _launch(logits, rows, flat)
 
 
 def sample_slots_begin(logits: torch.Tensor, records, slots: Sequence[int], prev_ids: Sequence[Sequence[int]],
@@ -147,8 +158,7 @@ def sample_slots_begin(logits: torch.Tensor, records, slots: Sequence[int], prev
     """:func:`sample_rows_begin` for requests whose settings and sampler state lie in their slots
     (``records``: :class:`~qwen25vl_lite_amd.cache.slots.SlotRecords`): row ``m`` of the logits belongs to the
     request in slot ``slots[m]``.  The rows' settings are gathered by slot index; only rows with
-    penalties (their generated tokens, ``prev_ids[m]``) and rows that draw (one generator each, by
-    the seed rule) are visited one by one."""
+    penalties (their generated tokens, ``prev_ids[m]``) and rows that draw without a seed are visited one by one."""
     if not logits.is_cuda:
         raise KernelError("sampling has no CPU path: logits must be on the GPU")
     if logits.dtype != torch.float32 or logits.dim() != 2 or not logits.is_contiguous():
@@ -167,35 +177,46 @@ def sample_slots_begin(logits: torch.Tensor, records, slots: Sequence[int], prev
     penal = (rows["repetition"] != 1.0) | (rows["presence"] != 0.0) | (rows["frequency"] != 0.0)
     for i in np.nonzero(penal)[0]:
         rows["prev_begin"][i] = len(flat)
-        flat.extend(int(t) for t in prev_ids[i])
+        flat.extend(prev_ids[i])
         rows["prev_end"][i] = len(flat)
-    for i in np.nonzero(draws)[0]:
-        seed = int(records.seed[at[i]])
-        rows["u"][i] = uniforms[i] if uniforms is not None else uniform_from(None if seed < 0 else seed,
-                                                                             int(records.generated[at[i]]))
-    return _launch(logits, rows, flat, bool(draws.any() or flat), bool((~draws & ~penal).any()))
+    if uniforms is not None:
+        for i in np.nonzero(draws)[0]:
+            rows["u"][i] = uniforms[i]
+    else:
+        seeds = records.seed[at]
+        seeded = draws & (seeds >= 0)
+        rows["seeded"] = seeded
+        rows["seed"] = np.where(seeded, _seed_words(seeds, records.generated[at]), 0)
+        for i in np.nonzero(draws & ~seeded)[0]:
+            rows["u"][i] = uniform_from(None, 0)
+    return _launch(logits, rows, flat)
 
 
-def _launch(logits: torch.Tensor, rows: np.ndarray, flat: List[int], need_scores: bool, plain: bool) -> PendingSample:
-    """Send the rows' settings to the device and queue the sampler.  ``need_scores``: some row scales
-    or penalises its logits (into a copy); ``plain``: some row is a plain argmax."""
+def _launch(logits: torch.Tensor, rows: np.ndarray, flat: List[int]) -> PendingSample:
+    """Send the rows' settings to the device and queue the sampler."""
     m, vocab = logits.shape
-    fn = _fn("sample", "qvl_sample_rows",
-             [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
-              ctypes.c_int, ctypes.c_int, ctypes.c_void_p])
+    c_ptr, c_int = ctypes.c_void_p, ctypes.c_int
+    fn = _fn("sample", "qvl_sample_rows", [c_ptr] * 7 + [c_int] * 4 + [c_ptr])
+    parts_bytes = _fn("sample", "qvl_sample_parts_bytes", [c_int], restype=ctypes.c_longlong)
+    scratch_bytes = _fn("sample", "qvl_sample_scratch_bytes", [], restype=ctypes.c_longlong)
     dev = logits.device
+    draws = rows["temperature"] > 0
     with torch.cuda.device(dev):
-        packed = np.concatenate([rows.view(np.int32), np.asarray(flat or [0], np.int32)])
+        try:
+            ids = np.asarray(flat or [0], np.int32)
+        except (TypeError, ValueError):          # ids of other types than Python's and numpy's
+            ids = np.asarray([int(t) for t in flat], np.int32)
+        packed = np.concatenate([rows.view(np.int32), ids])
         buf = _Staging.to_device(packed, dev)
         n_row_words = rows.view(np.int32).size
-        scores = torch.empty_like(logits) if need_scores else logits
+        some = bool(draws.any())
+        # rows that draw with penalties have their scores written out; the passes read the others' logits as they are
+        scores = torch.empty_like(logits) if bool((draws & (rows["prev_end"] > rows["prev_begin"])).any()) else None
+        scratch = torch.empty(m * scratch_bytes(), dtype=torch.uint8, device=dev) if some else None
+        parts = torch.empty(m * parts_bytes(vocab), dtype=torch.uint8, device=dev)
         out = torch.empty(m, dtype=torch.int32, device=dev)
-        # a greedy row without penalties is a plain argmax: several blocks scan it side by side
-        parts = None
-        if plain:
-            part_bytes = int(_fn("sample", "qvl_sample_argmax_part_bytes", [])())
-            parts = torch.empty(m * part_bytes, dtype=torch.uint8, device=dev)
-        _check(fn(logits.data_ptr(), scores.data_ptr(), buf.data_ptr(), buf[n_row_words:].data_ptr(),
-                  parts.data_ptr() if parts is not None else None, out.data_ptr(), m, vocab, _stream()),
-               "sample_rows")
+        _check(fn(logits.data_ptr(), None if scores is None else scores.data_ptr(), buf.data_ptr(),
+                  buf[n_row_words:].data_ptr(), None if scratch is None else scratch.data_ptr(), parts.data_ptr(),
+                  out.data_ptr(), m, vocab, int(bool((draws & (rows["top_k"] > 0) & (rows["top_k"] < vocab)).any())),
+                  int(bool((draws & (rows["top_p"] < 1.0)).any())), _stream()), "sample_rows")
         return PendingSample(out)

@@ -478,6 +478,48 @@ def test_sampler_kernel_against_plain():
     assert torch.allclose(freq, plain_filtered_probs(row, 1.0, top_k=4).double(), atol=2e-3)
 
 
+@pytest.mark.parametrize("vocab", [1, 7, 1023, 1025, 4096, 4097, 40001])
+def test_sampler_cuts_at_the_edges_of_its_pieces(vocab):
+    """Rows as long as a piece of the passes, one more, shorter than the draw's chunks; equal scores across a cut, tokens
+    that may not be drawn (-inf); every row with the number its seed stands for and with that number given."""
+    from qwen25vl_lite_amd.sampling import SamplingParams
+    from qwen25vl_lite_amd.sampling.sampler import sample_rows, uniform_for
+
+    g = torch.Generator().manual_seed(vocab)
+    kinds = [dict(temperature=1.0), dict(temperature=0.6, top_k=3), dict(temperature=1.0, top_k=vocab),
+             dict(temperature=1.1, top_p=0.5), dict(temperature=0.9, top_p=0.999), dict(temperature=0.8, min_p=0.2),
+             dict(temperature=0.9, top_k=20, top_p=0.7, min_p=0.01, repetition_penalty=1.3, frequency_penalty=0.2),
+             dict(temperature=0.0), dict(temperature=0.0, presence_penalty=0.7)]
+    seeds = [5, 2 ** 31 + 9, 2 ** 40 + 1, -3]
+    params = [SamplingParams(seed=seeds[i % len(seeds)], **k) for i, k in enumerate(kinds)]
+    for trial in range(3):
+        logits = torch.randn(len(params), vocab, generator=g) * 2
+        if trial == 1:
+            logits = logits.round()                       # many equal scores
+        if trial == 2 and vocab > 7:
+            logits[:, ::3] = float("-inf")
+        prev = [torch.randint(0, vocab, (trial * 9,), generator=g).tolist() for _ in params]
+        steps = [3 * trial + i for i in range(len(params))]
+        us = [uniform_for(p, s) for p, s in zip(params, steps)]
+        got = sample_rows(logits.cuda(), params, prev, steps)
+        assert got == sample_rows(logits.cuda(), params, prev, steps, uniforms=us)
+        for i, p in enumerate(params):
+            pen = plain_penalties(logits[i], prev[i], p.repetition_penalty, p.presence_penalty, p.frequency_penalty)
+            if p.temperature <= 0:
+                assert got[i] == int(torch.argmax(pen)), (trial, i)
+                continue
+            kept = plain_filtered_probs(pen, p.temperature, p.top_k, p.top_p, p.min_p) > 0
+            # every token tied with the last one kept stays too
+            probs = torch.softmax(pen.double() / p.temperature, 0) * (pen >= pen[kept].min())
+            cdf = torch.cumsum(probs, 0) / probs.sum()
+            want = int(torch.searchsorted(cdf, torch.tensor(us[i], dtype=torch.float64), right=True).clamp(max=vocab - 1))
+            if got[i] != want:
+                # a draw within rounding of a boundary of the distribution function: float32 sums of up to `vocab` masses
+                share = probs[got[i]] / probs.sum()
+                assert share > 0
+                assert min(abs(cdf[got[i]] - us[i]), abs(cdf[got[i]] - share - us[i])) < 1e-5, (trial, i)
+
+
 def test_trace_run_program(model_dirs, tmp_path):
     """bin/trace_run as a user calls it: JSON steps on standard input, `done <step>` lines,
     <step>.f32 files of little-endian float32 [wanted, vocab]."""
