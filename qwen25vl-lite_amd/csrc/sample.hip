@@ -16,7 +16,7 @@
 // Masses are whole numbers of 2^-40 of the largest score's (of more for rows beyond 2^23 scores, whose sum
 // would not fit 64 bits), which is finer than a float32 sum of them and lets the blocks add in any order.  One block a row that searched bit by bit, 32 passes for each
 // threshold, took 3.70 ms for 64 rows of 152,064 (greedy, top-p, top-k with top-p and penalties, min-p
-// in turn); these passes together take SAMPLE_US.
+// in turn); these passes together take 113 us.
 #include "common.h"
 #include <type_traits>
 

@@ -48,6 +48,16 @@ def _check(code: int, what: str) -> None:
         raise KernelError(f"{what}: the kernel refused its arguments ({_ERRORS.get(code, code)})")
 
 
+_cu_count: Dict[int, int] = {}
+
+
+def compute_units(device) -> int:
+    key = torch.device(device).index or 0
+    if key not in _cu_count:
+        _cu_count[key] = torch.cuda.get_device_properties(key).multi_processor_count
+    return _cu_count[key]
+
+
 def dtype_code(dtype: torch.dtype) -> int:
     if dtype == torch.float32:
         return 0
@@ -322,7 +332,7 @@ def gemm_f32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]
         out = torch.empty((m, n), dtype=torch.float32, device=x.device)
     _need(out.shape == (m, n) and out.dtype == torch.float32 and out.stride(1) == 1, "out must be float32 [M, N]")
     fn = _fn("gemm_f32", "qvl_gemm_f32",
-             [_c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr])
+             [_c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr])
     _check(fn(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), _ptr(out), out.stride(0), m, n, k,
-              _stream()), "gemm_f32")
+              compute_units(x.device), _stream()), "gemm_f32")
     return out

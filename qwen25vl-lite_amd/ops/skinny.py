@@ -14,6 +14,7 @@ from typing import Optional
 import torch
 
 from .kernels import _check, _fn, _ptr, _stream, dtype_code
+from .kernels import compute_units as _compute_units
 
 __all__ = ["resident_product", "takes_resident", "qkv_rope_product", "takes_qkv_rope", "RESIDENT_ROWS", "resident_norm_k", "resident_two_tile_k", "folds_norm", "ONE_BLOCK_ROWS", "split_product", "takes_split", "prefers_split", "SPLIT_ROWS",
            "takes_stack", "stack_product", "STORE", "RESIDUAL", "SWIGLU", "GEGLU", "RELU2", "GATED"]
@@ -28,14 +29,6 @@ _two_tile_k = None
 STORE, RESIDUAL, SWIGLU, GEGLU, RELU2 = 0, 1, 2, 4, 5
 GATED = {"silu": SWIGLU, "gelu_tanh": GEGLU}
 _c_int, _c_float, _c_ptr = ctypes.c_int, ctypes.c_float, ctypes.c_void_p
-_cu_count = {}
-
-
-def _compute_units(device) -> int:
-    key = torch.device(device).index or 0
-    if key not in _cu_count:
-        _cu_count[key] = torch.cuda.get_device_properties(key).multi_processor_count
-    return _cu_count[key]
 
 
 def _rows_aligned(t: torch.Tensor, elems: int) -> bool:

@@ -406,6 +406,27 @@ def test_gemm_f32_is_exact_and_row_independent(m, n, k):
     assert torch.equal(alone[0], out[m // 2])
 
 
+@pytest.mark.parametrize("n, k", [(5, 4), (64, 60), (130, 64), (33, 68), (509, 1000), (2560, 2048), (16390, 132)])
+@pytest.mark.parametrize("m", [1, 16, 17, 33, 64, 65, 130])
+def test_gemm_f32_tiles_give_the_chains_bits(m, n, k):
+    """The matrix-core tiles (rows on 16-byte boundaries) against the plain kernel, which takes any stride: one chain of
+    fused multiply-adds an output in either, so the same bits.  Sizes on either side of a tile, of a step of K, and of
+    where another shape of blocks is chosen; denormals and wide ranges among the values."""
+    from qwen25vl_lite_amd.ops import kernels
+    g = torch.Generator(device="cuda").manual_seed(m * n + k)
+    x = torch.randn(m, k, device="cuda", generator=g) * torch.exp2(torch.randint(-30, 30, (m, k), device="cuda", generator=g).float())
+    w = torch.randn(n, k, device="cuda", generator=g)
+    w[::7] *= 1e-38
+    b = torch.randn(n, device="cuda", generator=g)
+    wide = torch.zeros(m, k + 1, device="cuda")            # rows no multiple of 16 bytes apart: the plain kernel
+    wide[:, :k] = x
+    for bias in (None, b):
+        want = kernels.gemm_f32(wide[:, :k], w, bias)
+        assert torch.equal(kernels.gemm_f32(x, w, bias), want)
+    out = torch.empty(m, n + 3, device="cuda")[:, :n]
+    assert torch.equal(kernels.gemm_f32(x, w, b, out=out), want)
+
+
 @pytest.mark.parametrize("m, n, k", [(1, 509, 144), (8, 300, 200), (16, 17, 8), (9, 100, 8200), (17, 1000, 4104),
                                      (31, 130, 352), (64, 509, 3584), (5, 40, 100), (300, 64, 1000),
                                      (17, 4700, 3584), (32, 300, 3840), (24, 509, 3848), (20, 33, 8),
