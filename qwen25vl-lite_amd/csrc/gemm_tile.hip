@@ -1,0 +1,239 @@
+// Products with more rows than the decode kernels keep: out = X[M, K] . W[N, K]^T, bfloat16 operands, float32 sums, with what
+// follows the product done on the sums: a cast, the square of relu, a gated activation (gate and up rows of W in
+// groups of 8 + 8, or gate rows first), or float32 slabs over ranges of K for whoever adds them next.
+//
+// The inner loop is tile_product.h's.  Tiles of 256 x 256 run fastest, smaller ones where a device of 256
+// compute units would otherwise stand half empty; the choice is by an estimate of the time (plan_for).  Measured, the
+// library's product (with the activation's kernel behind it where there is one) in brackets: 2,048 x 37,888 x 3,584
+// gated 439 us (624), 2,048 x 3,584 x 18,944 in two ranges 204 (377), 280 x 22,016 x 2,048 gated 50 (55), 280 x 2,048 x
+// 11,008 in ranges 34 (50), 100 x 2,560 x 2,048 in ranges 15 (28), 700 x 3,584 x 18,944 in ranges 85 (182).
+//
+// Blocks go to the XCDs in turn, each with an L2 of its own: XCD x takes a contiguous run of the tiles, ordered so that
+// the 32 blocks it holds at a time share few rows of W and X (eight tiles of X's rows, then the next tile of W's).
+#include "tile_product.h"
+
+enum { OUT_BF16 = 0, OUT_F32 = 1, OUT_GROUPED = 2, OUT_HALVES = 3 };
+
+struct TileArgs {
+  const bf16_t* x;
+  long long ldx;
+  const bf16_t* w;
+  long long ldw;
+  void* out;
+  long long ldo;
+  int M, N, K;
+  int rows;              // OUT_HALVES: rows of W before its up rows (N = 2 rows); else N
+  int tiles_m, tiles_n, splits;
+  int relu2, gelu;
+  float alpha, limit, shift;
+};
+
+__device__ __forceinline__ uint32_t two_bf16(float a, float b) {
+  typedef __bf16 pair_t __attribute__((ext_vector_type(2)));
+  const pair_t v = {(__bf16)a, (__bf16)b};
+  return __builtin_bit_cast(uint32_t, v);
+}
+// four neighbouring results
+__device__ __forceinline__ void store4(bf16_t* o, const float* v, int n, bool whole) {
+  if (whole) {
+    *reinterpret_cast<uint2*>(o) = uint2{two_bf16(v[0], v[1]), two_bf16(v[2], v[3])};
+  } else {
+    for (int i = 0; i < n && i < 4; ++i) o[i] = f32_to_bf16(v[i]);
+  }
+}
+__device__ __forceinline__ void store4(float* o, const float* v, int n, bool whole) {
+  if (whole) {
+    *reinterpret_cast<float4*>(o) = float4{v[0], v[1], v[2], v[3]};
+  } else {
+    for (int i = 0; i < n && i < 4; ++i) o[i] = v[i];
+  }
+}
+__device__ __forceinline__ float clamped_gate(float g, float u, const TileArgs& p) {
+  if (p.limit > 0.f) {
+    g = fminf(g, p.limit);
+    u = fminf(fmaxf(u, -p.limit), p.limit);
+  }
+  return g / (1.0f + expf(-p.alpha * g)) * (u + p.shift);
+}
+
+template <typename T, int OUT>
+__global__ __launch_bounds__(512) void gemm_tile_kernel(TileArgs p) {
+  __shared__ __attribute__((aligned(16))) char lds[T::LDS];
+  T t;
+  const int tiles = p.tiles_m * p.tiles_n, all = tiles * p.splits, per = (all + 7) / 8;
+  const int turn = blockIdx.x >> 3, id = (blockIdx.x & 7) * per + turn;
+  if (turn >= per || id >= all) return;
+  const int split = id / tiles, at = id - split * tiles;
+  // eight tiles of X's rows beside each other, then the next tile of W's rows
+  const int band = at / (8 * p.tiles_n), in_band = at - band * 8 * p.tiles_n;
+  const int wide = min(8, p.tiles_m - 8 * band);
+  const int tile_m = 8 * band + in_band % wide, tile_n = in_band / wide;
+  constexpr int OUT_N = OUT == OUT_HALVES ? T::BN / 2 : T::BN;       // rows of W (of each half) from n0 on
+  const int n0 = tile_n * OUT_N, m0 = tile_m * T::BM;
+  // this split's range of K
+  const int steps_all = (p.K + 63) / 64;
+  const int s0 = (int)((long long)steps_all * split / p.splits), s1 = (int)((long long)steps_all * (split + 1) / p.splits);
+  const bf16_t* w = p.w + (size_t)n0 * p.ldw + (size_t)s0 * 64;
+  const bf16_t* x = p.x + (size_t)m0 * p.ldx + (size_t)s0 * 64;
+  // rows that do not exist are read from one that does; their sums are not stored
+  t.set_rows(
+      [&](int h, int rho) {
+        if (OUT == OUT_HALVES) {     // first half: gate rows, second half: their up rows
+          const int n = n0 + rho < p.rows ? rho : 0;
+          return (uint32_t)(((size_t)n + (h ? p.rows : 0)) * p.ldw * 2);
+        }
+        const int n = T::w_row(h, rho);
+        return (uint32_t)((size_t)(n0 + n < p.N ? n : 0) * p.ldw * 2);
+      },
+      [&](int h, int rho) {
+        const int m = T::x_row(h, rho);
+        return (uint32_t)((size_t)(m0 + m < p.M ? m : 0) * p.ldx * 2);
+      });
+  t.multiply(lds, w, x, s1 - s0, p.K % 64 != 0 && s1 == steps_all);
+  // a lane holds, of tile (n, m): X's row 16 m + r, W's rows 16 n + 4 g ... + 3
+#pragma unroll
+  for (int m = 0; m < T::MT; ++m) {
+    const int gm = m0 + (t.wm * T::MT + m) * 16 + t.r;
+    if (OUT == OUT_BF16 || OUT == OUT_F32) {
+      if (gm >= p.M) continue;
+#pragma unroll
+      for (int n = 0; n < T::NT; ++n) {
+        const int gn = n0 + (t.wn * T::NT + n) * 16 + 4 * t.g;
+        if (gn >= p.N) continue;
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          v[i] = t.acc[n][m][i];
+          if (p.relu2) {
+            v[i] = fmaxf(v[i], 0.f);
+            v[i] *= v[i];
+          }
+        }
+        const bool whole = gn + 4 <= p.N && p.ldo % 4 == 0;
+        if (OUT == OUT_BF16) store4(reinterpret_cast<bf16_t*>(p.out) + (size_t)gm * p.ldo + gn, v, p.N - gn, whole);
+        else store4(reinterpret_cast<float*>(p.out) + ((size_t)split * p.M + gm) * p.ldo + gn, v, p.N - gn, whole);
+      }
+    } else if (OUT == OUT_HALVES) {
+      if (gm >= p.M) continue;
+#pragma unroll
+      for (int n = 0; n < T::NH; ++n) {
+        const int gn = n0 + (t.wn * T::NH + n) * 16 + 4 * t.g;
+        if (gn >= p.rows) continue;
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = clamped_gate(t.acc[n][m][i], t.acc[n + T::NH][m][i], p);
+        store4(reinterpret_cast<bf16_t*>(p.out) + (size_t)gm * p.ldo + gn, v, p.rows - gn, gn + 4 <= p.rows && p.ldo % 4 == 0);
+      }
+    } else {
+      // rows 0 .. 7 of a tile of 16 are gate rows (lanes of g 0 and 1), rows 8 .. 15 their up rows.  Of two
+      // neighbouring tiles the lanes below 32 take the first, the others the second: one exchange of halves
+      // gives every lane a gate and its up value.
+#pragma unroll
+      for (int n = 0; n < T::NT; n += 2) {
+        float v[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float one = t.acc[n][m][i], next = t.acc[n + 1][m][i];
+          const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(one), __float_as_uint(next), false, false);
+          v[i] = gate_act(__uint_as_float((uint32_t)both[0]), p.gelu) * __uint_as_float((uint32_t)both[1]);
+        }
+        const int first = n0 + (t.wn * T::NT + n + (t.g >> 1)) * 16;      // the lane's tile's first row of W
+        if (gm < p.M && first < p.N)
+          store4(reinterpret_cast<bf16_t*>(p.out) + (size_t)gm * p.ldo + first / 2 + 4 * (t.g & 1), v, 4, p.ldo % 4 == 0);
+      }
+    }
+  }
+}
+
+// How a product is cut: the tile's shape and the ranges of K.  The estimate is of microseconds: a step of 64 values
+// costs a block `alone` where most compute units are idle and `full` where all work (a step of 256 x 256 takes 1.08 and
+// 1.43 us: with every matrix core busy the clock and the caches give way), a launch 8 us and each of its rounds 4 (the
+// first fetches, the stores); slabs are written and read once more, at 4.5 TB/s.
+struct Plan {
+  int tile, splits;
+  double us;
+};
+struct TileShape {
+  int bn, bm, a_unit;     // blocks a compute unit holds
+  double alone, full;
+};
+static const TileShape SHAPES[4] = {{256, 256, 1, 1.08, 1.43}, {128, 256, 1, 0.80, 0.96}, {256, 128, 1, 0.79, 0.94}, {128, 128, 2, 0.62, 1.02}};
+
+static Plan plan_for(int M, int N, int K, int most_splits, int cus) {
+  Plan best{0, 1, 1e30};
+  const int steps = (K + 63) / 64;
+  for (int i = 0; i < 4; ++i) {
+    const TileShape& s = SHAPES[i];
+    const long long tiles = (long long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+    for (int splits = 1; splits <= most_splits && (splits == 1 || splits * 4 <= steps); ++splits) {
+      const long long blocks = tiles * splits, room = (long long)cus * s.a_unit, whole = blocks / room;
+      const double rest = (double)(blocks - whole * room) / room;
+      const double depth = (steps + splits - 1) / splits;
+      double us = 8.0 + whole * (depth * s.full + 4.0);
+      if (rest > 0) us += depth * (s.alone + (s.full - s.alone) * rest) + 4.0;
+      if (splits > 1) us += splits * (double)M * N * 8.0 / 4.5e6;
+      if (us < best.us) best = Plan{i, splits, us};
+    }
+  }
+  return best;
+}
+
+#define MOST_SPLITS 12
+
+extern "C" int qvl_gemm_tile_splits(int M, int N, int K, int cus) {
+  if (M <= 0 || N <= 0 || K <= 0 || cus <= 0) return 0;
+  return plan_for(M, N, K, MOST_SPLITS, cus).splits;
+}
+// Blocks of the uncut product: with far fewer than compute units the library, which cuts K by itself, is faster.
+extern "C" int qvl_gemm_tile_blocks(int M, int N, int K, int cus) {
+  if (M <= 0 || N <= 0 || K <= 0 || cus <= 0) return 0;
+  const TileShape& s = SHAPES[plan_for(M, N, K, 1, cus).tile];
+  const long long blocks = (long long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+  return (int)(blocks < 0x7fffffff ? blocks : 0x7fffffff);
+}
+
+// x: bfloat16 [M, K], rows ldx apart; W: bfloat16 [N, K], rows ldw apart; both on 16-byte boundaries, K a multiple of 32.
+// mode 0: out bfloat16 [M, N] (relu2: max(product, 0)^2); 1: out float32 [splits][M][N], the slabs' sum is the product;
+// 2: N in groups of 8 gate + 8 up rows, out bfloat16 [M, N / 2] = act(gate) up (gelu: gelu's tanh form, else silu);
+// 3: N / 2 gate rows, then the up rows: out = g sigmoid(alpha g) (u + shift), g capped at limit, u clamped to +-limit.
+// tile: -1, or the shape to take (0 .. 3).
+extern "C" int qvl_gemm_tile(const void* x, long long ldx, const void* w, long long ldw, void* out, long long ldo, int M, int N,
+                             int K, int mode, int splits, int relu2, int gelu, float alpha, float limit, float shift, int tile,
+                             int cus, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return QVL_OK;
+  if (K <= 0 || K % 32 || ldx < K || ldw < K || ldx % 8 || ldw % 8 || !x || !w || !out || cus <= 0 || splits < 1 ||
+      ((uintptr_t)x % 16) || ((uintptr_t)w % 16) || ((uintptr_t)out % 16) || splits > (K + 63) / 64 || (mode != 1 && splits != 1))
+    return QVL_ERR_SHAPE;
+  if ((mode == 2 && N % 16) || (mode == 3 && N % 2) || ldo < (mode >= 2 ? N / 2 : N)) return QVL_ERR_SHAPE;
+  if (mode < 0 || mode > 3 || tile > 3) return QVL_ERR_SHAPE;
+  // byte offsets from a tile's first row are 32-bit (in mode 3 the up rows lie N / 2 rows further on)
+  const unsigned long long w_span = (mode == 3 ? (unsigned long long)N / 2 + 256 : 256ull) * ldw * 2, x_span = 256ull * ldx * 2;
+  if (w_span >= 0xffff0000ull || x_span >= 0xffff0000ull) return QVL_ERR_LIMIT;
+  TileArgs p;
+  p.x = (const bf16_t*)x; p.ldx = ldx; p.w = (const bf16_t*)w; p.ldw = ldw; p.out = out; p.ldo = ldo;
+  p.M = M; p.N = N; p.K = K; p.rows = mode == 3 ? N / 2 : N; p.splits = splits; p.relu2 = relu2; p.gelu = gelu;
+  p.alpha = alpha; p.limit = limit; p.shift = shift;
+  const int shape = tile >= 0 ? tile : plan_for(M, N, K, mode == 1 && splits > 1 ? MOST_SPLITS : 1, cus).tile;
+  const TileShape& s = SHAPES[shape];
+  const int out_n = mode == 3 ? s.bn / 2 : s.bn;
+  p.tiles_m = (M + s.bm - 1) / s.bm;
+  p.tiles_n = (p.rows + out_n - 1) / out_n;
+  const long long all = (long long)p.tiles_m * p.tiles_n * splits;
+  if (all > 0x7ffffff0ll / 8) return QVL_ERR_LIMIT;
+  const dim3 grid((unsigned)((all + 7) / 8 * 8));
+#define GO(OUT, WN, WM, NT, MT) hipLaunchKernelGGL((gemm_tile_kernel<Tile<WN, WM, NT, MT>, OUT>), grid, dim3(512), 0, stream, p)
+#define SHAPE(OUT)                       \
+  do {                                   \
+    if (shape == 0) GO(OUT, 2, 4, 8, 4); \
+    else if (shape == 1) GO(OUT, 2, 4, 4, 4); \
+    else if (shape == 2) GO(OUT, 4, 2, 4, 4); \
+    else GO(OUT, 2, 4, 4, 2);            \
+  } while (0)
+  if (mode == 0) SHAPE(OUT_BF16);
+  else if (mode == 1) SHAPE(OUT_F32);
+  else if (mode == 2) SHAPE(OUT_GROUPED);
+  else SHAPE(OUT_HALVES);
+#undef SHAPE
+#undef GO
+  return qvl_launch_status();
+}

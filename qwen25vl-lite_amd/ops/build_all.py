@@ -18,6 +18,7 @@ LIBRARIES = [
     ("gemm_resident", {}),
     ("gemm_resident", {"RK": 4}),
     ("gemm_split", {}),
+    ("gemm_tile", {}),
     ("peaks", {}),
     ("gated", {}),
     ("moe", {}),

@@ -3,8 +3,10 @@
 float32 runs through the hand-written FMA kernel (true 32-bit, fixed summation order).
 bfloat16 with up to 64 rows (a decode step) runs through the hand-written matrix-core kernel, which
 also folds the norm before a product, the residual add after it and the SwiGLU activation into
-itself; with more rows the vendor library's product runs, which is also what the
-reference's engine uses for its projections (reference src/qwen25vl_lite/text.py:61-66, 80-90).
+itself; with more rows the tiled kernel runs (:mod:`~qwen25vl_lite_amd.ops.tile`), with the activation on its sums, or
+cut along the inner size where the result joins a sum anyway.  The vendor library's product, which the
+reference's engine uses for its projections (reference src/qwen25vl_lite/text.py:61-66, 80-90), is left
+for what neither takes or does as fast.
 """
 
 from __future__ import annotations
@@ -13,7 +15,7 @@ from typing import Optional, Union
 
 import torch
 
-from . import kernels, skinny
+from . import kernels, skinny, tile
 
 __all__ = ["NormedRows", "linear", "linear_into", "linear_stack", "linear_relu2", "gate_up_swiglu", "tune_library_products"]
 
@@ -30,10 +32,14 @@ class NormedRows:
         return kernels.add_rmsnorm(self.h, None, self.weight, self.eps, self.dtype)
 
 
-def _library(x: torch.Tensor, weight: torch.Tensor, bias, out_dtype, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+def _many_rows(x: torch.Tensor, weight: torch.Tensor, bias, out_dtype, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     if out is not None:
+        if out.dtype == torch.bfloat16 and out.dim() == 2 and out.stride(1) == 1 and out.data_ptr() % 16 == 0 and tile.prefers_tile(x, weight):
+            return tile.tile_product(x, weight, out=out)
         return torch.mm(x, weight.t(), out=out)
-    if out_dtype == torch.float32:
+    if tile.prefers_tile(x, weight):
+        y = tile.tile_product(x, weight, out_dtype or torch.bfloat16)
+    elif out_dtype == torch.float32:
         y = torch.mm(x, weight.t(), out_dtype=torch.float32)  # float32 accumulator written out unrounded
     else:
         y = torch.nn.functional.linear(x, weight)
@@ -61,7 +67,7 @@ def linear(x: Union[torch.Tensor, NormedRows], weight: torch.Tensor, bias: Optio
             raise kernels.KernelError(f"linear: operands {x.dtype}/{weight.dtype} are not built")
         if few and skinny.takes_resident(m, k, weight) and _aligned(x):
             return skinny.resident_product(weight, x=x, bias=bias, out_dtype=out_dtype or torch.bfloat16)
-        return _library(x, weight, bias, out_dtype)
+        return _many_rows(x, weight, bias, out_dtype)
     if lazy:
         x = x.materialize()
     if not x.is_cuda:
@@ -86,7 +92,7 @@ def linear_stack(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
         elif m <= skinny.ONE_BLOCK_ROWS and skinny.takes_resident(m, k, weight[i]) and _aligned(x[i]):
             skinny.resident_product(weight[i], x=x[i], out=out[i], out_dtype=torch.bfloat16)
         else:
-            _library(x[i], weight[i], None, torch.bfloat16, out=out[i])
+            _many_rows(x[i], weight[i], None, torch.bfloat16, out=out[i])
     return out
 
 
@@ -98,6 +104,8 @@ def linear_relu2(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
             and skinny.takes_resident(m, k, weight) and _aligned(x)):
         return skinny.resident_product(weight, x=x, epilogue=skinny.RELU2, out_dtype=torch.bfloat16)
     from .rownorm import squared_relu_
+    if x.is_cuda and tile.prefers_tile(x, weight):
+        return tile.tile_product(x, weight, relu2=True)
     z = linear(x, weight)
     return squared_relu_(z if z.is_contiguous() else z.contiguous())
 
@@ -110,7 +118,7 @@ def linear_into(residual: Optional[torch.Tensor], x: torch.Tensor, weight: torch
     """``residual += x @ weight.T`` inside the product's kernel where that exists (few bfloat16
     rows): then None is returned.  Otherwise what is to be added is returned and the caller hands
     it on to whoever adds it (the next norm's kernel): the product ``[M, N]``, or float32
-    ``[slabs, M, N]`` whose slabs are added in order (the split kernel)."""
+    ``[slabs, M, N]`` whose slabs are added in order (the split kernel; the tiled one over ranges of the inner size)."""
     m, k = x.shape
     fast = x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and _aligned(x)
     if fast and skinny.prefers_split(m, k, weight):
@@ -119,8 +127,11 @@ def linear_into(residual: Optional[torch.Tensor], x: torch.Tensor, weight: torch
             and residual.dtype == torch.float32 and residual.shape == (m, weight.shape[0]) and residual.stride(1) == 1):
         skinny.resident_product(weight, x=x, epilogue=skinny.RESIDUAL, out=residual)
         return None
-    # More rows: the library's product.  Its bfloat16 output is the form it is tuned for (float32
-    # output costs a tenth of a 2,048-token prefill); the sum into the residual stays float32.
+    if fast:
+        slabs = tile.tile_slabs(x, weight)
+        if slabs is not None:
+            return slabs
+    # Uncut with more rows: in bfloat16 (half the traffic of float32); the sum into the residual stays float32.
     return linear(x, weight, out_dtype=torch.float32 if m <= skinny.ONE_BLOCK_ROWS else None)
 
 
@@ -153,4 +164,8 @@ def gate_up_swiglu(x: Union[torch.Tensor, NormedRows], weight: torch.Tensor, gro
             return skinny.resident_product(weight, h=x.h, norm_weight=x.weight, eps=x.eps, epilogue=skinny.GATED[act])
         if not lazy and x.dtype == torch.bfloat16 and skinny.takes_resident(m, k, weight) and _aligned(x):
             return skinny.resident_product(weight, x=x, epilogue=skinny.GATED[act])
+    if isinstance(x, NormedRows):
+        x = x.materialize()
+    if grouped and weight.shape[0] % 16 == 0 and x.is_cuda and tile.prefers_tile(x, weight):
+        return tile.tile_swiglu(x, weight, act)
     return kernels.swiglu(linear(x, weight), grouped=grouped, act=act)

@@ -1,0 +1,101 @@
+"""Dispatch of bfloat16 products with many rows to the tiled kernel (``csrc/gemm_tile.hip``)."""
+
+from __future__ import annotations
+
+import ctypes
+from typing import Optional
+
+import torch
+
+from .kernels import _check, _fn, _need, _ptr, _stream, compute_units
+
+__all__ = ["MANY_ROWS", "takes_tile", "prefers_tile", "tile_product", "tile_slabs", "tile_swiglu", "tile_gated"]
+
+_c_int, _c_ptr, _c_ll, _c_float = ctypes.c_int, ctypes.c_void_p, ctypes.c_longlong, ctypes.c_float
+_STORE, _SLABS, _GROUPED, _HALVES = range(4)
+_REACH = 0xffff0000      # bytes that a tile's rows may span from its first
+
+
+def _rows_aligned(t: torch.Tensor) -> bool:
+    return t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.stride(0) >= t.shape[1] and t.data_ptr() % 16 == 0
+
+
+def takes_tile(x: torch.Tensor, weight: torch.Tensor, halves: bool = False) -> bool:
+    """Whether the kernel takes ``x [M, K] @ weight[N, K].T``: bfloat16 rows on 16-byte boundaries, an inner size in steps
+    of 32, and rows that lie within 32-bit offsets of a tile's first (``halves``: the up rows, N / 2 further on, too)."""
+    if not (x.is_cuda and weight.is_cuda and x.dtype == weight.dtype == torch.bfloat16 and x.dim() == 2 and weight.dim() == 2
+            and x.shape[1] == weight.shape[1] and x.shape[0] > 0 and x.shape[1] > 0 and x.shape[1] % 32 == 0
+            and _rows_aligned(x) and _rows_aligned(weight)):
+        return False
+    span = 256 + (weight.shape[0] // 2 if halves else 0)
+    return span * weight.stride(0) * 2 < _REACH and 256 * x.stride(0) * 2 < _REACH
+
+
+MANY_ROWS = 64           # up to here the decode kernels and the library run
+
+
+def prefers_tile(x: torch.Tensor, weight: torch.Tensor, halves: bool = False) -> bool:
+    """Whether the kernel takes the product and is the faster way to it, uncut: more than ``MANY_ROWS`` rows, and tiles for
+    three quarters of the compute units (2,048 x 3,584 x 3,584: 224 tiles, 63 us against the library's 66; 280 x 2,560 x
+    2,048: 60 tiles, 34 against 24, the library cuts the inner size)."""
+    if x.shape[0] <= MANY_ROWS or not takes_tile(x, weight, halves):
+        return False
+    cus = compute_units(x.device)
+    blocks = int(_fn("gemm_tile", "qvl_gemm_tile_blocks", [_c_int] * 4)(x.shape[0], weight.shape[0], x.shape[1], cus))
+    return 4 * blocks >= 3 * cus
+
+
+def _launch(x, weight, out, ldo, mode, splits=1, relu2=0, gelu=0, alpha=1.0, limit=0.0, shift=0.0, shape=-1):
+    fn = _fn("gemm_tile", "qvl_gemm_tile", [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ll, _c_int, _c_int, _c_int, _c_int, _c_int,
+                                            _c_int, _c_int, _c_float, _c_float, _c_float, _c_int, _c_int, _c_ptr])
+    m, k = x.shape
+    _check(fn(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(out), ldo, m, weight.shape[0], k, mode, splits, relu2,
+              gelu, alpha, limit, shift, shape, compute_units(x.device), _stream()), "linear (tiles)")
+    return out
+
+
+def tile_product(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16,
+                 out: Optional[torch.Tensor] = None, relu2: bool = False, shape: int = -1) -> torch.Tensor:
+    """``x @ weight.T`` in ``out_dtype`` (``relu2``: the square of its positive part); ``shape`` names a tile (-1: by the
+    kernel's estimate)."""
+    _need(takes_tile(x, weight), "the tiled kernel does not take this product")
+    m, n = x.shape[0], weight.shape[0]
+    if out is None:
+        out = torch.empty((m, n), dtype=out_dtype, device=x.device)
+    _need(out.dtype == out_dtype and out_dtype in (torch.float32, torch.bfloat16) and tuple(out.shape) == (m, n)
+          and out.stride(1) == 1 and out.stride(0) >= n and out.data_ptr() % 16 == 0, "out must be [M, N] of the output's dtype")
+    return _launch(x, weight, out, out.stride(0), _SLABS if out_dtype == torch.float32 else _STORE, relu2=int(relu2), shape=shape)
+
+
+def tile_slabs(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:
+    """Float32 slabs ``[splits, M, N]`` over ranges of the inner size, whose sum in order is ``x @ weight.T``; None where the
+    kernel does not take the product or is faster without a cut.  Cutting pays where the tiles alone leave compute units
+    idle: 2,048 x 3,584 x 18,944 has 112 tiles of 256 x 256, two ranges take 204 us and one 282 (the library 377)."""
+    if x.shape[0] <= MANY_ROWS or not takes_tile(x, weight):
+        return None
+    m, k = x.shape
+    n = weight.shape[0]
+    splits = int(_fn("gemm_tile", "qvl_gemm_tile_splits", [_c_int] * 4)(m, n, k, compute_units(x.device)))
+    if splits <= 1:
+        return None
+    out = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
+    return _launch(x, weight, out, n, _SLABS, splits=splits)
+
+
+def tile_swiglu(x: torch.Tensor, weight: torch.Tensor, act: str = "silu", shape: int = -1) -> torch.Tensor:
+    """``act(gate) * up`` for a weight whose rows come in groups of 8 gate and 8 up rows: bfloat16 ``[M, N / 2]``."""
+    _need(takes_tile(x, weight) and weight.shape[0] % 16 == 0, "the tiled kernel does not take this product")
+    _need(act in ("silu", "gelu_tanh"), "the activation is silu or gelu_tanh")
+    half = weight.shape[0] // 2
+    out = torch.empty((x.shape[0], half), dtype=torch.bfloat16, device=x.device)
+    return _launch(x, weight, out, half, _GROUPED, gelu=int(act == "gelu_tanh"), shape=shape)
+
+
+def tile_gated(x: torch.Tensor, weight: torch.Tensor, alpha: float, limit: Optional[float], shift: float,
+               shape: int = -1) -> torch.Tensor:
+    """``g sigmoid(alpha g) (u + shift)`` for a weight of gate rows, then up rows: ``g`` capped at ``limit``, ``u`` clamped to
+    ``[-limit, limit]`` (None: neither); bfloat16 ``[M, N / 2]``."""
+    _need(takes_tile(x, weight, halves=True) and weight.shape[0] % 2 == 0, "the tiled kernel does not take this product")
+    half = weight.shape[0] // 2
+    out = torch.empty((x.shape[0], half), dtype=torch.bfloat16, device=x.device)
+    return _launch(x, weight, out, half, _HALVES, alpha=float(alpha), limit=float(limit or 0.0), shift=float(shift), shape=shape)

@@ -12,7 +12,7 @@ from typing import Dict, Optional
 
 import torch
 
-from ..ops import kernels, skinny
+from ..ops import kernels, skinny, tile
 from ..ops.attention import paged_attention
 from ..ops.linear import NormedRows, linear, linear_into
 from .base import (CacheNeed, LayerSlot, Mixer, ParamSpec, PartSpec, StateNeed, StepContext, build_part,
@@ -313,7 +313,12 @@ class PagedAttention(Mixer):
                 and x.data_ptr() % 16 == 0):
             qkv = skinny.split_product(self.w_in, x)   # slabs of partial sums: the rotation's kernel adds them
         else:
-            qkv = linear(x, self.w_in, out_dtype=torch.float32)
+            qkv = None
+            if (self.dtype == torch.bfloat16 and isinstance(x, torch.Tensor) and self.hd % 4 == 0
+                    and inv_freq.shape[0] % 4 == 0):
+                qkv = tile.tile_slabs(x, self.w_in)     # likewise, where many rows' tiles leave compute units idle
+            if qkv is None:
+                qkv = linear(x, self.w_in, out_dtype=torch.float32)
         cs = self._rotation_table(step, inv_freq, freq_row, m)
         return kernels.rope_kv_write(
             qkv, self.b_in, step.positions, inv_freq, freq_row,

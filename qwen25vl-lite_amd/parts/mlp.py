@@ -114,9 +114,13 @@ class ClampedGatedFF(FeedForward):
                 f"{self.names['down']}.weight": self.w_down}
 
     def forward(self, x, step: StepContext):
+        from ..ops import tile
         from ..ops.gated import gated_act
         from ..ops.linear import linear
 
+        if x.is_cuda and tile.prefers_tile(x, self.w_gate_up, halves=True):
+            act = tile.tile_gated(x, self.w_gate_up, self.alpha, self.limit, self.shift)
+            return linear_into(step.residual if step is not None else None, act, self.w_down)
         both = linear(x, self.w_gate_up)
         act = gated_act(both if both.is_contiguous() else both.contiguous(), self.alpha, self.limit, self.shift)
         return linear_into(step.residual if step is not None else None, act, self.w_down)

@@ -687,3 +687,67 @@ def test_projection_with_rotation_and_cache_write_folded_in(m, nq, nkv, hd, k, b
     assert not skinny.takes_qkv_rope(m, k, w, 24, 12, torch.bfloat16)
     assert not skinny.takes_qkv_rope(m, k, w, hd, half - 1, torch.bfloat16)
     assert not skinny.takes_qkv_rope(m, k, w, hd, half, torch.float32)
+
+
+@pytest.mark.parametrize("shape", [0, 1, 2, 3, -1])
+@pytest.mark.parametrize("m, n, k", [(65, 16, 32), (128, 256, 64), (129, 272, 96), (256, 500, 544), (257, 1040, 160), (300, 48, 2368)])
+def test_tiled_product(m, n, k, shape):
+    """The tiled kernel in every tile shape: rows and outputs at and beyond a tile's edges, inner sizes that end with
+    half a step, rows further apart than they are wide; stored as bfloat16 and float32, squared, gated both ways."""
+    from qwen25vl_lite_amd.ops import tile
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k + 8, device="cuda", generator=g).bfloat16()[:, :k]
+    w = (torch.randn(n, k + 16, device="cuda", generator=g) * 2 / k ** 0.5).bfloat16()[:, :k]
+    want = x.float() @ w.float().T
+    # float32 sums of k products of values about 1 and 2 / sqrt(k) in another order; bfloat16 keeps 8 bits
+    exact, rounded = dict(atol=2e-5, rtol=1e-4), dict(atol=1e-2, rtol=1e-2)
+    assert torch.allclose(tile.tile_product(x, w, torch.float32, shape=shape), want, **exact)
+    out = torch.empty(m, n + 24, dtype=torch.bfloat16, device="cuda")[:, 8:8 + n]
+    out[:] = 7.0
+    tile.tile_product(x, w, out=out, shape=shape)
+    assert torch.allclose(out.float(), want, **rounded)
+    assert torch.allclose(tile.tile_product(x, w, relu2=True, shape=shape).float(), want.clamp(min=0) ** 2, atol=2e-2, rtol=2e-2)
+    both = want.view(m, n // 16, 2, 8) if n % 16 == 0 else None
+    if both is not None:
+        for act, fn in (("silu", torch.nn.functional.silu), ("gelu_tanh", lambda z: torch.nn.functional.gelu(z, approximate="tanh"))):
+            ref = (fn(both[:, :, 0]) * both[:, :, 1]).reshape(m, n // 2)
+            assert torch.allclose(tile.tile_swiglu(x, w, act, shape=shape).float(), ref, atol=2e-2, rtol=2e-2)
+    gate, up = want[:, :n // 2].clamp(max=1.5), want[:, n // 2:].clamp(-1.5, 1.5)
+    ref = gate * torch.sigmoid(1.702 * gate) * (up + 1.0)
+    assert torch.allclose(tile.tile_gated(x, w, 1.702, 1.5, 1.0, shape=shape).float(), ref, atol=2e-2, rtol=2e-2)
+    gate, up = want[:, :n // 2], want[:, n // 2:]
+    assert torch.allclose(tile.tile_gated(x, w, 1.0, None, 0.0, shape=shape).float(), gate * torch.sigmoid(gate) * up, atol=3e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("m, n, k", [(65, 3584, 18944), (280, 2048, 11008), (100, 2560, 2048), (700, 272, 1376)])
+def test_tiled_product_in_ranges(m, n, k):
+    """Sums over ranges of the inner size that do not divide evenly, in float32 slabs; through the entry that joins them to
+    the residual sum too."""
+    from qwen25vl_lite_amd.ops import kernels, tile
+    from qwen25vl_lite_amd.ops.linear import linear_into
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(n, k, device="cuda", generator=g) * 2 / k ** 0.5).bfloat16()
+    want = x.float() @ w.float().T
+    slabs = tile.tile_slabs(x, w)
+    assert slabs is not None and slabs.shape[0] > 1 and slabs.dtype == torch.float32
+    assert torch.allclose(slabs.sum(0), want, atol=3e-5, rtol=1e-4)
+    h = torch.randn(m, n, device="cuda", generator=g)
+    gain = torch.rand(n, device="cuda", generator=g) + 0.5
+    total = h + want
+    normed = kernels.add_rmsnorm(h, linear_into(h, x, w), gain, 1e-6, torch.float32)
+    assert torch.allclose(h, total, atol=3e-5, rtol=1e-4)
+    ref = total * torch.rsqrt(total.pow(2).mean(-1, keepdim=True) + 1e-6) * gain
+    assert torch.allclose(normed, ref, atol=1e-4, rtol=1e-4)
+
+
+def test_tiled_product_leaves_what_it_does_not_take():
+    """Inner sizes off a step of 32, rows off 16 bytes, few rows: not taken, and the general entry still answers."""
+    from qwen25vl_lite_amd.ops import tile
+    from qwen25vl_lite_amd.ops.linear import linear
+    torch.manual_seed(0)
+    for m, n, k, off in ((100, 8192, 40, 0), (100, 8192, 64, 4), (64, 65536, 64, 0)):
+        x = torch.randn(m, k + off, device="cuda").bfloat16()[:, off:]
+        w = torch.randn(n, k, device="cuda").bfloat16()
+        assert not tile.prefers_tile(x, w)
+        assert torch.allclose(linear(x, w, out_dtype=torch.float32), x.float() @ w.float().T, atol=1e-3, rtol=1e-3)
