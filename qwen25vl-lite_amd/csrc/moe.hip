@@ -4,7 +4,7 @@
 //   products x W_e^T for every expert's pairs: gate|up with the gated activation, then down
 //   combine  the weighted sum of a token's experts, plus what a shared expert gave
 // float32 and bfloat16 storage; scores, weights and sums are float32.  A pair is p = token * top + choice.
-#include "common.h"
+#include "tile_product.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -204,6 +204,38 @@ __device__ __forceinline__ int expert_of(const int* offsets, int E, int i) {
   return e;
 }
 
+// Which expert the tile-th tile of `per` pairs belongs to, and the places of `sorted` it covers, first .. last - 1 at
+// most (e = E: there is no such tile).  Every lane looks at an expert of its own, so nothing waits for one load
+// after the other.
+struct ExpertTile {
+  int e, first, last;
+};
+__device__ __forceinline__ ExpertTile expert_tile(const int* __restrict__ offsets, int E, int tile, int per) {
+  const int lane = threadIdx.x & 63;
+  int before = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int e = e0 + lane;
+    const int f = e < E ? offsets[e] : 0, l = e < E ? offsets[e + 1] : 0;
+    const int nt = (l - f + per - 1) / per;
+    int upto = nt;                       // tiles of this expert and of those in lower lanes
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(upto, o, QVL_WAVE);
+      if (lane >= o) upto += v;
+    }
+    const int at = before + upto - nt;   // this expert's first tile
+    const unsigned long long mine = __ballot(tile >= at && tile < at + nt);
+    if (mine) {
+      const int src = __ffsll(mine) - 1;
+      const int skip = (tile - __shfl(at, src, QVL_WAVE)) * per;
+      return ExpertTile{__builtin_amdgcn_readfirstlane(e0 + src), __builtin_amdgcn_readfirstlane(__shfl(f, src, QVL_WAVE) + skip),
+                        __builtin_amdgcn_readfirstlane(__shfl(l, src, QVL_WAVE))};
+    }
+    before += __shfl(upto, 63, QVL_WAVE);
+  }
+  return ExpertTile{E, 0, 0};
+}
+
 template <typename T, typename TO>
 __global__ __launch_bounds__(256) void moe_rows_kernel(ExpertArgs a) {
   const int i = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -238,17 +270,9 @@ __global__ __launch_bounds__(256) void moe_rows_kernel(ExpertArgs a) {
 template <int MT, typename TO>
 __global__ __launch_bounds__(256) void moe_mfma_kernel(ExpertArgs a) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lg = lane >> 4, r = lane & 15;
-  constexpr int TM = 16 * MT;
-  int tile = blockIdx.x, e = 0, first = 0, last = 0;
-  for (; e < a.E; ++e) {
-    first = a.offsets[e];
-    last = a.offsets[e + 1];
-    const int nt = (last - first + TM - 1) / TM;
-    if (tile < nt) break;
-    tile -= nt;
-  }
+  const ExpertTile at_expert = expert_tile(a.offsets, a.E, blockIdx.x, 16 * MT);
+  const int e = at_expert.e, first = at_expert.first, last = at_expert.last;
   if (e >= a.E) return;
-  first += tile * TM;
   const int c0 = (blockIdx.y * 4 + wave) * 16;     // this wave's output columns
   if (c0 >= a.R) return;
   const int rows_w = a.gated ? 2 * a.R : a.R;
@@ -480,150 +504,78 @@ __global__ __launch_bounds__(256) void moe_tile_kernel(ExpertArgs a, int tiles_m
   }
 }
 
-// The same product with the fetches going straight from memory into LDS (global_load_lds_dwordx4: lane l
-// of a wave puts its 16 bytes at M0 + 16 l), up to ST_STAGES - 1 steps of K ahead of the step that is
-// multiplied, through ST_STAGES stages of LDS.  No register holds data on its way, so the waves can carry 128 x 256 tiles (8 tiles
-// of 16 rows of W each: 32 products from 12 operand reads a step) and a fetch is hidden by the steps before
-// it rather than by other waves.  Chunk c of row rho lies at place c ^ ((rho >> 2) & 3) of the row (the 16
-// lanes of an operand read hit all banks), so the lane that fills place s of row rho fetches chunk
-// s ^ ((rho >> 2) & 3).  Nothing can be replaced by zeros on this way: rows that do not exist are read from
-// rows that do (their sums are not stored), and K must be a multiple of 32.  Offsets within x and within an
-// expert's W are 32-bit.
-#define ST_K 32
-#define ST_NW 8
-#define ST_M 128
-#define ST_N (32 * ST_NW)
-#ifndef ST_STAGES
-#define ST_STAGES 5                                    // steps of K in LDS: one being multiplied, the others on their way
-#endif
-#define ST_X_SLOTS (ST_M * 4)                          // 16-byte places of x in a stage
-#define ST_SLOTS ((ST_M + ST_N) * 4)                   // and of x and W together
-#define ST_WAVE_LOADS (ST_SLOTS / 64 / 4)              // loads of 1 KB a wave issues a step
+// The same product through the inner loop of tile_product.h: tiles of 128 pairs x 256 rows of W (gated: 128 gate
+// rows and the up rows of the same outputs; a wave's gate and up values of an output end in one lane).  K must be a
+// multiple of 32 and offsets within x and within an expert's W 32-bit.  Measured on 12,384 pairs over 32 experts, K
+// 3,584: 2 x 2,368 rows 655 us (tiles of 128 x 256 with all waves in step: 874), 3,584 rows of K 2,368 320 us (480).
+typedef Tile<4, 2, 4, 4> ExpertsTile;
 
-__device__ __forceinline__ void fetch16_to_lds(const void* base, uint32_t lane_bytes, uint32_t lds_at) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_bytes), "s"(base), "s"(lds_at)
-               : "memory", "m0");
+template <typename TO>
+__device__ __forceinline__ void store_expert4(TO* o, const float* v, int n, bool whole);
+template <>
+__device__ __forceinline__ void store_expert4<float>(float* o, const float* v, int n, bool whole) {
+  if (whole) {
+    *reinterpret_cast<float4*>(o) = float4{v[0], v[1], v[2], v[3]};
+  } else {
+    for (int i = 0; i < 4; ++i)
+      if (i < n) o[i] = v[i];
+  }
 }
-// Wait until at most N of this wave's fetches are outstanding (they finish in order).
-template <int N>
-__device__ __forceinline__ void wait_fetches() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
+template <>
+__device__ __forceinline__ void store_expert4<bf16_t>(bf16_t* o, const float* v, int n, bool whole) {
+  if (whole) {
+    *reinterpret_cast<uint2*>(o) = uint2{(uint32_t)f32_to_bf16(v[0]) | (uint32_t)f32_to_bf16(v[1]) << 16,
+                                         (uint32_t)f32_to_bf16(v[2]) | (uint32_t)f32_to_bf16(v[3]) << 16};
+  } else {
+    for (int i = 0; i < 4; ++i)
+      if (i < n) o[i] = f32_to_bf16(v[i]);
+  }
 }
 
 template <bool GATED, typename TO>
-__global__ __launch_bounds__(256) void moe_stream_kernel(ExpertArgs a, int tiles_m, int tiles_n) {
-  __shared__ __attribute__((aligned(16))) uint4 stage[ST_STAGES][ST_SLOTS];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, lg = lane >> 4, r = lane & 15;
-  const int wm = wave >> 1, wn = wave & 1;
+__global__ __launch_bounds__(512) void moe_stream_kernel(ExpertArgs a, int tiles_m, int tiles_n, int whole4) {
+  typedef ExpertsTile T;
+  __shared__ __attribute__((aligned(16))) char lds[T::LDS];
+  // blocks of one XCD at a time: 4 tiles of pairs x 8 tiles of rows of W (see moe_tile_kernel)
   const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
   const int super = (idx >> 5) * 8 + xcd, inner = idx & 31;
   const int supers_m = (tiles_m + 3) / 4;
-  const int tile_n = (super / supers_m) * 8 + (inner >> 2);
-  int tile = (super % supers_m) * 4 + (inner & 3);
-  if (tile >= tiles_m || tile_n >= tiles_n) return;
-  int e = 0, first = 0, last = 0;
-  for (; e < a.E; ++e) {
-    first = a.offsets[e];
-    last = a.offsets[e + 1];
-    const int nt = (last - first + ST_M - 1) / ST_M;
-    if (tile < nt) break;
-    tile -= nt;
-  }
-  if (e >= a.E) return;
-  first += tile * ST_M;
-  constexpr int HALF = ST_N / 2;
-  constexpr int OUT_COLS = GATED ? HALF : ST_N;
+  const int tile_n = (super / supers_m) * 8 + (inner >> 2), tile_m = (super % supers_m) * 4 + (inner & 3);
+  if (tile_m >= tiles_m || tile_n >= tiles_n) return;
+  const ExpertTile at = expert_tile(a.offsets, a.E, tile_m, T::BM);
+  if (at.e >= a.E) return;
+  constexpr int OUT_COLS = GATED ? T::BN / 2 : T::BN;
   const int c0 = tile_n * OUT_COLS;
   const int rows_w = GATED ? 2 * a.R : a.R;
-  const bf16_t* we = (const bf16_t*)a.w + (size_t)e * rows_w * a.K;
-
-  // this wave's fetches of a step: places wave * ST_WAVE_LOADS * 64 ... of the stage, 64 a fetch
-  uint32_t from[ST_WAVE_LOADS];      // byte offset of this lane's 16 bytes at K = 0, within x or within W_e
+  const bf16_t* we = (const bf16_t*)a.w + (size_t)at.e * rows_w * a.K;
+  T t;
+  // rows that do not exist are read from one that does; their sums are not stored
+  t.set_rows(
+      [&](int h, int rho) {
+        if (GATED) return (uint32_t)(((size_t)(c0 + rho < a.R ? c0 + rho : 0) + (h ? a.R : 0)) * a.K * 2);
+        const int n = c0 + T::w_row(h, rho);
+        return (uint32_t)((size_t)(n < a.R ? n : 0) * a.K * 2);
+      },
+      [&](int h, int rho) {
+        const int i = at.first + T::x_row(h, rho);
+        return (uint32_t)((size_t)(a.sorted[i < at.last ? i : at.first] / a.div) * a.ldx * 2);
+      });
+  t.multiply(lds, we, a.x, (a.K + 63) / 64, a.K % 64 != 0);
 #pragma unroll
-  for (int j = 0; j < ST_WAVE_LOADS; ++j) {
-    const int place = (wave * ST_WAVE_LOADS + j) * 64 + lane;
-    if (place < ST_X_SLOTS) {
-      const int row = place >> 2, ch = (place & 3) ^ ((row >> 2) & 3);
-      const int i = first + row;
-      const int pair = a.sorted[i < last ? i : first];
-      from[j] = (uint32_t)(((size_t)(pair / a.div) * a.ldx + 8 * ch) * 2);
-    } else {
-      const int row = (place - ST_X_SLOTS) >> 2, ch = (place & 3) ^ ((row >> 2) & 3);
-      int wrow;
-      if (GATED) wrow = row < HALF ? c0 + row : a.R + c0 + (row - HALF);
-      else wrow = c0 + row;
-      const bool ok = GATED ? (c0 + (row % HALF) < a.R) : (wrow < a.R);
-      from[j] = (uint32_t)(((size_t)(ok ? wrow : 0) * a.K + 8 * ch) * 2);
-    }
-  }
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)&stage[0][0];
-  auto issue = [&](int step) {
-    const uint32_t at = lds0 + (uint32_t)(step % ST_STAGES) * (ST_SLOTS * 16) + (uint32_t)wave * (ST_WAVE_LOADS * 1024);
-    const uint32_t k_bytes = (uint32_t)step * (ST_K * 2);
+  for (int m = 0; m < T::MT; ++m) {
+    const int i = at.first + (t.wm * T::MT + m) * 16 + t.r;
+    if (i >= at.last) continue;
+    TO* o = (TO*)a.out + (size_t)a.sorted[i] * a.ldo;
 #pragma unroll
-    for (int j = 0; j < ST_WAVE_LOADS; ++j) {
-      // a fetch lies wholly in x's places or wholly in W's: the same base for all its lanes
-      const bool is_x = (wave * ST_WAVE_LOADS + j) * 64 < ST_X_SLOTS;
-      fetch16_to_lds(is_x ? (const void*)a.x : (const void*)we, from[j] + k_bytes, at + j * 1024);
-    }
-  };
-  f32x4_t acc[ST_NW][4];
+    for (int n = 0; n < (GATED ? T::NH : T::NT); ++n) {
+      const int c = c0 + (t.wn * (GATED ? T::NH : T::NT) + n) * 16 + 4 * t.g;
+      if (c >= a.R) continue;
+      float v[4];
 #pragma unroll
-  for (int n = 0; n < ST_NW; ++n)
-#pragma unroll
-    for (int m = 0; m < 4; ++m) acc[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  constexpr int PER_WAVE = GATED ? 8 * ST_NW : 16 * ST_NW;
-  int wrow0[ST_NW];
-#pragma unroll
-  for (int n = 0; n < ST_NW; ++n)
-    wrow0[n] = GATED ? (n < ST_NW / 2 ? wn * PER_WAVE + n * 16 : HALF + wn * PER_WAVE + (n - ST_NW / 2) * 16) : wn * PER_WAVE + n * 16;
-
-  const int steps = a.K / ST_K;
-#pragma unroll
-  for (int i = 0; i < ST_STAGES - 1; ++i)
-    if (i < steps) issue(i);
-  for (int s = 0; s < steps; ++s) {
-    // the steps after s that have been asked for may still be on their way: ST_STAGES - 2 of them, fewer at the end
-    const int ahead = steps - 1 - s < ST_STAGES - 2 ? steps - 1 - s : ST_STAGES - 2;
-    if (ahead >= 3) wait_fetches<3 * ST_WAVE_LOADS>();
-    else if (ahead == 2) wait_fetches<2 * ST_WAVE_LOADS>();
-    else if (ahead == 1) wait_fetches<ST_WAVE_LOADS>();
-    else wait_fetches<0>();
-    __syncthreads();                                    // every wave's part of step s is there, and step s - 1 has been multiplied
-    if (s + ST_STAGES - 1 < steps) issue(s + ST_STAGES - 1);
-    const uint4* sx = stage[s % ST_STAGES];
-    const uint4* sw = sx + ST_X_SLOTS;
-    bf16x8_t fx[4];
-#pragma unroll
-    for (int m = 0; m < 4; ++m) {
-      const int row = wm * 64 + m * 16 + r;
-      fx[m] = __builtin_bit_cast(bf16x8_t, sx[row * 4 + (lg ^ ((row >> 2) & 3))]);
-    }
-#pragma unroll
-    for (int n = 0; n < ST_NW; ++n) {
-      const int row = wrow0[n] + r;
-      const bf16x8_t fw = __builtin_bit_cast(bf16x8_t, sw[row * 4 + (lg ^ ((row >> 2) & 3))]);
-#pragma unroll
-      for (int m = 0; m < 4; ++m) acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fw, fx[m], acc[n][m], 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int m = 0; m < 4; ++m) {
-    const int i = first + wm * 64 + m * 16 + r;
-    if (i >= last) continue;
-    const int pair = a.sorted[i];
-    TO* o = (TO*)a.out + (size_t)pair * a.ldo;
-#pragma unroll
-    for (int n = 0; n < (GATED ? ST_NW / 2 : ST_NW); ++n) {
-      const int c = c0 + wn * PER_WAVE + n * 16 + 4 * lg;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (c + j >= a.R) break;
-        float v = acc[n][m][j];
-        if (GATED) v = gated_value(v, acc[n + ST_NW / 2][m][j], a.alpha, a.limit, a.shift);
-        else v = plain_value(v, a.act);
-        stf<TO>(o + c + j, v);
-      }
+      for (int j = 0; j < 4; ++j)
+        v[j] = GATED ? gated_value(t.acc[n][m][j], t.acc[n + (GATED ? T::NH : 0)][m][j], a.alpha, a.limit, a.shift)
+                     : plain_value(t.acc[n][m][j], a.act);
+      store_expert4<TO>(o + c, v, a.R - c, whole4 && c + 4 <= a.R);
     }
   }
 }
@@ -643,24 +595,23 @@ extern "C" int qvl_moe_experts(const void* x, long long ldx, int x_dtype, const 
   a.P = P; a.E = E; a.R = R; a.K = K; a.div = div; a.gated = gated; a.act = gated ? 0 : act; a.alpha = alpha; a.limit = limit; a.shift = shift;
   if (x_dtype == 1 && K % 8 == 0 && ldx % 8 == 0 && ((uintptr_t)x % 16) == 0 && ((uintptr_t)w % 16) == 0) {
     if (out_dtype != 0 && out_dtype != 1) return QVL_ERR_DTYPE;
-#ifndef MOE_NO_STREAM
     const unsigned long long x_rows = (unsigned long long)((P + div - 1) / div);
-    if (big_tiles && K % ST_K == 0 && x_rows * (unsigned long long)ldx * 2 < 0xffffff00ull &&
-        (unsigned long long)(gated ? 2 * R : R) * K * 2 < 0xffffff00ull) {
-      const int cols = gated ? ST_N / 2 : ST_N;
-      const int tiles_m = P / ST_M + (E < P ? E : P), tiles_n = (R + cols - 1) / cols;
+    if (big_tiles && K % 32 == 0 && x_rows * (unsigned long long)ldx * 2 < 0xffff0000ull &&
+        (unsigned long long)(gated ? 2 * R : R) * K * 2 < 0xffff0000ull) {
+      const int cols = gated ? ExpertsTile::BN / 2 : ExpertsTile::BN;
+      const int tiles_m = P / ExpertsTile::BM + (E < P ? E : P), tiles_n = (R + cols - 1) / cols;
       if ((long long)tiles_m * tiles_n > 0x7ffffff0ll) return QVL_ERR_LIMIT;
       const int supers = ((tiles_m + 3) / 4) * ((tiles_n + 7) / 8);
       const dim3 tgrid((unsigned)((supers + 7) / 8) * 8 * 32);
-      if (gated && out_dtype == 1)
-        hipLaunchKernelGGL((moe_stream_kernel<true, bf16_t>), tgrid, dim3(256), 0, stream, a, tiles_m, tiles_n);
-      else if (gated) hipLaunchKernelGGL((moe_stream_kernel<true, float>), tgrid, dim3(256), 0, stream, a, tiles_m, tiles_n);
-      else if (out_dtype == 1)
-        hipLaunchKernelGGL((moe_stream_kernel<false, bf16_t>), tgrid, dim3(256), 0, stream, a, tiles_m, tiles_n);
-      else hipLaunchKernelGGL((moe_stream_kernel<false, float>), tgrid, dim3(256), 0, stream, a, tiles_m, tiles_n);
+      const int whole4 = ldo % 4 == 0 && ((uintptr_t)out % 16) == 0;    // four neighbouring results as one store
+#define STREAM(G, TO) hipLaunchKernelGGL((moe_stream_kernel<G, TO>), tgrid, dim3(512), 0, stream, a, tiles_m, tiles_n, whole4)
+      if (gated && out_dtype == 1) STREAM(true, bf16_t);
+      else if (gated) STREAM(true, float);
+      else if (out_dtype == 1) STREAM(false, bf16_t);
+      else STREAM(false, float);
+#undef STREAM
       return qvl_launch_status();
     }
-#endif
     if (big_tiles) {
       const int cols = gated ? TILE_N / 2 : TILE_N;
       const int tiles_m = P / TILE_M + (E < P ? E : P), tiles_n = (R + cols - 1) / cols;
