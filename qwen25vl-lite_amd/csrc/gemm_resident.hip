@@ -4,36 +4,32 @@
 // between two products a short kernel of its own costs more than its arithmetic (its code and
 // data have just been flushed from the caches by the weights).
 //
-// A block of 16 waves owns row tiles of W (tile, tile + gridDim.x, ...).  A tile has `rows` <= 16
+// A block of 8 waves owns row tiles of W (tile, tile + gridDim.x, ...).  A tile has `rows` <= 16
 // rows of W (= outputs); the host picks `rows` so that the tiles divide evenly among the compute
-// units (3584 outputs on 256 units: 256 tiles of 14 rather than 224 of 16), the matrix-core tile's
-// other rows stay zero.
-// Wave w covers the 32 RK values of K from 32 RK w on (RK = 8: 256; a second build with RK = 4 serves
-// inner sizes up to 2,048, where with 256 values a wave half the waves would have none and the
-// other half would carry all loads), as the A operand (W rows) and B operand (X
-// rows) of v_mfma_f32_16x16x32_bf16; the 16 waves' sums meet in LDS and are added in wave order.
-// Up to 16 rows of X are one column tile of the matrix instruction; 17 to 32 rows are two (MT = 2):
-// every W fragment that is loaded is multiplied with both.  More rows are spread over teams of
-// blocks (below).
-// If K fits one pass (K <= 4096) the X operand stays in registers (the second column tile, if
-// there is one, in LDS, which takes K <= 32 * XHI_STEPS) for all of the block's tiles; W comes
-// through two half-tile buffers, each asked for again the moment its half is multiplied, so that
-// the next tile is on its way while a tile is multiplied and its sums are merged.  (A third buffer
-// fits the registers only if the compiler keeps every load in the place it was written; it does
-// not, and spills cost more than the deeper stream gains.)  A longer K is walked in passes of 4096
-// that take their turns in the same rotation (X is then read again for every pass).
+// units (3584 outputs on 256 units: 256 tiles of 14 rather than 224 of 16); the matrix-core tile's
+// other rows are read from one that exists and not stored.
+// Wave w covers the 32 RK values of K from 32 RK w on (RK = 16: 512; a second build with RK = 8 serves
+// inner sizes up to 2,048, where with 512 values a wave half the waves would have none), as the A operand (W rows)
+// and B operand (X rows) of v_mfma_f32_16x16x32_bf16; the waves' sums meet in LDS and are added in wave order.
+// Up to 16 rows of X are one column tile of the matrix instruction, 17 to 32 rows two (MT = 2): every W fragment is
+// multiplied with all of them.  X stays in the waves' registers for all of the block's tiles if K fits one pass
+// (K <= 256 RK); a longer K is walked in passes, X read again for each.  More rows are spread over
+// teams of blocks (below).
 //
-// Every load of the stream goes through a buffer descriptor (buffer_load with a byte offset that
-// the hardware checks against the buffer's size): a lane that has nothing to load (a row beyond
-// the tile, a column beyond K, a tile beyond the last) asks at an offset past the end and gets
-// zeros without any traffic.  So no load sits inside a branch, every wave issues the same loads
-// in the same order whatever its data, and the compiler can count exactly how many younger loads
-// may stay in flight at each wait (a load inside a branch costs a wait for everything: the
-// counter only says how many loads are outstanding, and the loads come back in order).
+// How W comes in decides the speed.  A load into registers in the instruction's own layout covers 16 rows of 64 bytes:
+// half a cache line a row, and each line is asked for twice (gate|up of the 7B decoder, 271.6 MB, 8 rows: 51 us = 5.3
+// TB/s; marked as read once, 54.7, the line's second half fetched anew).  So a wave brings its own columns of a tile into LDS with loads
+// that put their 16 bytes there directly, 256 bytes of 4 rows at a time, whole lines, marked as read once, and reads the
+// operands back from there.  Per call in a decode step of 8 rows of the 7B decoder: gate|up with its norm 49.9 us = 5.4
+// TB/s (51.0 with loads into registers), the head's 152,064 x 3,584 and the ranges of the down products, 16 and 128
+// calls, 40.9 on average (43.5).  A plain read of as much reaches 7.3 TB/s; without the norm gate|up takes 46: every
+// block reads and norms all rows first.  A wave waits for its own loads only (no
+// barrier but the one of the merge), four units of 128 columns go round, each asked for again the moment it has been
+// read, so that the next tile is on its way while a tile's sums are merged.
 //
 // What is folded in:
 //   prologue  PRO_NORM      X = rmsnorm(H) * w, from the float32 residual H (statistics in float32,
-//                           each wave sums its own 256 columns, the block adds the waves in order)
+//                           each wave sums its own columns, the block adds the waves in order)
 //   epilogue  EPI_RESIDUAL  out += product, out being the float32 residual
 //             EPI_SWIGLU    W's rows come in groups of 8 gate rows, 8 up rows; out[M, N/2] =
 //                           act(gate) * up, in bfloat16 (act: silu, or the tanh form of gelu)
@@ -41,6 +37,8 @@
 //                           key head takes 8 channels and the 8 channels they are rotated with
 //                           (half a head further), so the rotation happens here; queries are
 //                           written out, keys and values go straight into their page slots
+//   ranges of K             out[c] = the sums over range c of K (gemm_split below), for products whose result
+//                           joins the residual sum: the norm that follows adds the slabs in order
 #include "common.h"
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
@@ -66,26 +64,16 @@ __device__ __forceinline__ float buffer_load_f32(rsrc_t r, uint32_t byte_offset)
 
 #define HOLD_ORDER() __builtin_amdgcn_sched_barrier(0)   // nothing is scheduled across this point
 
-#ifdef QVL_TIMELINE
-// Measurement aid (never compiled into the package's library): every block's first wave stamps the
-// device's 100 MHz clock at a few places into a buffer set by qvl_gemm_resident_timeline().
-static unsigned long long* timeline_buffer = nullptr;
-extern "C" void qvl_gemm_resident_timeline(void* p) { timeline_buffer = (unsigned long long*)p; }
-#define STAMP(i)                                                                                    \
-  do {                                                                                              \
-    if (p.timeline && threadIdx.x == 0) p.timeline[blockIdx.x * 8 + (i)] = __builtin_amdgcn_s_memrealtime(); \
-  } while (0)
-#else
-#define STAMP(i)
-#endif
-
-#define W_RING 2   // half-step buffers of W that go round
-#define RW 16   // waves per block
+#define RW 8    // waves per block
 #ifndef RK
-#define RK 8    // 32-wide K steps per wave and pass (the host loads a build with 4 for inner sizes up to 2,048: all 16 waves then have columns)
+#define RK 16   // 32-wide K steps per wave and pass (the host loads a build with 8 for inner sizes up to 2,048: all waves then have columns)
 #endif
 #define PASS_K (RW * RK * 32)
-#define XHI_STEPS 120   // 32-wide K steps of the second column tile that fit LDS beside the sums: K <= 3840
+#define TWO_TILE_K (PASS_K - 256 < 3840 ? PASS_K : 3840)   // the longest K with 17 to 32 rows in one pass (4,096 would fit; the callers' rule is older and no decoder's width lies between)
+#define UNIT 4                  // K steps of a unit: 128 columns, 256 bytes a row
+#define UNIT_BYTES (16 * 256)
+#define UNIT_LOADS 4            // loads of 1 KB: 4 rows each
+#define UNITS (RK / UNIT)       // of a wave's columns
 
 enum { PRO_PLAIN = 0, PRO_NORM = 1 };
 enum { EPI_STORE = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_ROPE = 3 };
@@ -128,9 +116,7 @@ struct ResidentArgs {
   // i * stack_blocks .. and its operands and result lie i strides further on (in elements)
   int stack_blocks;      // 0: one product
   long long stack_x, stack_w, stack_o;
-#ifdef QVL_TIMELINE
-  unsigned long long* timeline;
-#endif
+  int all_k;             // ranges of one K: item i has the columns i * stack_x .. of all_k (0: every item has K columns)
 };
 
 __device__ __forceinline__ bf16x8_t load8(const bf16_t* p) {
@@ -145,19 +131,50 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
+// Lane l of the wave puts its 16 bytes at M0 + 16 l of LDS.  `once`: the lines are read by this block alone and need not stay in the caches.
+__device__ __forceinline__ void fetch16_to_lds(const void* base, uint32_t lane_bytes, uint32_t lds_at, bool once) {
+  if (once)
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(lane_bytes), "s"(base), "s"(lds_at)
+                 : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(lane_bytes), "s"(base), "s"(lds_at)
+                 : "memory", "m0");
+}
+// Wait until at most N of this wave's loads are outstanding (they finish in order).
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0f70);
+}
+__device__ __forceinline__ void wait_units(int younger) {   // all but the `younger` units asked for last have come
+  if (younger >= 3) wait_loads<3 * UNIT_LOADS>();
+  else if (younger == 2) wait_loads<2 * UNIT_LOADS>();
+  else if (younger == 1) wait_loads<UNIT_LOADS>();
+  else wait_loads<0>();
+}
+// A barrier that leaves loads from memory in flight.
+__device__ __forceinline__ void meet() {
+  __builtin_amdgcn_s_waitcnt(0xc07f);      // this wave's accesses to LDS are done
+  HOLD_ORDER();
+  __builtin_amdgcn_s_barrier();
+  HOLD_ORDER();
+}
+
 template <typename TO, int PRO, int EPI, bool ONE_PASS, int MT>
 __global__ __launch_bounds__(64 * RW) void gemm_resident_kernel(ResidentArgs p) {
   constexpr int COLS = 16 * MT;   // rows of X the block carries
-  // MT = 1: two buffers, a tile's sums are read while the next tile's are written.  MT = 2: one
-  // (LDS also holds the second column tile of X), and the norm weights borrow it before the first tile.
-  static_assert(MT == 1 || MT == 2, "one or two column tiles");
-  __shared__ __attribute__((aligned(16))) float red[MT == 1 ? 2 : 1][RW][16 * COLS];
+  constexpr int RING = MT <= 2 ? 4 : 3;
+  static_assert(MT <= 4 && (MT <= 2 || RK <= 8), "X fits the registers");
+  // MT = 1: two buffers, a tile's sums are read while the next tile's are written; else one, and a second barrier.
+  // The norm weights borrow the sums' place before the first tile.
+  constexpr int RED = MT == 1 ? 2 : 1;
+  static_assert(PRO != PRO_NORM || RK * 32 <= RED * 16 * COLS, "the norm weights fit");
+  __shared__ __attribute__((aligned(16))) char ring[RW][RING][UNIT_BYTES];
+  __shared__ __attribute__((aligned(16))) float red[RED][RW][16 * COLS];
   __shared__ float rowsq[RW][16];
-  __shared__ __attribute__((aligned(16))) float gains_own[(PRO == PRO_NORM && MT == 1) ? RW : 1][RK * 32];
-  __shared__ u32x4_t xhi[(MT == 2 && ONE_PASS) ? XHI_STEPS * 64 : 1];
-  float (*gains)[RK * 32] = MT == 1 ? gains_own : reinterpret_cast<float (*)[RK * 32]>(&red[0][0][0]);  // norm weights of each wave's columns
+  float (*gains)[RK * 32] = reinterpret_cast<float (*)[RK * 32]>(&red[0][0][0]);  // norm weights of each wave's columns
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, lg = lane >> 4, r = lane & 15;
-  const int k_lane = wave * RK * 32 + 8 * lg;  // first K index of this lane within a pass
+  const int k_wave = wave * RK * 32;           // the wave's first column within a pass
+  const int k_lane = k_wave + 8 * lg;          // first K index of this lane within a pass
   int block = blockIdx.x, blocks = gridDim.x;
   if (EPI == EPI_STORE && p.stack_blocks > 0) {
     const int item = block / p.stack_blocks;
@@ -166,13 +183,20 @@ __global__ __launch_bounds__(64 * RW) void gemm_resident_kernel(ResidentArgs p) 
     p.X += item * p.stack_x;
     p.W += item * p.stack_w;
     p.out = reinterpret_cast<TO*>(p.out) + item * p.stack_o;
+    if (p.all_k) p.K = min(p.K, p.all_k - item * (int)p.stack_x);
   }
-  STAMP(0);
   // how many of this lane's 32-wide steps of the pass that starts at k0 begin inside K (K is a
   // multiple of 8, as is every lane's first index: a step lies inside K or outside)
   auto steps_inside = [&](int k0) { return (p.K - k0 - k_lane + 31) >> 5; };
-  // what the kernel reads, each behind a descriptor that knows its size (a null pointer: size 0)
-  const rsrc_t w_buf = buffer_of(p.W, ((unsigned long long)(p.N - 1) * p.ldw + p.K) * 2);
+  // the same for the two halves of a lane's values under PRO_NORM, columns 4 lg .. and 16 + 4 lg .. of a step
+  const int inside_lo = (p.K - k_wave - 4 * lg + 31) >> 5, inside_hi = (p.K - k_wave - 16 - 4 * lg + 31) >> 5;
+  // how many units of the wave's columns of that pass hold any of K
+  auto units_inside = [&](int k0) {
+    const int n = (p.K - k0 - k_wave + 127) >> 7;
+    return n < 0 ? 0 : (n < UNITS ? n : UNITS);
+  };
+  // what the kernel reads beside W, each behind a descriptor that knows its size (a null pointer: size 0): a lane that has
+  // nothing to load asks past the end and gets zeros without traffic, so no load sits inside a branch
   const rsrc_t x_buf = buffer_of(p.X, ((unsigned long long)(p.M - 1) * p.ldx + p.K) * 2);
   const rsrc_t h_buf = buffer_of(p.H, ((unsigned long long)(p.M - 1) * p.ldh + p.K) * 4);
   const rsrc_t gain_buf = buffer_of(p.norm_w, (unsigned long long)p.K * 4);
@@ -189,77 +213,9 @@ __global__ __launch_bounds__(64 * RW) void gemm_resident_kernel(ResidentArgs p) 
     teams = (int)(gridDim.x >> 3) / p.groups * 8;
     m0 = (xcd_turn % p.groups) * COLS;
   }
-
-  // ---- the X operand of one pass ------------------------------------------------------------
-  // Column tile t holds rows 16 t .. 16 t + 15 of X.  first_w issues the block's first W loads at
-  // the point of the prologue where they fit best.  again: another column tile's norm came before
-  // (the norm weights are in LDS already, and the statistics' place may still be read).
-  auto load_x = [&](int t, int k0, bf16x8_t* xb, auto first_w, bool again = false) {
-    const int row = m0 + 16 * t + r;
-    const bool m_ok = row < p.M;
-    if (PRO == PRO_PLAIN) {
-      first_w();   // W first: it is the long wait
-      const uint32_t at = m_ok ? ((uint32_t)row * p.ldx + k0 + k_lane) * 2 : PAST_END;
-      const int inside = steps_inside(k0);
-#pragma unroll
-      for (int u = 0; u < RK; ++u)
-        xb[u] = __builtin_bit_cast(bf16x8_t, buffer_load16(x_buf, u < inside ? at : PAST_END, u * 64));
-    } else {
-      // rmsnorm of the float32 rows: this pass covers all of K (ONE_PASS), so the block's waves
-      // hold whole rows between them.  Loads return in the order they are issued: the rows and
-      // the norm weights are asked for first and W (by first_w) right behind them, so the
-      // statistics and the scaling run while W is still on its way.  A lane fetches 4 of its
-      // wave's 32 RK norm weights (the first 8 RK lanes do); they reach the lanes that need them
-      // through LDS.
-      const uint32_t at = m_ok ? ((uint32_t)row * p.ldh + k_lane) * 4 : PAST_END;
-      const int inside = steps_inside(0);
-      float4 v[RK][2];
-#pragma unroll
-      for (int u = 0; u < RK; ++u) {
-        const uint32_t o = u < inside ? at : PAST_END;
-        v[u][0] = __builtin_bit_cast(float4, buffer_load16(h_buf, o, u * 128));
-        v[u][1] = __builtin_bit_cast(float4, buffer_load16(h_buf, o, u * 128 + 16));
-      }
-      const int kg = wave * RK * 32 + 4 * lane;
-      const bool gain_lane = 4 * lane < RK * 32;
-      // beyond K the descriptor's own size gives zeros (K is a multiple of 8, kg of 4)
-      const float4 g4 =
-          __builtin_bit_cast(float4, buffer_load16(gain_buf, (again || !gain_lane) ? PAST_END : (uint32_t)kg * 4));
-      first_w();
-      float ss = 0.f;
-#pragma unroll
-      for (int u = 0; u < RK; ++u)
-        ss += v[u][0].x * v[u][0].x + v[u][0].y * v[u][0].y + v[u][0].z * v[u][0].z + v[u][0].w * v[u][0].w +
-              v[u][1].x * v[u][1].x + v[u][1].y * v[u][1].y + v[u][1].z * v[u][1].z + v[u][1].w * v[u][1].w;
-      ss += __shfl_xor(ss, 16, QVL_WAVE);
-      ss += __shfl_xor(ss, 32, QVL_WAVE);
-      asm volatile("s_nop 0" ::"v"(ss));
-      STAMP(6);   // this wave's rows have arrived
-      if (again) __syncthreads();   // the other column tile's statistics have been read
-      if (lg == 0) rowsq[wave][r] = ss;
-      if (!again && gain_lane) *reinterpret_cast<float4*>(&gains[wave][4 * lane]) = g4;
-      __syncthreads();
-      STAMP(7);   // every wave's have
-      float total = 0.f;
-#pragma unroll
-      for (int w = 0; w < RW; ++w) total += rowsq[w][r];
-      const float rs = 1.0f / sqrtf(total / (float)p.K + p.eps);
-#pragma unroll
-      for (int u = 0; u < RK; ++u) {
-        if (u < inside) {
-          const float4 g0 = *reinterpret_cast<const float4*>(&gains[wave][8 * lg + u * 32]);
-          const float4 g1 = *reinterpret_cast<const float4*>(&gains[wave][8 * lg + u * 32 + 4]);
-          u32x4_t o = {pack2((v[u][0].x * rs) * g0.x, (v[u][0].y * rs) * g0.y),
-                       pack2((v[u][0].z * rs) * g0.z, (v[u][0].w * rs) * g0.w),
-                       pack2((v[u][1].x * rs) * g1.x, (v[u][1].y * rs) * g1.y),
-                       pack2((v[u][1].z * rs) * g1.z, (v[u][1].w * rs) * g1.w)};
-          xb[u] = __builtin_bit_cast(bf16x8_t, o);
-        } else {
-          xb[u] = zero8();
-        }
-      }
-    }
-  };
+  const bool once = p.groups <= 1;            // nobody else reads the block's tiles of W
+  // Teams take tiles in turn: with runs of neighbouring tiles instead, blocks would read a multiple of a power of two
+  // of bytes apart (151,936 outputs of K 2,048: 114 us for 106).
   // the rows of a tile, and the row of W behind row i of a tile
   auto tile_rows = [&](int tile) { return (EPI == EPI_ROPE && tile < p.pair_tiles) ? 16 : p.rows; };
   auto w_row = [&](int tile, int i) {
@@ -277,37 +233,146 @@ __global__ __launch_bounds__(64 * RW) void gemm_resident_kernel(ResidentArgs p) 
     }
     return tile * p.rows + i;
   };
-  // steps u0 .. u0 + n - 1 of a tile's W operand
-  auto load_w_part = [&](int tile, int k0, int u0, int n, bf16x8_t* a) {
-    // a tile beyond the last has no rows: all of its loads are asked for past the end
-    const int row = tile < p.ntiles ? w_row(tile, r) : -1;
-    const bool row_ok = r < tile_rows(tile) && row >= 0 && row < p.N;
-    const uint32_t at = row_ok ? ((uint32_t)row * p.ldw + k0 + k_lane) * 2 : PAST_END;
-    const int inside = steps_inside(k0);
+
+  // ---- the stream of W ------------------------------------------------------------------------
+  // The wave's units in the order they are read: tile after tile, within a tile pass after pass, within a pass
+  // its units.  Row rho of a unit lies at 256 rho; place s of it holds the row's 16-byte chunk s ^ rho, so that the 16
+  // rows of an operand read touch all banks.  (ft, fp, fu): the unit asked for next.
+  const int passes = ONE_PASS ? 1 : (p.K + PASS_K - 1) / PASS_K;
+  int ft = team, fp = 0, fu = 0, f_units = units_inside(0), f_slot = 0, waiting = 0;   // waiting: units asked for and not read
+  uint32_t from[UNIT_LOADS];
+  auto set_from = [&](int tile) {
 #pragma unroll
-    for (int u = 0; u < n; ++u)
-      a[u] = __builtin_bit_cast(bf16x8_t, buffer_load16(w_buf, u0 + u < inside ? at : PAST_END, (u0 + u) * 64));
+    for (int j = 0; j < UNIT_LOADS; ++j) {
+      const int rho = 4 * j + lg;
+      int row = w_row(tile, rho);
+      if (rho >= tile_rows(tile) || row < 0 || row >= p.N) row = w_row(tile, 0);   // exists; its sums are stored once only
+      from[j] = ((uint32_t)row * p.ldw + k_wave + 8 * (r ^ rho)) * 2;
+    }
   };
-  auto load_w = [&](int tile, int k0, bf16x8_t* a) { load_w_part(tile, k0, 0, RK, a); };
+  const uint32_t ring0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)&ring[wave][0][0];
+  if (ft < p.ntiles) set_from(ft);
+  auto ask = [&]() {       // the next unit, if there is one
+    while (fu >= f_units) {
+      if (ft >= p.ntiles) return;
+      fu = 0;
+      if (++fp >= passes) {
+        fp = 0;
+        ft += teams;
+        if (ft < p.ntiles) set_from(ft);
+      }
+      f_units = units_inside(fp * PASS_K);
+      if (ft >= p.ntiles || (passes == 1 && f_units == 0)) {
+        ft = p.ntiles;
+        f_units = fu = 0;
+        return;
+      }
+    }
+    if (ft >= p.ntiles) return;
+    const int k = fp * PASS_K + fu * 128;
+    // a chunk beyond K is read from the row's first columns of the unit: it is not multiplied
+    const int left = p.K - k - k_wave;
+#pragma unroll
+    for (int j = 0; j < UNIT_LOADS; ++j) {
+      const int c = 8 * (r ^ (4 * j + lg));
+      const uint32_t at = from[j] + (uint32_t)k * 2 - (c < left ? 0u : (uint32_t)c * 2);
+      fetch16_to_lds(p.W, at, ring0 + f_slot * UNIT_BYTES + j * 1024, once);
+    }
+    f_slot = f_slot + 1 == RING ? 0 : f_slot + 1;
+    ++fu;
+    ++waiting;
+  };
+
+  auto ask_first = [&] {
+#pragma unroll
+    for (int i = 0; i < RING; ++i) ask();
+  };
+
+  // ---- the X operand of one pass ------------------------------------------------------------
+  // Column tile t holds rows 16 t .. 16 t + 15 of X.  again: another column tile's norm came before
+  // (the norm weights are in LDS already, and the statistics' place may still be read).
+  // first: the wave's first units are asked for right behind the rows.
+  auto load_x = [&](int t, int k0, bf16x8_t* xb, bool again, bool first) {
+    const int row = m0 + 16 * t + r;
+    const bool m_ok = row < p.M;
+    const int inside = steps_inside(k0);
+    if (PRO == PRO_PLAIN) {
+      const uint32_t at = m_ok ? ((uint32_t)row * p.ldx + k0 + k_lane) * 2 : PAST_END;
+#pragma unroll
+      for (int u = 0; u < RK; ++u)
+        xb[u] = __builtin_bit_cast(bf16x8_t, buffer_load16(x_buf, u < inside ? at : PAST_END, u * 64));
+      HOLD_ORDER();
+      if (first) ask_first();
+    } else {
+      // rmsnorm of the float32 rows: this pass covers all of K (ONE_PASS), so the block's waves
+      // hold whole rows between them.  A lane's eight values of a step are columns 4 lg .. and 16 + 4 lg .. (and W's
+      // operand is read likewise): a load then covers 64 neighbouring bytes of a row, not four times 16 of 128.  A lane fetches neighbouring norm weights of its wave; they reach the lanes that
+      // need them through LDS.
+      const uint32_t at = m_ok ? ((uint32_t)row * p.ldh + k_wave + 4 * lg) * 4 : PAST_END;
+      float4 v[RK][2];
+#pragma unroll
+      for (int u = 0; u < RK; ++u) {
+        v[u][0] = __builtin_bit_cast(float4, buffer_load16(h_buf, u < inside_lo ? at : PAST_END, u * 128));
+        v[u][1] = __builtin_bit_cast(float4, buffer_load16(h_buf, u < inside_hi ? at : PAST_END, u * 128 + 64));
+      }
+      constexpr int G = RK * 32 / 256;         // norm weights of the wave, 4 a lane, 256 a load
+      float4 g4[G];
+#pragma unroll
+      for (int i = 0; i < G; ++i)
+        g4[i] = __builtin_bit_cast(float4, buffer_load16(gain_buf, again ? PAST_END : (uint32_t)(k_wave + 256 * i + 4 * lane) * 4));
+      HOLD_ORDER();
+      if (first) ask_first();
+      float ss = 0.f;
+#pragma unroll
+      for (int u = 0; u < RK; ++u)
+        ss += v[u][0].x * v[u][0].x + v[u][0].y * v[u][0].y + v[u][0].z * v[u][0].z + v[u][0].w * v[u][0].w +
+              v[u][1].x * v[u][1].x + v[u][1].y * v[u][1].y + v[u][1].z * v[u][1].z + v[u][1].w * v[u][1].w;
+      ss += __shfl_xor(ss, 16, QVL_WAVE);
+      ss += __shfl_xor(ss, 32, QVL_WAVE);
+      if (again) meet();   // the other column tile's statistics have been read
+      if (lg == 0) rowsq[wave][r] = ss;
+      if (!again) {
+#pragma unroll
+        for (int i = 0; i < G; ++i) *reinterpret_cast<float4*>(&gains[wave][256 * i + 4 * lane]) = g4[i];
+      }
+      meet();
+      float total = 0.f;
+#pragma unroll
+      for (int w = 0; w < RW; ++w) total += rowsq[w][r];
+      const float rs = 1.0f / sqrtf(total / (float)p.K + p.eps);
+#pragma unroll
+      for (int u = 0; u < RK; ++u) {
+        if (u < inside_lo) {
+          const float4 g0 = *reinterpret_cast<const float4*>(&gains[wave][4 * lg + u * 32]);
+          const float4 g1 = *reinterpret_cast<const float4*>(&gains[wave][4 * lg + u * 32 + 16]);
+          u32x4_t o = {pack2((v[u][0].x * rs) * g0.x, (v[u][0].y * rs) * g0.y),
+                       pack2((v[u][0].z * rs) * g0.z, (v[u][0].w * rs) * g0.w),
+                       pack2((v[u][1].x * rs) * g1.x, (v[u][1].y * rs) * g1.y),
+                       pack2((v[u][1].z * rs) * g1.z, (v[u][1].w * rs) * g1.w)};
+          xb[u] = __builtin_bit_cast(bf16x8_t, o);
+        } else {
+          xb[u] = zero8();
+        }
+      }
+    }
+  };
   // What the epilogue of a tile reads from memory, for the element (m, nl) this thread finishes.
-  // Loads return in the order they are issued, so these are asked for before the W loads of the
-  // next tile: waiting for them must not wait for those.
   struct Epi {
     float bias, old;
     float2 cs;
     int slot;
   };
-  auto epi_load = [&](int tile) {
+  constexpr int EPT = (16 * COLS + 64 * RW - 1) / (64 * RW);   // elements of a tile a thread finishes
+  auto epi_load = [&](int tile, int i) {
     Epi e;
     e.bias = e.old = 0.f;
     e.cs = float2{1.f, 0.f};
     e.slot = -1;
-    if (EPI == EPI_SWIGLU) return e;
-    // Every thread asks, the ones without an element past the end (and gets zeros): the same loads
-    // on every path.  The waves beyond the first 16 COLS threads have no element at all.
-    const int m = m0 + (threadIdx.x >> 4), nl = threadIdx.x & 15;
+    if (EPI == EPI_SWIGLU || (EPI == EPI_STORE && !p.bias)) return e;
+    const int el = threadIdx.x + 64 * RW * i;
+    const int m = m0 + (el >> 4), nl = el & 15;
     const int n = tile < p.ntiles ? w_row(tile, nl) : -1;
-    const bool live = threadIdx.x < 16 * COLS && m < p.M && nl < tile_rows(tile) && n >= 0 && n < p.N;
+    const bool live = el < 16 * COLS && m < p.M && nl < tile_rows(tile) && n >= 0 && n < p.N;
     e.bias = buffer_load_f32(bias_buf, live ? (uint32_t)n * 4 : PAST_END);
     if (EPI == EPI_RESIDUAL) e.old = buffer_load_f32(old_buf, live ? ((uint32_t)m * p.ldo + n) * 4 : PAST_END);
     if (EPI == EPI_ROPE) {
@@ -325,20 +390,20 @@ __global__ __launch_bounds__(64 * RW) void gemm_resident_kernel(ResidentArgs p) 
   // A wave's sums lie as [row of X][row of the tile]: a lane writes its four at once, and the
   // thread that finishes element e = 16 m + nl reads word e of every wave.
   // MT = 1, one barrier per tile: the sums go into the buffer that was read two tiles ago; whoever
-  // reads it (the first four waves) has passed the barrier of the tile in between since.
-  // MT = 2, one buffer: a second barrier keeps the next tile's sums out until these are read.
-  struct Acc {
-    f32x4_t t[MT];
-  };
+  // reads it has passed the barrier of the tile in between since.
+  // Else one buffer: a second barrier keeps the next tile's sums out until these are read.
+  f32x4_t acc[MT];
   int parity = 0;
-  auto finish = [&](int tile, const Acc& acc, const Epi& epi) {
+  auto finish = [&](int tile, const Epi* epi) {
     float (*buf)[16 * COLS] = red[MT == 1 ? parity : 0];
     parity ^= 1;
 #pragma unroll
-    for (int t = 0; t < MT; ++t) *reinterpret_cast<f32x4_t*>(&buf[wave][(16 * t + r) * 16 + 4 * lg]) = acc.t[t];
-    __syncthreads();
-    if (threadIdx.x < 16 * COLS) {
-      const int e = threadIdx.x;
+    for (int t = 0; t < MT; ++t) *reinterpret_cast<f32x4_t*>(&buf[wave][(16 * t + r) * 16 + 4 * lg]) = acc[t];
+    meet();
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) {
+      const int e = threadIdx.x + 64 * RW * i;
+      if (e >= 16 * COLS) continue;
       const int m = m0 + (e >> 4), nl = e & 15, n = w_row(tile, nl);
       float sum = 0.f;
 #pragma unroll
@@ -350,17 +415,17 @@ __global__ __launch_bounds__(64 * RW) void gemm_resident_kernel(ResidentArgs p) 
           o[(size_t)m * p.ldo + (n >> 4) * 8 + (n & 7)] = f32_to_bf16(gate_act(sum, p.gelu) * up);
         }
       } else if (EPI == EPI_ROPE) {
-        sum += epi.bias;
+        sum += epi[i].bias;
         const float other = __shfl_xor(sum, 8, QVL_WAVE);   // the channel this one is rotated with
         const int head = n / p.hd, d = n - head * p.hd;
         if (m < p.M && nl < tile_rows(tile) && n < p.N) {
           // (cos, sin) is (1, 0) for value heads; rows 0..7 of a rotated tile are the first halves
-          const float val = (nl < 8 || head >= p.nq + p.nkv) ? sum * epi.cs.x - other * epi.cs.y
-                                                              : sum * epi.cs.x + other * epi.cs.y;
+          const float val = (nl < 8 || head >= p.nq + p.nkv) ? sum * epi[i].cs.x - other * epi[i].cs.y
+                                                              : sum * epi[i].cs.x + other * epi[i].cs.y;
           if (head < p.nq) {
             p.q_out[((size_t)m * p.nq + head) * p.hd + d] = f32_to_bf16(val);
-          } else if (epi.slot >= 0) {
-            const size_t page = (size_t)(epi.slot / p.ps), off = (size_t)(epi.slot % p.ps);
+          } else if (epi[i].slot >= 0) {
+            const size_t page = (size_t)(epi[i].slot / p.ps), off = (size_t)(epi[i].slot % p.ps);
             if (head < p.nq + p.nkv)
               p.kc[((page * p.nkv + (head - p.nq)) * p.ps + off) * p.hd + d] = f32_to_bf16(val);
             else
@@ -368,154 +433,96 @@ __global__ __launch_bounds__(64 * RW) void gemm_resident_kernel(ResidentArgs p) 
           }
         }
       } else if (m < p.M && nl < p.rows && n < p.N) {
-        sum += epi.bias;
+        sum += epi[i].bias;
         if (EPI == EPI_STORE && p.gelu == ACT_RELU2) {
           sum = fmaxf(sum, 0.f);
           sum *= sum;
         }
         if (EPI == EPI_RESIDUAL) {
           float* o = reinterpret_cast<float*>(p.out);
-          o[(size_t)m * p.ldo + n] = epi.old + sum;
+          o[(size_t)m * p.ldo + n] = epi[i].old + sum;
         } else {
           stf<TO>(reinterpret_cast<TO*>(p.out) + (size_t)m * p.ldo + n, sum);
         }
       }
     }
-    if (MT >= 2) __syncthreads();
+    if (MT >= 2) meet();
   };
-  // The W operand's steps come as two halves (a_lo, a_hi).  x1: the second column tile's operand in
-  // registers; null: it is in LDS (one pass), except for the waves whose steps lie beyond K then.
-  const bool hi_live = wave * RK < XHI_STEPS;
-  // steps u0 .. u0 + n - 1 of a tile, whose W operands are a[0 .. n - 1]
-  auto product_part = [&](const bf16x8_t* a, int u0, int n, const bf16x8_t* x0, const bf16x8_t* x1, Acc acc) {
-#pragma unroll
-    for (int i = 0; i < n; ++i) {
-      const int u = u0 + i;
-      acc.t[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], x0[u], acc.t[0], 0, 0, 0);
-      if (MT == 2) {
-        if (!ONE_PASS)
-          acc.t[MT - 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], x1[u], acc.t[MT - 1], 0, 0, 0);
-        else if (hi_live)
-          acc.t[MT - 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              a[i], __builtin_bit_cast(bf16x8_t, xhi[(wave * RK + u) * 64 + lane]), acc.t[MT - 1], 0, 0, 0);
-      }
-    }
-    return acc;
-  };
-  auto product = [&](const bf16x8_t* a_lo, const bf16x8_t* a_hi, const bf16x8_t* x0, const bf16x8_t* x1, Acc acc) {
-    acc = product_part(a_lo, 0, RK / 2, x0, x1, acc);
-    return product_part(a_hi, RK / 2, RK / 2, x0, x1, acc);
-  };
-  // half of the plain X operand of the pass that starts at k0 (column tile 0): steps half * RK / 2 ...
-  auto load_x_half = [&](int k0, int half, bf16x8_t* xb) {
-    const int row = m0 + r;
-    const bool m_ok = row < p.M;
-    const uint32_t at = m_ok ? ((uint32_t)row * p.ldx + k0 + k_lane) * 2 : PAST_END;
-    const int inside = steps_inside(k0);
-#pragma unroll
-    for (int i = 0; i < RK / 2; ++i) {
-      const int u = half * (RK / 2) + i;
-      xb[u] = __builtin_bit_cast(bf16x8_t, buffer_load16(x_buf, u < inside ? at : PAST_END, u * 64));
-    }
-  };
-  Acc zero;
-#pragma unroll
-  for (int t = 0; t < MT; ++t) zero.t[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
-  if (ONE_PASS || MT == 1) {
-    // The block's work is a sequence of steps: every tile of its own, and within a tile every pass
-    // over K (one, if X stays resident).  Two half-step buffers of W go round: each is asked for
-    // again, for the next step, as soon as the product has freed its registers, and arrives during
-    // the merge of the sums (or, between the passes of a tile, while the next rows of X come).
-    const int passes = ONE_PASS ? 1 : (p.K + PASS_K - 1) / PASS_K;
-    auto step_after = [&](int& t, int& ps) {
-      if (++ps >= passes) {
-        ps = 0;
-        t += teams;
-      }
-    };
-    bf16x8_t xb[RK];
-    bf16x8_t w[W_RING][RK / 2];
-    int tile = team, pass = 0;
-    if (MT == 1) {
-      load_x(0, 0, xb, [&] {
-        load_w_part(tile, 0, 0, RK / 2, w[0]);
-        load_w_part(tile, 0, RK / 2, RK / 2, w[1]);
-      });
-    } else {
-      // rows 16..31 first, while few registers are taken: each lane keeps its own operands of
-      // them in LDS and reads them back itself
-      bf16x8_t hi[RK];
-      load_x(1, 0, hi, [&] { load_w_part(tile, 0, 0, RK / 2, w[0]); });
+  bf16x8_t xb[MT][RK];
+  auto load_all_x = [&](int k0, bool first) {
 #pragma unroll
-      for (int u = 0; u < RK; ++u)
-        if (hi_live) xhi[(wave * RK + u) * 64 + lane] = __builtin_bit_cast(u32x4_t, hi[u]);
-      load_x(0, 0, xb, [&] { load_w_part(tile, 0, RK / 2, RK / 2, w[1]); }, true);
-      if (PRO == PRO_NORM) __syncthreads();   // the norm weights lie where the first tile's sums go
-    }
-    STAMP(1);   // the rows are in their registers, the first tile asked for
-    Epi e = epi_load(tile);
-    Acc acc = zero;
-    // one step whose halves are in a_lo and a_hi; false: it was the block's last
-    // A half buffer is asked for again the moment its steps are multiplied (not after the whole
-    // step).  Between the passes of a tile the next rows of X are asked for the same way, each half
-    // ahead of the W half that is needed with it (loads come back in the order they were asked
-    // for).  Every step issues the same loads, a step beyond the block's last one past the end of
-    // the buffers.  (A ring of three half buffers, the free one taking the first half of the step
-    // after next, needs more registers than a lane has: the compiler spills, and a spill's scratch
-    // store makes every wait a wait for everything.)
-    auto one = [&](bf16x8_t* a_lo, bf16x8_t* a_hi) {
-      int tn = tile, pn = pass;
-      step_after(tn, pn);
-      const bool tile_done = ONE_PASS || pn == 0;
-      // the order below is the order of the instructions: the compiler's scheduler would pull the
-      // loads of later steps ahead of the products and run out of registers for them
-      HOLD_ORDER();
-      acc = product_part(a_lo, 0, RK / 2, xb, nullptr, acc);
-      if (tile == team) { asm volatile("s_nop 0" :: "v"(acc.t[0])); STAMP(2); }   // the first half tile was there
-      HOLD_ORDER();
-      if (!ONE_PASS && MT == 1) load_x_half(pn * PASS_K, 0, xb);
-      load_w_part(tn, pn * PASS_K, 0, RK / 2, a_lo);
-      HOLD_ORDER();
-      acc = product_part(a_hi, RK / 2, RK / 2, xb, nullptr, acc);
-      HOLD_ORDER();
-      const Epi e_next = epi_load(tn);
-      if (!ONE_PASS && MT == 1) load_x_half(pn * PASS_K, 1, xb);
-      load_w_part(tn, pn * PASS_K, RK / 2, RK / 2, a_hi);
-      HOLD_ORDER();
-      if (tile_done) {
-        if (tile == team) STAMP(3);   // all of the first tile multiplied
-        finish(tile, acc, e);
-        if (tile == team) STAMP(4);   // and merged and written
-        acc = zero;
-        e = e_next;
+    for (int t = MT - 1; t >= 0; --t) load_x(t, k0, xb[t], t != MT - 1, first && t == MT - 1);
+    // From here on the waits are counted: the compiler, which does not know of the units, would wait for the rows
+    // behind units that are asked for later.
+    wait_loads<0>();
+    if (PRO == PRO_NORM) meet();   // the norm weights lie where the first tile's sums go
+  };
+  if (ONE_PASS) load_all_x(0, true);
+  else ask_first();
+  int slot = 0;
+  for (int tile = team; tile < p.ntiles; tile += teams) {
+    Epi e[EPT];
+#pragma unroll
+    for (int i = 0; i < EPT; ++i) e[i] = epi_load(tile, i);
+#pragma unroll
+    for (int t = 0; t < MT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int pass = 0; pass < passes; ++pass) {
+      const int k0 = pass * PASS_K;
+      if (!ONE_PASS) load_all_x(k0, false);
+      const int inside = steps_inside(k0), units = units_inside(k0);
+#pragma unroll
+      for (int u = 0; u < UNITS; ++u) {
+        if (u >= units) break;
+        HOLD_ORDER();
+        wait_units(waiting - 1);
+        HOLD_ORDER();
+        const char* at = &ring[wave][slot][r * 256];
+        bf16x8_t a[UNIT];
+#pragma unroll
+        for (int i = 0; i < UNIT; ++i) {
+          if (PRO == PRO_NORM) {
+            const int c = 4 * i + (lg >> 1), half = (lg & 1) * 8;
+            const uint2 lo = *reinterpret_cast<const uint2*>(at + ((c ^ r) << 4) + half);
+            const uint2 hi = *reinterpret_cast<const uint2*>(at + (((c + 2) ^ r) << 4) + half);
+            a[i] = __builtin_bit_cast(bf16x8_t, u32x4_t{lo.x, lo.y, hi.x, hi.y});
+          } else {
+            a[i] = *reinterpret_cast<const bf16x8_t*>(at + (((4 * i + lg) ^ r) << 4));
+          }
+        }
+        if (p.K - k0 - k_wave < 128 * (u + 1)) {     // the unit in which K ends: what lies beyond is no part of the sum
+#pragma unroll
+          for (int i = 0; i < UNIT; ++i) {
+            if (PRO == PRO_NORM) {
+              u32x4_t v = __builtin_bit_cast(u32x4_t, a[i]);
+              if (u * UNIT + i >= inside_lo) v.x = v.y = 0u;
+              if (u * UNIT + i >= inside_hi) v.z = v.w = 0u;
+              a[i] = __builtin_bit_cast(bf16x8_t, v);
+            } else if (u * UNIT + i >= inside) {
+              a[i] = zero8();
+            }
+          }
+        }
+        __builtin_amdgcn_s_waitcnt(0xc07f);          // the unit has been read: its place may be filled again
+        HOLD_ORDER();
+        slot = slot + 1 == RING ? 0 : slot + 1;
+        --waiting;
+        ask();
+        HOLD_ORDER();
+#pragma unroll
+        for (int i = 0; i < UNIT; ++i)
+#pragma unroll
+          for (int t = 0; t < MT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], xb[t][u * UNIT + i], acc[t], 0, 0, 0);
       }
-      tile = tn;
-      pass = pn;
-      return tn < p.ntiles;
-    };
-    while (tile < p.ntiles) {
-      if (!one(w[0], w[1])) break;
     }
-    STAMP(5);
-  } else {
-    for (int tile = team; tile < p.ntiles; tile += teams) {
-      Acc acc = zero;
-      const Epi e = epi_load(tile);
-      for (int k0 = 0; k0 < p.K; k0 += PASS_K) {
-        bf16x8_t xb[RK], x1[MT == 2 ? RK : 1], a[RK];
-        load_x(0, k0, xb, [&] { load_w(tile, k0, a); });
-        if (MT == 2) load_x(1, k0, x1, [] {}, true);
-        acc = product(a, a + RK / 2, xb, x1, acc);
-      }
-      finish(tile, acc, e);
-    }
+    finish(tile, e);
   }
+  wait_loads<0>();       // nothing may land in LDS that is no longer this block's
 }
 
 // How M rows are carried: column tiles per block (MT), blocks per team (groups), and whether X stays
 // in the block for all its tiles (one pass over K).  Up to 32 rows one block carries them all.
-// More rows, or 17 to 32 rows with a K too long for the second column tile's place in LDS, are
+// More rows, or 17 to 32 rows with a norm and a K too long for one pass, are
 // spread over the blocks of a team; a device with too few compute units for teams (fewer than 8
 // per group) is refused (mt = 0).
 struct Plan {
@@ -524,7 +531,7 @@ struct Plan {
 };
 static Plan plan_for(int M, int K, bool norm, int blocks) {
   if (M <= 16) return Plan{1, 1, K <= PASS_K};
-  const bool two_fit = K <= 32 * XHI_STEPS;
+  const bool two_fit = K <= TWO_TILE_K;
   if (M <= 32 && two_fit) return Plan{2, 1, true};
   if (two_fit && blocks >= 8 * ((M + 31) / 32)) return Plan{2, (M + 31) / 32, true};
   const int singles = (M + 15) / 16;
@@ -575,7 +582,7 @@ extern "C" unsigned long long qvl_gemm_resident_max_weight_bytes() { return BUFF
 
 extern "C" int qvl_gemm_resident_pass_k() { return PASS_K; }
 // the longest K with which 17 to 32 rows stay resident (and with which their norm is folded in)
-extern "C" int qvl_gemm_resident_two_tile_k() { return 32 * XHI_STEPS; }
+extern "C" int qvl_gemm_resident_two_tile_k() { return TWO_TILE_K; }
 
 // x: bfloat16 [M, K] (h null), or h: float32 [M, K] with norm_w [K] and eps (x null): X = rmsnorm(h) * norm_w.
 // epilogue 0: out[M, N] in out_dtype (0 float32, 1 bfloat16); 1: out (float32 [M, N]) += product;
@@ -610,10 +617,7 @@ extern "C" int qvl_gemm_resident(const void* x, int ldx, const void* h, int ldh,
   ResidentArgs p;
   p.X = (const bf16_t*)x; p.ldx = ldx; p.H = (const float*)h; p.ldh = ldh; p.norm_w = (const float*)norm_w;
   p.eps = eps; p.W = (const bf16_t*)W; p.ldw = ldw; p.bias = (const float*)bias; p.out = out; p.ldo = ldo;
-  p.M = M; p.N = N; p.K = K; p.gelu = gelu; p.stack_blocks = 0; p.stack_x = p.stack_w = p.stack_o = 0;
-#ifdef QVL_TIMELINE
-  p.timeline = timeline_buffer;
-#endif
+  p.M = M; p.N = N; p.K = K; p.gelu = gelu; p.stack_blocks = 0; p.stack_x = p.stack_w = p.stack_o = 0; p.all_k = 0;
   p.cs = nullptr; p.slot = nullptr;
   p.q_out = nullptr; p.kc = nullptr; p.vc = nullptr; p.nq = p.nkv = p.hd = p.ps = 0; p.pair_tiles = 0;
   // as many rounds of tiles as 16-row tiles need, with rows per tile cut down to what fills them evenly
@@ -661,9 +665,6 @@ extern "C" int qvl_gemm_resident_stack(const void* x, int ldx, long long x_strid
   ResidentArgs p;
   p.X = (const bf16_t*)x; p.ldx = ldx; p.H = nullptr; p.ldh = 0; p.norm_w = nullptr; p.eps = 0.f; p.W = (const bf16_t*)W;
   p.ldw = ldw; p.bias = nullptr; p.out = out; p.ldo = ldo; p.M = M; p.N = N; p.K = K; p.gelu = 0; p.groups = 1;
-#ifdef QVL_TIMELINE
-  p.timeline = nullptr;
-#endif
   p.cs = nullptr; p.slot = nullptr;
   p.q_out = nullptr; p.kc = nullptr; p.vc = nullptr; p.nq = p.nkv = p.hd = p.ps = 0; p.pair_tiles = 0;
   const long long rounds = (N + 16LL * share - 1) / (16LL * share);
@@ -671,7 +672,7 @@ extern "C" int qvl_gemm_resident_stack(const void* x, int ldx, long long x_strid
   p.ntiles = (N + p.rows - 1) / p.rows;
   p.whole_tiles = p.ntiles; p.parts = 1; p.pairs = 8;
   p.stack_blocks = share < p.ntiles ? share : p.ntiles;
-  p.stack_x = x_stride; p.stack_w = w_stride; p.stack_o = o_stride;
+  p.stack_x = x_stride; p.stack_w = w_stride; p.stack_o = o_stride; p.all_k = 0;
   const dim3 grid(p.stack_blocks * count), block(64 * RW);
 #define QVL_STACK(TO)                                                                                                      \
   if (pl.mt == 1) hipLaunchKernelGGL((gemm_resident_kernel<TO, PRO_PLAIN, EPI_STORE, true, 1>), grid, block, 0, stream, p); \
@@ -680,6 +681,73 @@ extern "C" int qvl_gemm_resident_stack(const void* x, int ldx, long long x_strid
   else if (out_dtype == 1) { QVL_STACK(bf16_t); }
   else return QVL_ERR_DTYPE;
 #undef QVL_STACK
+  return qvl_launch_status();
+}
+
+// Ranges of K over blocks: how a product is cut on a device with `cus` compute units.  A block carries all rows for at most
+// PASS_K columns; among the numbers of ranges around the least possible the one is taken whose busiest block
+// reads the fewest bytes (7B down projection, 3,584 x 18,944: 5 ranges of 51 blocks with up to 5 tiles of 15 rows), each
+// range beyond the least costing a slab more for the norm that adds them.
+struct Cut {
+  int chunks, chunk_k, per_chunk, rows, ntiles;
+};
+static Cut cut_for(int M, int N, int K, int cus) {
+  const int least = (K + PASS_K - 1) / PASS_K;
+  Cut best{0, 0, 0, 0, 0};
+  double best_cost = 1e30;
+  for (int chunks = least; chunks <= least + 6 && chunks <= cus; ++chunks) {
+    Cut c;
+    c.chunks = chunks;
+    c.chunk_k = ((K + chunks - 1) / chunks + 31) / 32 * 32;
+    if (c.chunk_k > PASS_K || (long long)c.chunk_k * (chunks - 1) >= K) continue;
+    c.per_chunk = cus / chunks;
+    const long long per_round = 16LL * c.per_chunk, rounds = (N + per_round - 1) / per_round;
+    c.rows = (int)((N + rounds * c.per_chunk - 1) / (rounds * c.per_chunk));
+    c.ntiles = (N + c.rows - 1) / c.rows;
+    if (c.per_chunk > c.ntiles) c.per_chunk = c.ntiles;
+    const long long tiles = (c.ntiles + c.per_chunk - 1) / c.per_chunk;
+    const double cost = (double)tiles * c.rows * c.chunk_k * 2 * cus + 16.0 * chunks * M * N;
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = c;
+    }
+  }
+  return best;
+}
+
+// Whether qvl_gemm_split takes these sizes, and how many slabs it then writes (0: it does not).  More than 32 rows are
+// taken by the build with RK = 8 only (a wave's columns of four column tiles fill its registers).
+extern "C" int qvl_gemm_split_chunks(int M, int N, int K, int cus) {
+  if (M <= 0 || M > (RK <= 8 ? 64 : 32) || N <= 0 || K <= 0 || K % 8 || cus <= 0) return 0;
+  return cut_for(M, N, K, cus).chunks;
+}
+
+// x: bfloat16 [M, K] (ldx elements a row).  W: bfloat16 [N, K].  out: float32 [chunks][M][N], chunks =
+// qvl_gemm_split_chunks(M, N, K, cus); the product is the sum of the slabs.  K a multiple of 8.
+extern "C" int qvl_gemm_split(const void* x, int ldx, const void* W, int ldw, void* out, int M, int N, int K, int cus,
+                              hipStream_t stream) {
+  if (M <= 0 || N <= 0) return QVL_OK;
+  if (M > 64) return QVL_ERR_LIMIT;
+  if (K <= 0 || K % 8 || ldw % 8 || ldw < K || ldx % 8 || ldx < K || cus <= 0 || !x || !W || !out) return QVL_ERR_SHAPE;
+  if (!fits_descriptors(M, N, K, ldw, ldx, 0, 0)) return QVL_ERR_LIMIT;
+  if (qvl_gemm_split_chunks(M, N, K, cus) == 0) return QVL_ERR_LIMIT;
+  const Cut c = cut_for(M, N, K, cus);
+  ResidentArgs p;
+  p.X = (const bf16_t*)x; p.ldx = ldx; p.H = nullptr; p.ldh = 0; p.norm_w = nullptr; p.eps = 0.f; p.W = (const bf16_t*)W;
+  p.ldw = ldw; p.bias = nullptr; p.out = out; p.ldo = N; p.M = M; p.N = N; p.K = c.chunk_k; p.gelu = 0; p.groups = 1;
+  p.cs = nullptr; p.slot = nullptr;
+  p.q_out = nullptr; p.kc = nullptr; p.vc = nullptr; p.nq = p.nkv = p.hd = p.ps = 0; p.pair_tiles = 0;
+  p.rows = c.rows; p.ntiles = c.ntiles; p.whole_tiles = c.ntiles; p.parts = 1; p.pairs = 8;
+  p.stack_blocks = c.per_chunk; p.stack_x = p.stack_w = c.chunk_k; p.stack_o = (long long)M * N; p.all_k = K;
+  const dim3 grid(c.chunks * c.per_chunk), block(64 * RW);
+#define QVL_SPLIT(MT) hipLaunchKernelGGL((gemm_resident_kernel<float, PRO_PLAIN, EPI_STORE, true, MT>), grid, block, 0, stream, p)
+  if (M <= 16) QVL_SPLIT(1);
+  else if (M <= 32) QVL_SPLIT(2);
+#if RK <= 8
+  else if (M <= 48) QVL_SPLIT(3);
+  else QVL_SPLIT(4);
+#endif
+#undef QVL_SPLIT
   return qvl_launch_status();
 }
 
@@ -714,10 +782,7 @@ extern "C" int qvl_gemm_resident_rope(const void* x, int ldx, const void* h, int
   ResidentArgs p;
   p.X = (const bf16_t*)x; p.ldx = ldx; p.H = (const float*)h; p.ldh = ldh; p.norm_w = (const float*)norm_w;
   p.eps = eps; p.W = (const bf16_t*)W; p.ldw = ldw; p.bias = (const float*)bias; p.out = nullptr; p.ldo = 0;
-  p.M = M; p.N = (nq + 2 * nkv) * hd; p.K = K; p.gelu = 0; p.stack_blocks = 0; p.stack_x = p.stack_w = p.stack_o = 0;
-#ifdef QVL_TIMELINE
-  p.timeline = timeline_buffer;
-#endif
+  p.M = M; p.N = (nq + 2 * nkv) * hd; p.K = K; p.gelu = 0; p.stack_blocks = 0; p.stack_x = p.stack_w = p.stack_o = 0; p.all_k = 0;
   // query and key heads in tiles of 8 + 8 rows, then the value rows in tiles as small as fills
   // the compute units evenly (36 heads of 128 on 256 units: 256 tiles of 16 and 256 of 2)
   p.pair_tiles = (nq + nkv) * (hd / 16);

@@ -16,8 +16,7 @@ LIBRARIES = [
     ("gemm_f32", {}),
     ("sample", {}),
     ("gemm_resident", {}),
-    ("gemm_resident", {"RK": 4}),
-    ("gemm_split", {}),
+    ("gemm_resident", {"RK": 8}),
     ("gemm_tile", {}),
     ("peaks", {}),
     ("gated", {}),

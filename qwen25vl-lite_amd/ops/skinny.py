@@ -35,14 +35,19 @@ def _rows_aligned(t: torch.Tensor, elems: int) -> bool:
     return t.stride(1) == 1 and t.stride(0) % elems == 0 and t.data_ptr() % 16 == 0
 
 
-NARROW_K = 2048   # up to this inner size the resident kernel's build with 128 columns a wave runs
+NARROW_K = 2048   # up to this inner size the resident kernel's build with 256 columns a wave runs
 
 
 def _build_for(k: int):
-    """The build of the resident kernel for an inner size: with 256 columns a wave, half of a
-    block's 16 waves have no columns of an inner size of 2,048 and the other half carry all loads
-    (the 3B decoder's gate | up product: 24.4 us against 17.7 with 128 columns a wave)."""
-    return {"RK": 4} if k <= NARROW_K else None
+    """The build of the resident kernel for an inner size: with 512 columns a wave, half of a
+    block's 8 waves have no columns of an inner size of 2,048 and the other half carry all loads."""
+    return {"RK": 8} if k <= NARROW_K else None
+
+
+def _split_build(m: int):
+    """The build that cuts a product of ``m`` rows into ranges of its inner size: up to 32 rows a wave keeps 512 columns of
+    them in registers, up to 64 rows 256."""
+    return None if m <= ONE_BLOCK_ROWS else {"RK": 8}
 
 
 def resident_norm_k() -> int:
@@ -218,7 +223,7 @@ SPLIT_ROWS = 64   # the most rows the split kernel is built for
 
 
 def takes_split(m: int, k: int, weight: torch.Tensor) -> bool:
-    """Whether the split kernel (``csrc/gemm_split.hip``) takes a product of ``m`` rows with this
+    """Whether the split kernel (in ``csrc/gemm_resident.hip``) takes a product of ``m`` rows with this
     weight: up to 64 bfloat16 rows, whose partial sums over chunks of the inner size come back as
     slabs."""
     if not (1 <= m <= SPLIT_ROWS and k % 8 == 0 and weight.dtype == torch.bfloat16 and _rows_aligned(weight, 8)):
@@ -227,7 +232,7 @@ def takes_split(m: int, k: int, weight: torch.Tensor) -> bool:
     if ((n - 1) * weight.stride(0) + k) * 2 >= _MAX_WEIGHT_BYTES:
         return False
     cus = _compute_units(weight.device)
-    return int(_fn("gemm_split", "qvl_gemm_split_chunks", [_c_int, _c_int, _c_int, _c_int])(m, n, k, cus)) > 0
+    return int(_fn("gemm_resident", "qvl_gemm_split_chunks", [_c_int, _c_int, _c_int, _c_int], _split_build(m))(m, n, k, cus)) > 0
 
 
 def prefers_split(m: int, k: int, weight: torch.Tensor) -> bool:
@@ -256,10 +261,10 @@ def split_product(weight: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     if x.dtype != torch.bfloat16 or not _rows_aligned(x, 8):
         raise ValueError("x must be bfloat16 with 16-byte aligned rows")
     cus = _compute_units(x.device)
-    chunks = int(_fn("gemm_split", "qvl_gemm_split_chunks", [_c_int, _c_int, _c_int, _c_int])(m, n, k, cus))
+    chunks = int(_fn("gemm_resident", "qvl_gemm_split_chunks", [_c_int, _c_int, _c_int, _c_int], _split_build(m))(m, n, k, cus))
     out = torch.empty((chunks, m, n), dtype=torch.float32, device=x.device)
-    fn = _fn("gemm_split", "qvl_gemm_split",
-             [_c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr])
+    fn = _fn("gemm_resident", "qvl_gemm_split",
+             [_c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr], _split_build(m))
     _check(fn(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(out), m, n, k, cus, _stream()),
            "linear (split)")
     return out
