@@ -37,7 +37,7 @@
 //                           key head takes 8 channels and the 8 channels they are rotated with
 //                           (half a head further), so the rotation happens here; queries are
 //                           written out, keys and values go straight into their page slots
-//   ranges of K             out[c] = the sums over range c of K (gemm_split below), for products whose result
+//   ranges of K             out[c] = the sums over range c of K (qvl_gemm_split below), for products whose result
 //                           joins the residual sum: the norm that follows adds the slabs in order
 #include "common.h"
 

@@ -602,6 +602,37 @@ def test_few_row_products_at_random_sizes():
         assert torch.allclose(total, before + want, atol=2e-2, rtol=2e-2), (m, n, k)
 
 
+@pytest.mark.parametrize("m", [1, 16, 17, 33, 64])
+@pytest.mark.parametrize("k", [8, 136, 1016, 2040, 2056, 3832])
+def test_few_row_products_read_nothing_beside_the_inner_size(m, k):
+    """The weight comes through LDS in units of 128 columns: with NaN behind the inner size in every row of both operands,
+    the last unit's columns beyond it must not be part of a sum, with the rows as they are, with their norm
+    formed inside, and over ranges of the inner size.  Each sum of k exact products is within k roundings of its terms."""
+    from qwen25vl_lite_amd.ops import kernels, skinny
+    torch.manual_seed(m + k)
+    n = 300
+    nan = float("nan")
+    wide_w, wide_x, wide_h = (torch.full((r, k + 128), nan, device="cuda") for r in (n, m, m))
+    wide_w, wide_x = wide_w.bfloat16(), wide_x.bfloat16()
+    w, x, h = wide_w[:, :k], wide_x[:, :k], wide_h[:, :k]
+    w.copy_(torch.randn(n, k) / math.sqrt(k))
+    x.copy_(torch.randn(m, k))
+    h.copy_(torch.randn(m, k))
+    g = (1 + 0.1 * torch.randn(k)).cuda()
+
+    def near(got, a, slack=0.0):
+        a, b = a.double().cpu(), w.double().cpu()
+        err = (got.double().cpu() - a @ b.T).abs()
+        assert bool((err <= (k * 2.0 ** -24 + slack) * (a.abs() @ b.abs().T) + 1e-30).all()), err.max()
+
+    near(skinny.resident_product(w, x=x), x)
+    near(skinny.split_product(w, x).sum(0), x)
+    if skinny.folds_norm(m, k):
+        # (a normed value may be rounded to bfloat16's other neighbour: the statistics are added up in another order)
+        near(skinny.resident_product(w, h=h, norm_weight=g, eps=1e-6), kernels.add_rmsnorm(h.contiguous(), None, g, 1e-6, torch.bfloat16),
+             2.0 ** -8)
+
+
 def test_no_cpu_path():
     from qwen25vl_lite_amd.ops import kernels
     from qwen25vl_lite_amd.ops.linear import linear
