@@ -162,8 +162,7 @@ __device__ __forceinline__ void meet() {
 template <typename TO, int PRO, int EPI, bool ONE_PASS, int MT>
 __global__ __launch_bounds__(64 * RW) void gemm_resident_kernel(ResidentArgs p) {
   constexpr int COLS = 16 * MT;   // rows of X the block carries
-  constexpr int RING = MT <= 2 ? 4 : 3;
-  static_assert(MT <= 4 && (MT <= 2 || RK <= 8), "X fits the registers");
+  constexpr int RING = 4;
   // MT = 1: two buffers, a tile's sums are read while the next tile's are written; else one, and a second barrier.
   // The norm weights borrow the sums' place before the first tile.
   constexpr int RED = MT == 1 ? 2 : 1;
@@ -715,10 +714,9 @@ static Cut cut_for(int M, int N, int K, int cus) {
   return best;
 }
 
-// Whether qvl_gemm_split takes these sizes, and how many slabs it then writes (0: it does not).  More than 32 rows are
-// taken by the build with RK = 8 only (a wave's columns of four column tiles fill its registers).
+// Whether qvl_gemm_split takes these sizes, and how many slabs it then writes (0: it does not).
 extern "C" int qvl_gemm_split_chunks(int M, int N, int K, int cus) {
-  if (M <= 0 || M > (RK <= 8 ? 64 : 32) || N <= 0 || K <= 0 || K % 8 || cus <= 0) return 0;
+  if (M <= 0 || M > 16 || N <= 0 || K <= 0 || K % 8 || cus <= 0) return 0;
   return cut_for(M, N, K, cus).chunks;
 }
 
@@ -727,7 +725,6 @@ extern "C" int qvl_gemm_split_chunks(int M, int N, int K, int cus) {
 extern "C" int qvl_gemm_split(const void* x, int ldx, const void* W, int ldw, void* out, int M, int N, int K, int cus,
                               hipStream_t stream) {
   if (M <= 0 || N <= 0) return QVL_OK;
-  if (M > 64) return QVL_ERR_LIMIT;
   if (K <= 0 || K % 8 || ldw % 8 || ldw < K || ldx % 8 || ldx < K || cus <= 0 || !x || !W || !out) return QVL_ERR_SHAPE;
   if (!fits_descriptors(M, N, K, ldw, ldx, 0, 0)) return QVL_ERR_LIMIT;
   if (qvl_gemm_split_chunks(M, N, K, cus) == 0) return QVL_ERR_LIMIT;
@@ -740,14 +737,7 @@ extern "C" int qvl_gemm_split(const void* x, int ldx, const void* W, int ldw, vo
   p.rows = c.rows; p.ntiles = c.ntiles; p.whole_tiles = c.ntiles; p.parts = 1; p.pairs = 8;
   p.stack_blocks = c.per_chunk; p.stack_x = p.stack_w = c.chunk_k; p.stack_o = (long long)M * N; p.all_k = K;
   const dim3 grid(c.chunks * c.per_chunk), block(64 * RW);
-#define QVL_SPLIT(MT) hipLaunchKernelGGL((gemm_resident_kernel<float, PRO_PLAIN, EPI_STORE, true, MT>), grid, block, 0, stream, p)
-  if (M <= 16) QVL_SPLIT(1);
-  else if (M <= 32) QVL_SPLIT(2);
-#if RK <= 8
-  else if (M <= 48) QVL_SPLIT(3);
-  else QVL_SPLIT(4);
-#endif
-#undef QVL_SPLIT
+  hipLaunchKernelGGL((gemm_resident_kernel<float, PRO_PLAIN, EPI_STORE, true, 1>), grid, block, 0, stream, p);
   return qvl_launch_status();
 }
 

@@ -1,0 +1,341 @@
+// Products with 17 to 64 rows: out = X[M, K] . W[N, K]^T, bfloat16 operands, float32 sums, stored as they are, as bfloat16, through
+// the gated activation of W's rows in groups of 8 gate and 8 up rows, or as one slab of sums for each range of K.
+//
+// What bounds it is reading W once.  A wave owns up to 32 rows of W and all rows of X (operands of
+// v_mfma_f32_32x32x16_bf16), eight waves are a block and a block has a compute unit to itself; the rows a wave takes at a time
+// are chosen so that all waves of the device have the same number of tiles (37,888 gated outputs on 2,048 waves: one
+// round of 10 channels).  Both operands come through LDS in steps of 64 values of K, all 160 KB of it being steps on
+// their way: W marked as read once, X out of the L2 for every tile again.  The steps of one tile follow those of the tile
+// before, so fetches stay in flight from the first tile to the last.  Where X is in the registers of waves that share
+// a tile of W (gemm_resident) it must fit them; here its rows and K are free, and eight waves read it at LDS's rate: 32 rows
+// of W a wave for 64 of X keep that below half of what LDS can do.
+//
+// Per call in a decode step: gate|up of the 7B decoder (37,888 x 3,584), 64 rows, 50.3 us = 5.4 TB/s (the library's product
+// 61.2 and the activation's kernel 5.0); of the 72B decoder (59,136 x 8,192), 19 rows, 145 = 6.7 TB/s (174 and 4.6); heads of
+// 152,064 x 3,584, 64 rows, 196 (212), x 8,192, 19 rows, 426 (465).  A plain read of as much reaches 7.3 TB/s.  Four waves a
+// block and two blocks a compute unit: 57 for 50; operands read and multiplied in turn, tile after tile of 16 rows: 65.
+#include "tile_product.h"
+
+#include <type_traits>
+
+#define ROWS_WAVES 8
+#define ROWS_LDS 163840
+
+enum { ROWS_BF16 = 0, ROWS_F32 = 1, ROWS_GATED = 2 };
+
+typedef float rows_f32x16 __attribute__((ext_vector_type(16)));
+
+struct RowsArgs {
+  const bf16_t* x;
+  long long ldx;
+  const bf16_t* w;
+  long long ldw;
+  void* out;
+  long long ldo;
+  int M, N, K;
+  int per;          // rows of W a wave takes at a time (ROWS_GATED: channels); even where results are bfloat16
+  int tiles;        // of all of W
+  int blocks;       // that share the tiles (of one range of K)
+  int rounds;       // tiles of a wave
+  int range_steps;  // steps of 64 values in a range of K; range i has the blocks i * blocks .. and the slab i of out
+  long long slab;
+  int gelu;
+  int pairs;        // bfloat16 results: two neighbouring ones may be stored at once
+};
+
+// Lane l of the wave puts its 16 bytes at M0 + 16 l of LDS; the lines are not kept in the caches.
+__device__ __forceinline__ void fetch16_once(const void* base, uint32_t lane_bytes, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(lane_bytes), "s"(base), "s"(lds_at)
+               : "memory", "m0");
+}
+template <int MOST, int LOADS>
+__device__ __forceinline__ void wait_steps(int ahead) {
+  if constexpr (MOST <= 0) {
+    tp_wait_fetches<0>();
+  } else {
+    if (ahead >= MOST) tp_wait_fetches<MOST * LOADS>();
+    else wait_steps<MOST - 1, LOADS>(ahead);
+  }
+}
+
+// MT column tiles of 32 rows of X; F fetches of 8 rows of W a step and wave: tiles of up to 8 F rows (4 F channels).
+template <int MT, int F, int OUT>
+__global__ __launch_bounds__(64 * ROWS_WAVES) void gemm_rows_kernel(RowsArgs p) {
+  constexpr int W_BYTES = ROWS_WAVES * F * 1024, STAGE = W_BYTES + MT * 4096, STAGES = ROWS_LDS / STAGE;
+  // MT = 1: X's four fetches of a step are made by two waves each (the same bytes to the same place), so that every wave
+  // waits for as many
+  constexpr int X_PLACES = 4 * MT;
+  constexpr int HALF = 2 * F;                 // ROWS_GATED: gates among a lane's 4 F sums
+  // float32 results: a lane holds one row of W (neighbouring lanes store neighbouring results); else neighbouring rows of W, so
+  // that gate and up value meet in a lane and two results of two bytes are stored at once
+  constexpr bool X_FIRST = OUT == ROWS_F32;
+  __shared__ __attribute__((aligned(16))) char lds[STAGES * STAGE];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, hi = lane >> 5, r = lane & 31;
+  const int range = blockIdx.x / p.blocks;
+  auto tile_of = [&](int round) { return (int)(blockIdx.x - range * p.blocks + round * p.blocks) * ROWS_WAVES + wave; };
+  const int k_first = range * p.range_steps * 64, k_values = min(p.K - k_first, p.range_steps * 64);
+  const int ksteps = (k_values + 63) / 64, steps = ksteps * p.rounds;
+  const int last_chunks = k_values % 64 ? (k_values % 64) / 8 : 8;     // of a last step, 8 values each
+  // row of W behind row i of a tile (-1: there is none).  ROWS_GATED: row i's sums are number 4 (i / 8) + i mod 4 of the lanes
+  // whose hi is (i / 4) mod 2, and the first half of a lane's sums are gates, the others their up values.
+  auto w_row = [&](int tile, int i) {
+    if (tile >= p.tiles) return -1;
+    if (OUT == ROWS_GATED) {
+      const int s = 4 * (i >> 3) + (i & 3), up = s >= HALF, j = ((i >> 2) & 1) * HALF + s - up * HALF, c = tile * p.per + j;
+      return (j < p.per && 2 * c < p.N) ? (c >> 3) * 16 + (c & 7) + 8 * up : -1;
+    }
+    const int n = tile * p.per + i;
+    return (i < p.per && n < p.N) ? n : -1;
+  };
+  // this lane's fetches: rows 8 j + lane / 8 of the wave's tile, the row's chunk (lane mod 8) ^ ((row / 2) mod 8), and of X
+  // row 8 x_place + lane / 8.  A row that does not exist is read from one that does; its sums are not stored.
+  uint32_t fw[F];
+  auto set_tile = [&](int tile) __attribute__((always_inline)) {
+    const int exists = max(w_row(tile, 0), 0);
+#pragma unroll
+    for (int j = 0; j < F; ++j) {
+      const int rho = 8 * j + (lane >> 3);
+      int n = w_row(tile, rho);
+      if (n < 0) n = exists;
+      fw[j] = (uint32_t)n * (uint32_t)p.ldw * 2 + 16 * ((lane & 7) ^ ((rho >> 1) & 7)) + (uint32_t)k_first * 2;
+    }
+  };
+  const int x_place = wave % X_PLACES, x_row = 8 * x_place + (lane >> 3);
+  const uint32_t fx = (uint32_t)(x_row < p.M ? x_row : 0) * (uint32_t)p.ldx * 2 + 16 * ((lane & 7) ^ ((x_row >> 1) & 7)) + (uint32_t)k_first * 2;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)&lds[0];
+  // Blocks begin a tile at different places of K and go round: all at the same place would ask the same few memory
+  // channels (rows lie a power of two of bytes apart in wide models; 59,136 x 8,192, 19 rows: 162 us for 200).
+  const int turn = (int)((blockIdx.x * 29u) % (unsigned)ksteps);
+  int asked = 0, ask_k = 0, ask_round = 0, ask_stage = 0, ask_at = turn;
+  auto ask = [&]() __attribute__((always_inline)) {          // the next step's fetches, if there is one
+    if (asked >= steps) return;
+    if (ask_k == 0) set_tile(tile_of(ask_round));
+    const uint32_t at = lds0 + ask_stage * STAGE, k = (uint32_t)ask_at * 128;
+    if (last_chunks == 8 || ask_at != ksteps - 1) {
+#pragma unroll
+      for (int j = 0; j < F; ++j) fetch16_once(p.w, fw[j] + k, at + (wave * F + j) * 1024);
+      tp_fetch16(p.x, fx + k, at + W_BYTES + x_place * 1024);
+    } else {
+      // chunks that lie beyond K are read from the step's first: they are not multiplied
+      auto back = [&](int row) { const int c = (lane & 7) ^ ((row >> 1) & 7); return c < last_chunks ? 0u : 16u * c; };
+#pragma unroll
+      for (int j = 0; j < F; ++j) fetch16_once(p.w, fw[j] + k - back(8 * j + (lane >> 3)), at + (wave * F + j) * 1024);
+      tp_fetch16(p.x, fx + k - back(x_row), at + W_BYTES + x_place * 1024);
+    }
+    ++asked;
+    ask_stage = ask_stage + 1 == STAGES ? 0 : ask_stage + 1;
+    if (++ask_at == ksteps) ask_at = 0;
+    if (++ask_k == ksteps) {
+      ask_k = 0;
+      ++ask_round;
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < STAGES - 1; ++i) ask();
+  const uint32_t sw = (r >> 1) & 7;
+  // rows of a tile beyond its 8 F are not fetched: their operand is another row's, their sums are not stored
+  const int wr = r < 8 * F ? r : r - 8 * F;
+  const uint32_t wsw = (wr >> 1) & 7;
+  rows_f32x16 acc[MT];
+  auto clear = [&] {
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[t][i] = 0.f;
+  };
+  auto finish = [&](int round) __attribute__((always_inline)) {
+    const int tile = tile_of(round);
+    if (tile >= p.tiles) return;
+    if constexpr (X_FIRST) {
+      const int n = tile * p.per + r;
+      float* out = reinterpret_cast<float*>(p.out) + range * p.slab + n;
+      if (r >= p.per || n >= p.N) return;
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int m = 32 * t + 8 * (i >> 2) + 4 * hi + (i & 3);
+          if (m < p.M) out[(size_t)m * p.ldo] = acc[t][i];
+        }
+    } else {
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        const int m = 32 * t + r;
+        if (m >= p.M) continue;
+        bf16_t* out = reinterpret_cast<bf16_t*>(p.out) + (size_t)m * p.ldo;
+        // results in pairs: numbers 2 i and 2 i + 1 of the lane's
+#pragma unroll
+        for (int i = 0; i < (OUT == ROWS_GATED ? HALF / 2 : HALF); ++i) {
+          float v0 = acc[t][2 * i], v1 = acc[t][2 * i + 1];
+          if (OUT == ROWS_GATED) {
+            v0 = gate_act(v0, p.gelu) * acc[t][HALF + 2 * i];
+            v1 = gate_act(v1, p.gelu) * acc[t][HALF + 2 * i + 1];
+          }
+          const int j = OUT == ROWS_GATED ? hi * HALF + 2 * i : 8 * (i >> 1) + 4 * hi + 2 * (i & 1);
+          const int n = tile * p.per + j, end = OUT == ROWS_GATED ? p.N / 2 : p.N;
+          if (j >= p.per || n >= end) continue;
+          if (p.pairs && n + 1 < end) {
+            *reinterpret_cast<uint32_t*>(out + n) = (uint32_t)f32_to_bf16(v0) | ((uint32_t)f32_to_bf16(v1) << 16);
+          } else {
+            out[n] = f32_to_bf16(v0);
+            if (n + 1 < end) out[n + 1] = f32_to_bf16(v1);
+          }
+        }
+      }
+    }
+  };
+  // The operands of a step are read from LDS while those of the step before are multiplied: all waves pass a barrier
+  // together, so that reading and multiplying would else take turns.
+  tp_bf16x8 w8[2][4], x8[2][MT][4];
+  int stage = 0, mul_k = turn, mul_left = ksteps, mul_round = 0;
+  auto read = [&](auto buf) __attribute__((always_inline)) {
+    constexpr int B = decltype(buf)::value;
+    const char* pw = lds + stage * STAGE + wave * F * 1024 + wr * 128;
+    const char* px = lds + stage * STAGE + W_BYTES + r * 128;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      w8[B][k] = *reinterpret_cast<const tp_bf16x8*>(pw + (((2 * k + hi) ^ wsw) << 4));
+#pragma unroll
+      for (int t = 0; t < MT; ++t) x8[B][t][k] = *reinterpret_cast<const tp_bf16x8*>(px + t * 4096 + (((2 * k + hi) ^ sw) << 4));
+    }
+    stage = stage + 1 == STAGES ? 0 : stage + 1;
+  };
+  auto multiply = [&](auto buf) __attribute__((always_inline)) {
+    constexpr int B = decltype(buf)::value;
+    if (last_chunks < 8 && mul_k == ksteps - 1) {      // chunks beyond K are no part of the sums
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (2 * k + hi >= last_chunks) {
+          w8[B][k] = tp_bf16x8{};
+#pragma unroll
+          for (int t = 0; t < MT; ++t) x8[B][t][k] = tp_bf16x8{};
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+        acc[t] = X_FIRST ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(x8[B][t][k], w8[B][k], acc[t], 0, 0, 0)
+                         : __builtin_amdgcn_mfma_f32_32x32x16_bf16(w8[B][k], x8[B][t][k], acc[t], 0, 0, 0);
+    if (++mul_k == ksteps) mul_k = 0;
+    if (--mul_left == 0) {
+      finish(mul_round++);
+      clear();
+      mul_left = ksteps;
+    }
+  };
+  auto step = [&](int s, auto here, auto before) __attribute__((always_inline)) {
+    if (s < steps) {
+      wait_steps<STAGES - 2, F + 1>(asked - 1 - s);      // all but the steps asked for behind this one have come
+      tp_wait_lds();
+      tp_barrier();                           // every wave's part of the step is there, and the step before has been read
+      ask();
+      read(here);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (s > 0) multiply(before);
+  };
+  clear();
+  constexpr std::integral_constant<int, 0> even{};
+  constexpr std::integral_constant<int, 1> odd{};
+  for (int s = 0; s <= steps; s += 2) {
+    step(s, even, odd);
+    if (s < steps) step(s + 1, odd, even);
+  }
+  tp_wait_fetches<0>();
+}
+
+static int rows_check(const RowsArgs& p, const void* x, const void* w, const void* out, int cus) {
+  if (p.M > 64) return QVL_ERR_LIMIT;
+  if (p.K <= 0 || p.K % 8 || p.ldx < p.K || p.ldw < p.K || p.ldx % 8 || p.ldw % 8 || !x || !w || !out || cus <= 0 ||
+      ((uintptr_t)x % 16) || ((uintptr_t)w % 16))
+    return QVL_ERR_SHAPE;
+  // offsets from the first row are 32-bit
+  if ((unsigned long long)((p.N - 1) * p.ldw + p.K) * 2 >= 0xffffff00ull || (unsigned long long)((p.M - 1) * p.ldx + p.K) * 2 >= 0xffffff00ull)
+    return QVL_ERR_LIMIT;
+  return QVL_OK;
+}
+static int rows_launch(RowsArgs& p, int ranges, int mode, hipStream_t stream) {
+  const int rows = mode == ROWS_GATED ? 2 * p.per : p.per, fetches = rows <= 16 ? 2 : (rows + 7) / 8;
+  const dim3 grid((unsigned)(p.blocks * ranges)), block(64 * ROWS_WAVES);
+#define GO(MT, F, OUT) hipLaunchKernelGGL((gemm_rows_kernel<MT, F, OUT>), grid, block, 0, stream, p)
+#define MODE(MT, F)                               \
+  do {                                            \
+    if (mode == ROWS_BF16) GO(MT, F, ROWS_BF16);  \
+    else if (mode == ROWS_F32) GO(MT, F, ROWS_F32); \
+    else GO(MT, F, ROWS_GATED);                   \
+  } while (0)
+#define FETCHES(MT)                     \
+  do {                                  \
+    if (fetches == 2) MODE(MT, 2);      \
+    else if (fetches == 3) MODE(MT, 3); \
+    else MODE(MT, 4);                   \
+  } while (0)
+  if (p.M <= 32) FETCHES(1);
+  else FETCHES(2);
+#undef FETCHES
+#undef MODE
+#undef GO
+  return qvl_launch_status();
+}
+
+// x: bfloat16 [M, K], rows ldx apart, M at most 64; w: bfloat16 [N, K], rows ldw apart; both on 16-byte boundaries, K a multiple
+// of 8.  mode 0: out bfloat16 [M, N]; 1: float32; 2: W's rows in groups of 8 gate + 8 up, out bfloat16 [M, N / 2] = act(gate) up.
+extern "C" int qvl_gemm_rows(const void* x, long long ldx, const void* w, long long ldw, void* out, long long ldo, int M, int N,
+                             int K, int mode, int gelu, int cus, hipStream_t stream) {
+  if (M <= 0 || N <= 0) return QVL_OK;
+  if (mode < 0 || mode > 2 || (mode == 2 && N % 16) || ldo < (mode == 2 ? N / 2 : N)) return QVL_ERR_SHAPE;
+  RowsArgs p;
+  p.x = (const bf16_t*)x; p.ldx = ldx; p.w = (const bf16_t*)w; p.ldw = ldw; p.out = out; p.ldo = ldo;
+  p.M = M; p.N = N; p.K = K; p.gelu = gelu; p.slab = 0; p.range_steps = (K + 63) / 64;
+  const int bad = rows_check(p, x, w, out, cus);
+  if (bad) return bad;
+  // the fewest rounds over a block a compute unit, then the fewest rows a wave that these rounds need
+  const long long items = mode == 2 ? N / 2 : N, most = mode == 2 ? 16 : 32, waves = (long long)cus * ROWS_WAVES;
+  const long long rounds = (items + most * waves - 1) / (most * waves);
+  p.per = (int)((items + rounds * waves - 1) / (rounds * waves));
+  if (mode != 1) p.per = (p.per + 1) / 2 * 2;
+  p.pairs = ldo % 2 == 0 && (uintptr_t)out % 4 == 0;
+  p.tiles = (int)((items + p.per - 1) / p.per);
+  p.blocks = min(cus, (p.tiles + ROWS_WAVES - 1) / ROWS_WAVES);
+  p.rounds = (p.tiles + p.blocks * ROWS_WAVES - 1) / (p.blocks * ROWS_WAVES);
+  return rows_launch(p, 1, mode, stream);
+}
+
+// Products whose result is added to something anyway, cut into ranges of K so that every compute unit has a block: out float32
+// [ranges, M, N], the sums over each range.  16 rows of W a wave: with 32 the operands of LDS last longer but there are twice
+// the slabs to write and add (3,584 x 18,944, 64 rows, with the norm that adds the slabs: 33 us, with 24 rows 35, with 8
+// 53).  A range has at least four steps.
+#define CUT_ROWS 16
+struct RowsCut {
+  int blocks, range_steps, ranges;
+};
+static RowsCut rows_cut(int N, int K, int cus) {
+  RowsCut c;
+  c.blocks = ((N + CUT_ROWS - 1) / CUT_ROWS + ROWS_WAVES - 1) / ROWS_WAVES;
+  const int steps = (K + 63) / 64, want = max(1, cus / c.blocks);
+  c.range_steps = max(4, (steps + want - 1) / want);
+  c.ranges = (steps + c.range_steps - 1) / c.range_steps;
+  return c;
+}
+// How many slabs qvl_gemm_rows_cut writes (0: it does not take these sizes).
+extern "C" int qvl_gemm_rows_ranges(int M, int N, int K, int cus) {
+  if (M <= 0 || M > 64 || N <= 0 || K <= 0 || K % 8 || cus <= 0) return 0;
+  return rows_cut(N, K, cus).ranges;
+}
+extern "C" int qvl_gemm_rows_cut(const void* x, long long ldx, const void* w, long long ldw, void* out, int M, int N, int K, int cus,
+                                 hipStream_t stream) {
+  if (M <= 0 || N <= 0) return QVL_OK;
+  RowsArgs p;
+  p.x = (const bf16_t*)x; p.ldx = ldx; p.w = (const bf16_t*)w; p.ldw = ldw; p.out = out; p.ldo = N;
+  p.M = M; p.N = N; p.K = K; p.gelu = 0; p.pairs = 0; p.slab = (long long)M * N;
+  const int bad = rows_check(p, x, w, out, cus);
+  if (bad) return bad;
+  const RowsCut c = rows_cut(N, K, cus);
+  p.per = CUT_ROWS;
+  p.tiles = (N + CUT_ROWS - 1) / CUT_ROWS;
+  p.blocks = c.blocks;
+  p.range_steps = c.range_steps;
+  p.rounds = 1;
+  return rows_launch(p, c.ranges, ROWS_F32, stream);
+}

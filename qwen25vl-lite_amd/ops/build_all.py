@@ -18,6 +18,7 @@ LIBRARIES = [
     ("gemm_resident", {}),
     ("gemm_resident", {"RK": 8}),
     ("gemm_tile", {}),
+    ("gemm_rows", {}),
     ("peaks", {}),
     ("gated", {}),
     ("moe", {}),

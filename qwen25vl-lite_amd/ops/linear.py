@@ -3,7 +3,7 @@
 float32 runs through the hand-written FMA kernel (true 32-bit, fixed summation order).
 bfloat16 with up to 64 rows (a decode step) runs through the hand-written matrix-core kernel, which
 also folds the norm before a product, the residual add after it and the SwiGLU activation into
-itself; with more rows the tiled kernel runs (:mod:`~qwen25vl_lite_amd.ops.tile`), with the activation on its sums, or
+itself, or through one that needs not keep the rows (:mod:`~qwen25vl_lite_amd.ops.rows`); with more rows the tiled kernel runs (:mod:`~qwen25vl_lite_amd.ops.tile`), with the activation on its sums, or
 cut along the inner size where the result joins a sum anyway.  The vendor library's product, which the
 reference's engine uses for its projections (reference src/qwen25vl_lite/text.py:61-66, 80-90), is left
 for what neither takes or does as fast.
@@ -15,7 +15,7 @@ from typing import Optional, Union
 
 import torch
 
-from . import kernels, skinny, tile
+from . import kernels, rows, skinny, tile
 
 __all__ = ["NormedRows", "linear", "linear_into", "linear_stack", "linear_relu2", "gate_up_swiglu", "tune_library_products"]
 
@@ -33,6 +33,9 @@ class NormedRows:
 
 
 def _many_rows(x: torch.Tensor, weight: torch.Tensor, bias, out_dtype, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    if rows.prefers_rows(x, weight) and (out is None or (out.dtype == torch.bfloat16 and out.stride(1) == 1 and out.stride(0) >= out.shape[1])):
+        y = rows.rows_product(x, weight, out_dtype or torch.bfloat16, out)
+        return y if bias is None else y + bias.to(y.dtype)
     if out is not None:
         if out.dtype == torch.bfloat16 and out.dim() == 2 and out.stride(1) == 1 and out.data_ptr() % 16 == 0 and tile.prefers_tile(x, weight):
             return tile.tile_product(x, weight, out=out)
@@ -57,7 +60,8 @@ def linear(x: Union[torch.Tensor, NormedRows], weight: torch.Tensor, bias: Optio
     if not weight.is_cuda:
         raise kernels.KernelError("linear has no CPU path: its tensors must be on the GPU")
     if weight.dtype == torch.bfloat16:
-        few = m <= skinny.ONE_BLOCK_ROWS     # beyond, the library streams a plain product faster
+        # with more rows teams of blocks lose to the library; with many outputs and more than a column tile of rows to `rows`
+        few = m <= skinny.ONE_BLOCK_ROWS and (bias is not None or not rows.wide(m, weight))
         if lazy and few and skinny.takes_resident(m, k, weight, norm=True):
             return skinny.resident_product(weight, h=x.h, norm_weight=x.weight, eps=x.eps, bias=bias,
                                            out_dtype=out_dtype or torch.bfloat16)
@@ -158,7 +162,7 @@ def gate_up_swiglu(x: Union[torch.Tensor, NormedRows], weight: torch.Tensor, gro
     and grouped rows the activation is applied inside the product's kernel."""
     m, k = x.shape
     if (grouped and weight.dtype == torch.bfloat16 and weight.is_cuda and weight.shape[0] % 16 == 0
-            and m <= skinny.ONE_BLOCK_ROWS):
+            and m <= skinny.ONE_BLOCK_ROWS and not rows.wide(m, weight)):
         lazy = isinstance(x, NormedRows)
         if lazy and skinny.takes_resident(m, k, weight, norm=True):
             return skinny.resident_product(weight, h=x.h, norm_weight=x.weight, eps=x.eps, epilogue=skinny.GATED[act])
@@ -166,6 +170,8 @@ def gate_up_swiglu(x: Union[torch.Tensor, NormedRows], weight: torch.Tensor, gro
             return skinny.resident_product(weight, x=x, epilogue=skinny.GATED[act])
     if isinstance(x, NormedRows):
         x = x.materialize()
+    if grouped and weight.shape[0] % 16 == 0 and rows.prefers_rows(x, weight):
+        return rows.rows_swiglu(x, weight, act)
     if grouped and weight.shape[0] % 16 == 0 and x.is_cuda and tile.prefers_tile(x, weight):
         return tile.tile_swiglu(x, weight, act)
     return kernels.swiglu(linear(x, weight), grouped=grouped, act=act)

@@ -1,0 +1,75 @@
+"""Dispatch of bfloat16 products with up to 64 rows and many outputs to ``csrc/gemm_rows.hip``, whose blocks need not keep the
+rows."""
+
+from __future__ import annotations
+
+import ctypes
+from typing import Optional
+
+import torch
+
+from . import skinny
+from .kernels import _check, _fn, _need, _ptr, _stream, compute_units
+
+__all__ = ["takes_rows", "prefers_rows", "rows_product", "rows_swiglu"]
+
+_c_int, _c_ptr, _c_ll = ctypes.c_int, ctypes.c_void_p, ctypes.c_longlong
+_REACH = 0xffffff00
+MOST_ROWS = 64
+
+
+def _aligned(t: torch.Tensor) -> bool:
+    return t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.stride(0) >= t.shape[1] and t.data_ptr() % 16 == 0
+
+
+def takes_rows(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether the kernel takes ``x [M, K] @ weight[N, K].T``: up to 64 bfloat16 rows on 16-byte boundaries, an inner size in
+    steps of 8, operands within 32-bit byte offsets."""
+    return (x.is_cuda and weight.is_cuda and x.dtype == weight.dtype == torch.bfloat16 and x.dim() == 2 and weight.dim() == 2
+            and x.shape[1] == weight.shape[1] and 0 < x.shape[0] <= MOST_ROWS and x.shape[1] > 0 and x.shape[1] % 8 == 0
+            and _aligned(x) and _aligned(weight) and ((weight.shape[0] - 1) * weight.stride(0) + x.shape[1]) * 2 < _REACH
+            and ((x.shape[0] - 1) * x.stride(0) + x.shape[1]) * 2 < _REACH)
+
+
+def wide(m: int, weight: torch.Tensor) -> bool:
+    """Whether a weight has the outputs that make the kernel the fastest way to ``m`` rows: at least 8 for each of a device's
+    waves (eight a compute unit; 10,240 x 8,192 at 19 rows 60 us, the library, which cuts the inner size, 41), and more
+    rows than the resident kernel carries in one column tile, or an inner size too long for it to keep them.  Against
+    the resident kernel at 32 rows: 22,016 x 2,048 gated 22 us for 27, with the norm in front 27 for 32; 37,888 x 3,584 45
+    for 54, 50 for 65; 152,064 x 3,584 186 for 200; with 8 rows, 3B and 7B sizes, the two lie within 3 us and the resident
+    kernel forms the norm by itself.  Against the library at 64 rows: 37,888 x 3,584 gated 49 us for 69 with the
+    activation's kernel, 59,136 x 8,192 151 for 199; heads of 152,064 x 3,584 194 for 219, x 8,192 438 for 500."""
+    n, k = weight.shape
+    return (m <= MOST_ROWS and n >= 64 * compute_units(weight.device)
+            and (m > skinny.ONE_TILE_ROWS or not skinny.takes_resident(m, k, weight)))
+
+
+def prefers_rows(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    return takes_rows(x, weight) and wide(x.shape[0], weight)
+
+
+def _launch(x, weight, out, mode, gelu=0):
+    fn = _fn("gemm_rows", "qvl_gemm_rows", [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ll] + [_c_int] * 6 + [_c_ptr])
+    _check(fn(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(out), out.stride(0), x.shape[0], weight.shape[0],
+              x.shape[1], mode, gelu, compute_units(x.device), _stream()), "linear (few rows)")
+    return out
+
+
+def rows_product(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype = torch.bfloat16,
+                 out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``x @ weight.T`` in ``out_dtype``."""
+    _need(takes_rows(x, weight), "the kernel does not take this product")
+    m, n = x.shape[0], weight.shape[0]
+    if out is None:
+        out = torch.empty((m, n), dtype=out_dtype, device=x.device)
+    _need(out.dtype == out_dtype and out_dtype in (torch.float32, torch.bfloat16) and tuple(out.shape) == (m, n)
+          and out.stride(1) == 1 and out.stride(0) >= n, "out must be [M, N] of the output's dtype")
+    return _launch(x, weight, out, int(out_dtype == torch.float32))
+
+
+def rows_swiglu(x: torch.Tensor, weight: torch.Tensor, act: str = "silu") -> torch.Tensor:
+    """``act(gate) * up`` for a weight whose rows come in groups of 8 gate and 8 up rows: bfloat16 ``[M, N / 2]``."""
+    _need(takes_rows(x, weight) and weight.shape[0] % 16 == 0, "the kernel does not take this product")
+    _need(act in ("silu", "gelu_tanh"), "the activation is silu or gelu_tanh")
+    out = torch.empty((x.shape[0], weight.shape[0] // 2), dtype=torch.bfloat16, device=x.device)
+    return _launch(x, weight, out, 2, int(act == "gelu_tanh"))

@@ -1,9 +1,10 @@
 """Dispatch of bfloat16 products with few rows to the hand-written kernels.
 
-Up to 64 rows: the resident kernel (``csrc/gemm_resident.hip``), which can also fold the RMSNorm
+Up to 64 rows, where their operands are kept by a block: the resident kernel (``csrc/gemm_resident.hip``), which can also fold the RMSNorm
 before the product, the residual add after it, the SwiGLU activation, or the rotation and cache
 write into itself.  One block carries up to 32 rows; more rows (or 17 to 32 with a long inner
-size) are spread over teams of blocks that walk the same weight tiles on one XCD.
+size) are spread over teams of blocks that walk the same weight tiles on one XCD.  Products of more than a few rows that are cut along their inner size run in
+``csrc/gemm_rows.hip``.
 """
 
 from __future__ import annotations
@@ -42,12 +43,6 @@ def _build_for(k: int):
     """The build of the resident kernel for an inner size: with 512 columns a wave, half of a
     block's 8 waves have no columns of an inner size of 2,048 and the other half carry all loads."""
     return {"RK": 8} if k <= NARROW_K else None
-
-
-def _split_build(m: int):
-    """The build that cuts a product of ``m`` rows into ranges of its inner size: up to 32 rows a wave keeps 512 columns of
-    them in registers, up to 64 rows 256."""
-    return None if m <= ONE_BLOCK_ROWS else {"RK": 8}
 
 
 def resident_norm_k() -> int:
@@ -219,20 +214,26 @@ def qkv_rope_product(weight: torch.Tensor, cs: torch.Tensor, *, x: Optional[torc
     return q_out
 
 
-SPLIT_ROWS = 64   # the most rows the split kernel is built for
+SPLIT_ROWS = 64   # the most rows that are cut along the inner size
+SPLIT_K = 2048 * 256   # the longest inner size
+# Up to here a block keeps its range of the rows and walks several tiles (csrc/gemm_resident.hip: few ranges; 2,048 x 11,008, one
+# row, with the norm that adds the slabs: a decode step of the 3B decoder 4.24 ms, cut by csrc/gemm_rows.hip 4.31), with more
+# rows csrc/gemm_rows.hip cuts (3,584 x 18,944: 8 rows 25.4 us for 26.9, 16 rows 25.4 for 28.3, 64 rows 28.3 for 36.7)
+KEPT_SPLIT_ROWS = 8
+
+
+def _ranges(m: int, n: int, k: int, cus: int) -> int:
+    if m <= KEPT_SPLIT_ROWS:
+        return int(_fn("gemm_resident", "qvl_gemm_split_chunks", [_c_int] * 4)(m, n, k, cus))
+    return int(_fn("gemm_rows", "qvl_gemm_rows_ranges", [_c_int] * 4)(m, n, k, cus))
 
 
 def takes_split(m: int, k: int, weight: torch.Tensor) -> bool:
-    """Whether the split kernel (in ``csrc/gemm_resident.hip``) takes a product of ``m`` rows with this
-    weight: up to 64 bfloat16 rows, whose partial sums over chunks of the inner size come back as
-    slabs."""
-    if not (1 <= m <= SPLIT_ROWS and k % 8 == 0 and weight.dtype == torch.bfloat16 and _rows_aligned(weight, 8)):
+    """Whether a product of ``m`` rows with this weight is taken in ranges of the inner size: up to
+    64 bfloat16 rows, whose partial sums come back as slabs."""
+    if not (1 <= m <= SPLIT_ROWS and k % 8 == 0 and k <= SPLIT_K and weight.dtype == torch.bfloat16 and _rows_aligned(weight, 8)):
         return False
-    n = weight.shape[0]
-    if ((n - 1) * weight.stride(0) + k) * 2 >= _MAX_WEIGHT_BYTES:
-        return False
-    cus = _compute_units(weight.device)
-    return int(_fn("gemm_resident", "qvl_gemm_split_chunks", [_c_int, _c_int, _c_int, _c_int], _split_build(m))(m, n, k, cus)) > 0
+    return ((weight.shape[0] - 1) * weight.stride(0) + k) * 2 < _MAX_WEIGHT_BYTES
 
 
 def prefers_split(m: int, k: int, weight: torch.Tensor) -> bool:
@@ -242,8 +243,8 @@ def prefers_split(m: int, k: int, weight: torch.Tensor) -> bool:
     pass over the weight (the down projection at 8 rows: 26.9 us against 37.3, which pays for the
     norm kernel that then adds the slabs, 5.7 us, where the resident kernel adds in place and the
     next product forms the norm itself); with more rows always (the output projection at 32 rows:
-    9.9 us and a norm kernel of 6 against 14.3 in place and 8 more for the norm inside the gate | up
-    product; at 64 rows 14.4 us against the library's 13.9 to 17.6, the down projection 36.2
+    10.3 us and a norm kernel of 6 against 14.2 in place and 11 more for the norm inside the gate | up
+    product; at 64 rows 12.3 us against the library's 13.9 to 17.6, the down projection 28.3
     against 46.6)."""
     if not takes_split(m, k, weight):
         return False
@@ -251,7 +252,7 @@ def prefers_split(m: int, k: int, weight: torch.Tensor) -> bool:
 
 
 def split_product(weight: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
-    """Partial sums of ``x @ weight.T`` over chunks of the inner size: float32 ``[chunks, M, N]``,
+    """Partial sums of ``x @ weight.T`` over ranges of the inner size: float32 ``[ranges, M, N]``,
     whose sum over the first axis (taken in order by whoever reads them: the norm that follows) is
     the product.  ``x`` is bfloat16 ``[M, K]``."""
     m = x.shape[0]
@@ -261,10 +262,12 @@ def split_product(weight: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
     if x.dtype != torch.bfloat16 or not _rows_aligned(x, 8):
         raise ValueError("x must be bfloat16 with 16-byte aligned rows")
     cus = _compute_units(x.device)
-    chunks = int(_fn("gemm_resident", "qvl_gemm_split_chunks", [_c_int, _c_int, _c_int, _c_int], _split_build(m))(m, n, k, cus))
-    out = torch.empty((chunks, m, n), dtype=torch.float32, device=x.device)
-    fn = _fn("gemm_resident", "qvl_gemm_split",
-             [_c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr], _split_build(m))
-    _check(fn(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(out), m, n, k, cus, _stream()),
-           "linear (split)")
+    out = torch.empty((_ranges(m, n, k, cus), m, n), dtype=torch.float32, device=x.device)
+    if m <= KEPT_SPLIT_ROWS:
+        fn = _fn("gemm_resident", "qvl_gemm_split",
+                 [_c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr])
+    else:
+        fn = _fn("gemm_rows", "qvl_gemm_rows_cut",
+                 [_c_ptr, ctypes.c_longlong, _c_ptr, ctypes.c_longlong, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr])
+    _check(fn(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(out), m, n, k, cus, _stream()), "linear (split)")
     return out

@@ -18,10 +18,12 @@ from ..ops.linear import NormedRows, linear, linear_into
 from .base import (CacheNeed, LayerSlot, Mixer, ParamSpec, PartSpec, StateNeed, StepContext, build_part,
                    register_part)
 
-# 33 to 48 rows: the projection cut along its inner size (slabs) and the rotation's kernel behind it beat the
-# fused kernel on teams of blocks (7B sizes: a step of 33 rows 4.14 ms against 4.24, of 48 rows 4.34 against 4.39,
-# of 64 rows 4.68 against 4.67)
-SPLIT_ROWS = (33, 48)
+# 17 to 48 rows: where the fused kernel does not run, the projection is cut along its inner size (slabs) and the rotation's
+# kernel adds them (10,240 x 8,192, 19 rows: 32 us, the library's product uncut 41).  From 33 rows on that also beats the fused
+# kernel on teams of blocks (7B sizes: a step of 33 rows 4.14 ms against 4.24, of 48 rows 4.34 against 4.39, of 64 rows
+# 4.68 against 4.67)
+SPLIT_ROWS = (17, 48)
+FUSED_ROWS = 32
 
 __all__ = ["PagedAttention"]
 
@@ -341,7 +343,7 @@ class PagedAttention(Mixer):
         kernel (the float32 sums never leave it)."""
         lazy = isinstance(x, NormedRows)
         m, k = x.shape
-        if not lazy and SPLIT_ROWS[0] <= m <= SPLIT_ROWS[1]:
+        if not lazy and FUSED_ROWS < m <= SPLIT_ROWS[1]:
             return None
         if self.dtype != torch.bfloat16 or not skinny.takes_qkv_rope(
                 m, k, self.w_in, self.hd, inv_freq.shape[0], slot.k_cache.dtype if write else None, norm=lazy):

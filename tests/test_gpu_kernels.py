@@ -633,6 +633,39 @@ def test_few_row_products_read_nothing_beside_the_inner_size(m, k):
              2.0 ** -8)
 
 
+@pytest.mark.parametrize("m", [1, 19, 32, 33, 64])
+@pytest.mark.parametrize("n, k", [(16, 8), (16400, 136), (37888, 72), (59136, 64), (81920, 200), (152064, 136), (36912, 2056)])
+def test_rows_against_many_outputs(m, n, k):
+    """The kernel for up to 64 rows and many outputs: two, three and four fetches of the weight's rows a wave, one round of tiles
+    and several, inner sizes that end inside a step, NaN behind the inner size in every row, an odd row stride of the
+    result; each sum of k exact products is within k roundings of its terms, a stored bfloat16 half a unit in its last place
+    further; gated values against the same activation of the float32 products."""
+    from qwen25vl_lite_amd.ops import rows
+    torch.manual_seed(m + n)
+    wide_w = torch.full((n, k + 64), float("nan"), device="cuda").bfloat16()
+    wide_x = torch.full((m, k + 64), float("nan"), device="cuda").bfloat16()
+    w, x = wide_w[:, :k], wide_x[:, :k]
+    w.copy_(torch.randn(n, k, device="cuda") / math.sqrt(k))
+    x.copy_(torch.randn(m, k, device="cuda"))
+    want = x.double() @ w.double().T
+    bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) + 1e-30
+    sums = rows.rows_product(x, w, torch.float32)
+    assert bool(((sums.double() - want).abs() <= bound).all())
+    for wider in (0, 1, 2):
+        out = torch.full((m, n + wider), 7.0, device="cuda").bfloat16()
+        rows.rows_product(x, w, out=out[:, :n])
+        assert bool(((out[:, :n].double() - want).abs() <= bound + 2.0 ** -8 * want.abs()).all())
+        assert bool((out[:, n:] == 7.0).all())
+    pairs = want.view(m, n // 16, 2, 8)
+    for act, fn in (("silu", torch.nn.functional.silu), ("gelu_tanh", lambda t: torch.nn.functional.gelu(t, approximate="tanh"))):
+        got = rows.rows_swiglu(x, w, act).double()
+        ref = (fn(pairs[:, :, 0]) * pairs[:, :, 1]).reshape(m, n // 2)
+        # both factors' sums within their bounds (an activation's slope is below 1.13), float32 rounding of the activation, one to bfloat16
+        b = bound.view(m, n // 16, 2, 8)
+        slack = (1.13 * b[:, :, 0] * (pairs[:, :, 1].abs() + b[:, :, 1]) + fn(pairs[:, :, 0]).abs() * b[:, :, 1]).reshape(m, n // 2)
+        assert bool(((got - ref).abs() <= slack + (2.0 ** -8 + 1e-5) * ref.abs() + 1e-5 * pairs[:, :, 1].abs().reshape(m, n // 2)).all())
+
+
 def test_no_cpu_path():
     from qwen25vl_lite_amd.ops import kernels
     from qwen25vl_lite_amd.ops.linear import linear
