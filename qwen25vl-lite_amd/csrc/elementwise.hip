@@ -286,10 +286,14 @@ __global__ void rope_kv_write_kernel(const TI* __restrict__ x, int x_stride, con
 }
 
 // The same for float32 sums, bfloat16 outputs and the table of cosines and sines in hand, with
-// all widths multiples of 4 (the prompt portions of a bfloat16 run): a block per token, a thread
-// per 4 neighbouring channels, 16-byte loads and 8-byte stores.
+// all widths multiples of 4: a thread per 4 neighbouring channels (and the 4 they are rotated with), 16-byte loads and 8-byte stores.
 // x may come as nslabs slabs, slab_stride elements apart (partial sums of a product cut along its inner
-// size): they are added in slab order, then the bias.
+// size): they are added in slab order, then the bias; AT_ONCE slabs are asked for before the first is added.
+// The y blocks of a token share its channels: a block each with many tokens, which fill the device and hide the loads of
+// one slab behind another's; with few, as many as make one item a thread and eight slabs at once, since one block would then
+// work through slab after slab of every item alone while the device idles (64 tokens, 28 + 2 x 4 heads of 128, 7
+// slabs: 14.0 us by one block a token and one slab at a time, 6.3; 2,048 tokens, 1 slab: 19.9 and 21.8).
+template <int AT_ONCE>
 __global__ __launch_bounds__(256) void rope_kv_write_wide_kernel(
     const float* __restrict__ x, int x_stride, const float* __restrict__ bias, const float2* __restrict__ cs,
     const int* __restrict__ slot, bf16_t* __restrict__ q_out, bf16_t* __restrict__ kc, bf16_t* __restrict__ vc, int nq,
@@ -298,40 +302,54 @@ __global__ __launch_bounds__(256) void rope_kv_write_wide_kernel(
   const float* src = x + (size_t)n * x_stride;
   auto sums = [&](int at) {
     float4 v = *reinterpret_cast<const float4*>(src + at);
-    for (int c = 1; c < nslabs; ++c) {
-      const float4 e = *reinterpret_cast<const float4*>(src + (size_t)c * slab_stride + at);
-      v.x += e.x; v.y += e.y; v.z += e.z; v.w += e.w;
+    for (int c0 = 1; c0 < nslabs; c0 += AT_ONCE) {
+      float4 e[AT_ONCE];
+#pragma unroll
+      for (int c = 0; c < AT_ONCE; ++c)
+        if (c0 + c < nslabs) e[c] = *reinterpret_cast<const float4*>(src + (size_t)(c0 + c) * slab_stride + at);
+#pragma unroll
+      for (int c = 0; c < AT_ONCE; ++c)
+        if (c0 + c < nslabs) { v.x += e[c].x; v.y += e[c].y; v.z += e[c].z; v.w += e[c].w; }
     }
-    return v;
-  };
-  const int s = nkv ? slot[n] : -1;
-  const size_t page = s >= 0 ? (size_t)(s / ps) : 0, off = s >= 0 ? (size_t)(s % ps) : 0;
-  auto add_bias = [&](float4 v, int at) {
     if (bias) {
       const float4 b = *reinterpret_cast<const float4*>(bias + at);
       v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w;
     }
     return v;
   };
+  const int s = nkv ? slot[n] : -1;
+  const size_t page = s >= 0 ? (size_t)(s / ps) : 0, off = s >= 0 ? (size_t)(s % ps) : 0;
   auto pack4 = [](float4 v) {
     uint2 o;
     o.x = (uint32_t)f32_to_bf16(v.x) | ((uint32_t)f32_to_bf16(v.y) << 16);
     o.y = (uint32_t)f32_to_bf16(v.z) | ((uint32_t)f32_to_bf16(v.w) << 16);
     return o;
   };
-  // rotated heads: items (head, 4 frequencies)
-  const int per_head = rot_half / 4, rotated = (nq + nkv) * per_head;
-  for (int it = threadIdx.x; it < rotated; it += blockDim.x) {
-    const int hh = it / per_head, f = (it - hh * per_head) * 4;
-    bf16_t* dst;
-    if (hh < nq) {
-      dst = q_out + ((size_t)n * nq + hh) * hd;
-    } else {
-      if (s < 0) continue;
-      dst = kc + ((page * nkv + (hh - nq)) * ps + off) * hd;
+  // items: (rotated head, 4 frequencies); (rotated head, 4 channels past the rotation); (value head, 4 channels)
+  const int per_head = rot_half / 4, rotated = (nq + nkv) * per_head, tail = (hd - 2 * rot_half) / 4;
+  const int rest = rotated + (nq + nkv) * tail, items = rest + (s >= 0 ? nkv * (hd / 4) : 0);
+  for (int it = blockIdx.y * 256 + threadIdx.x; it < items; it += gridDim.y * 256) {
+    if (it >= rest) {  // values: [page][kv head][channel][slot]
+      const int i = it - rest, kvh = i / (hd / 4), d = (i - kvh * (hd / 4)) * 4;
+      const float4 v = sums((nq + nkv + kvh) * hd + d);
+      bf16_t* dst = vc + ((page * nkv + kvh) * hd + d) * ps + off;
+      dst[0] = f32_to_bf16(v.x);
+      dst[(size_t)ps] = f32_to_bf16(v.y);
+      dst[(size_t)2 * ps] = f32_to_bf16(v.z);
+      dst[(size_t)3 * ps] = f32_to_bf16(v.w);
+      continue;
     }
-    const float4 x1 = add_bias(sums(hh * hd + f), hh * hd + f);
-    const float4 x2 = add_bias(sums(hh * hd + f + rot_half), hh * hd + f + rot_half);
+    const bool turns = it < rotated;
+    const int i = turns ? it : it - rotated, each = turns ? per_head : tail, hh = i / each;
+    const int f = (i - hh * each) * 4 + (turns ? 0 : 2 * rot_half);
+    if (hh >= nq && s < 0) continue;
+    bf16_t* dst = hh < nq ? q_out + ((size_t)n * nq + hh) * hd : kc + ((page * nkv + (hh - nq)) * ps + off) * hd;
+    const float4 x1 = sums(hh * hd + f);
+    if (!turns) {
+      *reinterpret_cast<uint2*>(dst + f) = pack4(x1);
+      continue;
+    }
+    const float4 x2 = sums(hh * hd + f + rot_half);
     const float4 c01 = *reinterpret_cast<const float4*>(cs + (size_t)n * rot_half + f);      // (c0, s0, c1, s1)
     const float4 c23 = *reinterpret_cast<const float4*>(cs + (size_t)n * rot_half + f + 2);
     const float4 lo = {x1.x * c01.x - x2.x * c01.y, x1.y * c01.z - x2.y * c01.w, x1.z * c23.x - x2.z * c23.y,
@@ -340,31 +358,6 @@ __global__ __launch_bounds__(256) void rope_kv_write_wide_kernel(
                        x2.w * c23.z + x1.w * c23.w};
     *reinterpret_cast<uint2*>(dst + f) = pack4(lo);
     *reinterpret_cast<uint2*>(dst + f + rot_half) = pack4(hi);
-  }
-  // channels past the rotation, unrotated
-  const int tail = (hd - 2 * rot_half) / 4;
-  for (int it = threadIdx.x; it < (nq + nkv) * tail; it += blockDim.x) {
-    const int hh = it / tail, d = 2 * rot_half + (it - hh * tail) * 4;
-    bf16_t* dst;
-    if (hh < nq) {
-      dst = q_out + ((size_t)n * nq + hh) * hd;
-    } else {
-      if (s < 0) continue;
-      dst = kc + ((page * nkv + (hh - nq)) * ps + off) * hd;
-    }
-    *reinterpret_cast<uint2*>(dst + d) = pack4(add_bias(sums(hh * hd + d), hh * hd + d));
-  }
-  // values: [page][kv head][channel][slot]
-  if (s >= 0) {
-    for (int it = threadIdx.x; it < nkv * (hd / 4); it += blockDim.x) {
-      const int kvh = it / (hd / 4), d = (it - kvh * (hd / 4)) * 4, at = (nq + nkv + kvh) * hd + d;
-      const float4 v = add_bias(sums(at), at);
-      bf16_t* dst = vc + ((page * nkv + kvh) * hd + d) * ps + off;
-      dst[0] = f32_to_bf16(v.x);
-      dst[(size_t)ps] = f32_to_bf16(v.y);
-      dst[(size_t)2 * ps] = f32_to_bf16(v.z);
-      dst[(size_t)3 * ps] = f32_to_bf16(v.w);
-    }
   }
 }
 
@@ -384,9 +377,14 @@ extern "C" int qvl_rope_kv_write(const void* x, int x_stride, const void* bias, 
   if (nq + 2 * nkv > 65535) return QVL_ERR_LIMIT;
   if (in_dtype == 0 && dtype == 1 && cs && hd % 4 == 0 && rot_half % 4 == 0 && x_stride % 4 == 0 &&
       (((uintptr_t)x | (uintptr_t)bias | (uintptr_t)cs) & 15) == 0 && (((uintptr_t)q_out | (uintptr_t)kc) & 7) == 0) {
-    hipLaunchKernelGGL(rope_kv_write_wide_kernel, dim3(N), dim3(256), 0, stream, (const float*)x, x_stride,
-                       (const float*)bias, (const float2*)cs, (const int*)slot, (bf16_t*)q_out, (bf16_t*)kc,
-                       (bf16_t*)vc, nq, nkv, hd, rot_half, ps, nslabs, slab_stride);
+    const int items = (nq + nkv) * (rot_half / 4 + (hd - 2 * rot_half) / 4) + nkv * (hd / 4);
+#define QVL_ROPE_WIDE(AT_ONCE, share)                                                                                      \
+  hipLaunchKernelGGL((rope_kv_write_wide_kernel<AT_ONCE>), dim3(N, share), dim3(256), 0, stream, (const float*)x, x_stride,   \
+                     (const float*)bias, (const float2*)cs, (const int*)slot, (bf16_t*)q_out, (bf16_t*)kc, (bf16_t*)vc, nq,  \
+                     nkv, hd, rot_half, ps, nslabs, slab_stride)
+    if (N >= 512) QVL_ROPE_WIDE(1, 1);
+    else QVL_ROPE_WIDE(8, min(64, (items + 255) / 256));
+#undef QVL_ROPE_WIDE
     return qvl_launch_status();
   }
   if (nslabs > 1) return QVL_ERR_SHAPE;
