@@ -23,8 +23,6 @@
 
 enum { ROWS_BF16 = 0, ROWS_F32 = 1, ROWS_GATED = 2 };
 
-typedef float rows_f32x16 __attribute__((ext_vector_type(16)));
-
 struct RowsArgs {
   const bf16_t* x;
   long long ldx;
@@ -42,21 +40,6 @@ struct RowsArgs {
   int gelu;
   int pairs;        // bfloat16 results: two neighbouring ones may be stored at once
 };
-
-// Lane l of the wave puts its 16 bytes at M0 + 16 l of LDS; the lines are not kept in the caches.
-__device__ __forceinline__ void fetch16_once(const void* base, uint32_t lane_bytes, uint32_t lds_at) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(lane_bytes), "s"(base), "s"(lds_at)
-               : "memory", "m0");
-}
-template <int MOST, int LOADS>
-__device__ __forceinline__ void wait_steps(int ahead) {
-  if constexpr (MOST <= 0) {
-    tp_wait_fetches<0>();
-  } else {
-    if (ahead >= MOST) tp_wait_fetches<MOST * LOADS>();
-    else wait_steps<MOST - 1, LOADS>(ahead);
-  }
-}
 
 // MT column tiles of 32 rows of X; F fetches of 8 rows of W a step and wave: tiles of up to 8 F rows (4 F channels).
 template <int MT, int F, int OUT>
@@ -113,13 +96,13 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) void gemm_rows_kernel(RowsArgs p) 
     const uint32_t at = lds0 + ask_stage * STAGE, k = (uint32_t)ask_at * 128;
     if (last_chunks == 8 || ask_at != ksteps - 1) {
 #pragma unroll
-      for (int j = 0; j < F; ++j) fetch16_once(p.w, fw[j] + k, at + (wave * F + j) * 1024);
+      for (int j = 0; j < F; ++j) tp_fetch16_once(p.w, fw[j] + k, at + (wave * F + j) * 1024);
       tp_fetch16(p.x, fx + k, at + W_BYTES + x_place * 1024);
     } else {
       // chunks that lie beyond K are read from the step's first: they are not multiplied
       auto back = [&](int row) { const int c = (lane & 7) ^ ((row >> 1) & 7); return c < last_chunks ? 0u : 16u * c; };
 #pragma unroll
-      for (int j = 0; j < F; ++j) fetch16_once(p.w, fw[j] + k - back(8 * j + (lane >> 3)), at + (wave * F + j) * 1024);
+      for (int j = 0; j < F; ++j) tp_fetch16_once(p.w, fw[j] + k - back(8 * j + (lane >> 3)), at + (wave * F + j) * 1024);
       tp_fetch16(p.x, fx + k - back(x_row), at + W_BYTES + x_place * 1024);
     }
     ++asked;
@@ -136,7 +119,7 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) void gemm_rows_kernel(RowsArgs p) 
   // rows of a tile beyond its 8 F are not fetched: their operand is another row's, their sums are not stored
   const int wr = r < 8 * F ? r : r - 8 * F;
   const uint32_t wsw = (wr >> 1) & 7;
-  rows_f32x16 acc[MT];
+  tp_f32x16 acc[MT];
   auto clear = [&] {
 #pragma unroll
     for (int t = 0; t < MT; ++t)
@@ -226,7 +209,7 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) void gemm_rows_kernel(RowsArgs p) 
   };
   auto step = [&](int s, auto here, auto before) __attribute__((always_inline)) {
     if (s < steps) {
-      wait_steps<STAGES - 2, F + 1>(asked - 1 - s);      // all but the steps asked for behind this one have come
+      tp_wait_steps<STAGES - 2, F + 1>(asked - 1 - s);      // all but the steps asked for behind this one have come
       tp_wait_lds();
       tp_barrier();                           // every wave's part of the step is there, and the step before has been read
       ask();

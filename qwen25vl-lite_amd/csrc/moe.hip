@@ -261,75 +261,144 @@ __global__ __launch_bounds__(256) void moe_rows_kernel(ExpertArgs a) {
   }
 }
 
-// bfloat16 on the matrix cores, few pairs an expert (a decode step: the experts' weights are read once
-// each and that is the time it takes).  A block of four waves owns 16 MT pairs of one expert and 64 output
-// columns; a wave takes 16 of the columns (rows of W: the instruction's first operand, straight from
-// memory: nobody else in the block reads them) and all MT tiles of 16 pairs (rows of x: the second
-// operand).  K in steps of 32, a multiple of 8.  Which expert a block serves follows from the
-// offsets: tile t of the grid is the (t - tiles before e)-th tile of 16 MT pairs of expert e.
-template <int MT, typename TO>
-__global__ __launch_bounds__(256) void moe_mfma_kernel(ExpertArgs a) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lg = lane >> 4, r = lane & 15;
-  const ExpertTile at_expert = expert_tile(a.offsets, a.E, blockIdx.x, 16 * MT);
-  const int e = at_expert.e, first = at_expert.first, last = at_expert.last;
-  if (e >= a.E) return;
-  const int c0 = (blockIdx.y * 4 + wave) * 16;     // this wave's output columns
-  if (c0 >= a.R) return;
-  const int rows_w = a.gated ? 2 * a.R : a.R;
-  const bf16_t* we = (const bf16_t*)a.w + (size_t)e * rows_w * a.K;
-  const bool col_ok = c0 + r < a.R;
-  const bf16_t* wg = we + (size_t)(col_ok ? c0 + r : 0) * a.K + 8 * lg;
-  const bf16_t* wu = wg + (size_t)a.R * a.K;      // only read if gated
-  const bf16_t* xr[MT];
-  int pair[MT];
+// bfloat16 on the matrix cores, few pairs an expert (a decode step: the experts' weights are read once each and that is
+// the time it takes).  An item is 32 pairs of an expert at most and the rows of W of a block of eight waves, `per` rows
+// (gated: channels) a wave, operands of v_mfma_f32_32x32x16_bf16.  One block a compute unit works through item after item:
+// how many experts have pairs is known on the device only, so `per` is chosen here, as the fewest that
+// take no more rounds of items over all blocks than the most would.  W and the gathered rows of x come through LDS in steps
+// of 64 values of K, W marked as read once, 144 KB of steps on their way, the steps of an item behind those of the item before.
+// 48 pairs over 32 experts, K 3,584, 2 x 2,368 rows: 134 us = 6.3 TB/s; K 2,368, 3,584 rows: 72 us = 5.9 TB/s.  16 rows of W a
+// wave straight into registers, half a line a row, 16 pairs a block: 235 and 118 us.
+#define FEW_WAVES 8
+#define FEW_PAIRS 32
+template <bool GATED, typename TO>
+__global__ __launch_bounds__(64 * FEW_WAVES) void moe_few_kernel(ExpertArgs a) {
+  constexpr int F = 4, W_BYTES = FEW_WAVES * F * 1024, STAGE = W_BYTES + 4096, STAGES = 4, HALF = 2 * F;
+  constexpr int MOST = GATED ? 16 : 32;
+  __shared__ __attribute__((aligned(16))) char lds[STAGES * STAGE];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, hi = lane >> 5, r = lane & 31;
+  int tiles = 0;                              // of at most 32 pairs, over all experts
+  for (int e0 = 0; e0 < a.E; e0 += 64) {
+    const int e = e0 + lane;
+    int n = e < a.E ? (a.offsets[e + 1] - a.offsets[e] + FEW_PAIRS - 1) / FEW_PAIRS : 0;
 #pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    const int i = first + 16 * t + r;
-    pair[t] = i < last ? a.sorted[i] : -1;
-    xr[t] = (const bf16_t*)a.x + (size_t)(pair[t] < 0 ? 0 : pair[t] / a.div) * a.ldx + 8 * lg;
+    for (int o = 32; o; o >>= 1) n += __shfl_xor(n, o, QVL_WAVE);
+    tiles += n;
   }
-  f32x4_t accg[MT], accu[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    accg[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    accu[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  }
-  // No load stands inside a branch (the compiler would wait for each before the next): what does not
-  // exist is read from a place that does (column 0 of the step, row 0) and replaced by zeros.
-  const bf16x8_t zero = __builtin_bit_cast(bf16x8_t, uint4{0u, 0u, 0u, 0u});
-  if (!a.gated) wu = wg;
-#pragma unroll 2
-  for (int k = 0; k < a.K; k += 32) {
-    const bool k_ok = k + 8 * lg < a.K;
-    const int at = k_ok ? k : k - 8 * lg;
-    bf16x8_t fg = *reinterpret_cast<const bf16x8_t*>(wg + at);
-    bf16x8_t fu = *reinterpret_cast<const bf16x8_t*>(wu + at);
-    bf16x8_t fx[MT];
-#pragma unroll
-    for (int t = 0; t < MT; ++t) fx[t] = *reinterpret_cast<const bf16x8_t*>(xr[t] + at);
-    fg = (k_ok && col_ok) ? fg : zero;
-    fu = (k_ok && col_ok) ? fu : zero;
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-      const bf16x8_t f = (k_ok && pair[t] >= 0) ? fx[t] : zero;
-      accg[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fg, f, accg[t], 0, 0, 0);
-      if (a.gated) accu[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fu, f, accu[t], 0, 0, 0);
+  tiles = __builtin_amdgcn_readfirstlane(tiles);
+  const int blocks = gridDim.x;
+  auto groups_of = [&](int per) { return (a.R + FEW_WAVES * per - 1) / (FEW_WAVES * per); };
+  const long long most_items = (long long)tiles * groups_of(MOST);
+  const long long rounds_all = (most_items + blocks - 1) / blocks;
+  const long long shares = max(1ll, rounds_all * blocks * FEW_WAVES);
+  int per = (int)max(1ll, min((long long)MOST, ((long long)tiles * a.R + shares - 1) / shares));
+  while (per < MOST && (long long)tiles * groups_of(per) > rounds_all * blocks) ++per;
+  const int groups = groups_of(per), items = tiles * groups;
+  const int first_item = blockIdx.x, rounds = first_item < items ? (items - first_item + blocks - 1) / blocks : 0;
+  const int ksteps = (a.K + 63) / 64, steps = ksteps * rounds;
+  const int last_chunks = a.K % 64 ? (a.K % 64) / 8 : 8;     // of a last step, 8 values each
+  // Row of W behind row i of a wave's tile (-1: there is none).  Row i's sums are number 4 (i / 8) + i mod 4 of the lanes whose
+  // hi is (i / 4) mod 2; gated: the first half of a lane's sums are gates, the others their up values.
+  auto w_row = [&](int c0, int i) {
+    int j = i, up = 0;
+    if (GATED) {
+      const int s = 4 * (i >> 3) + (i & 3);
+      up = s >= HALF;
+      j = ((i >> 2) & 1) * HALF + s - up * HALF;
     }
-  }
-  // a lane holds, of tile t, pair r and columns c0 + 4 lg .. + 3
+    return (j < per && c0 + j < a.R) ? c0 + j + up * a.R : -1;
+  };
+  // this lane's fetches: rows 8 j + lane / 8 of the wave's tile, the row's chunk (lane mod 8) ^ ((row / 2) mod 8), and of x
+  // row 8 (wave mod 4) + lane / 8 (two waves fetch the same: every wave then waits for as many).  A row that does not exist
+  // is read from one that does; its sums are not stored.
+  uint32_t fw[F], fx = 0;
+  const char* w_base = (const char*)a.w;
+  const int x_place = wave & 3, x_row = 8 * x_place + (lane >> 3);
+  auto column = [&](int item) { return ((item % groups) * FEW_WAVES + wave) * per; };
+  auto set_item = [&](int item) __attribute__((always_inline)) {
+    const ExpertTile at = expert_tile(a.offsets, a.E, item / groups, FEW_PAIRS);
+    w_base = (const char*)a.w + (size_t)at.e * (GATED ? 2 * a.R : a.R) * a.K * 2;
+    const int c0 = column(item), exists = max(w_row(c0, 0), 0);
 #pragma unroll
-  for (int t = 0; t < MT; ++t) {
-    if (pair[t] < 0) continue;
-    TO* o = (TO*)a.out + (size_t)pair[t] * a.ldo + c0 + 4 * lg;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (c0 + 4 * lg + j >= a.R) break;
-      float v = accg[t][j];
-      if (a.gated) v = gated_value(v, accu[t][j], a.alpha, a.limit, a.shift);
-      else v = plain_value(v, a.act);
-      stf<TO>(o + j, v);
+    for (int j = 0; j < F; ++j) {
+      const int rho = 8 * j + (lane >> 3);
+      int n = w_row(c0, rho);
+      if (n < 0) n = exists;
+      fw[j] = (uint32_t)n * (uint32_t)a.K * 2 + 16 * ((lane & 7) ^ ((rho >> 1) & 7));
     }
+    const int i = at.first + x_row;
+    fx = (uint32_t)(a.sorted[i < at.last ? i : at.first] / a.div) * (uint32_t)a.ldx * 2 + 16 * ((lane & 7) ^ ((x_row >> 1) & 7));
+  };
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)&lds[0];
+  // blocks begin an item at different places of K and go round, so that they do not all ask the same few memory channels
+  const int turn = (int)((blockIdx.x * 29u) % (unsigned)ksteps);
+  int asked = 0, ask_k = 0, ask_item = first_item, ask_stage = 0, ask_at = turn;
+  auto ask = [&]() __attribute__((always_inline)) {          // the next step's fetches, if there is one
+    if (asked >= steps) return;
+    if (ask_k == 0) set_item(ask_item);
+    const uint32_t at = lds0 + ask_stage * STAGE, k = (uint32_t)ask_at * 128;
+    // chunks of a last step that lie beyond K are read from its first: they are not multiplied
+    const int chunks = ask_at == ksteps - 1 ? last_chunks : 8;
+    auto back = [&](int row) { const int c = (lane & 7) ^ ((row >> 1) & 7); return c < chunks ? 0u : 16u * c; };
+#pragma unroll
+    for (int j = 0; j < F; ++j) tp_fetch16_once(w_base, fw[j] + k - back(8 * j + (lane >> 3)), at + (wave * F + j) * 1024);
+    tp_fetch16(a.x, fx + k - back(x_row), at + W_BYTES + x_place * 1024);
+    ++asked;
+    ask_stage = ask_stage + 1 == STAGES ? 0 : ask_stage + 1;
+    if (++ask_at == ksteps) ask_at = 0;
+    if (++ask_k == ksteps) {
+      ask_k = 0;
+      ask_item += blocks;
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < STAGES - 1; ++i) ask();
+  const uint32_t sw = (r >> 1) & 7;
+  tp_f32x16 acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  int stage = 0, at_k = turn, left = ksteps, item = first_item;
+  for (int s = 0; s < steps; ++s) {
+    tp_wait_steps<STAGES - 2, F + 1>(asked - 1 - s);      // all but the steps asked for behind this one have come
+    tp_wait_lds();
+    tp_barrier();                           // every wave's part of the step is there, and the step before has been read
+    ask();
+    const char* pw = lds + stage * STAGE + (wave * F * 8 + r) * 128;
+    const char* px = lds + stage * STAGE + W_BYTES + r * 128;
+    tp_bf16x8 w8[4], x8[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      w8[k] = *reinterpret_cast<const tp_bf16x8*>(pw + (((2 * k + hi) ^ sw) << 4));
+      x8[k] = *reinterpret_cast<const tp_bf16x8*>(px + (((2 * k + hi) ^ sw) << 4));
+    }
+    if (last_chunks < 8 && at_k == ksteps - 1) {           // chunks beyond K are no part of the sums
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (2 * k + hi >= last_chunks) w8[k] = x8[k] = tp_bf16x8{};
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w8[k], x8[k], acc, 0, 0, 0);
+    stage = stage + 1 == STAGES ? 0 : stage + 1;
+    if (++at_k == ksteps) at_k = 0;
+    if (--left) continue;
+    // an item's sums: a lane holds pair r of the tile
+    const ExpertTile at = expert_tile(a.offsets, a.E, item / groups, FEW_PAIRS);
+    const int c0 = column(item), i = at.first + r;
+    if (i < at.last) {
+      TO* o = (TO*)a.out + (size_t)a.sorted[i] * a.ldo + c0;
+#pragma unroll
+      for (int n = 0; n < (GATED ? HALF : 16); ++n) {
+        const int j = GATED ? hi * HALF + n : 8 * (n >> 2) + 4 * hi + (n & 3);
+        if (j >= per || c0 + j >= a.R) continue;
+        stf<TO>(o + j, GATED ? gated_value(acc[n], acc[n + HALF], a.alpha, a.limit, a.shift) : plain_value(acc[n], a.act));
+      }
+    }
+#pragma unroll
+    for (int n = 0; n < 16; ++n) acc[n] = 0.f;
+    left = ksteps;
+    item += blocks;
   }
+  tp_wait_fetches<0>();
 }
 
 // Many pairs an expert: tiles of TILE_M pairs x TILE_N rows of W (gated: TILE_N / 2 gate rows and the up rows
@@ -507,7 +576,8 @@ __global__ __launch_bounds__(256) void moe_tile_kernel(ExpertArgs a, int tiles_m
 // The same product through the inner loop of tile_product.h: tiles of 128 pairs x 256 rows of W (gated: 128 gate
 // rows and the up rows of the same outputs; a wave's gate and up values of an output end in one lane).  K must be a
 // multiple of 32 and offsets within x and within an expert's W 32-bit.  Measured on 12,384 pairs over 32 experts, K
-// 3,584: 2 x 2,368 rows 655 us (tiles of 128 x 256 with all waves in step: 874), 3,584 rows of K 2,368 320 us (480).
+// 3,584: 2 x 2,368 rows 655 us (tiles of 128 x 256 with all waves in step: 874); down and per-head products of a prompt's pass 207 us
+// on average (316).
 typedef Tile<4, 2, 4, 4> ExpertsTile;
 
 template <typename TO>
@@ -587,7 +657,7 @@ extern "C" int qvl_moe_experts(const void* x, long long ldx, int x_dtype, const 
                                const void* offsets, void* out, long long ldo, int out_dtype, int P, int E, int R, int K,
                                int div,
                                int gated, float alpha, float limit, float shift, int act, int big_tiles,
-                               hipStream_t stream) {
+                               int cus, hipStream_t stream) {
   if (P <= 0) return QVL_OK;
   if (E <= 0 || R <= 0 || K <= 0 || div <= 0 || ldx < K || ldo < R || !x || !w || !sorted || !offsets || !out) return QVL_ERR_SHAPE;
   ExpertArgs a;
@@ -627,13 +697,17 @@ extern "C" int qvl_moe_experts(const void* x, long long ldx, int x_dtype, const 
       else hipLaunchKernelGGL((moe_tile_kernel<false, float>), tgrid, dim3(256), 0, stream, a, tiles_m, tiles_n);
       return qvl_launch_status();
     }
-    const int tiles = P / 16 + (E < P ? E : P);
-    const dim3 grid(tiles, (R + 63) / 64);
-    if (grid.y > 65535) return QVL_ERR_LIMIT;
-    if (out_dtype == 1) hipLaunchKernelGGL((moe_mfma_kernel<1, bf16_t>), grid, dim3(256), 0, stream, a);
-    else if (out_dtype == 0) hipLaunchKernelGGL((moe_mfma_kernel<1, float>), grid, dim3(256), 0, stream, a);
-    else return QVL_ERR_DTYPE;
-    return qvl_launch_status();
+    if (cus <= 0) return QVL_ERR_SHAPE;
+    if (x_rows * (unsigned long long)ldx * 2 < 0xffff0000ull && (unsigned long long)(gated ? 2 * R : R) * K * 2 < 0xffff0000ull &&
+        (long long)(P / FEW_PAIRS + (E < P ? E : P)) * ((R + FEW_WAVES - 1) / FEW_WAVES) < 0x7ffffff0ll) {
+#define FEW(G, TO) hipLaunchKernelGGL((moe_few_kernel<G, TO>), dim3(cus), dim3(64 * FEW_WAVES), 0, stream, a)
+      if (gated && out_dtype == 1) FEW(true, bf16_t);
+      else if (gated) FEW(true, float);
+      else if (out_dtype == 1) FEW(false, bf16_t);
+      else FEW(false, float);
+#undef FEW
+      return qvl_launch_status();
+    }
   }
   int by = (R + 3) / 4;
   if (by > 64) by = 64;

@@ -20,6 +20,7 @@
 
 typedef __bf16 tp_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float tp_f32x4 __attribute__((ext_vector_type(4)));
+typedef float tp_f32x16 __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ void tp_fetch16(const void* base, uint32_t lane_bytes, uint32_t lds_at) {
   // lane l of the wave puts its 16 bytes at M0 + 16 l of LDS
@@ -37,6 +38,22 @@ __device__ __forceinline__ void tp_barrier() {
   __builtin_amdgcn_sched_barrier(0);
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
+}
+
+// Lane l of the wave puts its 16 bytes at M0 + 16 l of LDS; the lines are not kept in the caches.
+__device__ __forceinline__ void tp_fetch16_once(const void* base, uint32_t lane_bytes, uint32_t lds_at) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(lane_bytes), "s"(base), "s"(lds_at)
+               : "memory", "m0");
+}
+// All but the `ahead` steps of LOADS fetches asked for last have come (at most MOST are ahead).
+template <int MOST, int LOADS>
+__device__ __forceinline__ void tp_wait_steps(int ahead) {
+  if constexpr (MOST <= 0) {
+    tp_wait_fetches<0>();
+  } else {
+    if (ahead >= MOST) tp_wait_fetches<MOST * LOADS>();
+    else tp_wait_steps<MOST - 1, LOADS>(ahead);
+  }
 }
 
 template <int WN_, int WM_, int NT_, int MT_>

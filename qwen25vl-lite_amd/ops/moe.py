@@ -13,7 +13,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from .kernels import _check, _dev, _fn, _need, _ptr, _stream, dtype_code
+from .kernels import _check, _dev, _fn, _need, _ptr, _stream, compute_units, dtype_code
 
 __all__ = ["route", "sort_pairs", "pairs_by_column", "expert_products", "combine", "SCORE_FUNCTIONS", "BIG_TILE_PAIRS"]
 
@@ -100,10 +100,10 @@ def expert_products(x: torch.Tensor, weight: torch.Tensor, order: torch.Tensor, 
     alpha, limit, shift = gated if gated else (1.0, None, 0.0)
     fn = _fn("moe", "qvl_moe_experts", [_c_ptr, _c_ll, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ll, _c_int, _c_int,
                                         _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_float, _c_float, _c_int, _c_int,
-                                        _c_ptr])
+                                        _c_int, _c_ptr])
     _check(fn(_ptr(x), x.stride(0), dtype_code(x.dtype), _ptr(weight), _ptr(order), _ptr(offsets), _ptr(out),
               out.stride(0), dtype_code(out_dtype), int(pairs), e, r, k, int(div), int(bool(gated)), float(alpha), float(limit or 0.0),
-              float(shift), PLAIN_ACTS[act], int(pairs >= BIG_TILE_PAIRS * e), _stream()), "moe experts")
+              float(shift), PLAIN_ACTS[act], int(pairs >= BIG_TILE_PAIRS * e), compute_units(x.device), _stream()), "moe experts")
     return out
 
 

@@ -666,6 +666,44 @@ def test_rows_against_many_outputs(m, n, k):
         assert bool(((got - ref).abs() <= slack + (2.0 ** -8 + 1e-5) * ref.abs() + 1e-5 * pairs[:, :, 1].abs().reshape(m, n // 2)).all())
 
 
+@pytest.mark.parametrize("e, r, k, pairs", [(3, 40, 72, "one"), (8, 300, 200, "uneven"), (70, 129, 64, "uneven"), (4, 2368, 136, "all on one"),
+                                            (200, 1, 8, "uneven"), (32, 520, 2056, "few")])
+def test_experts_with_few_pairs(e, r, k, pairs):
+    """The experts' products of a decode step: experts with no pair, with one and with more than the 32 of a tile, rows and
+    inner sizes that fill no tile and no step, NaN beside the rows of x, more experts than lanes; plain, squared and
+    gated, both output types.  A sum of k exact products is within k roundings of its terms."""
+    from qwen25vl_lite_amd.ops import moe
+    torch.manual_seed(e + r)
+    top, n = 2, {"one": 1, "uneven": 45, "all on one": 20, "few": 8}[pairs]
+    ids = torch.randint(0, e, (n, top), dtype=torch.int32, device="cuda")
+    if pairs == "uneven":
+        ids[:, 0] = e // 2
+    elif pairs == "all on one":
+        ids[:] = 2
+    order, offsets = moe.sort_pairs(ids, e)
+    x = torch.full((n, k + 64), float("nan"), device="cuda").bfloat16()[:, :k]
+    x.copy_(torch.randn(n, k, device="cuda"))
+    w = (torch.randn(e, 2 * r, k, device="cuda") / math.sqrt(k)).bfloat16()
+    flat = ids.view(-1).long()
+    xs, ws = x.double().repeat_interleave(top, 0), w.double()[flat]
+    want = torch.einsum("pk,prk->pr", xs, ws)
+    bound = k * 2.0 ** -24 * torch.einsum("pk,prk->pr", xs.abs(), ws.abs()) + 1e-30
+    got = moe.expert_products(x, w, order, offsets, n * top, top, torch.float32)
+    assert bool(((got.double() - want).abs() <= bound).all())
+    room = torch.full((n * top, 2 * r + 3), 7.0, device="cuda").bfloat16()
+    moe.expert_products(x, w, order, offsets, n * top, top, torch.bfloat16, act="relu2", out=room[:, :2 * r])
+    ref = want.clamp(min=0) ** 2
+    slack = (2 * want.abs() + bound) * bound
+    assert bool(((room[:, :2 * r].double() - ref).abs() <= slack + (2.0 ** -8 + 1e-6) * ref).all()) and bool((room[:, 2 * r:] == 7.0).all())
+    g, u = want[:, :r].clamp(max=1.5), want[:, r:].clamp(-1.5, 1.5)
+    ref = g * torch.sigmoid(1.25 * g) * (u + 1.0)
+    # slopes: of g sigmoid(1.25 g) below 1.13, of u one; values |u + 1| <= 2.5, |g sigmoid| <= 1.5 above and 0.3 below
+    slack = 1.13 * 2.5 * bound[:, :r] + 1.5 * bound[:, r:]
+    for dtype, last in ((torch.float32, 0.0), (torch.bfloat16, 2.0 ** -8)):
+        got = moe.expert_products(x, w, order, offsets, n * top, top, dtype, gated=(1.25, 1.5, 1.0)).double()
+        assert bool(((got - ref).abs() <= slack + (last + 1e-6) * ref.abs() + 2e-6).all())
+
+
 def test_no_cpu_path():
     from qwen25vl_lite_amd.ops import kernels
     from qwen25vl_lite_amd.ops.linear import linear
