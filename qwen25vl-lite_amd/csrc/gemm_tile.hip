@@ -148,7 +148,9 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(TileArgs p) {
 // How a product is cut: the tile's shape and the ranges of K.  The estimate is of microseconds: a step of 64 values
 // costs a block `alone` where most compute units are idle and `full` where all work (a step of 256 x 256 takes 1.08 and
 // 1.43 us: with every matrix core busy the clock and the caches give way), a launch 8 us and each of its rounds 4 (the
-// first fetches, the stores); slabs are written and read once more, at 4.5 TB/s.
+// first fetches, the stores); slabs are written and read once more, at 4.5 TB/s.  Where two blocks share a compute unit, a
+// last round of up to half the room has a unit for each block, else some blocks have to share (22,016 x 2,048 gated: 172
+// blocks of 128 x 128 28 us, 344 43; of 128 x 256 172 36).
 struct Plan {
   int tile, splits;
   double us;
@@ -157,7 +159,7 @@ struct TileShape {
   int bn, bm, a_unit;     // blocks a compute unit holds
   double alone, full;
 };
-static const TileShape SHAPES[4] = {{256, 256, 1, 1.08, 1.43}, {128, 256, 1, 0.80, 0.96}, {256, 128, 1, 0.79, 0.94}, {128, 128, 2, 0.62, 1.02}};
+static const TileShape SHAPES[4] = {{256, 256, 1, 1.08, 1.43}, {128, 256, 1, 0.72, 0.96}, {256, 128, 1, 0.79, 0.94}, {128, 128, 2, 0.53, 1.02}};
 
 static Plan plan_for(int M, int N, int K, int most_splits, int cus) {
   Plan best{0, 1, 1e30};
@@ -170,7 +172,8 @@ static Plan plan_for(int M, int N, int K, int most_splits, int cus) {
       const double rest = (double)(blocks - whole * room) / room;
       const double depth = (steps + splits - 1) / splits;
       double us = 8.0 + whole * (depth * s.full + 4.0);
-      if (rest > 0) us += depth * (s.alone + (s.full - s.alone) * rest) + 4.0;
+      const double busy = s.a_unit == 1 ? rest : (2.0 * rest > 1.0 ? 1.0 : 0.0);
+      if (rest > 0) us += depth * (s.alone + (s.full - s.alone) * busy) + 4.0;
       if (splits > 1) us += splits * (double)M * N * 8.0 / 4.5e6;
       if (us < best.us) best = Plan{i, splits, us};
     }

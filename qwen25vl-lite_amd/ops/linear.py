@@ -172,6 +172,6 @@ def gate_up_swiglu(x: Union[torch.Tensor, NormedRows], weight: torch.Tensor, gro
         x = x.materialize()
     if grouped and weight.shape[0] % 16 == 0 and rows.prefers_rows(x, weight):
         return rows.rows_swiglu(x, weight, act)
-    if grouped and weight.shape[0] % 16 == 0 and x.is_cuda and tile.prefers_tile(x, weight):
+    if grouped and weight.shape[0] % 16 == 0 and x.is_cuda and tile.prefers_tile(x, weight, gated=True):
         return tile.tile_swiglu(x, weight, act)
     return kernels.swiglu(linear(x, weight), grouped=grouped, act=act)

@@ -34,15 +34,17 @@ def takes_tile(x: torch.Tensor, weight: torch.Tensor, halves: bool = False) -> b
 MANY_ROWS = 64           # up to here the decode kernels and the library run
 
 
-def prefers_tile(x: torch.Tensor, weight: torch.Tensor, halves: bool = False) -> bool:
+def prefers_tile(x: torch.Tensor, weight: torch.Tensor, halves: bool = False, gated: bool = False) -> bool:
     """Whether the kernel takes the product and is the faster way to it, uncut: more than ``MANY_ROWS`` rows, and tiles for
     three quarters of the compute units (2,048 x 3,584 x 3,584: 224 tiles, 63 us against the library's 66; 280 x 2,560 x
-    2,048: 60 tiles, 34 against 24, the library cuts the inner size)."""
+    2,048: 60 tiles, 34 against 24, the library cuts the inner size).  With a gated activation on the sums (``gated``), which
+    takes the library another kernel, half of them suffice (22,016 x 2,048: 100 rows, 172 tiles, 29 us against 35; 190 rows,
+    172 tiles, 37 against 41; 380 rows, 172 tiles, 52 against 53; 37,888 x 3,584, 190 rows, 148 tiles, 83 against 89)."""
     if x.shape[0] <= MANY_ROWS or not takes_tile(x, weight, halves):
         return False
     cus = compute_units(x.device)
     blocks = int(_fn("gemm_tile", "qvl_gemm_tile_blocks", [_c_int] * 4)(x.shape[0], weight.shape[0], x.shape[1], cus))
-    return 4 * blocks >= 3 * cus
+    return 2 * blocks >= cus if gated or halves else 4 * blocks >= 3 * cus
 
 
 def _launch(x, weight, out, ldo, mode, splits=1, relu2=0, gelu=0, alpha=1.0, limit=0.0, shift=0.0, shape=-1):
