@@ -1,5 +1,5 @@
 // Products with 17 to 64 rows: out = X[M, K] . W[N, K]^T, bfloat16 operands, float32 sums, stored as they are, as bfloat16, through
-// the gated activation of W's rows in groups of 8 gate and 8 up rows, or as one slab of sums for each range of K.
+// the gated activation of W's rows (groups of 8 gate and 8 up rows, or all gate rows first), or as one slab of sums for each range of K.
 //
 // What bounds it is reading W once.  A wave owns up to 32 rows of W and all rows of X (operands of
 // v_mfma_f32_32x32x16_bf16), eight waves are a block and a block has a compute unit to itself; the rows a wave takes at a time
@@ -21,7 +21,7 @@
 #define ROWS_WAVES 8
 #define ROWS_LDS 163840
 
-enum { ROWS_BF16 = 0, ROWS_F32 = 1, ROWS_GATED = 2 };
+enum { ROWS_BF16 = 0, ROWS_F32 = 1, ROWS_GATED = 2, ROWS_HALVES = 3 };
 
 struct RowsArgs {
   const bf16_t* x;
@@ -31,15 +31,25 @@ struct RowsArgs {
   void* out;
   long long ldo;
   int M, N, K;
-  int per;          // rows of W a wave takes at a time (ROWS_GATED: channels); even where results are bfloat16
+  int per;          // rows of W a wave takes at a time (gated: channels); even where results are bfloat16
   int tiles;        // of all of W
   int blocks;       // that share the tiles (of one range of K)
   int rounds;       // tiles of a wave
   int range_steps;  // steps of 64 values in a range of K; range i has the blocks i * blocks .. and the slab i of out
   long long slab;
   int gelu;
+  float alpha, limit, shift;
   int pairs;        // bfloat16 results: two neighbouring ones may be stored at once
 };
+
+// g sigmoid(alpha g) (u + shift); limit > 0: g capped at it, u clamped to +-limit.
+__device__ __forceinline__ float clamped_gate(const RowsArgs& p, float g, float u) {
+  if (p.limit > 0.f) {
+    g = fminf(g, p.limit);
+    u = fminf(fmaxf(u, -p.limit), p.limit);
+  }
+  return g / (1.0f + expf(-p.alpha * g)) * (u + p.shift);
+}
 
 // MT column tiles of 32 rows of X; F fetches of 8 rows of W a step and wave: tiles of up to 8 F rows (4 F channels).
 template <int MT, int F, int OUT>
@@ -48,10 +58,10 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) void gemm_rows_kernel(RowsArgs p) 
   // MT = 1: X's four fetches of a step are made by two waves each (the same bytes to the same place), so that every wave
   // waits for as many
   constexpr int X_PLACES = 4 * MT;
-  constexpr int HALF = 2 * F;                 // ROWS_GATED: gates among a lane's 4 F sums
+  constexpr int HALF = 2 * F;                 // gated: gates among a lane's 4 F sums
   // float32 results: a lane holds one row of W (neighbouring lanes store neighbouring results); else neighbouring rows of W, so
   // that gate and up value meet in a lane and two results of two bytes are stored at once
-  constexpr bool X_FIRST = OUT == ROWS_F32;
+  constexpr bool X_FIRST = OUT == ROWS_F32, GATED = OUT == ROWS_GATED || OUT == ROWS_HALVES;
   __shared__ __attribute__((aligned(16))) char lds[STAGES * STAGE];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, hi = lane >> 5, r = lane & 31;
   const int range = blockIdx.x / p.blocks;
@@ -59,13 +69,14 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) void gemm_rows_kernel(RowsArgs p) 
   const int k_first = range * p.range_steps * 64, k_values = min(p.K - k_first, p.range_steps * 64);
   const int ksteps = (k_values + 63) / 64, steps = ksteps * p.rounds;
   const int last_chunks = k_values % 64 ? (k_values % 64) / 8 : 8;     // of a last step, 8 values each
-  // row of W behind row i of a tile (-1: there is none).  ROWS_GATED: row i's sums are number 4 (i / 8) + i mod 4 of the lanes
+  // row of W behind row i of a tile (-1: there is none).  Gated: row i's sums are number 4 (i / 8) + i mod 4 of the lanes
   // whose hi is (i / 4) mod 2, and the first half of a lane's sums are gates, the others their up values.
   auto w_row = [&](int tile, int i) {
     if (tile >= p.tiles) return -1;
-    if (OUT == ROWS_GATED) {
+    if (GATED) {
       const int s = 4 * (i >> 3) + (i & 3), up = s >= HALF, j = ((i >> 2) & 1) * HALF + s - up * HALF, c = tile * p.per + j;
-      return (j < p.per && 2 * c < p.N) ? (c >> 3) * 16 + (c & 7) + 8 * up : -1;
+      if (j >= p.per || 2 * c >= p.N) return -1;
+      return OUT == ROWS_HALVES ? c + up * (p.N / 2) : (c >> 3) * 16 + (c & 7) + 8 * up;
     }
     const int n = tile * p.per + i;
     return (i < p.per && n < p.N) ? n : -1;
@@ -148,14 +159,17 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) void gemm_rows_kernel(RowsArgs p) 
         bf16_t* out = reinterpret_cast<bf16_t*>(p.out) + (size_t)m * p.ldo;
         // results in pairs: numbers 2 i and 2 i + 1 of the lane's
 #pragma unroll
-        for (int i = 0; i < (OUT == ROWS_GATED ? HALF / 2 : HALF); ++i) {
+        for (int i = 0; i < (GATED ? HALF / 2 : HALF); ++i) {
           float v0 = acc[t][2 * i], v1 = acc[t][2 * i + 1];
           if (OUT == ROWS_GATED) {
             v0 = gate_act(v0, p.gelu) * acc[t][HALF + 2 * i];
             v1 = gate_act(v1, p.gelu) * acc[t][HALF + 2 * i + 1];
+          } else if (OUT == ROWS_HALVES) {
+            v0 = clamped_gate(p, v0, acc[t][HALF + 2 * i]);
+            v1 = clamped_gate(p, v1, acc[t][HALF + 2 * i + 1]);
           }
-          const int j = OUT == ROWS_GATED ? hi * HALF + 2 * i : 8 * (i >> 1) + 4 * hi + 2 * (i & 1);
-          const int n = tile * p.per + j, end = OUT == ROWS_GATED ? p.N / 2 : p.N;
+          const int j = GATED ? hi * HALF + 2 * i : 8 * (i >> 1) + 4 * hi + 2 * (i & 1);
+          const int n = tile * p.per + j, end = GATED ? p.N / 2 : p.N;
           if (j >= p.per || n >= end) continue;
           if (p.pairs && n + 1 < end) {
             *reinterpret_cast<uint32_t*>(out + n) = (uint32_t)f32_to_bf16(v0) | ((uint32_t)f32_to_bf16(v1) << 16);
@@ -239,14 +253,15 @@ static int rows_check(const RowsArgs& p, const void* x, const void* w, const voi
   return QVL_OK;
 }
 static int rows_launch(RowsArgs& p, int ranges, int mode, hipStream_t stream) {
-  const int rows = mode == ROWS_GATED ? 2 * p.per : p.per, fetches = rows <= 16 ? 2 : (rows + 7) / 8;
+  const int rows = mode >= ROWS_GATED ? 2 * p.per : p.per, fetches = rows <= 16 ? 2 : (rows + 7) / 8;
   const dim3 grid((unsigned)(p.blocks * ranges)), block(64 * ROWS_WAVES);
 #define GO(MT, F, OUT) hipLaunchKernelGGL((gemm_rows_kernel<MT, F, OUT>), grid, block, 0, stream, p)
 #define MODE(MT, F)                               \
   do {                                            \
     if (mode == ROWS_BF16) GO(MT, F, ROWS_BF16);  \
     else if (mode == ROWS_F32) GO(MT, F, ROWS_F32); \
-    else GO(MT, F, ROWS_GATED);                   \
+    else if (mode == ROWS_GATED) GO(MT, F, ROWS_GATED); \
+    else GO(MT, F, ROWS_HALVES);                  \
   } while (0)
 #define FETCHES(MT)                     \
   do {                                  \
@@ -263,18 +278,19 @@ static int rows_launch(RowsArgs& p, int ranges, int mode, hipStream_t stream) {
 }
 
 // x: bfloat16 [M, K], rows ldx apart, M at most 64; w: bfloat16 [N, K], rows ldw apart; both on 16-byte boundaries, K a multiple
-// of 8.  mode 0: out bfloat16 [M, N]; 1: float32; 2: W's rows in groups of 8 gate + 8 up, out bfloat16 [M, N / 2] = act(gate) up.
+// of 8.  mode 0: out bfloat16 [M, N]; 1: float32; 2: W's rows in groups of 8 gate + 8 up, out bfloat16 [M, N / 2] = act(gate) up;
+// 3: N / 2 gate rows, then the up rows, out = g sigmoid(alpha g) (u + shift), g capped at limit, u clamped to +-limit.
 extern "C" int qvl_gemm_rows(const void* x, long long ldx, const void* w, long long ldw, void* out, long long ldo, int M, int N,
-                             int K, int mode, int gelu, int cus, hipStream_t stream) {
+                             int K, int mode, int gelu, float alpha, float limit, float shift, int cus, hipStream_t stream) {
   if (M <= 0 || N <= 0) return QVL_OK;
-  if (mode < 0 || mode > 2 || (mode == 2 && N % 16) || ldo < (mode == 2 ? N / 2 : N)) return QVL_ERR_SHAPE;
+  if (mode < 0 || mode > 3 || (mode == 2 && N % 16) || (mode == 3 && N % 2) || ldo < (mode >= 2 ? N / 2 : N)) return QVL_ERR_SHAPE;
   RowsArgs p;
   p.x = (const bf16_t*)x; p.ldx = ldx; p.w = (const bf16_t*)w; p.ldw = ldw; p.out = out; p.ldo = ldo;
-  p.M = M; p.N = N; p.K = K; p.gelu = gelu; p.slab = 0; p.range_steps = (K + 63) / 64;
+  p.M = M; p.N = N; p.K = K; p.gelu = gelu; p.alpha = alpha; p.limit = limit; p.shift = shift; p.slab = 0; p.range_steps = (K + 63) / 64;
   const int bad = rows_check(p, x, w, out, cus);
   if (bad) return bad;
   // the fewest rounds over a block a compute unit, then the fewest rows a wave that these rounds need
-  const long long items = mode == 2 ? N / 2 : N, most = mode == 2 ? 16 : 32, waves = (long long)cus * ROWS_WAVES;
+  const long long items = mode >= 2 ? N / 2 : N, most = mode >= 2 ? 16 : 32, waves = (long long)cus * ROWS_WAVES;
   const long long rounds = (items + most * waves - 1) / (most * waves);
   p.per = (int)((items + rounds * waves - 1) / (rounds * waves));
   if (mode != 1) p.per = (p.per + 1) / 2 * 2;
@@ -311,7 +327,7 @@ extern "C" int qvl_gemm_rows_cut(const void* x, long long ldx, const void* w, lo
   if (M <= 0 || N <= 0) return QVL_OK;
   RowsArgs p;
   p.x = (const bf16_t*)x; p.ldx = ldx; p.w = (const bf16_t*)w; p.ldw = ldw; p.out = out; p.ldo = N;
-  p.M = M; p.N = N; p.K = K; p.gelu = 0; p.pairs = 0; p.slab = (long long)M * N;
+  p.M = M; p.N = N; p.K = K; p.gelu = 0; p.alpha = 1.f; p.limit = p.shift = 0.f; p.pairs = 0; p.slab = (long long)M * N;
   const int bad = rows_check(p, x, w, out, cus);
   if (bad) return bad;
   const RowsCut c = rows_cut(N, K, cus);

@@ -11,9 +11,9 @@ import torch
 from . import skinny
 from .kernels import _check, _fn, _need, _ptr, _stream, compute_units
 
-__all__ = ["takes_rows", "prefers_rows", "rows_product", "rows_swiglu"]
+__all__ = ["takes_rows", "prefers_rows", "rows_product", "rows_swiglu", "many_outputs", "rows_gated"]
 
-_c_int, _c_ptr, _c_ll = ctypes.c_int, ctypes.c_void_p, ctypes.c_longlong
+_c_int, _c_ptr, _c_ll, _c_float = ctypes.c_int, ctypes.c_void_p, ctypes.c_longlong, ctypes.c_float
 _REACH = 0xffffff00
 MOST_ROWS = 64
 
@@ -31,16 +31,21 @@ def takes_rows(x: torch.Tensor, weight: torch.Tensor) -> bool:
             and ((x.shape[0] - 1) * x.stride(0) + x.shape[1]) * 2 < _REACH)
 
 
+def many_outputs(weight: torch.Tensor) -> bool:
+    """At least 8 for each of a device's waves, eight a compute unit (10,240 x 8,192 at 19 rows 60 us, the library, which
+    cuts the inner size, 41)."""
+    return weight.shape[0] >= 64 * compute_units(weight.device)
+
+
 def wide(m: int, weight: torch.Tensor) -> bool:
-    """Whether a weight has the outputs that make the kernel the fastest way to ``m`` rows: at least 8 for each of a device's
-    waves (eight a compute unit; 10,240 x 8,192 at 19 rows 60 us, the library, which cuts the inner size, 41), and more
-    rows than the resident kernel carries in one column tile, or an inner size too long for it to keep them.  Against
+    """Whether the kernel is the fastest way to ``m`` rows: many outputs, and more rows than the resident kernel carries in
+    one column tile, or an inner size too long for it to keep them.  Against
     the resident kernel at 32 rows: 22,016 x 2,048 gated 22 us for 27, with the norm in front 27 for 32; 37,888 x 3,584 45
     for 54, 50 for 65; 152,064 x 3,584 186 for 200; with 8 rows, 3B and 7B sizes, the two lie within 3 us and the resident
     kernel forms the norm by itself.  Against the library at 64 rows: 37,888 x 3,584 gated 49 us for 69 with the
     activation's kernel, 59,136 x 8,192 151 for 199; heads of 152,064 x 3,584 194 for 219, x 8,192 438 for 500."""
-    n, k = weight.shape
-    return (m <= MOST_ROWS and n >= 64 * compute_units(weight.device)
+    k = weight.shape[1]
+    return (m <= MOST_ROWS and many_outputs(weight)
             and (m > skinny.ONE_TILE_ROWS or not skinny.takes_resident(m, k, weight)))
 
 
@@ -48,10 +53,11 @@ def prefers_rows(x: torch.Tensor, weight: torch.Tensor) -> bool:
     return takes_rows(x, weight) and wide(x.shape[0], weight)
 
 
-def _launch(x, weight, out, mode, gelu=0):
-    fn = _fn("gemm_rows", "qvl_gemm_rows", [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ll] + [_c_int] * 6 + [_c_ptr])
+def _launch(x, weight, out, mode, gelu=0, alpha=1.0, limit=0.0, shift=0.0):
+    fn = _fn("gemm_rows", "qvl_gemm_rows", [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ll] + [_c_int] * 5
+             + [_c_float] * 3 + [_c_int, _c_ptr])
     _check(fn(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(out), out.stride(0), x.shape[0], weight.shape[0],
-              x.shape[1], mode, gelu, compute_units(x.device), _stream()), "linear (few rows)")
+              x.shape[1], mode, gelu, alpha, limit, shift, compute_units(x.device), _stream()), "linear (few rows)")
     return out
 
 
@@ -73,3 +79,11 @@ def rows_swiglu(x: torch.Tensor, weight: torch.Tensor, act: str = "silu") -> tor
     _need(act in ("silu", "gelu_tanh"), "the activation is silu or gelu_tanh")
     out = torch.empty((x.shape[0], weight.shape[0] // 2), dtype=torch.bfloat16, device=x.device)
     return _launch(x, weight, out, 2, int(act == "gelu_tanh"))
+
+
+def rows_gated(x: torch.Tensor, weight: torch.Tensor, alpha: float, limit: Optional[float], shift: float) -> torch.Tensor:
+    """``g sigmoid(alpha g) (u + shift)`` for a weight of gate rows, then up rows: ``g`` capped at ``limit``, ``u`` clamped to
+    ``[-limit, limit]`` (None: neither); bfloat16 ``[M, N / 2]``."""
+    _need(takes_rows(x, weight) and weight.shape[0] % 2 == 0, "the kernel does not take this product")
+    out = torch.empty((x.shape[0], weight.shape[0] // 2), dtype=torch.bfloat16, device=x.device)
+    return _launch(x, weight, out, 3, alpha=float(alpha), limit=float(limit or 0.0), shift=float(shift))

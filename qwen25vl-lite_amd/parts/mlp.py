@@ -114,10 +114,14 @@ class ClampedGatedFF(FeedForward):
                 f"{self.names['down']}.weight": self.w_down}
 
     def forward(self, x, step: StepContext):
-        from ..ops import tile
+        from ..ops import rows, tile
         from ..ops.gated import gated_act
         from ..ops.linear import linear
 
+        # (37,888 x 3,584, 8 rows: 44 us; the resident kernel's product 45 and the activation's kernel 5)
+        if x.is_cuda and self.w_gate_up.is_cuda and rows.takes_rows(x, self.w_gate_up) and rows.many_outputs(self.w_gate_up):
+            act = rows.rows_gated(x, self.w_gate_up, self.alpha, self.limit, self.shift)
+            return linear_into(step.residual if step is not None else None, act, self.w_down)
         if x.is_cuda and tile.prefers_tile(x, self.w_gate_up, halves=True):
             act = tile.tile_gated(x, self.w_gate_up, self.alpha, self.limit, self.shift)
             return linear_into(step.residual if step is not None else None, act, self.w_down)

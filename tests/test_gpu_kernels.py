@@ -664,6 +664,12 @@ def test_rows_against_many_outputs(m, n, k):
         b = bound.view(m, n // 16, 2, 8)
         slack = (1.13 * b[:, :, 0] * (pairs[:, :, 1].abs() + b[:, :, 1]) + fn(pairs[:, :, 0]).abs() * b[:, :, 1]).reshape(m, n // 2)
         assert bool(((got - ref).abs() <= slack + (2.0 ** -8 + 1e-5) * ref.abs() + 1e-5 * pairs[:, :, 1].abs().reshape(m, n // 2)).all())
+    # all gate rows, then the up rows; with clamps the values are at most 1.5 and 2.5, the slopes 1.13 and 1
+    got = rows.rows_gated(x, w, 1.25, 1.5, 1.0).double()
+    g, u = want[:, :n // 2].clamp(max=1.5), want[:, n // 2:].clamp(-1.5, 1.5)
+    ref = g * torch.sigmoid(1.25 * g) * (u + 1.0)
+    slack = 1.13 * 2.5 * bound[:, :n // 2] + 1.5 * bound[:, n // 2:]
+    assert bool(((got - ref).abs() <= slack + (2.0 ** -8 + 1e-6) * ref.abs() + 2e-6).all())
 
 
 @pytest.mark.parametrize("e, r, k, pairs", [(3, 40, 72, "one"), (8, 300, 200, "uneven"), (70, 129, 64, "uneven"), (4, 2368, 136, "all on one"),
