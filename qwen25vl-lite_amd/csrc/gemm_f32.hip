@@ -13,8 +13,10 @@
 // Both operands come through LDS with loads that put their 16 bytes there directly, several steps of K
 // ahead; a row's 16-byte chunks are exchanged by bits of the row's number, so that the 16 rows that one
 // operand read touches lie in different banks.  Measured at the 3B decoder's sizes, two layers and the head,
-// one step of 164 rows and three of 6 or 7: their products take 3.39 ms instead of the plain kernel's 21.0 ms.
+// one step of 164 rows and three of 6 or 7: their products take 3.18 ms instead of the plain kernel's 21.0 ms.
 #include "common.h"
+
+#include <type_traits>
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -117,7 +119,8 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_mfma_kernel(const float
   static_assert(ROWS_W % ROWS_LOAD == 0 && ROWS_A % ROWS_LOAD == 0, "a fetch lies in one operand");
   static_assert((STAGES - 2) * LOADS < 64, "the counter's range");
   __shared__ __attribute__((aligned(16))) float stage[STAGES][(ROWS_W + ROWS_A) * KT];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
+  const int wave = NWAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
   const int wn = wave % WN, wm = wave / WN;
   const int n0 = blockIdx.x * ROWS_W, m0 = blockIdx.y * ROWS_A;
   const float* wbase = W + (size_t)n0 * ldw;
@@ -161,35 +164,83 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_mfma_kernel(const float
 #pragma unroll
   for (int i = 0; i < STAGES - 1; ++i)
     if (i < steps) issue(i);
-  for (int s = 0; s < steps; ++s) {
-    const int ahead = steps - 1 - s < STAGES - 2 ? steps - 1 - s : STAGES - 2;
-    wait_steps<STAGES - 2, LOADS>(ahead);
-    __syncthreads();                       // every wave's part of step s is there, and step s - 1 has been multiplied
-    if (s + STAGES - 1 < steps) issue(s + STAGES - 1);
-    const float* sw = stage[s % STAGES];
-    const float* sa = sw + ROWS_W * KT;
-    auto multiply = [&](int c) {           // chunk c: four values of K, lane group g has the g-th
-      float fw[TNW], fa[TMW];
+  // With one tile a wave, a step's operands are read from LDS while those of the step before are multiplied: the chain of
+  // products of one sum is all there is to hide the reads behind (8 x 2,048 x 11,008: 140 -> 118 us; 64 rows 169 -> 153).  Four waves
+  // side by side on many outputs hide it behind each other (22,016 x 2,048: 43.8, so 44.6).
+  if constexpr (TNW == 1 && TMW == 1 && WN < 4) {
+    float fw[2][CH], fa[2][CH];
+    auto read = [&](int s, auto buf) __attribute__((always_inline)) {
+      constexpr int B = decltype(buf)::value;
+      const float* sw = stage[s % STAGES];
+      const float* sa = sw + ROWS_W * KT;
 #pragma unroll
-      for (int n = 0; n < TNW; ++n) {
-        const int row = (wn * TNW + n) * 16 + r;
-        fw[n] = sw[row * KT + 4 * (c ^ (row & (CH - 1))) + g];
+      for (int c = 0; c < CH; ++c) {
+        const int row = wn * 16 + r;
+        fw[B][c] = sw[row * KT + 4 * (c ^ (row & (CH - 1))) + g];
+        const int ra = wm * 16 + r;
+        fa[B][c] = sa[ra * KT + 4 * (c ^ ((ROWS_W + ra) & (CH - 1))) + g];
       }
-#pragma unroll
-      for (int m = 0; m < TMW; ++m) {
-        const int row = (wm * TMW + m) * 16 + r;
-        fa[m] = sa[row * KT + 4 * (c ^ ((ROWS_W + row) & (CH - 1))) + g];
-      }
-#pragma unroll
-      for (int n = 0; n < TNW; ++n)
-#pragma unroll
-        for (int m = 0; m < TMW; ++m) acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[n], fa[m], acc[n][m], 0, 0, 0);
     };
-    if (s + 1 < steps || K % KT == 0) {
+    auto multiply = [&](int s, auto buf) __attribute__((always_inline)) {
+      constexpr int B = decltype(buf)::value;
+      const int chunks = s + 1 < steps || K % KT == 0 ? CH : (K % KT) / 4;
+      if (chunks == CH) {
 #pragma unroll
-      for (int c = 0; c < CH; ++c) multiply(c);
-    } else {
-      for (int c = 0; c < (K % KT) / 4; ++c) multiply(c);
+        for (int c = 0; c < CH; ++c) acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[B][c], fa[B][c], acc[0][0], 0, 0, 0);
+      } else {
+#pragma unroll
+        for (int c = 0; c < CH; ++c)       // (unrolled, a branch each: an index at run time would move the operands about)
+          if (c < chunks) acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[B][c], fa[B][c], acc[0][0], 0, 0, 0);
+      }
+    };
+    auto step = [&](int s, auto here, auto before) __attribute__((always_inline)) {
+      if (s < steps) {
+        const int ahead = steps - 1 - s < STAGES - 2 ? steps - 1 - s : STAGES - 2;
+        wait_steps<STAGES - 2, LOADS>(ahead);
+        __syncthreads();                     // every wave's part of step s is there, and step s - 1 has been read
+        if (s + STAGES - 1 < steps) issue(s + STAGES - 1);
+        read(s, here);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (s > 0) multiply(s - 1, before);
+    };
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    for (int s = 0; s <= steps; s += 2) {
+      step(s, even, odd);
+      if (s < steps) step(s + 1, odd, even);
+    }
+  } else {
+    for (int s = 0; s < steps; ++s) {
+      const int ahead = steps - 1 - s < STAGES - 2 ? steps - 1 - s : STAGES - 2;
+      wait_steps<STAGES - 2, LOADS>(ahead);
+      __syncthreads();                       // every wave's part of step s is there, and step s - 1 has been multiplied
+      if (s + STAGES - 1 < steps) issue(s + STAGES - 1);
+      const float* sw = stage[s % STAGES];
+      const float* sa = sw + ROWS_W * KT;
+      auto multiply = [&](int c) {           // chunk c: four values of K, lane group g has the g-th
+        float fw[TNW], fa[TMW];
+#pragma unroll
+        for (int n = 0; n < TNW; ++n) {
+          const int row = (wn * TNW + n) * 16 + r;
+          fw[n] = sw[row * KT + 4 * (c ^ (row & (CH - 1))) + g];
+        }
+#pragma unroll
+        for (int m = 0; m < TMW; ++m) {
+          const int row = (wm * TMW + m) * 16 + r;
+          fa[m] = sa[row * KT + 4 * (c ^ ((ROWS_W + row) & (CH - 1))) + g];
+        }
+#pragma unroll
+        for (int n = 0; n < TNW; ++n)
+#pragma unroll
+          for (int m = 0; m < TMW; ++m) acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[n], fa[m], acc[n][m], 0, 0, 0);
+      };
+      if (s + 1 < steps || K % KT == 0) {
+#pragma unroll
+        for (int c = 0; c < CH; ++c) multiply(c);
+      } else {
+        for (int c = 0; c < (K % KT) / 4; ++c) multiply(c);
+      }
     }
   }
   // a lane holds, of (n, m): row 16 (wm TMW + m) + r of A, outputs 16 (wn TNW + n) + 4 g ...
