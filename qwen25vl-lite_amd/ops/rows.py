@@ -38,17 +38,18 @@ def many_outputs(weight: torch.Tensor) -> bool:
 
 
 def wide(m: int, weight: torch.Tensor) -> bool:
-    """Whether the kernel is the fastest way to ``m`` rows: many outputs, and more rows than the resident kernel carries in
-    one column tile, or an inner size too long for it to keep them, or more than 8 rows of the wider build's inner sizes, whose norm
-    takes it longer than a kernel of its own.  Against
+    """Whether the kernel is the fastest way to ``m`` rows: many outputs, and an inner size beyond the resident kernel's
+    narrow build (a norm formed in each of its blocks takes longer than a kernel of its own), or more rows than that
+    carries in one column tile.  Against
     the resident kernel at 32 rows: 22,016 x 2,048 gated 22 us for 27, with the norm in front 27 for 32; 37,888 x 3,584 45
     for 54, 50 for 65; 152,064 x 3,584 186 for 200; with 9 rows and the norm
-    37,888 x 3,584 49.7 us for 52.5, with 16 50.1 for 55.6 (22,016 x 2,048 26.3 for 25.5); with 8 rows the two lie within 3 us
-    and the resident kernel needs a launch less.  Against the library at 64 rows: 37,888 x 3,584 gated 49 us for 69 with the
+    37,888 x 3,584 49.7 us for 52.5, with 16 50.1 for 55.6 (22,016 x 2,048 26.3 for 25.5); a pass of 8 decode steps, 7B sizes, 8
+    layers, 1 row 8,291 us for 8,347, 4 rows 8,498 for 8,727, 8 rows 8,757 for 9,006, 16 rows 9,150 for 9,651; 3B sizes, 16
+    rows, 5,730 for 5,723.  Against the library at 64 rows: 37,888 x 3,584 gated 49 us for 69 with the
     activation's kernel, 59,136 x 8,192 151 for 199; heads of 152,064 x 3,584 194 for 219, x 8,192 438 for 500."""
     k = weight.shape[1]
     return (m <= MOST_ROWS and many_outputs(weight)
-            and (m > (8 if k > skinny.NARROW_K else skinny.ONE_TILE_ROWS) or not skinny.takes_resident(m, k, weight)))
+            and (k > skinny.NARROW_K or m > skinny.ONE_TILE_ROWS or not skinny.takes_resident(m, k, weight)))
 
 
 def prefers_rows(x: torch.Tensor, weight: torch.Tensor) -> bool:
