@@ -189,10 +189,10 @@ extern "C" int qvl_add_rmsnorm(void* h, const void* delta, const void* w, void* 
                                float eps, int delta_dtype, int out_dtype, int nslabs, long long slab_stride,
                                hipStream_t stream) {
   if (M <= 0) return QVL_OK;
-  if (H <= 0 || nslabs < 1 || (nslabs > 1 && (slab_stride < H || slab_stride % 4))) return QVL_ERR_SHAPE;
+  if (H <= 0 || nslabs < 1 || (nslabs > 1 && slab_stride < H)) return QVL_ERR_SHAPE;
   const int threads = H >= 2048 ? 512 : 256;
   const bool vec = H % 4 == 0 && H <= NORM_VEC_MAX * 4 * 256 && nslabs == 1;
-  if (nslabs > 1 && delta && delta_dtype == 0 && H % 4 == 0 && H <= SLAB_VEC_MAX * 4096) {
+  if (nslabs > 1 && delta && delta_dtype == 0 && H % 4 == 0 && slab_stride % 4 == 0 && H <= SLAB_VEC_MAX * 4096) {
     if (out_dtype == 0)
       hipLaunchKernelGGL((add_rmsnorm_slabs_kernel<float>), dim3(M), dim3(1024), 0, stream, (float*)h, (const float*)delta,
                          (const float*)w, (float*)out, (const int*)rows, H, eps, nslabs, slab_stride);

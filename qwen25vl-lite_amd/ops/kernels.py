@@ -125,8 +125,8 @@ def add_rmsnorm(h: torch.Tensor, delta: Optional[torch.Tensor], weight: torch.Te
           "norm weight must be float32 [H]")
     nslabs, slab_stride = 1, 0
     if delta is not None and delta.dim() == 3:
-        _need(delta.dtype == torch.float32 and tuple(delta.shape[1:]) == tuple(h.shape) and delta.is_contiguous()
-              and width % 4 == 0, "slabs of delta must be contiguous float32 [slabs, N, H] with H in steps of 4")
+        _need(delta.dtype == torch.float32 and tuple(delta.shape[1:]) == tuple(h.shape) and delta.is_contiguous(),
+              "slabs of delta must be contiguous float32 [slabs, N, H]")
         nslabs, slab_stride = delta.shape[0], n * width
     elif delta is not None:
         _need(delta.shape == h.shape and delta.is_contiguous(), "delta must match h's shape")

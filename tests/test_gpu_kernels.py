@@ -849,6 +849,32 @@ def test_tiled_product_in_ranges(m, n, k):
     assert torch.allclose(normed, ref, atol=1e-4, rtol=1e-4)
 
 
+@pytest.mark.parametrize("m, n, k", [(20, 50, 512), (33, 51, 1032), (64, 1, 2056), (100, 50, 512), (100, 49, 1024), (300, 37, 2080)])
+def test_products_of_any_width_join_the_residual_sum(m, n, k):
+    """Widths off steps of 4: what linear_into hands on, as slabs too, is taken by the norm behind it, whole and for chosen
+    rows.  Each sum of k products and the addition into the residual is within k + 1 roundings of its terms."""
+    from qwen25vl_lite_amd.ops import kernels
+    from qwen25vl_lite_amd.ops.linear import linear_into
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(n, k, device="cuda", generator=g) / k ** 0.5).bfloat16()
+    h = torch.randn(m, n, device="cuda", generator=g)
+    gain = torch.rand(n, device="cuda", generator=g) + 0.5
+    total = h.double() + x.double() @ w.double().T
+    slack = (k + 1) * 2.0 ** -24 * (h.double().abs() + x.double().abs() @ w.double().abs().T)
+    left = linear_into(None, x, w)
+    if left.dtype == torch.bfloat16:              # uncut: one rounding of the product
+        slack = slack + 2.0 ** -8 * (total - h.double()).abs()
+    ref = total * torch.rsqrt(total.pow(2).mean(-1, keepdim=True) + 1e-6) * gain
+    rows = torch.tensor([m - 1, 0], dtype=torch.int32, device="cuda")
+    picked = kernels.add_rmsnorm(h, left, gain, 1e-6, torch.float32, rows=rows)
+    normed = kernels.add_rmsnorm(h, left, gain, 1e-6, torch.float32)
+    assert bool(((h.double() - total).abs() <= slack).all())
+    # (a row's scale follows its sums: no term of it is off by more than the largest relative error of a row of one value)
+    assert torch.allclose(normed.double(), ref, atol=2e-2 if left.dtype == torch.bfloat16 else 1e-3, rtol=1e-2)
+    assert torch.equal(picked, normed[rows.long()])
+
+
 def test_tiled_product_leaves_what_it_does_not_take():
     """Inner sizes off a step of 32, rows off 16 bytes, few rows: not taken, and the general entry still answers."""
     from qwen25vl_lite_amd.ops import tile
