@@ -274,7 +274,8 @@ __device__ void search_state(RowScratch& r, const RowParams& p, int level, bool 
         if (threadIdx.x < o) s_sum[threadIdx.x] += s_sum[threadIdx.x + o];
         __syncthreads();
       }
-      target = (unsigned long long)ceil((double)p.top_p * (double)s_sum[0]);
+      // (a top_p below float32's range is 0 here: the largest score stays)
+      target = max(1ull, (unsigned long long)ceil((double)p.top_p * (double)s_sum[0]));
       __syncthreads();
     } else {
       target = (unsigned long long)p.top_k;

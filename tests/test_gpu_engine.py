@@ -520,6 +520,23 @@ def test_sampler_cuts_at_the_edges_of_its_pieces(vocab):
                 assert min(abs(cdf[got[i]] - us[i]), abs(cdf[got[i]] - share - us[i])) < 1e-5, (trial, i)
 
 
+@pytest.mark.parametrize("top_p", [1e-50, 1e-30, 1e-7])
+def test_sampler_keeps_the_most_likely_token_at_any_top_p(top_p):
+    """A top_p that float32 rounds to zero, one whose share of the mass is less than a unit of it, a small one: the token that
+    crosses it stays, and it is the most likely one, whatever is drawn."""
+    from qwen25vl_lite_amd.sampling import SamplingParams
+    from qwen25vl_lite_amd.sampling.sampler import sample_rows
+
+    g = torch.Generator().manual_seed(1)
+    logits = torch.randn(6, 5003, generator=g)
+    kinds = [dict(), dict(top_k=40), dict(min_p=0.01), dict(repetition_penalty=1.2), dict(temperature=0.3), dict(temperature=5.0)]
+    params = [SamplingParams(**{"temperature": 1.0, "top_p": top_p, **k}) for k in kinds]
+    for p in params:
+        p.validate()
+    for u in (0.0, 0.5, 0.999):
+        assert sample_rows(logits.cuda(), params, [[]] * 6, [0] * 6, uniforms=[u] * 6) == logits.argmax(-1).tolist()
+
+
 def test_trace_run_program(model_dirs, tmp_path):
     """bin/trace_run as a user calls it: JSON steps on standard input, `done <step>` lines,
     <step>.f32 files of little-endian float32 [wanted, vocab]."""
