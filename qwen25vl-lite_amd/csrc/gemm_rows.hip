@@ -130,26 +130,25 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) void gemm_rows_kernel(RowsArgs p) 
   // rows of a tile beyond its 8 F are not fetched: their operand is another row's, their sums are not stored
   const int wr = r < 8 * F ? r : r - 8 * F;
   const uint32_t wsw = (wr >> 1) & 7;
-  tp_f32x16 acc[MT];
-  auto clear = [&] {
-#pragma unroll
-    for (int t = 0; t < MT; ++t)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[t][i] = 0.f;
-  };
+  // A sum is formed of short runs: the products of a step go to CHAINS sums in turn, and these join the rest every eight steps.
+  // What an addition rounds off then stays small: 64 rows x 152,064 x 3,584, error against 64 bits 1.0e-7 of the result, in one chain of
+  // 224 products 3.7e-7 (the library's product likewise), for 204 and 205 us.  Joined every two or four steps, the waits for the products show:
+  // 37,888 x 3,584 gated, 64 rows, 54 us for 52.
+  constexpr int CHAINS = MT == 1 ? 4 : 2;
+  tp_f32x16 run[CHAINS][MT], acc[MT];
   auto finish = [&](int round) __attribute__((always_inline)) {
     const int tile = tile_of(round);
     if (tile >= p.tiles) return;
     if constexpr (X_FIRST) {
       const int n = tile * p.per + r;
-      float* out = reinterpret_cast<float*>(p.out) + range * p.slab + n;
       if (r >= p.per || n >= p.N) return;
+      float* out = reinterpret_cast<float*>(p.out) + range * p.slab + n + 4 * hi * p.ldo;
 #pragma unroll
       for (int t = 0; t < MT; ++t)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const int m = 32 * t + 8 * (i >> 2) + 4 * hi + (i & 3);
-          if (m < p.M) out[(size_t)m * p.ldo] = acc[t][i];
+          if (32 * t + 8 * (i >> 2) + 4 * hi + (i & 3) < p.M) *out = acc[t][i];
+          out += (i & 3) == 3 ? 5 * p.ldo : p.ldo;
         }
     } else {
 #pragma unroll
@@ -211,14 +210,26 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) void gemm_rows_kernel(RowsArgs p) 
 #pragma unroll
     for (int k = 0; k < 4; ++k)
 #pragma unroll
-      for (int t = 0; t < MT; ++t)
-        acc[t] = X_FIRST ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(x8[B][t][k], w8[B][k], acc[t], 0, 0, 0)
-                         : __builtin_amdgcn_mfma_f32_32x32x16_bf16(w8[B][k], x8[B][t][k], acc[t], 0, 0, 0);
+      for (int t = 0; t < MT; ++t) {
+        tp_f32x16& c = run[k % CHAINS][t];
+        c = X_FIRST ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(x8[B][t][k], w8[B][k], c, 0, 0, 0)
+                    : __builtin_amdgcn_mfma_f32_32x32x16_bf16(w8[B][k], x8[B][t][k], c, 0, 0, 0);
+      }
     if (++mul_k == ksteps) mul_k = 0;
-    if (--mul_left == 0) {
-      finish(mul_round++);
-      clear();
-      mul_left = ksteps;
+    if ((--mul_left & 7) == 0) {
+      __builtin_amdgcn_sched_barrier(0);      // (a branch: the additions wait for the products, and are not for every step)
+#pragma unroll
+      for (int t = 0; t < MT; ++t) {
+        acc[t] += CHAINS == 4 ? (run[0][t] + run[1][t]) + (run[CHAINS - 2][t] + run[CHAINS - 1][t]) : run[0][t] + run[1][t];
+#pragma unroll
+        for (int c = 0; c < CHAINS; ++c) run[c][t] = tp_f32x16{};
+      }
+      if (mul_left == 0) {
+        finish(mul_round++);
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[t] = tp_f32x16{};
+        mul_left = ksteps;
+      }
     }
   };
   auto step = [&](int s, auto here, auto before) __attribute__((always_inline)) {
@@ -232,7 +243,12 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) void gemm_rows_kernel(RowsArgs p) 
     }
     if (s > 0) multiply(before);
   };
-  clear();
+#pragma unroll
+  for (int t = 0; t < MT; ++t) {
+    acc[t] = tp_f32x16{};
+#pragma unroll
+    for (int c = 0; c < CHAINS; ++c) run[c][t] = tp_f32x16{};
+  }
   constexpr std::integral_constant<int, 0> even{};
   constexpr std::integral_constant<int, 1> odd{};
   for (int s = 0; s <= steps; s += 2) {

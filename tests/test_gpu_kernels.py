@@ -633,6 +633,29 @@ def test_few_row_products_read_nothing_beside_the_inner_size(m, k):
              2.0 ** -8)
 
 
+def _off(got, x, w):
+    """Error of a product against 64 bits, 2-norm over 2-norm."""
+    want = x.double() @ w.double().T
+    return float((got.double() - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("m", [1, 16, 19, 40, 64])
+@pytest.mark.parametrize("k", [1024, 3584, 8192])
+def test_float32_sums_of_the_streaming_kernel(m, k):
+    """A chain of additions is off by a random walk: each rounds off up to half a unit of 24 bits (2^-24 / sqrt(3) on
+    average) of a sum that grows evenly, sqrt(n / 2) of them in the end.  Sums are formed of chains of 16 at most, two levels of
+    joins and a join for every 512 values: no more than sqrt(8 + 2 + k / 1024) of them."""
+    from qwen25vl_lite_amd.ops import rows, skinny
+    torch.manual_seed(m + k)
+    x = torch.randn(m, k, device="cuda").bfloat16()
+    w = (torch.randn(2048, k, device="cuda") / math.sqrt(k)).bfloat16()
+    bound = 2.0 ** -24 / math.sqrt(3.0) * math.sqrt(10 + k / 1024)
+    assert _off(rows.rows_product(x, w, torch.float32), x, w) < bound
+    if m > skinny.KEPT_SPLIT_ROWS:
+        slabs = skinny.split_product(w, x)
+        assert _off(slabs.double().sum(0), x, w) < bound
+
+
 @pytest.mark.parametrize("m", [1, 19, 32, 33, 64])
 @pytest.mark.parametrize("n, k", [(16, 8), (16400, 136), (37888, 72), (59136, 64), (81920, 200), (152064, 136), (36912, 2056)])
 def test_rows_against_many_outputs(m, n, k):
