@@ -639,6 +639,21 @@ def _off(got, x, w):
     return float((got.double() - want).norm() / want.norm())
 
 
+@pytest.mark.parametrize("m", [1, 8, 16, 24])
+@pytest.mark.parametrize("k", [896, 1024, 1536, 2048, 3584, 4096])
+def test_float32_sums_of_the_resident_kernel(m, k):
+    """As below: chains of at most 8 products of 32 values, which the instruction adds in two halves, a join of the two halves of
+    a wave's columns and one sum for each of up to 8 waves: sqrt(8 + 1 / 2 + 4) of 2^-24 / sqrt(3) at most."""
+    from qwen25vl_lite_amd.ops import skinny
+    torch.manual_seed(m + k)
+    x = torch.randn(m, k, device="cuda").bfloat16()
+    w = (torch.randn(2048, k, device="cuda") / math.sqrt(k)).bfloat16()
+    bound = 2.0 ** -24 / math.sqrt(3.0) * math.sqrt(12.5)
+    assert _off(skinny.resident_product(w, x=x), x, w) < bound
+    if m <= skinny.KEPT_SPLIT_ROWS:
+        assert _off(skinny.split_product(w, x).double().sum(0), x, w) < bound
+
+
 @pytest.mark.parametrize("m", [1, 16, 19, 40, 64])
 @pytest.mark.parametrize("k", [1024, 3584, 8192])
 def test_float32_sums_of_the_streaming_kernel(m, k):
