@@ -215,7 +215,7 @@ def qkv_rope_product(weight: torch.Tensor, cs: torch.Tensor, *, x: Optional[torc
 
 
 SPLIT_ROWS = 64   # the most rows that are cut along the inner size
-SPLIT_K = 2048 * 256   # the longest inner size
+SPLIT_K = 2048    # the longest inner size, for each compute unit: with more of it a block of the few rows' kernel could not keep its range
 # Up to here a block keeps its range of the rows and walks several tiles (csrc/gemm_resident.hip: few ranges; 2,048 x 11,008, one
 # row, with the norm that adds the slabs: a decode step of the 3B decoder 4.24 ms, cut by csrc/gemm_rows.hip 4.31), with more
 # rows csrc/gemm_rows.hip cuts (3,584 x 18,944: 8 rows 25.4 us for 26.9, 16 rows 25.4 for 28.3, 64 rows 28.3 for 36.7)
@@ -231,7 +231,8 @@ def _ranges(m: int, n: int, k: int, cus: int) -> int:
 def takes_split(m: int, k: int, weight: torch.Tensor) -> bool:
     """Whether a product of ``m`` rows with this weight is taken in ranges of the inner size: up to
     64 bfloat16 rows, whose partial sums come back as slabs."""
-    if not (1 <= m <= SPLIT_ROWS and k % 8 == 0 and k <= SPLIT_K and weight.dtype == torch.bfloat16 and _rows_aligned(weight, 8)):
+    if not (1 <= m <= SPLIT_ROWS and k % 8 == 0 and weight.dtype == torch.bfloat16 and _rows_aligned(weight, 8)
+            and k <= SPLIT_K * _compute_units(weight.device)):
         return False
     return ((weight.shape[0] - 1) * weight.stride(0) + k) * 2 < _MAX_WEIGHT_BYTES
 
