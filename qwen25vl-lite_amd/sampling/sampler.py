@@ -46,6 +46,17 @@ def _seed_words(seeds: np.ndarray, steps: np.ndarray) -> np.ndarray:
     return (seeds.astype(np.uint64) + steps.astype(np.uint64)).astype(np.uint32)
 
 
+def _int32_ids(flat: Sequence) -> np.ndarray:
+    """Token ids as int32 ``[L]`` (one zero for none)."""
+    try:
+        ids = np.asarray(flat or [0], np.int32)
+        if ids.ndim == 1:
+            return ids
+    except (TypeError, ValueError):
+        pass
+    return np.asarray([int(t) for t in flat], np.int32)   # other types than Python's and numpy's, or arrays of one id each
+
+
 class _Staging:
     """Pinned host buffers that take turns carrying the sampler's per-row settings to the device:
     a copy from pinned memory does not make the host wait for the work queued before it."""
@@ -202,11 +213,7 @@ def _launch(logits: torch.Tensor, rows: np.ndarray, flat: List[int]) -> PendingS
     dev = logits.device
     draws = rows["temperature"] > 0
     with torch.cuda.device(dev):
-        try:
-            ids = np.asarray(flat or [0], np.int32)
-        except (TypeError, ValueError):          # ids of other types than Python's and numpy's
-            ids = np.asarray([int(t) for t in flat], np.int32)
-        packed = np.concatenate([rows.view(np.int32), ids])
+        packed = np.concatenate([rows.view(np.int32), _int32_ids(flat)])
         buf = _Staging.to_device(packed, dev)
         n_row_words = rows.view(np.int32).size
         some = bool(draws.any())

@@ -1,4 +1,4 @@
-"""Rules that choose a kernel by sizes: what can be checked without a GPU."""
+"""Rules that choose a kernel by sizes, and what the sampler is handed: what can be checked without a GPU."""
 
 import numpy as np
 import pytest
@@ -18,3 +18,17 @@ def test_products_are_cut_where_the_kernel_takes_the_cut(cus, rows, monkeypatch)
             taken += 1
             assert skinny._ranges(rows, 3, k, cus) > 0, k
     assert taken >= 5
+
+
+def test_sampler_takes_token_ids_of_any_kind():
+    """Lists of Python's and numpy's integers, 0-d tensors, arrays and tensors of one id each; what is no id is refused."""
+    from qwen25vl_lite_amd.sampling.sampler import _int32_ids
+    for flat in ([3, 4], [np.int64(3), np.uint8(4)], list(torch.tensor([3, 4])), list(torch.tensor([[3], [4]])),
+                 list(np.array([[3], [4]], np.int64)), ["3", 4]):
+        got = _int32_ids(flat)
+        assert got.dtype == np.int32 and got.tolist() == [3, 4], flat
+    assert _int32_ids([]).tolist() == [0]
+    for flat, error in (([1 << 40], OverflowError), ([np.int64(1 << 40)], OverflowError), ([None], TypeError),
+                        (list(torch.tensor([[3, 4], [5, 6]])), (RuntimeError, TypeError, ValueError))):
+        with pytest.raises(error):
+            _int32_ids(flat)
