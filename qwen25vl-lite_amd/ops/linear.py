@@ -168,10 +168,11 @@ def gate_up_swiglu(x: Union[torch.Tensor, NormedRows], weight: torch.Tensor, gro
             return skinny.resident_product(weight, h=x.h, norm_weight=x.weight, eps=x.eps, epilogue=skinny.GATED[act])
         if not lazy and x.dtype == torch.bfloat16 and skinny.takes_resident(m, k, weight) and _aligned(x):
             return skinny.resident_product(weight, x=x, epilogue=skinny.GATED[act])
-    if isinstance(x, NormedRows):
-        x = x.materialize()
-    if grouped and weight.shape[0] % 16 == 0 and rows.prefers_rows(x, weight):
-        return rows.rows_swiglu(x, weight, act)
-    if grouped and weight.shape[0] % 16 == 0 and x.is_cuda and tile.prefers_tile(x, weight, gated=True):
-        return tile.tile_swiglu(x, weight, act)
+    if grouped and weight.shape[0] % 16 == 0:
+        if isinstance(x, NormedRows):
+            x = x.materialize()
+        if rows.prefers_rows(x, weight):
+            return rows.rows_swiglu(x, weight, act)
+        if x.is_cuda and tile.prefers_tile(x, weight, gated=True):
+            return tile.tile_swiglu(x, weight, act)
     return kernels.swiglu(linear(x, weight), grouped=grouped, act=act)

@@ -748,6 +748,32 @@ def test_experts_with_few_pairs(e, r, k, pairs):
         assert bool(((got - ref).abs() <= slack + (last + 1e-6) * ref.abs() + 2e-6).all())
 
 
+@pytest.mark.parametrize("m", [1, 16, 32])
+def test_rows_of_gate_and_up_that_form_no_groups_keep_the_norm_in_the_product(m, monkeypatch):
+    """An inner size of the feed-forward off steps of 8: the product forms the norm of a decode step's rows itself, without a
+    kernel in front of it.  The normed rows and the product are rounded to bfloat16, the activation's factors likewise."""
+    from qwen25vl_lite_amd.ops import linear as products
+    torch.manual_seed(m)
+    h = torch.randn(m, 512, device="cuda")
+    gain = torch.rand(512, device="cuda") + 0.5
+    w = (torch.randn(2 * 1003, 512, device="cuda") / math.sqrt(512)).bfloat16()
+    normed = products.NormedRows(h, gain, 1e-6, torch.bfloat16)
+    x = normed.materialize().double()
+
+    def apart(self):
+        raise AssertionError("the norm ran apart from the product")
+    monkeypatch.setattr(products.NormedRows, "materialize", apart)
+    got = products.gate_up_swiglu(normed, w, grouped=False).double()
+    both = x @ w.double().T
+    # each normed value may be the neighbouring bfloat16; float32 sums of 512 products; the product's rounding to bfloat16
+    off = (2.0 ** -8 + 512 * 2.0 ** -24) * (x.abs() @ w.double().abs().T) + 2.0 ** -8 * both.abs()
+    g, u = both[:, :1003], both[:, 1003:]
+    ref = torch.nn.functional.silu(g) * u
+    # (the activation's slope is below 1.13)
+    slack = 1.13 * off[:, :1003] * (u.abs() + off[:, 1003:]) + torch.nn.functional.silu(g).abs() * off[:, 1003:]
+    assert bool(((got - ref).abs() <= slack + 2.0 ** -8 * (ref.abs() + slack)).all())
+
+
 def test_no_cpu_path():
     from qwen25vl_lite_amd.ops import kernels
     from qwen25vl_lite_amd.ops.linear import linear
