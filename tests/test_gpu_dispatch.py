@@ -1,0 +1,139 @@
+"""Products on both sides of the row counts and inner sizes at which another kernel takes over: each entry against 64 bits."""
+
+import math
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+ROWS = [1, 8, 9, 16, 17, 32, 33, 48, 49, 64, 65, 100]
+INNER = [2040, 2048, 2056, 4104]
+
+
+def _operands(m, n, k):
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(n, k, device="cuda", generator=g) / math.sqrt(k)).bfloat16()
+    want = x.double() @ w.double().T
+    return x, w, want, k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)     # k roundings of a sum's terms
+
+
+@pytest.mark.parametrize("k", INNER)
+@pytest.mark.parametrize("n", [272, 16400])
+def test_products(n, k):
+    """Few outputs and many (64 for each compute unit), plain, with a bias, in float32, joined to a sum."""
+    from qwen25vl_lite_amd.ops import linear as products
+    bias = torch.randn(n, device="cuda")
+    for m in ROWS:
+        x, w, want, slack = _operands(m, n, k)
+        assert bool(((products.linear(x, w, out_dtype=torch.float32).double() - want).abs() <= slack).all()), m
+        assert bool(((products.linear(x, w).double() - want).abs() <= slack + 2.0 ** -8 * want.abs()).all()), m
+        got = products.linear(x, w, bias, out_dtype=torch.float32).double()
+        total = want + bias.double()
+        assert bool(((got - total).abs() <= slack + 2.0 ** -23 * (want.abs() + total.abs())).all()), m
+        for residual in (None, torch.randn(m, n, device="cuda")):
+            before = 0.0 if residual is None else residual.double()
+            left = products.linear_into(residual, x, w)
+            got = (before if left is None or residual is None else residual.double()) + (
+                0.0 if left is None else left.double().sum(0) if left.dim() == 3 else left.double())
+            if left is None:
+                got = residual.double()
+            last = 2.0 ** -8 if left is not None and left.dtype == torch.bfloat16 else 2.0 ** -23
+            assert bool(((got - (want + before)).abs() <= slack + last * (want.abs() + (want + before).abs())).all()), m
+
+
+@pytest.mark.parametrize("k", INNER)
+@pytest.mark.parametrize("n", [272, 16400])
+def test_gate_and_up(n, k):
+    """Grouped and plain rows of gate and up, plain rows of x and rows whose norm may be formed on the way."""
+    from qwen25vl_lite_amd.ops import linear as products
+    gain = torch.rand(k, device="cuda") + 0.5
+    for m in ROWS:
+        x, w, want, slack = _operands(m, n, k)
+        for grouped in (True, False):
+            both, off = ((t.view(m, n // 16, 2, 8).transpose(1, 2).reshape(m, 2, n // 2) if grouped else t.view(m, 2, n // 2))
+                         for t in (want, slack))
+            # a product may be rounded to bfloat16 before the activation (whose slope is below 1.13)
+            off = off + 2.0 ** -8 * (both.abs() + off)
+            g, u = both[:, 0], both[:, 1]
+            ref = torch.nn.functional.silu(g) * u
+            bound = 1.13 * off[:, 0] * (u.abs() + off[:, 1]) + torch.nn.functional.silu(g).abs() * off[:, 1]
+            got = products.gate_up_swiglu(x, w, grouped).double()
+            assert bool(((got - ref).abs() <= bound + 2.0 ** -8 * (ref.abs() + bound)).all()), (m, grouped)
+        h = torch.randn(m, k, device="cuda")
+        lazy = products.NormedRows(h, gain, 1e-6, torch.bfloat16)
+        x = lazy.materialize()
+        got, ref = (products.gate_up_swiglu(t, w, True).double() for t in (lazy, x))
+        # a normed value may be the neighbouring bfloat16, and so may a result
+        moved = 2.0 ** -8 * (x.double().abs() @ w.double().abs().T)
+        both, moved = ((t.view(m, n // 16, 2, 8).transpose(1, 2).reshape(m, 2, n // 2)) for t in (x.double() @ w.double().T, moved))
+        bound = 1.13 * moved[:, 0] * (both[:, 1].abs() + moved[:, 1]) + (both[:, 0].abs() + moved[:, 0]) * moved[:, 1]
+        assert bool(((got - ref).abs() <= bound + 2.0 ** -7 * ref.abs() + 1e-6).all()), m
+
+
+@pytest.mark.parametrize("k", INNER)
+def test_projection_with_rotation_and_cache(k):
+    """The stacked projection of an attention: in one kernel with the rotation, cut along its inner size with the rotation's
+    kernel adding the slabs, uncut.  Queries, keys and values against 64 bits, a token without a slot among them."""
+    from qwen25vl_lite_amd.ops import kernels
+    from qwen25vl_lite_amd.ops.linear import NormedRows
+    from qwen25vl_lite_amd.parts import PartSpec, build_part
+    nq, nkv, hd, ps = 4, 2, 32, 16
+    part = build_part("mixer", PartSpec("paged_attention", {
+        "hidden_size": k, "num_heads": nq, "num_kv_heads": nkv, "head_dim": hd, "qkv_bias": True,
+        "position": PartSpec("rope", {"theta": 1e4})}), torch.bfloat16, torch.device("cuda:0"))
+    torch.manual_seed(k)
+    specs = part.param_specs()
+    weights = {name: torch.randn(s.shape, device="cuda") / (math.sqrt(k) if len(s.shape) == 2 else 1.0) for name, s in specs.items()}
+    part.load({name: t.bfloat16() if t.dim() == 2 else t for name, t in weights.items()})
+    inv_freq, freq_row = part.position.rotary_tables(hd)
+    gain = torch.rand(k, device="cuda") + 0.5
+    for m in ROWS:
+        h = torch.randn(m, k, device="cuda")
+        lazy = NormedRows(h, gain, 1e-6, torch.bfloat16)
+        x = lazy.materialize()
+        pages = m // ps + 2
+        slots = torch.randperm(pages * ps, device="cuda")[:m].int()
+        if m > 2:
+            slots[1] = -1
+        group = SimpleNamespace(slot_mapping=slots, page_size=ps)
+        positions = torch.randint(0, 900, (1, m), dtype=torch.int32, device="cuda")
+        want = x.double() @ part.w_in.double().T + part.b_in.double()
+        off = (k + 1) * 2.0 ** -24 * (x.double().abs() @ part.w_in.double().abs().T + part.b_in.double().abs())
+        neighbour = 2.0 ** -8 * (x.double().abs() @ part.w_in.double().abs().T)   # norms formed in another order
+        cs = kernels.rope_table(positions, inv_freq, freq_row, m).double()
+        for rows in (x, lazy):
+            if rows is lazy and m > 32:
+                continue
+            kc = torch.zeros(pages, nkv, ps, hd, dtype=torch.bfloat16, device="cuda")
+            vc = torch.zeros(pages, nkv, hd, ps, dtype=torch.bfloat16, device="cuda")
+            slot = SimpleNamespace(k_cache=kc, v_cache=vc)
+            step = SimpleNamespace(positions=positions, per_pass={})
+            args = (rows, step, group, slot, True, inv_freq, freq_row)
+            q = part._project_few_rows(*args)
+            if q is None:
+                q = part._project(*args)
+
+            def turned(t, bound):
+                c, s = cs[:, None, :, 0], cs[:, None, :, 1]
+                a, b = t[..., :hd // 2], t[..., hd // 2:]
+                if bound:
+                    c, s = c.abs(), s.abs()
+                    return torch.cat([a * c + b * s, b * c + a * s], -1)
+                return torch.cat([a * c - b * s, b * c + a * s], -1)
+            slack = off + (neighbour if rows is lazy else 0.0)
+            heads, bound = (t.view(m, nq + 2 * nkv, hd) for t in (want, slack))
+            ref = torch.cat([turned(heads[:, :nq + nkv], False), heads[:, nq + nkv:]], 1)
+            bound = torch.cat([turned(bound[:, :nq + nkv] + 2.0 ** -22 * heads[:, :nq + nkv].abs(), True), bound[:, nq + nkv:]], 1)
+            bound = bound + 2.0 ** -8 * (ref.abs() + bound)
+            assert bool(((q.view(m, nq, hd).double() - ref[:, :nq]).abs() <= bound[:, :nq]).all()), (m, rows is lazy)
+            live = slots >= 0
+            page, at = slots[live].long() // ps, slots[live].long() % ps
+            keys, values = kc[page, :, at].double(), vc[page, :, :, at].double()
+            assert bool(((keys - ref[live][:, nq:nq + nkv]).abs() <= bound[live][:, nq:nq + nkv]).all()), (m, rows is lazy)
+            assert bool(((values - ref[live][:, nq + nkv:]).abs() <= bound[live][:, nq + nkv:]).all()), (m, rows is lazy)
+            untouched = torch.ones(pages, ps, dtype=torch.bool, device="cuda")
+            untouched[page, at] = False
+            assert bool((kc.transpose(1, 2)[untouched] == 0).all()) and bool((vc.permute(0, 3, 1, 2)[untouched] == 0).all())

@@ -142,6 +142,49 @@ def test_rope_kv_write_from_slabs():
                               out_dtype=torch.bfloat16)
 
 
+@pytest.mark.parametrize("n", [1, 40, 520])
+@pytest.mark.parametrize("count", [2, 9, 10, 17])
+def test_rope_kv_write_adds_any_number_of_slabs(count, n):
+    """One batch of slabs that are asked for together, several, the last one partly filled; tokens that share the device's blocks
+    and a block each; rotation of a part of the head, tokens without a slot: the bits of the slabs' sum taken in order."""
+    from qwen25vl_lite_amd.ops import kernels
+    torch.manual_seed(count + n)
+    nq, nkv, hd, ps, half, pages = 6, 2, 48, 16, 16, n // 16 + 2
+    cols = (nq + 2 * nkv) * hd
+    slabs = torch.randn(count, n, cols).cuda()
+    total = slabs[0]
+    for s in slabs[1:]:
+        total = total + s
+    bias = torch.randn(cols).cuda()
+    pos = torch.randint(0, 500, (1, n), dtype=torch.int32).cuda()
+    inv_freq = plain_inv_freq(2 * half, 10000.0).cuda()
+    freq_row = torch.zeros(half, dtype=torch.int32).cuda()
+    slots = torch.randperm(pages * ps)[:n].to(torch.int32)
+    slots[1::7] = -1
+    slots = slots.cuda()
+    cs = kernels.rope_table(pos, inv_freq, freq_row, n)
+    outs = []
+    for x in (slabs, total):
+        kc = torch.full((pages, nkv, ps, hd), 7.0, dtype=torch.bfloat16).cuda()
+        vc = torch.full((pages, nkv, hd, ps), 7.0, dtype=torch.bfloat16).cuda()
+        q = kernels.rope_kv_write(x, bias, pos, inv_freq, freq_row, slots, kc, vc, nq, nkv, hd, ps,
+                                  out_dtype=torch.bfloat16, cs=cs)
+        outs.append((q, kc, vc))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)
+    # what is not turned is the sum with the bias, rounded once
+    plain = (total + bias).bfloat16().view(n, nq + 2 * nkv, hd)
+    q, kc, vc = outs[0]
+    assert torch.equal(q.view(n, nq, hd)[..., 2 * half:], plain[:, :nq, 2 * half:])
+    live = slots >= 0
+    page, at = slots[live].long() // ps, slots[live].long() % ps
+    assert torch.equal(kc[page, :, at][..., 2 * half:], plain[live][:, nq:nq + nkv, 2 * half:])
+    assert torch.equal(vc[page, :, :, at], plain[live][:, nq + nkv:])
+    free = torch.ones(pages, ps, dtype=torch.bool, device="cuda")
+    free[page, at] = False
+    assert bool((kc.transpose(1, 2)[free] == 7.0).all()) and bool((vc.permute(0, 3, 1, 2)[free] == 7.0).all())
+
+
 def _paged(k, v, ps, pages, dtype, seed):
     """Scatter per-request keys/values [nkv, T, hd] into shuffled pages; returns caches and tables."""
     g = torch.Generator().manual_seed(seed)
@@ -889,6 +932,59 @@ def test_tiled_product(m, n, k, shape):
     assert torch.allclose(tile.tile_gated(x, w, 1.702, 1.5, 1.0, shape=shape).float(), ref, atol=2e-2, rtol=2e-2)
     gate, up = want[:, :n // 2], want[:, n // 2:]
     assert torch.allclose(tile.tile_gated(x, w, 1.0, None, 0.0, shape=shape).float(), gate * torch.sigmoid(gate) * up, atol=3e-2, rtol=2e-2)
+
+
+@pytest.mark.parametrize("shape", [0, 1, 2, 3])
+@pytest.mark.parametrize("beside", [0, 1, 6])
+@pytest.mark.parametrize("m, n, k", [(65, 509, 96), (130, 1018, 160), (257, 38, 64)])
+def test_tiled_product_off_steps_of_four(m, n, k, beside, shape):
+    """Outputs and row strides off steps of 4: every result in its place, nothing written beside them.  A sum of k exact products
+    is within k roundings of its terms, a stored bfloat16 half a unit in its last place further."""
+    from qwen25vl_lite_amd.ops import tile
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(n, k, device="cuda", generator=g) / k ** 0.5).bfloat16()
+    want = x.double() @ w.double().T
+    bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    for dtype, last in ((torch.float32, 0.0), (torch.bfloat16, 2.0 ** -8)):
+        room = torch.full((m + 2, 8 + n + beside), 7.0, device="cuda", dtype=dtype)
+        inside = room.view(-1)[8:][:m * (8 + n + beside)].view(m, 8 + n + beside)[:, :n]
+        tile.tile_product(x, w, dtype, out=inside, shape=shape)
+        assert bool(((inside.double() - want).abs() <= bound + last * want.abs()).all())
+        inside.fill_(7.0)
+        assert bool((room == 7.0).all())
+    if n % 2:
+        return
+    g, u = want[:, :n // 2].clamp(max=1.5), want[:, n // 2:].clamp(-1.5, 1.5)
+    ref = g * torch.sigmoid(1.25 * g) * (u + 1.0)
+    slack = 1.13 * 2.5 * bound[:, :n // 2] + 1.5 * bound[:, n // 2:]      # (slopes: see the rows kernel's test)
+    got = tile.tile_gated(x, w, 1.25, 1.5, 1.0, shape=shape).double()
+    assert bool(((got - ref).abs() <= slack + (2.0 ** -8 + 1e-6) * ref.abs() + 2e-6).all())
+
+
+@pytest.mark.parametrize("m", [1, 19, 40])
+@pytest.mark.parametrize("n", [2, 34, 16401, 40970])
+def test_rows_with_a_last_output_alone(m, n):
+    """An odd number of outputs, or of channels of a gated product: the last one has no neighbour to be stored with."""
+    from qwen25vl_lite_amd.ops import rows
+    torch.manual_seed(m + n)
+    k = 72
+    x = torch.randn(m, k, device="cuda").bfloat16()
+    w = (torch.randn(n, k, device="cuda") / math.sqrt(k)).bfloat16()
+    want = x.double() @ w.double().T
+    bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    for wider in (n % 2, 1 - n % 2):       # an even row stride, whose results are stored in pairs, and an odd one
+        room = torch.full((m + 1, n + wider), 7.0, device="cuda").bfloat16()
+        rows.rows_product(x, w, out=room[:m, :n])
+        assert bool(((room[:m, :n].double() - want).abs() <= bound + 2.0 ** -8 * want.abs()).all())
+        assert bool((room[:m, n:] == 7.0).all()) and bool((room[m] == 7.0).all())
+    if n % 2:
+        return
+    got = rows.rows_gated(x, w, 1.25, 1.5, 1.0).double()
+    g, u = want[:, :n // 2].clamp(max=1.5), want[:, n // 2:].clamp(-1.5, 1.5)
+    ref = g * torch.sigmoid(1.25 * g) * (u + 1.0)
+    slack = 1.13 * 2.5 * bound[:, :n // 2] + 1.5 * bound[:, n // 2:]
+    assert bool(((got - ref).abs() <= slack + (2.0 ** -8 + 1e-6) * ref.abs() + 2e-6).all())
 
 
 @pytest.mark.parametrize("m, n, k", [(65, 3584, 18944), (280, 2048, 11008), (100, 2560, 2048), (700, 272, 1376)])
