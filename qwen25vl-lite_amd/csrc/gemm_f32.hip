@@ -9,7 +9,8 @@
 // what the plain kernel at the end gives.
 //
 // What bounds the product: up to 64 rows (a decode step) reading W once; with more rows the matrix
-// cores, and for few outputs the chain itself: 32 cycles for four values of K (K = 11,008: 37 us).
+// cores.  With few outputs a block has one chain and little to hide its reads of LDS behind: 8 x 2,048 x 11,008 takes 118 us, of which
+// the chain, 32 cycles for four values of K, is 37.
 // Both operands come through LDS with loads that put their 16 bytes there directly, several steps of K
 // ahead; a row's 16-byte chunks are exchanged by bits of the row's number, so that the 16 rows that one
 // operand read touches lie in different banks.  Measured at the 3B decoder's sizes, two layers and the head,

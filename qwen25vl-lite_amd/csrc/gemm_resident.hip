@@ -20,10 +20,10 @@
 // half a cache line a row, and each line is asked for twice (gate|up of the 7B decoder, 271.6 MB, 8 rows: 51 us = 5.3
 // TB/s; marked as read once, 54.7, the line's second half fetched anew).  So a wave brings its own columns of a tile into LDS with loads
 // that put their 16 bytes there directly, 256 bytes of 4 rows at a time, whole lines, marked as read once, and reads the
-// operands back from there.  Per call in a decode step of 8 rows of the 7B decoder: gate|up with its norm 49.9 us = 5.4
-// TB/s (51.0 with loads into registers), the head's 152,064 x 3,584 and the ranges of the down products, 16 and 128
-// calls, 40.9 on average (43.5).  A plain read of as much reaches 7.3 TB/s; without the norm gate|up takes 46: every
-// block reads and norms all rows first.  A wave waits for its own loads only (no
+// operands back from there (that product with its norm 49.9 us; without the norm 46, every block reads and norms all rows
+// first: with K beyond 2,048 products of so many outputs go to gemm_rows.hip, 43 and a norm kernel of 5).  Per call in a decode step: 7B
+// decoder, 8 rows, the down product's ranges 24.8 us = 5.5 TB/s, q|k|v 12.4, o 8.2; 3B decoder, 1 row, gate|up with its norm 20.6 us
+// = 4.4 TB/s.  A plain read of much memory reaches 7.3 TB/s.  A wave waits for its own loads only (no
 // barrier but the one of the merge), four units of 128 columns go round, each asked for again the moment it has been
 // read, so that the next tile is on its way while a tile's sums are merged.
 //

@@ -1,4 +1,4 @@
-// Products with 17 to 64 rows: out = X[M, K] . W[N, K]^T, bfloat16 operands, float32 sums, stored as they are, as bfloat16, through
+// Products with up to 64 rows: out = X[M, K] . W[N, K]^T, bfloat16 operands, float32 sums, stored as they are, as bfloat16, through
 // the gated activation of W's rows (groups of 8 gate and 8 up rows, or all gate rows first), or as one slab of sums for each range of K.
 //
 // What bounds it is reading W once.  A wave owns up to 32 rows of W and all rows of X (operands of
@@ -10,9 +10,10 @@
 // a tile of W (gemm_resident) it must fit them; here its rows and K are free, and eight waves read it at LDS's rate: 32 rows
 // of W a wave for 64 of X keep that below half of what LDS can do.
 //
-// Per call in a decode step: gate|up of the 7B decoder (37,888 x 3,584), 64 rows, 50.3 us = 5.4 TB/s (the library's product
-// 61.2 and the activation's kernel 5.0); of the 72B decoder (59,136 x 8,192), 19 rows, 145 = 6.7 TB/s (174 and 4.6); heads of
-// 152,064 x 3,584, 64 rows, 196 (212), x 8,192, 19 rows, 426 (465).  A plain read of as much reaches 7.3 TB/s.  Four waves a
+// Per call in a decode step: gate|up of the 7B decoder (37,888 x 3,584), 8 rows, 43.0 us = 6.3 TB/s (gemm_resident, with the
+// norm inside, 50), 64 rows, 50.0 = 5.4 TB/s (the library's product 61.2 and the activation's kernel 5.0); of the 72B decoder
+// (59,136 x 8,192), 19 rows, 149 = 6.5 TB/s (174 and 4.6); heads of 152,064 x 3,584, 8 rows, 164, 64 rows, 194 (212), x 8,192, 19
+// rows, 433 (465).  A plain read of as much reaches 7.3 TB/s.  Four waves a
 // block and two blocks a compute unit: 57 for 50; operands read and multiplied in turn, tile after tile of 16 rows: 65.
 #include "tile_product.h"
 

@@ -1,10 +1,12 @@
 """Matrix products of the step: ``x @ weight.T`` for ``weight`` as a Linear stores it.
 
-float32 runs through the hand-written FMA kernel (true 32-bit, fixed summation order).
-bfloat16 with up to 64 rows (a decode step) runs through the hand-written matrix-core kernel, which
-also folds the norm before a product, the residual add after it and the SwiGLU activation into
-itself, or through one that needs not keep the rows (:mod:`~qwen25vl_lite_amd.ops.rows`); with more rows the tiled kernel runs (:mod:`~qwen25vl_lite_amd.ops.tile`), with the activation on its sums, or
-cut along the inner size where the result joins a sum anyway.  The vendor library's product, which the
+float32 runs through hand-written kernels on the matrix cores' float32 instruction (true 32-bit, fixed summation order; plain
+multiply-adds where strides or sizes do not suit it).
+bfloat16 with up to 32 rows (a decode step) runs through the hand-written matrix-core kernel that keeps the rows
+(:mod:`~qwen25vl_lite_amd.ops.skinny`), which also folds the norm before a product, the residual add after it and the SwiGLU
+activation into itself; up to 64 rows with many outputs through one that needs not keep them (:mod:`~qwen25vl_lite_amd.ops.rows`);
+with more rows the tiled kernel runs (:mod:`~qwen25vl_lite_amd.ops.tile`), with the activation on its sums.  Where the result
+joins a sum anyway products may be cut along the inner size.  The vendor library's product, which the
 reference's engine uses for its projections (reference src/qwen25vl_lite/text.py:61-66, 80-90), is left
 for what neither takes or does as fast.
 """
@@ -60,7 +62,7 @@ def linear(x: Union[torch.Tensor, NormedRows], weight: torch.Tensor, bias: Optio
     if not weight.is_cuda:
         raise kernels.KernelError("linear has no CPU path: its tensors must be on the GPU")
     if weight.dtype == torch.bfloat16:
-        # with more rows teams of blocks lose to the library; with many outputs and more than a column tile of rows to `rows`
+        # with more rows teams of blocks lose to the library, with many outputs to `rows` (see `wide`; it adds no bias)
         few = m <= skinny.ONE_BLOCK_ROWS and (bias is not None or not rows.wide(m, weight))
         if lazy and few and skinny.takes_resident(m, k, weight, norm=True):
             return skinny.resident_product(weight, h=x.h, norm_weight=x.weight, eps=x.eps, bias=bias,

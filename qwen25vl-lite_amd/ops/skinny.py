@@ -216,9 +216,11 @@ def qkv_rope_product(weight: torch.Tensor, cs: torch.Tensor, *, x: Optional[torc
 
 SPLIT_ROWS = 64   # the most rows that are cut along the inner size
 SPLIT_K = 2048    # the longest inner size, for each compute unit: with more of it a block of the few rows' kernel could not keep its range
-# Up to here a block keeps its range of the rows and walks several tiles (csrc/gemm_resident.hip: few ranges; 2,048 x 11,008, one
-# row, with the norm that adds the slabs: a decode step of the 3B decoder 4.24 ms, cut by csrc/gemm_rows.hip 4.31), with more
-# rows csrc/gemm_rows.hip cuts (3,584 x 18,944: 8 rows 25.4 us for 26.9, 16 rows 25.4 for 28.3, 64 rows 28.3 for 36.7)
+# Up to here a block keeps its range of the rows and walks several tiles (csrc/gemm_resident.hip: few ranges, so few slabs for the
+# norm behind to add), with more rows csrc/gemm_rows.hip cuts (3,584 x 18,944 alone: 8 rows 25.4 us for 26.9, 16 rows 25.4 for 28.3, 64
+# rows 28.3 for 36.7).  A pass of 8 decode steps with the norms, cut by gemm_rows.hip for this kernel: 3B sizes, 8 layers, 1 row 4,698
+# us for 4,579, 8 rows 5,207 for 5,095; 7B, 8 layers, 1 row 8,248 for 8,298, 4 rows 8,420 for 8,432, 8 rows 8,701 for 8,678; 72B, 2
+# layers, 1 row 8,686 for 8,637, 8 rows 8,958 for 9,010: within 0.6 per cent at the long inner sizes, 2 per cent slower at 11,008.
 KEPT_SPLIT_ROWS = 8
 
 
@@ -241,9 +243,11 @@ def prefers_split(m: int, k: int, weight: torch.Tensor) -> bool:
     """Where the split kernel is the fastest way to a product that is added to the residual
     (measured on MI355X at the 3B, 7B and 72B decoders' output and down projections): up to 16 rows
     when the inner size is too long for a block of the resident kernel to keep its rows for one
-    pass over the weight (the down projection at 8 rows: 26.9 us against 37.3, which pays for the
-    norm kernel that then adds the slabs, 5.7 us, where the resident kernel adds in place and the
-    next product forms the norm itself); with more rows always (the output projection at 32 rows:
+    pass over the weight (the down projection at 8 rows: 26.9 us against 37.3).  A shorter one adds into the sum in place: the
+    next product may form the norm itself, and where it does not (many outputs, an inner size beyond 2,048) a norm
+    without slabs stands in front of it (the output projection in slabs for in place, a pass of 8 decode steps: 3B sizes, 1 row 4,703 us for
+    4,579, 8 rows 5,255 for 5,095; 7B, 1 row 8,318 for 8,298, 8 rows 8,699 for 8,678, 16 rows 9,023 for 9,095; 72B, 1 row 8,654 for 8,637,
+    8 rows 8,923 for 9,010).  With more rows always (the output projection at 32 rows:
     10.3 us and a norm kernel of 6 against 14.2 in place and 11 more for the norm inside the gate | up
     product; at 64 rows 12.3 us against the library's 13.9 to 17.6, the down projection 28.3
     against 46.6)."""
