@@ -222,10 +222,18 @@ SPLIT_K = 2048    # the longest inner size, for each compute unit: with more of 
 # us for 4,579, 8 rows 5,207 for 5,095; 7B, 8 layers, 1 row 8,248 for 8,298, 4 rows 8,420 for 8,432, 8 rows 8,701 for 8,678; 72B, 2
 # layers, 1 row 8,686 for 8,637, 8 rows 8,958 for 9,010: within 0.6 per cent at the long inner sizes, 2 per cent slower at 11,008.
 KEPT_SPLIT_ROWS = 8
+# Up to 16 rows likewise where the weight has no more values than this: its few slabs then count for more than the pace of the stream.  A pass of
+# 6 decode steps, 3B sizes, 6 layers (2,048 x 11,008), kept for cut by gemm_rows.hip: 9 rows 3,136 us for 3,180, 12 rows 3,163 for 3,211,
+# 16 rows 3,299 for 3,340; 7B, 4 layers (3,584 x 18,944), 16 rows 4,232 for 4,213; 72B, 2 layers (8,192 x 29,568), 16 rows 6,956 for 6,848
+KEPT_WEIGHTS = 1 << 25
+
+
+def _keeps(m: int, n: int, k: int) -> bool:
+    return m <= KEPT_SPLIT_ROWS or (m <= ONE_TILE_ROWS and n * k <= KEPT_WEIGHTS)
 
 
 def _ranges(m: int, n: int, k: int, cus: int) -> int:
-    if m <= KEPT_SPLIT_ROWS:
+    if _keeps(m, n, k):
         return int(_fn("gemm_resident", "qvl_gemm_split_chunks", [_c_int] * 4)(m, n, k, cus))
     return int(_fn("gemm_rows", "qvl_gemm_rows_ranges", [_c_int] * 4)(m, n, k, cus))
 
@@ -268,7 +276,7 @@ def split_product(weight: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
         raise ValueError("x must be bfloat16 with 16-byte aligned rows")
     cus = _compute_units(x.device)
     out = torch.empty((_ranges(m, n, k, cus), m, n), dtype=torch.float32, device=x.device)
-    if m <= KEPT_SPLIT_ROWS:
+    if _keeps(m, n, k):
         fn = _fn("gemm_resident", "qvl_gemm_split",
                  [_c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr])
     else:

@@ -137,3 +137,17 @@ def test_projection_with_rotation_and_cache(k):
             untouched = torch.ones(pages, ps, dtype=torch.bool, device="cuda")
             untouched[page, at] = False
             assert bool((kc.transpose(1, 2)[untouched] == 0).all()) and bool((vc.permute(0, 3, 1, 2)[untouched] == 0).all())
+
+
+@pytest.mark.parametrize("n, k, most", [(2048, 11008, 16), (2048, 16384, 16), (2048, 16392, 8), (3584, 18944, 8)])
+def test_few_rows_cut_along_k(n, k, most):
+    """Up to 8 rows, or 16 with a small weight, few ranges whose rows stay in their blocks; beyond, the streaming kernel's: as many
+    slabs as the kernel that then runs writes, each against 64 bits in their sum."""
+    from qwen25vl_lite_amd.ops import kernels, skinny
+    cus = kernels.compute_units("cuda:0")
+    for m in (1, 8, 9, 16, 17):
+        x, w, want, slack = _operands(m, n, k)
+        slabs = skinny.split_product(w, x)
+        stem, name = ("gemm_resident", "qvl_gemm_split_chunks") if m <= most else ("gemm_rows", "qvl_gemm_rows_ranges")
+        assert slabs.shape[0] == kernels._fn(stem, name, [skinny._c_int] * 4)(m, n, k, cus), m
+        assert bool(((slabs.double().sum(0) - want).abs() <= slack).all()), m
