@@ -209,21 +209,25 @@ def _launch(logits: torch.Tensor, rows: np.ndarray, flat: List[int]) -> PendingS
     c_ptr, c_int = ctypes.c_void_p, ctypes.c_int
     fn = _fn("sample", "qvl_sample_rows", [c_ptr] * 7 + [c_int] * 4 + [c_ptr])
     parts_bytes = _fn("sample", "qvl_sample_parts_bytes", [c_int], restype=ctypes.c_longlong)
-    scratch_bytes = _fn("sample", "qvl_sample_scratch_bytes", [], restype=ctypes.c_longlong)
     dev = logits.device
     draws = rows["temperature"] > 0
     with torch.cuda.device(dev):
         packed = np.concatenate([rows.view(np.int32), _int32_ids(flat)])
         buf = _Staging.to_device(packed, dev)
         n_row_words = rows.view(np.int32).size
-        some = bool(draws.any())
-        # rows that draw with penalties have their scores written out; the passes read the others' logits as they are
-        scores = torch.empty_like(logits) if bool((draws & (rows["prev_end"] > rows["prev_begin"])).any()) else None
-        scratch = torch.empty(m * scratch_bytes(), dtype=torch.uint8, device=dev) if some else None
+        scores = scratch = None
+        top_k = top_p = 0
+        if draws.any():
+            scratch_bytes = _fn("sample", "qvl_sample_scratch_bytes", [], restype=ctypes.c_longlong)
+            scratch = torch.empty(m * scratch_bytes(), dtype=torch.uint8, device=dev)
+            # rows that draw with penalties have their scores written out; the passes read the others' logits as they are
+            if (draws & (rows["prev_end"] > rows["prev_begin"])).any():
+                scores = torch.empty_like(logits)
+            top_k = int((draws & (rows["top_k"] > 0) & (rows["top_k"] < vocab)).any())
+            top_p = int((draws & (rows["top_p"] < 1.0)).any())
         parts = torch.empty(m * parts_bytes(vocab), dtype=torch.uint8, device=dev)
         out = torch.empty(m, dtype=torch.int32, device=dev)
         _check(fn(logits.data_ptr(), None if scores is None else scores.data_ptr(), buf.data_ptr(),
                   buf[n_row_words:].data_ptr(), None if scratch is None else scratch.data_ptr(), parts.data_ptr(),
-                  out.data_ptr(), m, vocab, int(bool((draws & (rows["top_k"] > 0) & (rows["top_k"] < vocab)).any())),
-                  int(bool((draws & (rows["top_p"] < 1.0)).any())), _stream()), "sample_rows")
+                  out.data_ptr(), m, vocab, top_k, top_p, _stream()), "sample_rows")
         return PendingSample(out)
