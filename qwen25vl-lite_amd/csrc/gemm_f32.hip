@@ -1,20 +1,22 @@
 // True float32 matrix product  C[M,N] = A[M,K] * W[N,K]^T (+ bias[N]),  W as a Linear stores it.
-// Every output element sums its K products in index order 0..K-1 in one accumulator, one fused
-// multiply-add after the other, so a row's result does not depend on M or on the tile it falls in.
+// Every output's sum has one order that K alone sets, so a row's result does not depend on M or on the tile it falls
+// in: K is cut into at most eight ranges (range_of) and these into runs of 32 values.  A run's products join one
+// accumulator that begins at zero, one fused multiply-add after the other, 16 values at a time with k mod 16 in the order 0
+// 4 8 12 1 5 9 13 2 6 10 14 3 7 11 15; the runs' sums are added from the range's first to its last, then the ranges'.
 //
 // v_mfma_f32_16x16x4_f32 takes float32 operands as they are and forms its four products of an output
-// the same way, in order of the inner index with one rounding each: on random, widely scaled, denormal
+// in order of the inner index with one rounding each: on random, widely scaled, denormal
 // and mixed inputs its results have the bits of a chain of fmaf.  So the tiles below run on the matrix
 // cores (157 TFLOP/s of float32, twice what single multiply-adds of the vector units reach) and give
-// what the plain kernel at the end gives.
+// what the plain kernel at the end gives.  The order within 16 values is that of lanes which each read 16 bytes: lane group g
+// holds values 4 g ... 4 g + 3, and the t-th instruction takes the t-th of each.
 //
-// What bounds the product: up to 64 rows (a decode step) reading W once; with more rows the matrix
-// cores.  With few outputs a block has one chain and little to hide its reads of LDS behind: 8 x 2,048 x 11,008 takes 118 us, of which
-// the chain, 32 cycles for four values of K, is 37.
-// Both operands come through LDS with loads that put their 16 bytes there directly, several steps of K
-// ahead; a row's 16-byte chunks are exchanged by bits of the row's number, so that the 16 rows that one
-// operand read touches lie in different banks.  Measured at the 3B decoder's sizes, two layers and the head,
-// one step of 164 rows and three of 6 or 7: their products take 3.19 ms instead of the plain kernel's 21.0 ms.
+// Why ranges: one chain an output is 32 cycles for four values of K wherever the outputs are few (8 x 2,048 x 11,008: 37 us at
+// least, 118 as measured), and cannot be shared out; ranges run in waves and blocks beside each other.  Short
+// runs round off less (error against 64 bits at K = 2,048 1.3e-7 of the
+// result, one chain 8.1e-7; at 11,008 1.7e-7 and 1.9e-6).  Before and after: 6 x 2,048 x 11,008 117 and 24 us, 6 x 22,016 x 2,048 44 and 33
+// (5.4 TB/s), 6 x 151,936 x 2,048 233 and 198 (6.3 TB/s), 6 x 2,048 x 2,048 24 and 7; 164 x 2,048 x 11,008 188 and 92, 164 x 22,016 x
+// 2,048 230 and 190, 700 x 22,016 x 2,048 874 and 550 (115 TFLOP/s).
 #include "common.h"
 
 #include <type_traits>
@@ -24,6 +26,14 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 #define TM 64
 #define TN 64
 #define TK 16
+#define MOST_RANGES 8
+#define RUN 32
+
+// Values of K in a range: an eighth, in steps of 64, 256 at least.
+__host__ __device__ __forceinline__ int range_of(int K) {
+  const int r = ((K + MOST_RANGES - 1) / MOST_RANGES + 63) / 64 * 64;
+  return r < 256 ? 256 : r;
+}
 
 // Any strides and any K: 64x64 tile per block, 16x16 threads, 4x4 outputs per thread, K step 16.
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ A, int lda,
@@ -34,13 +44,25 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
   __shared__ float sw[TK][TN + 4];
   const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
   const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-  float acc[4][4];
+  const int range = range_of(K);
+  float run[4][4], acc[4][4], total[4][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+    for (int j = 0; j < 4; ++j) run[i][j] = acc[i][j] = total[i][j] = 0.f;
+  auto join = [](float (&to)[4][4], float (&from)[4][4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        to[i][j] += from[i][j];
+        from[i][j] = 0.f;
+      }
+  };
 
   for (int k0 = 0; k0 < K; k0 += TK) {
+    if (k0 && k0 % RUN == 0) join(acc, run);
+    if (k0 && k0 % range == 0) join(total, acc);
     // 64 rows x 16 k per operand: 1024 elements, 4 per thread
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -52,7 +74,8 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
     }
     __syncthreads();
 #pragma unroll
-    for (int kk = 0; kk < TK; ++kk) {
+    for (int step = 0; step < TK; ++step) {
+      const int kk = 4 * (step & 3) + (step >> 2);
       float a[4], b[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) a[i] = sa[kk][ty * 4 + i];
@@ -61,10 +84,11 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+        for (int j = 0; j < 4; ++j) run[i][j] = fmaf(a[i], b[j], run[i][j]);
     }
     __syncthreads();
   }
+  join(acc, run);
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int gm = m0 + ty * 4 + i;
@@ -72,7 +96,7 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int gn = n0 + tx * 4 + j;
-      if (gn < N) C[(size_t)gm * ldc + gn] = acc[i][j] + (bias ? bias[gn] : 0.f);
+      if (gn < N) C[(size_t)gm * ldc + gn] = (total[i][j] + acc[i][j]) + (bias ? bias[gn] : 0.f);
     }
   }
 }
@@ -105,37 +129,151 @@ __device__ __forceinline__ void wait_steps(int ahead) {
   }
 }
 
-// WN x WM waves, each with TNW x TMW tiles of 16 outputs (rows of W) by 16 rows of A; K in steps of KT values
-// through STAGES stages of LDS.  K a multiple of 4, rows of A and W on 16-byte boundaries.
-template <int WN, int WM, int TNW, int TMW, int KT, int STAGES>
-__global__ __launch_bounds__(64 * WN * WM) void gemm_f32_mfma_kernel(const float* __restrict__ A, int lda,
+// Up to 16 rows: reading W once is the bound.  A block of eight waves has 8 WF outputs at a time, each wave one of K's
+// ranges.  A wave fetches its steps of 32 values ahead through a ring of LDS of its own, across its tiles, W's lines
+// whole (8 rows of 128 bytes an instruction) and marked as read once: no barrier stands between a fetch and its use, only
+// the sums of the ranges meet once a tile.  XF fetches of 8 rows of A a step.  WF = 1 where that leaves a tile for each compute
+// unit at most: one unit fetches some 40 GB/s, so all should (6 x 2,048 x 11,008 with 16 outputs a block, on half of them, 29 us for 24).
+#define F32_STREAM_ROWS 16
+template <int WF, int XF>
+__global__ __launch_bounds__(64 * MOST_RANGES) void gemm_f32_stream_kernel(const float* __restrict__ A, int lda,
+                                                                           const float* __restrict__ W, int ldw,
+                                                                           const float* __restrict__ bias, float* __restrict__ C,
+                                                                           int ldc, int M, int N, int K, int tiles) {
+  constexpr int STEP = 32, ROWS_W = 8 * WF, FETCHES = WF + XF, STAGE = FETCHES * 1024, SUMS = MOST_RANGES * 1024;   // SUMS: bytes of a tile's
+  constexpr int STAGES = (163840 - 2 * SUMS) / MOST_RANGES / STAGE;
+  __shared__ __attribute__((aligned(16))) char lds[MOST_RANGES * STAGES * STAGE + 2 * SUMS];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
+  const int range = range_of(K), ranges = (K + range - 1) / range;
+  const int k_first = wave * range, ksteps = wave < ranges ? (min(K - k_first, range) + STEP - 1) / STEP : 0;
+  const int my_tiles = (tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x, steps = ksteps * my_tiles;
+  char* sums = lds + MOST_RANGES * STAGES * STAGE;
+  const char* mine = lds + wave * STAGES * STAGE;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + wave * STAGES * STAGE;
+  // a fetch brings rows 8 j ... 8 j + 7; place s of row rho holds chunk s ^ ((rho / 2) mod 8).  Rows that do not exist are read
+  // from ones that do, their sums are not stored; so are chunks beyond K, which the multiplication replaces by zeros.
+  const int row8 = lane >> 3;
+  auto chunk_at = [&](int j) { return (lane & 7) ^ (((8 * j + row8) >> 1) & 7); };
+  uint32_t fa[XF], fw[WF];
+#pragma unroll
+  for (int j = 0; j < XF; ++j) fa[j] = (uint32_t)min(8 * j + row8, M - 1) * (uint32_t)lda * 4;
+  int asked = 0, ask_k = 0, ask_tile = blockIdx.x, ask_stage = 0;
+  const float* wbase = W;
+  auto ask = [&]() __attribute__((always_inline)) {
+    if (asked >= steps) return;
+    if (ask_k == 0) {
+      wbase = W + (size_t)ask_tile * ROWS_W * ldw;
+#pragma unroll
+      for (int j = 0; j < WF; ++j) {
+        const int n = 8 * j + row8;
+        fw[j] = (uint32_t)(ask_tile * ROWS_W + n < N ? n : 0) * (uint32_t)ldw * 4;
+      }
+    }
+    const uint32_t at = lds0 + ask_stage * STAGE;
+    const int k0 = k_first + ask_k * STEP;
+    auto bytes = [&](int j) {
+      const int k = k0 + 4 * chunk_at(j);
+      return (uint32_t)(k < K ? k : 0) * 4;
+    };
+#pragma unroll
+    for (int j = 0; j < WF; ++j) fetch16_to_lds<false>(wbase, fw[j] + bytes(j), at + j * 1024);
+#pragma unroll
+    for (int j = 0; j < XF; ++j) fetch16_to_lds<true>(A, fa[j] + bytes(j), at + (WF + j) * 1024);
+    ++asked;
+    ask_stage = ask_stage + 1 == STAGES ? 0 : ask_stage + 1;
+    if (++ask_k == ksteps) {
+      ask_k = 0;
+      ask_tile += gridDim.x;
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < STAGES - 1; ++i) ask();
+  f32x4_t acc{0.f, 0.f, 0.f, 0.f};
+  const int wr = WF == 1 ? r & 7 : r, xr = XF == 1 ? r & 7 : r;       // (sums of rows twice there are not stored)
+  const uint32_t sw = (wr >> 1) & 7, xsw = (xr >> 1) & 7;
+  int stage = 0, s = 0;
+  for (int i = 0; i < my_tiles; ++i) {
+    for (int k = 0; k < ksteps; ++k, ++s) {
+      wait_steps<STAGES - 2, FETCHES>(asked - 1 - s);
+      __builtin_amdgcn_sched_barrier(0);
+      const char* pw = mine + stage * STAGE + wr * 128;
+      const char* px = mine + stage * STAGE + WF * 1024 + xr * 128;
+      f32x4_t w4[2], x4[2];
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        w4[c] = *reinterpret_cast<const f32x4_t*>(pw + (((4 * c + g) ^ sw) << 4));
+        x4[c] = *reinterpret_cast<const f32x4_t*>(px + (((4 * c + g) ^ xsw) << 4));
+      }
+      __builtin_amdgcn_s_waitcnt(0xc07f);       // read: the next fetches go where the step before this one lay
+      __builtin_amdgcn_sched_barrier(0);
+      ask();
+      const int left = K - (k_first + k * STEP);
+      if (left < STEP) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+          if (4 * (4 * c + g) >= left) w4[c] = x4[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
+      f32x4_t run{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) run = __builtin_amdgcn_mfma_f32_16x16x4f32(w4[c][e], x4[c][e], run, 0, 0, 0);
+      acc += run;
+      stage = stage + 1 == STAGES ? 0 : stage + 1;
+    }
+    char* here = sums + (i & 1) * SUMS;
+    if (wave < ranges) {
+      *reinterpret_cast<f32x4_t*>(here + wave * 1024 + lane * 16) = acc;
+      acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();               // (fetches stay in flight.)  The sums of the tile before the last have been read, too
+    __builtin_amdgcn_sched_barrier(0);
+    // output n of row m: lane 16 (n / 4) + m holds it as its number n mod 4
+    const int m = threadIdx.x >> 4, n = threadIdx.x & 15, gn = ((int)blockIdx.x + i * (int)gridDim.x) * ROWS_W + n;
+    if (m < M && n < ROWS_W && gn < N) {
+      const float* q = reinterpret_cast<const float*>(here) + ((n >> 2) * 16 + m) * 4 + (n & 3);
+      float total = 0.f;
+      for (int w = 0; w < ranges; ++w) total += q[w * 256];
+      C[(size_t)m * ldc + gn] = total + (bias ? bias[gn] : 0.f);
+    }
+  }
+  wait_fetches<0>();
+}
+
+// More rows: WN x WM waves, each with TNW x TMW tiles of 16 outputs (rows of W) by 16 rows of A; K in steps of 32 values
+// through STAGES stages of LDS, the matrix cores the bound.  Registers and LDS leave room for four blocks a compute unit, which
+// hide each other's barriers (1,500 x 2,048 x 11,008: 595 us; tiles of 128 x 128, a block a unit, 757).  A block has `per` of K's ranges.  slabs: the sums of
+// range i go to slab i, so many floats apart; otherwise (one block has all ranges) their sum goes to C.
+// ONCE: no other block reads these rows of W.
+template <int WN, int WM, int TNW, int TMW, int STAGES, bool ONCE>
+__global__ __launch_bounds__(64 * WN * WM, 4) void gemm_f32_tile_kernel(const float* __restrict__ A, int lda,
                                                                      const float* __restrict__ W, int ldw,
                                                                      const float* __restrict__ bias, float* __restrict__ C,
-                                                                     int ldc, int M, int N, int K) {
-  constexpr int NWAVES = WN * WM, ROWS_W = 16 * WN * TNW, ROWS_A = 16 * WM * TMW;
-  constexpr int CH = KT / 4;                                  // 16-byte chunks of a row of a stage
-  constexpr int ROWS_LOAD = 64 / CH;                          // rows one wave's fetch covers (1 KB)
-  constexpr int LOADS = (ROWS_W + ROWS_A) / ROWS_LOAD / NWAVES;
-  static_assert(LOADS * ROWS_LOAD * NWAVES == ROWS_W + ROWS_A, "the fetches divide evenly among the waves");
-  static_assert(ROWS_W % ROWS_LOAD == 0 && ROWS_A % ROWS_LOAD == 0, "a fetch lies in one operand");
+                                                                     int ldc, int M, int N, int K, int per, long long slabs) {
+  constexpr int NWAVES = WN * WM, ROWS_W = 16 * WN * TNW, ROWS_A = 16 * WM * TMW, KT = 32;
+  constexpr int LOADS = (ROWS_W + ROWS_A) / 8 / NWAVES, STAGE = (ROWS_W + ROWS_A) * KT * 4;
+  static_assert(LOADS * 8 * NWAVES == ROWS_W + ROWS_A, "the fetches divide evenly among the waves");
   static_assert((STAGES - 2) * LOADS < 64, "the counter's range");
-  __shared__ __attribute__((aligned(16))) float stage[STAGES][(ROWS_W + ROWS_A) * KT];
-  const int wave = NWAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  __shared__ __attribute__((aligned(16))) char lds[STAGES * STAGE];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
   const int wn = wave % WN, wm = wave / WN;
   const int n0 = blockIdx.x * ROWS_W, m0 = blockIdx.y * ROWS_A;
   const float* wbase = W + (size_t)n0 * ldw;
   const float* abase = A + (size_t)m0 * lda;
+  const int range = range_of(K), k_first = blockIdx.z * per * range, k_end = min(K, k_first + per * range);
 
-  // this wave's fetches of a step: rows (wave LOADS + j) ROWS_LOAD ... of the stage, W's rows first.  Place s of row
-  // rho holds chunk s ^ (rho mod CH).  A row that does not exist is read from one that does (its sums are not stored).
+  // this wave's fetches of a step: 8 rows each, W's first.  Place s of row rho holds chunk s ^ ((rho / 2) mod 8).  Rows and
+  // chunks that do not exist are read from ones that do.
   uint32_t from[LOADS];
   int chunk[LOADS];
 #pragma unroll
   for (int j = 0; j < LOADS; ++j) {
-    const int rho = (wave * LOADS + j) * ROWS_LOAD + lane / CH;
-    chunk[j] = (lane % CH) ^ (rho & (CH - 1));
-    if ((wave * LOADS + j) * ROWS_LOAD < ROWS_W) {
+    const int rho = (wave * LOADS + j) * 8 + (lane >> 3);
+    chunk[j] = (lane & 7) ^ ((rho >> 1) & 7);
+    if ((wave * LOADS + j) * 8 < ROWS_W) {
       const int n = n0 + rho < N ? rho : 0;
       from[j] = (uint32_t)((size_t)n * ldw * 4);
     } else {
@@ -143,160 +281,212 @@ __global__ __launch_bounds__(64 * WN * WM) void gemm_f32_mfma_kernel(const float
       from[j] = (uint32_t)((size_t)m * lda * 4);
     }
   }
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)&stage[0][0];
-  auto issue = [&](int step) {
-    const uint32_t at = lds0 + (uint32_t)(step % STAGES) * ((ROWS_W + ROWS_A) * KT * 4) + (uint32_t)wave * (LOADS * 1024);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
+  int ask_stage = 0;
+  auto issue = [&](int step) __attribute__((always_inline)) {
+    const uint32_t at = lds0 + (uint32_t)ask_stage * STAGE + (uint32_t)wave * (LOADS * 1024);
+    ask_stage = ask_stage + 1 == STAGES ? 0 : ask_stage + 1;
 #pragma unroll
     for (int j = 0; j < LOADS; ++j) {
-      // a chunk beyond K (in the last step) is read from the row's first: it is not multiplied
-      const int k = step * KT + 4 * chunk[j];
+      const int k = k_first + step * KT + 4 * chunk[j];
       const uint32_t bytes = from[j] + (uint32_t)(k < K ? k : 0) * 4;
-      if ((wave * LOADS + j) * ROWS_LOAD < ROWS_W) fetch16_to_lds<(WM > 1)>(wbase, bytes, at + j * 1024);
+      if ((wave * LOADS + j) * 8 < ROWS_W) fetch16_to_lds<!ONCE>(wbase, bytes, at + j * 1024);
       else fetch16_to_lds<true>(abase, bytes, at + j * 1024);
     }
   };
-  f32x4_t acc[TNW][TMW];
+  f32x4_t acc[TNW][TMW], total[TNW][TMW];
 #pragma unroll
   for (int n = 0; n < TNW; ++n)
 #pragma unroll
-    for (int m = 0; m < TMW; ++m) acc[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < TMW; ++m) acc[n][m] = total[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // a lane holds, of (n, m): row 16 (wm TMW + m) + r of A, outputs 16 (wn TNW + n) + 4 g ...
+  auto store = [&](float* to, int ld, const f32x4_t (*v)[TMW], const float* add) __attribute__((always_inline)) {
+    const bool fours = ld % 4 == 0 && (uintptr_t)to % 16 == 0;
+#pragma unroll
+    for (int m = 0; m < TMW; ++m) {
+      const int gm = m0 + (wm * TMW + m) * 16 + r;
+      if (gm >= M) continue;
+#pragma unroll
+      for (int n = 0; n < TNW; ++n) {
+        const int gn = n0 + (wn * TNW + n) * 16 + 4 * g;
+        float* o = to + (size_t)gm * ld + gn;
+        f32x4_t x = v[n][m];
+        if (add) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) x[i] += gn + i < N ? add[gn + i] : 0.f;
+        }
+        if (fours && gn + 4 <= N) {
+          *reinterpret_cast<f32x4_t*>(o) = x;
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (gn + i < N) o[i] = x[i];
+        }
+      }
+    }
+  };
 
-  const int steps = (K + KT - 1) / KT;
+  const int steps = (k_end - k_first + KT - 1) / KT;
 #pragma unroll
   for (int i = 0; i < STAGES - 1; ++i)
     if (i < steps) issue(i);
-  // With one tile a wave, a step's operands are read from LDS while those of the step before are multiplied: the chain of
-  // products of one sum is all there is to hide the reads behind (8 x 2,048 x 11,008: 140 -> 118 us; 64 rows 169 -> 153).  Four waves
-  // side by side on many outputs hide it behind each other (22,016 x 2,048: 43.8, so 44.6).
-  if constexpr (TNW == 1 && TMW == 1 && WN < 4) {
-    float fw[2][CH], fa[2][CH];
-    auto read = [&](int s, auto buf) __attribute__((always_inline)) {
-      constexpr int B = decltype(buf)::value;
-      const float* sw = stage[s % STAGES];
-      const float* sa = sw + ROWS_W * KT;
+  // Half a step's operands are read from LDS while those of the half before are multiplied: all waves pass a barrier
+  // together, so that reading and multiplying would else take turns.
+  const uint32_t sw = (r >> 1) & 7;
+  f32x4_t w4[2][TNW], x4[2][TMW], run[TNW][TMW];
+  int stage = 0, left = min(range, k_end - k_first), slab = blockIdx.z * per;
+  auto read = [&](auto half) __attribute__((always_inline)) {
+    constexpr int H = decltype(half)::value;
+    const char* p = lds + stage * STAGE + r * 128 + (((4 * H + g) ^ sw) << 4);
 #pragma unroll
-      for (int c = 0; c < CH; ++c) {
-        const int row = wn * 16 + r;
-        fw[B][c] = sw[row * KT + 4 * (c ^ (row & (CH - 1))) + g];
-        const int ra = wm * 16 + r;
-        fa[B][c] = sa[ra * KT + 4 * (c ^ ((ROWS_W + ra) & (CH - 1))) + g];
-      }
-    };
-    auto multiply = [&](int s, auto buf) __attribute__((always_inline)) {
-      constexpr int B = decltype(buf)::value;
-      const int chunks = s + 1 < steps || K % KT == 0 ? CH : (K % KT) / 4;
-      if (chunks == CH) {
+    for (int n = 0; n < TNW; ++n) w4[H][n] = *reinterpret_cast<const f32x4_t*>(p + (wn * TNW + n) * 2048);
 #pragma unroll
-        for (int c = 0; c < CH; ++c) acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[B][c], fa[B][c], acc[0][0], 0, 0, 0);
-      } else {
+    for (int m = 0; m < TMW; ++m) x4[H][m] = *reinterpret_cast<const f32x4_t*>(p + (ROWS_W + (wm * TMW + m) * 16) * 128);
+  };
+  auto multiply = [&](auto half) __attribute__((always_inline)) {
+    constexpr int H = decltype(half)::value;
+    if (left < KT && 4 * (4 * H + g) >= left) {          // chunks beyond K are no part of the sums
 #pragma unroll
-        for (int c = 0; c < CH; ++c)       // (unrolled, a branch each: an index at run time would move the operands about)
-          if (c < chunks) acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[B][c], fa[B][c], acc[0][0], 0, 0, 0);
-      }
-    };
-    auto step = [&](int s, auto here, auto before) __attribute__((always_inline)) {
-      if (s < steps) {
-        const int ahead = steps - 1 - s < STAGES - 2 ? steps - 1 - s : STAGES - 2;
-        wait_steps<STAGES - 2, LOADS>(ahead);
-        __syncthreads();                     // every wave's part of step s is there, and step s - 1 has been read
-        if (s + STAGES - 1 < steps) issue(s + STAGES - 1);
-        read(s, here);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if (s > 0) multiply(s - 1, before);
-    };
-    constexpr std::integral_constant<int, 0> even{};
-    constexpr std::integral_constant<int, 1> odd{};
-    for (int s = 0; s <= steps; s += 2) {
-      step(s, even, odd);
-      if (s < steps) step(s + 1, odd, even);
+      for (int n = 0; n < TNW; ++n) w4[H][n] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int m = 0; m < TMW; ++m) x4[H][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
-  } else {
-    for (int s = 0; s < steps; ++s) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+      for (int n = 0; n < TNW; ++n)
+#pragma unroll
+        for (int m = 0; m < TMW; ++m)
+          run[n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w4[H][n][e], x4[H][m][e],
+                                                           H == 0 && e == 0 ? f32x4_t{0.f, 0.f, 0.f, 0.f} : run[n][m], 0, 0, 0);
+  };
+  auto join = [&](f32x4_t (&to)[TNW][TMW], const f32x4_t (&from)[TNW][TMW]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int n = 0; n < TNW; ++n)
+#pragma unroll
+      for (int m = 0; m < TMW; ++m) to[n][m] += from[n][m];
+  };
+  constexpr std::integral_constant<int, 0> first{};
+  constexpr std::integral_constant<int, 1> second{};
+  for (int s = 0; s <= steps; ++s) {
+    if (s < steps) {
       const int ahead = steps - 1 - s < STAGES - 2 ? steps - 1 - s : STAGES - 2;
       wait_steps<STAGES - 2, LOADS>(ahead);
-      __syncthreads();                       // every wave's part of step s is there, and step s - 1 has been multiplied
+      __builtin_amdgcn_s_waitcnt(0xc07f);
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();        // every wave's part of step s is there, and step s - 1 has been read
+      __builtin_amdgcn_sched_barrier(0);
       if (s + STAGES - 1 < steps) issue(s + STAGES - 1);
-      const float* sw = stage[s % STAGES];
-      const float* sa = sw + ROWS_W * KT;
-      auto multiply = [&](int c) {           // chunk c: four values of K, lane group g has the g-th
-        float fw[TNW], fa[TMW];
-#pragma unroll
-        for (int n = 0; n < TNW; ++n) {
-          const int row = (wn * TNW + n) * 16 + r;
-          fw[n] = sw[row * KT + 4 * (c ^ (row & (CH - 1))) + g];
-        }
-#pragma unroll
-        for (int m = 0; m < TMW; ++m) {
-          const int row = (wm * TMW + m) * 16 + r;
-          fa[m] = sa[row * KT + 4 * (c ^ ((ROWS_W + row) & (CH - 1))) + g];
-        }
+      read(first);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (s > 0) {
+      multiply(second);
+      join(acc, run);
+      left -= KT;
+      if (left <= 0) {
+        left = min(range, k_end - k_first - s * KT);
+        if (slabs) store(C + (slab++) * slabs, N, acc, nullptr);
+        join(total, acc);
 #pragma unroll
         for (int n = 0; n < TNW; ++n)
 #pragma unroll
-          for (int m = 0; m < TMW; ++m) acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[n], fa[m], acc[n][m], 0, 0, 0);
-      };
-      if (s + 1 < steps || K % KT == 0) {
-#pragma unroll
-        for (int c = 0; c < CH; ++c) multiply(c);
-      } else {
-        for (int c = 0; c < (K % KT) / 4; ++c) multiply(c);
+          for (int m = 0; m < TMW; ++m) acc[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
       }
     }
-  }
-  // a lane holds, of (n, m): row 16 (wm TMW + m) + r of A, outputs 16 (wn TNW + n) + 4 g ...
-#pragma unroll
-  for (int m = 0; m < TMW; ++m) {
-    const int gm = m0 + (wm * TMW + m) * 16 + r;
-    if (gm >= M) continue;
-#pragma unroll
-    for (int n = 0; n < TNW; ++n) {
-      const int gn = n0 + (wn * TNW + n) * 16 + 4 * g;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        if (gn + i < N) C[(size_t)gm * ldc + gn + i] = acc[n][m][i] + (bias ? bias[gn + i] : 0.f);
+    if (s < steps) {
+      __builtin_amdgcn_sched_barrier(0);
+      read(second);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(first);
+      stage = stage + 1 == STAGES ? 0 : stage + 1;
     }
   }
+  if (!slabs) store(C, ldc, total, bias);
 }
 
-extern "C" int qvl_gemm_f32(const void* A, int lda, const void* W, int ldw, const void* bias, void* C, int ldc, int M,
+// The ranges' sums, added from the first to the last.
+__global__ __launch_bounds__(256) void gemm_f32_add_kernel(const float* __restrict__ sums, int ranges, long long slab,
+                                                           const float* __restrict__ bias, float* __restrict__ C, int ldc, int N) {
+  const int n = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
+  if (n >= N) return;
+  const float* p = sums + (size_t)m * N + n;
+  float v[MOST_RANGES];
+#pragma unroll
+  for (int i = 0; i < MOST_RANGES; ++i) v[i] = i < ranges ? p[i * slab] : 0.f;
+  float total = 0.f;
+#pragma unroll
+  for (int i = 0; i < MOST_RANGES; ++i)
+    if (i < ranges) total += v[i];
+  C[(size_t)m * ldc + n] = total + (bias ? bias[n] : 0.f);
+}
+
+// How a product of more than 16 rows is cut.  Tiles of 64 outputs by 64 rows (`rows`), by 32 where that is all rows.  Where there
+// are fewer tiles than 7 for 4 compute units each of K's ranges has blocks of its own; their sums are then added by a kernel
+// behind (5 us and the slabs' traffic).  Measured, cut and uncut: 164 x 2,048 x 11,008 (96 tiles) 91 us and 275, 512 x 2,560 x 2,048
+// (320) 63 and 83, 700 x 2,048 x 11,008 (352) 285 and 433, 700 x 2,560 x 2,048 (440) 84 and 84, 100 x 22,016 x 2,048 (688) 127 and 119,
+// 1,500 x 2,048 x 2,048 (768) 137 and 116.  Two or four ranges a block were never the best by more than 2 per cent.
+struct F32Plan {
+  int rows, per, parts;      // per: ranges of a block
+};
+static F32Plan f32_plan(int M, int N, int K, int cus) {
+  const int range = range_of(K), ranges = (K + range - 1) / range, rows = M <= 32 ? 32 : 64;
+  const bool cut = 4 * (long long)((N + 63) / 64) * ((M + rows - 1) / rows) < 7LL * cus;
+  return cut ? F32Plan{rows, 1, ranges} : F32Plan{rows, ranges, 1};
+}
+static bool f32_tiles(int lda, int ldw, int K) {      // 128 rows of W or A from a block's first one lie within 32 bits of bytes
+  return K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && lda < (1 << 22) && ldw < (1 << 22);
+}
+
+// Floats that qvl_gemm_f32 needs beside its operands (0: none).
+extern "C" long long qvl_gemm_f32_scratch(int lda, int ldw, int M, int N, int K, int cus) {
+  if (M <= F32_STREAM_ROWS || N <= 0 || K <= 0 || cus <= 0 || !f32_tiles(lda, ldw, K)) return 0;
+  const F32Plan p = f32_plan(M, N, K, cus);
+  const int range = range_of(K);
+  return p.parts > 1 ? (long long)((K + range - 1) / range) * M * N : 0;
+}
+
+// scratch: qvl_gemm_f32_scratch floats.
+extern "C" int qvl_gemm_f32(const void* A, int lda, const void* W, int ldw, const void* bias, void* C, int ldc, void* scratch, int M,
                             int N, int K, int cus, hipStream_t stream) {
   if (M <= 0 || N <= 0) return QVL_OK;
   if (K <= 0 || lda < K || ldw < K || ldc < N || cus <= 0) return QVL_ERR_SHAPE;
-  // 128 rows of W or A from a block's first one lie within 32 bits of bytes
-  const bool tiles = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0 &&
-                     lda < (1 << 22) && ldw < (1 << 22);
-#define GO(WN, WM, TNW, TMW, KT, STAGES)                                                                             \
-  do {                                                                                                               \
-    const dim3 grid((N + 16 * WN * TNW - 1) / (16 * WN * TNW), (M + 16 * WM * TMW - 1) / (16 * WM * TMW));             \
-    if (grid.y > 65535) return QVL_ERR_LIMIT;                                                                        \
-    hipLaunchKernelGGL((gemm_f32_mfma_kernel<WN, WM, TNW, TMW, KT, STAGES>), grid, dim3(64 * WN * WM), 0, stream,    \
-                       (const float*)A, lda, (const float*)W, ldw, (const float*)bias, (float*)C, ldc, M, N, K);     \
-    return qvl_launch_status();                                                                                      \
-  } while (0)
-  if (tiles) {
-    // Few rows: a block of four waves takes 64 outputs of all rows, so that W is read once, where that fills the
-    // device; fewer outputs are spread over blocks of one wave (16 outputs) or, with more than 16 rows, of 32 x 32.
-    const bool wide = (long long)N >= 64LL * cus;
-    if (M <= 16) {
-      if (wide) GO(4, 1, 1, 1, 64, 4);
-      GO(1, 1, 1, 1, 64, 9);
-    }
-    if (M <= 64 && wide) {
-      if (M <= 32) GO(4, 1, 1, 2, 64, 3);
-      if (M <= 48) GO(4, 1, 1, 3, 64, 4);
-      GO(4, 1, 1, 4, 64, 4);
-    }
-    // The largest tiles of which there are two for every compute unit; the chain of one tile is short only in small ones.
-    const long long big = (long long)((N + 127) / 128) * ((M + 127) / 128), mid = (long long)((N + 63) / 64) * ((M + 63) / 64);
-    if (big >= 2LL * cus) GO(2, 2, 4, 4, 32, 4);
-    if (mid >= 2LL * cus) GO(2, 2, 2, 2, 32, 4);
-    GO(2, 2, 1, 1, 32, 4);
-  }
+  const float* a = (const float*)A;
+  const float* w = (const float*)W;
+  const float* b = (const float*)bias;
+  if (f32_tiles(lda, ldw, K) && ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0) {
+    if (M <= F32_STREAM_ROWS) {
+      const bool narrow = N <= 8 * cus;
+      const int tiles = narrow ? (N + 7) / 8 : (N + 15) / 16;
+      const dim3 grid(tiles < cus ? tiles : cus), block(64 * MOST_RANGES);
+#define GO(WF, XF) hipLaunchKernelGGL((gemm_f32_stream_kernel<WF, XF>), grid, block, 0, stream, a, lda, w, ldw, b, (float*)C, ldc, M, N, K, tiles)
+      if (narrow && M <= 8) GO(1, 1);
+      else if (narrow) GO(1, 2);
+      else if (M <= 8) GO(2, 1);
+      else GO(2, 2);
 #undef GO
+      return qvl_launch_status();
+    }
+    const F32Plan p = f32_plan(M, N, K, cus);
+    if (p.parts > 1 && !scratch) return QVL_ERR_SHAPE;
+    float* to = p.parts > 1 ? (float*)scratch : (float*)C;
+    const long long slab = p.parts > 1 ? (long long)M * N : 0;
+    const dim3 grid((N + 63) / 64, (M + p.rows - 1) / p.rows, p.parts);
+    if (grid.y > 65535 || (p.parts > 1 && M > 65535)) return QVL_ERR_LIMIT;
+#define GO(...) hipLaunchKernelGGL((gemm_f32_tile_kernel<__VA_ARGS__>), grid, dim3(256), 0, stream, a, lda, w, ldw, b, to, ldc, M, N, K, p.per, slab)
+    if (p.rows == 64 && grid.y == 1) GO(2, 2, 2, 2, 2, true);
+    else if (p.rows == 64) GO(2, 2, 2, 2, 2, false);
+    else GO(4, 1, 1, 2, 3, true);
+#undef GO
+    if (p.parts > 1) {
+      const int range = range_of(K);
+      hipLaunchKernelGGL(gemm_f32_add_kernel, dim3((N + 255) / 256, M), dim3(256), 0, stream, (const float*)scratch, (K + range - 1) / range,
+                         slab, b, (float*)C, ldc, N);
+    }
+    return qvl_launch_status();
+  }
   const dim3 grid((N + TN - 1) / TN, (M + TM - 1) / TM);
   if (grid.y > 65535) return QVL_ERR_LIMIT;
-  hipLaunchKernelGGL(gemm_f32_kernel, grid, dim3(256), 0, stream, (const float*)A, lda, (const float*)W, ldw,
-                     (const float*)bias, (float*)C, ldc, M, N, K);
+  hipLaunchKernelGGL(gemm_f32_kernel, grid, dim3(256), 0, stream, a, lda, w, ldw, b, (float*)C, ldc, M, N, K);
   return qvl_launch_status();
 }

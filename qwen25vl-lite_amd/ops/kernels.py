@@ -331,8 +331,11 @@ def gemm_f32(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor]
     if out is None:
         out = torch.empty((m, n), dtype=torch.float32, device=x.device)
     _need(out.shape == (m, n) and out.dtype == torch.float32 and out.stride(1) == 1, "out must be float32 [M, N]")
+    cus = compute_units(x.device)
+    need = int(_fn("gemm_f32", "qvl_gemm_f32_scratch", [_c_int] * 6, restype=ctypes.c_longlong)(x.stride(0), weight.stride(0), m, n, k, cus))
+    sums = torch.empty(need, dtype=torch.float32, device=x.device) if need else None
     fn = _fn("gemm_f32", "qvl_gemm_f32",
-             [_c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_ptr])
-    _check(fn(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), _ptr(out), out.stride(0), m, n, k,
-              compute_units(x.device), _stream()), "gemm_f32")
+             [_c_ptr, _c_int, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr])
+    _check(fn(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), _ptr(out), out.stride(0), _ptr(sums), m, n, k,
+              cus, _stream()), "gemm_f32")
     return out

@@ -470,6 +470,24 @@ def test_gemm_f32_tiles_give_the_chains_bits(m, n, k):
     assert torch.equal(kernels.gemm_f32(x, w, b, out=out), want)
 
 
+@pytest.mark.parametrize("n, k", [(2048, 11008), (2049, 2308), (4100, 2052), (70, 8200), (17, 2044), (28700, 260)])
+@pytest.mark.parametrize("m", [1, 8, 9, 16, 17, 32, 33, 130])
+def test_gemm_f32_ranges_of_k(m, n, k):
+    """K in several ranges, the last one short and off the steps of 32; one and several tiles a block, outputs on both
+    sides of where a block takes 8 or 16, cut and uncut.  Against 64 bits (a run of 32 products and at most 43 + 8 sums on the way: each
+    rounds off half of 2^-23 of a partial sum at most, 2^-23 sqrt(91 / 2) of the result's scale as random errors add) and the plain kernel's bits."""
+    from qwen25vl_lite_amd.ops import kernels
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x, w = torch.randn(m, k, device="cuda", generator=g), torch.randn(n, k, device="cuda", generator=g)
+    b = torch.randn(n, device="cuda", generator=g)
+    got = kernels.gemm_f32(x, w, b)
+    want = x.double() @ w.double().t() + b.double()
+    assert ((got - want).norm() / want.norm()).item() < 2 ** -23 * (91 / 2) ** 0.5
+    wide = torch.zeros(m, k + 1, device="cuda")
+    wide[:, :k] = x
+    assert torch.equal(kernels.gemm_f32(wide[:, :k], w, b), got)
+
+
 @pytest.mark.parametrize("m, n, k", [(1, 509, 144), (8, 300, 200), (16, 17, 8), (9, 100, 8200), (17, 1000, 4104),
                                      (31, 130, 352), (64, 509, 3584), (5, 40, 100), (300, 64, 1000),
                                      (17, 4700, 3584), (32, 300, 3840), (24, 509, 3848), (20, 33, 8),
