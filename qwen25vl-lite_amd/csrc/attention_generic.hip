@@ -1,5 +1,5 @@
 // Paged attention for any head size, float32 or bfloat16 storage, float32 arithmetic.
-// One wave per (token, query head).  It serves prompt portions and decoded tokens alike: a
+// One wave (four where sizes are multiples of four) per (token, query head).  It serves prompt portions and decoded tokens alike: a
 // token at sequence index p sees keys lo..p of its request, lo = max(0, p - window + 1) with
 // a window, else 0 (reference attention.py:336-402 for the mask, text.py:78 for the scale); with
 // a window it also sees the request's first `keep_first` keys, wherever the window stands.  With `chunk` it
@@ -110,6 +110,157 @@ __global__ void attn_generic_kernel(const T* __restrict__ q, const T* __restrict
   }
 }
 
+// Four values from memory, as float32.
+__device__ __forceinline__ float4 load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+__device__ __forceinline__ float4 load4(const bf16_t* p) {
+  const uint2 v = *reinterpret_cast<const uint2*>(p);
+  return float4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u)};
+}
+
+// The same where head size and page size are multiples of four.  What bounds a token's few keys is the time until a load comes
+// back, so loads are wide and many are in flight: four waves take the blocks of 64 keys in turn, each with a
+// softmax of its own (joined at the end, in the waves' order); eight lanes read a key's row side by side, and a lane
+// reads a channel's values of four keys at once.  CH: channels of a value, in sixteens, at most.
+// float32, 16 heads of 128 over 2 of keys: 7 tokens at 25 to 100 keys 51 us with the wave above, 11 with these; 164 tokens of two prompts 57 and 33.
+#define ATTN_WAVES 4
+template <typename T, int CH>
+__global__ __launch_bounds__(64 * ATTN_WAVES) void attn_generic_vec_kernel(
+    const T* __restrict__ q, const T* __restrict__ kc, const T* __restrict__ vc, const int* __restrict__ block_table, int table_width,
+    const int* __restrict__ token_req, const int* __restrict__ token_seqpos, T* __restrict__ out, int nh, int nkv, int hd, int vd, int ps,
+    int window, int keep_first, int chunk, float scale, const float* __restrict__ sinks, const float2* __restrict__ turn, int turn_pairs) {
+  __shared__ __attribute__((aligned(16))) float sq[ATTN_MAX_HD];
+  __shared__ __attribute__((aligned(16))) float prob[ATTN_WAVES][64];
+  __shared__ float part[ATTN_WAVES][CH * 16], part_m[ATTN_WAVES], part_l[ATTN_WAVES];
+  const int n = blockIdx.x, h = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int r = token_req[n], p = token_seqpos[n];
+  const int kvh = h / (nh / nkv);
+  int lo = (window > 0 && p - window + 1 > 0) ? p - window + 1 : 0;
+  if (chunk > 0) lo = max(lo, p - p % chunk);
+  const int kept = keep_first < lo ? keep_first : lo;       // keys [0, kept) are seen besides [lo, p]
+  const int skip_from = (kept + 63) / 64, skipped = max(lo / 64 - skip_from, 0);  // blocks of 64 keys with nothing to see
+  const T* qr = q + ((size_t)n * nh + h) * hd;
+  for (int d = threadIdx.x; d < hd; d += 64 * ATTN_WAVES) sq[d] = ldf<T>(qr + d);
+  __syncthreads();
+  const int* bt = block_table + (size_t)r * table_width;
+
+  float m = -INFINITY, l = 0.f;
+  float acc[CH];       // channel 16 i + lane / 4, of the keys whose number / 4 has the rest lane mod 4
+#pragma unroll
+  for (int i = 0; i < CH; ++i) acc[i] = 0.f;
+  const int sub = lane & 7, quad = lane & 3, chan = lane >> 2, blocks = p < 0 ? 0 : p / 64 + 1 - skipped;
+  for (int b = wave; b < blocks; b += ATTN_WAVES) {
+    const int first = 64 * (b < skip_from ? b : b + skipped);
+    // scores: in pass i, eight lanes have key 8 (lane / 8) + i; it is lane number 8 (lane / 8) + i that keeps it
+    float s = -INFINITY;
+    const int mine = first + lane;
+    const bool valid = (mine >= lo || mine < kept) && mine <= p;
+    const T* row[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const int j = min(first + (lane & 56) + i, p), pk = bt[j / ps];
+      const size_t page = (size_t)(pk < 0 ? 0 : pk);   // a table without this page: read page 0, never out of bounds
+      row[i] = kc + ((page * nkv + kvh) * ps + (size_t)(j % ps)) * hd;
+    }
+    float dot[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int d = 4 * sub; d < hd; d += 32) {
+      const float4 a = *reinterpret_cast<const float4*>(sq + d);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float4 k = load4(row[i] + d);
+        dot[i] += a.x * k.x;
+        dot[i] += a.y * k.y;
+        dot[i] += a.z * k.z;
+        dot[i] += a.w * k.w;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+#pragma unroll
+      for (int o = 1; o < 8; o <<= 1) dot[i] += __shfl_xor(dot[i], o, QVL_WAVE);
+      if (sub == i && valid) s = dot[i] * scale;
+    }
+    const float m_new = fmaxf(m, wave_max(s));
+    const float pj = valid ? expf(s - m_new) : 0.f;
+    const float alpha = expf(m - m_new);  // m = -inf at first: alpha = 0
+    l = l * alpha + wave_sum(pj);
+    m = m_new;
+    prob[wave][lane] = pj;
+#pragma unroll
+    for (int i = 0; i < CH; ++i) acc[i] *= alpha;
+    __builtin_amdgcn_wave_barrier();       // (a wave's own lines: its writes come before its reads)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int j0 = first + 16 * t + 4 * quad;
+      if (first + 16 * t > p) break;
+      const int at = min(j0, p & ~3), pk = bt[at / ps];
+      const size_t page = (size_t)(pk < 0 ? 0 : pk);
+      const T* v = vc + ((page * nkv + kvh) * vd) * ps + (size_t)(at % ps);
+      const float4 w = *reinterpret_cast<const float4*>(&prob[wave][16 * t + 4 * quad]);
+      // values of keys that are not seen may be anything
+      auto seen = [&](int j) { return (j >= lo || j < kept) && j <= p; };
+      const bool s0 = seen(j0), s1 = seen(j0 + 1), s2 = seen(j0 + 2), s3 = seen(j0 + 3);
+      float4 x[CH];
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        const int d = 16 * i + chan;
+        if (16 * i < vd) x[i] = load4(v + (size_t)(d < vd ? d : 0) * ps);
+      }
+#pragma unroll
+      for (int i = 0; i < CH; ++i) {
+        if (16 * i >= vd) break;
+        acc[i] += s0 ? w.x * x[i].x : 0.f;
+        acc[i] += s1 ? w.y * x[i].y : 0.f;
+        acc[i] += s2 ? w.z * x[i].z : 0.f;
+        acc[i] += s3 ? w.w * x[i].w : 0.f;
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+#pragma unroll
+    for (int o = 1; o < 4; o <<= 1) acc[i] += __shfl_xor(acc[i], o, QVL_WAVE);
+    if (quad == 0) part[wave][16 * i + chan] = acc[i];
+  }
+  if (lane == 0) {
+    part_m[wave] = m;
+    part_l[wave] = l;
+  }
+  __syncthreads();
+  const float sk = sinks ? sinks[h] : -INFINITY;
+  float top = sk;
+#pragma unroll
+  for (int w = 0; w < ATTN_WAVES; ++w) top = fmaxf(top, part_m[w]);
+  float factor[ATTN_WAVES], total = 0.f;
+#pragma unroll
+  for (int w = 0; w < ATTN_WAVES; ++w) {
+    factor[w] = w < blocks ? expf(part_m[w] - top) : 0.f;
+    total += part_l[w] * factor[w];
+  }
+  if (sinks) total += expf(sk - top);
+  const float inv = 1.0f / total;
+  auto value = [&](int d) {
+    float v = 0.f;
+#pragma unroll
+    for (int w = 0; w < ATTN_WAVES; ++w) v += part[w][d] * factor[w];
+    return v * inv;
+  };
+  T* o = out + ((size_t)n * nh + h) * vd;
+  const int half = vd >> 1;
+  const float2* tn = turn + (size_t)n * half;
+  for (int d = threadIdx.x; d < vd; d += 64 * ATTN_WAVES) {
+    const float v = value(d);
+    if (turn) {
+      const bool one = turn_pairs ? !(d & 1) : d < half;
+      const float2 t = tn[turn_pairs ? d >> 1 : (one ? d : d - half)];
+      const float w = value(turn_pairs ? d ^ 1 : (one ? d + half : d - half));
+      stf<T>(o + d, one ? v * t.x + w * t.y : v * t.x - w * t.y);
+    } else {
+      stf<T>(o + d, v);
+    }
+  }
+}
+
 extern "C" int qvl_attn_generic(const void* q, const void* kc, const void* vc, const void* block_table,
                                 int table_width, const void* token_req, const void* token_seqpos, void* out, int N,
                                 int nh, int nkv, int hd, int vd, int ps, int window, int keep_first, int chunk,
@@ -121,6 +272,20 @@ extern "C" int qvl_attn_generic(const void* q, const void* kc, const void* vc, c
     return QVL_ERR_SHAPE;
   if (hd > ATTN_MAX_HD || vd > ATTN_MAX_HD || nh > 65535) return QVL_ERR_LIMIT;
   const dim3 grid(N, nh);
+  const bool vec = hd % 4 == 0 && ps % 4 == 0 && ((uintptr_t)kc % 16) == 0 && ((uintptr_t)vc % 16) == 0;
+#define VEC(T, CH)                                                                                                       \
+  hipLaunchKernelGGL((attn_generic_vec_kernel<T, CH>), grid, dim3(64 * ATTN_WAVES), 0, stream, (const T*)q, (const T*)kc,  \
+                     (const T*)vc, (const int*)block_table, table_width, (const int*)token_req, (const int*)token_seqpos, \
+                     (T*)out, nh, nkv, hd, vd, ps, window, keep_first, chunk, scale, (const float*)sinks,                 \
+                     (const float2*)turn, turn_pairs)
+  if (vec && (dtype == 0 || dtype == 1)) {
+    if (dtype == 0 && vd <= 128) VEC(float, 8);
+    else if (dtype == 0) VEC(float, ATTN_MAX_HD / 16);
+    else if (vd <= 128) VEC(bf16_t, 8);
+    else VEC(bf16_t, ATTN_MAX_HD / 16);
+    return qvl_launch_status();
+  }
+#undef VEC
   if (dtype == 0)
     hipLaunchKernelGGL(attn_generic_kernel<float>, grid, dim3(64), 0, stream, (const float*)q, (const float*)kc,
                        (const float*)vc, (const int*)block_table, table_width, (const int*)token_req,

@@ -258,6 +258,44 @@ def test_paged_attention_generic(dtype, nq, nkv, hd, window, ps):
     assert torch.allclose(out.float().cpu(), c["want"], **tol), (out.float().cpu() - c["want"]).abs().max()
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("nq, nkv, hd, vd, ps, window, keep, chunk", [
+    (4, 2, 128, 128, 16, None, 0, None), (4, 2, 100, 132, 4, None, 0, None), (3, 1, 36, 20, 12, 150, 5, None),
+    (4, 4, 4, 512, 8, 64, 130, None), (2, 1, 64, 64, 16, None, 0, 130), (4, 2, 30, 24, 16, 150, 5, None), (4, 2, 32, 24, 6, None, 0, 90)])
+def test_generic_attention_of_long_contexts(dtype, nq, nkv, hd, vd, ps, window, keep, chunk):
+    """More blocks of 64 keys than waves, blocks skipped between kept keys and a window, the last block short; head and page sizes the
+    wide loads take and do not take.  Every slot that a token does not see holds NaN."""
+    from qwen25vl_lite_amd.ops import kernels
+    torch.manual_seed(nq + hd + vd)
+    n, length = 5, 601
+    pages = (length + ps - 1) // ps
+    seen = torch.zeros(n, length, dtype=torch.bool)
+    at = [600, 300, 63, 64, 0]
+    for i, p in enumerate(at):
+        lo = max(0, p - window + 1) if window else 0
+        lo = max(lo, p - p % chunk) if chunk else lo
+        seen[i, lo:p + 1] = True
+        seen[i, :min(keep, lo)] = True
+    q, sinks = torch.randn(n, nq, hd).to(dtype), torch.randn(nq)
+    k, v = torch.randn(n, nkv, length, hd).to(dtype), torch.randn(n, nkv, length, vd).to(dtype)
+    kc = torch.full((n * pages, nkv, ps, hd), math.nan, dtype=dtype)
+    vc = torch.full((n * pages, nkv, vd, ps), math.nan, dtype=dtype)
+    table = torch.randperm(n * pages).view(n, pages).to(torch.int32)
+    for i in range(n):
+        for j in torch.nonzero(seen[i]).flatten().tolist():
+            kc[table[i, j // ps], :, j % ps] = k[i, :, j]
+            vc[table[i, j // ps], :, :, j % ps] = v[i, :, j]
+    got = kernels.paged_attention_generic(q.reshape(n, -1).cuda(), kc.cuda(), vc.cuda(), table.cuda(), torch.arange(n, dtype=torch.int32).cuda(),
+                                          torch.tensor(at, dtype=torch.int32).cuda(), nq, window, hd ** -0.5, keep_first=keep,
+                                          chunk=chunk, sinks=sinks.cuda())
+    per = nq // nkv
+    s = torch.einsum("nhd,nhtd->nht", q.double(), k.double().repeat_interleave(per, 1)) * hd ** -0.5
+    s = torch.cat([s.masked_fill(~seen[:, None], -math.inf), sinks.double().view(1, nq, 1).expand(n, nq, 1)], 2)
+    want = torch.einsum("nht,nhtd->nhd", torch.softmax(s, 2)[:, :, :length], v.double().repeat_interleave(per, 1)).reshape(n, -1)
+    tol = dict(atol=2e-5, rtol=1e-4) if dtype == torch.float32 else dict(atol=1.5e-2, rtol=2e-2)
+    assert torch.allclose(got.double().cpu(), want, **tol), (got.double().cpu() - want).abs().max()
+
+
 @pytest.mark.parametrize("split", ["tile", "tile_two_groups", "coop", "coop_split", "coop_split_two_kernels"])
 @pytest.mark.parametrize("nq, nkv, hd, window, ps", [(*s, 16) for s in ATTN_SHAPES if s[2] % 16 == 0]
                          + [s for s in PAGE_SIZES if s[2] % 16 == 0])
