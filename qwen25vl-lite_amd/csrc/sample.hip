@@ -17,13 +17,25 @@
 // would not fit 64 bits), which is finer than a float32 sum of them and lets the blocks add in any order.  One block a row that searched bit by bit, 32 passes for each
 // threshold, took 3.70 ms for 64 rows of 152,064 (greedy, top-p, top-k with top-p and penalties, min-p
 // in turn); these passes together take 113 us.
+//
+// Most rows need none of these passes: what their cuts leave is a short list.  Each 64 scores of a row have a
+// largest one; the k-th largest of those is no larger than the k-th largest score, and scores that far below the largest one that
+// all of a row's could not make up 1 - top_p never matter.  So one pass gathers what such a bound leaves (and adds up all
+// mass, where top-p needs it), and a block a row finds the thresholds among these few and draws, with the same sums.  Rows
+// whose list is longer than LIST, or whose list does not reach top-p, go the long way; the others' blocks there end at once.
+// The 64 rows above: 43 us in three kernels, all of it reading and finding, the passes 117 in nine.
 #include "common.h"
+#include <cstddef>
 #include <type_traits>
 
 #define PIECE 4096          // scores a block owns in a pass over a row
 #define THREADS 256
 #define BINS 2048           // bins of a threshold's search: 11 bits of a score's key at a time
 #define CHUNKS 1024         // contiguous ranges of a row whose masses the draw adds one after the other
+#define GROUPS 16           // groups of 256 scores of a piece, whose largest are kept
+#define LIST 1024           // scores of a short list
+#define GUESS 384           // how many groups' largest scores top-p is expected to reach at most
+#define STEPS 2048          // steps of 1/64 below a row's largest score that bounds are told apart by; the last one is open
 
 struct RowParams {
   float temperature, top_p, min_p, u;
@@ -51,11 +63,17 @@ struct Threshold {
 struct RowScratch {
   Threshold found[2];
   float u;
-  int pad[3];
+  unsigned int listed;          // scores asked into the list (more than LIST: it is of no use)
+  int todo_row;                 // of the i-th row: the i-th of those that go the long way
+  int pad;
+  unsigned long long all_mass, pad2;
+  float list_score[LIST];
+  int list_index[LIST];
   unsigned int count[3][BINS];
   unsigned long long mass[3][BINS];
   float chunk_mass[CHUNKS];
 };
+static_assert(offsetof(RowScratch, chunk_mass) % 16 == 0 && sizeof(RowScratch) % 16 == 0, "the chunks' masses are read four at a time");
 
 __device__ __forceinline__ uint32_t order_key(float f) {
   uint32_t u = __float_as_uint(f);
@@ -77,6 +95,26 @@ struct Scores {
 __device__ __forceinline__ Scores scores_of(const RowParams& p, const float* logits, const float* scores, int m, int V) {
   const bool out = penalised(p);
   return Scores{(out ? scores : logits) + (size_t)m * V, out || p.temperature <= 0.f ? 1.f : p.temperature};
+}
+
+// Thread t's scores of a piece: number j is the piece's score piece_index(j, t), those beyond n the first one again.
+__device__ __forceinline__ int piece_index(int j, int tid) { return (j >> 2) * 4 * THREADS + 4 * tid + (j & 3); }
+__device__ __forceinline__ void load_piece(const float* at, int n, int V, float (&v)[PIECE / THREADS]) {
+  const int tid = threadIdx.x;
+  if (V % 4 == 0 && (uintptr_t)at % 16 == 0) {        // then a piece's end is a multiple of four, too
+#pragma unroll
+    for (int j = 0; j < PIECE / THREADS; j += 4) {
+      const int i = piece_index(j, tid);
+      const float4 x = *reinterpret_cast<const float4*>(at + (i < n ? i : 0));
+      v[j] = x.x; v[j + 1] = x.y; v[j + 2] = x.z; v[j + 3] = x.w;
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < PIECE / THREADS; ++j) {
+      const int i = piece_index(j, tid);
+      v[j] = at[i < n ? i : 0];
+    }
+  }
 }
 
 __device__ __forceinline__ void better(float& bv, int& bi, float ov, int oi) {
@@ -126,39 +164,39 @@ __device__ float first_uniform(uint32_t seed) {
 }
 
 // The first pass: a piece's largest score (of penalised rows the penalised and scaled scores, which are
-// written to `scores`), and empty bins for the searches.  With scratch there is one block more a row,
+// written to `scores`) and, of rows that draw, its groups' largest.  With scratch there is one block more a row,
 // which draws the row's uniform number.
 __global__ __launch_bounds__(THREADS) void sample_scan_kernel(const float* __restrict__ logits, float* __restrict__ scores,
                                                               const RowParams* __restrict__ params,
                                                               const int* __restrict__ prev_ids,
                                                               RowScratch* __restrict__ scratch,
-                                                              ArgmaxPart* __restrict__ parts, int V, int pieces) {
+                                                              ArgmaxPart* __restrict__ parts, float* __restrict__ groups,
+                                                              int* __restrict__ todo, int M, int V, int pieces) {
   __shared__ int seen[PIECE];     // how often each of the piece's tokens has been generated
   __shared__ float vals[THREADS / 64];
   __shared__ int idxs[THREADS / 64];
-  const int m = blockIdx.y, s = blockIdx.x, tid = threadIdx.x;
+  const int tid = threadIdx.x;
+  int at = blockIdx.x;
+  if (scratch) {
+    // the rows' own blocks come first: a seed's first number is a chain of 397 products
+    if (at < M) {
+      if (tid == 0) {
+        const RowParams p = params[at];
+        scratch[at].listed = 0u;
+        scratch[at].all_mass = 0ull;
+        if (at == 0) *todo = 0;
+        scratch[at].u = p.temperature > 0.f && p.seeded ? first_uniform(p.seed) : p.u;
+      }
+      return;
+    }
+    at -= M;
+  }
+  const int m = at / pieces, s = at - m * pieces;
   const RowParams p = params[m];
   const bool draws = p.temperature > 0.f;
-  if (scratch && draws) {
-    // empty bins: the blocks of the row share them out
-    const int step = gridDim.x * THREADS;
-    if (cuts_k(p, V))
-      for (int i = s * THREADS + tid; i < 3 * BINS; i += step) (&scratch[m].count[0][0])[i] = 0u;
-    if (cuts_p(p))
-      for (int i = s * THREADS + tid; i < 3 * BINS; i += step) (&scratch[m].mass[0][0])[i] = 0ull;
-  }
-  if (s == pieces) {
-    if (tid == 0) scratch[m].u = p.seeded ? first_uniform(p.seed) : p.u;
-    return;
-  }
-  const float* lg = logits + (size_t)m * V;
   const int lo = s * PIECE, n = min(PIECE, V - lo);
   float v[PIECE / THREADS];
-#pragma unroll
-  for (int j = 0; j < PIECE / THREADS; ++j) {
-    const int i = j * THREADS + tid;
-    v[j] = lg[lo + (i < n ? i : 0)];
-  }
+  load_piece(logits + (size_t)m * V + lo, n, V, v);
   if (penalised(p)) {
 #pragma unroll
     for (int j = 0; j < PIECE / THREADS; ++j) seen[j * THREADS + tid] = 0;
@@ -172,7 +210,7 @@ __global__ __launch_bounds__(THREADS) void sample_scan_kernel(const float* __res
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < PIECE / THREADS; ++j) {
-      const int count = seen[j * THREADS + tid];
+      const int count = seen[piece_index(j, tid)];
       if (count == 0) continue;
       float x = v[j];
       if (p.repetition != 1.f) x = x > 0.f ? x / p.repetition : x * p.repetition;
@@ -180,7 +218,7 @@ __global__ __launch_bounds__(THREADS) void sample_scan_kernel(const float* __res
     }
 #pragma unroll
     for (int j = 0; j < PIECE / THREADS; ++j) {
-      const int i = j * THREADS + tid;
+      const int i = piece_index(j, tid);
       if (draws) v[j] = v[j] / p.temperature;
       if (draws && i < n) scores[(size_t)m * V + lo + i] = v[j];
     }
@@ -192,8 +230,14 @@ __global__ __launch_bounds__(THREADS) void sample_scan_kernel(const float* __res
   int bi = V;
 #pragma unroll
   for (int j = 0; j < PIECE / THREADS; ++j) {
-    const int i = j * THREADS + tid;
+    const int i = piece_index(j, tid);
     if (i < n && v[j] > bv) { bv = v[j]; bi = lo + i; }   // indices rise within a thread: the first of equals stays
+  }
+  if (scratch && draws) {
+    float top = fmaxf(bv, __shfl_xor(bv, 1, QVL_WAVE));
+#pragma unroll
+    for (int o = 2; o < THREADS / GROUPS; o <<= 1) top = fmaxf(top, __shfl_xor(top, o, QVL_WAVE));
+    if (tid % (THREADS / GROUPS) == 0) groups[((size_t)m * pieces + s) * GROUPS + tid / (THREADS / GROUPS)] = top;
   }
   wave_argmax(bv, bi);
   if ((tid & 63) == 0) { vals[tid >> 6] = bv; idxs[tid >> 6] = bi; }
@@ -206,6 +250,334 @@ __global__ __launch_bounds__(THREADS) void sample_scan_kernel(const float* __res
 
 // `one`: the largest score's mass, a power of two
 __device__ __forceinline__ unsigned long long mass_of(float e, float one) { return e > 0.f ? (unsigned long long)(e * one) : 0ull; }
+
+// The sum of the threads before this one (whole block; one place for each wave in s_wave).
+template <typename T>
+__device__ __forceinline__ T sum_before(T own, T* s_wave) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  T sum = own;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const T x = __shfl_up(sum, o, QVL_WAVE);
+    if (lane >= o) sum += x;
+  }
+  if (lane == 63) s_wave[wave] = sum;
+  __syncthreads();
+  sum -= own;
+  for (int w = 0; w < wave; ++w) sum += s_wave[w];
+  return sum;
+}
+
+// How far below the row's largest score a score is, in steps.
+__device__ __forceinline__ int step_of(float x, float mx) { return (int)fminf((mx - x) * 64.f, (float)(STEPS - 1)); }
+
+// Gathers the scores that the row's cuts can leave, and all mass where top-p alone cuts.
+__global__ __launch_bounds__(THREADS) void sample_list_kernel(const float* __restrict__ logits, const float* __restrict__ scores,
+                                                              const RowParams* __restrict__ params,
+                                                              RowScratch* __restrict__ scratch,
+                                                              const ArgmaxPart* __restrict__ parts,
+                                                              const float* __restrict__ groups, int V, int pieces, float one) {
+  __shared__ unsigned int steps[STEPS], sums[THREADS / 64];
+  __shared__ unsigned long long mass[THREADS / 64];
+  __shared__ ArgmaxPart s_best;
+  __shared__ int s_k, s_p;
+  __shared__ unsigned int s_count, s_base;
+  const int m = blockIdx.y, s = blockIdx.x, tid = threadIdx.x;
+  const RowParams p = params[m];
+  if (p.temperature <= 0.f) return;
+  RowScratch& r = scratch[m];
+  const Scores score = scores_of(p, logits, scores, m, V);
+  const int lo = s * PIECE, n = min(PIECE, V - lo);
+  float v[PIECE / THREADS];
+  load_piece(score.at + lo, n, V, v);
+  const bool k_cut = cuts_k(p, V), p_cut = cuts_p(p);
+  const float mx = row_argmax(parts, m, pieces, V, &s_best).value;
+  int bound = STEPS - 1;          // scores up to this many steps below the largest go into the list
+  if (p.min_p > 0.f) bound = min(bound, (int)fminf(-logf(p.min_p) * 64.f + 2.f, (float)(STEPS - 1)));
+  if (k_cut || (p_cut && !(p.min_p > 0.f))) {
+    for (int i = tid; i < STEPS; i += THREADS) steps[i] = 0u;
+    if (tid == 0) s_k = s_p = STEPS - 1;
+    __syncthreads();
+    const float* top = groups + (size_t)m * pieces * GROUPS;
+    for (int i = tid; i < pieces * GROUPS; i += THREADS) {
+      const float x = top[i];
+      if (x > -INFINITY) atomicAdd(&steps[step_of(x, mx)], 1u);
+    }
+    __syncthreads();
+    constexpr int PER = STEPS / THREADS;
+    unsigned int own[PER], sum = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      own[i] = steps[tid * PER + i];
+      sum += own[i];
+    }
+    const unsigned int k = (unsigned int)p.top_k;
+    unsigned int before = sum_before(sum, sums);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      if (before < k && before + own[i] >= k) s_k = tid * PER + i;
+      if (before < GUESS && before + own[i] >= GUESS) s_p = tid * PER + i;
+      before += own[i];
+    }
+    __syncthreads();
+    if (k_cut) bound = min(bound, s_k);
+    else bound = min(s_p, (int)fminf(logf((float)V / fmaxf(1.f - p.top_p, 1e-7f)) * 64.f + 2.f, (float)(STEPS - 1)));
+  }
+  if (bound == STEPS - 1 && V > LIST) {        // every score
+    if (s == 0 && tid == 0) atomicAdd(&r.listed, LIST + 1u);
+    return;
+  }
+  if (tid == 0) s_count = 0u;
+  __syncthreads();
+  // a score that is no number, or none that is: the long way
+  bool odd = !(fabsf(mx) < INFINITY);
+  const bool sum_all = p_cut && !k_cut && !(p.min_p > 0.f);
+  unsigned long long own_mass = 0;
+  unsigned int place[PIECE / THREADS];
+#pragma unroll
+  for (int j = 0; j < PIECE / THREADS; ++j) {
+    place[j] = 0xffffffffu;
+    if (piece_index(j, tid) >= n) continue;
+    v[j] = v[j] / score.temperature;
+    odd |= v[j] != v[j];
+    if (sum_all) own_mass += mass_of(expf(v[j] - mx), one);
+    if (step_of(v[j], mx) <= bound) place[j] = atomicAdd(&s_count, 1u);
+  }
+  if (odd) atomicAdd(&s_count, LIST + 1u);
+  if (sum_all) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) own_mass += __shfl_xor(own_mass, o, QVL_WAVE);
+    if ((tid & 63) == 0) mass[tid >> 6] = own_mass;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    s_base = s_count ? atomicAdd(&r.listed, s_count < LIST + 1u ? s_count : LIST + 1u) : 0u;
+    if (sum_all) {
+      unsigned long long sum = 0;
+      for (int w = 0; w < THREADS / 64; ++w) sum += mass[w];
+      if (sum) atomicAdd(&r.all_mass, sum);
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < PIECE / THREADS; ++j) {
+    if (place[j] == 0xffffffffu) continue;
+    const unsigned int at = s_base + place[j];
+    if (at < LIST) {
+      r.list_score[at] = v[j];
+      r.list_index[at] = lo + piece_index(j, tid);
+    }
+  }
+}
+
+// A row's token from its list, by the rules of the long way: thresholds by the keys' bits, masses of chunks added from their first
+// index on, chunks one after the other (chunks without mass add nothing, so those of the list are enough).  A threshold is found
+// by steps below the largest score first, then among the scores of its step.
+__global__ __launch_bounds__(THREADS) void sample_short_kernel(const RowParams* __restrict__ params,
+                                                               RowScratch* __restrict__ scratch,
+                                                               const ArgmaxPart* __restrict__ parts, int* __restrict__ out,
+                                                               int* __restrict__ todo, int V, int pieces, float one) {
+  constexpr int PER = LIST / THREADS, OWN = STEPS / THREADS;
+  __shared__ unsigned long long steps[STEPS], s_sum[THREADS / 64], s_above;
+  __shared__ unsigned long long in_mass[LIST];        // the threshold's step: its scores' masses (or ones) and keys
+  __shared__ uint32_t in_key[LIST], s_cut;
+  __shared__ __attribute__((aligned(16))) int index[LIST], kept_index[LIST];
+  __shared__ float weight[LIST], kept_weight[LIST], run_mass[LIST], run_before[LIST];
+  __shared__ int run_at[LIST], s_wave[THREADS / 64], s_step, s_in, s_kept, s_runs, s_chosen, s_last;
+  __shared__ float s_z;
+  __shared__ ArgmaxPart s_best;
+  const int m = blockIdx.x, tid = threadIdx.x;
+  const RowParams p = params[m];
+  const ArgmaxPart best = row_argmax(parts, m, pieces, V, &s_best);
+  if (p.temperature <= 0.f) {
+    if (tid == 0) out[m] = best.index < V ? best.index : 0;
+    return;
+  }
+  RowScratch& r = scratch[m];
+  const bool k_cut = cuts_k(p, V), p_cut = cuts_p(p);
+  const float mx = best.value;
+  const int n = r.listed <= LIST ? (int)r.listed : 0;       // (0: the long way; a list has the largest score at least)
+  float w[PER];
+  uint32_t key[PER];
+  int ix[PER], st[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int at = i * THREADS + tid;
+    const float x = at < n ? r.list_score[at] : -INFINITY;
+    ix[i] = at < n ? r.list_index[at] : 0;
+    key[i] = order_key(x);
+    st[i] = at < n ? step_of(x, mx) : -1;
+    w[i] = at < n ? expf(x - mx) : 0.f;
+    if (p.min_p > 0.f && w[i] < p.min_p) w[i] = 0.f;
+  }
+  if (tid == 0) s_kept = s_runs = s_last = 0;
+  // the key at which the parts of the scores from the largest down reach the target: false if they do not
+  auto threshold = [&](auto part, unsigned long long target) -> bool {
+    for (int i = tid; i < STEPS; i += THREADS) steps[i] = 0ull;
+    if (tid == 0) {
+      s_step = -1;
+      s_in = 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const unsigned long long x = part(i);
+      if (st[i] >= 0 && x) atomicAdd(&steps[st[i]], x);
+    }
+    __syncthreads();
+    unsigned long long own[OWN], sum = 0;
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+      own[i] = steps[tid * OWN + i];
+      sum += own[i];
+    }
+    unsigned long long before = sum_before(sum, s_sum);
+#pragma unroll
+    for (int i = 0; i < OWN; ++i) {
+      if (before < target && before + own[i] >= target) {
+        s_step = tid * OWN + i;
+        s_above = before;
+      }
+      before += own[i];
+    }
+    __syncthreads();
+    if (s_step < 0) return false;
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+      if (st[i] == s_step) {
+        const int at = atomicAdd(&s_in, 1);
+        in_key[at] = key[i];
+        in_mass[at] = part(i);
+      }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      if (st[i] != s_step) continue;
+      unsigned long long above = s_above, reach = s_above;
+      for (int j = 0; j < s_in; ++j) {
+        above += in_key[j] > key[i] ? in_mass[j] : 0ull;
+        reach += in_key[j] >= key[i] ? in_mass[j] : 0ull;
+      }
+      if (above < target && reach >= target) s_cut = key[i];
+    }
+    __syncthreads();
+    return true;
+  };
+  if (k_cut && n > 0) {
+    // (fewer than k in the list: the others have no mass by min-p)
+    if (threshold([&](int i) { return 1ull; }, (unsigned long long)p.top_k)) {
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+        if (key[i] < s_cut) w[i] = 0.f;
+    }
+    __syncthreads();
+  }
+  bool done = n > 0;
+  if (p_cut && done) {
+    // the mass of what top-k and min-p leave; without them every score has a part
+    unsigned long long all = r.all_mass;
+    if (k_cut || p.min_p > 0.f) {
+      unsigned long long sum = 0;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) sum += mass_of(w[i], one);
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, QVL_WAVE);
+      if ((tid & 63) == 0) s_sum[tid >> 6] = sum;
+      __syncthreads();
+      all = 0;
+      for (int i = 0; i < THREADS / 64; ++i) all += s_sum[i];
+      __syncthreads();
+    }
+    done = threshold([&](int i) { return mass_of(w[i], one); }, max(1ull, (unsigned long long)ceil((double)p.top_p * (double)all)));
+    if (done) {
+#pragma unroll
+      for (int i = 0; i < PER; ++i)
+        if (key[i] < s_cut) w[i] = 0.f;
+    }
+  }
+  if (!done) {
+    for (int i = tid; i < 3 * BINS; i += THREADS) {
+      (&r.count[0][0])[i] = 0u;
+      (&r.mass[0][0])[i] = 0ull;
+    }
+    if (tid == 0) scratch[atomicAdd(todo, 1)].todo_row = m;
+    return;
+  }
+  // what is left, in the order of the indices
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < PER; ++i)
+    if (w[i] > 0.f) {
+      const int at = atomicAdd(&s_kept, 1);
+      kept_index[at] = ix[i];
+      kept_weight[at] = w[i];
+    }
+  __syncthreads();
+  const int kept = s_kept;
+  for (int i = tid; i < kept; i += THREADS) {
+    const int own = kept_index[i];
+    int rank = 0;
+#pragma unroll 8
+    for (int j = 0; j < kept; ++j) rank += kept_index[j] < own;
+    index[rank] = own;
+    weight[rank] = kept_weight[i];
+  }
+  if (tid == 0) s_chosen = LIST;
+  __syncthreads();
+  // the runs of one chunk, each added by the thread of its first score
+  const int C = (V + CHUNKS - 1) / CHUNKS;
+  for (int i = 0; i * THREADS < kept; ++i) {
+    const int at = i * THREADS + tid;
+    const bool first = at < kept && (at == 0 || index[at] / C != index[at - 1] / C);
+    const unsigned long long votes = __ballot(first);
+    if ((tid & 63) == 0) s_wave[tid >> 6] = __popcll(votes);
+    __syncthreads();
+    int before = s_runs;
+    for (int x = 0; x < (tid >> 6); ++x) before += s_wave[x];
+    before += __popcll(votes & ((1ull << (tid & 63)) - 1ull));
+    if (first) {
+      const int chunk = index[at] / C;
+      float acc = 0.f;
+      for (int j = at; j < kept && index[j] / C == chunk; ++j) acc += weight[j];
+      run_at[before] = at;
+      run_mass[before] = acc;
+    }
+    __syncthreads();
+    if (tid == 0)
+      for (int x = 0; x < THREADS / 64; ++x) s_runs += s_wave[x];
+    __syncthreads();
+  }
+  const int runs = s_runs;
+  if (tid == 0) {
+    float acc = 0.f;
+#pragma unroll 8
+    for (int t = 0; t < runs; ++t) {
+      run_before[t] = acc;
+      acc += run_mass[t];
+    }
+    s_z = acc;
+  }
+  __syncthreads();
+  const float aim = r.u * s_z;
+  for (int t = tid; t < runs; t += THREADS) {
+    if (run_before[t] + run_mass[t] > aim) atomicMin(&s_chosen, t);
+    atomicMax(&s_last, t);
+  }
+  __syncthreads();
+  if (tid == 0) {
+    const bool found = s_chosen < LIST;
+    const int t = found ? s_chosen : s_last, from = run_at[t], to = t + 1 < runs ? run_at[t + 1] : kept;
+    const float pick = found ? aim - run_before[t] : INFINITY;
+    float acc = 0.f;
+    int token = index[from];
+    for (int j = from; j < to; ++j) {
+      token = index[j];
+      acc += weight[j];
+      if (acc > pick) break;
+    }
+    out[m] = token;
+  }
+}
 
 // The highest of the bins at which the sum of the bins from the top down reaches `target` (the lowest
 // bin if none does), and what the bins above it bring.  Whole block; T the bins' type.
@@ -312,25 +684,23 @@ template <bool MASS>
 __global__ __launch_bounds__(THREADS) void sample_bins_kernel(const float* __restrict__ logits, const float* __restrict__ scores,
                                                               const RowParams* __restrict__ params,
                                                               RowScratch* __restrict__ scratch,
-                                                              const ArgmaxPart* __restrict__ parts, int V, int pieces,
+                                                              const ArgmaxPart* __restrict__ parts,
+                                                              const int* __restrict__ todo, int V, int pieces,
                                                               int level, float one) {
   typedef typename std::conditional<MASS, unsigned long long, unsigned int>::type bin_t;
   __shared__ bin_t bins[BINS];
   __shared__ unsigned long long s_sum[THREADS], s_above;
   __shared__ int s_bin;
   __shared__ ArgmaxPart s_best;
-  const int m = blockIdx.y, s = blockIdx.x, tid = threadIdx.x;
+  if ((int)blockIdx.y >= *todo) return;
+  const int m = scratch[blockIdx.y].todo_row, s = blockIdx.x, tid = threadIdx.x;
   const RowParams p = params[m];
   if (!(MASS ? cuts_p(p) : cuts_k(p, V))) return;
   RowScratch& r = scratch[m];
   const Scores score = scores_of(p, logits, scores, m, V);
   const int lo = s * PIECE, n = min(PIECE, V - lo);
   float v[PIECE / THREADS];
-#pragma unroll
-  for (int j = 0; j < PIECE / THREADS; ++j) {
-    const int i = j * THREADS + tid;
-    v[j] = score.at[lo + (i < n ? i : 0)];
-  }
+  load_piece(score.at + lo, n, V, v);
   for (int i = tid; i < BINS; i += THREADS) bins[i] = 0;
   const float mx = MASS ? row_argmax(parts, m, pieces, V, &s_best).value : 0.f;
   uint32_t key;
@@ -343,7 +713,7 @@ __global__ __launch_bounds__(THREADS) void sample_bins_kernel(const float* __res
   const uint32_t fixed = level == 0 ? 0u : (0xffffffffu << level_shift(level - 1)), low = level == 2 ? 0x3ffu : 0x7ffu;
 #pragma unroll
   for (int j = 0; j < PIECE / THREADS; ++j) {
-    if (j * THREADS + tid >= n) break;
+    if (piece_index(j, tid) >= n) continue;
     const float x = v[j] / score.temperature;
     const uint32_t k = order_key(x);
     if ((k & fixed) != key) continue;
@@ -368,14 +738,15 @@ __global__ __launch_bounds__(THREADS) void sample_bins_kernel(const float* __res
 __global__ __launch_bounds__(THREADS) void sample_chunks_kernel(const float* __restrict__ logits, const float* __restrict__ scores,
                                                                 const RowParams* __restrict__ params,
                                                                 RowScratch* __restrict__ scratch,
-                                                                const ArgmaxPart* __restrict__ parts, int V, int pieces) {
+                                                                const ArgmaxPart* __restrict__ parts,
+                                                                const int* __restrict__ todo, int V, int pieces) {
   __shared__ float tile[CHUNKS_A_BLOCK][65];
   __shared__ unsigned long long s_sum[THREADS], s_above;
   __shared__ int s_bin;
   __shared__ ArgmaxPart s_best;
-  const int m = blockIdx.y, tid = threadIdx.x;
+  if ((int)blockIdx.y >= *todo) return;
+  const int m = scratch[blockIdx.y].todo_row, tid = threadIdx.x;
   const RowParams p = params[m];
-  if (p.temperature <= 0.f) return;
   RowScratch& r = scratch[m];
   const Scores score = scores_of(p, logits, scores, m, V);
   const float mx = row_argmax(parts, m, pieces, V, &s_best).value;
@@ -417,17 +788,22 @@ __global__ __launch_bounds__(THREADS) void sample_pick_kernel(const float* __res
                                                               const RowParams* __restrict__ params,
                                                               RowScratch* __restrict__ scratch,
                                                               const ArgmaxPart* __restrict__ parts, int* __restrict__ out,
-                                                              int V, int pieces) {
+                                                              const int* __restrict__ todo, int V, int pieces) {
   __shared__ __attribute__((aligned(16))) float sums[CHUNKS];
   __shared__ float prefix[CHUNKS];
   __shared__ __attribute__((aligned(16))) float tile[THREADS];
   __shared__ ArgmaxPart s_best;
   __shared__ int s_chunk, s_last, s_token;
   __shared__ float s_z;
-  const int m = blockIdx.x, tid = threadIdx.x;
+  int m = blockIdx.x;
+  const int tid = threadIdx.x;
+  if (scratch) {
+    if ((int)blockIdx.x >= *todo) return;
+    m = scratch[blockIdx.x].todo_row;
+  }
   const RowParams p = params[m];
   const ArgmaxPart best = row_argmax(parts, m, pieces, V, &s_best);
-  if (p.temperature <= 0.f) {
+  if (!scratch) {                      // no row draws
     if (tid == 0) out[m] = best.index < V ? best.index : 0;
     return;
   }
@@ -503,38 +879,53 @@ __global__ __launch_bounds__(THREADS) void sample_pick_kernel(const float* __res
 static int pieces_of(int V) { return (V + PIECE - 1) / PIECE; }
 
 // Room a row needs: in `parts` always, in `scratch` if any row draws.
-extern "C" long long qvl_sample_parts_bytes(int V) { return (long long)pieces_of(V) * (long long)sizeof(ArgmaxPart); }
+extern "C" long long qvl_sample_parts_bytes(int V) { return (long long)pieces_of(V) * (long long)(sizeof(ArgmaxPart) + GROUPS * sizeof(float)); }
 extern "C" long long qvl_sample_scratch_bytes() { return (long long)sizeof(RowScratch); }
 extern "C" int qvl_sample_params_size() { return (int)sizeof(RowParams); }
 
 // logits: float32 [M, V].  scores: as large, written for rows that draw with penalties (null if there are none).
 // scratch: M * qvl_sample_scratch_bytes() bytes on a 16-byte boundary, null if no row draws.  parts: M * qvl_sample_parts_bytes(V).
+// out: the rows' tokens, and behind them, if rows draw, how many rows go the long way.
 // top_k, top_p: whether any row has that cut (the passes for it are left out otherwise).
+// ways: 1 the short way, after which out[M] rows have no token yet; 2 the long way for these, with all buffers as the short
+// one left them; 3 both.
 extern "C" int qvl_sample_rows(const void* logits, void* scores, const void* params, const void* prev_ids, void* scratch,
-                               void* parts, void* out, int M, int V, int top_k, int top_p, hipStream_t stream) {
+                               void* parts, void* out, int M, int V, int top_k, int top_p, int ways, hipStream_t stream) {
   if (M <= 0) return QVL_OK;
   if (V <= 0 || !logits || !params || !prev_ids || !parts || !out) return QVL_ERR_SHAPE;
-  if (((uintptr_t)scratch % 16) != 0) return QVL_ERR_SHAPE;
-  if (M > 65535) return QVL_ERR_LIMIT;
+  if (((uintptr_t)scratch % 16) != 0 || ways < 1 || ways > 3) return QVL_ERR_SHAPE;
+  const int pieces = pieces_of(V);
+  if (M > 65535 || (long long)M * (pieces + 1) > 0x7fffffffll) return QVL_ERR_LIMIT;
   const float* lg = (const float*)logits;
   float* sc = (float*)scores;
   const RowParams* rp = (const RowParams*)params;
   RowScratch* rs = (RowScratch*)scratch;
   ArgmaxPart* ap = (ArgmaxPart*)parts;
-  const int pieces = pieces_of(V);
+  float* groups = (float*)(ap + (size_t)M * pieces);
+  int* ids = (int*)out;
+  int* todo = ids + M;
   float one = 1099511627776.0f;                                   // 2^40
   for (long long v = 1ll << 23; v < V; v <<= 1) one *= 0.5f;      // the sum of a row's masses fits 63 bits
-  hipLaunchKernelGGL(sample_scan_kernel, dim3(pieces + (scratch ? 1 : 0), M), dim3(THREADS), 0, stream, lg, sc, rp,
-                     (const int*)prev_ids, rs, ap, V, pieces);
-  if (scratch) {
+  const dim3 block(THREADS);
+  if (ways & 1) {
+    hipLaunchKernelGGL(sample_scan_kernel, dim3(M * pieces + (scratch ? M : 0)), block, 0, stream, lg, sc, rp, (const int*)prev_ids, rs, ap,
+                       groups, todo, M, V, pieces);
+    if (scratch) {
+      hipLaunchKernelGGL(sample_list_kernel, dim3(pieces, M), block, 0, stream, lg, sc, rp, rs, ap, groups, V, pieces, one);
+      hipLaunchKernelGGL(sample_short_kernel, dim3(M), block, 0, stream, rp, rs, ap, ids, todo, V, pieces, one);
+    } else {
+      hipLaunchKernelGGL(sample_pick_kernel, dim3(M), block, 0, stream, lg, sc, rp, rs, ap, ids, todo, V, pieces);
+    }
+  }
+  if ((ways & 2) && scratch) {
     if (top_k)
       for (int level = 0; level < 3; ++level)
-        hipLaunchKernelGGL(sample_bins_kernel<false>, dim3(pieces, M), dim3(THREADS), 0, stream, lg, sc, rp, rs, ap, V, pieces, level, one);
+        hipLaunchKernelGGL(sample_bins_kernel<false>, dim3(pieces, M), block, 0, stream, lg, sc, rp, rs, ap, todo, V, pieces, level, one);
     if (top_p)
       for (int level = 0; level < 3; ++level)
-        hipLaunchKernelGGL(sample_bins_kernel<true>, dim3(pieces, M), dim3(THREADS), 0, stream, lg, sc, rp, rs, ap, V, pieces, level, one);
-    hipLaunchKernelGGL(sample_chunks_kernel, dim3(CHUNKS / CHUNKS_A_BLOCK, M), dim3(THREADS), 0, stream, lg, sc, rp, rs, ap, V, pieces);
+        hipLaunchKernelGGL(sample_bins_kernel<true>, dim3(pieces, M), block, 0, stream, lg, sc, rp, rs, ap, todo, V, pieces, level, one);
+    hipLaunchKernelGGL(sample_chunks_kernel, dim3(CHUNKS / CHUNKS_A_BLOCK, M), block, 0, stream, lg, sc, rp, rs, ap, todo, V, pieces);
+    hipLaunchKernelGGL(sample_pick_kernel, dim3(M), block, 0, stream, lg, sc, rp, rs, ap, ids, todo, V, pieces);
   }
-  hipLaunchKernelGGL(sample_pick_kernel, dim3(M), dim3(THREADS), 0, stream, lg, sc, rp, rs, ap, (int*)out, V, pieces);
   return qvl_launch_status();
 }

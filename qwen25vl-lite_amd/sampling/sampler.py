@@ -118,14 +118,17 @@ def sample_rows(logits: torch.Tensor, params: Sequence[SamplingParams], prev_ids
     ``prev_ids[m]`` are the tokens request ``m`` has generated so far (for the penalties) and
     ``steps[m]`` their number (for the seed rule).  ``uniforms`` overrides the random numbers.
     """
-    pending = sample_rows_begin(logits, params, prev_ids, steps, uniforms)
-    return pending.result() if pending is not None else []
+    return _sample_rows(logits, params, prev_ids, steps, uniforms, wait=True) or []
 
 
 def sample_rows_begin(logits: torch.Tensor, params: Sequence[SamplingParams], prev_ids: Sequence[Sequence[int]],
                       steps: Sequence[int], uniforms: Optional[Sequence[float]] = None) -> Optional[PendingSample]:
     """Queue the sampling of :func:`sample_rows` and the copy of its ids to the host; nothing is
     waited for.  None for no rows."""
+    return _sample_rows(logits, params, prev_ids, steps, uniforms, wait=False)
+
+
+def _sample_rows(logits, params, prev_ids, steps, uniforms, wait: bool):
     if not logits.is_cuda:
         raise KernelError("sampling has no CPU path: logits must be on the GPU")
     if logits.dtype != torch.float32 or logits.dim() != 2 or not logits.is_contiguous():
@@ -142,7 +145,7 @@ def sample_rows_begin(logits: torch.Tensor, params: Sequence[SamplingParams], pr
             and first.frequency_penalty == 0.0 and all(p is first or p == first for p in params)):
         # one greedy setting for the whole batch (the usual decode step): fill the rows at once
         rows[:] = (first.temperature, first.top_p, first.min_p, 0.0, 1.0, 0.0, 0.0, first.top_k if first.top_k else -1, 0, 0, 0, 0)
-        return _launch(logits, rows, flat)
+        return _launch(logits, rows, flat, wait)
     filled = []
     for i, p in enumerate(params):
         need_prev = p.repetition_penalty != 1.0 or p.presence_penalty != 0.0 or p.frequency_penalty != 0.0
@@ -161,7 +164,7 @@ def sample_rows_begin(logits: torch.Tensor, params: Sequence[SamplingParams], pr
         filled.append((p.temperature, p.top_p, p.min_p, u, p.repetition_penalty, p.presence_penalty, p.frequency_penalty,
                        p.top_k if p.top_k else -1, begin, len(flat), word, seeded))
     rows[:] = filled
-    return _launch(logits, rows, flat)
+    return _launch(logits, rows, flat, wait)
 
 
 def sample_slots_begin(logits: torch.Tensor, records, slots: Sequence[int], prev_ids: Sequence[Sequence[int]],
@@ -203,11 +206,15 @@ def sample_slots_begin(logits: torch.Tensor, records, slots: Sequence[int], prev
     return _launch(logits, rows, flat)
 
 
-def _launch(logits: torch.Tensor, rows: np.ndarray, flat: List[int]) -> PendingSample:
-    """Send the rows' settings to the device and queue the sampler."""
+_SHORT, _LONG = 1, 2      # the kernel's ways to a row's token
+
+
+def _launch(logits: torch.Tensor, rows: np.ndarray, flat: List[int], wait: bool = False):
+    """Send the rows' settings to the device and queue the sampler: a :class:`PendingSample`.  With ``wait`` the ids,
+    and the passes for rows that the short way does not settle are queued only if there are any."""
     m, vocab = logits.shape
     c_ptr, c_int = ctypes.c_void_p, ctypes.c_int
-    fn = _fn("sample", "qvl_sample_rows", [c_ptr] * 7 + [c_int] * 4 + [c_ptr])
+    fn = _fn("sample", "qvl_sample_rows", [c_ptr] * 7 + [c_int] * 5 + [c_ptr])
     parts_bytes = _fn("sample", "qvl_sample_parts_bytes", [c_int], restype=ctypes.c_longlong)
     dev = logits.device
     draws = rows["temperature"] > 0
@@ -226,8 +233,19 @@ def _launch(logits: torch.Tensor, rows: np.ndarray, flat: List[int]) -> PendingS
             top_k = int((draws & (rows["top_k"] > 0) & (rows["top_k"] < vocab)).any())
             top_p = int((draws & (rows["top_p"] < 1.0)).any())
         parts = torch.empty(m * parts_bytes(vocab), dtype=torch.uint8, device=dev)
-        out = torch.empty(m, dtype=torch.int32, device=dev)
-        _check(fn(logits.data_ptr(), None if scores is None else scores.data_ptr(), buf.data_ptr(),
-                  buf[n_row_words:].data_ptr(), None if scratch is None else scratch.data_ptr(), parts.data_ptr(),
-                  out.data_ptr(), m, vocab, top_k, top_p, _stream()), "sample_rows")
-        return PendingSample(out)
+        out = torch.empty(m + 1, dtype=torch.int32, device=dev)      # the ids, and how many rows go the long way
+
+        def queue(ways):
+            _check(fn(logits.data_ptr(), None if scores is None else scores.data_ptr(), buf.data_ptr(),
+                      buf.data_ptr() + 4 * n_row_words, None if scratch is None else scratch.data_ptr(), parts.data_ptr(),
+                      out.data_ptr(), m, vocab, top_k, top_p, ways, _stream()), "sample_rows")
+        if not wait or scratch is None:
+            queue(_SHORT | _LONG)
+            pending = PendingSample(out[:m])
+            return pending.result() if wait else pending
+        queue(_SHORT)
+        ids = PendingSample(out).result()
+        if ids.pop():
+            queue(_LONG)
+            ids = PendingSample(out[:m]).result()
+        return ids

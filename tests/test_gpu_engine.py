@@ -537,6 +537,54 @@ def test_sampler_keeps_the_most_likely_token_at_any_top_p(top_p):
         assert sample_rows(logits.cuda(), params, [[]] * 6, [0] * 6, uniforms=[u] * 6) == logits.argmax(-1).tolist()
 
 
+@pytest.mark.parametrize("vocab", [1000, 5003, 152064, 151937])
+def test_sampler_of_lists_and_of_whole_rows(vocab):
+    """Rows whose cuts leave a short list beside rows that keep more than one holds, or whose list does not reach top-p
+    (flat rows, ties of thousands, values that are no number): the same tokens as float64 gives, queued at once
+    or waited for."""
+    from qwen25vl_lite_amd.sampling import SamplingParams
+    from qwen25vl_lite_amd.sampling.sampler import sample_rows, sample_rows_begin
+
+    g = torch.Generator().manual_seed(vocab)
+    kinds = [dict(temperature=0.7, top_p=0.9), dict(temperature=1.0, top_k=50, top_p=0.95, frequency_penalty=0.1),
+             dict(temperature=0.8, min_p=0.05), dict(temperature=4.0, top_p=0.97), dict(temperature=1.0), dict(temperature=1.0, top_k=900),
+             dict(temperature=1.0, min_p=1e-6, top_p=0.99), dict(temperature=0.0), dict(temperature=1.0, top_k=7), dict(temperature=0.5, top_k=300, min_p=0.1)]
+    params = [SamplingParams(**k) for k in kinds]
+    n = len(params)
+    for trial in range(3):
+        logits = torch.randn(n, vocab, generator=g) * 2
+        logits.scatter_add_(1, torch.randint(0, vocab, (n, 40), generator=g), torch.randn(n, 40, generator=g) * 3 + 7)
+        if trial == 1:
+            logits = (logits * 2).round() / 2            # thousands of equal scores at a cut
+        if trial == 2:
+            logits[:, 1::2] = float("-inf")
+        prev = [torch.randint(0, vocab, (20,), generator=g).tolist() for _ in params]
+        us = torch.rand(n, generator=g).tolist()
+        dev = logits.cuda()
+        got = sample_rows(dev, params, prev, [20] * n, uniforms=us)
+        queued = sample_rows_begin(dev, params, prev, [20] * n, uniforms=us)
+        assert queued.device_ids.tolist() == got and queued.result() == got
+        alone = [sample_rows(dev[i:i + 1].contiguous(), [p], [prev[i]], [20], uniforms=[us[i]])[0] for i, p in enumerate(params)]
+        assert alone == got
+        for i, p in enumerate(params):
+            pen = plain_penalties(logits[i], prev[i], p.repetition_penalty, p.presence_penalty, p.frequency_penalty)
+            if p.temperature <= 0:
+                assert got[i] == int(torch.argmax(pen))
+                continue
+            kept = plain_filtered_probs(pen, p.temperature, p.top_k, p.top_p, p.min_p) > 0
+            probs = torch.softmax(pen.double() / p.temperature, 0) * (pen >= pen[kept].min())
+            cdf = torch.cumsum(probs, 0) / probs.sum()
+            share = probs[got[i]] / probs.sum()
+            # within rounding of float32 sums of up to `vocab` masses, and of one score more or less at a cut
+            edge = 2e-5 + float(probs[pen == pen[kept].min()].max() / probs.sum())
+            assert cdf[got[i]] - share - edge <= us[i] <= cdf[got[i]] + edge, (trial, i)
+    logits = torch.randn(2, vocab, generator=g)
+    logits[0, 3] = float("nan")
+    logits[1] = float("-inf")
+    ids = sample_rows(logits.cuda(), params[:2], [[], []], [0, 0], uniforms=[0.5, 0.5])
+    assert all(0 <= t < vocab for t in ids)
+
+
 def test_trace_run_program(model_dirs, tmp_path):
     """bin/trace_run as a user calls it: JSON steps on standard input, `done <step>` lines,
     <step>.f32 files of little-endian float32 [wanted, vocab]."""
