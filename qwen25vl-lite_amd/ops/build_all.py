@@ -15,6 +15,7 @@ LIBRARIES = [
     ("attention_generic", {}),
     ("gemm_f32", {}),
     ("sample", {}),
+    ("sample_gather", {}),
     ("gemm_resident", {}),
     ("gemm_resident", {"RK": 8}),
     ("gemm_tile", {}),

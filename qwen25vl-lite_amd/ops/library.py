@@ -16,6 +16,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import tempfile
 import threading
 import time
@@ -31,7 +32,8 @@ HIPCC_FLAGS = ("-O3", "-std=c++17", f"--offload-arch={ARCH}", "-shared", "-fPIC"
 # Flags of single sources.  The matrix-core attention takes maxima of scores that are never NaN
 # (masked ones are -inf): told so, the compiler drops the instruction that would quiet a signalling
 # NaN before every maximum, a third of the vector instructions of its softmax.
-SOURCE_FLAGS = {"attention_mfma": ("-fno-honor-nans",)}
+SOURCE_FLAGS = {"attention_mfma": ("-fno-honor-nans",),
+                "sample_gather": (f"-I{sysconfig.get_path('include')}",)}     # host code that reads Python objects
 
 _loaded: Dict[Tuple[str, Tuple[Tuple[str, str], ...]], ctypes.CDLL] = {}
 _lock = threading.Lock()
@@ -162,14 +164,15 @@ def build_library(stem: str, defines: Optional[Mapping[str, object]] = None, *, 
     return out
 
 
-def load_library(stem: str, defines: Optional[Mapping[str, object]] = None) -> ctypes.CDLL:
-    """The loaded library of ``csrc/<stem>.hip``; built first if it is not there."""
+def load_library(stem: str, defines: Optional[Mapping[str, object]] = None, loader=ctypes.CDLL) -> ctypes.CDLL:
+    """The loaded library of ``csrc/<stem>.hip``; built first if it is not there.  ``loader``: ``ctypes.PyDLL`` for one whose functions
+    are called with the interpreter's lock held."""
     defines = dict(defines or {})
     key = (stem, tuple(sorted((k, str(v)) for k, v in defines.items())))
     with _lock:
         lib = _loaded.get(key)
         if lib is None:
             path = build_library(stem, defines)
-            lib = ctypes.CDLL(path)
+            lib = loader(path)
             _loaded[key] = lib
         return lib

@@ -16,6 +16,7 @@ import numpy as np
 import torch
 
 from ..ops.kernels import KernelError, _check, _fn, _stream
+from ..ops.library import load_library
 from .params import SamplingParams
 
 __all__ = ["sample_rows", "sample_rows_begin", "sample_slots_begin", "PendingSample", "uniform_for", "uniform_from"]
@@ -64,22 +65,50 @@ class _Staging:
     _rings = {}
 
     @classmethod
-    def to_device(cls, packed: np.ndarray, device: torch.device) -> torch.Tensor:
+    def take(cls, words: int, device: torch.device):
+        """A buffer of at least ``words`` int32 that no copy reads any more: ``(host tensor, event)``."""
         key = device.index or 0
         ring = cls._rings.setdefault(key, {"turn": -1, "slots": [None] * 4})
         turn = ring["turn"] = (ring["turn"] + 1) % len(ring["slots"])
         slot = ring["slots"][turn]
-        if slot is None or slot[0].numel() < packed.size:
-            slot = ring["slots"][turn] = (torch.empty(max(1024, 2 * packed.size), dtype=torch.int32, pin_memory=True),
-                                         torch.cuda.Event())
+        if slot is None or slot[0].numel() < words:
+            slot = ring["slots"][turn] = (torch.empty(max(8192, 2 * words), dtype=torch.int32, pin_memory=True), torch.cuda.Event())
         else:
             slot[1].synchronize()       # the copy that last read this buffer is done
+        return slot
+
+    @staticmethod
+    def send(slot, words: int, device: torch.device) -> torch.Tensor:
         host, copied = slot
-        host.numpy()[:packed.size] = packed
-        buf = torch.empty(packed.size, dtype=torch.int32, device=device)
-        buf.copy_(host[:packed.size], non_blocking=True)
+        buf = torch.empty(words, dtype=torch.int32, device=device)
+        buf.copy_(host[:words], non_blocking=True)
         copied.record()
         return buf
+
+    @classmethod
+    def to_device(cls, packed: np.ndarray, device: torch.device) -> torch.Tensor:
+        slot = cls.take(packed.size, device)
+        slot[0].numpy()[:packed.size] = packed
+        return cls.send(slot, packed.size, device)
+
+
+_ROW_WORDS = _ROW.itemsize // 4
+
+
+def _gather(params, prev_ids, steps, vocab: int, host: torch.Tensor):
+    """The rows' settings and ids into ``host`` by native code: ``(words, flags)``; words are -1 where a row is not of
+    the usual kind, below that minus the words needed."""
+    global _gather_fn
+    if _gather_fn is None:
+        lib = load_library("sample_gather", loader=ctypes.PyDLL)
+        _gather_fn = lib.qvl_sample_gather
+        _gather_fn.restype = ctypes.c_long
+        _gather_fn.argtypes = [ctypes.py_object] * 3 + [ctypes.c_long] * 2 + [ctypes.c_void_p, ctypes.c_long, ctypes.c_void_p]
+    flags = (ctypes.c_int32 * 4)()
+    return _gather_fn(params, prev_ids, steps, len(params), vocab, host.data_ptr(), host.numel(), ctypes.addressof(flags)), flags
+
+
+_gather_fn = None
 
 
 class PendingSample:
@@ -146,6 +175,15 @@ def _sample_rows(logits, params, prev_ids, steps, uniforms, wait: bool):
         # one greedy setting for the whole batch (the usual decode step): fill the rows at once
         rows[:] = (first.temperature, first.top_p, first.min_p, 0.0, 1.0, 0.0, 0.0, first.top_k if first.top_k else -1, 0, 0, 0, 0)
         return _launch(logits, rows, flat, wait)
+    if uniforms is None:
+        with torch.cuda.device(logits.device):
+            slot = _Staging.take(m * _ROW_WORDS + 1, logits.device)
+            words, flags = _gather(params, prev_ids, steps, vocab, slot[0])
+            if words < -1:
+                slot = _Staging.take(-words, logits.device)
+                words, flags = _gather(params, prev_ids, steps, vocab, slot[0])
+            if words > 0:
+                return _queue(logits, _Staging.send(slot, words, logits.device), *flags, wait)
     filled = []
     for i, p in enumerate(params):
         need_prev = p.repetition_penalty != 1.0 or p.presence_penalty != 0.0 or p.frequency_penalty != 0.0
@@ -210,42 +248,47 @@ _SHORT, _LONG = 1, 2      # the kernel's ways to a row's token
 
 
 def _launch(logits: torch.Tensor, rows: np.ndarray, flat: List[int], wait: bool = False):
-    """Send the rows' settings to the device and queue the sampler: a :class:`PendingSample`.  With ``wait`` the ids,
-    and the passes for rows that the short way does not settle are queued only if there are any."""
+    """Send the rows' settings to the device and queue the sampler (see :func:`_queue`)."""
+    vocab = logits.shape[1]
+    draws = rows["temperature"] > 0
+    flags = (draws.any(), (draws & (rows["prev_end"] > rows["prev_begin"])).any(),
+             (draws & (rows["top_k"] > 0) & (rows["top_k"] < vocab)).any(), (draws & (rows["top_p"] < 1.0)).any())
+    with torch.cuda.device(logits.device):
+        buf = _Staging.to_device(np.concatenate([rows.view(np.int32), _int32_ids(flat)]), logits.device)
+        return _queue(logits, buf, *flags, wait)
+
+
+def _queue(logits: torch.Tensor, buf: torch.Tensor, draws, penalised, top_k, top_p, wait: bool):
+    """Queue the sampler for the settings in ``buf`` (the rows, then generated ids): a :class:`PendingSample`.  With ``wait``
+    the ids, and the passes for rows that the short way does not settle are queued only if there are any.
+    ``draws``, ``penalised``, ``top_k``, ``top_p``: whether any row draws, draws with generated ids, has these cuts."""
     m, vocab = logits.shape
     c_ptr, c_int = ctypes.c_void_p, ctypes.c_int
     fn = _fn("sample", "qvl_sample_rows", [c_ptr] * 7 + [c_int] * 5 + [c_ptr])
     parts_bytes = _fn("sample", "qvl_sample_parts_bytes", [c_int], restype=ctypes.c_longlong)
     dev = logits.device
-    draws = rows["temperature"] > 0
-    with torch.cuda.device(dev):
-        packed = np.concatenate([rows.view(np.int32), _int32_ids(flat)])
-        buf = _Staging.to_device(packed, dev)
-        n_row_words = rows.view(np.int32).size
-        scores = scratch = None
-        top_k = top_p = 0
-        if draws.any():
-            scratch_bytes = _fn("sample", "qvl_sample_scratch_bytes", [], restype=ctypes.c_longlong)
-            scratch = torch.empty(m * scratch_bytes(), dtype=torch.uint8, device=dev)
-            # rows that draw with penalties have their scores written out; the passes read the others' logits as they are
-            if (draws & (rows["prev_end"] > rows["prev_begin"])).any():
-                scores = torch.empty_like(logits)
-            top_k = int((draws & (rows["top_k"] > 0) & (rows["top_k"] < vocab)).any())
-            top_p = int((draws & (rows["top_p"] < 1.0)).any())
-        parts = torch.empty(m * parts_bytes(vocab), dtype=torch.uint8, device=dev)
-        out = torch.empty(m + 1, dtype=torch.int32, device=dev)      # the ids, and how many rows go the long way
+    scores = scratch = None
+    if draws:
+        scratch_bytes = _fn("sample", "qvl_sample_scratch_bytes", [], restype=ctypes.c_longlong)
+        scratch = torch.empty(m * scratch_bytes(), dtype=torch.uint8, device=dev)
+        # rows that draw with penalties have their scores written out; the passes read the others' logits as they are
+        if penalised:
+            scores = torch.empty_like(logits)
+    parts = torch.empty(m * parts_bytes(vocab), dtype=torch.uint8, device=dev)
+    out = torch.empty(m + 1, dtype=torch.int32, device=dev)      # the ids, and how many rows go the long way
 
-        def queue(ways):
-            _check(fn(logits.data_ptr(), None if scores is None else scores.data_ptr(), buf.data_ptr(),
-                      buf.data_ptr() + 4 * n_row_words, None if scratch is None else scratch.data_ptr(), parts.data_ptr(),
-                      out.data_ptr(), m, vocab, top_k, top_p, ways, _stream()), "sample_rows")
-        if not wait or scratch is None:
-            queue(_SHORT | _LONG)
-            pending = PendingSample(out[:m])
-            return pending.result() if wait else pending
-        queue(_SHORT)
-        ids = PendingSample(out).result()
-        if ids.pop():
-            queue(_LONG)
-            ids = PendingSample(out[:m]).result()
-        return ids
+    def queue(ways):
+        at = buf.data_ptr()
+        _check(fn(logits.data_ptr(), None if scores is None else scores.data_ptr(), at, at + 4 * _ROW_WORDS * m,
+                  None if scratch is None else scratch.data_ptr(), parts.data_ptr(), out.data_ptr(), m, vocab, int(top_k),
+                  int(top_p), ways, _stream()), "sample_rows")
+    if not wait or scratch is None:
+        queue(_SHORT | _LONG)
+        pending = PendingSample(out[:m])
+        return pending.result() if wait else pending
+    queue(_SHORT)
+    ids = PendingSample(out).result()
+    if ids.pop():
+        queue(_LONG)
+        ids = PendingSample(out[:m]).result()
+    return ids

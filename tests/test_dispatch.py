@@ -32,3 +32,38 @@ def test_sampler_takes_token_ids_of_any_kind():
                         (list(torch.tensor([[3, 4], [5, 6]])), (RuntimeError, TypeError, ValueError))):
         with pytest.raises(error):
             _int32_ids(flat)
+
+
+def test_sampler_settings_gathered_by_native_code():
+    """The words that go to the device are those that Python's loop makes, at any settings, number of ids and room; what is
+    not of the usual kind is left to that loop."""
+    from qwen25vl_lite_amd.sampling import SamplingParams
+    from qwen25vl_lite_amd.sampling import sampler as S
+    kinds = [dict(temperature=0.0), dict(temperature=0.7, top_p=0.9, seed=3), dict(temperature=1, top_k=50, repetition_penalty=1.05, seed=-9),
+             dict(temperature=0.8, min_p=0.05, seed=2 ** 40 + 7), dict(temperature=0.0, presence_penalty=0.5), dict(temperature=2.0, top_k=0, seed=1)]
+    params = [SamplingParams(**k) for k in kinds]
+    prev = [[5], (1, 2), [2 ** 30 - 1, 0, 2 ** 30, -1, 2 ** 31 - 1], [], list(range(300)), []]
+    steps = [1, 2, 5, 0, 300, 7]
+    rows, ids = np.zeros(len(params), S._ROW), []
+    for i, p in enumerate(params):
+        begin = len(ids)
+        if p.repetition_penalty != 1.0 or p.presence_penalty != 0.0 or p.frequency_penalty != 0.0:
+            ids.extend(prev[i])
+        seeded = p.temperature > 0
+        rows[i] = (p.temperature, p.top_p, p.min_p, 0.0, p.repetition_penalty, p.presence_penalty, p.frequency_penalty, p.top_k or -1, begin,
+                   len(ids), (p.seed + steps[i]) & 0xffffffff if seeded else 0, seeded)
+    want = np.concatenate([rows.view(np.int32), np.asarray(ids, np.int32)])
+    host = torch.full((want.size + 3,), 77, dtype=torch.int32)
+    words, flags = S._gather(params, prev, steps, 100, host)
+    assert words == want.size and host[:words].tolist() == want.tolist() and host[words:].tolist() == [77] * 3
+    assert list(flags) == [1, 1, 1, 1]
+    small = torch.full((80,), 77, dtype=torch.int32)
+    assert S._gather(params, prev, steps, 100, small[:76])[0] == -want.size and small[76:].tolist() == [77] * 4
+    assert S._gather(params[:1], prev[:1], steps[:1], 100, host)[0] == 13 and host[12] == 0        # no ids: one zero
+    for odd in (dict(params=[SamplingParams(temperature=0.5)]), dict(params=[SamplingParams(temperature="1")]), dict(params=[None]),
+                dict(params=[SamplingParams(temperature=1.0, seed=2 ** 70)]), dict(prev=[np.array([3])]), dict(prev=[[2 ** 31]]),
+                dict(prev=[[np.int64(3)]]), dict(prev=[[True]]), dict(steps=[np.int64(1)]), dict(prev=[]), dict(steps=np.array([1]))):
+        call = dict(params=[SamplingParams(temperature=1.0, seed=4, presence_penalty=0.1)], prev=[[3]], steps=[1])
+        assert S._gather(call["params"], call["prev"], call["steps"], 100, host)[0] == 13
+        call.update(odd)
+        assert S._gather(call["params"], call["prev"], call["steps"], 100, host)[0] == -1, odd
