@@ -2,15 +2,17 @@
 // follows the product done on the sums: a cast, the square of relu, a gated activation (gate and up rows of W in
 // groups of 8 + 8, or gate rows first), or float32 slabs over ranges of K for whoever adds them next.
 //
-// The inner loop is tile_product.h's.  Tiles of 256 x 256 run fastest, smaller ones where a device of 256
-// compute units would otherwise stand half empty; the choice is by an estimate of the time (plan_for).  Measured, the
+// The inner loop is tile_product.h's.  Tiles of 256 x 256 run fastest, others where a device of 256
+// compute units would otherwise stand half empty or rows be padded; the choice is by an estimate of the time (plan_for).  Measured, the
 // library's product (with the activation's kernel behind it where there is one) in brackets: 2,048 x 37,888 x 3,584
-// gated 439 us (624), 2,048 x 3,584 x 18,944 in two ranges 204 (377), 280 x 22,016 x 2,048 gated 50 (55), 280 x 2,048 x
-// 11,008 in ranges 34 (50), 100 x 2,560 x 2,048 in ranges 15 (28), 700 x 3,584 x 18,944 in ranges 85 (182).
+// gated 421 us (624), 2,048 x 3,584 x 18,944 in two ranges 204 (377), 281 x 22,016 x 2,048 gated 37 (55), 281 x 2,048 x 11,008 in ranges 23
+// (50), 281 x 2,048 x 2,048 in ranges 10 (20).
 //
 // Blocks go to the XCDs in turn, each with an L2 of its own: XCD x takes a contiguous run of the tiles, ordered so that
 // the 32 blocks it holds at a time share few rows of W and X (eight tiles of X's rows, then the next tile of W's).
 #include "tile_product.h"
+
+#include <cmath>
 
 enum { OUT_BF16 = 0, OUT_F32 = 1, OUT_GROUPED = 2, OUT_HALVES = 3 };
 
@@ -130,6 +132,7 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(TileArgs p) {
       // gives every lane a gate and its up value.
 #pragma unroll
       for (int n = 0; n < T::NT; n += 2) {
+        static_assert(T::NT % 2 == 0, "tiles in pairs");
         float v[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -146,11 +149,12 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(TileArgs p) {
 }
 
 // How a product is cut: the tile's shape and the ranges of K.  The estimate is of microseconds: a step of 64 values
-// costs a block `alone` where most compute units are idle and `full` where all work (a step of 256 x 256 takes 1.08 and
-// 1.43 us: with every matrix core busy the clock and the caches give way), a launch 8 us and each of its rounds 4 (the
-// first fetches, the stores); slabs are written and read once more, at 4.5 TB/s.  Where two blocks share a compute unit, a
-// last round of up to half the room has a unit for each block, else some blocks have to share (22,016 x 2,048 gated: 172
-// blocks of 128 x 128 28 us, 344 43; of 128 x 256 172 36).
+// costs a block `alone` where most compute units are idle and `full` where all work (with every matrix core busy the clock and the
+// caches give way), a launch 3 us and each of its rounds 2.9 (the first fetches, the stores); results are written at 5.9 TB/s and read once
+// more at 4.5; and W comes at 7.5 TB/s at most, which joins the rest as the root of squares.  Where two blocks share a compute unit, a last
+// round of up to half the room has a unit for each block, else some blocks have to share.  Fitted to 124 products of 70 to 4,096 rows at
+// the 3B, 7B and 72B decoders' sizes, each with all shapes and cuts (rms 6 per cent): what it chooses takes 0.8 per cent longer than the best
+// on average, 12 at most; the estimate before, among the first four shapes, 5.0 and 36.
 struct Plan {
   int tile, splits;
   double us;
@@ -159,22 +163,27 @@ struct TileShape {
   int bn, bm, a_unit;     // blocks a compute unit holds
   double alone, full;
 };
-static const TileShape SHAPES[4] = {{256, 256, 1, 1.08, 1.43}, {128, 256, 1, 0.72, 0.96}, {256, 128, 1, 0.79, 0.94}, {128, 128, 2, 0.53, 1.02}};
+#define SHAPES_N 10
+static const TileShape SHAPES[SHAPES_N] = {{256, 256, 1, 0.967, 1.361}, {128, 256, 1, 0.629, 0.816}, {256, 128, 1, 0.678, 0.825},
+                                           {128, 128, 2, 0.502, 0.884}, {192, 192, 1, 0.727, 0.922}, {128, 192, 2, 0.597, 1.164},
+                                           {192, 256, 1, 0.784, 1.089}, {192, 320, 1, 0.992, 1.362}, {128, 320, 1, 0.758, 0.985},
+                                           {256, 192, 1, 0.888, 1.129}};
 
 static Plan plan_for(int M, int N, int K, int most_splits, int cus) {
   Plan best{0, 1, 1e30};
   const int steps = (K + 63) / 64;
-  for (int i = 0; i < 4; ++i) {
+  const double memory = 3.0 + (double)N * K * 2.0 / 7.52e6;
+  for (int i = 0; i < SHAPES_N; ++i) {
     const TileShape& s = SHAPES[i];
     const long long tiles = (long long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
     for (int splits = 1; splits <= most_splits && (splits == 1 || splits * 4 <= steps); ++splits) {
       const long long blocks = tiles * splits, room = (long long)cus * s.a_unit, whole = blocks / room;
       const double rest = (double)(blocks - whole * room) / room;
-      const double depth = (steps + splits - 1) / splits;
-      double us = 8.0 + whole * (depth * s.full + 4.0);
+      const double depth = (steps + splits - 1) / splits, bytes = (double)M * N * (splits > 1 ? 4.0 * splits : 2.0);
+      double us = 3.0 + whole * (depth * s.full + 2.9) + bytes / 5.92e6;
       const double busy = s.a_unit == 1 ? rest : (2.0 * rest > 1.0 ? 1.0 : 0.0);
-      if (rest > 0) us += depth * (s.alone + (s.full - s.alone) * busy) + 4.0;
-      if (splits > 1) us += splits * (double)M * N * 8.0 / 4.5e6;
+      if (rest > 0) us += depth * (s.alone + (s.full - s.alone) * busy) + 2.9;
+      us = sqrt(us * us + memory * memory) + bytes / 4.5e6;
       if (us < best.us) best = Plan{i, splits, us};
     }
   }
@@ -199,7 +208,7 @@ extern "C" int qvl_gemm_tile_blocks(int M, int N, int K, int cus) {
 // mode 0: out bfloat16 [M, N] (relu2: max(product, 0)^2); 1: out float32 [splits][M][N], the slabs' sum is the product;
 // 2: N in groups of 8 gate + 8 up rows, out bfloat16 [M, N / 2] = act(gate) up (gelu: gelu's tanh form, else silu);
 // 3: N / 2 gate rows, then the up rows: out = g sigmoid(alpha g) (u + shift), g capped at limit, u clamped to +-limit.
-// tile: -1, or the shape to take (0 .. 3).
+// tile: -1, or the shape to take (0 .. 9).
 extern "C" int qvl_gemm_tile(const void* x, long long ldx, const void* w, long long ldw, void* out, long long ldo, int M, int N,
                              int K, int mode, int splits, int relu2, int gelu, float alpha, float limit, float shift, int tile,
                              int cus, hipStream_t stream) {
@@ -208,7 +217,7 @@ extern "C" int qvl_gemm_tile(const void* x, long long ldx, const void* w, long l
       ((uintptr_t)x % 16) || ((uintptr_t)w % 16) || ((uintptr_t)out % 16) || splits > (K + 63) / 64 || (mode != 1 && splits != 1))
     return QVL_ERR_SHAPE;
   if ((mode == 2 && N % 16) || (mode == 3 && N % 2) || ldo < (mode >= 2 ? N / 2 : N)) return QVL_ERR_SHAPE;
-  if (mode < 0 || mode > 3 || tile > 3) return QVL_ERR_SHAPE;
+  if (mode < 0 || mode > 3 || tile >= SHAPES_N) return QVL_ERR_SHAPE;
   // byte offsets from a tile's first row are 32-bit (in mode 3 the up rows lie N / 2 rows further on)
   const unsigned long long w_span = (mode == 3 ? (unsigned long long)N / 2 + 256 : 256ull) * ldw * 2, x_span = 256ull * ldx * 2;
   if (w_span >= 0xffff0000ull || x_span >= 0xffff0000ull) return QVL_ERR_LIMIT;
@@ -216,7 +225,8 @@ extern "C" int qvl_gemm_tile(const void* x, long long ldx, const void* w, long l
   p.x = (const bf16_t*)x; p.ldx = ldx; p.w = (const bf16_t*)w; p.ldw = ldw; p.out = out; p.ldo = ldo;
   p.M = M; p.N = N; p.K = K; p.rows = mode == 3 ? N / 2 : N; p.splits = splits; p.relu2 = relu2; p.gelu = gelu;
   p.alpha = alpha; p.limit = limit; p.shift = shift;
-  const int shape = tile >= 0 ? tile : plan_for(M, N, K, mode == 1 && splits > 1 ? MOST_SPLITS : 1, cus).tile;
+  int shape = tile >= 0 ? tile : plan_for(M, N, K, mode == 1 && splits > 1 ? MOST_SPLITS : 1, cus).tile;
+  if ((unsigned long long)SHAPES[shape].bm * ldx * 2 >= 0xffff0000ull) shape = 0;
   const TileShape& s = SHAPES[shape];
   const int out_n = mode == 3 ? s.bn / 2 : s.bn;
   p.tiles_m = (M + s.bm - 1) / s.bm;
@@ -230,7 +240,13 @@ extern "C" int qvl_gemm_tile(const void* x, long long ldx, const void* w, long l
     if (shape == 0) GO(OUT, 2, 4, 8, 4); \
     else if (shape == 1) GO(OUT, 2, 4, 4, 4); \
     else if (shape == 2) GO(OUT, 4, 2, 4, 4); \
-    else GO(OUT, 2, 4, 4, 2);            \
+    else if (shape == 3) GO(OUT, 2, 4, 4, 2); \
+    else if (shape == 4) GO(OUT, 2, 4, 6, 3); \
+    else if (shape == 5) GO(OUT, 2, 4, 4, 3); \
+    else if (shape == 6) GO(OUT, 2, 4, 6, 4); \
+    else if (shape == 7) GO(OUT, 2, 4, 6, 5); \
+    else if (shape == 8) GO(OUT, 2, 4, 4, 5); \
+    else GO(OUT, 2, 4, 8, 3);            \
   } while (0)
   if (mode == 0) SHAPE(OUT_BF16);
   else if (mode == 1) SHAPE(OUT_F32);

@@ -9,14 +9,21 @@
 //
 // A step's operands lie in four regions: W's rows of the waves' first and second halves, X's likewise.  A
 // region is fetched again, for the step after next, one phase after its last reader has passed, so a fetch
-// (straight into LDS) has more than a step's time to arrive with only two buffers.  Rows of 128 bytes; the
+// (straight into LDS) has more than a step's time to arrive with only two buffers (three or four: no faster).  Rows of 128 bytes; the
 // 16-byte chunk c of row rho lies at place c ^ ((rho >> 1) & 7), which spreads the 16 rows of an operand read over
 // all banks.
 //
-// Measured on 4,096 x 8,192 x 8,192 with tiles of 256 x 256: 1.48 PFLOP/s; the same tiles with all waves in step and
-// one step of prefetch 1.29; the library's product of 8,192 cubed 1.34.
+// Each phase reads one region: W's first half, X's second, W's second, and X's first of the next step, into registers of
+// its own.  With both first halves in one phase that phase's reads take longer than the other group's products, and one
+// phase has none.  Steps come in pairs, so that a region's place is a constant.  Both, against one step a round and the halves together:
+// 4,096 x 37,888 x 3,584 gated 820 us for 853 (the places alone 834), 2,048 x 3,584 x 18,944 in two ranges 204 for 212, 2,048 x 22,016 x
+// 2,048 gated in tiles of 128 x 256 195 for 209, 281 x 2,048 x 2,048 of 128 x 128 9.5 for 10.3.
+//
+// Measured on 4,096 x 37,888 x 3,584 gated with tiles of 256 x 256: 820 us = 1.36 PFLOP/s; the library's product of 8,192 cubed 1.34.
 #pragma once
 #include "common.h"
+
+#include <type_traits>
 
 typedef __bf16 tp_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float tp_f32x4 __attribute__((ext_vector_type(4)));
@@ -56,18 +63,29 @@ __device__ __forceinline__ void tp_wait_steps(int ahead) {
   }
 }
 
+// An address that is the same for the whole wave, in scalar registers.
+__device__ __forceinline__ const void* tp_uniform(const void* p) {
+  const unsigned long long a = (unsigned long long)(uintptr_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)a), hi = __builtin_amdgcn_readfirstlane((uint32_t)(a >> 32));
+  return (const void*)(uintptr_t)((unsigned long long)hi << 32 | lo);
+}
+
 template <int WN_, int WM_, int NT_, int MT_>
 struct Tile {
   static constexpr int WN = WN_, WM = WM_, NT = NT_, MT = MT_;
-  static constexpr int BN = 16 * WN * NT, BM = 16 * WM * MT, NH = NT / 2, MH = MT / 2;
-  static constexpr int LA = BN / 128, LB = BM / 128;         // fetches of 8 rows a wave has in a region of W, of X
-  static constexpr int RA = BN * 64, RB = BM * 64;           // bytes of a region
-  static constexpr int BUF = 2 * RA + 2 * RB, LDS = 2 * BUF;
-  static_assert(WN * WM == 8 && NT % 2 == 0 && MT % 2 == 0 && BN % 128 == 0 && BM % 128 == 0, "eight waves, whole fetches");
+  static constexpr int BN = 16 * WN * NT, BM = 16 * WM * MT;
+  // of a wave's tiles the first half (the larger one) and the second
+  static constexpr int N0 = (NT + 1) / 2, N1 = NT / 2, M0 = (MT + 1) / 2, M1 = MT / 2, NH = N0, MH = M0;
+  static constexpr int rows_w(int h) { return 16 * WN * (h ? N1 : N0); }         // of a region
+  static constexpr int rows_x(int h) { return 16 * WM * (h ? M1 : M0); }
+  // fetches of 8 rows a wave has in a region; where they do not divide evenly some rows are fetched twice (the same
+  // bytes to the same place), so that all waves wait for as many
+  static constexpr int LW0 = (rows_w(0) + 63) / 64, LW1 = (rows_w(1) + 63) / 64, LX0 = (rows_x(0) + 63) / 64, LX1 = (rows_x(1) + 63) / 64;
+  static constexpr int BUF = (BN + BM) * 128, LDS = 2 * BUF;
+  static_assert(WN * WM == 8 && NT >= 2 && MT >= 2 && LDS <= 163840, "eight waves, two halves, what LDS holds");
 
   int wave, lane, g, r, wn, wm;
-  uint32_t fa[2][LA], fb[2][LB];   // byte offset of this lane's 16 bytes at K = 0, from W's and from X's base
-  uint32_t back;                   // bytes a lane steps back in a last step of 32 values (its chunk lies beyond K)
+  uint32_t fa[2][LW0], fb[2][LX0];   // byte offset of this lane's 16 bytes at K = 0, from W's and from X's base
   tp_f32x4 acc[NT][MT];
 
   __device__ __forceinline__ Tile() {
@@ -78,32 +96,50 @@ struct Tile {
     wn = wave % WN;
     wm = wave / WN;
   }
-  // chunk of its row that this lane fetches, for the fetch whose rows begin at a multiple of 8
+  // group of 8 rows that this wave's fetch j in a region of `rows` rows brings, L fetches a wave
+  template <int L>
+  __device__ __forceinline__ int group_of(int j, int rows) const {
+    const int i = wave * L + j;
+    return rows % (64 * L) == 0 || i < rows / 8 ? i : i - rows / 8;
+  }
+  // chunk of its row that this lane fetches
   __device__ __forceinline__ int chunk_of(int rho) const { return (lane & 7) ^ ((rho >> 1) & 7); }
   // w_at(h, rho), x_at(h, rho): byte offset of row rho of region h (rows of a wave's half one after the other,
   // waves in order): of the tile's row w_row(h, rho), x_row(h, rho)
-  __device__ static __forceinline__ int w_row(int h, int rho) { return rho / (16 * NH) * (16 * NT) + h * 16 * NH + rho % (16 * NH); }
-  __device__ static __forceinline__ int x_row(int h, int rho) { return rho / (16 * MH) * (16 * MT) + h * 16 * MH + rho % (16 * MH); }
+  __device__ static __forceinline__ int w_row(int h, int rho) {
+    const int n = 16 * (h ? N1 : N0);
+    return rho / n * (16 * NT) + h * 16 * N0 + rho % n;
+  }
+  __device__ static __forceinline__ int x_row(int h, int rho) {
+    const int m = 16 * (h ? M1 : M0);
+    return rho / m * (16 * MT) + h * 16 * M0 + rho % m;
+  }
   template <typename WAt, typename XAt>
   __device__ __forceinline__ void set_rows(WAt w_at, XAt x_at) {
+    auto region = [&](auto half) __attribute__((always_inline)) {
+      constexpr int h = decltype(half)::value, LW = h ? LW1 : LW0, LX = h ? LX1 : LX0;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-#pragma unroll
-      for (int j = 0; j < LA; ++j) {
-        const int rho = (wave * LA + j) * 8 + (lane >> 3);
+      for (int j = 0; j < LW; ++j) {
+        const int rho = group_of<LW>(j, rows_w(h)) * 8 + (lane >> 3);
         fa[h][j] = w_at(h, rho) + 16 * chunk_of(rho);
       }
 #pragma unroll
-      for (int j = 0; j < LB; ++j) {
-        const int rho = (wave * LB + j) * 8 + (lane >> 3);
+      for (int j = 0; j < LX; ++j) {
+        const int rho = group_of<LX>(j, rows_x(h)) * 8 + (lane >> 3);
         fb[h][j] = x_at(h, rho) + 16 * chunk_of(rho);
       }
-    }
+    };
+    region(std::integral_constant<int, 0>{});
+    region(std::integral_constant<int, 1>{});
   }
 
   // acc = the tile's products over `steps` steps of 64 values from w and x on.  half_last: the last step has 32
   // values only.
   __device__ __forceinline__ void multiply(char* lds, const void* w, const void* x, int steps, bool half_last) {
+    constexpr std::integral_constant<int, 0> I{};
+    constexpr std::integral_constant<int, 1> II{};
+    w = tp_uniform(w);
+    x = tp_uniform(x);
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
@@ -111,87 +147,103 @@ struct Tile {
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
     // A fetch asked for beyond the last step brings the last step's values again, to a region nobody reads any
     // more: every step has the same fetches, so the waits can count them.
-    auto at_step = [&](int s, uint32_t rho8) {
+    auto at_step = [&](int s, uint32_t rho) {
       const int t = s < steps ? s : steps - 1;
       uint32_t bytes = (uint32_t)t * 128;
-      if (half_last && t == steps - 1 && (((uint32_t)lane & 7) ^ ((rho8 >> 1) & 7)) >= 4) bytes -= 64;
+      if (half_last && t == steps - 1 && (((uint32_t)lane & 7) ^ ((rho >> 1) & 7)) >= 4) bytes -= 64;
       return bytes;
     };
-    auto issue_w = [&](int h, int s) {
-      const uint32_t at = lds0 + (s & 1) * BUF + h * RA + wave * (LA * 1024);
+    auto issue_w = [&](auto half, int s, int buf) __attribute__((always_inline)) {
+      constexpr int h = decltype(half)::value, L = h ? LW1 : LW0;
+      const uint32_t at = lds0 + buf + h * rows_w(0) * 128;
 #pragma unroll
-      for (int j = 0; j < LA; ++j) tp_fetch16(w, fa[h][j] + at_step(s, (wave * LA + j) * 8 + (lane >> 3)), at + j * 1024);
+      for (int j = 0; j < L; ++j) {
+        const int group = group_of<L>(j, rows_w(h));
+        tp_fetch16(w, fa[h][j] + at_step(s, group * 8 + (lane >> 3)), at + group * 1024);
+      }
     };
-    auto issue_x = [&](int h, int s) {
-      const uint32_t at = lds0 + (s & 1) * BUF + 2 * RA + h * RB + wave * (LB * 1024);
+    auto issue_x = [&](auto half, int s, int buf) __attribute__((always_inline)) {
+      constexpr int h = decltype(half)::value, L = h ? LX1 : LX0;
+      const uint32_t at = lds0 + buf + (BN + h * rows_x(0)) * 128;
 #pragma unroll
-      for (int j = 0; j < LB; ++j) tp_fetch16(x, fb[h][j] + at_step(s, (wave * LB + j) * 8 + (lane >> 3)), at + j * 1024);
+      for (int j = 0; j < L; ++j) {
+        const int group = group_of<L>(j, rows_x(h));
+        tp_fetch16(x, fb[h][j] + at_step(s, group * 8 + (lane >> 3)), at + group * 1024);
+      }
     };
     const uint32_t sw = (r >> 1) & 7;
-    uint32_t ra[2], rb[2];
+    uint32_t chunk[2];
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      ra[k] = (uint32_t)((wn * 16 * NH + r) * 128) + (((4 * k + g) ^ sw) << 4);
-      rb[k] = (uint32_t)((wm * 16 * MH + r) * 128) + (((4 * k + g) ^ sw) << 4);
-    }
-    tp_bf16x8 a[NH][2], b0[MH][2], b1[MH][2];
-    auto read_w = [&](int h, int s) {
-      const char* p = lds + (s & 1) * BUF + h * RA;
+    for (int k = 0; k < 2; ++k) chunk[k] = (uint32_t)(r * 128) + (((4 * k + g) ^ sw) << 4);
+    tp_bf16x8 a[N0][2], b0[2][M0][2], b1[M1][2];
+    auto read_w = [&](auto half, int buf) __attribute__((always_inline)) {
+      constexpr int h = decltype(half)::value, N = h ? N1 : N0;
+      const char* p = lds + buf + h * rows_w(0) * 128 + wn * (16 * N) * 128;
 #pragma unroll
-      for (int i = 0; i < NH; ++i)
+      for (int i = 0; i < N; ++i)
 #pragma unroll
-        for (int k = 0; k < 2; ++k) a[i][k] = *reinterpret_cast<const tp_bf16x8*>(p + ra[k] + i * 2048);
+        for (int k = 0; k < 2; ++k) a[i][k] = *reinterpret_cast<const tp_bf16x8*>(p + chunk[k] + i * 2048);
     };
-    auto read_x = [&](int h, int s, tp_bf16x8 (*b)[2]) {
-      const char* p = lds + (s & 1) * BUF + 2 * RA + h * RB;
+    auto read_x = [&](auto half, int buf, auto& b) __attribute__((always_inline)) {
+      constexpr int h = decltype(half)::value, M = h ? M1 : M0;
+      const char* p = lds + buf + (BN + h * rows_x(0)) * 128 + wm * (16 * M) * 128;
 #pragma unroll
-      for (int i = 0; i < MH; ++i)
+      for (int i = 0; i < M; ++i)
 #pragma unroll
-        for (int k = 0; k < 2; ++k) b[i][k] = *reinterpret_cast<const tp_bf16x8*>(p + rb[k] + i * 2048);
+        for (int k = 0; k < 2; ++k) b[i][k] = *reinterpret_cast<const tp_bf16x8*>(p + chunk[k] + i * 2048);
     };
-    auto part = [&](int hn, int hm, int k, tp_bf16x8 (*b)[2]) {
+    auto quarter = [&](auto half_n, auto half_m, int s, auto& b) __attribute__((always_inline)) {
+      constexpr int hn = decltype(half_n)::value, hm = decltype(half_m)::value;
+      auto part = [&](int k) __attribute__((always_inline)) {
 #pragma unroll
-      for (int n = 0; n < NH; ++n)
+        for (int n = 0; n < (hn ? N1 : N0); ++n)
 #pragma unroll
-        for (int m = 0; m < MH; ++m)
-          acc[hn * NH + n][hm * MH + m] =
-              __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[n][k], b[m][k], acc[hn * NH + n][hm * MH + m], 0, 0, 0);
+          for (int m = 0; m < (hm ? M1 : M0); ++m)
+            acc[hn * N0 + n][hm * M0 + m] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[n][k], b[m][k], acc[hn * N0 + n][hm * M0 + m], 0, 0, 0);
+      };
+      part(0);
+      if (!half_last || s + 1 < steps) part(1);
     };
-    auto quarter = [&](int hn, int hm, int s, tp_bf16x8 (*b)[2]) {
-      part(hn, hm, 0, b);
-      if (!half_last || s + 1 < steps) part(hn, hm, 1, b);
-    };
-    issue_w(0, 0); issue_x(0, 0); issue_x(1, 0); issue_w(1, 0); issue_w(0, 1); issue_x(0, 1); issue_x(1, 1);
-    tp_wait_fetches<2 * LA + 3 * LB>();     // the first halves of step 0
-    tp_barrier();
-    if (wave >= 4) tp_barrier();            // the second group, a phase behind
-    for (int s = 0; s < steps; ++s) {
-      read_w(0, s);
-      read_x(0, s, b0);
-      issue_w(1, s + 1);
-      tp_wait_fetches<3 * LA + 2 * LB>();   // X's second half of step s (behind it: W1 W0 X0 X1 W1)
+    // One step; its first half of X is in b already, the next step's goes to b_next.
+    auto step = [&](int s, int here, auto& b, auto& b_next) __attribute__((always_inline)) {
+      const int other = BUF - here;
+      read_w(I, here);
+      issue_w(II, s + 1, other);
+      tp_wait_fetches<LW1 + LW0 + LX0 + LX1 + LW1>();   // X's second half of step s (behind it: W1 W0 X0 X1 W1)
       tp_wait_lds();                        // this wave has read: the regions may be filled again
       tp_barrier();
-      quarter(0, 0, s, b0);
+      quarter(I, I, s, b);
       tp_barrier();
-      read_x(1, s, b1);
-      issue_w(0, s + 2);
-      tp_wait_fetches<3 * LA + 2 * LB>();   // W's second half of step s
+      read_x(II, here, b1);
+      issue_w(I, s + 2, here);
+      tp_wait_fetches<LW0 + LX0 + LX1 + LW1 + LW0>();   // W's second half of step s
       tp_wait_lds();
       tp_barrier();
-      quarter(0, 1, s, b1);
+      quarter(I, II, s, b1);
       tp_barrier();
-      read_w(1, s);
-      issue_x(0, s + 2);
+      read_w(II, here);
+      issue_x(I, s + 2, here);
+      tp_wait_fetches<LX1 + LW1 + LW0 + LX0>();         // the first halves of step s + 1
       tp_wait_lds();
       tp_barrier();
-      quarter(1, 1, s, b1);
+      quarter(II, II, s, b1);
       tp_barrier();
-      issue_x(1, s + 2);
-      tp_wait_fetches<2 * LA + 3 * LB>();   // the first halves of step s + 1
+      read_x(I, other, b_next);             // (behind the last step: what lies there, for nothing)
+      issue_x(II, s + 2, here);
+      tp_wait_lds();
       tp_barrier();
-      quarter(1, 0, s, b0);
+      quarter(II, I, s, b);
       tp_barrier();
+    };
+    issue_w(I, 0, 0); issue_x(I, 0, 0); issue_x(II, 0, 0); issue_w(II, 0, 0); issue_w(I, 1, BUF); issue_x(I, 1, BUF); issue_x(II, 1, BUF);
+    tp_wait_fetches<LX1 + LW1 + LW0 + LX0 + LX1>();     // the first halves of step 0
+    tp_barrier();
+    if (wave >= 4) tp_barrier();            // the second group, a phase behind
+    read_x(I, 0, b0[0]);
+    for (int s = 0; s < steps; s += 2) {
+      step(s, 0, b0[0], b0[1]);
+      if (s + 1 < steps) step(s + 1, BUF, b0[1], b0[0]);
     }
     if (wave < 4) tp_barrier();
     tp_wait_fetches<0>();                   // nothing may land in LDS that is no longer this block's

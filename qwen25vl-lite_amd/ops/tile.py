@@ -36,7 +36,7 @@ MANY_ROWS = 64           # up to here the decode kernels and the library run
 
 def prefers_tile(x: torch.Tensor, weight: torch.Tensor, halves: bool = False, gated: bool = False) -> bool:
     """Whether the kernel takes the product and is the faster way to it, uncut: more than ``MANY_ROWS`` rows, and tiles for
-    three quarters of the compute units (2,048 x 3,584 x 3,584: 224 tiles, 63 us against the library's 66; 280 x 2,560 x
+    three quarters of the compute units (2,048 x 3,584 x 3,584: 224 tiles, 54 us against the library's 66; 280 x 2,560 x
     2,048: 60 tiles, 34 against 24, the library cuts the inner size).  With a gated activation on the sums (``gated``), which
     takes the library another kernel, half of them suffice (22,016 x 2,048: 100 rows, 172 tiles, 29 us against 35; 190 rows,
     172 tiles, 37 against 41; 380 rows, 172 tiles, 52 against 53; 37,888 x 3,584, 190 rows, 148 tiles, 83 against 89)."""
@@ -69,16 +69,27 @@ def tile_product(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype =
     return _launch(x, weight, out, out.stride(0), _SLABS if out_dtype == torch.float32 else _STORE, relu2=int(relu2), shape=shape)
 
 
+# An uncut product that joins the residual is stored in bfloat16 up to this inner size, and from some number of results on up to a longer one.
+# Beyond, products are cut at most numbers of rows, and keep their float32 sums at the others too: which shape and cut is faster
+# changes from one number of rows to the next (3,584 x 18,944: 1,500 rows in ranges, 1,600 not, 2,000 in ranges), a result's precision does
+# not.  That is 10 us of 410 at 4,096 rows of the latter.
+WHOLE_K, WHOLE_RESULTS, LONG_K = 2560, 6 << 20, 6144
+
+
+def _stored_whole(results: int, k: int) -> bool:
+    return k <= WHOLE_K or (k <= LONG_K and results >= WHOLE_RESULTS)
+
+
 def tile_slabs(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:
     """Float32 slabs ``[splits, M, N]`` over ranges of the inner size, whose sum in order is ``x @ weight.T``; None where the
-    kernel does not take the product or is faster without a cut.  Cutting pays where the tiles alone leave compute units
-    idle: 2,048 x 3,584 x 18,944 has 112 tiles of 256 x 256, two ranges take 204 us and one 282 (the library 377)."""
+    kernel does not take the product or is faster without a cut (long inner sizes: one slab).  Cutting pays where the tiles alone leave compute units
+    idle: 2,048 x 3,584 x 18,944 has 112 tiles of 256 x 256, two ranges take 204 us and one of 192 x 256 234 (the library 377)."""
     if x.shape[0] <= MANY_ROWS or not takes_tile(x, weight):
         return None
     m, k = x.shape
     n = weight.shape[0]
     splits = int(_fn("gemm_tile", "qvl_gemm_tile_splits", [_c_int] * 4)(m, n, k, compute_units(x.device)))
-    if splits <= 1:
+    if splits <= 1 and (_stored_whole(m * n, k) or not prefers_tile(x, weight)):
         return None
     out = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
     return _launch(x, weight, out, n, _SLABS, splits=splits)

@@ -1018,6 +1018,35 @@ def test_tiled_product_off_steps_of_four(m, n, k, beside, shape):
     assert bool(((got - ref).abs() <= slack + (2.0 ** -8 + 1e-6) * ref.abs() + 2e-6).all())
 
 
+@pytest.mark.parametrize("shape, bn, bm", [(4, 192, 192), (5, 128, 192), (6, 192, 256), (7, 192, 320), (8, 128, 320), (9, 256, 192)])
+@pytest.mark.parametrize("rows, outputs, k", [(-1, -2, 32), (1, 16, 64), (-80, 2, 96), (-126, -94, 160), (64, 48, 192)])
+def test_tiled_product_in_shapes_that_do_not_halve(shape, bn, bm, rows, outputs, k):
+    """Shapes whose halves are unequal or whose rows no number of whole fetches brings: rows and outputs around a tile's edges, an
+    odd and an even number of steps, a last one of half its size.  A sum of k exact products is within k roundings of its terms."""
+    from qwen25vl_lite_amd.ops import tile
+    m, n = bm + rows, bn + outputs
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x = torch.randn(m, k, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(n, k, device="cuda", generator=g) / k ** 0.5).bfloat16()
+    want = x.double() @ w.double().T
+    bound = k * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    for dtype, last in ((torch.float32, 0.0), (torch.bfloat16, 2.0 ** -8)):
+        got = tile.tile_product(x, w, dtype, shape=shape).double()
+        assert bool(((got - want).abs() <= bound + last * want.abs()).all())
+    slope = 1.13 * (1.0 + 2.0 ** -8)
+    if n % 16 == 0:
+        two, b = want.view(m, n // 16, 2, 8), bound.view(m, n // 16, 2, 8)
+        ref = torch.nn.functional.silu(two[:, :, 0]) * two[:, :, 1]
+        slack = slope * (b[:, :, 0] * (two[:, :, 1].abs() + b[:, :, 1]) + two[:, :, 0].abs() * b[:, :, 1])
+        got = tile.tile_swiglu(x, w, shape=shape).double().view(m, n // 16, 8)
+        assert bool(((got - ref).abs() <= slack + (2.0 ** -8 + 1e-5) * ref.abs() + 2e-6).all())
+    g, u = want[:, :n // 2].clamp(max=1.5), want[:, n // 2:].clamp(-1.5, 1.5)
+    ref = g * torch.sigmoid(1.25 * g) * (u + 1.0)
+    slack = 1.13 * 2.5 * bound[:, :n // 2] + 1.5 * bound[:, n // 2:]
+    got = tile.tile_gated(x, w, 1.25, 1.5, 1.0, shape=shape).double()
+    assert bool(((got - ref).abs() <= slack + (2.0 ** -8 + 1e-6) * ref.abs() + 2e-6).all())
+
+
 @pytest.mark.parametrize("m", [1, 19, 40])
 @pytest.mark.parametrize("n", [2, 34, 16401, 40970])
 def test_rows_with_a_last_output_alone(m, n):
