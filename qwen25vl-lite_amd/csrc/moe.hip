@@ -576,9 +576,15 @@ __global__ __launch_bounds__(256) void moe_tile_kernel(ExpertArgs a, int tiles_m
 // The same product through the inner loop of tile_product.h: tiles of 128 pairs x 256 rows of W (gated: 128 gate
 // rows and the up rows of the same outputs; a wave's gate and up values of an output end in one lane).  K must be a
 // multiple of 32 and offsets within x and within an expert's W 32-bit.  Measured on 12,384 pairs over 32 experts, K
-// 3,584: 2 x 2,368 rows 655 us (tiles of 128 x 256 with all waves in step: 874); down and per-head products of a prompt's pass 207 us
-// on average (316).
+// 3,584: 2 x 2,368 rows 574 us (tiles of 128 x 256 with all waves in step: 874); down 291.
+// From WIDE_PAIRS pairs an expert on (on average) tiles of 256 pairs: LDS gives each operand to twice the products, for half a tile more
+// of padding an expert.  2 x 2,368 x 3,584 gated and 3,584 x 2,368, 32 experts, of 128 and of 256: 131 pairs 324 and 329 us, 180 and 175,
+// 188 319 and 356, 183 and 189, 262 453 and 446, 246 and 241, 387 574 and 449, 291 and 246, 562 723 and 717, 376 and 369, 768 1,030 and 887,
+// 536 and 444; 2 x 1,376 x 2,048 and 2,048 x 1,376: 188 134 and 174, 80 and 98, 262 187 and 182, 108 and 100, 562 262 and 279, 173 and 146,
+// 768 358 and 342, 232 and 192.
 typedef Tile<4, 2, 4, 4> ExpertsTile;
+typedef Tile<2, 4, 8, 4> WideTile;
+#define WIDE_PAIRS 256
 
 template <typename TO>
 __device__ __forceinline__ void store_expert4(TO* o, const float* v, int n, bool whole);
@@ -602,9 +608,8 @@ __device__ __forceinline__ void store_expert4<bf16_t>(bf16_t* o, const float* v,
   }
 }
 
-template <bool GATED, typename TO>
+template <typename T, bool GATED, typename TO>
 __global__ __launch_bounds__(512) void moe_stream_kernel(ExpertArgs a, int tiles_m, int tiles_n, int whole4) {
-  typedef ExpertsTile T;
   __shared__ __attribute__((aligned(16))) char lds[T::LDS];
   // blocks of one XCD at a time: 4 tiles of pairs x 8 tiles of rows of W (see moe_tile_kernel)
   const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
@@ -652,7 +657,7 @@ __global__ __launch_bounds__(512) void moe_stream_kernel(ExpertArgs a, int tiles
 
 // x_dtype / out_dtype: 0 float32, 1 bfloat16.  float32 operands write float32; bfloat16 operands
 // write either.  The matrix-core kernel runs for bfloat16 with K a multiple of 8 and rows of x on
-// 16-byte boundaries; `big_tiles` asks for the kernel with tiles of 128 pairs through LDS (many pairs an expert).
+// 16-byte boundaries; `big_tiles` asks for the kernels with tiles of 128 or 256 pairs through LDS (many pairs an expert).
 extern "C" int qvl_moe_experts(const void* x, long long ldx, int x_dtype, const void* w, const void* sorted,
                                const void* offsets, void* out, long long ldo, int out_dtype, int P, int E, int R, int K,
                                int div,
@@ -668,17 +673,25 @@ extern "C" int qvl_moe_experts(const void* x, long long ldx, int x_dtype, const 
     const unsigned long long x_rows = (unsigned long long)((P + div - 1) / div);
     if (big_tiles && K % 32 == 0 && x_rows * (unsigned long long)ldx * 2 < 0xffff0000ull &&
         (unsigned long long)(gated ? 2 * R : R) * K * 2 < 0xffff0000ull) {
+      const bool wide = P >= WIDE_PAIRS * (long long)E;
+      const int bm = wide ? WideTile::BM : ExpertsTile::BM;
       const int cols = gated ? ExpertsTile::BN / 2 : ExpertsTile::BN;
-      const int tiles_m = P / ExpertsTile::BM + (E < P ? E : P), tiles_n = (R + cols - 1) / cols;
+      const int tiles_m = P / bm + (E < P ? E : P), tiles_n = (R + cols - 1) / cols;
       if ((long long)tiles_m * tiles_n > 0x7ffffff0ll) return QVL_ERR_LIMIT;
       const int supers = ((tiles_m + 3) / 4) * ((tiles_n + 7) / 8);
       const dim3 tgrid((unsigned)((supers + 7) / 8) * 8 * 32);
       const int whole4 = ldo % 4 == 0 && ((uintptr_t)out % 16) == 0;    // four neighbouring results as one store
-#define STREAM(G, TO) hipLaunchKernelGGL((moe_stream_kernel<G, TO>), tgrid, dim3(512), 0, stream, a, tiles_m, tiles_n, whole4)
-      if (gated && out_dtype == 1) STREAM(true, bf16_t);
-      else if (gated) STREAM(true, float);
-      else if (out_dtype == 1) STREAM(false, bf16_t);
-      else STREAM(false, float);
+#define STREAM(T, G, TO) hipLaunchKernelGGL((moe_stream_kernel<T, G, TO>), tgrid, dim3(512), 0, stream, a, tiles_m, tiles_n, whole4)
+#define SHAPE(G, TO)                     \
+  do {                                   \
+    if (wide) STREAM(WideTile, G, TO);   \
+    else STREAM(ExpertsTile, G, TO);     \
+  } while (0)
+      if (gated && out_dtype == 1) SHAPE(true, bf16_t);
+      else if (gated) SHAPE(true, float);
+      else if (out_dtype == 1) SHAPE(false, bf16_t);
+      else SHAPE(false, float);
+#undef SHAPE
 #undef STREAM
       return qvl_launch_status();
     }

@@ -847,6 +847,33 @@ def test_experts_with_few_pairs(e, r, k, pairs):
         assert bool(((got - ref).abs() <= slack + (last + 1e-6) * ref.abs() + 2e-6).all())
 
 
+@pytest.mark.parametrize("e, r, k, per", [(2, 300, 160, 255), (2, 300, 160, 257), (3, 128, 96, 700), (1, 129, 64, 256), (5, 8, 32, 300)])
+def test_experts_with_many_pairs(e, r, k, per):
+    """On both sides of where tiles of 256 pairs begin; experts whose pairs fill no tile, outputs that fill none, one expert without
+    pairs.  A sum of k exact products is within k roundings of its terms."""
+    from qwen25vl_lite_amd.ops import moe
+    torch.manual_seed(e + per)
+    n, top = per * e // 2 + (per * e) % 2, 2
+    ids = torch.randint(0, max(1, e - 1), (n, top), dtype=torch.int32, device="cuda")
+    order, offsets = moe.sort_pairs(ids, e)
+    x = torch.randn(n, k, device="cuda").bfloat16()
+    w = (torch.randn(e, 2 * r, k, device="cuda") / math.sqrt(k)).bfloat16()
+    flat = ids.view(-1).long()
+    want = torch.zeros(n * top, 2 * r, dtype=torch.float64, device="cuda")
+    bound = torch.zeros_like(want)
+    for i in range(e):
+        at = (flat == i).nonzero()[:, 0]
+        want[at] = x[at // top].double() @ w[i].double().t()
+        bound[at] = k * 2.0 ** -24 * (x[at // top].double().abs() @ w[i].double().abs().t()) + 1e-30
+    got = moe.expert_products(x, w, order, offsets, n * top, top, torch.float32)
+    assert bool(((got.double() - want).abs() <= bound).all())
+    g, u = want[:, :r].clamp(max=1.5), want[:, r:].clamp(-1.5, 1.5)
+    ref = g * torch.sigmoid(1.25 * g) * (u + 1.0)
+    slack = 1.13 * 2.5 * bound[:, :r] + 1.5 * bound[:, r:]
+    got = moe.expert_products(x, w, order, offsets, n * top, top, torch.bfloat16, gated=(1.25, 1.5, 1.0)).double()
+    assert bool(((got - ref).abs() <= slack + (2.0 ** -8 + 1e-6) * ref.abs() + 2e-6).all())
+
+
 @pytest.mark.parametrize("m", [1, 16, 32])
 def test_rows_of_gate_and_up_that_form_no_groups_keep_the_norm_in_the_product(m, monkeypatch):
     """An inner size of the feed-forward off steps of 8: the product forms the norm of a decode step's rows itself, without a
