@@ -18,12 +18,20 @@ from ..ops.linear import NormedRows, linear, linear_into
 from .base import (CacheNeed, LayerSlot, Mixer, ParamSpec, PartSpec, StateNeed, StepContext, build_part,
                    register_part)
 
-# 17 to 48 rows: where the fused kernel does not run, the projection is cut along its inner size (slabs) and the rotation's
+# 17 to 64 rows: where the fused kernel does not run, the projection is cut along its inner size (slabs) and the rotation's
 # kernel adds them (10,240 x 8,192, 19 rows: 32 us, the library's product uncut 41).  From 33 rows on that also beats the fused
-# kernel on teams of blocks (7B sizes: a step of 33 rows 4.14 ms against 4.24, of 48 rows 4.34 against 4.39, of 64 rows
-# 4.68 against 4.67)
-SPLIT_ROWS = (17, 48)
+# kernel on teams of blocks: up to 48 rows at any inner size (7B sizes: a step of 33 rows 4.14 ms against 4.24, of 48 rows 4.34 against
+# 4.39), up to 64 where it is beyond LONG_K (8 decode steps at 768 keys, 72B sizes, 2 layers: 64 rows 9,962 us against 10,157, 56 9,818
+# and 10,041; 7B sizes, K = 3,584, 8 layers, 64 rows 11,160 and 11,124; 3B sizes, K = 2,048, 6 steps at 256 keys 4,922 and 4,820).
+SPLIT_ROWS = (17, 64)
+SHORT_SPLIT_ROWS = 48
+LONG_K = 4096
 FUSED_ROWS = 32
+
+
+def _splits(m: int, k: int) -> bool:
+    return SPLIT_ROWS[0] <= m <= (SPLIT_ROWS[1] if k > LONG_K else SHORT_SPLIT_ROWS)
+
 
 __all__ = ["PagedAttention"]
 
@@ -309,7 +317,7 @@ class PagedAttention(Mixer):
         # Projections are written out in float32 (the accumulator, unrounded): bias, rotation and
         # the residual sum then happen in float32 and each stored value is rounded once.
         m, k = x.shape
-        if (SPLIT_ROWS[0] <= m <= SPLIT_ROWS[1] and self.dtype == torch.bfloat16 and isinstance(x, torch.Tensor)
+        if (_splits(m, k) and self.dtype == torch.bfloat16 and isinstance(x, torch.Tensor)
                 and x.dtype == torch.bfloat16 and self.hd % 4 == 0 and inv_freq.shape[0] % 4 == 0
                 and skinny.takes_split(m, k, self.w_in) and x.stride(1) == 1 and x.stride(0) % 8 == 0
                 and x.data_ptr() % 16 == 0):
@@ -343,7 +351,7 @@ class PagedAttention(Mixer):
         kernel (the float32 sums never leave it)."""
         lazy = isinstance(x, NormedRows)
         m, k = x.shape
-        if not lazy and FUSED_ROWS < m <= SPLIT_ROWS[1]:
+        if not lazy and m > FUSED_ROWS and _splits(m, k):
             return None
         if self.dtype != torch.bfloat16 or not skinny.takes_qkv_rope(
                 m, k, self.w_in, self.hd, inv_freq.shape[0], slot.k_cache.dtype if write else None, norm=lazy):
