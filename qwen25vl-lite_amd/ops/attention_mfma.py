@@ -14,7 +14,7 @@ from typing import Optional, Tuple
 import numpy as np
 import torch
 
-from .kernels import _check, _fn, _need, _ptr, _stream
+from .kernels import _check, _fn, _need, _ptr, _stream, int32_to_device
 
 __all__ = ["try_attention", "supports", "tiles_for", "plan_splits"]
 
@@ -144,7 +144,7 @@ def _step_tiles(step, group: int, tile_ct: int, device, by_length: bool = False,
         if only is not None:
             keep = np.asarray(only, dtype=bool)[req]
             req, ct = req[keep], ct[keep]
-        both = torch.from_numpy(np.concatenate([req, ct])).to(device, non_blocking=True)
+        both = int32_to_device(np.concatenate([req, ct]), device)
         cache[key] = (both[:len(req)], both[len(req):], len(req))
     return cache[key]
 
@@ -167,6 +167,13 @@ def long_single_tiles(step, group: int, nkv: int, device=None):
     own their contexts are split among blocks (measured at the 7B decoder's heads: 8 decoded tokens
     at 8,192 keys beside a portion of 256 take 87 us together, 32 and 13 apart).  Below
     ``ALONE_KEYS`` the two launches, one after the other, cost more than the walks they shorten."""
+    key = ("long single tiles", group, nkv)       # the same for every layer of the step
+    if key not in step.derived:
+        step.derived[key] = _long_single_tiles(step, group, nkv, device)
+    return step.derived[key]
+
+
+def _long_single_tiles(step, group: int, nkv: int, device):
     q = np.diff(np.asarray(step.cu_q_host, dtype=np.int64))
     single = (q > 0) & (q * group <= 16)
     if not single.any() or single.all():

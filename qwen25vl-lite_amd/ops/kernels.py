@@ -33,7 +33,7 @@ _functions: Dict[Tuple[str, str, Tuple], ctypes._CFuncPtr] = {}
 
 
 def _fn(stem: str, name: str, argtypes, defines=None, restype=_c_int):
-    key = (stem, name, tuple(sorted((defines or {}).items())))
+    key = (stem, name, tuple(sorted(defines.items())) if defines else ())
     fn = _functions.get(key)
     if fn is None:
         fn = getattr(load_library(stem, defines), name)
@@ -52,10 +52,11 @@ _cu_count: Dict[int, int] = {}
 
 
 def compute_units(device) -> int:
-    key = torch.device(device).index or 0
-    if key not in _cu_count:
-        _cu_count[key] = torch.cuda.get_device_properties(key).multi_processor_count
-    return _cu_count[key]
+    key = (device if isinstance(device, torch.device) else torch.device(device)).index or 0
+    count = _cu_count.get(key)
+    if count is None:
+        count = _cu_count[key] = torch.cuda.get_device_properties(key).multi_processor_count
+    return count
 
 
 def dtype_code(dtype: torch.dtype) -> int:
@@ -77,19 +78,28 @@ def _ptr(t: Optional[torch.Tensor]):
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)    # (the tensors at hand have initialised the device)
 
 
 def _stream():
     """The current HIP stream's handle (the short way where this PyTorch has it: the call is made
     once per kernel launch)."""
     if _raw_stream is not None:
-        return _raw_stream(torch.cuda.current_device())
+        return _raw_stream(_current_device())
     return torch.cuda.current_stream().cuda_stream
 
 
 def _need(cond: bool, msg: str) -> None:
     if not cond:
         raise KernelError(msg)
+
+
+def int32_to_device(host, device) -> torch.Tensor:
+    """A numpy int32 array on the device.  On a GPU it goes by way of pinned memory: the copy takes its place in the stream, where one
+    from other memory makes the host wait for all work queued before it."""
+    staged = torch.empty(host.size, dtype=torch.int32, pin_memory=torch.device(device).type == "cuda")
+    staged.numpy()[:] = host
+    return staged.to(device, non_blocking=True)
 
 
 # --------------------------------------------------------------------------------------------

@@ -14,7 +14,7 @@ import numpy as np
 
 import torch
 
-from .kernels import _check, _dev, _fn, _need, _ptr, _stream, dtype_code
+from .kernels import _check, _dev, _fn, _need, _ptr, _stream, dtype_code, int32_to_device
 
 __all__ = ["decayed_scan", "scan_groups", "chunked_scan", "plan_chunks", "ChunkPlan", "MAX_KEY_SIZE", "CHUNK"]
 
@@ -163,7 +163,7 @@ def plan_chunks(cu_q_host: Sequence[int], device, chunk_len: int = CHUNK) -> Chu
         first.append(len(bounds) - 1)
     n = len(bounds) - 1
     host = np.concatenate([np.asarray(bounds, np.int32), np.arange(n, dtype=np.int32), np.asarray(first, np.int32)])
-    dev = torch.from_numpy(host).to(device)
+    dev = int32_to_device(host, device)
     return ChunkPlan(n, chunk_len, dev[:n + 1], dev[n + 1:2 * n + 1], dev[2 * n + 1:])
 
 
