@@ -251,8 +251,10 @@ def _launch(logits: torch.Tensor, rows: np.ndarray, flat: List[int], wait: bool 
     """Send the rows' settings to the device and queue the sampler (see :func:`_queue`)."""
     vocab = logits.shape[1]
     draws = rows["temperature"] > 0
-    flags = (draws.any(), (draws & (rows["prev_end"] > rows["prev_begin"])).any(),
-             (draws & (rows["top_k"] > 0) & (rows["top_k"] < vocab)).any(), (draws & (rows["top_p"] < 1.0)).any())
+    flags = (False,) * 4
+    if draws.any():
+        flags = (True, (draws & (rows["prev_end"] > rows["prev_begin"])).any(),
+                 (draws & (rows["top_k"] > 0) & (rows["top_k"] < vocab)).any(), (draws & (rows["top_p"] < 1.0)).any())
     with torch.cuda.device(logits.device):
         buf = _Staging.to_device(np.concatenate([rows.view(np.int32), _int32_ids(flat)]), logits.device)
         return _queue(logits, buf, *flags, wait)
