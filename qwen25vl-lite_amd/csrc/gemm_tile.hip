@@ -192,15 +192,47 @@ static Plan plan_for(int M, int N, int K, int most_splits, int cus) {
 
 #define MOST_SPLITS 12
 
+// Where the library is left a product: by an estimate among the four shapes of powers of two alone.  With far fewer blocks
+// than compute units the library, which cuts K by itself, is faster, and the other shapes' more blocks for the same work do not move that
+// line: of 40 products that they alone would take over it the library was the faster in 35 (2,560 x 8,192, 1,991 rows: 79 us against 87;
+// 7,168 x 2,368, 605: 29 and 36; 3,584 x 4,736, 2,396: 77 and 75), by 4 per cent on average.
+struct Count {
+  long long blocks;
+  int splits;
+};
+static Count count_for(int M, int N, int K, int most_splits, int cus) {
+  static const TileShape COUNTED[4] = {{256, 256, 1, 1.08, 1.43}, {128, 256, 1, 0.72, 0.96}, {256, 128, 1, 0.79, 0.94}, {128, 128, 2, 0.53, 1.02}};
+  const int steps = (K + 63) / 64;
+  double least = 1e30;
+  Count count{0, 1};
+  for (const TileShape& s : COUNTED) {
+    const long long tiles = (long long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+    for (int splits = 1; splits <= most_splits && (splits == 1 || splits * 4 <= steps); ++splits) {
+      const long long blocks = tiles * splits, room = (long long)cus * s.a_unit, whole = blocks / room;
+      const double rest = (double)(blocks - whole * room) / room, depth = (steps + splits - 1) / splits;
+      const double busy = s.a_unit == 1 ? rest : (2.0 * rest > 1.0 ? 1.0 : 0.0);
+      double us = whole * (depth * s.full + 4.0);
+      if (rest > 0) us += depth * (s.alone + (s.full - s.alone) * busy) + 4.0;
+      if (splits > 1) us += splits * (double)M * N * 8.0 / 4.5e6;
+      if (us < least) least = us, count = Count{tiles, splits};
+    }
+  }
+  return count;
+}
+static long long uncut_blocks(int M, int N, int K, int cus) { return count_for(M, N, K, 1, cus).blocks; }
+
+// Ranges of K that tile_slabs (tile.py) takes; 0: the library's product, which a cut does not beat and whose tiles are too few (as in
+// prefers_tile, under three quarters of the compute units).  Measured where the shapes of count_for would not be cut, one float32 slab by the
+// others against the library: 8,192 x 3,584, 626 rows, 50 us and 41; 4,608 x 9,472, 2,155 rows, 167 and 151; by 7 per cent on average of 14.
 extern "C" int qvl_gemm_tile_splits(int M, int N, int K, int cus) {
   if (M <= 0 || N <= 0 || K <= 0 || cus <= 0) return 0;
+  if (4 * uncut_blocks(M, N, K, cus) < 3ll * cus && count_for(M, N, K, MOST_SPLITS, cus).splits == 1) return 0;
   return plan_for(M, N, K, MOST_SPLITS, cus).splits;
 }
-// Blocks of the uncut product: with far fewer than compute units the library, which cuts K by itself, is faster.
+// Blocks of the uncut product, which prefers_tile (tile.py) holds against the compute units.
 extern "C" int qvl_gemm_tile_blocks(int M, int N, int K, int cus) {
   if (M <= 0 || N <= 0 || K <= 0 || cus <= 0) return 0;
-  const TileShape& s = SHAPES[plan_for(M, N, K, 1, cus).tile];
-  const long long blocks = (long long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+  const long long blocks = uncut_blocks(M, N, K, cus);
   return (int)(blocks < 0x7fffffff ? blocks : 0x7fffffff);
 }
 

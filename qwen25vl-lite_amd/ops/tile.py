@@ -38,8 +38,8 @@ def prefers_tile(x: torch.Tensor, weight: torch.Tensor, halves: bool = False, ga
     """Whether the kernel takes the product and is the faster way to it, uncut: more than ``MANY_ROWS`` rows, and tiles for
     three quarters of the compute units (2,048 x 3,584 x 3,584: 224 tiles, 54 us against the library's 66; 280 x 2,560 x
     2,048: 60 tiles, 34 against 24, the library cuts the inner size).  With a gated activation on the sums (``gated``), which
-    takes the library another kernel, half of them suffice (22,016 x 2,048: 100 rows, 172 tiles, 29 us against 35; 190 rows,
-    172 tiles, 37 against 41; 380 rows, 172 tiles, 52 against 53; 37,888 x 3,584, 190 rows, 148 tiles, 83 against 89)."""
+    takes the library another kernel, half of them suffice (22,016 x 2,048: 100 rows, 29 us against
+    35; 200 rows, 35 against 41; 350 rows, 42 against 53; 37,888 x 3,584, 200 rows, 76 against 89)."""
     if x.shape[0] <= MANY_ROWS or not takes_tile(x, weight, halves):
         return False
     cus = compute_units(x.device)
@@ -89,7 +89,7 @@ def tile_slabs(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:
     m, k = x.shape
     n = weight.shape[0]
     splits = int(_fn("gemm_tile", "qvl_gemm_tile_splits", [_c_int] * 4)(m, n, k, compute_units(x.device)))
-    if splits <= 1 and (_stored_whole(m * n, k) or not prefers_tile(x, weight)):
+    if splits < 1 or (splits == 1 and _stored_whole(m * n, k)):
         return None
     out = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
     return _launch(x, weight, out, n, _SLABS, splits=splits)
