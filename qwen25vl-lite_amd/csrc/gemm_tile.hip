@@ -3,7 +3,7 @@
 // groups of 8 + 8, or gate rows first), or float32 slabs over ranges of K for whoever adds them next.
 //
 // The inner loop is tile_product.h's.  Tiles of 256 x 256 run fastest, others where a device of 256
-// compute units would otherwise stand half empty or rows be padded; the choice is by an estimate of the time (plan_for).  Measured, the
+// compute units would otherwise stand half empty or rows be padded; the choice is by an estimate of the time (shape_for).  Measured, the
 // library's product (with the activation's kernel behind it where there is one) in brackets: 2,048 x 37,888 x 3,584
 // gated 421 us (624), 2,048 x 3,584 x 18,944 in two ranges 204 (377), 281 x 22,016 x 2,048 gated 37 (55), 281 x 2,048 x 11,008 in ranges 23
 // (50), 281 x 2,048 x 2,048 in ranges 10 (20).
@@ -148,17 +148,12 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(TileArgs p) {
   }
 }
 
-// How a product is cut: the tile's shape and the ranges of K.  The estimate is of microseconds: a step of 64 values
+// The tile's shape for a product in `splits` ranges of K.  The estimate is of microseconds: a step of 64 values
 // costs a block `alone` where most compute units are idle and `full` where all work (with every matrix core busy the clock and the
 // caches give way), a launch 3 us and each of its rounds 2.9 (the first fetches, the stores); results are written at 5.9 TB/s and read once
 // more at 4.5; and W comes at 7.5 TB/s at most, which joins the rest as the root of squares.  Where two blocks share a compute unit, a last
 // round of up to half the room has a unit for each block, else some blocks have to share.  Fitted to 124 products of 70 to 4,096 rows at
-// the 3B, 7B and 72B decoders' sizes, each with all shapes and cuts (rms 6 per cent): what it chooses takes 0.8 per cent longer than the best
-// on average, 12 at most; the estimate before, among the first four shapes, 5.0 and 36.
-struct Plan {
-  int tile, splits;
-  double us;
-};
+// the 3B, 7B and 72B decoders' sizes, each with all shapes and cuts (rms 6 per cent).
 struct TileShape {
   int bn, bm, a_unit;     // blocks a compute unit holds
   double alone, full;
@@ -169,33 +164,39 @@ static const TileShape SHAPES[SHAPES_N] = {{256, 256, 1, 0.967, 1.361}, {128, 25
                                            {192, 256, 1, 0.784, 1.089}, {192, 320, 1, 0.992, 1.362}, {128, 320, 1, 0.758, 0.985},
                                            {256, 192, 1, 0.888, 1.129}};
 
-static Plan plan_for(int M, int N, int K, int most_splits, int cus) {
-  Plan best{0, 1, 1e30};
+static int shape_for(int M, int N, int K, int splits, int cus) {
+  int best = 0;
+  double least = 1e30;
   const int steps = (K + 63) / 64;
   const double memory = 3.0 + (double)N * K * 2.0 / 7.52e6;
   for (int i = 0; i < SHAPES_N; ++i) {
     const TileShape& s = SHAPES[i];
-    const long long tiles = (long long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
-    for (int splits = 1; splits <= most_splits && (splits == 1 || splits * 4 <= steps); ++splits) {
-      const long long blocks = tiles * splits, room = (long long)cus * s.a_unit, whole = blocks / room;
-      const double rest = (double)(blocks - whole * room) / room;
-      const double depth = (steps + splits - 1) / splits, bytes = (double)M * N * (splits > 1 ? 4.0 * splits : 2.0);
-      double us = 3.0 + whole * (depth * s.full + 2.9) + bytes / 5.92e6;
-      const double busy = s.a_unit == 1 ? rest : (2.0 * rest > 1.0 ? 1.0 : 0.0);
-      if (rest > 0) us += depth * (s.alone + (s.full - s.alone) * busy) + 2.9;
-      us = sqrt(us * us + memory * memory) + bytes / 4.5e6;
-      if (us < best.us) best = Plan{i, splits, us};
-    }
+    const long long blocks = (long long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn) * splits, room = (long long)cus * s.a_unit;
+    const long long whole = blocks / room;
+    const double rest = (double)(blocks - whole * room) / room;
+    const double depth = (steps + splits - 1) / splits, bytes = (double)M * N * (splits > 1 ? 4.0 * splits : 2.0);
+    double us = 3.0 + whole * (depth * s.full + 2.9) + bytes / 5.92e6;
+    const double busy = s.a_unit == 1 ? rest : (2.0 * rest > 1.0 ? 1.0 : 0.0);
+    if (rest > 0) us += depth * (s.alone + (s.full - s.alone) * busy) + 2.9;
+    us = sqrt(us * us + memory * memory) + bytes / 4.5e6;
+    if (us < least) least = us, best = i;
   }
   return best;
 }
 
 #define MOST_SPLITS 12
 
-// Where the library is left a product: by an estimate among the four shapes of powers of two alone.  With far fewer blocks
-// than compute units the library, which cuts K by itself, is faster, and the other shapes' more blocks for the same work do not move that
-// line: of 40 products that they alone would take over it the library was the faster in 35 (2,560 x 8,192, 1,991 rows: 79 us against 87;
-// 7,168 x 2,368, 605: 29 and 36; 3,584 x 4,736, 2,396: 77 and 75), by 4 per cent on average.
+// How many ranges K is cut into, and which products are left to the library: by an estimate among the four shapes of powers of two alone,
+// whatever shape then runs.
+//
+// The ranges set the order of an output's sum, and a product that is cut hands its sums on in float32 where one that is not may round them to
+// bfloat16: the shapes above change neither.  Ranges by the estimate above, fitted on 256 compute units, gave up float32 sums on parts of a
+// device (2,048 x 2,048, 1,031 rows, 128 units: three slabs here, none by it) and gained nothing over sixteen whole passes (fitted and here: 2,048
+// rows at 7B sizes 7,239 us and 7,265, portions of 2,048 beside long contexts 28.67 ms and 28.84, a Gogudra pass 12.35 and 12.23).
+//
+// With far fewer blocks than compute units the library, which cuts K by itself, is faster, and the other shapes' more blocks for the same
+// work do not move that line: of 40 products that they alone would take over it the library was the faster in 35 (2,560 x 8,192, 1,991 rows:
+// 79 us against 87; 7,168 x 2,368, 605: 29 and 36; 3,584 x 4,736, 2,396: 77 and 75), by 4 per cent on average.
 struct Count {
   long long blocks;
   int splits;
@@ -211,7 +212,7 @@ static Count count_for(int M, int N, int K, int most_splits, int cus) {
       const long long blocks = tiles * splits, room = (long long)cus * s.a_unit, whole = blocks / room;
       const double rest = (double)(blocks - whole * room) / room, depth = (steps + splits - 1) / splits;
       const double busy = s.a_unit == 1 ? rest : (2.0 * rest > 1.0 ? 1.0 : 0.0);
-      double us = whole * (depth * s.full + 4.0);
+      double us = 8.0 + whole * (depth * s.full + 4.0);
       if (rest > 0) us += depth * (s.alone + (s.full - s.alone) * busy) + 4.0;
       if (splits > 1) us += splits * (double)M * N * 8.0 / 4.5e6;
       if (us < least) least = us, count = Count{tiles, splits};
@@ -219,20 +220,16 @@ static Count count_for(int M, int N, int K, int most_splits, int cus) {
   }
   return count;
 }
-static long long uncut_blocks(int M, int N, int K, int cus) { return count_for(M, N, K, 1, cus).blocks; }
 
-// Ranges of K that tile_slabs (tile.py) takes; 0: the library's product, which a cut does not beat and whose tiles are too few (as in
-// prefers_tile, under three quarters of the compute units).  Measured where the shapes of count_for would not be cut, one float32 slab by the
-// others against the library: 8,192 x 3,584, 626 rows, 50 us and 41; 4,608 x 9,472, 2,155 rows, 167 and 151; by 7 per cent on average of 14.
+// Ranges of K that tile_slabs (tile.py) takes.
 extern "C" int qvl_gemm_tile_splits(int M, int N, int K, int cus) {
   if (M <= 0 || N <= 0 || K <= 0 || cus <= 0) return 0;
-  if (4 * uncut_blocks(M, N, K, cus) < 3ll * cus && count_for(M, N, K, MOST_SPLITS, cus).splits == 1) return 0;
-  return plan_for(M, N, K, MOST_SPLITS, cus).splits;
+  return count_for(M, N, K, MOST_SPLITS, cus).splits;
 }
 // Blocks of the uncut product, which prefers_tile (tile.py) holds against the compute units.
 extern "C" int qvl_gemm_tile_blocks(int M, int N, int K, int cus) {
   if (M <= 0 || N <= 0 || K <= 0 || cus <= 0) return 0;
-  const long long blocks = uncut_blocks(M, N, K, cus);
+  const long long blocks = count_for(M, N, K, 1, cus).blocks;
   return (int)(blocks < 0x7fffffff ? blocks : 0x7fffffff);
 }
 
@@ -257,7 +254,7 @@ extern "C" int qvl_gemm_tile(const void* x, long long ldx, const void* w, long l
   p.x = (const bf16_t*)x; p.ldx = ldx; p.w = (const bf16_t*)w; p.ldw = ldw; p.out = out; p.ldo = ldo;
   p.M = M; p.N = N; p.K = K; p.rows = mode == 3 ? N / 2 : N; p.splits = splits; p.relu2 = relu2; p.gelu = gelu;
   p.alpha = alpha; p.limit = limit; p.shift = shift;
-  int shape = tile >= 0 ? tile : plan_for(M, N, K, mode == 1 && splits > 1 ? MOST_SPLITS : 1, cus).tile;
+  int shape = tile >= 0 ? tile : shape_for(M, N, K, splits, cus);
   if ((unsigned long long)SHAPES[shape].bm * ldx * 2 >= 0xffff0000ull) shape = 0;
   const TileShape& s = SHAPES[shape];
   const int out_n = mode == 3 ? s.bn / 2 : s.bn;

@@ -69,27 +69,16 @@ def tile_product(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype =
     return _launch(x, weight, out, out.stride(0), _SLABS if out_dtype == torch.float32 else _STORE, relu2=int(relu2), shape=shape)
 
 
-# An uncut product that joins the residual is stored in bfloat16 up to this inner size, and from some number of results on up to a longer one.
-# Beyond, products are cut at most numbers of rows, and keep their float32 sums at the others too: which shape and cut is faster
-# changes from one number of rows to the next (3,584 x 18,944: 1,500 rows in ranges, 1,600 not, 2,000 in ranges), a result's precision does
-# not.  That is 10 us of 410 at 4,096 rows of the latter.
-WHOLE_K, WHOLE_RESULTS, LONG_K = 2560, 6 << 20, 6144
-
-
-def _stored_whole(results: int, k: int) -> bool:
-    return k <= WHOLE_K or (k <= LONG_K and results >= WHOLE_RESULTS)
-
-
 def tile_slabs(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:
     """Float32 slabs ``[splits, M, N]`` over ranges of the inner size, whose sum in order is ``x @ weight.T``; None where the
-    kernel does not take the product or is faster without a cut (long inner sizes: one slab).  Cutting pays where the tiles alone leave compute units
+    kernel does not take the product or is faster without a cut.  Cutting pays where the tiles alone leave compute units
     idle: 2,048 x 3,584 x 18,944 has 112 tiles of 256 x 256, two ranges take 204 us and one of 192 x 256 234 (the library 377)."""
     if x.shape[0] <= MANY_ROWS or not takes_tile(x, weight):
         return None
     m, k = x.shape
     n = weight.shape[0]
     splits = int(_fn("gemm_tile", "qvl_gemm_tile_splits", [_c_int] * 4)(m, n, k, compute_units(x.device)))
-    if splits < 1 or (splits == 1 and _stored_whole(m * n, k)):
+    if splits <= 1:
         return None
     out = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
     return _launch(x, weight, out, n, _SLABS, splits=splits)

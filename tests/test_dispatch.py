@@ -67,3 +67,16 @@ def test_sampler_settings_gathered_by_native_code():
         assert S._gather(call["params"], call["prev"], call["steps"], 100, host)[0] == 13
         call.update(odd)
         assert S._gather(call["params"], call["prev"], call["steps"], 100, host)[0] == -1, odd
+
+
+@pytest.mark.parametrize("m, n, k, units, ranges", [
+    (1031, 2048, 2048, 128, 3), (1031, 2048, 2048, 256, 1), (281, 2048, 2048, 256, 4), (281, 2048, 11008, 256, 5), (512, 3584, 3584, 256, 2),
+    (1600, 3584, 18944, 256, 2), (2048, 3584, 18944, 256, 2), (3200, 3584, 18944, 256, 1), (700, 8192, 29568, 256, 5),
+    (200, 2560, 2048, 64, 3), (300, 4608, 3584, 32, 1), (65, 64, 32, 256, 1), (5000, 8192, 8192, 304, 1)])
+def test_ranges_of_the_inner_size_do_not_follow_the_tiles_shape(m, n, k, units, ranges):
+    """How many ranges a product is cut into decides the order of its sums and whether they stay in float32: by the four
+    shapes' estimate on any number of compute units, as these counts were before there were more shapes."""
+    import ctypes
+
+    from qwen25vl_lite_amd.ops.kernels import _fn
+    assert _fn("gemm_tile", "qvl_gemm_tile_splits", [ctypes.c_int] * 4)(m, n, k, units) == ranges
