@@ -495,6 +495,10 @@ __global__ __launch_bounds__(THREADS) void sample_short_kernel(const RowParams* 
         if (key[i] < s_cut) w[i] = 0.f;
     }
   }
+  bool left = false;        // (a min-p above 1 leaves nothing)
+#pragma unroll
+  for (int i = 0; i < PER; ++i) left |= w[i] > 0.f;
+  done = __syncthreads_or(done && left);
   if (!done) {
     for (int i = tid; i < 3 * BINS; i += THREADS) {
       (&r.count[0][0])[i] = 0u;
@@ -504,7 +508,6 @@ __global__ __launch_bounds__(THREADS) void sample_short_kernel(const RowParams* 
     return;
   }
   // what is left, in the order of the indices
-  __syncthreads();
 #pragma unroll
   for (int i = 0; i < PER; ++i)
     if (w[i] > 0.f) {

@@ -585,6 +585,22 @@ def test_sampler_of_lists_and_of_whole_rows(vocab):
     assert all(0 <= t < vocab for t in ids)
 
 
+@pytest.mark.parametrize("vocab", [900, 5003, 152064])
+def test_sampler_where_min_p_leaves_nothing(vocab):
+    """A min_p above 1 (which the engine refuses, the sampler takes) leaves no token: the first one, whether or not the
+    largest score is within rounding of the bound, beside rows that are as they are alone."""
+    from qwen25vl_lite_amd.sampling import SamplingParams
+    from qwen25vl_lite_amd.sampling.sampler import sample_rows, sample_rows_begin
+    kinds = [dict(min_p=p, **more) for p in (1.001, 1.02, 1.04, 1.05, 2.0) for more in ({}, dict(top_k=20), dict(top_p=0.9))] + [dict(top_k=1)]
+    params = [SamplingParams(temperature=1.0, seed=i, **k) for i, k in enumerate(kinds)]
+    n = len(params)
+    logits = torch.randn(n, vocab, generator=torch.Generator().manual_seed(vocab))
+    logits[:, 7] = 20.0
+    want = [0] * (n - 1) + [7]
+    assert sample_rows(logits.cuda(), params, [[]] * n, [0] * n) == want
+    assert sample_rows_begin(logits.cuda(), params, [[]] * n, [0] * n).result() == want
+
+
 def test_trace_run_program(model_dirs, tmp_path):
     """bin/trace_run as a user calls it: JSON steps on standard input, `done <step>` lines,
     <step>.f32 files of little-endian float32 [wanted, vocab]."""
