@@ -10,6 +10,7 @@ without a seed draw theirs here, from the global generator.
 from __future__ import annotations
 
 import ctypes
+from collections import deque
 from typing import List, Optional, Sequence
 
 import numpy as np
@@ -58,38 +59,43 @@ def _int32_ids(flat: Sequence) -> np.ndarray:
     return np.asarray([int(t) for t in flat], np.int32)   # other types than Python's and numpy's, or arrays of one id each
 
 
-class _Staging:
-    """Pinned host buffers that take turns carrying the sampler's per-row settings to the device:
-    a copy from pinned memory does not make the host wait for the work queued before it."""
+class _Pinned:
+    """Pinned host buffers of int32, each with its event and one holder from :meth:`take` to :meth:`give`, on any thread.
+    Of those given back ``KEPT`` a device stay; ``idle`` of them are left alone, so that a copy asked for lately is not waited for."""
+    KEPT = 8
 
-    _rings = {}
+    def __init__(self, idle: int, least: int):
+        self._idle, self._least, self._free = idle, least, {}
 
-    @classmethod
-    def take(cls, words: int, device: torch.device):
-        """A buffer of at least ``words`` int32 that no copy reads any more: ``(host tensor, event)``."""
-        key = device.index or 0
-        ring = cls._rings.setdefault(key, {"turn": -1, "slots": [None] * 4})
-        turn = ring["turn"] = (ring["turn"] + 1) % len(ring["slots"])
-        slot = ring["slots"][turn]
+    def take(self, words: int, device: torch.device):
+        """A buffer of at least ``words`` that no copy uses any more: ``(host tensor, event)``."""
+        free = self._free.setdefault(device.index or 0, deque())
+        try:
+            slot = free.popleft() if len(free) > self._idle else None
+        except IndexError:          # (another thread was faster)
+            slot = None
         if slot is None or slot[0].numel() < words:
-            slot = ring["slots"][turn] = (torch.empty(max(8192, 2 * words), dtype=torch.int32, pin_memory=True), torch.cuda.Event())
-        else:
-            slot[1].synchronize()       # the copy that last read this buffer is done
+            return torch.empty(max(self._least, 2 * words), dtype=torch.int32, pin_memory=True), torch.cuda.Event()
+        slot[1].synchronize()       # the copy that last used this buffer is done
         return slot
 
-    @staticmethod
-    def send(slot, words: int, device: torch.device) -> torch.Tensor:
-        host, copied = slot
-        buf = torch.empty(words, dtype=torch.int32, device=device)
-        buf.copy_(host[:words], non_blocking=True)
-        copied.record()
-        return buf
+    def give(self, slot, device: torch.device) -> None:
+        free = self._free.setdefault(device.index or 0, deque())
+        if len(free) < self.KEPT:
+            free.append(slot)
 
-    @classmethod
-    def to_device(cls, packed: np.ndarray, device: torch.device) -> torch.Tensor:
-        slot = cls.take(packed.size, device)
-        slot[0].numpy()[:packed.size] = packed
-        return cls.send(slot, packed.size, device)
+
+_up, _down = _Pinned(3, 8192), _Pinned(0, 256)      # the rows' settings on their way to the device, sampled ids on theirs to the host
+
+
+def _send(slot, words: int, device: torch.device) -> torch.Tensor:
+    """The buffer's first ``words`` on the device; the buffer is given back."""
+    host, copied = slot
+    buf = torch.empty(words, dtype=torch.int32, device=device)
+    buf.copy_(host[:words], non_blocking=True)
+    copied.record()
+    _up.give(slot, device)
+    return buf
 
 
 _ROW_WORDS = _ROW.itemsize // 4
@@ -113,30 +119,24 @@ _gather_fn = None
 
 class PendingSample:
     """Sampled ids that are on their way: ``device_ids`` (int32 ``[M]``, valid for kernels queued
-    after the sampler on the same stream) and a copy to pinned host memory whose end an event
-    marks.  :meth:`result` waits for that copy only, not for work queued after it."""
+    after the sampler on the same stream) and :meth:`result`, which waits for the host copy."""
 
-    _pinned = {}     # device index -> ring of pinned int32 buffers, so that two samples can be pending
-    _turn = {}
+    _slot = None
 
     def __init__(self, device_ids: torch.Tensor):
-        m = device_ids.numel()
-        key = device_ids.device.index or 0
-        ring = self._pinned.setdefault(key, [None] * 4)
-        turn = self._turn[key] = (self._turn.get(key, -1) + 1) % len(ring)
-        if ring[turn] is None or ring[turn].numel() < m:
-            ring[turn] = torch.empty(max(256, m), dtype=torch.int32, pin_memory=True)
         self.device_ids = device_ids
-        self._host = ring[turn][:m]
-        self._host.copy_(device_ids, non_blocking=True)
-        self._event = torch.cuda.Event()
-        self._event.record()
-        self._ids: Optional[List[int]] = None
+        self._slot = host, event = _down.take(device_ids.numel(), device_ids.device)
+        host[:device_ids.numel()].copy_(device_ids, non_blocking=True)
+        event.record()
 
     def result(self) -> List[int]:
-        if self._ids is None:
-            self._event.synchronize()
-            self._ids = self._host.tolist()
+        slot = self._slot
+        if slot is not None:
+            slot[1].synchronize()
+            # of several threads the first keeps its ids, and gives the buffer back only then
+            self.__dict__.setdefault("_ids", slot[0][:self.device_ids.numel()].tolist())
+            if self.__dict__.pop("_slot", None) is not None:
+                _down.give(slot, self.device_ids.device)
         return self._ids
 
 
@@ -177,13 +177,15 @@ def _sample_rows(logits, params, prev_ids, steps, uniforms, wait: bool):
         return _launch(logits, rows, flat, wait)
     if uniforms is None:
         with torch.cuda.device(logits.device):
-            slot = _Staging.take(m * _ROW_WORDS + 1, logits.device)
+            slot = _up.take(m * _ROW_WORDS + 1, logits.device)
             words, flags = _gather(params, prev_ids, steps, vocab, slot[0])
             if words < -1:
-                slot = _Staging.take(-words, logits.device)
+                _up.give(slot, logits.device)
+                slot = _up.take(-words, logits.device)
                 words, flags = _gather(params, prev_ids, steps, vocab, slot[0])
             if words > 0:
-                return _queue(logits, _Staging.send(slot, words, logits.device), *flags, wait)
+                return _queue(logits, _send(slot, words, logits.device), *flags, wait)
+            _up.give(slot, logits.device)
     filled = []
     for i, p in enumerate(params):
         need_prev = p.repetition_penalty != 1.0 or p.presence_penalty != 0.0 or p.frequency_penalty != 0.0
@@ -256,8 +258,10 @@ def _launch(logits: torch.Tensor, rows: np.ndarray, flat: List[int], wait: bool 
         flags = (True, (draws & (rows["prev_end"] > rows["prev_begin"])).any(),
                  (draws & (rows["top_k"] > 0) & (rows["top_k"] < vocab)).any(), (draws & (rows["top_p"] < 1.0)).any())
     with torch.cuda.device(logits.device):
-        buf = _Staging.to_device(np.concatenate([rows.view(np.int32), _int32_ids(flat)]), logits.device)
-        return _queue(logits, buf, *flags, wait)
+        packed = np.concatenate([rows.view(np.int32), _int32_ids(flat)])
+        slot = _up.take(packed.size, logits.device)
+        slot[0].numpy()[:packed.size] = packed
+        return _queue(logits, _send(slot, packed.size, logits.device), *flags, wait)
 
 
 def _queue(logits: torch.Tensor, buf: torch.Tensor, draws, penalised, top_k, top_p, wait: bool):

@@ -601,6 +601,32 @@ def test_sampler_where_min_p_leaves_nothing(vocab):
     assert sample_rows_begin(logits.cuda(), params, [[]] * n, [0] * n).result() == want
 
 
+def test_pending_samples_keep_their_ids():
+    """Ids that are read late are the call's own, however many calls came in between, each of them waited for or not, and of whole rows
+    or not; so are settings that another holder's buffer stands between."""
+    from qwen25vl_lite_amd.sampling import SamplingParams
+    from qwen25vl_lite_amd.sampling import sampler as S
+    m, vocab = 3, 4000
+    greedy, whole = SamplingParams(), SamplingParams(temperature=1.0, seed=1)
+
+    def logits(token):
+        return torch.zeros(m, vocab, device="cuda").index_fill_(1, torch.tensor([token], device="cuda"), 60.0)
+    first = S.sample_rows_begin(logits(11), [greedy] * m, [[]] * m, [0] * m)
+    for token in (21, 22, 23):
+        assert S.sample_rows(logits(token), [whole] * m, [[]] * m, [0] * m) == [token] * m
+    later = [S.sample_rows_begin(logits(30 + i), [whole if i % 2 else greedy] * m, [[]] * m, [0] * m) for i in range(12)]
+    torch.cuda.synchronize()
+    assert first.result() == [11] * m
+    assert [p.result() for p in reversed(later)] == [[30 + i] * m for i in range(11, -1, -1)]
+    assert first.result() == [11] * m and later[0].result() == [30] * m
+    device = torch.device("cuda", torch.cuda.current_device())
+    held = [S._up.take(100, device) for _ in range(10)]
+    assert len({host.data_ptr() for host, _ in held}) == 10
+    for slot in held:
+        S._up.give(slot, device)
+    assert len(S._up._free[device.index]) == S._Pinned.KEPT
+
+
 def test_trace_run_program(model_dirs, tmp_path):
     """bin/trace_run as a user calls it: JSON steps on standard input, `done <step>` lines,
     <step>.f32 files of little-endian float32 [wanted, vocab]."""
