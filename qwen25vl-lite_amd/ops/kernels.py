@@ -96,8 +96,11 @@ def _need(cond: bool, msg: str) -> None:
 
 def int32_to_device(host, device) -> torch.Tensor:
     """A numpy int32 array on the device.  On a GPU it goes by way of pinned memory: the copy takes its place in the stream, where one
-    from other memory makes the host wait for all work queued before it."""
-    staged = torch.empty(host.size, dtype=torch.int32, pin_memory=torch.device(device).type == "cuda")
+    from other memory makes the host wait for all work queued before it.  A graph would replay the copy from memory that has gone
+    back to its pool: none is recorded into one."""
+    cuda = torch.device(device).type == "cuda"
+    _need(not (cuda and torch.cuda.is_current_stream_capturing()), "a step's lists are made before its graph is captured, not inside")
+    staged = torch.empty(host.size, dtype=torch.int32, pin_memory=cuda)
     staged.numpy()[:] = host
     return staged.to(device, non_blocking=True)
 

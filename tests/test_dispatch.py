@@ -80,3 +80,23 @@ def test_ranges_of_the_inner_size_do_not_follow_the_tiles_shape(m, n, k, units, 
 
     from qwen25vl_lite_amd.ops.kernels import _fn
     assert _fn("gemm_tile", "qvl_gemm_tile_splits", [ctypes.c_int] * 4)(m, n, k, units) == ranges
+
+
+def test_a_steps_lists_are_not_made_inside_a_graph(monkeypatch):
+    """Their way to the device is by host memory that another list takes later: a recorded copy would read that one's numbers."""
+    from qwen25vl_lite_amd.ops import attention_mfma, kernels, linear_attention
+    lists = np.arange(5, dtype=np.int32)
+    assert kernels.int32_to_device(lists, "cpu").tolist() == lists.tolist()
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    assert kernels.int32_to_device(lists, "cpu").tolist() == lists.tolist()
+    for device in ("cuda:0", torch.device("cuda")):
+        with pytest.raises(kernels.KernelError, match="captured"):
+            kernels.int32_to_device(lists, device)
+        with pytest.raises(kernels.KernelError, match="captured"):
+            linear_attention.plan_chunks([0, 7, 9], device)
+
+        class Step:
+            derived, cu_q_host, ctx_len_host = {}, [0, 7, 9], [7, 2]
+        with pytest.raises(kernels.KernelError, match="captured"):
+            attention_mfma._step_tiles(Step, 4, 1, device)
+        assert not Step.derived
