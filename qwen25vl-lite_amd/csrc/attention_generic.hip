@@ -54,8 +54,9 @@ __global__ void attn_generic_kernel(const T* __restrict__ q, const T* __restrict
       s = dot * scale;
     }
     const float m_new = fmaxf(m, wave_max(s));
-    const float pj = valid ? expf(s - m_new) : 0.f;
-    const float alpha = expf(m - m_new);  // m = -inf at first: alpha = 0
+    const float base = m_new > -INFINITY ? m_new : 0.f;   // (scores of -inf alone have no weight beside later ones)
+    const float pj = valid ? expf(s - base) : 0.f;
+    const float alpha = expf(m - base);   // m = -inf at first: alpha = 0
     l = l * alpha + wave_sum(pj);
 #pragma unroll
     for (int i = 0; i < ATTN_MAX_HD / 64; ++i) acc[i] *= alpha;
@@ -180,8 +181,9 @@ __global__ __launch_bounds__(64 * ATTN_WAVES) void attn_generic_vec_kernel(
       if (sub == i && valid) s = dot[i] * scale;
     }
     const float m_new = fmaxf(m, wave_max(s));
-    const float pj = valid ? expf(s - m_new) : 0.f;
-    const float alpha = expf(m - m_new);  // m = -inf at first: alpha = 0
+    const float base = m_new > -INFINITY ? m_new : 0.f;   // (scores of -inf alone have no weight beside later ones or other waves')
+    const float pj = valid ? expf(s - base) : 0.f;
+    const float alpha = expf(m - base);   // m = -inf at first: alpha = 0
     l = l * alpha + wave_sum(pj);
     m = m_new;
     prob[wave][lane] = pj;

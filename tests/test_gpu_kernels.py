@@ -296,6 +296,34 @@ def test_generic_attention_of_long_contexts(dtype, nq, nkv, hd, vd, ps, window, 
     assert torch.allclose(got.double().cpu(), want, **tol), (got.double().cpu() - want).abs().max()
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("hd", [64, 62])
+@pytest.mark.parametrize("low", [(64, 128), (0, 64), (0, 256), (130, 301)])
+def test_generic_attention_beside_scores_of_minus_infinity(dtype, hd, low):
+    """Keys whose scores overflow to minus infinity, whole blocks of them, have no weight beside others: wherever the blocks stand
+    among those that the waves share, with and without a sink."""
+    from qwen25vl_lite_amd.ops import kernels
+    g = torch.Generator().manual_seed(hd + low[0])
+    length, ps = 301, 16
+    q = torch.full((1, 1, hd), 1e20).to(dtype)
+    k = torch.randn(length, hd, generator=g) * 1e-20
+    k[low[0]:low[1]] = -1e20
+    k, v = k.to(dtype), torch.randn(length, hd, generator=g).to(dtype)
+    pages = (length + ps - 1) // ps
+    kc, vc = torch.zeros(pages, 1, ps, hd, dtype=dtype), torch.zeros(pages, 1, hd, ps, dtype=dtype)
+    for j in range(length):
+        kc[j // ps, 0, j % ps], vc[j // ps, 0, :, j % ps] = k[j], v[j]
+    s = (k.double() @ q[0, 0].double()) * hd ** -0.5
+    for sinks in (None, torch.tensor([0.5])):
+        terms = s if sinks is None else torch.cat([s, sinks.double()])
+        want = torch.softmax(terms, 0)[:length] @ v.double()
+        got = kernels.paged_attention_generic(q.reshape(1, -1).cuda(), kc.cuda(), vc.cuda(), torch.arange(pages, dtype=torch.int32).view(1, -1).cuda(),
+                                              torch.zeros(1, dtype=torch.int32).cuda(), torch.tensor([length - 1], dtype=torch.int32).cuda(), 1,
+                                              None, hd ** -0.5, sinks=None if sinks is None else sinks.cuda())
+        tol = dict(atol=2e-5, rtol=1e-4) if dtype == torch.float32 else dict(atol=1.5e-2, rtol=2e-2)
+        assert torch.allclose(got[0].double().cpu(), want, **tol), (sinks, (got[0].double().cpu() - want).abs().max())
+
+
 @pytest.mark.parametrize("split", ["tile", "tile_two_groups", "coop", "coop_split", "coop_split_two_kernels"])
 @pytest.mark.parametrize("nq, nkv, hd, window, ps", [(*s, 16) for s in ATTN_SHAPES if s[2] % 16 == 0]
                          + [s for s in PAGE_SIZES if s[2] % 16 == 0])
