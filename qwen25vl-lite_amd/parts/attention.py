@@ -19,10 +19,11 @@ from .base import (CacheNeed, LayerSlot, Mixer, ParamSpec, PartSpec, StateNeed, 
                    register_part)
 
 # 17 to 64 rows: where the fused kernel does not run, the projection is cut along its inner size (slabs) and the rotation's
-# kernel adds them (10,240 x 8,192, 19 rows: 32 us, the library's product uncut 41).  From 33 rows on that also beats the fused
-# kernel on teams of blocks: up to 48 rows at any inner size (7B sizes: a step of 33 rows 4.14 ms against 4.24, of 48 rows 4.34 against
-# 4.39), up to 64 where it is beyond LONG_K (8 decode steps at 768 keys, 72B sizes, 2 layers: 64 rows 9,962 us against 10,157, 56 9,818
-# and 10,041; 7B sizes, K = 3,584, 8 layers, 64 rows 11,160 and 11,124; 3B sizes, K = 2,048, 6 steps at 256 keys 4,922 and 4,820).
+# kernel adds them (10,240 x 8,192, 19 rows: 32 us, the library's product uncut 41): up to 48 rows at any inner size, up to 64 where it is
+# beyond LONG_K, which the fused kernel does not take with as many rows (8 decode steps at 768 keys, 72B sizes, 2 layers: 64 rows 9,962 us
+# against 10,157 with the library's product, 56 9,818 and 10,041).  From 33 to 48 rows that also beats the fused kernel on teams of blocks (7B
+# sizes: a step of 33 rows 4.14 ms against 4.24, of 48 rows 4.34 against 4.39); from 49 on it does not (7B sizes, K = 3,584, 8 layers, 64 rows
+# 11,160 and 11,124; 3B sizes, K = 2,048, 6 steps at 256 keys 4,922 and 4,820).
 SPLIT_ROWS = (17, 64)
 SHORT_SPLIT_ROWS = 48
 LONG_K = 4096
