@@ -85,6 +85,10 @@ __device__ __forceinline__ bool penalised(const RowParams& p) {
 }
 __device__ __forceinline__ bool cuts_k(const RowParams& p, int V) { return p.temperature > 0.f && p.top_k > 0 && p.top_k < V; }
 __device__ __forceinline__ bool cuts_p(const RowParams& p) { return p.temperature > 0.f && p.top_p < 1.f; }
+// A row that draws from all of its scores, too many for a list.
+__device__ __forceinline__ bool draws_whole(const RowParams& p, int V) {
+  return p.temperature > 0.f && V > LIST && !cuts_k(p, V) && !cuts_p(p) && !(p.min_p > 0.f);
+}
 
 // The row's scores: the penalised ones have been written out, already divided by the temperature.
 struct Scores {
@@ -182,7 +186,7 @@ __global__ __launch_bounds__(THREADS) void sample_scan_kernel(const float* __res
     if (at < M) {
       if (tid == 0) {
         const RowParams p = params[at];
-        scratch[at].listed = 0u;
+        scratch[at].listed = draws_whole(p, V) ? LIST + 1u : 0u;
         scratch[at].all_mass = 0ull;
         if (at == 0) *todo = 0;
         scratch[at].u = p.temperature > 0.f && p.seeded ? first_uniform(p.seed) : p.u;
@@ -284,7 +288,7 @@ __global__ __launch_bounds__(THREADS) void sample_list_kernel(const float* __res
   __shared__ unsigned int s_count, s_base;
   const int m = blockIdx.y, s = blockIdx.x, tid = threadIdx.x;
   const RowParams p = params[m];
-  if (p.temperature <= 0.f) return;
+  if (p.temperature <= 0.f || draws_whole(p, V)) return;
   RowScratch& r = scratch[m];
   const Scores score = scores_of(p, logits, scores, m, V);
   const int lo = s * PIECE, n = min(PIECE, V - lo);
@@ -889,11 +893,13 @@ extern "C" int qvl_sample_params_size() { return (int)sizeof(RowParams); }
 // logits: float32 [M, V].  scores: as large, written for rows that draw with penalties (null if there are none).
 // scratch: M * qvl_sample_scratch_bytes() bytes on a 16-byte boundary, null if no row draws.  parts: M * qvl_sample_parts_bytes(V).
 // out: the rows' tokens, and behind them, if rows draw, how many rows go the long way.
-// top_k, top_p: whether any row has that cut (the passes for it are left out otherwise).
+// top_k, top_p: whether any row has that cut (the passes for it are left out otherwise); cuts: whether any row that draws has a
+// cut (the lists are left out otherwise).
 // ways: 1 the short way, after which out[M] rows have no token yet; 2 the long way for these, with all buffers as the short
 // one left them; 3 both.
 extern "C" int qvl_sample_rows(const void* logits, void* scores, const void* params, const void* prev_ids, void* scratch,
-                               void* parts, void* out, int M, int V, int top_k, int top_p, int ways, hipStream_t stream) {
+                               void* parts, void* out, int M, int V, int top_k, int top_p, int cuts, int ways,
+                               hipStream_t stream) {
   if (M <= 0) return QVL_OK;
   if (V <= 0 || !logits || !params || !prev_ids || !parts || !out) return QVL_ERR_SHAPE;
   if (((uintptr_t)scratch % 16) != 0 || ways < 1 || ways > 3) return QVL_ERR_SHAPE;
@@ -914,7 +920,8 @@ extern "C" int qvl_sample_rows(const void* logits, void* scores, const void* par
     hipLaunchKernelGGL(sample_scan_kernel, dim3(M * pieces + (scratch ? M : 0)), block, 0, stream, lg, sc, rp, (const int*)prev_ids, rs, ap,
                        groups, todo, M, V, pieces);
     if (scratch) {
-      hipLaunchKernelGGL(sample_list_kernel, dim3(pieces, M), block, 0, stream, lg, sc, rp, rs, ap, groups, V, pieces, one);
+      if (cuts || V <= LIST)
+        hipLaunchKernelGGL(sample_list_kernel, dim3(pieces, M), block, 0, stream, lg, sc, rp, rs, ap, groups, V, pieces, one);
       hipLaunchKernelGGL(sample_short_kernel, dim3(M), block, 0, stream, rp, rs, ap, ids, todo, V, pieces, one);
     } else {
       hipLaunchKernelGGL(sample_pick_kernel, dim3(M), block, 0, stream, lg, sc, rp, rs, ap, ids, todo, V, pieces);

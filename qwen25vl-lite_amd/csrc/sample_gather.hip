@@ -63,14 +63,15 @@ bool one_digit(PyObject* v, long& out) {
 }
 bool items(PyObject* s) { return PyList_CheckExact(s) || PyTuple_CheckExact(s); }
 
-long gather(PyObject* params, PyObject* prev, PyObject* steps, long M, long vocab, int32_t* out, long room, int32_t* flags) {
+long gather(PyObject* params, PyObject* prev, PyObject* steps, long M, long vocab, int32_t* out, long room, int32_t* flags,
+            int32_t* more) {
   if (!items(params) || !items(prev) || !items(steps)) return -1;
   if (M * ROW_WORDS + 1 > room) return -(M * ROW_WORDS + 1);
   Row* rows = reinterpret_cast<Row*>(out);
   int32_t* ids = out + M * ROW_WORDS;
   const long id_room = room - M * ROW_WORDS;
   long count = 0;
-  bool draws = false, scores = false, top_k = false, top_p = false;
+  bool draws = false, scores = false, top_k = false, top_p = false, cut = false, whole = false;
   for (long i = 0; i < M; ++i) {
     if (PySequence_Fast_GET_SIZE(params) != M || PySequence_Fast_GET_SIZE(prev) != M || PySequence_Fast_GET_SIZE(steps) != M) return -1;
     PyObject* p = PySequence_Fast_GET_ITEM(params, i);
@@ -127,8 +128,11 @@ long gather(PyObject* params, PyObject* prev, PyObject* steps, long M, long voca
     if (r.temperature > 0.f) {
       draws = true;
       scores |= r.prev_end > r.prev_begin;
-      top_k |= r.top_k > 0 && r.top_k < vocab;
-      top_p |= r.top_p < 1.f;
+      const bool k_cut = r.top_k > 0 && r.top_k < vocab, p_cut = r.top_p < 1.f, any = k_cut || p_cut || r.min_p > 0.f;
+      top_k |= k_cut;
+      top_p |= p_cut;
+      cut |= any;
+      whole |= !any;
     }
   }
   if (count > id_room) return -(M * ROW_WORDS + count);
@@ -137,16 +141,22 @@ long gather(PyObject* params, PyObject* prev, PyObject* steps, long M, long voca
   flags[1] = scores;
   flags[2] = top_k;
   flags[3] = top_p;
+  if (more) {
+    more[0] = cut;
+    more[1] = whole;
+  }
   return M * ROW_WORDS + count;
 }
 
 }  // namespace
 
 // Called with the interpreter's lock held.  out: `room` 32-bit words: M rows, then the generated ids of rows with penalties (one zero
-// if there are none).  flags: whether any row draws, draws with ids, cuts by top-k, by top-p.  Returns the words written;
+// if there are none).  flags: whether any row draws, draws with ids, cuts by top-k, by top-p; more (or null): draws
+// with any cut, with none.  Returns the words written;
 // -1: not taken; -n below that: n words are needed.  No exception is left behind.
-extern "C" long qvl_sample_gather(PyObject* params, PyObject* prev, PyObject* steps, long M, long vocab, void* out, long room, void* flags) {
-  const long n = M < 1 ? -1 : gather(params, prev, steps, M, vocab, (int32_t*)out, room, (int32_t*)flags);
+extern "C" long qvl_sample_gather(PyObject* params, PyObject* prev, PyObject* steps, long M, long vocab, void* out, long room, void* flags,
+                                  void* more) {
+  const long n = M < 1 ? -1 : gather(params, prev, steps, M, vocab, (int32_t*)out, room, (int32_t*)flags, (int32_t*)more);
   if (PyErr_Occurred()) PyErr_Clear();
   return n;
 }

@@ -101,17 +101,18 @@ def _send(slot, words: int, device: torch.device) -> torch.Tensor:
 _ROW_WORDS = _ROW.itemsize // 4
 
 
-def _gather(params, prev_ids, steps, vocab: int, host: torch.Tensor):
+def _gather(params, prev_ids, steps, vocab: int, host: torch.Tensor, more=None):
     """The rows' settings and ids into ``host`` by native code: ``(words, flags)``; words are -1 where a row is not of
-    the usual kind, below that minus the words needed."""
+    the usual kind, below that minus the words needed.  ``more``: two int32 that are told whether any row that draws has a cut, has none."""
     global _gather_fn
     if _gather_fn is None:
         lib = load_library("sample_gather", loader=ctypes.PyDLL)
         _gather_fn = lib.qvl_sample_gather
         _gather_fn.restype = ctypes.c_long
-        _gather_fn.argtypes = [ctypes.py_object] * 3 + [ctypes.c_long] * 2 + [ctypes.c_void_p, ctypes.c_long, ctypes.c_void_p]
+        _gather_fn.argtypes = [ctypes.py_object] * 3 + [ctypes.c_long] * 2 + [ctypes.c_void_p, ctypes.c_long] + [ctypes.c_void_p] * 2
     flags = (ctypes.c_int32 * 4)()
-    return _gather_fn(params, prev_ids, steps, len(params), vocab, host.data_ptr(), host.numel(), ctypes.addressof(flags)), flags
+    return _gather_fn(params, prev_ids, steps, len(params), vocab, host.data_ptr(), host.numel(), ctypes.addressof(flags),
+                      None if more is None else ctypes.addressof(more)), flags
 
 
 _gather_fn = None
@@ -177,14 +178,14 @@ def _sample_rows(logits, params, prev_ids, steps, uniforms, wait: bool):
         return _launch(logits, rows, flat, wait)
     if uniforms is None:
         with torch.cuda.device(logits.device):
-            slot = _up.take(m * _ROW_WORDS + 1, logits.device)
-            words, flags = _gather(params, prev_ids, steps, vocab, slot[0])
+            slot, more = _up.take(m * _ROW_WORDS + 1, logits.device), (ctypes.c_int32 * 2)()
+            words, flags = _gather(params, prev_ids, steps, vocab, slot[0], more)
             if words < -1:
                 _up.give(slot, logits.device)
                 slot = _up.take(-words, logits.device)
-                words, flags = _gather(params, prev_ids, steps, vocab, slot[0])
+                words, flags = _gather(params, prev_ids, steps, vocab, slot[0], more)
             if words > 0:
-                return _queue(logits, _send(slot, words, logits.device), *flags, wait)
+                return _queue(logits, _send(slot, words, logits.device), *flags, *more, wait)
             _up.give(slot, logits.device)
     filled = []
     for i, p in enumerate(params):
@@ -253,10 +254,12 @@ def _launch(logits: torch.Tensor, rows: np.ndarray, flat: List[int], wait: bool 
     """Send the rows' settings to the device and queue the sampler (see :func:`_queue`)."""
     vocab = logits.shape[1]
     draws = rows["temperature"] > 0
-    flags = (False,) * 4
+    flags = (False,) * 6
     if draws.any():
-        flags = (True, (draws & (rows["prev_end"] > rows["prev_begin"])).any(),
-                 (draws & (rows["top_k"] > 0) & (rows["top_k"] < vocab)).any(), (draws & (rows["top_p"] < 1.0)).any())
+        top_k, top_p = (rows["top_k"] > 0) & (rows["top_k"] < vocab), rows["top_p"] < 1.0
+        cut = top_k | top_p | (rows["min_p"] > 0)
+        flags = (True, (draws & (rows["prev_end"] > rows["prev_begin"])).any(), (draws & top_k).any(), (draws & top_p).any(),
+                 (draws & cut).any(), (draws & ~cut).any())
     with torch.cuda.device(logits.device):
         packed = np.concatenate([rows.view(np.int32), _int32_ids(flat)])
         slot = _up.take(packed.size, logits.device)
@@ -264,13 +267,15 @@ def _launch(logits: torch.Tensor, rows: np.ndarray, flat: List[int], wait: bool 
         return _queue(logits, _send(slot, packed.size, logits.device), *flags, wait)
 
 
-def _queue(logits: torch.Tensor, buf: torch.Tensor, draws, penalised, top_k, top_p, wait: bool):
+def _queue(logits: torch.Tensor, buf: torch.Tensor, draws, penalised, top_k, top_p, cut, whole, wait: bool):
     """Queue the sampler for the settings in ``buf`` (the rows, then generated ids): a :class:`PendingSample`.  With ``wait``
-    the ids, and the passes for rows that the short way does not settle are queued only if there are any.
-    ``draws``, ``penalised``, ``top_k``, ``top_p``: whether any row draws, draws with generated ids, has these cuts."""
+    the ids, and the passes for rows that the short way does not settle are queued only if there are any (a row that draws from all of its
+    scores is one, which is known before).
+    ``draws``, ``penalised``, ``top_k``, ``top_p``: whether any row draws, draws with generated ids, has these cuts; ``cut``, ``whole``: draws
+    with a cut, with none."""
     m, vocab = logits.shape
     c_ptr, c_int = ctypes.c_void_p, ctypes.c_int
-    fn = _fn("sample", "qvl_sample_rows", [c_ptr] * 7 + [c_int] * 5 + [c_ptr])
+    fn = _fn("sample", "qvl_sample_rows", [c_ptr] * 7 + [c_int] * 6 + [c_ptr])
     parts_bytes = _fn("sample", "qvl_sample_parts_bytes", [c_int], restype=ctypes.c_longlong)
     dev = logits.device
     scores = scratch = None
@@ -287,8 +292,8 @@ def _queue(logits: torch.Tensor, buf: torch.Tensor, draws, penalised, top_k, top
         at = buf.data_ptr()
         _check(fn(logits.data_ptr(), None if scores is None else scores.data_ptr(), at, at + 4 * _ROW_WORDS * m,
                   None if scratch is None else scratch.data_ptr(), parts.data_ptr(), out.data_ptr(), m, vocab, int(top_k),
-                  int(top_p), ways, _stream()), "sample_rows")
-    if not wait or scratch is None:
+                  int(top_p), int(cut), ways, _stream()), "sample_rows")
+    if not wait or scratch is None or whole:
         queue(_SHORT | _LONG)
         pending = PendingSample(out[:m])
         return pending.result() if wait else pending

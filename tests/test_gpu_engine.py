@@ -627,6 +627,32 @@ def test_pending_samples_keep_their_ids():
     assert len(S._up._free[device.index]) == S._Pinned.KEPT
 
 
+@pytest.mark.parametrize("vocab", [900, 33000])
+def test_rows_without_a_cut_are_waited_for_once(vocab, monkeypatch):
+    """A row that draws from all of its scores has no list, which is known before: its ids are not waited for twice, by any
+    way the settings come, alone and beside rows with lists and greedy ones."""
+    from qwen25vl_lite_amd.sampling import SamplingParams
+    from qwen25vl_lite_amd.sampling import sampler as S
+    g = torch.Generator(device="cuda").manual_seed(vocab)
+    logits = torch.randn(4, vocab, device="cuda", generator=g)
+    whole = [SamplingParams(temperature=1.0, seed=i) for i in range(4)]
+    mixed = [whole[0], SamplingParams(temperature=0.9, top_k=40, seed=1), SamplingParams(), SamplingParams(temperature=1.0, min_p=0.1, top_k=5, seed=9)]
+    for params in (whole, mixed):
+        us = [S.uniform_for(p, 3) for p in params]
+        want = S.sample_rows_begin(logits, params, [[]] * 4, [3] * 4).result()
+        waits, real = [], S.PendingSample
+        monkeypatch.setattr(S, "PendingSample", lambda ids: waits.append(1) or real(ids))
+        assert S.sample_rows(logits, params, [[]] * 4, [3] * 4) == want and len(waits) == 1
+        assert S.sample_rows(logits, params, [[]] * 4, [3] * 4, uniforms=us) == want and len(waits) == 2
+        monkeypatch.setattr(S, "PendingSample", real)
+        for i, p in enumerate(params):
+            probs = torch.softmax(logits[i].double() / (p.temperature or 1.0), 0)
+            if p is whole[i]:          # within rounding of float32 sums of `vocab` masses
+                cdf = float(probs[:want[i] + 1].sum())
+                assert cdf - float(probs[want[i]]) - 2e-5 <= us[i] <= cdf + 2e-5
+        assert [S.sample_rows(logits[i:i + 1], [p], [[]], [3])[0] for i, p in enumerate(params)] == want
+
+
 def test_trace_run_program(model_dirs, tmp_path):
     """bin/trace_run as a user calls it: JSON steps on standard input, `done <step>` lines,
     <step>.f32 files of little-endian float32 [wanted, vocab]."""
