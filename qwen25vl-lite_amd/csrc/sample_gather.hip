@@ -1,7 +1,7 @@
 // Host code: the settings of a sampler call's rows, from the requests' Python objects into the block of 32-bit words that goes to
 // the device.  A loop over 64 requests and 3,100 generated ids in Python takes longer than the sampler's kernels (90 us on the host of
 // an MI355X for 64 requests, this 12).  Whatever is not the usual kind (settings that are no numbers, ids in
-// other containers than lists and tuples or other than Python's integers, rows that draw without a seed) is left to the caller's Python.
+// other containers than lists and tuples or other than Python's integers) is left to the caller's Python.
 #include <Python.h>
 
 #include <cstdint>
@@ -72,6 +72,7 @@ long gather(PyObject* params, PyObject* prev, PyObject* steps, long M, long voca
   const long id_room = room - M * ROW_WORDS;
   long count = 0;
   bool draws = false, scores = false, top_k = false, top_p = false, cut = false, whole = false;
+  int32_t unseeded = 0;
   for (long i = 0; i < M; ++i) {
     if (PySequence_Fast_GET_SIZE(params) != M || PySequence_Fast_GET_SIZE(prev) != M || PySequence_Fast_GET_SIZE(steps) != M) return -1;
     PyObject* p = PySequence_Fast_GET_ITEM(params, i);
@@ -96,7 +97,10 @@ long gather(PyObject* params, PyObject* prev, PyObject* steps, long M, long voca
     r.seed = 0;
     r.seeded = 0;
     r.prev_begin = (int32_t)count;
-    if (v[0] > 0) {
+    if (v[0] > 0 && seed_kind == 2 && more) {
+      r.seeded = -1;        // the caller's to fill in
+      ++unseeded;
+    } else if (v[0] > 0) {
       // the generator's seed: the request's and the number of its tokens
       if (PySequence_Fast_GET_SIZE(steps) != M) return -1;
       long long step = 0;
@@ -144,6 +148,7 @@ long gather(PyObject* params, PyObject* prev, PyObject* steps, long M, long voca
   if (more) {
     more[0] = cut;
     more[1] = whole;
+    more[2] = unseeded;
   }
   return M * ROW_WORDS + count;
 }
@@ -152,7 +157,7 @@ long gather(PyObject* params, PyObject* prev, PyObject* steps, long M, long voca
 
 // Called with the interpreter's lock held.  out: `room` 32-bit words: M rows, then the generated ids of rows with penalties (one zero
 // if there are none).  flags: whether any row draws, draws with ids, cuts by top-k, by top-p; more (or null): draws
-// with any cut, with none.  Returns the words written;
+// with any cut, with none, and how many draw without a seed (`seeded` is -1 in these; without `more` they are not taken).  Returns the words written;
 // -1: not taken; -n below that: n words are needed.  No exception is left behind.
 extern "C" long qvl_sample_gather(PyObject* params, PyObject* prev, PyObject* steps, long M, long vocab, void* out, long room, void* flags,
                                   void* more) {

@@ -103,7 +103,8 @@ _ROW_WORDS = _ROW.itemsize // 4
 
 def _gather(params, prev_ids, steps, vocab: int, host: torch.Tensor, more=None):
     """The rows' settings and ids into ``host`` by native code: ``(words, flags)``; words are -1 where a row is not of
-    the usual kind, below that minus the words needed.  ``more``: two int32 that are told whether any row that draws has a cut, has none."""
+    the usual kind, below that minus the words needed.  ``more``: three int32 that are told whether any row that draws has a cut, has none,
+    and how many draw without a seed; their ``seeded`` is -1 then, where without ``more`` they are not of the usual kind."""
     global _gather_fn
     if _gather_fn is None:
         lib = load_library("sample_gather", loader=ctypes.PyDLL)
@@ -178,14 +179,18 @@ def _sample_rows(logits, params, prev_ids, steps, uniforms, wait: bool):
         return _launch(logits, rows, flat, wait)
     if uniforms is None:
         with torch.cuda.device(logits.device):
-            slot, more = _up.take(m * _ROW_WORDS + 1, logits.device), (ctypes.c_int32 * 2)()
+            slot, more = _up.take(m * _ROW_WORDS + 1, logits.device), (ctypes.c_int32 * 3)()
             words, flags = _gather(params, prev_ids, steps, vocab, slot[0], more)
             if words < -1:
                 _up.give(slot, logits.device)
                 slot = _up.take(-words, logits.device)
                 words, flags = _gather(params, prev_ids, steps, vocab, slot[0], more)
             if words > 0:
-                return _queue(logits, _send(slot, words, logits.device), *flags, *more, wait)
+                if more[2]:
+                    rows = slot[0].numpy()[:m * _ROW_WORDS].view(_ROW)
+                    for i in np.nonzero(rows["seeded"] < 0)[0]:
+                        rows["u"][i], rows["seeded"][i] = uniform_from(None, 0), 0
+                return _queue(logits, _send(slot, words, logits.device), *flags, *more[:2], wait)
             _up.give(slot, logits.device)
     filled = []
     for i, p in enumerate(params):

@@ -110,3 +110,21 @@ def test_which_rows_of_the_stacked_projection_are_cut():
     assert cut[2048] == cut[4096] == list(range(17, 49)) and cut[4104] == cut[8192] == list(range(17, 65))
     for k in (4104, 8192):        # what ran there before is the library's product, not the fused kernel
         assert not any(skinny.takes_resident(m, k, torch.empty((10240, k), dtype=torch.bfloat16, device="meta")) for m in range(33, 65))
+
+
+def test_sampler_settings_of_rows_without_a_seed():
+    """Rows that draw without a seed are gathered with the others and marked, whatever their place among the steps."""
+    import ctypes
+
+    from qwen25vl_lite_amd.sampling import SamplingParams
+    from qwen25vl_lite_amd.sampling import sampler as S
+    params = [SamplingParams(temperature=1.0), SamplingParams(temperature=0.8, top_k=9, seed=5), SamplingParams(), SamplingParams(temperature=0.5, min_p=0.1),
+              SamplingParams(temperature=1e-50)]
+    host, more = torch.zeros(200, dtype=torch.int32), (ctypes.c_int32 * 3)()
+    words, flags = S._gather(params, [[]] * 5, ["any", 2, None, 1.5, 0], 100, host, more)
+    rows = host.numpy()[:60].view(S._ROW)
+    assert words == 61 and list(flags) == [1, 0, 1, 0] and list(more) == [1, 1, 3]
+    assert rows["seeded"].tolist() == [-1, 1, 0, -1, -1] and rows["seed"][1] == 7 and not rows["u"].any()
+    assert S._gather(params, [[]] * 5, [0, 2, 0, 0, 0], 100, host)[0] == -1
+    assert S._gather(params[1:3], [[]] * 2, [2, 0], 100, host, more)[0] == 25 and list(more) == [1, 0, 0]
+    assert S._gather(params[1:3], [[]] * 2, ["2", 0], 100, host, more)[0] == -1

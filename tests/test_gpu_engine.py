@@ -653,6 +653,25 @@ def test_rows_without_a_cut_are_waited_for_once(vocab, monkeypatch):
         assert [S.sample_rows(logits[i:i + 1], [p], [[]], [3])[0] for i, p in enumerate(params)] == want
 
 
+def test_rows_without_a_seed_draw_from_the_global_generator(monkeypatch):
+    """One number a row that draws, in the rows' order, whichever code gathers the settings."""
+    from qwen25vl_lite_amd.sampling import SamplingParams
+    from qwen25vl_lite_amd.sampling import sampler as S
+    logits = torch.randn(5, 30000, device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
+    params = [SamplingParams(temperature=1.0), SamplingParams(), SamplingParams(temperature=1.0, top_k=50), SamplingParams(temperature=1.0, seed=4),
+              SamplingParams(temperature=0.9, top_p=0.8, frequency_penalty=0.1)]
+    args = (logits, params, [[]] * 4 + [[1, 2]], [0, 0, 0, 6, 2])
+    torch.manual_seed(77)
+    us = [S.uniform_for(p, n) for p, n in zip(params, args[3])]
+    after = torch.rand(1).item()
+    want = S.sample_rows(*args, uniforms=us)
+    torch.manual_seed(77)
+    assert S.sample_rows(*args) == want and torch.rand(1).item() == after
+    monkeypatch.setattr(S, "_gather", lambda *a: (-1, None))
+    torch.manual_seed(77)
+    assert S.sample_rows(*args) == want and torch.rand(1).item() == after
+
+
 def test_trace_run_program(model_dirs, tmp_path):
     """bin/trace_run as a user calls it: JSON steps on standard input, `done <step>` lines,
     <step>.f32 files of little-endian float32 [wanted, vocab]."""
