@@ -5,7 +5,7 @@ from __future__ import annotations
 import os
 from typing import List
 
-from .library import build_library
+from .library import build_library, python_headers
 
 __all__ = ["LIBRARIES", "build_everything"]
 
@@ -73,7 +73,9 @@ LIBRARIES = [
 
 
 def build_everything(force: bool = False, quiet: bool = False) -> List[str]:
-    built = [build_library(stem, defines, force=force, quiet=quiet) for stem, defines in LIBRARIES]
+    # (without the interpreter's headers the sampler's settings are gathered in Python)
+    built = [build_library(stem, defines, force=force, quiet=quiet) for stem, defines in LIBRARIES
+             if stem != "sample_gather" or python_headers()]
     # libraries of sources that have changed since are of no use to anyone
     keep = {os.path.basename(p) for p in built}
     for directory in {os.path.dirname(p) for p in built}:

@@ -35,7 +35,7 @@ HIPCC_FLAGS = ("-O3", "-std=c++17", f"--offload-arch={ARCH}", "-shared", "-fPIC"
 SOURCE_FLAGS = {"attention_mfma": ("-fno-honor-nans",),
                 "sample_gather": (f"-I{sysconfig.get_path('include')}",)}     # host code that reads Python objects
 
-_loaded: Dict[Tuple[str, Tuple[Tuple[str, str], ...]], ctypes.CDLL] = {}
+_loaded: Dict[Tuple[str, Tuple[Tuple[str, str], ...], type], ctypes.CDLL] = {}
 _lock = threading.Lock()
 
 
@@ -164,11 +164,16 @@ def build_library(stem: str, defines: Optional[Mapping[str, object]] = None, *, 
     return out
 
 
+def python_headers() -> bool:
+    """Whether this interpreter's headers are there, which one host library needs."""
+    return os.path.isfile(os.path.join(sysconfig.get_path("include"), "Python.h"))
+
+
 def load_library(stem: str, defines: Optional[Mapping[str, object]] = None, loader=ctypes.CDLL) -> ctypes.CDLL:
     """The loaded library of ``csrc/<stem>.hip``; built first if it is not there.  ``loader``: ``ctypes.PyDLL`` for one whose functions
     are called with the interpreter's lock held."""
     defines = dict(defines or {})
-    key = (stem, tuple(sorted((k, str(v)) for k, v in defines.items())))
+    key = (stem, tuple(sorted((k, str(v)) for k, v in defines.items())), loader)
     with _lock:
         lib = _loaded.get(key)
         if lib is None:

@@ -17,7 +17,7 @@ import numpy as np
 import torch
 
 from ..ops.kernels import KernelError, _check, _fn, _stream
-from ..ops.library import load_library
+from ..ops.library import KernelBuildError, load_library
 from .params import SamplingParams
 
 __all__ = ["sample_rows", "sample_rows_begin", "sample_slots_begin", "PendingSample", "uniform_for", "uniform_from"]
@@ -107,11 +107,18 @@ def _gather(params, prev_ids, steps, vocab: int, host: torch.Tensor, more=None):
     and how many draw without a seed; their ``seeded`` is -1 then, where without ``more`` they are not of the usual kind."""
     global _gather_fn
     if _gather_fn is None:
-        lib = load_library("sample_gather", loader=ctypes.PyDLL)
-        _gather_fn = lib.qvl_sample_gather
-        _gather_fn.restype = ctypes.c_long
-        _gather_fn.argtypes = [ctypes.py_object] * 3 + [ctypes.c_long] * 2 + [ctypes.c_void_p, ctypes.c_long] + [ctypes.c_void_p] * 2
+        try:
+            lib = load_library("sample_gather", loader=ctypes.PyDLL)
+        except (KernelBuildError, OSError):      # (no headers of this interpreter, say.)  The caller's loop does the same
+            _gather_fn = False
+        else:
+            fn = lib.qvl_sample_gather
+            fn.restype = ctypes.c_long
+            fn.argtypes = [ctypes.py_object] * 3 + [ctypes.c_long] * 2 + [ctypes.c_void_p, ctypes.c_long] + [ctypes.c_void_p] * 2
+            _gather_fn = fn
     flags = (ctypes.c_int32 * 4)()
+    if _gather_fn is False:
+        return -1, flags
     return _gather_fn(params, prev_ids, steps, len(params), vocab, host.data_ptr(), host.numel(), ctypes.addressof(flags),
                       None if more is None else ctypes.addressof(more)), flags
 

@@ -128,3 +128,42 @@ def test_sampler_settings_of_rows_without_a_seed():
     assert S._gather(params, [[]] * 5, [0, 2, 0, 0, 0], 100, host)[0] == -1
     assert S._gather(params[1:3], [[]] * 2, [2, 0], 100, host, more)[0] == 25 and list(more) == [1, 0, 0]
     assert S._gather(params[1:3], [[]] * 2, ["2", 0], 100, host, more)[0] == -1
+
+
+@pytest.mark.parametrize("error", ["build", "load"])
+def test_sampler_without_its_native_gather(error, monkeypatch):
+    """Where the interpreter's headers are missing the settings are gathered by Python's loop: tried once, refused from then on."""
+    from qwen25vl_lite_amd.ops.library import KernelBuildError
+    from qwen25vl_lite_amd.sampling import SamplingParams
+    from qwen25vl_lite_amd.sampling import sampler as S
+    tried = []
+
+    def missing(stem, **how):
+        tried.append(stem)
+        raise KernelBuildError("Python.h: no such file") if error == "build" else OSError("undefined symbol")
+    monkeypatch.setattr(S, "_gather_fn", None)
+    monkeypatch.setattr(S, "load_library", missing)
+    host = torch.zeros(40, dtype=torch.int32)
+    for _ in range(3):
+        assert S._gather([SamplingParams()], [[]], [0], 100, host)[0] == -1
+    assert tried == ["sample_gather"]
+
+
+@pytest.mark.parametrize("there", [True, False])
+def test_everything_else_is_built_without_the_interpreters_headers(there, monkeypatch, tmp_path):
+    from qwen25vl_lite_amd.ops import build_all
+    stems = []
+    monkeypatch.setattr(build_all, "python_headers", lambda: there)
+    monkeypatch.setattr(build_all, "build_library", lambda stem, defines, **how: stems.append(stem) or str(tmp_path / f"{len(stems)}.so"))
+    assert len(build_all.build_everything()) == len(build_all.LIBRARIES) - (not there)
+    assert ("sample_gather" in stems) == there
+
+
+def test_a_library_is_loaded_as_it_is_asked_for():
+    """A handle whose calls let go of the interpreter's lock is not given to whoever asked for one that keeps it."""
+    import ctypes
+
+    from qwen25vl_lite_amd.ops.library import load_library
+    plain, held = load_library("sample_gather"), load_library("sample_gather", loader=ctypes.PyDLL)
+    assert not isinstance(plain, ctypes.PyDLL) and isinstance(held, ctypes.PyDLL)
+    assert load_library("sample_gather") is plain and load_library("sample_gather", loader=ctypes.PyDLL) is held
