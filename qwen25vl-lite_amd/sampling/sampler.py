@@ -10,7 +10,7 @@ without a seed draw theirs here, from the global generator.
 from __future__ import annotations
 
 import ctypes
-from collections import deque
+from collections import defaultdict, deque
 from typing import List, Optional, Sequence
 
 import numpy as np
@@ -61,26 +61,28 @@ def _int32_ids(flat: Sequence) -> np.ndarray:
 
 class _Pinned:
     """Pinned host buffers of int32, each with its event and one holder from :meth:`take` to :meth:`give`, on any thread.
-    Of those given back ``KEPT`` a device stay; ``idle`` of them are left alone, so that a copy asked for lately is not waited for."""
+    Of those given back ``KEPT`` a device stay; ``idle`` of them are left alone, so that a copy asked for lately is not waited for
+    (0: buffers are given back when their copy is done)."""
     KEPT = 8
 
     def __init__(self, idle: int, least: int):
-        self._idle, self._least, self._free = idle, least, {}
+        self._idle, self._least, self._free = idle, least, defaultdict(deque)
 
     def take(self, words: int, device: torch.device):
         """A buffer of at least ``words`` that no copy uses any more: ``(host tensor, event)``."""
-        free = self._free.setdefault(device.index or 0, deque())
+        free = self._free[device.index or 0]
         try:
             slot = free.popleft() if len(free) > self._idle else None
         except IndexError:          # (another thread was faster)
             slot = None
         if slot is None or slot[0].numel() < words:
             return torch.empty(max(self._least, 2 * words), dtype=torch.int32, pin_memory=True), torch.cuda.Event()
-        slot[1].synchronize()       # the copy that last used this buffer is done
+        if self._idle:
+            slot[1].synchronize()       # the copy that last used this buffer is done (those given back at once have been waited for)
         return slot
 
     def give(self, slot, device: torch.device) -> None:
-        free = self._free.setdefault(device.index or 0, deque())
+        free = self._free[device.index or 0]
         if len(free) < self.KEPT:
             free.append(slot)
 
@@ -133,9 +135,11 @@ class PendingSample:
     _slot = None
 
     def __init__(self, device_ids: torch.Tensor):
+        m = device_ids.numel()
         self.device_ids = device_ids
-        self._slot = host, event = _down.take(device_ids.numel(), device_ids.device)
-        host[:device_ids.numel()].copy_(device_ids, non_blocking=True)
+        self._slot = host, event = _down.take(m, device_ids.device)
+        self._host = host[:m]
+        self._host.copy_(device_ids, non_blocking=True)
         event.record()
 
     def result(self) -> List[int]:
@@ -143,7 +147,7 @@ class PendingSample:
         if slot is not None:
             slot[1].synchronize()
             # of several threads the first keeps its ids, and gives the buffer back only then
-            self.__dict__.setdefault("_ids", slot[0][:self.device_ids.numel()].tolist())
+            self.__dict__.setdefault("_ids", self._host.tolist())
             if self.__dict__.pop("_slot", None) is not None:
                 _down.give(slot, self.device_ids.device)
         return self._ids

@@ -672,6 +672,28 @@ def test_rows_without_a_seed_draw_from_the_global_generator(monkeypatch):
     assert S.sample_rows(*args) == want and torch.rand(1).item() == after
 
 
+@pytest.mark.parametrize("vocab, first, count", [(152064, 74000, 900), (152064, 148, 3), (5003, 5003 - 700, 700), (1024, 0, 1024), (1000, 300, 1),
+                                                 (40000, 39000, 1000), (40000, 30, 1024), (40000, 0, 1100)])
+def test_sampler_where_what_is_left_lies_close_together(vocab, first, count):
+    """Scores of one chunk or of neighbouring ones, as many as a list holds and more, chunks of one score and of 149: every part of
+    the draw, by the list and by the passes over the whole row."""
+    from qwen25vl_lite_amd.sampling import SamplingParams
+    from qwen25vl_lite_amd.sampling.sampler import sample_rows
+    g = torch.Generator().manual_seed(first + count)
+    row = torch.full((vocab,), -30.0)
+    row[first:first + count] = torch.rand(count, generator=g) * 2
+    us = torch.tensor([0.0, 1e-6, 0.25, 0.5, 0.75, 0.999999])
+    us = torch.cat([us, torch.rand(10, generator=g)]).tolist()
+    n = len(us)
+    probs = torch.softmax(row.double(), 0)
+    cdf = torch.cumsum(probs, 0)
+    for kind in (dict(min_p=1e-3), dict(min_p=1e-3, top_k=2 * vocab), dict(top_k=max(1, count)), {}):
+        got = sample_rows(row.expand(n, -1).contiguous().cuda(), [SamplingParams(temperature=1.0, **kind)] * n, [[]] * n, [0] * n, uniforms=us)
+        for token, u in zip(got, us):      # within rounding of float32 sums of `vocab` masses
+            assert not kind or first <= token < first + count, (kind, token, u)      # (uncut, each of the others has e^-30)
+            assert cdf[token] - probs[token] - 2e-5 <= u <= cdf[token] + 2e-5, (kind, token, u)
+
+
 def test_trace_run_program(model_dirs, tmp_path):
     """bin/trace_run as a user calls it: JSON steps on standard input, `done <step>` lines,
     <step>.f32 files of little-endian float32 [wanted, vocab]."""
