@@ -25,6 +25,7 @@
 // whose list is longer than LIST, or whose list does not reach top-p, go the long way; the others' blocks there end at once.
 // The 64 rows above: 43 us in three kernels, all of it reading and finding, the passes 117 in nine.
 #include "common.h"
+#include <cmath>
 #include <cstddef>
 #include <type_traits>
 
@@ -34,7 +35,7 @@
 #define CHUNKS 1024         // contiguous ranges of a row whose masses the draw adds one after the other
 #define GROUPS 16           // groups of 256 scores of a piece, whose largest are kept
 #define LIST 1024           // scores of a short list
-#define GUESS 384           // how many groups' largest scores top-p is expected to reach at most
+#define GUESS 620           // scores that are expected in a list where top-p alone cuts: some below LIST, since their number is guessed
 #define STEPS 2048          // steps of 1/64 below a row's largest score that bounds are told apart by; the last one is open
 
 struct RowParams {
@@ -325,7 +326,7 @@ __global__ __launch_bounds__(THREADS) void sample_list_kernel(const float* __res
                                                               const RowParams* __restrict__ params,
                                                               RowScratch* __restrict__ scratch,
                                                               const ArgmaxPart* __restrict__ parts,
-                                                              const float* __restrict__ groups, int V, int pieces, float one) {
+                                                              const float* __restrict__ groups, int V, int pieces, int guess, float one) {
   __shared__ unsigned int steps[STEPS], sums[THREADS / 64];
   __shared__ unsigned long long mass[THREADS / 64];
   __shared__ ArgmaxPart s_best;
@@ -365,7 +366,7 @@ __global__ __launch_bounds__(THREADS) void sample_list_kernel(const float* __res
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       if (before < k && before + own[i] >= k) s_k = tid * PER + i;
-      if (before < GUESS && before + own[i] >= GUESS) s_p = tid * PER + i;
+      if (before < (unsigned int)guess && before + own[i] >= (unsigned int)guess) s_p = tid * PER + i;
       before += own[i];
     }
     __syncthreads();
@@ -918,6 +919,14 @@ __global__ __launch_bounds__(THREADS) void sample_pick_kernel(const float* __res
 
 static int pieces_of(int V) { return (V + PIECE - 1) / PIECE; }
 
+// Of the groups of a row's whole pieces, how many have a score above the one with GUESS scores above it, if these lie anywhere: a
+// group has none with probability exp(-GUESS / groups).  (384 of the 592 groups of 151,936 scores; all but one of 32,000's 112.  As many
+// groups at any size left rows of less than 98,304 scores without a guess: eight of 32,000 at top-p 0.9, peaked, 116 us, with it 63.)
+static int guess_of(int V) {
+  const double groups = (double)(V / PIECE) * GROUPS;
+  return V <= LIST || groups < 1 ? 0x7fffffff : (int)lround(groups * (1.0 - exp(-GUESS / groups)));
+}
+
 // Room a row needs: in `parts` always, in `scratch` if any row draws.
 extern "C" long long qvl_sample_parts_bytes(int V) { return (long long)pieces_of(V) * (long long)(sizeof(ArgmaxPart) + GROUPS * sizeof(float)); }
 extern "C" long long qvl_sample_scratch_bytes() { return (long long)sizeof(RowScratch); }
@@ -954,7 +963,7 @@ extern "C" int qvl_sample_rows(const void* logits, void* scores, const void* par
                        groups, todo, M, V, pieces);
     if (scratch) {
       if (cuts || V <= LIST)
-        hipLaunchKernelGGL(sample_list_kernel, dim3(pieces, M), block, 0, stream, lg, sc, rp, rs, ap, groups, V, pieces, one);
+        hipLaunchKernelGGL(sample_list_kernel, dim3(pieces, M), block, 0, stream, lg, sc, rp, rs, ap, groups, V, pieces, guess_of(V), one);
       hipLaunchKernelGGL(sample_short_kernel, dim3(M), block, 0, stream, rp, rs, ap, ids, todo, V, pieces, one);
     } else {
       hipLaunchKernelGGL(sample_pick_kernel, dim3(M), block, 0, stream, lg, sc, rp, rs, ap, ids, todo, V, pieces);

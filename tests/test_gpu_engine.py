@@ -694,6 +694,24 @@ def test_sampler_where_what_is_left_lies_close_together(vocab, first, count):
             assert cdf[token] - probs[token] - 2e-5 <= u <= cdf[token] + 2e-5, (kind, token, u)
 
 
+@pytest.mark.parametrize("vocab", [4097, 8192, 32000, 65000, 98303, 152064])
+def test_peaked_rows_of_any_vocabulary_are_settled_by_their_list(vocab, monkeypatch):
+    """Five tokens with most of the mass, a bell near enough below them that the others could add up to a tenth of it: a list that
+    top-p alone bounds holds the five, whatever the number of groups its bound is guessed from, and nothing is waited for twice."""
+    from qwen25vl_lite_amd.sampling import SamplingParams
+    from qwen25vl_lite_amd.sampling import sampler as S
+    n = 16
+    logits = torch.randn(n, vocab, device="cuda", generator=torch.Generator(device="cuda").manual_seed(vocab))
+    logits[:, 100:105] = 11.0
+    us = [(i + 0.5) / n for i in range(n)]
+    waits, real = [], S.PendingSample
+    monkeypatch.setattr(S, "PendingSample", lambda ids: waits.append(1) or real(ids))
+    for p, kept in ((0.9, 5), (0.5, 5)):          # (equal scores stay together)
+        waits.clear()
+        got = S.sample_rows(logits, [SamplingParams(temperature=0.8, top_p=p)] * n, [[]] * n, [0] * n, uniforms=us)
+        assert got == [100 + int(u * kept) for u in us] and len(waits) == 1
+
+
 def test_trace_run_program(model_dirs, tmp_path):
     """bin/trace_run as a user calls it: JSON steps on standard input, `done <step>` lines,
     <step>.f32 files of little-endian float32 [wanted, vocab]."""
