@@ -6,6 +6,8 @@
 // float32 and bfloat16 storage; scores, weights and sums are float32.  A pair is p = token * top + choice.
 #include "tile_product.h"
 
+#include <cmath>
+
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
@@ -577,11 +579,10 @@ __global__ __launch_bounds__(256) void moe_tile_kernel(ExpertArgs a, int tiles_m
 // rows and the up rows of the same outputs; a wave's gate and up values of an output end in one lane).  K must be a
 // multiple of 32 and offsets within x and within an expert's W 32-bit.  Measured on 12,384 pairs over 32 experts, K
 // 3,584: 2 x 2,368 rows 574 us (tiles of 128 x 256 with all waves in step: 874); down 291.
-// From WIDE_PAIRS pairs an expert on (on average) tiles of 256 pairs: LDS gives each operand to twice the products, for half a tile more
-// of padding an expert.  2 x 2,368 x 3,584 gated and 3,584 x 2,368, 32 experts, of 128 and of 256: 131 pairs 324 and 329 us, 180 and 175,
-// 188 319 and 356, 183 and 189, 262 453 and 446, 246 and 241, 387 574 and 449, 291 and 246, 562 723 and 717, 376 and 369, 768 1,030 and 887,
-// 536 and 444; 2 x 1,376 x 2,048 and 2,048 x 1,376: 188 134 and 174, 80 and 98, 262 187 and 182, 108 and 100, 562 262 and 279, 173 and 146,
-// 768 358 and 342, 232 and 192.
+// Tiles of 256 pairs give each operand in LDS to twice the products, for half a tile more of padding an expert: from WIDE_PAIRS pairs an
+// expert on (on average), where that comes out in fewer or shorter rounds of blocks (qvl_moe_wide_pairs).  Of 128 and of 256, gated | down: 32 experts, 2 x
+// 2,368 x 3,584, 387 pairs 604 and 475 us | 304 and 260, 450 604 and 614 | 302 and 357; 8 experts, 2 x 1,376 x 2,048, 387 pairs 72 and 105 |
+// 35 and 48, 562 104 and 108 | 58 and 51.
 typedef Tile<4, 2, 4, 4> ExpertsTile;
 typedef Tile<2, 4, 8, 4> WideTile;
 #define WIDE_PAIRS 256
@@ -655,6 +656,34 @@ __global__ __launch_bounds__(512) void moe_stream_kernel(ExpertArgs a, int tiles
   }
 }
 
+// How long tiles of bm pairs take, in microseconds: the rounds of the XCD that gets most blocks (they go there in groups of 4 x 8 tiles),
+// each a step of 64 values of K after the other, `alone` where most compute units are idle and `full` where all work, and 2.9 more for its
+// first fetches and its stores.  The pairs' shares are not known on the host: an expert is taken to waste 0.4 of a tile.
+static double stream_us(int P, int E, int bm, int tiles_n, int K, double alone, double full, int cus) {
+  const int there = P / bm + (E < P ? E : P), used = (int)((double)P / bm + 0.4 * E + 0.5), real = used < there ? used : there;
+  const int supers_m = (there + 3) / 4, supers = supers_m * ((tiles_n + 7) / 8);
+  double most = (double)real * tiles_n / 8;
+  if (supers <= 1024) {
+    long long blocks[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int s = 0; s < supers; ++s) {
+      const int m = real - 4 * (s % supers_m), n = tiles_n - 8 * (s / supers_m);
+      blocks[s & 7] += (m < 0 ? 0 : m < 4 ? m : 4) * (n < 8 ? n : 8);
+    }
+    for (long long b : blocks) most = (double)b > most ? (double)b : most;
+  }
+  const double rounds = most * 8 / cus, whole = floor(rounds), rest = rounds - whole;
+  const int steps = (K + 63) / 64;
+  return whole * (steps * full + 2.9) + (rest > 0 ? steps * (alone + (full - alone) * rest) + 2.9 : 0.0);
+}
+// Whether tiles of 256 pairs are the faster ones.  Of 264 products (8, 32 and 64 experts of 768 to 4,096 outputs, 262 to 1,300 pairs each) two are
+// over 2 per cent slower than with tiles of 128 (8 and 12), and 0.8 per cent of the time is lost on average; by the number of pairs alone 66 were
+// (up to 46), and 4.9 per cent was lost.
+extern "C" int qvl_moe_wide_pairs(int P, int E, int R, int K, int gated, int cus) {
+  if (P <= 0 || E <= 0 || R <= 0 || K <= 0 || cus <= 0 || P < WIDE_PAIRS * (long long)E) return 0;
+  const int cols = gated ? ExpertsTile::BN / 2 : ExpertsTile::BN, tiles_n = (R + cols - 1) / cols;
+  return stream_us(P, E, WideTile::BM, tiles_n, K, 0.967, 1.361, cus) < stream_us(P, E, ExpertsTile::BM, tiles_n, K, 0.678, 0.825, cus);
+}
+
 // x_dtype / out_dtype: 0 float32, 1 bfloat16.  float32 operands write float32; bfloat16 operands
 // write either.  The matrix-core kernel runs for bfloat16 with K a multiple of 8 and rows of x on
 // 16-byte boundaries; `big_tiles` asks for the kernels with tiles of 128 or 256 pairs through LDS (many pairs an expert).
@@ -673,7 +702,7 @@ extern "C" int qvl_moe_experts(const void* x, long long ldx, int x_dtype, const 
     const unsigned long long x_rows = (unsigned long long)((P + div - 1) / div);
     if (big_tiles && K % 32 == 0 && x_rows * (unsigned long long)ldx * 2 < 0xffff0000ull &&
         (unsigned long long)(gated ? 2 * R : R) * K * 2 < 0xffff0000ull) {
-      const bool wide = P >= WIDE_PAIRS * (long long)E;
+      const bool wide = qvl_moe_wide_pairs(P, E, R, K, gated, cus);
       const int bm = wide ? WideTile::BM : ExpertsTile::BM;
       const int cols = gated ? ExpertsTile::BN / 2 : ExpertsTile::BN;
       const int tiles_m = P / bm + (E < P ? E : P), tiles_n = (R + cols - 1) / cols;

@@ -902,6 +902,17 @@ def test_experts_with_many_pairs(e, r, k, per):
     assert bool(((got - ref).abs() <= slack + (2.0 ** -8 + 1e-6) * ref.abs() + 2e-6).all())
 
 
+@pytest.mark.parametrize("e, r, k, per", [(3, 1029, 96, 700), (7, 1030, 160, 260), (2, 1033, 32, 1030)])
+def test_experts_in_tiles_of_256_pairs(e, r, k, per):
+    """Sizes at which these are taken for both products: experts whose pairs fill no tile, outputs off steps of four, a last step of
+    half its size."""
+    from qwen25vl_lite_amd.ops import kernels
+    wide = kernels._fn("moe", "qvl_moe_wide_pairs", [kernels._c_int] * 6)
+    pairs = per * e + (per * e) % 2
+    assert wide(pairs, e, 2 * r, k, 0, kernels.compute_units("cuda:0")) and wide(pairs, e, r, k, 1, kernels.compute_units("cuda:0"))
+    test_experts_with_many_pairs(e, r, k, per)
+
+
 @pytest.mark.parametrize("m", [1, 16, 32])
 def test_rows_of_gate_and_up_that_form_no_groups_keep_the_norm_in_the_product(m, monkeypatch):
     """An inner size of the feed-forward off steps of 8: the product forms the norm of a decode step's rows itself, without a
