@@ -123,6 +123,8 @@ __device__ __forceinline__ float4 load4(const bf16_t* p) {
 // softmax of its own (joined at the end, in the waves' order); eight lanes read a key's row side by side, and a lane
 // reads a channel's values of four keys at once.  CH: channels of a value, in sixteens, at most.
 // float32, 16 heads of 128 over 2 of keys: 7 tokens at 25 to 100 keys 51 us with the wave above, 11 with these; 164 tokens of two prompts 57 and 33.
+// Values of more than 128 channels are read 128 at a time: with all of a value's reads in one array the compiler kept it in scratch memory (28 heads of
+// 512, bfloat16, 64 tokens at 1,000 keys 3,697 us, so 937, with the wave above 1,973; of 256, 64 tokens at 64 keys 224, 88 and 67).
 #define ATTN_WAVES 4
 template <typename T, int CH>
 __global__ __launch_bounds__(64 * ATTN_WAVES) void attn_generic_vec_kernel(
@@ -201,19 +203,24 @@ __global__ __launch_bounds__(64 * ATTN_WAVES) void attn_generic_vec_kernel(
       // values of keys that are not seen may be anything
       auto seen = [&](int j) { return (j >= lo || j < kept) && j <= p; };
       const bool s0 = seen(j0), s1 = seen(j0 + 1), s2 = seen(j0 + 2), s3 = seen(j0 + 3);
-      float4 x[CH];
+      // (eight at a time: more in flight cost the registers that other waves would have)
 #pragma unroll
-      for (int i = 0; i < CH; ++i) {
-        const int d = 16 * i + chan;
-        if (16 * i < vd) x[i] = load4(v + (size_t)(d < vd ? d : 0) * ps);
-      }
+      for (int c = 0; c < CH; c += 8) {
+        if (c && 16 * c >= vd) break;
+        float4 x[8];
 #pragma unroll
-      for (int i = 0; i < CH; ++i) {
-        if (16 * i >= vd) break;
-        acc[i] += s0 ? w.x * x[i].x : 0.f;
-        acc[i] += s1 ? w.y * x[i].y : 0.f;
-        acc[i] += s2 ? w.z * x[i].z : 0.f;
-        acc[i] += s3 ? w.w * x[i].w : 0.f;
+        for (int i = 0; i < 8; ++i) {
+          const int d = 16 * (c + i) + chan;
+          if (16 * (c + i) < vd) x[i] = load4(v + (size_t)(d < vd ? d : 0) * ps);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          if (16 * (c + i) >= vd) break;
+          acc[c + i] += s0 ? w.x * x[i].x : 0.f;
+          acc[c + i] += s1 ? w.y * x[i].y : 0.f;
+          acc[c + i] += s2 ? w.z * x[i].z : 0.f;
+          acc[c + i] += s3 ? w.w * x[i].w : 0.f;
+        }
       }
     }
     __builtin_amdgcn_wave_barrier();
@@ -282,8 +289,10 @@ extern "C" int qvl_attn_generic(const void* q, const void* kc, const void* vc, c
                      (const float2*)turn, turn_pairs)
   if (vec && (dtype == 0 || dtype == 1)) {
     if (dtype == 0 && vd <= 128) VEC(float, 8);
+    else if (dtype == 0 && vd <= 256) VEC(float, 16);
     else if (dtype == 0) VEC(float, ATTN_MAX_HD / 16);
     else if (vd <= 128) VEC(bf16_t, 8);
+    else if (vd <= 256) VEC(bf16_t, 16);
     else VEC(bf16_t, ATTN_MAX_HD / 16);
     return qvl_launch_status();
   }

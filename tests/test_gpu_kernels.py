@@ -297,6 +297,13 @@ def test_generic_attention_of_long_contexts(dtype, nq, nkv, hd, vd, ps, window, 
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("hd, vd", [(256, 256), (64, 129), (64, 257), (8, 511)])
+def test_generic_attention_of_wide_values(dtype, hd, vd):
+    """Values of more channels than are read at a time, the last ones alone."""
+    test_generic_attention_of_long_contexts(dtype, 2, 1, hd, vd, 8, 150, 5, None)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("hd", [64, 62])
 @pytest.mark.parametrize("low", [(64, 128), (0, 64), (0, 256), (130, 301)])
 def test_generic_attention_beside_scores_of_minus_infinity(dtype, hd, low):
