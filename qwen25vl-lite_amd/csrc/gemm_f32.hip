@@ -28,6 +28,7 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 #define TK 16
 #define MOST_RANGES 8
 #define RUN 32
+static_assert(RUN == 2 * TK, "the plain kernel joins a run's sums every second step");
 
 // Values of K in a range: an eighth, in steps of 64, 256 at least.
 __host__ __device__ __forceinline__ int range_of(int K) {
@@ -59,20 +60,34 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
         from[i][j] = 0.f;
       }
   };
-
-  for (int k0 = 0; k0 < K; k0 += TK) {
-    if (k0 && k0 % RUN == 0) join(acc, run);
-    if (k0 && k0 % range == 0) join(total, acc);
-    // 64 rows x 16 k per operand: 1024 elements, 4 per thread
+  // 64 rows x 16 k per operand: 1024 elements, 4 per thread, asked for while the 16 values of k before are multiplied
+  const int kk = threadIdx.x % TK, r0 = threadIdx.x / TK;
+  const float* pa[4];
+  const float* pw[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {       // (rows that do not exist are read from the last one that does; their sums are not stored)
+    pa[e] = A + (size_t)min(m0 + r0 + 16 * e, M - 1) * lda;
+    pw[e] = W + (size_t)min(n0 + r0 + 16 * e, N - 1) * ldw;
+  }
+  float va[4], vw[4];
+  auto load = [&](int k0) {
+    const int gk = min(k0 + kk, K - 1);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const int idx = threadIdx.x + 256 * e;
-      const int rr = idx / TK, kk = idx % TK;
-      const int gm = m0 + rr, gn = n0 + rr, gk = k0 + kk;
-      sa[kk][rr] = (gm < M && gk < K) ? A[(size_t)gm * lda + gk] : 0.f;
-      sw[kk][rr] = (gn < N && gk < K) ? W[(size_t)gn * ldw + gk] : 0.f;
+      va[e] = pa[e][gk];
+      vw[e] = pw[e][gk];
+    }
+  };
+  load(0);
+  int next = range;
+  for (int k0 = 0; k0 < K; k0 += TK) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      sa[kk][r0 + 16 * e] = k0 + kk < K ? va[e] : 0.f;
+      sw[kk][r0 + 16 * e] = k0 + kk < K ? vw[e] : 0.f;
     }
     __syncthreads();
+    load(k0 + TK);
 #pragma unroll
     for (int step = 0; step < TK; ++step) {
       const int kk = 4 * (step & 3) + (step >> 2);
@@ -87,6 +102,11 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
         for (int j = 0; j < 4; ++j) run[i][j] = fmaf(a[i], b[j], run[i][j]);
     }
     __syncthreads();
+    if (k0 % RUN != 0) join(acc, run);          // (a run is two steps)
+    if (k0 + TK == next) {
+      join(total, acc);
+      next += range;
+    }
   }
   join(acc, run);
 #pragma unroll

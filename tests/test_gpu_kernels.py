@@ -561,6 +561,25 @@ def test_gemm_f32_ranges_of_k(m, n, k):
     assert torch.equal(kernels.gemm_f32(wide[:, :k], w, b), got)
 
 
+@pytest.mark.parametrize("n, k", [(40005, 64), (33001, 700), (5000, 1000), (4099, 256), (70, 64), (1030, 516), (300, 2052)])
+@pytest.mark.parametrize("m", [1, 16, 17, 33, 64, 100, 300])
+def test_gemm_f32_of_few_ranges(m, n, k):
+    """One to four ranges, so that the waves of a block of few rows have several tiles of outputs; small tiles and large ones, cut
+    and uncut, the last ones not full: against 64 bits, with the plain kernel's bits."""
+    from qwen25vl_lite_amd.ops import kernels
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x, w = torch.randn(m, k, device="cuda", generator=g), torch.randn(n, k, device="cuda", generator=g)
+    b = torch.randn(n, device="cuda", generator=g)
+    got = kernels.gemm_f32(x, w, b)
+    want = x.double() @ w.double().t() + b.double()
+    assert ((got - want).norm() / want.norm()).item() < 2 ** -23 * (91 / 2) ** 0.5       # as for more ranges
+    wide = torch.full((m, k + 1), math.nan, device="cuda")
+    wide[:, :k] = x
+    assert torch.equal(kernels.gemm_f32(wide[:, :k], w, b), got)
+    out = torch.full((m, n + 3), 7.0, device="cuda")
+    assert torch.equal(kernels.gemm_f32(x, w, b, out=out[:, 1:n + 1]), got) and bool((out[:, 0] == 7).all()) and bool((out[:, n + 1:] == 7).all())
+
+
 @pytest.mark.parametrize("m, n, k", [(1, 509, 144), (8, 300, 200), (16, 17, 8), (9, 100, 8200), (17, 1000, 4104),
                                      (31, 130, 352), (64, 509, 3584), (5, 40, 100), (300, 64, 1000),
                                      (17, 4700, 3584), (32, 300, 3840), (24, 509, 3848), (20, 33, 8),
