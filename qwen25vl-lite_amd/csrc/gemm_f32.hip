@@ -159,14 +159,15 @@ template <int WF, int XF>
 __global__ __launch_bounds__(64 * MOST_RANGES) void gemm_f32_stream_kernel(const float* __restrict__ A, int lda,
                                                                            const float* __restrict__ W, int ldw,
                                                                            const float* __restrict__ bias, float* __restrict__ C,
-                                                                           int ldc, int M, int N, int K, int tiles) {
+                                                                           int ldc, int M, int N, int K, int tiles, int groups) {
   constexpr int STEP = 32, ROWS_W = 8 * WF, FETCHES = WF + XF, STAGE = FETCHES * 1024, SUMS = MOST_RANGES * 1024;   // SUMS: bytes of a tile's
   constexpr int STAGES = (163840 - 2 * SUMS) / MOST_RANGES / STAGE;
   __shared__ __attribute__((aligned(16))) char lds[MOST_RANGES * STAGES * STAGE + 2 * SUMS];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
-  const int range = range_of(K), ranges = (K + range - 1) / range;
-  const int k_first = wave * range, ksteps = wave < ranges ? (min(K - k_first, range) + STEP - 1) / STEP : 0;
-  const int my_tiles = (tiles - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x, steps = ksteps * my_tiles;
+  const int range = range_of(K), ranges = (K + range - 1) / range, group = wave / ranges;
+  const int k_first = (wave - group * ranges) * range, ksteps = group < groups ? (min(K - k_first, range) + STEP - 1) / STEP : 0;
+  const int turns = (tiles + groups - 1) / groups;
+  const int my_tiles = (turns - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x, steps = ksteps * my_tiles;
   char* sums = lds + MOST_RANGES * STAGES * STAGE;
   const char* mine = lds + wave * STAGES * STAGE;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds + wave * STAGES * STAGE;
@@ -177,11 +178,12 @@ __global__ __launch_bounds__(64 * MOST_RANGES) void gemm_f32_stream_kernel(const
   uint32_t fa[XF], fw[WF];
 #pragma unroll
   for (int j = 0; j < XF; ++j) fa[j] = (uint32_t)min(8 * j + row8, M - 1) * (uint32_t)lda * 4;
-  int asked = 0, ask_k = 0, ask_tile = blockIdx.x, ask_stage = 0;
+  int asked = 0, ask_k = 0, ask_turn = blockIdx.x, ask_stage = 0;
   const float* wbase = W;
   auto ask = [&]() __attribute__((always_inline)) {
     if (asked >= steps) return;
     if (ask_k == 0) {
+      const int ask_tile = min(ask_turn * groups + group, tiles - 1);
       wbase = W + (size_t)ask_tile * ROWS_W * ldw;
 #pragma unroll
       for (int j = 0; j < WF; ++j) {
@@ -203,7 +205,7 @@ __global__ __launch_bounds__(64 * MOST_RANGES) void gemm_f32_stream_kernel(const
     ask_stage = ask_stage + 1 == STAGES ? 0 : ask_stage + 1;
     if (++ask_k == ksteps) {
       ask_k = 0;
-      ask_tile += gridDim.x;
+      ask_turn += gridDim.x;
     }
   };
 #pragma unroll
@@ -242,7 +244,7 @@ __global__ __launch_bounds__(64 * MOST_RANGES) void gemm_f32_stream_kernel(const
       stage = stage + 1 == STAGES ? 0 : stage + 1;
     }
     char* here = sums + (i & 1) * SUMS;
-    if (wave < ranges) {
+    if (group < groups) {
       *reinterpret_cast<f32x4_t*>(here + wave * 1024 + lane * 16) = acc;
       acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
@@ -251,9 +253,11 @@ __global__ __launch_bounds__(64 * MOST_RANGES) void gemm_f32_stream_kernel(const
     __builtin_amdgcn_s_barrier();               // (fetches stay in flight.)  The sums of the tile before the last have been read, too
     __builtin_amdgcn_sched_barrier(0);
     // output n of row m: lane 16 (n / 4) + m holds it as its number n mod 4
-    const int m = threadIdx.x >> 4, n = threadIdx.x & 15, gn = ((int)blockIdx.x + i * (int)gridDim.x) * ROWS_W + n;
-    if (m < M && n < ROWS_W && gn < N) {
-      const float* q = reinterpret_cast<const float*>(here) + ((n >> 2) * 16 + m) * 4 + (n & 3);
+    const int m = threadIdx.x >> 4 & 15, n = threadIdx.x & 15;
+    for (int at = threadIdx.x >> 8; at < groups; at += 2) {
+      const int gn = (((int)blockIdx.x + i * (int)gridDim.x) * groups + at) * ROWS_W + n;
+      if (m >= M || n >= ROWS_W || gn >= N) continue;
+      const float* q = reinterpret_cast<const float*>(here) + (at * ranges * 64 + (n >> 2) * 16 + m) * 4 + (n & 3);
       float total = 0.f;
       for (int w = 0; w < ranges; ++w) total += q[w * 256];
       C[(size_t)m * ldc + gn] = total + (bias ? bias[gn] : 0.f);
@@ -478,8 +482,18 @@ extern "C" int qvl_gemm_f32(const void* A, int lda, const void* W, int ldw, cons
     if (M <= F32_STREAM_ROWS) {
       const bool narrow = N <= 8 * cus;
       const int tiles = narrow ? (N + 7) / 8 : (N + 15) / 16;
-      const dim3 grid(tiles < cus ? tiles : cus), block(64 * MOST_RANGES);
-#define GO(WF, XF) hipLaunchKernelGGL((gemm_f32_stream_kernel<WF, XF>), grid, block, 0, stream, a, lda, w, ldw, b, (float*)C, ldc, M, N, K, tiles)
+      // Tiles beside each other in a block where there are fewer ranges than waves: as many as make the longest block short, whose unit five
+      // waves keep busy (40,000 outputs, 4 rows, K = 256: 32 us with one wave, 14 with five; K = 64 12.8 and 8).
+      const int range = range_of(K), ranges = (K + range - 1) / range;
+      int groups = 1;
+      double least = 1e300;
+      for (int n = 1; n * ranges <= MOST_RANGES; ++n) {
+        const double cost = (double)(((tiles + n - 1) / n + cus - 1) / cus) * n / (n * ranges < 5 ? n * ranges / 5.0 : 1.0);
+        if (cost < least) least = cost, groups = n;
+      }
+      const int turns = (tiles + groups - 1) / groups;
+      const dim3 grid(turns < cus ? turns : cus), block(64 * MOST_RANGES);
+#define GO(WF, XF) hipLaunchKernelGGL((gemm_f32_stream_kernel<WF, XF>), grid, block, 0, stream, a, lda, w, ldw, b, (float*)C, ldc, M, N, K, tiles, groups)
       if (narrow && M <= 8) GO(1, 1);
       else if (narrow) GO(1, 2);
       else if (M <= 8) GO(2, 1);
