@@ -268,8 +268,8 @@ __global__ __launch_bounds__(64 * MOST_RANGES) void gemm_f32_stream_kernel(const
 
 // More rows: WN x WM waves, each with TNW x TMW tiles of 16 outputs (rows of W) by 16 rows of A; K in steps of 32 values
 // through STAGES stages of LDS, the matrix cores the bound.  Registers and LDS leave room for four blocks a compute unit, which
-// hide each other's barriers (1,500 x 2,048 x 11,008: 595 us; tiles of 128 x 128, a block a unit, 757).  A block has `per` of K's ranges.  slabs: the sums of
-// range i go to slab i, so many floats apart; otherwise (one block has all ranges) their sum goes to C.
+// hide each other's barriers (1,500 x 2,048 x 11,008: 595 us; tiles of 128 x 128, a block a unit, 757).  A block has all of K's ranges or one (`per`).  slabs: the
+// sums of range i go to slab i, so many floats apart; otherwise their sum goes to C.
 // ONCE: no other block reads these rows of W.
 template <int WN, int WM, int TNW, int TMW, int STAGES, bool ONCE>
 __global__ __launch_bounds__(64 * WN * WM, 4) void gemm_f32_tile_kernel(const float* __restrict__ A, int lda,
@@ -284,10 +284,10 @@ __global__ __launch_bounds__(64 * WN * WM, 4) void gemm_f32_tile_kernel(const fl
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
   const int wn = wave % WN, wm = wave / WN;
-  const int n0 = blockIdx.x * ROWS_W, m0 = blockIdx.y * ROWS_A;
+  const int tiles_n = (N + ROWS_W - 1) / ROWS_W, n0 = blockIdx.x % tiles_n * ROWS_W, m0 = blockIdx.x / tiles_n * ROWS_A;
   const float* wbase = W + (size_t)n0 * ldw;
   const float* abase = A + (size_t)m0 * lda;
-  const int range = range_of(K), k_first = blockIdx.z * per * range, k_end = min(K, k_first + per * range);
+  const int range = range_of(K), k_first = blockIdx.y * per * range, k_end = min(K, k_first + per * range);
 
   // this wave's fetches of a step: 8 rows each, W's first.  Place s of row rho holds chunk s ^ ((rho / 2) mod 8).  Rows and
   // chunks that do not exist are read from ones that do.
@@ -358,7 +358,7 @@ __global__ __launch_bounds__(64 * WN * WM, 4) void gemm_f32_tile_kernel(const fl
   // together, so that reading and multiplying would else take turns.
   const uint32_t sw = (r >> 1) & 7;
   f32x4_t w4[2][TNW], x4[2][TMW], run[TNW][TMW];
-  int stage = 0, left = min(range, k_end - k_first), slab = blockIdx.z * per;
+  int stage = 0, left = min(range, k_end - k_first), slab = blockIdx.y * per;
   auto read = [&](auto half) __attribute__((always_inline)) {
     constexpr int H = decltype(half)::value;
     const char* p = lds + stage * STAGE + r * 128 + (((4 * H + g) ^ sw) << 4);
@@ -431,18 +431,20 @@ __global__ __launch_bounds__(64 * WN * WM, 4) void gemm_f32_tile_kernel(const fl
 
 // The ranges' sums, added from the first to the last.
 __global__ __launch_bounds__(256) void gemm_f32_add_kernel(const float* __restrict__ sums, int ranges, long long slab,
-                                                           const float* __restrict__ bias, float* __restrict__ C, int ldc, int N) {
-  const int n = blockIdx.x * 256 + threadIdx.x, m = blockIdx.y;
+                                                           const float* __restrict__ bias, float* __restrict__ C, int ldc, int M, int N) {
+  const int n = blockIdx.x * 256 + threadIdx.x;
   if (n >= N) return;
-  const float* p = sums + (size_t)m * N + n;
-  float v[MOST_RANGES];
+  for (int m = blockIdx.y; m < M; m += gridDim.y) {
+    const float* p = sums + (size_t)m * N + n;
+    float v[MOST_RANGES];
 #pragma unroll
-  for (int i = 0; i < MOST_RANGES; ++i) v[i] = i < ranges ? p[i * slab] : 0.f;
-  float total = 0.f;
+    for (int i = 0; i < MOST_RANGES; ++i) v[i] = i < ranges ? p[i * slab] : 0.f;
+    float total = 0.f;
 #pragma unroll
-  for (int i = 0; i < MOST_RANGES; ++i)
-    if (i < ranges) total += v[i];
-  C[(size_t)m * ldc + n] = total + (bias ? bias[n] : 0.f);
+    for (int i = 0; i < MOST_RANGES; ++i)
+      if (i < ranges) total += v[i];
+    C[(size_t)m * ldc + n] = total + (bias ? bias[n] : 0.f);
+  }
 }
 
 // How a product of more than 16 rows is cut.  Tiles of 64 outputs by 64 rows (`rows`), by 32 where that is all rows.  Where there
@@ -458,7 +460,7 @@ static F32Plan f32_plan(int M, int N, int K, int cus) {
   const bool cut = 4 * (long long)((N + 63) / 64) * ((M + rows - 1) / rows) < 7LL * cus;
   return cut ? F32Plan{rows, 1, ranges} : F32Plan{rows, ranges, 1};
 }
-static bool f32_tiles(int lda, int ldw, int K) {      // 128 rows of W or A from a block's first one lie within 32 bits of bytes
+static bool f32_tiles(int lda, int ldw, int K) {      // 64 rows of W or A from a block's first one lie within 32 bits of bytes
   return K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && lda < (1 << 22) && ldw < (1 << 22);
 }
 
@@ -505,17 +507,18 @@ extern "C" int qvl_gemm_f32(const void* A, int lda, const void* W, int ldw, cons
     if (p.parts > 1 && !scratch) return QVL_ERR_SHAPE;
     float* to = p.parts > 1 ? (float*)scratch : (float*)C;
     const long long slab = p.parts > 1 ? (long long)M * N : 0;
-    const dim3 grid((N + 63) / 64, (M + p.rows - 1) / p.rows, p.parts);
-    if (grid.y > 65535 || (p.parts > 1 && M > 65535)) return QVL_ERR_LIMIT;
+    const long long tiles_n = (N + 63) / 64, tiles_m = (M + p.rows - 1) / p.rows;
+    if (tiles_n * tiles_m > 0xffffffffll / 256) return QVL_ERR_LIMIT;      // threads of a grid
+    const dim3 grid((unsigned)(tiles_n * tiles_m), p.parts);
 #define GO(...) hipLaunchKernelGGL((gemm_f32_tile_kernel<__VA_ARGS__>), grid, dim3(256), 0, stream, a, lda, w, ldw, b, to, ldc, M, N, K, p.per, slab)
-    if (p.rows == 64 && grid.y == 1) GO(2, 2, 2, 2, 2, true);
+    if (p.rows == 64 && tiles_m == 1) GO(2, 2, 2, 2, 2, true);
     else if (p.rows == 64) GO(2, 2, 2, 2, 2, false);
     else GO(4, 1, 1, 2, 3, true);
 #undef GO
     if (p.parts > 1) {
       const int range = range_of(K);
-      hipLaunchKernelGGL(gemm_f32_add_kernel, dim3((N + 255) / 256, M), dim3(256), 0, stream, (const float*)scratch, (K + range - 1) / range,
-                         slab, b, (float*)C, ldc, N);
+      hipLaunchKernelGGL(gemm_f32_add_kernel, dim3((N + 255) / 256, M < 65535 ? M : 65535), dim3(256), 0, stream, (const float*)scratch, (K + range - 1) / range,
+                         slab, b, (float*)C, ldc, M, N);
     }
     return qvl_launch_status();
   }

@@ -580,6 +580,15 @@ def test_gemm_f32_of_few_ranges(m, n, k):
     assert torch.equal(kernels.gemm_f32(x, w, b, out=out[:, 1:n + 1]), got) and bool((out[:, 0] == 7).all()) and bool((out[:, n + 1:] == 7).all())
 
 
+def test_gemm_f32_of_more_rows_than_a_grid_has_places_for_tiles_of_64():
+    from qwen25vl_lite_amd.ops import kernels
+    m, n, k = 65535 * 64 + 65, 3, 32
+    x, w = torch.randn(m, k, device="cuda"), torch.randn(n, k, device="cuda")
+    got = kernels.gemm_f32(x, w)
+    for at in (0, 65535 * 32, 65535 * 64 - 40, m - 100):
+        assert torch.equal(got[at:at + 100], kernels.gemm_f32(x[at:at + 100], w))
+
+
 @pytest.mark.parametrize("m, n, k", [(1, 509, 144), (8, 300, 200), (16, 17, 8), (9, 100, 8200), (17, 1000, 4104),
                                      (31, 130, 352), (64, 509, 3584), (5, 40, 100), (300, 64, 1000),
                                      (17, 4700, 3584), (32, 300, 3840), (24, 509, 3848), (20, 33, 8),
