@@ -19,6 +19,7 @@
 // 2,048 230 and 190, 700 x 22,016 x 2,048 874 and 550 (115 TFLOP/s).
 #include "common.h"
 
+#include <cmath>
 #include <type_traits>
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -447,18 +448,37 @@ __global__ __launch_bounds__(256) void gemm_f32_add_kernel(const float* __restri
   }
 }
 
-// How a product of more than 16 rows is cut.  Tiles of 64 outputs by 64 rows (`rows`), by 32 where that is all rows.  Where there
-// are fewer tiles than 7 for 4 compute units each of K's ranges has blocks of its own; their sums are then added by a kernel
-// behind (5 us and the slabs' traffic).  Measured, cut and uncut: 164 x 2,048 x 11,008 (96 tiles) 91 us and 275, 512 x 2,560 x 2,048
-// (320) 63 and 83, 700 x 2,048 x 11,008 (352) 285 and 433, 700 x 2,560 x 2,048 (440) 84 and 84, 100 x 22,016 x 2,048 (688) 127 and 119,
-// 1,500 x 2,048 x 2,048 (768) 137 and 116.  Two or four ranges a block were never the best by more than 2 per cent.
+// How a product of more than 16 rows is cut: tiles of 64 outputs by 64 rows (by 32 where that is all rows) or of 32 by 32, and a block for all of
+// K or one for each range, whose sums a kernel behind then adds.  The estimate is of microseconds: a step of 32 values takes a block `alone`
+// where a compute unit has no other and each one `full` where they share its matrix cores; 0.92 more for the first fetches and the stores of each
+// round of four blocks a unit; W read and the results written at 8.8 TB/s, which joins that as the root of squares; the adding kernel 1.8 and the slabs
+// read at 6.5 TB/s (a cut has to be 4 per cent shorter).  Fitted to 1,326 products of 17 to 1,500 rows, 64 to 80,000 outputs and K of 64 to 11,008, each in all four forms (rms 7 per
+// cent): what it chooses takes 0.4 per cent longer than the best on average.  Large tiles alone, cut by their number: 12, most where K or the
+// outputs are few (64 x 256 x 256 11 us and 8, 164 x 64 x 11,008 42 and 25).
 struct F32Plan {
-  int rows, per, parts;      // per: ranges of a block
+  int rows_w, rows, per, parts;      // of W and of A in a tile; per: ranges of a block
 };
 static F32Plan f32_plan(int M, int N, int K, int cus) {
-  const int range = range_of(K), ranges = (K + range - 1) / range, rows = M <= 32 ? 32 : 64;
-  const bool cut = 4 * (long long)((N + 63) / 64) * ((M + rows - 1) / rows) < 7LL * cus;
-  return cut ? F32Plan{rows, 1, ranges} : F32Plan{rows, ranges, 1};
+  const int range = range_of(K), ranges = (K + range - 1) / range;
+  F32Plan best{};
+  double least = 1e300;
+  for (int form = 0; form < (ranges > 1 ? 4 : 2); ++form) {
+    const bool small = form & 1, cut = form & 2;
+    const int rows_w = small ? 32 : 64, rows = small || M <= 32 ? 32 : 64;
+    const double full = small ? 0.222 : rows == 32 ? 0.402 : 0.616, alone = small ? 0.406 : rows == 32 ? 0.584 : 0.772;
+    const long long tiles = (long long)((N + rows_w - 1) / rows_w) * ((M + rows - 1) / rows);
+    const int steps = ((cut ? range : K) + 31) / 32;
+    const double blocks = (double)tiles * (cut ? ranges : 1) / cus, sharing = blocks < 8 ? ceil(blocks) : blocks;
+    const double results = 4.0 * M * N * (cut ? ranges : 1), memory = (4.0 * N * K + results) / 8.8e6;
+    double us = steps * (alone > full * sharing ? alone : full * sharing) + 0.92 * ceil(blocks / 4);
+    us = sqrt(us * us + memory * memory);
+    if (cut) us = 1.04 * (us + 1.8 + results / 6.45e6);
+    if (us < least) {
+      least = us;
+      best = F32Plan{rows_w, rows, cut ? 1 : ranges, cut ? ranges : 1};
+    }
+  }
+  return best;
 }
 static bool f32_tiles(int lda, int ldw, int K) {      // 64 rows of W or A from a block's first one lie within 32 bits of bytes
   return K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && lda < (1 << 22) && ldw < (1 << 22);
@@ -507,11 +527,12 @@ extern "C" int qvl_gemm_f32(const void* A, int lda, const void* W, int ldw, cons
     if (p.parts > 1 && !scratch) return QVL_ERR_SHAPE;
     float* to = p.parts > 1 ? (float*)scratch : (float*)C;
     const long long slab = p.parts > 1 ? (long long)M * N : 0;
-    const long long tiles_n = (N + 63) / 64, tiles_m = (M + p.rows - 1) / p.rows;
+    const long long tiles_n = (N + p.rows_w - 1) / p.rows_w, tiles_m = (M + p.rows - 1) / p.rows;
     if (tiles_n * tiles_m > 0xffffffffll / 256) return QVL_ERR_LIMIT;      // threads of a grid
     const dim3 grid((unsigned)(tiles_n * tiles_m), p.parts);
 #define GO(...) hipLaunchKernelGGL((gemm_f32_tile_kernel<__VA_ARGS__>), grid, dim3(256), 0, stream, a, lda, w, ldw, b, to, ldc, M, N, K, p.per, slab)
-    if (p.rows == 64 && tiles_m == 1) GO(2, 2, 2, 2, 2, true);
+    if (p.rows_w == 32) GO(2, 2, 1, 1, 4, false);
+    else if (p.rows == 64 && tiles_m == 1) GO(2, 2, 2, 2, 2, true);
     else if (p.rows == 64) GO(2, 2, 2, 2, 2, false);
     else GO(4, 1, 1, 2, 3, true);
 #undef GO
