@@ -19,19 +19,21 @@ from .base import (CacheNeed, LayerSlot, Mixer, ParamSpec, PartSpec, StateNeed, 
                    register_part)
 
 # 17 to 64 rows: where the fused kernel does not run, the projection is cut along its inner size (slabs) and the rotation's
-# kernel adds them (10,240 x 8,192, 19 rows: 32 us, the library's product uncut 41): up to 48 rows at any inner size, up to 64 where it is
-# beyond LONG_K, which the fused kernel does not take with as many rows (8 decode steps at 768 keys, 72B sizes, 2 layers: 64 rows 9,962 us
-# against 10,157 with the library's product, 56 9,818 and 10,041).  From 33 to 48 rows that also beats the fused kernel on teams of blocks (7B
+# kernel adds them (10,240 x 8,192, 19 rows: 32 us, the library's product uncut 41): up to 48 rows at any size, up to 64 where the inner size is
+# beyond LONG_K, which the fused kernel does not take with as many rows, and the weight has LARGE_WEIGHT values or more (49 rows, with the
+# library's product and in slabs: 512 x 4,608 12 us and 17, 7,168 x 5,120 23 and 27, 5,120 x 8,192 31 and 27, 10,240 x 6,144 46 and 36, 10,240 x 8,192
+# 49 and 40, 14,336 x 12,288 88 and 74, 18,432 x 16,384 176 and 164).  From 33 to 48 rows that also beats the fused kernel on teams of blocks (7B
 # sizes: a step of 33 rows 4.14 ms against 4.24, of 48 rows 4.34 against 4.39); from 49 on it does not (7B sizes, K = 3,584, 8 layers, 64 rows
 # 11,160 and 11,124; 3B sizes, K = 2,048, 6 steps at 256 keys 4,922 and 4,820).
 SPLIT_ROWS = (17, 64)
 SHORT_SPLIT_ROWS = 48
 LONG_K = 4096
+LARGE_WEIGHT = 40 << 20
 FUSED_ROWS = 32
 
 
-def _splits(m: int, k: int) -> bool:
-    return SPLIT_ROWS[0] <= m <= (SPLIT_ROWS[1] if k > LONG_K else SHORT_SPLIT_ROWS)
+def _splits(m: int, n: int, k: int) -> bool:
+    return SPLIT_ROWS[0] <= m <= (SPLIT_ROWS[1] if k > LONG_K and n * k >= LARGE_WEIGHT else SHORT_SPLIT_ROWS)
 
 
 __all__ = ["PagedAttention"]
@@ -318,7 +320,7 @@ class PagedAttention(Mixer):
         # Projections are written out in float32 (the accumulator, unrounded): bias, rotation and
         # the residual sum then happen in float32 and each stored value is rounded once.
         m, k = x.shape
-        if (_splits(m, k) and self.dtype == torch.bfloat16 and isinstance(x, torch.Tensor)
+        if (_splits(m, self.w_in.shape[0], k) and self.dtype == torch.bfloat16 and isinstance(x, torch.Tensor)
                 and x.dtype == torch.bfloat16 and self.hd % 4 == 0 and inv_freq.shape[0] % 4 == 0
                 and skinny.takes_split(m, k, self.w_in) and x.stride(1) == 1 and x.stride(0) % 8 == 0
                 and x.data_ptr() % 16 == 0):
@@ -352,7 +354,7 @@ class PagedAttention(Mixer):
         kernel (the float32 sums never leave it)."""
         lazy = isinstance(x, NormedRows)
         m, k = x.shape
-        if not lazy and m > FUSED_ROWS and _splits(m, k):
+        if not lazy and m > FUSED_ROWS and _splits(m, self.w_in.shape[0], k):
             return None
         if self.dtype != torch.bfloat16 or not skinny.takes_qkv_rope(
                 m, k, self.w_in, self.hd, inv_freq.shape[0], slot.k_cache.dtype if write else None, norm=lazy):

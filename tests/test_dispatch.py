@@ -103,11 +103,17 @@ def test_a_steps_lists_are_not_made_inside_a_graph(monkeypatch):
 
 
 def test_which_rows_of_the_stacked_projection_are_cut():
-    """17 to 48 rows at any inner size, up to 64 beyond the one that the kernel with the rotation inside keeps in one pass."""
+    """17 to 48 rows at any size, up to 64 of large weights beyond the inner size that the kernel with the rotation inside keeps in one
+    pass."""
     from qwen25vl_lite_amd.ops import skinny
     from qwen25vl_lite_amd.parts import attention
-    cut = {k: [m for m in range(1, 70) if attention._splits(m, k)] for k in (2048, 4096, 4104, 8192)}
-    assert cut[2048] == cut[4096] == list(range(17, 49)) and cut[4104] == cut[8192] == list(range(17, 65))
+
+    def cut(n, k):
+        return [m for m in range(1, 70) if attention._splits(m, n, k)]
+    for n, k in ((2560, 2048), (4608, 3584), (40960, 4096), (512, 4608), (7168, 5120), (1280, 8192), (5119, 8192)):
+        assert cut(n, k) == list(range(17, 49)), (n, k)
+    for n, k in ((10240, 4104), (5120, 8192), (10240, 6144), (10240, 8192), (18432, 16384)):
+        assert cut(n, k) == list(range(17, 65)), (n, k)
     for k in (4104, 8192):        # what ran there before is the library's product, not the fused kernel
         assert not any(skinny.takes_resident(m, k, torch.empty((10240, k), dtype=torch.bfloat16, device="meta")) for m in range(33, 65))
 

@@ -139,6 +139,13 @@ def test_projection_with_rotation_and_cache(k):
             assert bool((kc.transpose(1, 2)[untouched] == 0).all()) and bool((vc.permute(0, 3, 1, 2)[untouched] == 0).all())
 
 
+def test_projection_in_slabs_up_to_64_rows(monkeypatch):
+    """As a large weight's, whose 49 to 64 rows are cut, too."""
+    from qwen25vl_lite_amd.parts import attention
+    monkeypatch.setattr(attention, "LARGE_WEIGHT", 0)
+    test_projection_with_rotation_and_cache(4104)
+
+
 @pytest.mark.parametrize("n, k, most", [(2048, 11008, 16), (2048, 16384, 16), (2048, 16392, 8), (3584, 18944, 8)])
 def test_few_rows_cut_along_k(n, k, most):
     """Up to 8 rows, or 16 with a small weight, few ranges whose rows stay in their blocks; beyond, the streaming kernel's: as many
