@@ -1148,6 +1148,26 @@ def test_tiled_product_in_shapes_that_do_not_halve(shape, bn, bm, rows, outputs,
     assert bool(((got - ref).abs() <= slack + (2.0 ** -8 + 1e-6) * ref.abs() + 2e-6).all())
 
 
+@pytest.mark.parametrize("shape, bn, bm", [(0, 256, 256), (1, 128, 256), (2, 256, 128), (3, 128, 128), (4, 192, 192), (5, 128, 192), (6, 192, 256), (7, 192, 320),
+                                           (8, 128, 320), (9, 256, 192)])
+@pytest.mark.parametrize("k, splits", [(160, 3), (96, 2), (608, 9), (1056, 12), (1024, 7)])
+def test_tiled_product_in_ranges_of_every_shape(shape, bn, bm, k, splits):
+    """Ranges that do not divide the steps of 64, of one step and of several, with a last one of half its size: each slab holds its
+    own range's sums, a sum of k exact products within k roundings of its terms."""
+    from qwen25vl_lite_amd.ops import tile
+    m, n = bm + 33, bn + 22
+    g = torch.Generator(device="cuda").manual_seed(shape + k)
+    x = torch.randn(m, k, device="cuda", generator=g).bfloat16()
+    w = (torch.randn(n, k, device="cuda", generator=g) / k ** 0.5).bfloat16()
+    out = torch.full((splits, m, n), math.nan, device="cuda")
+    tile._launch(x, w, out, n, tile._SLABS, splits=splits, shape=shape)
+    steps = (k + 63) // 64
+    for i in range(splits):
+        at = slice(64 * (steps * i // splits), 64 * (steps * (i + 1) // splits))
+        a, b = x[:, at].double(), w[:, at].double()
+        assert bool(((out[i].double() - a @ b.T).abs() <= k * 2.0 ** -24 * (a.abs() @ b.abs().T)).all()), i
+
+
 @pytest.mark.parametrize("m", [1, 19, 40])
 @pytest.mark.parametrize("n", [2, 34, 16401, 40970])
 def test_rows_with_a_last_output_alone(m, n):
