@@ -14,9 +14,9 @@
 // Why ranges: one chain an output is 32 cycles for four values of K wherever the outputs are few (8 x 2,048 x 11,008: 37 us at
 // least, 118 as measured), and cannot be shared out; ranges run in waves and blocks beside each other.  Short
 // runs round off less (error against 64 bits at K = 2,048 1.3e-7 of the
-// result, one chain 8.1e-7; at 11,008 1.7e-7 and 1.9e-6).  Before and after: 6 x 2,048 x 11,008 117 and 24 us, 6 x 22,016 x 2,048 44 and 33
-// (5.4 TB/s), 6 x 151,936 x 2,048 233 and 198 (6.3 TB/s), 6 x 2,048 x 2,048 24 and 7; 164 x 2,048 x 11,008 188 and 92, 164 x 22,016 x
-// 2,048 230 and 190, 700 x 22,016 x 2,048 874 and 550 (115 TFLOP/s).
+// result, one chain 8.1e-7; at 11,008 1.7e-7 and 1.9e-6).  Before and after, weights from memory: 6 x 2,048 x 11,008 118 and 25 us, 6 x 22,016 x
+// 2,048 46 and 35 (5.1 TB/s), 6 x 151,936 x 2,048 240 and 202 (6.2 TB/s), 6 x 2,048 x 2,048 25 and 9; 164 x 2,048 x 11,008 193 and 95, 164 x 22,016 x
+// 2,048 237 and 201, 700 x 22,016 x 2,048 872 and 588 (107 TFLOP/s).
 #include "common.h"
 
 #include <cmath>
@@ -154,7 +154,7 @@ __device__ __forceinline__ void wait_steps(int ahead) {
 // ranges.  A wave fetches its steps of 32 values ahead through a ring of LDS of its own, across its tiles, W's lines
 // whole (8 rows of 128 bytes an instruction) and marked as read once: no barrier stands between a fetch and its use, only
 // the sums of the ranges meet once a tile.  XF fetches of 8 rows of A a step.  WF = 1 where that leaves a tile for each compute
-// unit at most: one unit fetches some 40 GB/s, so all should (6 x 2,048 x 11,008 with 16 outputs a block, on half of them, 29 us for 24).
+// unit at most: one unit fetches some 40 GB/s, so all should (6 x 2,048 x 11,008 with 16 outputs a block, on half of them, 29 us for 25).
 #define F32_STREAM_ROWS 16
 template <int WF, int XF>
 __global__ __launch_bounds__(64 * MOST_RANGES) void gemm_f32_stream_kernel(const float* __restrict__ A, int lda,

@@ -16,14 +16,14 @@
 // Masses are whole numbers of 2^-40 of the largest score's (of more for rows beyond 2^23 scores, whose sum
 // would not fit 64 bits), which is finer than a float32 sum of them and lets the blocks add in any order.  One block a row that searched bit by bit, 32 passes for each
 // threshold, took 3.70 ms for 64 rows of 152,064 (greedy, top-p, top-k with top-p and penalties, min-p
-// in turn); these passes together take 113 us.
+// in turn); these passes together 117 in nine kernels.
 //
-// Most rows need none of these passes: what their cuts leave is a short list.  Each 64 scores of a row have a
+// Most rows need none of these passes: what their cuts leave is a short list.  Each group of 256 scores of a row has a
 // largest one; the k-th largest of those is no larger than the k-th largest score, and scores that far below the largest one that
 // all of a row's could not make up 1 - top_p never matter.  So one pass gathers what such a bound leaves (and adds up all
 // mass, where top-p needs it), and a block a row finds the thresholds among these few and draws, with the same sums.  Rows
 // whose list is longer than LIST, or whose list does not reach top-p, go the long way; the others' blocks there end at once.
-// The 64 rows above: 43 us in three kernels, all of it reading and finding, the passes 117 in nine.
+// The 64 rows above: 45 us in three kernels, all of it reading and finding.  Rows that draw from all of their scores are not tried.
 #include "common.h"
 #include <cmath>
 #include <cstddef>
