@@ -712,6 +712,28 @@ def test_peaked_rows_of_any_vocabulary_are_settled_by_their_list(vocab, monkeypa
         assert got == [100 + int(u * kept) for u in us] and len(waits) == 1
 
 
+def test_sampling_from_slot_records_is_that_of_the_rows_settings():
+    """A served step's way to the sampler and sample_rows: the same ids for every kind of row, slots in any order, rows of short lists, long ones
+    and none."""
+    from qwen25vl_lite_amd.cache.slots import SlotRecords
+    from qwen25vl_lite_amd.sampling import SamplingParams
+    from qwen25vl_lite_amd.sampling.sampler import sample_rows, sample_slots_begin
+    kinds = [dict(), dict(temperature=0.7, top_p=0.9), dict(temperature=1.0, top_k=50, top_p=0.95, repetition_penalty=1.1), dict(temperature=0.8, min_p=0.05),
+             dict(temperature=1.0), dict(temperature=0.0, presence_penalty=0.5), dict(temperature=3.0, top_p=0.97), dict(temperature=1.0, top_k=900)]
+    params = [SamplingParams(seed=None if k.get("temperature", 0.0) == 0.0 else 3 * i, **k) for i, k in enumerate(kinds)]
+    n, vocab = len(params), 40001
+    g = torch.Generator().manual_seed(5)
+    slots = torch.randperm(n + 5, generator=g)[:n].tolist()
+    records = SlotRecords(n + 5)
+    for trial in range(4):
+        prev = [torch.randint(0, vocab, (trial * 9 + i,), generator=g).tolist() for i in range(n)]
+        for slot, p, ids in zip(slots, params, prev):
+            records.assign(slot, p, generated=len(ids))
+        logits = (torch.randn(n, vocab, generator=g) * (1 + 2 * (trial % 2))).cuda()
+        want = sample_rows(logits, params, prev, [len(ids) for ids in prev])
+        assert sample_slots_begin(logits, records, slots, prev).result() == want
+
+
 def test_trace_run_program(model_dirs, tmp_path):
     """bin/trace_run as a user calls it: JSON steps on standard input, `done <step>` lines,
     <step>.f32 files of little-endian float32 [wanted, vocab]."""
