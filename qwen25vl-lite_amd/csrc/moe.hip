@@ -658,9 +658,10 @@ __global__ __launch_bounds__(512) void moe_stream_kernel(ExpertArgs a, int tiles
 
 // How long tiles of bm pairs take, in microseconds: the rounds of the XCD that gets most blocks (they go there in groups of 4 x 8 tiles),
 // each a step of 64 values of K after the other, `alone` where most compute units are idle and `full` where all work, and 2.9 more for its
-// first fetches and its stores.  The pairs' shares are not known on the host: an expert is taken to waste 0.4 of a tile.
-static double stream_us(int P, int E, int bm, int tiles_n, int K, double alone, double full, int cus) {
-  const int there = P / bm + (E < P ? E : P), used = (int)((double)P / bm + 0.4 * E + 0.5), real = used < there ? used : there;
+// first fetches and its stores.  The pairs' shares are not known on the host: an expert is taken to waste
+// `waste` of a tile.
+static double stream_us(int P, int E, int bm, double waste, int tiles_n, int K, double alone, double full, int cus) {
+  const int there = P / bm + (E < P ? E : P), used = (int)((double)P / bm + waste * E + 0.5), real = used < there ? used : there;
   const int supers_m = (there + 3) / 4, supers = supers_m * ((tiles_n + 7) / 8);
   double most = (double)real * tiles_n / 8;
   if (supers <= 1024) {
@@ -676,12 +677,15 @@ static double stream_us(int P, int E, int bm, int tiles_n, int K, double alone, 
   return whole * (steps * full + 2.9) + (rest > 0 ? steps * (alone + (full - alone) * rest) + 2.9 : 0.0);
 }
 // Whether tiles of 256 pairs are the faster ones.  Of 264 products (8, 32 and 64 experts of 768 to 4,096 outputs, 262 to 1,300 pairs each) two are
-// over 2 per cent slower than with tiles of 128 (8 and 12), and 0.8 per cent of the time is lost on average; by the number of pairs alone 66 were
+// over 2 per cent slower than with tiles of 128 (8 and 12), and 1.7 per cent of the time is lost on average; by the number of pairs alone 66 were
 // (up to 46), and 4.9 per cent was lost.
 extern "C" int qvl_moe_wide_pairs(int P, int E, int R, int K, int gated, int cus) {
   if (P <= 0 || E <= 0 || R <= 0 || K <= 0 || cus <= 0 || P < WIDE_PAIRS * (long long)E) return 0;
   const int cols = gated ? ExpertsTile::BN / 2 : ExpertsTile::BN, tiles_n = (R + cols - 1) / cols;
-  return stream_us(P, E, WideTile::BM, tiles_n, K, 0.967, 1.361, cus) < stream_us(P, E, ExpertsTile::BM, tiles_n, K, 0.678, 0.825, cus);
+  // (0.4 is what routers' choices at random wasted; 0.55 as well, so that some pairs more in one expert's tile are not a round more)
+  const double narrow = stream_us(P, E, ExpertsTile::BM, 0.4, tiles_n, K, 0.678, 0.825, cus);
+  return stream_us(P, E, WideTile::BM, 0.4, tiles_n, K, 0.967, 1.361, cus) < narrow &&
+         stream_us(P, E, WideTile::BM, 0.55, tiles_n, K, 0.967, 1.361, cus) < narrow;
 }
 
 // x_dtype / out_dtype: 0 float32, 1 bfloat16.  float32 operands write float32; bfloat16 operands

@@ -179,7 +179,7 @@ def test_a_library_is_loaded_as_it_is_asked_for():
     (3096, 8, 1376, 2048, 1, 256, 0), (3096, 8, 2048, 1376, 0, 256, 0), (2560, 8, 768, 2048, 1, 256, 0), (12384, 32, 2368, 3584, 1, 256, 1),
     (12384, 32, 3584, 2368, 0, 256, 1), (17982, 32, 1376, 2048, 1, 256, 0), (17982, 32, 2048, 1376, 0, 256, 1), (24576, 32, 1376, 2048, 1, 256, 1),
     (8191, 32, 2368, 3584, 1, 256, 0), (65536, 64, 768, 2048, 1, 256, 1), (1 << 20, 16, 4096, 4096, 1, 256, 1), (24576, 32, 1376, 2048, 1, 64, 1),
-    (5, 8, 64, 64, 1, 256, 0), (0, 8, 64, 64, 1, 256, 0), (4096, 8, 64, 64, 1, 0, 0)])
+    (12798, 32, 768, 2048, 1, 256, 0), (5, 8, 64, 64, 1, 256, 0), (0, 8, 64, 64, 1, 256, 0), (4096, 8, 64, 64, 1, 0, 0)])
 def test_where_experts_take_tiles_of_256_pairs(pairs, experts, outputs, k, gated, units, wide):
     """By the rounds of blocks that they come out in, which cross at other numbers of pairs for few experts than for many and for a
     gated product than for the one behind it."""
