@@ -118,15 +118,14 @@ __device__ __forceinline__ float4 load4(const bf16_t* p) {
   return float4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16), __uint_as_float(v.y & 0xffff0000u)};
 }
 
-// The same where head size and page size are multiples of four.  What bounds a token's few keys is the time until a load comes
+// The same where head size and page size are multiples of four, in one, two or four waves.  What bounds a token's few keys is the time until a load comes
 // back, so loads are wide and many are in flight: four waves take the blocks of 64 keys in turn, each with a
 // softmax of its own (joined at the end, in the waves' order); eight lanes read a key's row side by side, and a lane
 // reads a channel's values of four keys at once.  CH: channels of a value, in sixteens, at most.
 // float32, 16 heads of 128 over 2 of keys: 7 tokens at 25 to 100 keys 51 us with the wave above, 11 with these; 164 tokens of two prompts 57 and 33.
 // Values of more than 128 channels are read 128 at a time: with all of a value's reads in one array the compiler kept it in scratch memory (28 heads of
 // 512, bfloat16, 64 tokens at 1,000 keys 3,697 us, so 937, with the wave above 1,973; of 256, 64 tokens at 64 keys 224, 88 and 67).
-#define ATTN_WAVES 4
-template <typename T, int CH>
+template <typename T, int CH, int ATTN_WAVES>
 __global__ __launch_bounds__(64 * ATTN_WAVES) void attn_generic_vec_kernel(
     const T* __restrict__ q, const T* __restrict__ kc, const T* __restrict__ vc, const int* __restrict__ block_table, int table_width,
     const int* __restrict__ token_req, const int* __restrict__ token_seqpos, T* __restrict__ out, int nh, int nkv, int hd, int vd, int ps,
@@ -160,7 +159,9 @@ __global__ __launch_bounds__(64 * ATTN_WAVES) void attn_generic_vec_kernel(
     const T* row[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const int j = min(first + (lane & 56) + i, p), pk = bt[j / ps];
+      int j = min(first + (lane & 56) + i, p);
+      if constexpr (ATTN_WAVES < 4) j = j < lo && j >= kept ? p : j;       // (a key that is not seen: one that is; its score is left out)
+      const int pk = bt[j / ps];
       const size_t page = (size_t)(pk < 0 ? 0 : pk);   // a table without this page: read page 0, never out of bounds
       row[i] = kc + ((page * nkv + kvh) * ps + (size_t)(j % ps)) * hd;
     }
@@ -196,6 +197,8 @@ __global__ __launch_bounds__(64 * ATTN_WAVES) void attn_generic_vec_kernel(
     for (int t = 0; t < 4; ++t) {
       const int j0 = first + 16 * t + 4 * quad;
       if (first + 16 * t > p) break;
+      if constexpr (ATTN_WAVES < 4)
+        if (first + 16 * t + 15 < lo && first + 16 * t >= kept) continue;      // none of the sixteen is seen
       const int at = min(j0, p & ~3), pk = bt[at / ps];
       const size_t page = (size_t)(pk < 0 ? 0 : pk);
       const T* v = vc + ((page * nkv + kvh) * vd) * ps + (size_t)(at % ps);
@@ -282,20 +285,32 @@ extern "C" int qvl_attn_generic(const void* q, const void* kc, const void* vc, c
   if (hd > ATTN_MAX_HD || vd > ATTN_MAX_HD || nh > 65535) return QVL_ERR_LIMIT;
   const dim3 grid(N, nh);
   const bool vec = hd % 4 == 0 && ps % 4 == 0 && ((uintptr_t)kc % 16) == 0 && ((uintptr_t)vc % 16) == 0;
-#define VEC(T, CH)                                                                                                       \
-  hipLaunchKernelGGL((attn_generic_vec_kernel<T, CH>), grid, dim3(64 * ATTN_WAVES), 0, stream, (const T*)q, (const T*)kc,  \
+#define VEC(T, CH, WAVES)                                                                                                \
+  hipLaunchKernelGGL((attn_generic_vec_kernel<T, CH, WAVES>), grid, dim3(64 * WAVES), 0, stream, (const T*)q, (const T*)kc, \
                      (const T*)vc, (const int*)block_table, table_width, (const int*)token_req, (const int*)token_seqpos, \
                      (T*)out, nh, nkv, hd, vd, ps, window, keep_first, chunk, scale, (const float*)sinks,                 \
                      (const float2*)turn, turn_pairs)
+#define CHANNELS(T, WAVES)                       \
+  do {                                           \
+    if (vd <= 128) VEC(T, 8, WAVES);             \
+    else if (vd <= 256) VEC(T, 16, WAVES);       \
+    else VEC(T, ATTN_MAX_HD / 16, WAVES);        \
+  } while (0)
   if (vec && (dtype == 0 || dtype == 1)) {
-    if (dtype == 0 && vd <= 128) VEC(float, 8);
-    else if (dtype == 0 && vd <= 256) VEC(float, 16);
-    else if (dtype == 0) VEC(float, ATTN_MAX_HD / 16);
-    else if (vd <= 128) VEC(bf16_t, 8);
-    else if (vd <= 256) VEC(bf16_t, 16);
-    else VEC(bf16_t, ATTN_MAX_HD / 16);
+    // A token that sees few keys, in two blocks of 64 at most, has no work for four waves (16 heads of 64 over 2, bfloat16, 2,000 tokens, windows of 16
+    // and 64 keys: the kernel above 100 and 278 us, four waves 305 and 327, one 91 and two 164)
+    long long most = window > 0 ? window : 0x7fffffff;
+    if (chunk > 0 && chunk < most) most = chunk;
+    if (keep_first > 0) most += keep_first;
+    if (dtype == 0 && most <= 32) CHANNELS(float, 1);
+    else if (dtype == 0 && most <= 64) CHANNELS(float, 2);
+    else if (dtype == 0) CHANNELS(float, 4);
+    else if (most <= 32) CHANNELS(bf16_t, 1);
+    else if (most <= 64) CHANNELS(bf16_t, 2);
+    else CHANNELS(bf16_t, 4);
     return qvl_launch_status();
   }
+#undef CHANNELS
 #undef VEC
   if (dtype == 0)
     hipLaunchKernelGGL(attn_generic_kernel<float>, grid, dim3(64), 0, stream, (const float*)q, (const float*)kc,

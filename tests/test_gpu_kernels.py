@@ -304,6 +304,15 @@ def test_generic_attention_of_wide_values(dtype, hd, vd):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("hd, vd, window, keep, chunk", [(64, 64, 16, 0, None), (16, 24, 1, 0, None), (100, 132, 20, 12, None), (32, 260, 33, 0, None),
+                                                         (64, 64, 40, 24, None), (128, 128, 64, 0, None), (64, 64, None, 0, 24), (64, 200, None, 0, 50),
+                                                         (8, 8, 30, 0, 17)])
+def test_generic_attention_of_few_keys(dtype, hd, vd, window, keep, chunk):
+    """Windows and chunks of so few keys that one wave looks at them, or two, the kept ones among them."""
+    test_generic_attention_of_long_contexts(dtype, 4, 2, hd, vd, 8, window, keep, chunk)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("hd", [64, 62])
 @pytest.mark.parametrize("low", [(64, 128), (0, 64), (0, 256), (130, 301)])
 def test_generic_attention_beside_scores_of_minus_infinity(dtype, hd, low):
