@@ -160,14 +160,14 @@ template <int WF, int XF>
 __global__ __launch_bounds__(64 * MOST_RANGES) void gemm_f32_stream_kernel(const float* __restrict__ A, int lda,
                                                                            const float* __restrict__ W, int ldw,
                                                                            const float* __restrict__ bias, float* __restrict__ C,
-                                                                           int ldc, int M, int N, int K, int tiles, int groups) {
+                                                                           int ldc, int M, int N, int K, int tiles, int groups, int turns,
+                                                                           int ranges, int part) {
   constexpr int STEP = 32, ROWS_W = 8 * WF, FETCHES = WF + XF, STAGE = FETCHES * 1024, SUMS = MOST_RANGES * 1024;   // SUMS: bytes of a tile's
   constexpr int STAGES = (163840 - 2 * SUMS) / MOST_RANGES / STAGE;
   __shared__ __attribute__((aligned(16))) char lds[MOST_RANGES * STAGES * STAGE + 2 * SUMS];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
-  const int range = range_of(K), ranges = (K + range - 1) / range, group = wave / ranges;
+  const int range = range_of(K), group = wave * part >> 16;       // wave / ranges
   const int k_first = (wave - group * ranges) * range, ksteps = group < groups ? (min(K - k_first, range) + STEP - 1) / STEP : 0;
-  const int turns = (tiles + groups - 1) / groups;
   const int my_tiles = (turns - (int)blockIdx.x + (int)gridDim.x - 1) / (int)gridDim.x, steps = ksteps * my_tiles;
   char* sums = lds + MOST_RANGES * STAGES * STAGE;
   const char* mine = lds + wave * STAGES * STAGE;
@@ -513,9 +513,9 @@ extern "C" int qvl_gemm_f32(const void* A, int lda, const void* W, int ldw, cons
         const double cost = (double)(((tiles + n - 1) / n + cus - 1) / cus) * n / (n * ranges < 5 ? n * ranges / 5.0 : 1.0);
         if (cost < least) least = cost, groups = n;
       }
-      const int turns = (tiles + groups - 1) / groups;
+      const int turns = (tiles + groups - 1) / groups, part = 65536 / ranges + 1;
       const dim3 grid(turns < cus ? turns : cus), block(64 * MOST_RANGES);
-#define GO(WF, XF) hipLaunchKernelGGL((gemm_f32_stream_kernel<WF, XF>), grid, block, 0, stream, a, lda, w, ldw, b, (float*)C, ldc, M, N, K, tiles, groups)
+#define GO(WF, XF) hipLaunchKernelGGL((gemm_f32_stream_kernel<WF, XF>), grid, block, 0, stream, a, lda, w, ldw, b, (float*)C, ldc, M, N, K, tiles, groups, turns, ranges, part)
       if (narrow && M <= 8) GO(1, 1);
       else if (narrow) GO(1, 2);
       else if (M <= 8) GO(2, 1);
