@@ -118,14 +118,14 @@ def _gather(params, prev_ids, steps, vocab: int, host: torch.Tensor, more=None):
             fn.restype = ctypes.c_long
             fn.argtypes = [ctypes.py_object] * 3 + [ctypes.c_long] * 2 + [ctypes.c_void_p, ctypes.c_long] + [ctypes.c_void_p] * 2
             _gather_fn = fn
-    flags = (ctypes.c_int32 * 4)()
+    flags = _Flags()
     if _gather_fn is False:
         return -1, flags
-    return _gather_fn(params, prev_ids, steps, len(params), vocab, host.data_ptr(), host.numel(), ctypes.addressof(flags),
-                      None if more is None else ctypes.addressof(more)), flags
+    return _gather_fn(params, prev_ids, steps, len(params), vocab, host.data_ptr(), host.numel(), flags, more), flags
 
 
 _gather_fn = None
+_Flags, _More = ctypes.c_int32 * 4, ctypes.c_int32 * 3
 
 
 class PendingSample:
@@ -190,7 +190,7 @@ def _sample_rows(logits, params, prev_ids, steps, uniforms, wait: bool):
         return _launch(logits, rows, flat, wait)
     if uniforms is None:
         with torch.cuda.device(logits.device):
-            slot, more = _up.take(m * _ROW_WORDS + 1, logits.device), (ctypes.c_int32 * 3)()
+            slot, more = _up.take(m * _ROW_WORDS + 1, logits.device), _More()
             words, flags = _gather(params, prev_ids, steps, vocab, slot[0], more)
             if words < -1:
                 _up.give(slot, logits.device)
@@ -201,7 +201,7 @@ def _sample_rows(logits, params, prev_ids, steps, uniforms, wait: bool):
                     rows = slot[0].numpy()[:m * _ROW_WORDS].view(_ROW)
                     for i in np.nonzero(rows["seeded"] < 0)[0]:
                         rows["u"][i], rows["seeded"][i] = uniform_from(None, 0), 0
-                return _queue(logits, _send(slot, words, logits.device), *flags, *more[:2], wait)
+                return _queue(logits, _send(slot, words, logits.device), *flags, more[0], more[1], wait)
             _up.give(slot, logits.device)
     filled = []
     for i, p in enumerate(params):
