@@ -25,7 +25,11 @@
 #include "common.h"
 #include <type_traits>
 #include "attention_mfma.h"
+#include <algorithm>
 #include <atomic>
+#include <functional>
+#include <utility>
+#include <vector>
 #include <mutex>
 
 #ifndef HD
@@ -626,10 +630,7 @@ __device__ __forceinline__ void init_state(TileState& st) {
 // With head sizes up to 128 the kernel also comes with GROUPS = 2 such groups of BLK_WAVES waves in
 // a workgroup, on the same column tiles: group g walks the key blocks g, g + 2, ... through stages
 // of its own, and the groups' sums are merged through LDS at the end.  One such workgroup fills a
-// compute unit where two of the plain kind do, and a walk takes half as long.  That pays where a
-// step has no more walks than the plain kind has places and they differ much in length (one
-// prompt of 2,048 tokens: the first tiles see few keys, the last ones all); with more walks the
-// plain kind's independent workgroups overlap their matrix and vector phases better.
+// compute unit where two of the plain kind do, and a walk takes half as long.
 #define BLK_WAVES 4
 #if HD <= 128
 #ifndef BLK_CT
@@ -760,36 +761,122 @@ __device__ __forceinline__ void operands_from_lds(const bf16_t* ks, const bf16_t
   for (int dt = 0; dt < NT; ++dt) rg.v[dt] = load8(vs + (vslot + 32 * dt) * 8);
 }
 
-// One entry of the block list for one key/value head.  blk_cb counts in units of
-// BLK_WAVES * BLK_CT column tiles.
+// One entry of the plan (see qvl_attn_mfma_block_plan): BLK_WAVES * BLK_CT column tiles of a request over the 32-key blocks
+// kb_first .. kb_last, the first part of a walk from the first block its columns see and the last part to the last one, whatever the
+// plan took the request's length for (a captured step is planned once, for contexts that grow).
+#define ITEM_INTS 8
+struct BlockItem {
+  int req, cb;             // the request, and which of its runs of BLK_WAVES * BLK_CT column tiles
+  int head;                // key/value head
+  int kb_first, kb_last;
+  int part, parts;         // of the run's whole walk
+  int slot, counter;       // parts > 1: where the walk's first partial result is, and its counter
+};
 template <int GROUPS>
 struct BlockShared {
   __attribute__((aligned(16))) bf16_t stage[GROUPS][BLK_STAGES][STAGE_ELEMS];   // K rows, then V^T rows
-  int wave_range[GROUPS * BLK_WAVES][2];
-  int work;
+  int is_last, next;
 };
 // what a lane of the second group hands over per column tile: its sums, the reference and its share of the total
 #define MERGE_REGS (NT * 4 + 2)
 static_assert(BLK_MAX_GROUPS == 1 || BLK_CT * MERGE_REGS * BLK_WAVES * 64 * 4 <= BLK_STAGES * STAGE_ELEMS * 2,
               "the second group's sums do not fit its stages");
 
+// Device-scope ("agent") stores and loads: visible across the XCDs' L2 caches.
+__device__ __forceinline__ void store_device_scope(float* p, float v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float load_device_scope(const float* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void store_device_scope(unsigned long long* p, float a, float b) {
+  __hip_atomic_store(p, (unsigned long long)__float_as_uint(a) | (unsigned long long)__float_as_uint(b) << 32, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ float2 load_device_scope(const unsigned long long* p) {
+  const unsigned long long v = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return float2{__uint_as_float((uint32_t)v), __uint_as_float((uint32_t)(v >> 32))};
+}
+
+// A part of a walk leaves, per wave and column tile, PART_PAIRS pairs of floats a lane (its sums, then reference and total),
+// pair by pair for the 64 lanes: whole lines, and a lane finds the same lane's.
+#define PART_PAIRS (NT * 2 + 1)
+#define PART_ULLS (BLK_WAVES * BLK_CT * PART_PAIRS * 64)
+
+// The sums of all parts of a walk, in their order, into st; at: the lane's first pair of part 0.  All tiles of a part are asked
+// for together: what bounds this is the trip to memory, once a part.
+__device__ __forceinline__ void merge_parts(const unsigned long long* at, int parts, TileState* st) {
+#pragma unroll
+  for (int t = 0; t < BLK_CT; ++t) init_state(st[t]);
+  for (int p = 0; p < parts; ++p) {
+    float2 v[BLK_CT][PART_PAIRS];
+#pragma unroll
+    for (int t = 0; t < BLK_CT; ++t)
+#pragma unroll
+      for (int j = 0; j < PART_PAIRS; ++j) v[t][j] = load_device_scope(at + (size_t)p * PART_ULLS + (t * PART_PAIRS + j) * 64);
+#pragma unroll
+    for (int t = 0; t < BLK_CT; ++t) {
+      const float m_p = v[t][2 * NT].x, m = fmaxf(st[t].m, m_p);
+      const float ref = m == -INFINITY ? 0.f : m;      // no key of the column so far: all sums are zero
+      const float keep = __builtin_amdgcn_exp2f(st[t].m - ref), wgt = __builtin_amdgcn_exp2f(m_p - ref);
+      st[t].m = m;
+#pragma unroll
+      for (int dt = 0; dt < NT; ++dt) {
+        f32x4_t& o = st[t].acc[dt];
+        o[0] = o[0] * keep + v[t][2 * dt].x * wgt;
+        o[1] = o[1] * keep + v[t][2 * dt].y * wgt;
+        o[2] = o[2] * keep + v[t][2 * dt + 1].x * wgt;
+        o[3] = o[3] * keep + v[t][2 * dt + 1].y * wgt;
+      }
+      st[t].acc[NT][0] = st[t].acc[NT][0] * keep + v[t][2 * NT].y * wgt;
+    }
+  }
+}
+
+// This lane's part of its column's row of the output.
+__device__ __forceinline__ void store_column(const TileInfo& t, const TileState& st, const HeadEnd& end, bf16_t* __restrict__ out,
+                                             int nq, int lg) {
+  if (!t.valid) return;
+  const float inv = head_end(end, t.token, t.head, st.acc[NT][0], st.m);
+  bf16_t* orow = out + ((size_t)t.token * nq + t.head) * HD;
+#pragma unroll
+  for (int dt = 0; dt < NT; ++dt) {
+    const int d = dt * 16 + 4 * lg;
+    uint2 wv;
+    wv.x = pack2(st.acc[dt][0] * inv, st.acc[dt][1] * inv);
+    wv.y = pack2(st.acc[dt][2] * inv, st.acc[dt][3] * inv);
+    *reinterpret_cast<uint2*>(orow + d) = wv;
+  }
+}
+
 template <int GROUPS>
-__device__ __forceinline__ void attend_block(BlockShared<GROUPS>& sh, int item, int kvh, const bf16_t* __restrict__ q,
+__device__ __forceinline__ void attend_block(BlockShared<GROUPS>& sh, const BlockItem& item, const bf16_t* __restrict__ q,
                                              const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
                                              const int* __restrict__ bt, int table_width,
                                              const int* __restrict__ cu_q, const int* __restrict__ ctx_len,
-                                             const int* __restrict__ blk_req, const int* __restrict__ blk_cb,
                                              bf16_t* __restrict__ out, int nq, int nkv, int ps, int window,
-                                             float scale, const HeadEnd& end) {
+                                             float scale, unsigned long long* __restrict__ partials, int* __restrict__ counters,
+                                             const HeadEnd& end, int* __restrict__ tickets, int& ticket) {
+  const int kvh = item.head;
   const int g = nq / nkv;
   const int wave_of_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int group = wave_of_all / BLK_WAVES, wave = wave_of_all % BLK_WAVES;
-  const int r = blk_req[item], ct0 = (blk_cb[item] * BLK_WAVES + wave) * BLK_CT;
+  const int r = item.req, ct0 = (item.cb * BLK_WAVES + wave) * BLK_CT;
   const int ncols = (cu_q[r + 1] - cu_q[r]) * g;
   TileInfo t[BLK_CT];
   bf16x8_t qb[BLK_CT][KS];
   TileState st[BLK_CT];
   int lo = 0x7fffffff, hi = -1;
+  // the key blocks of this part
+  int kb_first = item.kb_first, kb_last = item.kb_last;
+  {
+    const int qlen = cu_q[r + 1] - cu_q[r], before = ctx_len[r] - qlen;
+    const int column = item.cb * (BLK_WAVES * BLK_CT * 16), most = qlen - 1;
+    const int from = before + column / g - window + 1, to = (column + BLK_WAVES * BLK_CT * 16 - 1) / g;
+    const int kb_lo = window > 0 && from > 0 ? from >> 5 : 0, kb_hi = (before + (to < most ? to : most)) >> 5;
+    kb_first = item.part == 0 || kb_first < kb_lo ? kb_lo : kb_first;
+    kb_last = item.part == item.parts - 1 || kb_last > kb_hi ? kb_hi : kb_last;
+  }
   Walk<BLK_CT> w;
 #pragma unroll
   for (int i = 0; i < BLK_CT; ++i) {
@@ -805,20 +892,6 @@ __device__ __forceinline__ void attend_block(BlockShared<GROUPS>& sh, int item, 
       hi = t[i].hi_tile > hi ? t[i].hi_tile : hi;
     }
   }
-  if (lane == 0) {
-    sh.wave_range[wave_of_all][0] = lo;
-    sh.wave_range[wave_of_all][1] = hi;
-  }
-  __syncthreads();
-  int blo = 0x7fffffff, bhi = -1;
-#pragma unroll
-  for (int i = 0; i < GROUPS * BLK_WAVES; ++i) {
-    blo = min(blo, sh.wave_range[i][0]);
-    bhi = max(bhi, sh.wave_range[i][1]);
-  }
-  if (bhi < 0) return;  // uniform over the block
-  blo = __builtin_amdgcn_readfirstlane(blo);
-  bhi = __builtin_amdgcn_readfirstlane(bhi);
   w.key_begin = lo; w.key_end = hi;
   w.scale_log2 = scale * LOG2E; w.lg = lane >> 4; w.r = lane & 15;
   {  // the range every column of this wave sees
@@ -842,7 +915,7 @@ __device__ __forceinline__ void attend_block(BlockShared<GROUPS>& sh, int item, 
   ld.table_width = table_width; ld.ps = ps; ld.wave = wave;
   // this group's blocks are kb0, kb0 + GROUPS, ...: nblk of them; every group goes round the
   // loop (and through its barrier) as often as the first
-  const int kb0 = (blo >> 5) + group, all_blocks = (bhi >> 5) - (blo >> 5) + 1;
+  const int kb0 = kb_first + group, all_blocks = kb_last - kb_first + 1;   // (a part may have none)
   const int nblk = (all_blocks - group + GROUPS - 1) / GROUPS;
   const int rounds = (all_blocks + GROUPS - 1) / GROUPS;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)&sh.stage[group][0][0];
@@ -898,7 +971,16 @@ __device__ __forceinline__ void attend_block(BlockShared<GROUPS>& sh, int item, 
   };
   int i = 0;
   for (; i < nblk - (BLK_STAGES - 1); ++i) round(i, std::true_type{});
+  // The ticket for the workgroup's next item is on its way during the last rounds.  (It stands behind loads that these wait for
+  // with the counts of loads alone: they wait for one load more.)
+  if (tickets && threadIdx.x == 0) ticket = __hip_atomic_fetch_add(tickets, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   for (; i < rounds; ++i) round(i, std::false_type{});
+  // The sums stay where they are up to here: what follows is told of new values, or the compiler, with two ways to store them,
+  // moves all of them from one register to another in every round (8,192 tokens 505 us for 460).
+#pragma unroll
+  for (int t = 0; t < BLK_CT; ++t)
+#pragma unroll
+    for (int dt = 0; dt <= NT; ++dt) asm volatile("" : "+v"(st[t].acc[dt]));
   if (GROUPS > 1) {
     // The second group's sums reach the first through the second group's stages, which nobody reads
     // or fills any more: word (tile, register, wave, lane), so every lane finds its partner's.
@@ -917,9 +999,9 @@ __device__ __forceinline__ void attend_block(BlockShared<GROUPS>& sh, int item, 
       }
     }
     __syncthreads();
-    if (group > 0) return;
 #pragma unroll
     for (int i = 0; i < BLK_CT; ++i) {
+      if (group > 0) break;
       const float* theirs = hand + ((size_t)i * MERGE_REGS * BLK_WAVES + wave) * 64 + lane;
       const float m_b = theirs[(NT * 4) * BLK_WAVES * 64], l_b = theirs[(NT * 4 + 1) * BLK_WAVES * 64];
       const float m = fmaxf(st[i].m, m_b);
@@ -931,36 +1013,55 @@ __device__ __forceinline__ void attend_block(BlockShared<GROUPS>& sh, int item, 
 #pragma unroll
         for (int j = 0; j < 4; ++j)
           st[i].acc[dt][j] = st[i].acc[dt][j] * sa + theirs[(dt * 4 + j) * BLK_WAVES * 64] * sb;
-      st[i].m = ref;
+      st[i].m = m;
     }
   }
-  const int lg = lane >> 4;
+  if (item.parts > 1) {   // uniform over the workgroup
+    // The part that finishes last adds up all of them.  Parts may run on different XCDs: as with the splits of the kernel for
+    // few tiles, the results go through memory at device scope, and every thread waits for its stores before the workgroup is
+    // counted in.  It leaves the counter at zero.
+    unsigned long long* walk = partials + (size_t)item.slot * PART_ULLS + (size_t)wave * (BLK_CT * PART_PAIRS * 64) + lane;
+    if (group == 0) {
+      unsigned long long* mine = walk + (size_t)item.part * PART_ULLS;
 #pragma unroll
-  for (int i = 0; i < BLK_CT; ++i) {
-    if (!t[i].valid) continue;
-    const float inv = head_end(end, t[i].token, t[i].head, st[i].acc[NT][0], st[i].m);
-    bf16_t* orow = out + ((size_t)t[i].token * nq + t[i].head) * HD;
+      for (int i = 0; i < BLK_CT; ++i) {
 #pragma unroll
-    for (int dt = 0; dt < NT; ++dt) {
-      const int d = dt * 16 + 4 * lg;
-      uint2 wv;
-      wv.x = pack2(st[i].acc[dt][0] * inv, st[i].acc[dt][1] * inv);
-      wv.y = pack2(st[i].acc[dt][2] * inv, st[i].acc[dt][3] * inv);
-      *reinterpret_cast<uint2*>(orow + d) = wv;
+        for (int dt = 0; dt < NT; ++dt) {
+          store_device_scope(mine + (i * PART_PAIRS + 2 * dt) * 64, st[i].acc[dt][0], st[i].acc[dt][1]);
+          store_device_scope(mine + (i * PART_PAIRS + 2 * dt + 1) * 64, st[i].acc[dt][2], st[i].acc[dt][3]);
+        }
+        store_device_scope(mine + (i * PART_PAIRS + 2 * NT) * 64, st[i].m, st[i].acc[NT][0]);
+      }
     }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int* count = counters + item.counter;
+      const int before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      sh.is_last = before == item.parts - 1;
+      if (sh.is_last) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!sh.is_last) return;   // uniform over the workgroup
+    if (group > 0) return;
+    merge_parts(walk, item.parts, st);
   }
+  if (group > 0) return;
+#pragma unroll
+  for (int i = 0; i < BLK_CT; ++i) store_column(t[i], st[i], end, out, nq, lane >> 4);
 }
 
-// The workgroups take (entry, head) pairs from queues in global memory until these are empty: the
-// host lists the entries longest walk first, so the long walks start at once and the short ones
-// fill in behind them, whatever mix of requests the step has.  Workgroups go to the 8 XCDs in
-// turn; when the key/value heads divide 8 there is a queue per head and a workgroup serves the
-// head of its XCD first (that XCD's L2 then holds one head's keys) and the others when its own
-// queue is empty.  queue[i] is the next entry of queue i, queue[QUEUE_DONE] counts the workgroups
-// that have found every queue empty; the last of them puts all counters back to zero for the
-// next launch (launches that share the counters must not overlap).
-#define QUEUE_DONE 8
-#define QUEUE_INTS 16
+// The plan's items are listed longest first.  Workgroup w begins with item `place` and then takes the next that nobody has
+// taken, by tickets from a counter: the list is balanced by blocks, and what is left of the differences between compute
+// units evens out.  Workgroups go to the 8 XCDs in turn; when the key/value
+// heads divide 8, the list is of one head's walks, workgroup w serves head (w % 8) % nkv (an XCD's L2 then holds few heads'
+// keys) and is place w / 8 * (8 / nkv) + (w % 8) / nkv of that head, and every head has a counter; otherwise the items name their heads.  Counters lie
+// 256 bytes apart, and no workgroup asks another head's: with 512 workgroups raising neighbouring counters, each all of them,
+// eight prompts of 300 tokens took 47 us for 20.  A list that is no longer than the places needs none.
+// The last workgroup of a list puts its counters back to zero (launches that share them must not overlap).
+// head_slots, head_walks: the plan's partial results and cut walks, of one head.
+#define TICKET_INTS 64                  // from one head's counters to the next: tickets, and 128 bytes on the workgroups that found no more
+#define WALK_COUNTERS_AT (8 * TICKET_INTS)
 #if HD <= 128
 #define BLK_PER_CU 2   // of the plain kind (GROUPS = 1); the kind with two groups fills a compute unit alone
 #else
@@ -970,29 +1071,33 @@ template <int GROUPS>
 __global__ __launch_bounds__(64 * BLK_WAVES * GROUPS, GROUPS == 1 ? BLK_PER_CU : 1) void attn_mfma_block_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
     const int* __restrict__ bt, int table_width, const int* __restrict__ cu_q, const int* __restrict__ ctx_len,
-    const int* __restrict__ blk_req, const int* __restrict__ blk_cb, int num_blocks, bf16_t* __restrict__ out, int nq,
-    int nkv, int ps, int window, float scale, int* __restrict__ queue, HeadEnd end) {
+    const int* __restrict__ items, int count, int places, int head_slots, int head_walks,
+    bf16_t* __restrict__ out, int nq, int nkv, int ps, int window, float scale, unsigned long long* __restrict__ partials,
+    int* __restrict__ counters, HeadEnd end) {
   __shared__ BlockShared<GROUPS> sh;
   const bool per_head = 8 % nkv == 0;
-  const int queues = per_head ? nkv : 1;
-  const int per_queue = per_head ? num_blocks : num_blocks * nkv;
-  const int home = (blockIdx.x & 7) % queues;
-  for (int turn = 0; turn < queues; ++turn) {
-    const int qi = (home + turn) % queues;
-    for (;;) {
-      if (threadIdx.x == 0) sh.work = atomicAdd(&queue[qi], 1);
-      __syncthreads();
-      const int work = __builtin_amdgcn_readfirstlane(sh.work);   // the same for all: keep it scalar
-      if (work >= per_queue) break;  // uniform over the block; every workgroup gets here for every queue
-      attend_block(sh, per_head ? work : work / nkv, per_head ? qi : work % nkv, q, kc, vc, bt, table_width, cu_q,
-                   ctx_len, blk_req, blk_cb, out, nq, nkv, ps, window, scale, end);
-      __syncthreads();               // everybody has read sh.work and is done with the stages
-    }
-    __syncthreads();
+  const int w = blockIdx.x, head = per_head ? (w & 7) % nkv : 0;
+  const int place = per_head ? (w >> 3) * (8 / nkv) + (w & 7) / nkv : w;
+  if (place >= places) return;
+  int* tickets = count > places ? counters + head * TICKET_INTS : nullptr;
+  int ticket = 0;
+  for (int i = place; i < count;) {
+    const int* it = items + (size_t)i * ITEM_INTS;
+    const BlockItem item{it[0], it[1], per_head ? head : it[2], it[3], it[4], it[5] & 0xffff, it[5] >> 16,
+                         it[6] + head * head_slots, it[7] + head * head_walks};
+    attend_block(sh, item, q, kc, vc, bt, table_width, cu_q, ctx_len, out, nq, nkv, ps, window, scale, partials,
+                 counters + WALK_COUNTERS_AT, end, tickets, ticket);
+    if (!tickets) return;
+    if (threadIdx.x == 0) sh.next = places + ticket;
+    __syncthreads();   // and everybody is done with the stages
+    i = __builtin_amdgcn_readfirstlane(sh.next);
   }
-  if (threadIdx.x == 0 && atomicAdd(&queue[QUEUE_DONE], 1) == (int)gridDim.x - 1) {
-    for (int i = 0; i < queues; ++i) atomicExch(&queue[i], 0);  // nobody takes work any more
-    atomicExch(&queue[QUEUE_DONE], 0);
+  if (threadIdx.x == 0) {
+    int* ended = tickets + TICKET_INTS / 2;
+    if (__hip_atomic_fetch_add(ended, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == places - 1) {   // nobody asks any more
+      __hip_atomic_store(tickets, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(ended, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
 }
 
@@ -1017,14 +1122,6 @@ __global__ __launch_bounds__(64 * BLK_WAVES * GROUPS, GROUPS == 1 ? BLK_PER_CU :
 #else
 #define COOP_WAVES 2
 #endif
-
-// Device-scope ("agent") stores and loads: visible across the XCDs' L2 caches.
-__device__ __forceinline__ void store_device_scope(float* p, float v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float load_device_scope(const float* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 
 // Merge the nsplit partial results of one (tile, kv head) and write the tile's rows of the output:
 // thread -> (column, 4 channels); splits are summed in order.  ACROSS: the partial results were
@@ -1206,35 +1303,190 @@ static int check_common(int num_tiles, int nq, int nkv, int ps, int table_width)
   return -1;
 }
 
-// Column tiles per entry of the block list that qvl_attn_mfma_block expects, and how many of its
-// workgroups a compute unit holds at a time.
+// Column tiles a walk of the kernel for many tiles has, and how many of its workgroups a compute unit holds at a time.
 extern "C" int qvl_attn_mfma_block_tiles() { return BLK_WAVES * BLK_CT; }
 extern "C" int qvl_attn_mfma_block_per_cu() { return BLK_PER_CU; }
 extern "C" int qvl_attn_mfma_block_max_groups() { return BLK_MAX_GROUPS; }
-extern "C" int qvl_attn_mfma_queue_ints() { return QUEUE_INTS; }
+// What the kernel for many tiles does, as a list: every run of BLK_WAVES * BLK_CT column tiles of every request has one walk
+// over the key blocks it sees, whose length the host knows, and walks are cut into parts where whole ones would leave places
+// (workgroups that a device runs at a time) without work.
+//
+// Longest first, a walk goes to the place with least to do if that place is then done at time T; walks that fit nowhere are
+// cut and fill what room is left, place by place.  T starts at the mean and grows until everything has a place (uncut, all
+// have one at the latest when T is what longest-first alone gives).  Times are in blocks of 32 keys: a block costs one, a
+// walk ITEM_COST more (its queries, its first blocks on their way, its results), a part of a cut one PART_COST more (it stores its sums) and
+// MERGE_COST for each part its walk has (one of them reads all).  Half and twice these costs give the same times to 3 per cent.
+//
+// Measured at the 7B decoder's heads, before there were lists (one entry of a queue for each walk, uncut) and now: 4,096 tokens at 8,192 and 12,288
+// keys 441 us and 363, 797 and 580 (600 walks of nearly one length came out as two rounds on 512 places); 2,048 at 2,048 keys 65 and 53, at
+// 8,192 266 and 220; 512 at 4,096 81 and 51; eight prompts of 300 47 and 20; 2,048 with 64 query heads 131 and 87; 16,384 1,724 and 1,701.
+#define ITEM_COST 4
+#define PART_COST 2
+#define MERGE_COST 2
+#define LEAST_PART 8
+
+struct PlanWalk {
+  int req, cb, head, kb_first, kb_last;
+};
+struct PlanPart {
+  int walk, kb_first, kb_last, part;
+};
+// Tries to have everything done at time T; parts of place p in placed[p].
+static bool plan_at(const std::vector<PlanWalk>& walks, const std::vector<int>& order, int places, int groups, int T, int most_cut,
+                    std::vector<std::vector<PlanPart>>& placed, std::vector<int>& parts_of) {
+  for (auto& p : placed) p.clear();
+  typedef std::pair<int, int> Load;   // (time, place)
+  std::vector<Load> heap;
+  heap.reserve(places);
+  for (int p = 0; p < places; ++p) heap.push_back(Load{0, p});   // (a heap already: all loads are equal)
+  const auto later = std::greater<Load>();
+  std::vector<int> left;
+  auto blocks = [&](int i) { return walks[i].kb_last - walks[i].kb_first + 1; };
+  auto rounds = [&](int n) { return (n + groups - 1) / groups; };
+  for (int i : order) {
+    const int cost = rounds(blocks(i)) + ITEM_COST;
+    if (heap[0].first + cost > T) {
+      left.push_back(i);
+      continue;
+    }
+    std::pop_heap(heap.begin(), heap.end(), later);
+    heap.back().first += cost;
+    placed[heap.back().second].push_back(PlanPart{i, walks[i].kb_first, walks[i].kb_last, 0});
+    parts_of[i] = 1;
+    std::push_heap(heap.begin(), heap.end(), later);
+  }
+  if (left.empty()) return true;
+  std::sort(heap.begin(), heap.end());   // most room first
+  size_t at = 0;
+  int cut = 0;
+  for (int i : left) {
+    int from = walks[i].kb_first, rest = blocks(i), part = 0;
+    const int inside = T - ITEM_COST - PART_COST > 0 ? T - ITEM_COST - PART_COST : 1;
+    const int extra = ITEM_COST + PART_COST + MERGE_COST * ((rounds(rest) + inside - 1) / inside + 1);
+    while (rest > 0) {
+      if (at == heap.size() || part >= 0x7fff) return false;
+      const bool whole = part == 0 && heap[at].first + ITEM_COST + rounds(rest) <= T;
+      int take = whole ? rest : (T - heap[at].first - extra) * groups;
+      if (take < rest && rest - take < LEAST_PART * groups) take = whole ? rest : rest - LEAST_PART * groups;
+      if (take > rest) take = rest;
+      if (!whole && take < LEAST_PART * groups && take < rest) {
+        ++at;
+        continue;
+      }
+      placed[heap[at].second].push_back(PlanPart{i, from, from + take - 1, part++});
+      heap[at].first += rounds(take) + (whole ? ITEM_COST : extra);
+      from += take;
+      rest -= take;
+      if (rest > 0) ++at;
+    }
+    parts_of[i] = part;
+    cut += part > 1;
+  }
+  return cut <= most_cut;
+}
+
+// The list for requests whose tokens stand at cu_q[i] .. cu_q[i + 1] - 1 of the step and whose contexts after it are ctx[i] long
+// (host memory; only: null, or 0 for requests to leave out), nq / nkv = g, on `places` workgroups of `groups` wave groups.
+// out: ITEM_INTS for each item, `room` items at most; at most most_cut walks are cut.  head: workgroups to launch, items, places taken,
+// partial results (of all heads), partial results and cut walks of one head (0 where the items name their heads).
+extern "C" int qvl_attn_mfma_block_plan(const int* cu_q, const int* ctx, const unsigned char* only, int reqs, int g, int nkv,
+                                        int window, int places, int groups, int most_cut, int* out, long long room, int* head) {
+  if (!cu_q || !ctx || !out || !head || reqs <= 0 || g <= 0 || nkv <= 0 || places <= 0 || groups < 1 || groups > BLK_MAX_GROUPS || most_cut < 0)
+    return QVL_ERR_SHAPE;
+  try {
+    const bool per_head = 8 % nkv == 0;
+    const int columns = 16 * BLK_WAVES * BLK_CT;
+    if (per_head) places = places / 8 * 8 / nkv > 0 ? places / 8 * 8 / nkv : 8 / nkv;
+    if (per_head) most_cut /= nkv;
+    std::vector<PlanWalk> walks;
+    long long total = 0;
+    for (int r = 0; r < reqs; ++r) {
+      const long long q = (long long)cu_q[r + 1] - cu_q[r];
+      if (q <= 0 || (only && !only[r])) continue;
+      if (ctx[r] < q) return QVL_ERR_SHAPE;
+      const long long runs = (q * g + columns - 1) / columns;
+      for (long long cb = 0; cb < runs; ++cb) {
+        const long long a = cb * columns / g, b = std::min((cb * columns + columns - 1) / g, q - 1);
+        const long long lo = window > 0 ? std::max(0ll, ctx[r] - q + a - window + 1) : 0, hi = ctx[r] - q + b;
+        for (int h = 0; h < (per_head ? 1 : nkv); ++h) {
+          walks.push_back(PlanWalk{r, (int)cb, h, (int)(lo >> 5), (int)(hi >> 5)});
+          total += ((hi >> 5) - (lo >> 5) + groups) / groups + ITEM_COST;
+        }
+      }
+    }
+    if (walks.size() > 0x7fffffffull / 64) return QVL_ERR_LIMIT;
+    const int n = (int)walks.size();
+    std::vector<int> order(n), parts_of(n);
+    for (int i = 0; i < n; ++i) order[i] = i;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+      return walks[a].kb_last - walks[a].kb_first > walks[b].kb_last - walks[b].kb_first;
+    });
+    std::vector<std::vector<PlanPart>> placed(places);
+    int T = (int)std::min<long long>(total / places + 1, 0x3fffffff);
+    while (!plan_at(walks, order, places, groups, T, most_cut, placed, parts_of)) T += T / 32 + 1;
+    struct Listed {
+      int blocks;
+      PlanPart part;
+    };
+    std::vector<Listed> list;
+    for (const auto& parts : placed)
+      for (const PlanPart& part : parts) list.push_back(Listed{part.kb_last - part.kb_first + 1, part});
+    std::sort(list.begin(), list.end(), [](const Listed& a, const Listed& b) {
+      return a.blocks != b.blocks ? a.blocks > b.blocks : a.part.walk != b.part.walk ? a.part.walk < b.part.walk : a.part.part < b.part.part;
+    });
+    if ((long long)list.size() > room) return QVL_ERR_LIMIT;
+    std::vector<int> slot(n), counter(n);
+    long long slots = 0;
+    int counters = 0;
+    for (int i = 0; i < n; ++i) {
+      slot[i] = (int)slots;
+      counter[i] = counters;
+      if (parts_of[i] > 1) slots += parts_of[i], ++counters;
+    }
+    if (slots * (per_head ? nkv : 1) > 0x7fffffffll) return QVL_ERR_LIMIT;
+    int* it = out;
+    for (const Listed& l : list) {
+      const PlanWalk& w = walks[l.part.walk];
+      it[0] = w.req; it[1] = w.cb; it[2] = w.head; it[3] = l.part.kb_first; it[4] = l.part.kb_last;
+      it[5] = l.part.part | parts_of[l.part.walk] << 16; it[6] = slot[l.part.walk]; it[7] = counter[l.part.walk];
+      it += ITEM_INTS;
+    }
+    const int count = (int)list.size(), taken = std::min(count, places), per8 = per_head ? 8 / nkv : 1;
+    head[0] = per_head ? (taken + per8 - 1) / per8 * 8 : taken;
+    head[1] = count;
+    head[2] = taken;
+    head[3] = (int)(slots * (per_head ? nkv : 1));
+    head[4] = per_head ? (int)slots : 0;
+    head[5] = per_head ? counters : 0;
+    return QVL_OK;
+  } catch (...) {
+    return QVL_ERR_LIMIT;
+  }
+}
+
+// Bytes of one partial result.
+extern "C" long long qvl_attn_mfma_block_part_bytes() { return PART_ULLS * 8ll; }
 
 extern "C" int qvl_attn_mfma_block(const void* q, const void* kc, const void* vc, const void* bt, int table_width,
-                                   const void* cu_q, const void* ctx_len, const void* blk_req, const void* blk_cb,
-                                   int num_blocks, void* out, const void* sinks, const void* gates,
-                                   long long gate_stride, int nq, int nkv, int ps, int window, float scale, void* queue, int max_workgroups, int groups, hipStream_t stream) {
+                                   const void* cu_q, const void* ctx_len, const void* items, int grid, int count, int places,
+                                   int head_slots, int head_walks, void* out, const void* sinks, const void* gates,
+                                   long long gate_stride, int nq, int nkv, int ps, int window, float scale, void* partials,
+                                   void* counters, int groups, hipStream_t stream) {
   // sinks: float32 [nq] or null: one more term exp(sink) in each query head's softmax denominator.
   // gates: float32, a row of gate_stride values per token, or null: head h's output times sigmoid(row[h]).
-  // queue: qvl_attn_mfma_queue_ints() ints, zero before the first launch that uses them.
-  // groups: wave groups per workgroup, 1 .. qvl_attn_mfma_block_max_groups(); max_workgroups should
-  // be what the device holds at a time (qvl_attn_mfma_block_per_cu() per compute unit with one group, one with two).
-  const int c = check_common(num_blocks, nq, nkv, ps, table_width);
+  // items, grid, count, places, head_slots, head_walks: as qvl_attn_mfma_block_plan gives them, the items on the device.
+  // partials: room for the partial results that the plan counts; counters: WALK_COUNTERS_AT + most_cut ints, zero before
+  // the launch, which leaves them at zero.  groups: as the plan was made for.
+  const int c = check_common(grid, nq, nkv, ps, table_width);
   if (c >= 0) return c;
-  if (!(scale > 0.f) || !queue || max_workgroups <= 0) return QVL_ERR_SHAPE;
+  if (!(scale > 0.f) || !items || !counters || count <= 0 || places <= 0 || places > count || ((uintptr_t)partials % 8)) return QVL_ERR_SHAPE;
   if (groups < 1 || groups > BLK_MAX_GROUPS) return QVL_ERR_LIMIT;
-  const long long total = (long long)num_blocks * nkv;
-  if (total > 0x7fffffffLL) return QVL_ERR_LIMIT;
-  const unsigned grid = (unsigned)(total < max_workgroups ? total : max_workgroups);
   const HeadEnd end{(const float*)sinks, (const float*)gates, gate_stride};
 #define QVL_BLOCK_LAUNCH(G)                                                                                          \
   hipLaunchKernelGGL(attn_mfma_block_kernel<G>, dim3(grid), dim3(64 * BLK_WAVES * G), 0, stream, (const bf16_t*)q,    \
                      (const bf16_t*)kc, (const bf16_t*)vc, (const int*)bt, table_width, (const int*)cu_q,              \
-                     (const int*)ctx_len, (const int*)blk_req, (const int*)blk_cb, num_blocks, (bf16_t*)out, nq, nkv, \
-                     ps, window, scale, (int*)queue, end)
+                     (const int*)ctx_len, (const int*)items, count, places, head_slots, head_walks,               \
+                     (bf16_t*)out, nq, nkv, ps, window, scale, (unsigned long long*)partials, (int*)counters, end)
   if (groups == 1) QVL_BLOCK_LAUNCH(1);
 #if BLK_MAX_GROUPS > 1
   else QVL_BLOCK_LAUNCH(2);

@@ -9,7 +9,7 @@ from __future__ import annotations
 
 import collections
 import ctypes
-from typing import Optional, Tuple
+from typing import NamedTuple, Optional, Tuple
 
 import numpy as np
 import torch
@@ -24,8 +24,11 @@ _MAX_HD = 256
 # them hold a number instead of None where a caller (a test) fixes the count itself.
 TARGET_PER_CU = 2          # from this many (tile, head) pairs a compute unit on, a wave per tile fills the device
 FILL_PER_CU = 1            # with fewer cooperative blocks than this, contexts are split among blocks
-WIDE_WALKS_PER_CU = 3      # the kind of the kernel whose waves carry three column tiles: from this many walks on
-WIDE_BLOCKS_PER_CU = 586   # ... that have this many 32-key blocks to walk between them (150,000 on 256 units)
+WIDE_WALK_BLOCKS = 80      # the kind of the kernel whose waves carry three column tiles: walks of this many 32-key blocks on average
+WIDE_BLOCKS_PER_CU = 160   # ... and this many between them (41,000 on 256 units); measured with 16, 28 and 64 query heads: 43,000 blocks of 96 a walk
+                           # 111 us for 116, 98,000 of 192 217 for 235, 115,000 of 128 252 for 258, 229,000 of 224 454 for 471; but 31,000 of 240
+                           # 94 for 91, 13,000 of 120 65 for 52 (fewer walks, more cuts), and 33,000 and 57,000 of 64 the same within 3 per cent
+GROUPS_WALK_BLOCKS = 64    # two wave groups (block_groups): walks this long on average (64 walks of 24 blocks 26 us for 24)
 TARGET_BLOCKS = None
 FILL_BLOCKS = None
 MIN_KEYS_PER_SPLIT = 256   # keys a split has at least
@@ -34,6 +37,8 @@ SPLIT_FROM_KEYS = 768      # shorter contexts are walked by one block: merging s
                            # (one compute unit by itself fetches its keys and values at about 40 GB/s); measured at batch 1 and 8:
                            # 527 keys 11.5 us whole, 11.9 in two splits; 1,024 keys 17.8 whole, 12.0 in four
 MERGE_COUNTERS = 1 << 16   # (tile, kv head) pairs whose splits one launch can merge by itself
+TICKET_COUNTERS = 8 * 64   # WALK_COUNTERS_AT in the source
+CUT_WALKS = 1 << 13        # walks of one launch that may be cut into parts
 ALONE_KEYS = 4096          # decoded tokens beside prompt portions get a launch of their own from this context on
 WIDE_CT = 3
 _cu_count = {}
@@ -69,8 +74,7 @@ def block_defines(head_dim: int, wide: bool) -> dict:
     """The library of the kernel for many tiles: compiled per head size, and for head sizes up to 128
     in a second kind whose waves carry three column tiles instead of two.  That kind reads its operands
     from LDS once for three tiles (a third less LDS traffic and bookkeeping per product) at the price
-    of longer walks and no second group of waves: 6 % faster from about 8,192 prompt tokens on at the
-    7B decoder's heads, slower below."""
+    of longer walks and no second group of waves (where it is taken: ``WIDE_WALK_BLOCKS``)."""
     return {"HD": head_dim, "BLK_CT": WIDE_CT} if wide and head_dim <= 128 else {"HD": head_dim}
 
 
@@ -124,29 +128,67 @@ def _counters(device: torch.device) -> torch.Tensor:
 
 
 def _work_queue(device: torch.device):
-    """Per device: the counters of the block kernel's work queues and how many workgroups fill
-    the device.  A launch finds the counters at zero and leaves them at zero; launches on one
+    """Per device: the counters of the kernel for many tiles (from which workgroups take tickets for their next walk, and by which
+    the parts of a cut walk find out which of them finishes last) and how many compute units there are.  A launch finds the counters at zero and leaves them at zero; launches on one
     device share them, so they must follow each other on one stream (the engine has one).  A launch
     that reports an error has them cleared."""
     key = torch.device(device).index or 0
     if key not in _queues:
         cus = torch.cuda.get_device_properties(device).multi_processor_count
-        _queues[key] = (torch.zeros(16, dtype=torch.int32, device=device), cus)
+        _queues[key] = (torch.zeros(TICKET_COUNTERS + CUT_WALKS, dtype=torch.int32, device=device), cus)
     return _queues[key]
 
 
-def _step_tiles(step, group: int, tile_ct: int, device, by_length: bool = False, only=None):
+class BlockPlan(NamedTuple):
+    """What the kernel for many tiles does in which order (csrc/attention_mfma.hip, qvl_attn_mfma_block_plan)."""
+
+    items: np.ndarray       # [n, 8]: request, run of column tiles, head, first and last key block, part | parts << 16, slot, counter
+    grid: int               # workgroups to launch
+    places: int             # of a head (or of all, where the items name their heads): workgroups that have an item to begin with
+    partials: int           # partial results of all heads
+    head_slots: int         # partial results and cut walks of one head (0: the items name their heads)
+    head_walks: int
+
+
+def plan_walks(cu_q, ctx_len, group: int, nkv: int, window: int, places: int, groups: int, defines: dict, only=None) -> BlockPlan:
+    """The walks of a step's runs of column tiles, cut where that keeps more of ``places`` workgroups of ``groups`` wave groups busy."""
+    cu = np.ascontiguousarray(cu_q, dtype=np.int32)
+    ctx = np.ascontiguousarray(ctx_len, dtype=np.int32)
+    keep = None if only is None else np.ascontiguousarray(only, dtype=np.uint8)
+    cols = 16 * int(_fn("attention_mfma", "qvl_attn_mfma_block_tiles", [], defines)())
+    runs = int(((np.diff(cu.astype(np.int64)) * group + cols - 1) // cols).sum())
+    room = runs * nkv + places       # a part that is cut off fills its place or ends its walk
+    out, head = np.empty((room, 8), dtype=np.int32), np.zeros(6, dtype=np.int32)
+    fn = _fn("attention_mfma", "qvl_attn_mfma_block_plan", [_c_ptr] * 3 + [_c_int] * 7 + [_c_ptr, _c_ll, _c_ptr], defines)
+    _check(fn(cu.ctypes.data, ctx.ctypes.data, None if keep is None else keep.ctypes.data, len(ctx), group, nkv, window, places,
+              groups, CUT_WALKS, out.ctypes.data, room, head.ctypes.data), "paged_attention (plan of the walks)")
+    grid, count, taken_places, partials, head_slots, head_walks = (int(x) for x in head)
+    return BlockPlan(out[:count], grid, taken_places, partials, head_slots, head_walks)
+
+
+def _step_tiles(step, group: int, tile_ct: int, device, only=None):
     """The step's entries on the device; ``only``: a tuple of 0/1 per request, entries of the others left out."""
     cache = step.derived
-    key = ("tiles", group, tile_ct, by_length, only)
+    key = ("tiles", group, tile_ct, only)
     if key not in cache:
-        req, ct = tiles_for(step.cu_q_host, group, tile_ct, step.ctx_len_host if by_length else None)
+        req, ct = tiles_for(step.cu_q_host, group, tile_ct)
         if only is not None:
             keep = np.asarray(only, dtype=bool)[req]
             req, ct = req[keep], ct[keep]
         both = int32_to_device(np.concatenate([req, ct]), device)
         cache[key] = (both[:len(req)], both[len(req):], len(req))
     return cache[key]
+
+
+def _count_tiles(step, group: int, tile_ct: int, only=None) -> int:
+    """Entries of ``tile_ct`` column tiles that the step's requests make."""
+    key = ("count of tiles", group, tile_ct, only)       # the same for every layer of the step
+    if key not in step.derived:
+        q = np.diff(np.asarray(step.cu_q_host, dtype=np.int64))
+        if only is not None:
+            q = q * np.asarray(only, dtype=np.int64)
+        step.derived[key] = int(((q * group + 16 * tile_ct - 1) // (16 * tile_ct)).sum())
+    return step.derived[key]
 
 
 def _walk_blocks(step, group: int, tile_ct: int, only=None) -> int:
@@ -157,6 +199,29 @@ def _walk_blocks(step, group: int, tile_ct: int, only=None) -> int:
         q = q * np.asarray(only, dtype=np.int64)
     entries = (q * group + 16 * tile_ct - 1) // (16 * tile_ct)
     return int((entries * np.maximum(1, (ctx - q // 2 + 31) // 32)).sum())
+
+
+def _step_walks(step, group: int, nkv: int, hd: int, window: int, device, only=None, force_wide=None, force_groups=None):
+    """``(wide, wave groups, defines, plan, its items on the device)`` of the step's prompt portions, the same for every layer with
+    these heads."""
+    key = ("walks", group, nkv, hd, window, only, force_wide, force_groups)
+    if key in step.derived:
+        return step.derived[key]
+    cus = _work_queue(device)[1]
+    num_tiles, blocks = _count_tiles(step, group, block_tiles(hd), only), _walk_blocks(step, group, block_tiles(hd), only)
+    wide = force_wide
+    if wide is None:
+        # a run of twelve tiles that ends early walks for nothing more often than one of eight
+        wide = (hd <= 128 and blocks >= WIDE_WALK_BLOCKS * num_tiles and blocks * nkv >= WIDE_BLOCKS_PER_CU * cus
+                and _walk_blocks(step, group, block_tiles(hd, True), only) * WIDE_CT <= 1.04 * 2 * blocks)
+    defines = block_defines(hd, wide)
+    per_cu = int(_fn("attention_mfma", "qvl_attn_mfma_block_per_cu", [], defines)())
+    groups = force_groups
+    if groups is None:
+        groups = block_groups(num_tiles * nkv, cus * per_cu, hd) if not wide and blocks >= GROUPS_WALK_BLOCKS * num_tiles else 1
+    plan = plan_walks(step.cu_q_host, step.ctx_len_host, group, nkv, window, cus * (per_cu if groups == 1 else 1), groups, defines, only)
+    step.derived[key] = (wide, groups, defines, plan, int32_to_device(plan.items.reshape(-1), device))
+    return step.derived[key]
 
 
 def long_single_tiles(step, group: int, nkv: int, device=None):
@@ -187,10 +252,11 @@ def _long_single_tiles(step, group: int, nkv: int, device):
 def block_groups(walks: int, places: int, head_dim: int) -> int:
     """Wave groups per workgroup for a step of ``walks`` (entry, head) pairs on a device that holds
     ``places`` plain workgroups at a time.  Two groups (head sizes up to 128) halve a walk's time at
-    a tenth less throughput (measured at 2,048 to 8,192 tokens): they pay when all walks start at
-    once and the longest decides, not when places are taken several times over."""
+    a tenth less throughput: they pay where walks are so few that they are cut into many parts, of which one then adds up
+    half as many (on 512 places, 68 walks of 124 key blocks 43 us for 50, of 247 62 for 71; 112 of 120 and 128 of 240 the same within 5
+    per cent; 224 of 240 149 for 146)."""
     most = int(_fn("attention_mfma", "qvl_attn_mfma_block_max_groups", [], {"HD": head_dim})())
-    return 2 if most >= 2 and walks <= places else 1
+    return 2 if most >= 2 and 4 * walks <= places else 1
 
 
 def try_attention(q, k_cache, v_cache, block_table, step, num_q_heads: int, window: Optional[int],
@@ -219,35 +285,28 @@ def try_attention(q, k_cache, v_cache, block_table, step, num_q_heads: int, wind
     _need(gate is None or (gate.is_cuda and gate.dtype == torch.float32 and gate.shape == (n, nq) and gate.stride(1) == 1),
           "gate must be float32 [N, nq] on the GPU with contiguous rows")
     gate_args = (_ptr(gate), 0 if gate is None else gate.stride(0))
-    tile_req, tile_ct, num_tiles = _step_tiles(step, nq // nkv, 1, q.device)
     out = torch.empty_like(q)
     defines = {"HD": hd}
-    kind, nsplit, per = plan_splits(num_tiles, nkv, step.max_ctx_len, q.device)
+    kind, nsplit, per = plan_splits(_count_tiles(step, nq // nkv, 1), nkv, step.max_ctx_len, q.device)
 
     def many_tiles(only):
-        tile_req, tile_ct, num_tiles = _step_tiles(step, nq // nkv, block_tiles(hd), q.device, by_length=True, only=only)
-        wide = force_wide
-        if wide is None:   # many and long walks: measured at the 7B decoder's heads, the wide kind wins from one prompt of about 8,192 tokens on
-            cus = _compute_units(q.device)
-            wide = (hd <= 128 and num_tiles * nkv >= WIDE_WALKS_PER_CU * cus
-                    and _walk_blocks(step, nq // nkv, block_tiles(hd), only) * nkv >= WIDE_BLOCKS_PER_CU * cus)
-        defines = block_defines(hd, wide)
-        if wide:
-            tile_req, tile_ct, num_tiles = _step_tiles(step, nq // nkv, block_tiles(hd, True), q.device, by_length=True, only=only)
+        wide, groups, defines, plan, items = _step_walks(step, nq // nkv, nkv, hd, int(window or 0), q.device, only, force_wide, force_groups)
         fn = _fn("attention_mfma", "qvl_attn_mfma_block",
-                 [_c_ptr] * 4 + [_c_int] + [_c_ptr] * 4 + [_c_int, _c_ptr, _c_ptr, _c_ptr, _c_ll] + [_c_int] * 4
-                 + [_c_float, _c_ptr, _c_int, _c_int, _c_ptr], defines)
-        queue, cus = _work_queue(q.device)
-        per_cu = int(_fn("attention_mfma", "qvl_attn_mfma_block_per_cu", [], defines)())
-        most = int(_fn("attention_mfma", "qvl_attn_mfma_block_max_groups", [], defines)())
-        groups = block_groups(num_tiles * nkv, cus * per_cu, hd) if force_groups is None else force_groups
-        groups = min(groups, most) if force_groups is None else groups
+                 [_c_ptr] * 4 + [_c_int] + [_c_ptr] * 3 + [_c_int] * 5 + [_c_ptr, _c_ptr, _c_ptr, _c_ll] + [_c_int] * 4
+                 + [_c_float, _c_ptr, _c_ptr, _c_int, _c_ptr], defines)
+        counters = _work_queue(q.device)[0]
+        partials = None
+        if plan.partials:
+            size = _fn("attention_mfma", "qvl_attn_mfma_block_part_bytes", [], defines)
+            size.restype = ctypes.c_longlong
+            partials = torch.empty(plan.partials * int(size()), dtype=torch.uint8, device=q.device)
         code = fn(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), block_table.shape[1], _ptr(step.cu_q),
-                  _ptr(step.ctx_len), _ptr(tile_req), _ptr(tile_ct), num_tiles, _ptr(out), _ptr(sinks), *gate_args, nq, nkv, ps, int(window or 0),
-                  float(scale), _ptr(queue), cus * (per_cu if groups == 1 else 1), groups, _stream())
+                  _ptr(step.ctx_len), _ptr(items), plan.grid, len(plan.items), plan.places, plan.head_slots, plan.head_walks,
+                  _ptr(out), _ptr(sinks), *gate_args, nq, nkv, ps, int(window or 0), float(scale), _ptr(partials), _ptr(counters),
+                  groups, _stream())
         if code:
             # whatever a launch that went wrong did to the counters, the next one starts from zero
-            queue.zero_()
+            counters.zero_()
         _check(code, "paged_attention (matrix cores)")
         taken[f"many tiles, {WIDE_CT if wide else 2} column tiles a wave, {groups} wave group{'s' if groups > 1 else ''}"] += 1
 
@@ -294,7 +353,7 @@ def try_attention(q, k_cache, v_cache, block_table, step, num_q_heads: int, wind
         _, nsplit1, per1 = plan_splits(sum(single), nkv, longest, q.device)   # fewer blocks than fill the device: the kernel that splits
         shared_tiles(single, nsplit1, per1)
         rest = tuple(1 - s for s in single)
-        kind, nsplit, per = plan_splits(_step_tiles(step, nq // nkv, 1, q.device, only=rest)[2], nkv,
+        kind, nsplit, per = plan_splits(_count_tiles(step, nq // nkv, 1, rest), nkv,
                                         max(c for c, s in zip(step.ctx_len_host, rest) if s), q.device)
         if kind == "tile":
             many_tiles(rest)

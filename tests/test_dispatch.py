@@ -102,6 +102,58 @@ def test_a_steps_lists_are_not_made_inside_a_graph(monkeypatch):
         assert not Step.derived
 
 
+@pytest.mark.parametrize("qlens, lens, group, nkv, window", [([2048], [2048], 7, 4, 0), ([512], [8192], 7, 4, 0), ([1], [40000], 8, 1, 0),
+                                                             ([700, 1, 33], [3000, 9000, 33], 1, 6, 0), ([300, 0, 90], [5000, 7, 90], 5, 8, 1000),
+                                                             ([1], [1], 1, 16, 0), ([20000], [30000], 16, 2, 0)])
+@pytest.mark.parametrize("places, groups, wide", [(512, 1, False), (256, 2, False), (512, 1, True), (13, 1, False)])
+def test_walks_of_prompt_portions(qlens, lens, group, nkv, window, places, groups, wide):
+    """Every run of column tiles of every head has its key blocks once, in parts that follow each other, longest first; the parts of
+    cut walks have places of their own for their results; workgroups there are for all, and with few walks each has less than the longest walk."""
+    from qwen25vl_lite_amd.ops import attention_mfma as attn
+    cu = np.concatenate([[0], np.cumsum(qlens)])
+    defines = attn.block_defines(128, wide)
+    plan = attn.plan_walks(cu, lens, group, nkv, window, places, groups, defines)
+    cols, per_head = 16 * attn.block_tiles(128, wide), 8 % nkv == 0
+    heads = 1 if per_head else nkv
+    walks = {}
+    for req, cb, head, first, last, packed, slot, counter in plan.items.tolist():
+        walks.setdefault((req, cb, head), []).append((packed & 0xffff, packed >> 16, first, last, slot, counter))
+    want = {(r, cb, h) for r, q in enumerate(qlens) for cb in range(-(-q * group // cols)) for h in range(heads)}
+    assert set(walks) == want
+    slots, counters = [], []
+    for (r, cb, _), parts in walks.items():
+        parts.sort()
+        before = lens[r] - qlens[r]
+        lo = max(0, before + cb * cols // group - window + 1) if window else 0
+        hi = before + min((cb * cols + cols - 1) // group, qlens[r] - 1)
+        assert [p[0] for p in parts] == list(range(len(parts))) and {p[1] for p in parts} == {len(parts)}
+        assert parts[0][2] == lo >> 5 and parts[-1][3] == hi >> 5
+        assert all(a[3] + 1 == b[2] for a, b in zip(parts, parts[1:])) and all(p[2] <= p[3] for p in parts)
+        if len(parts) > 1:
+            slots += list(range(parts[0][4], parts[0][4] + len(parts)))
+            counters.append(parts[0][5])
+            assert len({p[4] for p in parts}) == len({p[5] for p in parts}) == 1
+    assert sorted(slots) == list(range(len(slots))) and sorted(counters) == list(range(len(counters)))
+    assert plan.partials == len(slots) * (nkv if per_head else 1)
+    assert (plan.head_slots, plan.head_walks) == ((len(slots), len(counters)) if per_head else (0, 0))
+    n = plan.items[:, 4] - plan.items[:, 3]
+    assert (np.diff(n) <= 0).all()
+    most = max(8 // nkv, places // 8 * 8 // nkv) if per_head else places
+    assert plan.places == min(most, len(plan.items))
+    # the workgroups launched reach every place of every head, and no more than eight beyond
+    assert plan.grid >= plan.places * (nkv if per_head else 1) > plan.grid - 8
+    if len(want) * 4 < most and n.max() >= 64:
+        assert counters
+
+
+@pytest.mark.parametrize("bad", [dict(lens=[3]), dict(groups=3), dict(nkv=0), dict(places=0)])
+def test_walks_that_cannot_be_listed(bad):
+    from qwen25vl_lite_amd.ops import attention_mfma as attn, kernels
+    kw = {**dict(lens=[9], nkv=2, places=16, groups=1), **bad}
+    with pytest.raises(kernels.KernelError):
+        attn.plan_walks([0, 4], kw["lens"], 2, kw["nkv"], 0, kw["places"], kw["groups"], {"HD": 128})
+
+
 def test_which_rows_of_the_stacked_projection_are_cut():
     """17 to 48 rows at any size, up to 64 of large weights beyond the inner size that the kernel with the rotation inside keeps in one
     pass."""

@@ -454,6 +454,36 @@ def test_mixed_step_with_few_long_decoded_tokens(nq, nkv, hd, window, monkeypatc
     assert torch.allclose(out.float().cpu(), c["want"], atol=1.5e-2, rtol=2e-2), err
 
 
+@pytest.mark.parametrize("kind", ["narrow", "two_groups", "wide", "planned_longer"])
+@pytest.mark.parametrize("nq, nkv, hd, window, ps", [(14, 2, 128, None, 16), (6, 6, 48, None, 48), (3, 3, 128, 1200, 32), (4, 1, 256, None, 16)])
+def test_paged_attention_walks_in_parts(nq, nkv, hd, window, ps, kind):
+    """Walks long and few enough to be cut: parts that end inside the context, that hold none of some columns' keys, and (a step
+    planned for longer contexts than it has, as a captured one is) no key at all.  The counters are back at zero behind every launch, and a second
+    one gives the same bits."""
+    from types import SimpleNamespace
+    import unittest.mock as mock
+    from qwen25vl_lite_amd.ops import attention_mfma
+    if hd == 256 and kind in ("two_groups", "wide"):
+        pytest.skip("built for head sizes up to 128")
+    lens, qlens = (1501, 64, 1030), (37, 20, 1)
+    c = _attention_case(torch.bfloat16, nq, nkv, hd, window, lens, qlens, ps=ps)
+    cu = [0, 37, 57, 58]
+    planned = [4096] * 3 if kind == "planned_longer" else list(lens)
+    cu_q, ctx_len = (torch.tensor(x, dtype=torch.int32).cuda() for x in (cu, lens))
+    step = SimpleNamespace(num_reqs=3, cu_q=cu_q, cu_q_host=cu, ctx_len=ctx_len, ctx_len_host=planned, max_q_len=37,
+                           max_ctx_len=max(planned), derived={})
+    with mock.patch.object(attention_mfma, "plan_splits", lambda t, n, m, d=None: ("tile", 1, 0)):
+        outs = [attention_mfma.try_attention(c["q"], c["kc"], c["vc"], c["table"], step, nq, window, c["scale"],
+                                             force_groups=2 if kind == "two_groups" else 1, force_wide=kind == "wide") for _ in range(3)]
+    plan = next(v for k, v in step.derived.items() if k[0] == "walks")[3]
+    assert plan.partials >= 2
+    torch.cuda.synchronize()
+    assert int(attention_mfma._work_queue(c["q"].device)[0].abs().sum()) == 0
+    for out in outs:
+        assert torch.equal(out, outs[0])
+        assert torch.allclose(out.float().cpu(), c["want"], atol=1.5e-2, rtol=2e-2), (out.float().cpu() - c["want"]).abs().max()
+
+
 @pytest.mark.parametrize("nq, nkv, hd, window, ps", [(28, 4, 128, None, 16), (6, 2, 48, 100, 16), (4, 4, 256, 257, 16),
                                                      (5, 1, 16, None, 16), (28, 4, 128, None, 48), (6, 2, 48, 100, 32),
                                                      (4, 4, 256, 257, 64), (4, 2, 32, None, 16), (8, 2, 64, 70, 32),
