@@ -14,7 +14,7 @@
 
 #include <cmath>
 
-enum { OUT_BF16 = 0, OUT_F32 = 1, OUT_GROUPED = 2, OUT_HALVES = 3 };
+enum { OUT_BF16 = 0, OUT_F32 = 1, OUT_GROUPED = 2, OUT_HALVES = 3, OUT_HEADS = 4 };
 
 struct TileArgs {
   const bf16_t* x;
@@ -28,7 +28,15 @@ struct TileArgs {
   int tiles_m, tiles_n, splits;
   int relu2, gelu;
   float alpha, limit, shift;
+  // OUT_HEADS: W holds nq query, nkv key and nkv value heads of HEAD rows; out takes the rotated queries [M, nq, HEAD]
+  const float* bias;     // [N] or null
+  const float4* cs;      // [M, HEAD / 2]: cosine and sine, two frequencies a value
+  const int* slot;       // [M]: page * ps + place in it, or -1
+  bf16_t* kc;            // [page][nkv][ps][HEAD]
+  bf16_t* vc;            // [page][nkv][HEAD][ps]
+  int nq, nkv, ps;
 };
+#define HEAD 128
 
 __device__ __forceinline__ uint32_t two_bf16(float a, float b) {
   typedef __bf16 pair_t __attribute__((ext_vector_type(2)));
@@ -58,6 +66,73 @@ __device__ __forceinline__ float clamped_gate(float g, float u, const TileArgs& 
   return g / (1.0f + expf(-p.alpha * g)) * (u + p.shift);
 }
 
+// OUT_HEADS: channels f and f + 64 of a head are rotated together, so the waves that share a head (one of 8 tiles of W's rows, two of
+// 4) have half of their tiles in either half of the head: tile n < NT / 2 and tile n + NT / 2 meet in a lane.
+// The row of W behind row rho of region h:
+template <typename T>
+__device__ __forceinline__ int head_row(int h, int rho) {
+  constexpr int SHARE = 8 / T::NT > 0 ? 8 / T::NT : 1, RUN = 16 * (T::NT / 2);
+  const int wave = rho / RUN;
+  return wave / SHARE * HEAD + h * (HEAD / 2) + wave % SHARE * RUN + rho % RUN;
+}
+
+// The sums of a tile of OUT_HEADS: bias, rotation, queries out, keys and values into their pages, each rounded once.  What this saves is
+// the float32 product's way to memory and back and a launch: 2,048 rows x 4,608 x 3,584 70 us, the library's product and the rotation's
+// kernel 62 + 20 (with one chain of sums for each output both, the same bits), 4,096 rows 135 for 162.
+template <typename T>
+__device__ __forceinline__ void store_heads(const T& t, const TileArgs& p, int n0, int m0) {
+  constexpr int SHARE = 8 / T::NT > 0 ? 8 / T::NT : 1, RUN = 16 * (T::NT / 2);
+  const int head = n0 / HEAD + t.wn / SHARE, kind = head < p.nq ? 0 : head < p.nq + p.nkv ? 1 : 2;      // the same for a wave
+  if (head * HEAD >= p.N) return;
+  const int f0 = t.wn % SHARE * RUN + 4 * t.g;      // and f0 + 16 n, of the lane's sums
+  float4 b[T::NT];
+#pragma unroll
+  for (int n = 0; n < T::NT; ++n)
+    b[n] = p.bias ? *reinterpret_cast<const float4*>(p.bias + head * HEAD + f0 + n % (T::NT / 2) * 16 + n / (T::NT / 2) * (HEAD / 2))
+                  : float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int m = 0; m < T::MT; ++m) {
+    const int gm = m0 + (t.wm * T::MT + m) * 16 + t.r;
+    if (gm >= p.M) continue;
+    bf16_t* to = reinterpret_cast<bf16_t*>(p.out) + ((size_t)gm * p.nq + head) * HEAD;
+    int apart = 1;       // from a channel to the next
+    if (kind) {
+      const int s = p.slot[gm];
+      if (s < 0) continue;
+      const int page = s / p.ps, place = s - page * p.ps;
+      const size_t of = (size_t)page * p.nkv + (head - p.nq - (kind == 2 ? p.nkv : 0));
+      to = kind == 1 ? p.kc + (of * p.ps + place) * HEAD : p.vc + of * HEAD * p.ps + place;
+      if (kind == 2) apart = p.ps;
+    }
+#pragma unroll
+    for (int n = 0; n < T::NT / 2; ++n) {
+      const int f = f0 + 16 * n;
+      const tp_f32x4 s1 = t.acc[n][m], s2 = t.acc[n + T::NT / 2][m];
+      const float4 b1 = b[n], b2 = b[n + T::NT / 2];
+      const float x1[4] = {s1[0] + b1.x, s1[1] + b1.y, s1[2] + b1.z, s1[3] + b1.w};
+      const float x2[4] = {s2[0] + b2.x, s2[1] + b2.y, s2[2] + b2.z, s2[3] + b2.w};
+      if (kind == 2) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          to[(size_t)(f + i) * apart] = f32_to_bf16(x1[i]);
+          to[(size_t)(f + i + HEAD / 2) * apart] = f32_to_bf16(x2[i]);
+        }
+        continue;
+      }
+      const float4 c01 = p.cs[(size_t)gm * (HEAD / 4) + f / 2], c23 = p.cs[(size_t)gm * (HEAD / 4) + f / 2 + 1];     // (c0, s0, c1, s1)
+      const float c[4] = {c01.x, c01.z, c23.x, c23.z}, sn[4] = {c01.y, c01.w, c23.y, c23.w};
+      float lo[4], hi[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        lo[i] = x1[i] * c[i] - x2[i] * sn[i];
+        hi[i] = x2[i] * c[i] + x1[i] * sn[i];
+      }
+      store4(to + f, lo, 4, true);
+      store4(to + f + HEAD / 2, hi, 4, true);
+    }
+  }
+}
+
 template <typename T, int OUT>
 __global__ __launch_bounds__(512) void gemm_tile_kernel(TileArgs p) {
   __shared__ __attribute__((aligned(16))) char lds[T::LDS];
@@ -84,7 +159,7 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(TileArgs p) {
           const int n = n0 + rho < p.rows ? rho : 0;
           return (uint32_t)(((size_t)n + (h ? p.rows : 0)) * p.ldw * 2);
         }
-        const int n = T::w_row(h, rho);
+        const int n = OUT == OUT_HEADS ? head_row<T>(h, rho) : T::w_row(h, rho);
         return (uint32_t)((size_t)(n0 + n < p.N ? n : 0) * p.ldw * 2);
       },
       [&](int h, int rho) {
@@ -93,6 +168,10 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(TileArgs p) {
       });
   t.multiply(lds, w, x, s1 - s0, p.K % 64 != 0 && s1 == steps_all);
   // a lane holds, of tile (n, m): X's row 16 m + r, W's rows 16 n + 4 g ... + 3
+  if constexpr (OUT == OUT_HEADS) {
+    store_heads(t, p, n0, m0);
+    return;
+  }
 #pragma unroll
   for (int m = 0; m < T::MT; ++m) {
     const int gm = m0 + (t.wm * T::MT + m) * 16 + t.r;
@@ -164,12 +243,13 @@ static const TileShape SHAPES[SHAPES_N] = {{256, 256, 1, 0.967, 1.361}, {128, 25
                                            {192, 256, 1, 0.784, 1.089}, {192, 320, 1, 0.992, 1.362}, {128, 320, 1, 0.758, 0.985},
                                            {256, 192, 1, 0.888, 1.129}};
 
-static int shape_for(int M, int N, int K, int splits, int cus) {
+static int shape_for(int M, int N, int K, int splits, int cus, unsigned may = ~0u) {      // may: a bit for each shape
   int best = 0;
   double least = 1e30;
   const int steps = (K + 63) / 64;
   const double memory = 3.0 + (double)N * K * 2.0 / 7.52e6;
   for (int i = 0; i < SHAPES_N; ++i) {
+    if (!(may >> i & 1)) continue;
     const TileShape& s = SHAPES[i];
     const long long blocks = (long long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn) * splits, room = (long long)cus * s.a_unit;
     const long long whole = blocks / room;
@@ -282,6 +362,49 @@ extern "C" int qvl_gemm_tile(const void* x, long long ldx, const void* w, long l
   else if (mode == 2) SHAPE(OUT_GROUPED);
   else SHAPE(OUT_HALVES);
 #undef SHAPE
+#undef GO
+  return qvl_launch_status();
+}
+
+// Shapes whose waves hold both halves of a head (8 or 4 tiles of W's rows).
+#define HEAD_SHAPES ((1u << 0) | (1u << 1) | (1u << 2) | (1u << 3) | (1u << 5) | (1u << 8) | (1u << 9))
+
+// The stacked projection of nq query, nkv key and nkv value heads of 128 channels with what follows it in the kernel: q_out bfloat16
+// [M, nq, 128] rotated; rotated keys and values into the page slots of their tokens, kc [page][nkv][ps][128], vc [page][nkv][128][ps]
+// (slot[m] = page * ps + place, or -1: not written).  bias: float32 [(nq + 2 nkv) 128] or null; cs: float32 [M, 64, 2].  x, w, tile
+// as in qvl_gemm_tile; everything on 16-byte boundaries.
+extern "C" int qvl_gemm_tile_heads(const void* x, long long ldx, const void* w, long long ldw, const void* bias, const void* cs,
+                                   const void* slot, void* q_out, void* kc, void* vc, int M, int K, int nq, int nkv, int ps, int tile,
+                                   int cus, hipStream_t stream) {
+  if (M <= 0) return QVL_OK;
+  if (nq <= 0 || nkv < 0 || nq > 0xffff || nkv > 0xffff || (nkv && (ps <= 0 || !slot || !kc || !vc))) return QVL_ERR_SHAPE;
+  const int N = (nq + 2 * nkv) * HEAD;
+  if (K <= 0 || K % 32 || ldx < K || ldw < K || ldx % 8 || ldw % 8 || !x || !w || !cs || !q_out || cus <= 0 ||
+      (((uintptr_t)x | (uintptr_t)w | (uintptr_t)bias | (uintptr_t)cs | (uintptr_t)q_out | (uintptr_t)kc | (uintptr_t)vc) % 16))
+    return QVL_ERR_SHAPE;
+  if (tile >= SHAPES_N || (tile >= 0 && !(HEAD_SHAPES >> tile & 1))) return QVL_ERR_SHAPE;
+  // byte offsets from a tile's first row are 32-bit
+  if (256ull * ldw * 2 >= 0xffff0000ull || 256ull * ldx * 2 >= 0xffff0000ull) return QVL_ERR_LIMIT;
+  TileArgs p;
+  p.x = (const bf16_t*)x; p.ldx = ldx; p.w = (const bf16_t*)w; p.ldw = ldw; p.out = q_out; p.ldo = 0;
+  p.M = M; p.N = N; p.K = K; p.rows = N; p.splits = 1; p.relu2 = p.gelu = 0; p.alpha = p.limit = p.shift = 0.f;
+  p.bias = (const float*)bias; p.cs = (const float4*)cs; p.slot = (const int*)slot; p.kc = (bf16_t*)kc; p.vc = (bf16_t*)vc;
+  p.nq = nq; p.nkv = nkv; p.ps = ps;
+  int shape = tile >= 0 ? tile : shape_for(M, N, K, 1, cus, HEAD_SHAPES);
+  if ((unsigned long long)SHAPES[shape].bm * ldx * 2 >= 0xffff0000ull) shape = 0;
+  p.tiles_m = (M + SHAPES[shape].bm - 1) / SHAPES[shape].bm;
+  p.tiles_n = (N + SHAPES[shape].bn - 1) / SHAPES[shape].bn;
+  const long long all = (long long)p.tiles_m * p.tiles_n;
+  if (all > 0x7ffffff0ll / 8) return QVL_ERR_LIMIT;
+  const dim3 grid((unsigned)((all + 7) / 8 * 8));
+#define GO(WN, WM, NT, MT) hipLaunchKernelGGL((gemm_tile_kernel<Tile<WN, WM, NT, MT>, OUT_HEADS>), grid, dim3(512), 0, stream, p)
+  if (shape == 0) GO(2, 4, 8, 4);
+  else if (shape == 1) GO(2, 4, 4, 4);
+  else if (shape == 2) GO(4, 2, 4, 4);
+  else if (shape == 3) GO(2, 4, 4, 2);
+  else if (shape == 5) GO(2, 4, 4, 3);
+  else if (shape == 8) GO(2, 4, 4, 5);
+  else GO(2, 4, 8, 3);
 #undef GO
   return qvl_launch_status();
 }

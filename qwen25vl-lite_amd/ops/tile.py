@@ -9,7 +9,8 @@ import torch
 
 from .kernels import _check, _fn, _need, _ptr, _stream, compute_units
 
-__all__ = ["MANY_ROWS", "takes_tile", "prefers_tile", "tile_product", "tile_slabs", "tile_swiglu", "tile_gated"]
+__all__ = ["MANY_ROWS", "takes_tile", "prefers_tile", "tile_product", "slab_ranges", "tile_slabs", "prefers_heads", "tile_heads", "tile_swiglu",
+           "tile_gated"]
 
 _c_int, _c_ptr, _c_ll, _c_float = ctypes.c_int, ctypes.c_void_p, ctypes.c_longlong, ctypes.c_float
 _STORE, _SLABS, _GROUPED, _HALVES = range(4)
@@ -69,19 +70,67 @@ def tile_product(x: torch.Tensor, weight: torch.Tensor, out_dtype: torch.dtype =
     return _launch(x, weight, out, out.stride(0), _SLABS if out_dtype == torch.float32 else _STORE, relu2=int(relu2), shape=shape)
 
 
-def tile_slabs(x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:
-    """Float32 slabs ``[splits, M, N]`` over ranges of the inner size, whose sum in order is ``x @ weight.T``; None where the
-    kernel does not take the product or is faster without a cut.  Cutting pays where the tiles alone leave compute units
-    idle: 2,048 x 3,584 x 18,944 has 112 tiles of 256 x 256, two ranges take 204 us and one of 192 x 256 234 (the library 377)."""
+def slab_ranges(x: torch.Tensor, weight: torch.Tensor) -> int:
+    """Ranges of the inner size that :func:`tile_slabs` cuts a product into: 1 where tiles alone are faster, 0 where the kernel does
+    not take the product or has few rows."""
     if x.shape[0] <= MANY_ROWS or not takes_tile(x, weight):
+        return 0
+    return int(_fn("gemm_tile", "qvl_gemm_tile_splits", [_c_int] * 4)(x.shape[0], weight.shape[0], x.shape[1], compute_units(x.device)))
+
+
+def tile_slabs(x: torch.Tensor, weight: torch.Tensor, ranges: Optional[int] = None) -> Optional[torch.Tensor]:
+    """Float32 slabs ``[ranges, M, N]`` over ranges of the inner size, whose sum in order is ``x @ weight.T``; None where the
+    kernel does not take the product or is faster without a cut.  Cutting pays where the tiles alone leave compute units
+    idle: 2,048 x 3,584 x 18,944 has 112 tiles of 256 x 256, two ranges take 204 us and one of 192 x 256 234 (the library 377).
+    ``ranges``: :func:`slab_ranges` of the same, if the caller has it."""
+    if ranges is None:
+        ranges = slab_ranges(x, weight)
+    if ranges <= 1:
         return None
+    m, n = x.shape[0], weight.shape[0]
+    out = torch.empty((ranges, m, n), dtype=torch.float32, device=x.device)
+    return _launch(x, weight, out, n, _SLABS, splits=ranges)
+
+
+def prefers_heads(x: torch.Tensor, weight: torch.Tensor, ranges: int, head_dim: int, rot_half: int, *rest: Optional[torch.Tensor]) -> bool:
+    """Whether the stacked projection goes through :func:`tile_heads`: heads of 128 channels rotated whole, ``rest`` (bias, cache) on
+    16-byte boundaries, and a product that is not cut along the inner size (``ranges``: :func:`slab_ranges`), or into three ranges at most of an inner
+    size up to 2,048.
+
+    Measured, the product (the library's, or slabs) and the rotation's kernel in brackets: 16 + 2 x 2 heads, inner size 2,048, 512 rows 23 us (26, three
+    slabs), 375 rows 23 (23), 256 rows 23 (21, four slabs), 2,048 rows 31 (39); 28 + 2 x 4 heads, 3,584, 512 rows 38 (41), 2,048 rows 70 (82), 4,096 rows 135
+    (162), 375 rows 37 (32, two slabs); 64 + 2 x 8 heads, 8,192, 2,048 rows 303 (326), 512 rows 96 (96, three slabs)."""
+    return ((ranges == 1 or (1 < ranges <= 3 and x.shape[1] <= 2048)) and head_dim == 128 and rot_half == 64
+            and all(t is None or t.data_ptr() % 16 == 0 for t in rest))
+
+
+def tile_heads(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], cs: torch.Tensor, slots: Optional[torch.Tensor],
+               k_cache: Optional[torch.Tensor], v_cache: Optional[torch.Tensor], num_q_heads: int, num_kv_heads: int, page_size: int,
+               shape: int = -1) -> torch.Tensor:
+    """The stacked query | key | value projection with bias, rotation and cache write on the float32 sums: the rotated queries
+    ``[M, nq 128]`` (bfloat16); rotated keys and values are in their page slots.  ``cs``: :func:`kernels.rope_table`.  With ``num_kv_heads == 0`` the
+    weight holds query rows only."""
     m, k = x.shape
-    n = weight.shape[0]
-    splits = int(_fn("gemm_tile", "qvl_gemm_tile_splits", [_c_int] * 4)(m, n, k, compute_units(x.device)))
-    if splits <= 1:
-        return None
-    out = torch.empty((splits, m, n), dtype=torch.float32, device=x.device)
-    return _launch(x, weight, out, n, _SLABS, splits=splits)
+    nq, nkv = int(num_q_heads), int(num_kv_heads)
+    n = (nq + 2 * nkv) * 128
+    _need(takes_tile(x, weight) and weight.shape[0] == n, "the tiled kernel does not take this projection")
+    _need(bias is None or (bias.dtype == torch.float32 and bias.shape == (n,) and bias.is_contiguous() and bias.is_cuda),
+          "bias must be float32 [(nq + 2 nkv) 128]")
+    _need(cs.is_cuda and cs.dtype == torch.float32 and cs.dim() == 3 and cs.shape[0] >= m and tuple(cs.shape[1:]) == (64, 2)
+          and cs.is_contiguous(), "cs must be float32 [M, 64, 2]")
+    if nkv:
+        _need(slots is not None and slots.is_cuda and slots.dtype == torch.int32 and slots.shape == (m,) and slots.is_contiguous(),
+              "slots must be int32 [M]")
+        _need(k_cache is not None and v_cache is not None and k_cache.is_cuda and v_cache.is_cuda
+              and k_cache.dtype == v_cache.dtype == torch.bfloat16 and k_cache.is_contiguous() and v_cache.is_contiguous()
+              and tuple(k_cache.shape[1:]) == (nkv, page_size, 128) and tuple(v_cache.shape[1:]) == (nkv, 128, page_size)
+              and v_cache.shape[0] == k_cache.shape[0], "caches must be bfloat16 [pages, nkv, ps, 128] / [pages, nkv, 128, ps]")
+    q_out = torch.empty((m, nq * 128), dtype=torch.bfloat16, device=x.device)
+    fn = _fn("gemm_tile", "qvl_gemm_tile_heads", [_c_ptr, _c_ll, _c_ptr, _c_ll] + [_c_ptr] * 6 + [_c_int] * 7 + [_c_ptr])
+    _check(fn(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), _ptr(cs), _ptr(slots if nkv else None), _ptr(q_out),
+              _ptr(k_cache if nkv else None), _ptr(v_cache if nkv else None), m, k, nq, nkv, int(page_size), shape,
+              compute_units(x.device), _stream()), "linear (tiles, rotation and cache write)")
+    return q_out
 
 
 def tile_swiglu(x: torch.Tensor, weight: torch.Tensor, act: str = "silu", shape: int = -1) -> torch.Tensor:

@@ -320,6 +320,15 @@ class PagedAttention(Mixer):
         # Projections are written out in float32 (the accumulator, unrounded): bias, rotation and
         # the residual sum then happen in float32 and each stored value is rounded once.
         m, k = x.shape
+        nkv = self.nkv if write else 0
+        many = self.dtype == torch.bfloat16 and isinstance(x, torch.Tensor)
+        ranges = tile.slab_ranges(x, self.w_in) if many else 0
+        if many and self.w_in.shape[0] == (self.nq + 2 * nkv) * self.hd and tile.prefers_heads(
+                x, self.w_in, ranges, self.hd, inv_freq.shape[0], self.b_in, slot.k_cache if write else None,
+                slot.v_cache if write else None):
+            return tile.tile_heads(x, self.w_in, self.b_in, self._rotation_table(step, inv_freq, freq_row, m),
+                                   group.slot_mapping if write else None, slot.k_cache if write else None,
+                                   slot.v_cache if write else None, self.nq, nkv, group.page_size)
         if (_splits(m, self.w_in.shape[0], k) and self.dtype == torch.bfloat16 and isinstance(x, torch.Tensor)
                 and x.dtype == torch.bfloat16 and self.hd % 4 == 0 and inv_freq.shape[0] % 4 == 0
                 and skinny.takes_split(m, k, self.w_in) and x.stride(1) == 1 and x.stride(0) % 8 == 0
@@ -327,16 +336,15 @@ class PagedAttention(Mixer):
             qkv = skinny.split_product(self.w_in, x)   # slabs of partial sums: the rotation's kernel adds them
         else:
             qkv = None
-            if (self.dtype == torch.bfloat16 and isinstance(x, torch.Tensor) and self.hd % 4 == 0
-                    and inv_freq.shape[0] % 4 == 0):
-                qkv = tile.tile_slabs(x, self.w_in)     # likewise, where many rows' tiles leave compute units idle
+            if many and self.hd % 4 == 0 and inv_freq.shape[0] % 4 == 0:
+                qkv = tile.tile_slabs(x, self.w_in, ranges)     # likewise, where many rows' tiles leave compute units idle
             if qkv is None:
                 qkv = linear(x, self.w_in, out_dtype=torch.float32)
         cs = self._rotation_table(step, inv_freq, freq_row, m)
         return kernels.rope_kv_write(
             qkv, self.b_in, step.positions, inv_freq, freq_row,
             group.slot_mapping if write else None, slot.k_cache if write else None, slot.v_cache if write else None,
-            self.nq, self.nkv if write else 0, self.hd, group.page_size, out_dtype=self.dtype, cs=cs)
+            self.nq, nkv, self.hd, group.page_size, out_dtype=self.dtype, cs=cs)
 
     def _rotation_table(self, step, inv_freq, freq_row, n: int, position=None, width: Optional[int] = None) -> torch.Tensor:
         """Cosines and sines of the step's angles: computed once per pass and position encoding,

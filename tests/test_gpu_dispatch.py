@@ -139,6 +139,61 @@ def test_projection_with_rotation_and_cache(k):
             assert bool((kc.transpose(1, 2)[untouched] == 0).all()) and bool((vc.permute(0, 3, 1, 2)[untouched] == 0).all())
 
 
+@pytest.mark.parametrize("shape", [-1, 0, 1, 2, 3, 5, 8, 9])
+@pytest.mark.parametrize("m, k, nq, nkv, ps, bias", [(65, 96, 3, 1, 16, True), (321, 160, 5, 2, 48, True), (129, 64, 4, 0, 16, False),
+                                                     (256, 32, 1, 1, 32, False)])
+def test_projection_of_many_rows_with_rotation_and_cache(m, k, nq, nkv, ps, bias, shape):
+    """Every tile that holds both halves of a head, at rows, heads and inner sizes that leave the last tile and the last step part
+    empty.  Queries, keys and values against 64 bits, tokens without a slot among them; nothing else of the pages is written."""
+    from qwen25vl_lite_amd.ops import kernels, tile
+    hd, n = 128, (nq + 2 * nkv) * 128
+    torch.manual_seed(m + k)
+    x, w = torch.randn(m, k, device="cuda").bfloat16(), (torch.randn(n, k, device="cuda") / math.sqrt(k)).bfloat16()
+    b = torch.randn(n, device="cuda") if bias else None
+    pages = m // ps + 2
+    slots = torch.randperm(pages * ps, device="cuda")[:m].int()
+    slots[1] = slots[m - 1] = -1
+    kc = torch.zeros(pages, max(nkv, 1), ps, hd, dtype=torch.bfloat16, device="cuda")
+    vc = torch.zeros(pages, max(nkv, 1), hd, ps, dtype=torch.bfloat16, device="cuda")
+    positions = torch.randint(0, 900, (1, m), dtype=torch.int32, device="cuda")
+    inv_freq = 1e4 ** (-torch.arange(0, hd, 2, device="cuda").float() / hd)
+    cs = kernels.rope_table(positions, inv_freq, torch.zeros(hd // 2, dtype=torch.int32, device="cuda"), m)
+    q = tile.tile_heads(x, w, b, cs, slots if nkv else None, kc if nkv else None, vc if nkv else None, nq, nkv, ps, shape=shape)
+    want, off = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    if bias:
+        want, off = want + b.double(), off + b.double().abs()
+    want, off = want.view(m, -1, hd), ((k + 1) * 2.0 ** -24 * off).view(m, -1, hd)
+    c, s = cs.double()[:, None, :, 0], cs.double()[:, None, :, 1]
+
+    def turned(t, c, s, sign):
+        return torch.cat([t[..., :64] * c - sign * t[..., 64:] * s, t[..., 64:] * c + t[..., :64] * s], -1)
+    ref, bound = turned(want, c, s, 1.0), turned(off, c.abs(), s.abs(), -1.0)
+    # two products and a sum in float32 each rounded, then bfloat16
+    bound = bound + 2.0 ** -22 * turned(want.abs(), c.abs(), s.abs(), -1.0) + 2.0 ** -8 * ref.abs() + 1e-30
+    assert bool(((q.view(m, nq, hd).double() - ref[:, :nq]).abs() <= bound[:, :nq]).all())
+    if nkv:
+        live = slots >= 0
+        page, at = (slots[live] // ps).long(), (slots[live] % ps).long()
+        assert bool(((kc[page, :, at].double() - ref[live][:, nq:nq + nkv]).abs() <= bound[live][:, nq:nq + nkv]).all())
+        wv, ov = want[live][:, nq + nkv:], off[live][:, nq + nkv:]
+        assert bool(((vc[page, :, :, at].double() - wv).abs() <= ov + 2.0 ** -8 * wv.abs() + 1e-30).all())
+        untouched = torch.ones(pages, ps, dtype=torch.bool, device="cuda")
+        untouched[page, at] = False
+        assert bool((kc.transpose(1, 2)[untouched] == 0).all()) and bool((vc.permute(0, 3, 1, 2)[untouched] == 0).all())
+
+
+def test_which_projections_take_the_rotation_with_them():
+    from qwen25vl_lite_amd.ops import kernels, tile
+    w = torch.empty(4608, 3584, dtype=torch.bfloat16, device="cuda")
+    x = torch.empty(2048, 3584, dtype=torch.bfloat16, device="cuda")
+    assert tile.slab_ranges(x, w) == 1 and tile.prefers_heads(x, w, 1, 128, 64)
+    assert tile.slab_ranges(x[:64], w) == 0 and not tile.prefers_heads(x[:64], w, 0, 128, 64)
+    assert not tile.prefers_heads(x, w, 1, 128, 32) and not tile.prefers_heads(x, w, 1, 64, 32) and not tile.prefers_heads(x, w, 2, 128, 64)
+    assert not tile.prefers_heads(x, w, 1, 128, 64, torch.empty(4609, device="cuda")[1:])
+    if kernels.compute_units("cuda:0") == 256:
+        assert tile.slab_ranges(x[:256], w) == 3
+
+
 def test_projection_in_slabs_up_to_64_rows(monkeypatch):
     """As a large weight's, whose 49 to 64 rows are cut, too."""
     from qwen25vl_lite_amd.parts import attention
