@@ -20,6 +20,7 @@ LIBRARIES = [
     ("gemm_resident", {"RK": 8}),
     ("gemm_tile", {}),
     ("gemm_rows", {}),
+    ("gemm_slice", {}),
     ("peaks", {}),
     ("gated", {}),
     ("moe", {}),

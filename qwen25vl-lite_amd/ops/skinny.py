@@ -18,7 +18,7 @@ from .kernels import _check, _fn, _ptr, _stream, dtype_code
 from .kernels import compute_units as _compute_units
 
 __all__ = ["resident_product", "takes_resident", "qkv_rope_product", "takes_qkv_rope", "RESIDENT_ROWS", "resident_norm_k", "resident_two_tile_k", "folds_norm", "ONE_BLOCK_ROWS", "split_product", "takes_split", "prefers_split", "SPLIT_ROWS",
-           "takes_stack", "stack_product", "STORE", "RESIDUAL", "SWIGLU", "GEGLU", "RELU2", "GATED"]
+           "takes_stack", "stack_product", "takes_slice", "slice_qkv_rope", "STORE", "RESIDUAL", "SWIGLU", "GEGLU", "RELU2", "GATED"]
 
 RESIDENT_ROWS = 64       # up to here the resident kernel runs
 ONE_TILE_ROWS = 16       # the rows of one column tile of the matrix instruction
@@ -211,6 +211,42 @@ def qkv_rope_product(weight: torch.Tensor, cs: torch.Tensor, *, x: Optional[torc
               _ptr(slots if nkv else None), _ptr(q_out), _ptr(k_cache if nkv else None),
               _ptr(v_cache if nkv else None), nq, nkv, hd, int(page_size), _compute_units(src.device), _stream()),
            "linear (resident, rotation and cache write)")
+    return q_out
+
+
+def takes_slice(m: int, k: int, weight: torch.Tensor, head_dim: int, rot_half: int, cache_dtype) -> bool:
+    """Whether :func:`slice_qkv_rope` takes the stacked projection of ``m`` rows: bfloat16, a rotation over the whole head, inner sizes up to
+    4,096 and 32 weight rows a compute unit (csrc/gemm_slice.hip).  There it is the fastest way at every number of rows."""
+    if (weight.dtype != torch.bfloat16 or 2 * rot_half != head_dim or cache_dtype not in (None, torch.bfloat16)
+            or not _rows_aligned(weight, 8) or weight.shape[0] * weight.stride(0) * 2 >= 0x7fffff00):
+        return False
+    return bool(_fn("gemm_slice", "qvl_gemm_slice_takes", [_c_int] * 4)(m, weight.shape[0], k, _compute_units(weight.device)))
+
+
+def slice_qkv_rope(weight: torch.Tensor, cs: torch.Tensor, x: torch.Tensor, bias: Optional[torch.Tensor], slots: Optional[torch.Tensor],
+                   k_cache: Optional[torch.Tensor], v_cache: Optional[torch.Tensor], num_q_heads: int, num_kv_heads: int, head_dim: int,
+                   page_size: int) -> torch.Tensor:
+    """As :func:`qkv_rope_product`, where :func:`takes_slice` says so."""
+    m, k = x.shape
+    nq, nkv, hd = int(num_q_heads), int(num_kv_heads), int(head_dim)
+    if (weight.shape != ((nq + 2 * nkv) * hd, k) or not takes_slice(m, k, weight, hd, cs.shape[1], None) or x.dtype != torch.bfloat16
+            or not _rows_aligned(x, 8) or m * x.stride(0) * 2 >= 0x7fffff00):
+        raise ValueError("the kernel does not take this projection")
+    if bias is not None and (bias.dtype != torch.float32 or not bias.is_contiguous() or bias.shape != (weight.shape[0],)):
+        raise ValueError("bias must be float32 [(nq + 2 nkv) hd]")
+    if cs.dtype != torch.float32 or cs.dim() != 3 or cs.shape[0] < m or tuple(cs.shape[1:]) != (hd // 2, 2) or not cs.is_contiguous():
+        raise ValueError("cs must be float32 [M, hd/2, 2]")
+    if nkv and (slots is None or slots.dtype != torch.int32 or slots.shape != (m,) or not slots.is_contiguous()
+                or k_cache is None or v_cache is None or k_cache.dtype != torch.bfloat16 or v_cache.dtype != torch.bfloat16
+                or not k_cache.is_contiguous() or not v_cache.is_contiguous()
+                or tuple(k_cache.shape[1:]) != (nkv, page_size, hd) or tuple(v_cache.shape[1:]) != (nkv, hd, page_size)
+                or v_cache.shape[0] != k_cache.shape[0]):
+        raise ValueError("slots int32 [M] and bfloat16 caches [pages, nkv, ps, hd] / [pages, nkv, hd, ps] are needed")
+    q_out = torch.empty((m, nq * hd), dtype=torch.bfloat16, device=x.device)
+    fn = _fn("gemm_slice", "qvl_gemm_slice_rope", [_c_ptr, _c_int, _c_ptr, _c_int] + [_c_ptr] * 6 + [_c_int] * 7 + [_c_ptr])
+    _check(fn(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), _ptr(cs), _ptr(slots if nkv else None), _ptr(q_out),
+              _ptr(k_cache if nkv else None), _ptr(v_cache if nkv else None), m, k, nq, nkv, hd, int(page_size),
+              _compute_units(x.device), _stream()), "linear (slices, rotation and cache write)")
     return q_out
 
 

@@ -18,18 +18,21 @@ from ..ops.linear import NormedRows, linear, linear_into
 from .base import (CacheNeed, LayerSlot, Mixer, ParamSpec, PartSpec, StateNeed, StepContext, build_part,
                    register_part)
 
-# 17 to 64 rows: where the fused kernel does not run, the projection is cut along its inner size (slabs) and the rotation's
+# 17 to 64 rows that neither csrc/gemm_slice.hip takes (an inner size beyond 4,096, or more than 32 weight rows a compute unit) nor the fused kernel:
+# the projection is cut along its inner size (slabs) and the rotation's
 # kernel adds them (10,240 x 8,192, 19 rows: 32 us, the library's product uncut 41): up to 48 rows at any size, up to 64 where the inner size is
 # beyond LONG_K, which the fused kernel does not take with as many rows, and the weight has LARGE_WEIGHT values or more (49 rows, with the
 # library's product and in slabs: 512 x 4,608 12 us and 17, 7,168 x 5,120 23 and 27, 5,120 x 8,192 31 and 27, 10,240 x 6,144 46 and 36, 10,240 x 8,192
-# 49 and 40, 14,336 x 12,288 88 and 74, 18,432 x 16,384 176 and 164).  From 33 to 48 rows that also beats the fused kernel on teams of blocks (7B
-# sizes: a step of 33 rows 4.14 ms against 4.24, of 48 rows 4.34 against 4.39); from 49 on it does not (7B sizes, K = 3,584, 8 layers, 64 rows
-# 11,160 and 11,124; 3B sizes, K = 2,048, 6 steps at 256 keys 4,922 and 4,820).
+# 49 and 40, 14,336 x 12,288 88 and 74, 18,432 x 16,384 176 and 164).
 SPLIT_ROWS = (17, 64)
 SHORT_SPLIT_ROWS = 48
 LONG_K = 4096
 LARGE_WEIGHT = 40 << 20
 FUSED_ROWS = 32
+# A first layer's rows, still to be normed: up to here, and an inner size up to 2,048, the fused kernel forms the norm by itself (1 row of 2,560 x
+# 2,048 9.5 us for a norm kernel of 4.6 and 5.5; with more of either it takes longer: 8 rows of 4,608 x 3,584 17.9 for 4.8 and 9.8, 24 rows of
+# 2,560 x 2,048 18.1 for 4.6 and 6.7)
+LAZY_ROWS = 8
 
 
 def _splits(m: int, n: int, k: int) -> bool:
@@ -362,6 +365,14 @@ class PagedAttention(Mixer):
         kernel (the float32 sums never leave it)."""
         lazy = isinstance(x, NormedRows)
         m, k = x.shape
+        if self.dtype == torch.bfloat16 and m <= skinny.RESIDENT_ROWS and (not lazy or m > LAZY_ROWS or k > skinny.NARROW_K) and skinny.takes_slice(
+                m, k, self.w_in, self.hd, inv_freq.shape[0], slot.k_cache.dtype if write else None):
+            rows = x.materialize() if lazy else x
+            if rows.dtype == torch.bfloat16 and rows.stride(1) == 1 and rows.stride(0) % 8 == 0 and rows.data_ptr() % 16 == 0:
+                return skinny.slice_qkv_rope(
+                    self.w_in, self._rotation_table(step, inv_freq, freq_row, m), rows, self.b_in, group.slot_mapping if write else None,
+                    slot.k_cache if write else None, slot.v_cache if write else None, self.nq, self.nkv if write else 0, self.hd,
+                    group.page_size)
         if not lazy and m > FUSED_ROWS and _splits(m, self.w_in.shape[0], k):
             return None
         if self.dtype != torch.bfloat16 or not skinny.takes_qkv_rope(

@@ -139,26 +139,24 @@ def test_projection_with_rotation_and_cache(k):
             assert bool((kc.transpose(1, 2)[untouched] == 0).all()) and bool((vc.permute(0, 3, 1, 2)[untouched] == 0).all())
 
 
-@pytest.mark.parametrize("shape", [-1, 0, 1, 2, 3, 5, 8, 9])
-@pytest.mark.parametrize("m, k, nq, nkv, ps, bias", [(65, 96, 3, 1, 16, True), (321, 160, 5, 2, 48, True), (129, 64, 4, 0, 16, False),
-                                                     (256, 32, 1, 1, 32, False)])
-def test_projection_of_many_rows_with_rotation_and_cache(m, k, nq, nkv, ps, bias, shape):
-    """Every tile that holds both halves of a head, at rows, heads and inner sizes that leave the last tile and the last step part
-    empty.  Queries, keys and values against 64 bits, tokens without a slot among them; nothing else of the pages is written."""
-    from qwen25vl_lite_amd.ops import kernels, tile
-    hd, n = 128, (nq + 2 * nkv) * 128
+def _stacked_projection(m, k, nq, nkv, hd, ps, bias, call):
+    """``call(x, w, bias, cs, slots, k cache, v cache)`` returns the rotated queries: these, keys and values against 64 bits, tokens without a
+    slot among them; nothing else of the pages is written."""
+    from qwen25vl_lite_amd.ops import kernels
+    n, half = (nq + 2 * nkv) * hd, hd // 2
     torch.manual_seed(m + k)
     x, w = torch.randn(m, k, device="cuda").bfloat16(), (torch.randn(n, k, device="cuda") / math.sqrt(k)).bfloat16()
     b = torch.randn(n, device="cuda") if bias else None
     pages = m // ps + 2
     slots = torch.randperm(pages * ps, device="cuda")[:m].int()
-    slots[1] = slots[m - 1] = -1
+    if m > 2:
+        slots[1] = slots[m - 1] = -1
     kc = torch.zeros(pages, max(nkv, 1), ps, hd, dtype=torch.bfloat16, device="cuda")
     vc = torch.zeros(pages, max(nkv, 1), hd, ps, dtype=torch.bfloat16, device="cuda")
     positions = torch.randint(0, 900, (1, m), dtype=torch.int32, device="cuda")
     inv_freq = 1e4 ** (-torch.arange(0, hd, 2, device="cuda").float() / hd)
-    cs = kernels.rope_table(positions, inv_freq, torch.zeros(hd // 2, dtype=torch.int32, device="cuda"), m)
-    q = tile.tile_heads(x, w, b, cs, slots if nkv else None, kc if nkv else None, vc if nkv else None, nq, nkv, ps, shape=shape)
+    cs = kernels.rope_table(positions, inv_freq, torch.zeros(half, dtype=torch.int32, device="cuda"), m)
+    q = call(x, w, b, cs, *((slots, kc, vc) if nkv else (None, None, None)))
     want, off = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
     if bias:
         want, off = want + b.double(), off + b.double().abs()
@@ -166,20 +164,43 @@ def test_projection_of_many_rows_with_rotation_and_cache(m, k, nq, nkv, ps, bias
     c, s = cs.double()[:, None, :, 0], cs.double()[:, None, :, 1]
 
     def turned(t, c, s, sign):
-        return torch.cat([t[..., :64] * c - sign * t[..., 64:] * s, t[..., 64:] * c + t[..., :64] * s], -1)
+        return torch.cat([t[..., :half] * c - sign * t[..., half:] * s, t[..., half:] * c + t[..., :half] * s], -1)
     ref, bound = turned(want, c, s, 1.0), turned(off, c.abs(), s.abs(), -1.0)
     # two products and a sum in float32 each rounded, then bfloat16
     bound = bound + 2.0 ** -22 * turned(want.abs(), c.abs(), s.abs(), -1.0) + 2.0 ** -8 * ref.abs() + 1e-30
-    assert bool(((q.view(m, nq, hd).double() - ref[:, :nq]).abs() <= bound[:, :nq]).all())
+    assert bool(((q.view(m, nq, hd).double() - ref[:, :nq]).abs() <= bound[:, :nq]).all()), m
     if nkv:
         live = slots >= 0
         page, at = (slots[live] // ps).long(), (slots[live] % ps).long()
-        assert bool(((kc[page, :, at].double() - ref[live][:, nq:nq + nkv]).abs() <= bound[live][:, nq:nq + nkv]).all())
+        assert bool(((kc[page, :, at].double() - ref[live][:, nq:nq + nkv]).abs() <= bound[live][:, nq:nq + nkv]).all()), m
         wv, ov = want[live][:, nq + nkv:], off[live][:, nq + nkv:]
-        assert bool(((vc[page, :, :, at].double() - wv).abs() <= ov + 2.0 ** -8 * wv.abs() + 1e-30).all())
+        assert bool(((vc[page, :, :, at].double() - wv).abs() <= ov + 2.0 ** -8 * wv.abs() + 1e-30).all()), m
         untouched = torch.ones(pages, ps, dtype=torch.bool, device="cuda")
         untouched[page, at] = False
         assert bool((kc.transpose(1, 2)[untouched] == 0).all()) and bool((vc.permute(0, 3, 1, 2)[untouched] == 0).all())
+
+
+@pytest.mark.parametrize("shape", [-1, 0, 1, 2, 3, 5, 8, 9])
+@pytest.mark.parametrize("m, k, nq, nkv, ps, bias", [(65, 96, 3, 1, 16, True), (321, 160, 5, 2, 48, True), (129, 64, 4, 0, 16, False),
+                                                     (256, 32, 1, 1, 32, False)])
+def test_projection_of_many_rows_with_rotation_and_cache(m, k, nq, nkv, ps, bias, shape):
+    """Every tile that holds both halves of a head, at rows, heads and inner sizes that leave the last tile and the last step part empty."""
+    from qwen25vl_lite_amd.ops import tile
+    _stacked_projection(m, k, nq, nkv, 128, ps, bias,
+                        lambda x, w, b, cs, slots, kc, vc: tile.tile_heads(x, w, b, cs, slots, kc, vc, nq, nkv, ps, shape=shape))
+
+
+@pytest.mark.parametrize("k, nq, nkv, hd, ps, bias", [(8, 3, 1, 10, 16, True), (2056, 5, 2, 48, 48, False), (3584, 28, 4, 128, 16, True),
+                                                      (4096, 50, 7, 128, 32, True), (72, 64, 0, 128, 16, False), (3320, 1, 1, 2, 16, True)])
+def test_projection_of_few_rows_in_slices(k, nq, nkv, hd, ps, bias):
+    """Inner sizes that leave waves without any of it, one pair of channels a block and sixteen, rows on both sides of the column tiles."""
+    from qwen25vl_lite_amd.ops import skinny
+    for m in (1, 7, 8, 9, 16, 17, 32, 33, 48, 49, 64):
+        _stacked_projection(m, k, nq, nkv, hd, ps, bias,
+                            lambda x, w, b, cs, slots, kc, vc: skinny.slice_qkv_rope(w, cs, x, b, slots, kc, vc, nq, nkv, hd, ps))
+    w = torch.empty(128, 4104, dtype=torch.bfloat16, device="cuda")
+    assert not skinny.takes_slice(8, 4104, w, 32, 16, None) and not skinny.takes_slice(65, 4096, w[:, :4096], 32, 16, None)
+    assert not skinny.takes_slice(8, 4096, w[:, :4096], 32, 8, None) and skinny.takes_slice(8, 4096, w[:, :4096], 32, 16, None)
 
 
 def test_which_projections_take_the_rotation_with_them():
