@@ -309,3 +309,35 @@ def test_random_lifetimes_lose_nothing(seed):
     if cm.prefix_cache is not None:
         cm.prefix_cache.evict(10 ** 9)
     assert cm.pages_in_use() == [0, 0]
+
+
+def test_a_steps_single_tokens_are_laid_out_as_runs_are():
+    """Decoded tokens beside a portion, by the way of single tokens and by the general one (tokens that are not plain integers)."""
+    import numpy as np
+    import torch
+    from qwen25vl_lite_amd.engine.batch import StepEntry, build_step
+    cm = CacheManager([CacheGroupSpec(CacheNeed(1, 8), 1), CacheGroupSpec(CacheNeed(1, 8, 20), 1)], 64, 16, 8, enable_prefix_cache=False)
+    for r, n in enumerate((0, 31, 32, 5)):
+        cm.admit(r)
+        cm.reserve(r, n + 40)
+        cm.commit(r, n)
+
+    def step(kind, want=(0,), token=7, vocab=100):
+        entries = [StepEntry(r, [kind(token)], n, want, rope_delta=d) for r, n, d in ((1, 31, 0), (2, 32, -3), (3, 5, 9))]
+        entries.insert(1, StepEntry(0, list(range(37)), 0, [2, 36]))
+        return build_step(entries, cm, 3, torch.float32, torch.device("cpu"), vocab)
+    a, b = step(int), step(np.int64)
+    for name in ("token_ids", "positions", "token_req", "token_seqpos", "cu_q", "ctx_len", "req_slots", "logit_rows"):
+        assert torch.equal(getattr(a, name), getattr(b, name)), name
+    for g in range(2):
+        assert torch.equal(a.groups[g].slot_mapping, b.groups[g].slot_mapping) and torch.equal(a.groups[g].block_table, b.groups[g].block_table)
+        assert a.groups[g].slot_mapping.tolist() == sum((cm.slot_mapping(r, g, s, s + n) for r, s, n in ((1, 31, 1), (0, 0, 37), (2, 32, 1), (3, 5, 1))), [])
+    assert (a.cu_q_host, a.ctx_len_host, a.max_q_len) == (b.cu_q_host, b.ctx_len_host, b.max_q_len)
+    for kind in (int, np.int64):
+        for bad in (dict(want=(1,)), dict(token=100), dict(token=-1)):
+            with pytest.raises(ValueError):
+                step(kind, **bad)
+    cm.requests[2].tables[1][2] = -1
+    for kind in (int, np.int64):
+        with pytest.raises(RuntimeError, match="given back"):
+            step(kind)
