@@ -173,9 +173,9 @@ class LatentAttention(Mixer):
         q = q if q.is_contiguous() else q.contiguous()
         # the query in the latent's space, head by head: [N, heads, kv_rank | rot_dim]
         q_lat = torch.empty((n, h, r + rot), dtype=self.dtype, device=x.device)
-        by_head = step.per_pass.get(("pairs_by_head", h))
+        by_head = step.derived.get(("pairs_by_head", h))      # set by the step's shape alone: a captured step makes them once
         if by_head is None:
-            by_head = step.per_pass[("pairs_by_head", h)] = moe_ops.pairs_by_column(n, h, x.device)
+            by_head = step.derived[("pairs_by_head", h)] = moe_ops.pairs_by_column(n, h, x.device)
         moe_ops.expert_products(q.view(n * h, self.dim + rot)[:, :self.dim], self.w_uk_t, *by_head, n * h, 1, self.dtype,
                                 out=q_lat.view(n * h, r + rot)[:, :r])
         latent.latent_query_rotate_(q, h, self.dim, rot, r, cs, q_lat, interleaved=self.interleaved)

@@ -166,7 +166,9 @@ class LinearAttention(Mixer):
         z = None
         if self.decay_kind == "channel":
             at = self._offset("a1")
-            low = proj[:, at:at + self.rank].contiguous()      # a few columns: copied to rows of their own
+            low = proj[:, at:at + self.rank]                   # a few columns: as they lie where bfloat16 products take them, else copied
+            if low.dtype != torch.bfloat16 or low.stride(0) % 8 or low.data_ptr() % 16:
+                low = low.contiguous()
             z = linear(low, self.w_a2, self.b_a2, out_dtype=torch.float32)
         elif forget:
             at = self._offset("f")
