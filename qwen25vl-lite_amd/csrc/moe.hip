@@ -23,135 +23,214 @@ __device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + expf
 // ---------------------------------------------------------------------------------------
 #define MOE_MAX_E 512
 
-__global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict__ z, int* __restrict__ ids,
-                                                        float* __restrict__ wts, int N, int E, int top, int groups,
-                                                        int keep, float scale, int score_fn, int normalize,
-                                                        float floor_) {
-  __shared__ float s_all[4][MOE_MAX_E];
-  __shared__ float g_all[4][64];
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int n = blockIdx.x * 4 + wave;
-  if (n >= N) return;
-  float* s = s_all[wave];
-  float* gs = g_all[wave];
-  const float* zr = z + (size_t)n * E;
-  if (score_fn == 1) {
-    float mx = -INFINITY;
-    for (int e = lane; e < E; e += 64) mx = fmaxf(mx, zr[e]);
-    mx = wave_max(mx);
-    float sum = 0.f;
-    for (int e = lane; e < E; e += 64) {
-      const float v = expf(zr[e] - mx);
-      s[e] = v;
-      sum += v;
-    }
-    sum = wave_sum(sum);
-    for (int e = lane; e < E; e += 64) s[e] = s[e] / sum;
-  } else {
-    for (int e = lane; e < E; e += 64) s[e] = sigmoid_f(zr[e]);
-  }
-  __builtin_amdgcn_wave_barrier();
-  const int per = E / groups;
-  if (lane < groups) {
-    float a = -INFINITY, b = -INFINITY;   // the two largest
-    for (int i = 0; i < per; ++i) {
-      const float v = s[lane * per + i];
-      if (v > a) { b = a; a = v; }
-      else if (v > b) b = v;
-    }
-    gs[lane] = per > 1 ? a + b : a;
-  }
-  __builtin_amdgcn_wave_barrier();
-  bool allowed_group = false;
-  if (lane < groups) {
-    int ahead = 0;
-    const float mine = gs[lane];
-    for (int g = 0; g < groups; ++g) ahead += (gs[g] > mine || (gs[g] == mine && g < lane)) ? 1 : 0;
-    allowed_group = ahead < keep;
-  }
-  const unsigned long long allowed = __ballot(allowed_group);
-  // this lane's experts: e = lane + 64 i; a score of -1 can never be chosen before an allowed one
-  float cand[MOE_MAX_E / 64];
+struct RouteArgs {
+  const float* z;
+  int* ids;
+  float* wts;
+  int N, E, top, groups, keep, score_fn, normalize;
+  float scale, floor_;
+};
+
+// The largest of a wave's values (no NaN among them) in every lane: within rows of 16 lanes by rotations, across them by swaps.
+__device__ __forceinline__ float largest(float v) {
+  auto turned = [&](auto by) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), 0x120 + decltype(by)::value, 0xf, 0xf, true));
+  };
+  v = fmaxf(v, turned(std::integral_constant<int, 8>{}));
+  v = fmaxf(v, turned(std::integral_constant<int, 4>{}));
+  v = fmaxf(v, turned(std::integral_constant<int, 2>{}));
+  v = fmaxf(v, turned(std::integral_constant<int, 1>{}));
+  const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float((uint32_t)x[0]), __uint_as_float((uint32_t)x[1]));
+  const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float((uint32_t)y[0]), __uint_as_float((uint32_t)y[1]));
+}
+
+// Token n by one wave; s and gs: this wave's MOE_MAX_E and 64 floats of LDS (read where there are groups).  What bounds it is the chain of
+// choices: each takes a maximum over the wave (rotations and swaps of registers; by way of LDS six choices of 32 experts took 4 us
+// more) and one lane's answer, the lowest index where several lanes hold the largest score.
+__device__ __forceinline__ void route_token(const RouteArgs& p, int n, float* s, float* gs) {
+  const int lane = threadIdx.x & 63, E = p.E;
+  const float* zr = p.z + (size_t)n * E;
+  float score[MOE_MAX_E / 64];      // of this lane's experts, e = lane + 64 i
 #pragma unroll
   for (int i = 0; i < MOE_MAX_E / 64; ++i) {
     const int e = lane + 64 * i;
-    cand[i] = (e < E && ((allowed >> (e / per)) & 1ull)) ? s[e] : -1.0f;
+    score[i] = e < E ? zr[e] : -INFINITY;
+  }
+  if (p.score_fn == 1) {
+    float mx = -INFINITY, sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < MOE_MAX_E / 64; ++i)
+      if (64 * i < E) mx = fmaxf(mx, score[i]);
+    mx = largest(mx);
+#pragma unroll
+    for (int i = 0; i < MOE_MAX_E / 64; ++i)
+      if (lane + 64 * i < E) {
+        score[i] = expf(score[i] - mx);
+        sum += score[i];
+      }
+    sum = wave_sum(sum);
+#pragma unroll
+    for (int i = 0; i < MOE_MAX_E / 64; ++i) score[i] = score[i] / sum;
+  } else {
+#pragma unroll
+    for (int i = 0; i < MOE_MAX_E / 64; ++i)
+      if (64 * i < E) score[i] = sigmoid_f(score[i]);
+  }
+  unsigned long long allowed = ~0ull;
+  const int per = E / p.groups;
+  if (p.groups > 1) {
+#pragma unroll
+    for (int i = 0; i < MOE_MAX_E / 64; ++i)
+      if (lane + 64 * i < E) s[lane + 64 * i] = score[i];
+    __builtin_amdgcn_wave_barrier();
+    if (lane < p.groups) {
+      float a = -INFINITY, b = -INFINITY;   // the two largest
+      for (int i = 0; i < per; ++i) {
+        const float v = s[lane * per + i];
+        if (v > a) { b = a; a = v; }
+        else if (v > b) b = v;
+      }
+      gs[lane] = per > 1 ? a + b : a;
+    }
+    __builtin_amdgcn_wave_barrier();
+    bool allowed_group = false;
+    if (lane < p.groups) {
+      int ahead = 0;
+      const float mine = gs[lane];
+      for (int g = 0; g < p.groups; ++g) ahead += (gs[g] > mine || (gs[g] == mine && g < lane)) ? 1 : 0;
+      allowed_group = ahead < p.keep;
+    }
+    allowed = __ballot(allowed_group);
+    __builtin_amdgcn_wave_barrier();      // (the next token's scores go to the same place)
+  }
+  // a score of -1 can never be chosen before an allowed one
+#pragma unroll
+  for (int i = 0; i < MOE_MAX_E / 64; ++i) {
+    const int e = lane + 64 * i;
+    score[i] = (e < E && ((allowed >> (p.groups > 1 ? e / per : 0)) & 1ull)) ? score[i] : -1.0f;
   }
   float total = 0.f;
   float my_w = 0.f;   // lane t keeps the weight of choice t (top <= 64)
   int my_id = 0;
-  for (int t = 0; t < top; ++t) {
-    float best = -2.0f;
+  for (int t = 0; t < p.top; ++t) {
+    float mine = -2.0f;
     int at = 0x7fffffff;
 #pragma unroll
     for (int i = 0; i < MOE_MAX_E / 64; ++i)
-      if (cand[i] > best) { best = cand[i]; at = lane + 64 * i; }
+      if (64 * i < E && score[i] > mine) { mine = score[i]; at = lane + 64 * i; }
     // the wave's best: larger score first, then the lower index
+    const float best = largest(mine);
+    const unsigned long long equal = __ballot(mine == best);
+    if (__popcll(equal) > 1) {
+      if (mine != best) at = 0x7fffffff;
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ob = __shfl_xor(best, o, QVL_WAVE);
-      const int oa = __shfl_xor(at, o, QVL_WAVE);
-      if (ob > best || (ob == best && oa < at)) { best = ob; at = oa; }
+      for (int o = 32; o > 0; o >>= 1) at = min(at, __shfl_xor(at, o, QVL_WAVE));
+    } else {
+      at = __builtin_amdgcn_readlane(at, __ffsll(equal) - 1);
     }
-    if ((at & 63) == lane) {
 #pragma unroll
-      for (int i = 0; i < MOE_MAX_E / 64; ++i)
-        if (at == lane + 64 * i) cand[i] = -3.0f;
-    }
+    for (int i = 0; i < MOE_MAX_E / 64; ++i)
+      if (at == lane + 64 * i) score[i] = -3.0f;
     total += best;
     if (lane == t) { my_w = best; my_id = at; }
   }
-  if (lane < top) {
-    const float w = normalize ? my_w / (total + floor_) : my_w;
-    ids[(size_t)n * top + lane] = my_id;
-    wts[(size_t)n * top + lane] = w * scale;
+  if (lane < p.top) {
+    const float w = p.normalize ? my_w / (total + p.floor_) : my_w;
+    p.ids[(size_t)n * p.top + lane] = my_id;
+    p.wts[(size_t)n * p.top + lane] = w * p.scale;
   }
 }
 
-extern "C" int qvl_moe_route(const void* z, void* ids, void* wts, int N, int E, int top, int groups, int keep,
-                             float scale, int score_fn, int normalize, float floor_, hipStream_t stream) {
-  if (N <= 0) return QVL_OK;
-  if (E <= 0 || top <= 0 || groups <= 0 || keep <= 0 || keep > groups || E % groups || top > keep * (E / groups))
-    return QVL_ERR_SHAPE;
-  if (E > MOE_MAX_E || groups > 64 || top > 64) return QVL_ERR_LIMIT;
-  hipLaunchKernelGGL(moe_route_kernel, dim3((N + 3) / 4), dim3(256), 0, stream, (const float*)z, (int*)ids, (float*)wts, N,
-                     E, top, groups, keep, scale, score_fn, normalize, floor_);
-  return qvl_launch_status();
+__global__ __launch_bounds__(256) void moe_route_kernel(RouteArgs p) {
+  __shared__ float s_all[4][MOE_MAX_E];
+  __shared__ float g_all[4][64];
+  const int wave = threadIdx.x >> 6, n = blockIdx.x * 4 + wave;
+  if (n < p.N) route_token(p, n, s_all[wave], g_all[wave]);
 }
 
 // ---------------------------------------------------------------------------------------
 // Pairs listed by expert: offsets[e] .. offsets[e + 1] of `sorted` hold the pairs that chose expert
-// e (in no fixed order: a pair's row of a product does not depend on its neighbours).  One block.
+// e (in no fixed order: a pair's row of a product does not depend on its neighbours).  One block of 1024 threads.
 // ---------------------------------------------------------------------------------------
+struct SortSpace {
+  int count[MOE_MAX_E], start[MOE_MAX_E + 1];
+};
+__device__ __forceinline__ void sort_block(SortSpace& sh, const int* ids, int* __restrict__ sorted, int* __restrict__ offsets, int P, int E) {
+  for (int e = threadIdx.x; e < E; e += blockDim.x) sh.count[e] = 0;
+  __syncthreads();
+  for (int p = threadIdx.x; p < P; p += blockDim.x) {
+    const int e = ids[p];
+    if (e >= 0 && e < E) atomicAdd(&sh.count[e], 1);
+  }
+  __syncthreads();
+  if (threadIdx.x < 64) {      // the first wave adds up the counts before each expert
+    int before = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + threadIdx.x, mine = e < E ? sh.count[e] : 0;
+      int upto = mine;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(upto, o, QVL_WAVE);
+        if ((int)threadIdx.x >= o) upto += v;
+      }
+      if (e < E) {
+        sh.start[e] = before + upto - mine;
+        sh.count[e] = 0;
+      }
+      before += __shfl(upto, 63, QVL_WAVE);
+    }
+    if (threadIdx.x == 0) sh.start[E] = before;
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e <= E; e += blockDim.x) offsets[e] = sh.start[e];
+  for (int p = threadIdx.x; p < P; p += blockDim.x) {
+    const int e = ids[p];
+    if (e >= 0 && e < E) sorted[sh.start[e] + atomicAdd(&sh.count[e], 1)] = p;
+  }
+}
+
 __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ ids, int* __restrict__ sorted,
                                                         int* __restrict__ offsets, int P, int E) {
-  __shared__ int count[MOE_MAX_E + 1];
-  __shared__ int start[MOE_MAX_E + 1];
-  for (int e = threadIdx.x; e <= E; e += blockDim.x) count[e] = 0;
-  __syncthreads();
-  for (int p = threadIdx.x; p < P; p += blockDim.x) {
-    const int e = ids[p];
-    if (e >= 0 && e < E) atomicAdd(&count[e], 1);
+  __shared__ SortSpace sh;
+  sort_block(sh, ids, sorted, offsets, P, E);
+}
+
+// Both for the few tokens of a decode step, one block: 8 tokens of 32 experts, six of them, 9.9 us and 4.8 in two launches as they were.
+#define ROUTE_SORT_TOKENS 64
+__global__ __launch_bounds__(1024) void moe_route_sort_kernel(RouteArgs p, int* __restrict__ sorted, int* __restrict__ offsets) {
+  __shared__ float s_all[16][MOE_MAX_E];
+  __shared__ float g_all[16][64];
+  __shared__ SortSpace sh;
+  const int wave = threadIdx.x >> 6;
+  for (int n = wave; n < p.N; n += 16) route_token(p, n, s_all[wave], g_all[wave]);
+  __syncthreads();      // (a block's stores are seen by all of it)
+  sort_block(sh, p.ids, sorted, offsets, p.N * p.top, p.E);
+}
+
+static int route_check(const RouteArgs& p) {
+  if (p.E <= 0 || p.top <= 0 || p.groups <= 0 || p.keep <= 0 || p.keep > p.groups || p.E % p.groups || p.top > p.keep * (p.E / p.groups))
+    return QVL_ERR_SHAPE;
+  return p.E > MOE_MAX_E || p.groups > 64 || p.top > 64 ? QVL_ERR_LIMIT : QVL_OK;
+}
+
+// sorted, offsets: null, or also the pairs by expert as qvl_moe_sort gives them.
+extern "C" int qvl_moe_route(const void* z, void* ids, void* wts, void* sorted, void* offsets, int N, int E, int top, int groups, int keep,
+                             float scale, int score_fn, int normalize, float floor_, hipStream_t stream) {
+  if (N <= 0) return QVL_OK;
+  const RouteArgs p{(const float*)z, (int*)ids, (float*)wts, N, E, top, groups, keep, score_fn, normalize, scale, floor_};
+  const int bad = route_check(p);
+  if (bad) return bad;
+  if (sorted && offsets && N <= ROUTE_SORT_TOKENS) {
+    hipLaunchKernelGGL(moe_route_sort_kernel, dim3(1), dim3(1024), 0, stream, p, (int*)sorted, (int*)offsets);
+    return qvl_launch_status();
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int at = 0;
-    for (int e = 0; e < E; ++e) {
-      start[e] = at;
-      at += count[e];
-    }
-    start[E] = at;
-  }
-  __syncthreads();
-  for (int e = threadIdx.x; e <= E; e += blockDim.x) {
-    offsets[e] = start[e];
-    count[e] = 0;
-  }
-  __syncthreads();
-  for (int p = threadIdx.x; p < P; p += blockDim.x) {
-    const int e = ids[p];
-    if (e >= 0 && e < E) sorted[start[e] + atomicAdd(&count[e], 1)] = p;
-  }
+  hipLaunchKernelGGL(moe_route_kernel, dim3((N + 3) / 4), dim3(256), 0, stream, p);
+  if (hipGetLastError() != hipSuccess) return QVL_ERR_LAUNCH;
+  if (sorted && offsets)
+    hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, stream, (const int*)ids, (int*)sorted, (int*)offsets, N * top, E);
+  return qvl_launch_status();
 }
 
 extern "C" int qvl_moe_sort(const void* ids, void* sorted, void* offsets, int P, int E, hipStream_t stream) {

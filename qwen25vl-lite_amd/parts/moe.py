@@ -130,14 +130,16 @@ class RoutedExperts(FeedForward):
 
     def route(self, x: torch.Tensor):
         """``(chosen int32 [N, top], weights float32 [N, top])`` of the rows of ``x``."""
+        return self._route(x, moe_ops.route)
+
+    def _route(self, x: torch.Tensor, how):
         z = linear(x, self.w_router, self.b_router, out_dtype=torch.float32)
-        return moe_ops.route(z if z.is_contiguous() else z.contiguous(), self.top, self.groups, self.keep, self.scale,
-                             self.score, self.normalize, self.floor)
+        return how(z if z.is_contiguous() else z.contiguous(), self.top, self.groups, self.keep, self.scale,
+                   self.score, self.normalize, self.floor)
 
     def forward(self, x, step: StepContext):
         n = x.shape[0]
-        ids, weights = self.route(x)
-        order, offsets = moe_ops.sort_pairs(ids, self.experts)
+        _, weights, order, offsets = self._route(x, moe_ops.route_sorted)
         pairs = n * self.top
         if self.expert_kind == "gated":
             how = dict(gated=(self.alpha, self.limit, self.shift))

@@ -911,6 +911,37 @@ def test_rows_against_many_outputs(m, n, k):
     assert bool(((got - ref).abs() <= slack + (2.0 ** -8 + 1e-6) * ref.abs() + 2e-6).all())
 
 
+@pytest.mark.parametrize("e, top, groups, keep, score", [(1, 1, 1, 1, "softmax"), (32, 6, 1, 1, "softmax"), (64, 8, 1, 1, "sigmoid"),
+                                                         (65, 64, 1, 1, "sigmoid"), (512, 8, 1, 1, "softmax"), (72, 5, 8, 3, "sigmoid")])
+def test_routes_listed_by_expert(e, top, groups, keep, score):
+    """Rows for one wave and for several of a block, and one more than it takes; logits from a few values, so that most choices are
+    among equals and the lower index has to win; the listing holds every pair once, under its expert."""
+    from qwen25vl_lite_amd.ops import moe
+    for n in (1, 16, 17, 64, 65, 200):
+        torch.manual_seed(n)
+        z = torch.randint(0, 5, (n, e), device="cuda").float()
+        ids, wts, order, offsets = moe.route_sorted(z, top, groups, keep, 1.5, score)
+        s = torch.softmax(z.double(), -1) if score == "softmax" else torch.sigmoid(z.double())
+        if groups > 1:
+            members = s.view(n, groups, e // groups)
+            best = members.topk(2, -1).values.sum(-1)
+            rank = (best[:, None, :] > best[:, :, None]).sum(-1) + ((best[:, None, :] == best[:, :, None])
+                                                                      & (torch.arange(groups, device="cuda")[None, None] < torch.arange(groups, device="cuda")[None, :, None])).sum(-1)
+            members = members.masked_fill((rank >= keep)[:, :, None], -1.0)
+            s = members.reshape(n, e)
+        # the lower index first among equals: a stable sort downwards
+        want = torch.sort(s, dim=-1, descending=True, stable=True)
+        assert torch.equal(ids.long(), want.indices[:, :top]), n
+        w = want.values[:, :top]
+        assert torch.allclose(wts.double(), 1.5 * w / w.sum(-1, keepdim=True), rtol=1e-5, atol=0)
+        flat = ids.view(-1).long()
+        assert torch.equal(offsets.long(), torch.cat([torch.zeros(1, device="cuda").long(), torch.bincount(flat, minlength=e).cumsum(0)]))
+        assert torch.equal(order.long().sort().values, torch.arange(n * top, device="cuda"))
+        assert torch.equal(flat[order.long()], flat.sort().values)
+        again = moe.route(z, top, groups, keep, 1.5, score)
+        assert torch.equal(again[0], ids) and torch.equal(again[1], wts)
+
+
 @pytest.mark.parametrize("e, r, k, pairs", [(3, 40, 72, "one"), (8, 300, 200, "uneven"), (70, 129, 64, "uneven"), (4, 2368, 136, "all on one"),
                                             (200, 1, 8, "uneven"), (32, 520, 2056, "few")])
 def test_experts_with_few_pairs(e, r, k, pairs):
