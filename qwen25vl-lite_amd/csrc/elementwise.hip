@@ -6,29 +6,91 @@
 // ---------------------------------------------------------------------------------------
 // Embedding gather: out[n, :] = scale * float32(table[ids[n], :])       (reference text.py:213)
 // ---------------------------------------------------------------------------------------
-template <typename T>
-__global__ void embed_gather_kernel(const int* __restrict__ ids, const T* __restrict__ table,
-                                    float* __restrict__ out, int H, int V, float scale) {
-  const int n = blockIdx.x;
-  int id = ids[n];
-  id = id < 0 ? 0 : (id >= V ? V - 1 : id);  // ids are validated on the host; never read outside the table
-  const T* row = table + (size_t)id * H;
-  float* o = out + (size_t)n * H;
-  for (int i = threadIdx.x; i < H; i += blockDim.x) o[i] = ldf<T>(row + i) * scale;
+// With it the step's tables of cosines and sines (see rope_table_kernel): both need the step's integers alone, and a decode step's launch
+// costs more than either (one row each of 3,584: rows 7.4 us with values one by one and their launch 4.7).
+#define EMBED_TABLES 4
+struct RotationTable {
+  const float* inv_freq;
+  const int* freq_row;
+  float2* out;
+  int rot_half;
+  float amplitude;
+};
+struct EmbedArgs {
+  const int* ids;
+  const void* table;
+  float* out;
+  int H, V;
+  float scale;
+  const int* pos;
+  int pos_stride;
+  RotationTable tables[EMBED_TABLES];
+};
+
+__device__ __forceinline__ void rotation_row(const RotationTable& t, const int* __restrict__ pos, int pos_stride, int n) {
+  for (int f = threadIdx.x; f < t.rot_half; f += blockDim.x) {
+    const int row = t.freq_row[f];
+    float c = 1.f, s = 0.f;
+    if (row >= 0) {
+      sincosf((float)pos[(size_t)row * pos_stride + n] * t.inv_freq[f], &s, &c);
+      c *= t.amplitude;
+      s *= t.amplitude;
+    }
+    t.out[(size_t)n * t.rot_half + f] = float2{c, s};
+  }
 }
 
-extern "C" int qvl_embed_gather(const void* ids, const void* table, void* out, int N, int H, int V, int dtype,
-                                float scale, hipStream_t stream) {
+// grid (N, 1 + tables).  WIDE: 16 bytes of a row at a time (rows and their number of values allow it).
+template <typename T, bool WIDE>
+__global__ __launch_bounds__(256) void embed_kernel(EmbedArgs p) {
+  const int n = blockIdx.x;
+  if (blockIdx.y > 0) {
+    rotation_row(p.tables[blockIdx.y - 1], p.pos, p.pos_stride, n);
+    return;
+  }
+  int id = p.ids[n];
+  id = id < 0 ? 0 : (id >= p.V ? p.V - 1 : id);  // ids are validated on the host; never read outside the table
+  const T* row = reinterpret_cast<const T*>(p.table) + (size_t)id * p.H;
+  float* o = p.out + (size_t)n * p.H;
+  if constexpr (WIDE) {
+    constexpr int E = 16 / sizeof(T);
+    for (int i = threadIdx.x * E; i < p.H; i += 256 * E) {
+      const uint4 v = *reinterpret_cast<const uint4*>(row + i);
+      const T* e = reinterpret_cast<const T*>(&v);
+#pragma unroll
+      for (int k = 0; k < E; k += 4)
+        *reinterpret_cast<float4*>(o + i + k) = float4{ldf<T>(e + k) * p.scale, ldf<T>(e + k + 1) * p.scale, ldf<T>(e + k + 2) * p.scale,
+                                                       ldf<T>(e + k + 3) * p.scale};
+    }
+  } else {
+    for (int i = threadIdx.x; i < p.H; i += 256) o[i] = ldf<T>(row + i) * p.scale;
+  }
+}
+
+// inv_freq, freq_row, rotated, rot_half, amplitude: arrays (on the host) of `tables` at most EMBED_TABLES; pos as in qvl_rope_table.
+extern "C" int qvl_embed_gather(const void* ids, const void* table, void* out, int N, int H, int V, int dtype, float scale,
+                                const void* pos, int pos_stride, int tables, const void* const* inv_freq, const void* const* freq_row,
+                                void* const* rotated, const int* rot_half, const float* amplitude, hipStream_t stream) {
   if (N <= 0) return QVL_OK;
-  if (H <= 0 || V <= 0) return QVL_ERR_SHAPE;
-  if (dtype == 0)
-    hipLaunchKernelGGL(embed_gather_kernel<float>, dim3(N), dim3(256), 0, stream, (const int*)ids,
-                       (const float*)table, (float*)out, H, V, scale);
-  else if (dtype == 1)
-    hipLaunchKernelGGL(embed_gather_kernel<bf16_t>, dim3(N), dim3(256), 0, stream, (const int*)ids,
-                       (const bf16_t*)table, (float*)out, H, V, scale);
-  else
+  if (H <= 0 || V <= 0 || tables < 0 || tables > EMBED_TABLES || (tables && (!pos || pos_stride < N || !inv_freq || !freq_row || !rotated || !rot_half || !amplitude)))
+    return QVL_ERR_SHAPE;
+  EmbedArgs p;
+  p.ids = (const int*)ids; p.table = table; p.out = (float*)out; p.H = H; p.V = V; p.scale = scale; p.pos = (const int*)pos; p.pos_stride = pos_stride;
+  for (int t = 0; t < tables; ++t) {
+    if (rot_half[t] < 0) return QVL_ERR_SHAPE;
+    p.tables[t] = RotationTable{(const float*)inv_freq[t], (const int*)freq_row[t], (float2*)rotated[t], rot_half[t], amplitude[t]};
+  }
+  const dim3 grid(N, 1 + tables);
+  const bool aligned = (((uintptr_t)table | (uintptr_t)out) & 15) == 0;
+  if (dtype == 0) {
+    if (aligned && H % 4 == 0) hipLaunchKernelGGL((embed_kernel<float, true>), grid, dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((embed_kernel<float, false>), grid, dim3(256), 0, stream, p);
+  } else if (dtype == 1) {
+    if (aligned && H % 8 == 0) hipLaunchKernelGGL((embed_kernel<bf16_t, true>), grid, dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((embed_kernel<bf16_t, false>), grid, dim3(256), 0, stream, p);
+  } else {
     return QVL_ERR_DTYPE;
+  }
   return qvl_launch_status();
 }
 
@@ -408,20 +470,8 @@ extern "C" int qvl_rope_kv_write(const void* x, int x_stride, const void* bias, 
 // The rotation's cosines and sines of a step, for kernels that rotate without computing angles:
 // out[n, f] = amplitude * (cos, sin) of pos[freq_row[f], n] * inv_freq[f], or (1, 0) where freq_row[f] < 0.
 // ---------------------------------------------------------------------------------------
-__global__ void rope_table_kernel(const int* __restrict__ pos, int pos_stride, const float* __restrict__ inv_freq,
-                                  const int* __restrict__ freq_row, float2* __restrict__ out, int rot_half,
-                                  float amplitude) {
-  const int n = blockIdx.x;
-  for (int f = threadIdx.x; f < rot_half; f += blockDim.x) {
-    const int row = freq_row[f];
-    float c = 1.f, s = 0.f;
-    if (row >= 0) {
-      sincosf((float)pos[(size_t)row * pos_stride + n] * inv_freq[f], &s, &c);
-      c *= amplitude;
-      s *= amplitude;
-    }
-    out[(size_t)n * rot_half + f] = float2{c, s};
-  }
+__global__ void rope_table_kernel(const int* __restrict__ pos, int pos_stride, RotationTable table) {
+  rotation_row(table, pos, pos_stride, blockIdx.x);
 }
 
 extern "C" int qvl_rope_table(const void* pos, int pos_stride, const void* inv_freq, const void* freq_row, void* out,
@@ -429,7 +479,7 @@ extern "C" int qvl_rope_table(const void* pos, int pos_stride, const void* inv_f
   if (N <= 0 || rot_half <= 0) return QVL_OK;
   if (pos_stride < N) return QVL_ERR_SHAPE;
   hipLaunchKernelGGL(rope_table_kernel, dim3(N), dim3(64), 0, stream, (const int*)pos, pos_stride,
-                     (const float*)inv_freq, (const int*)freq_row, (float2*)out, rot_half, amplitude);
+                     RotationTable{(const float*)inv_freq, (const int*)freq_row, (float2*)out, rot_half, amplitude});
   return qvl_launch_status();
 }
 

@@ -10,7 +10,7 @@ from typing import Dict, List, Optional, Tuple
 import torch
 
 from ..cache.manager import CacheGroupSpec
-from ..parts.base import (Block, CacheNeed, LayerSlot, Mixer, ParamSpec, Part, PartSpec, ResidualStream, StateNeed,
+from ..parts.base import (Block, CacheNeed, LayerSlot, Mixer, ParamSpec, Part, PartSpec, ResidualStream, StateNeed, rotation_key,
                           StepContext, build_part)
 from .spec import ModelSpec
 
@@ -138,6 +138,7 @@ class DecoderModel:
         self.embedding = build_part("embedding", spec.embed or PartSpec("token_table", sizes), dtype, self.device)
         self.head_part = build_part("head", spec.head or PartSpec("linear", sizes), dtype, self.device)
         self._has_weights = False
+        self._rotation_list: Optional[list] = None
         self.pass_vectors: Optional[PassVectors] = None
         if spec.pass_vectors_name is not None:
             if not spec.pass_vectors_name.endswith(".weight") or spec.pass_vectors_rows <= 0:
@@ -304,12 +305,26 @@ class DecoderModel:
         return slots
 
     # ------------------------------------------------------------------ the step
+    def _rotations(self) -> list:
+        """The rotation tables that the mixers of a pass look for, each once."""
+        if self._rotation_list is None:
+            found, parts = {}, list(self.blocks)
+            while parts:
+                part = parts.pop(0)
+                if isinstance(part, Mixer):
+                    for position, width in part.rotations():
+                        found.setdefault(rotation_key(position, width), (position, width))
+                parts.extend(part.sub_parts().values())
+            self._rotation_list = [(key, *what) for key, what in found.items()]
+        return self._rotation_list
+
     def forward(self, step: StepContext, slots: List[LayerSlot]) -> torch.Tensor:
         """Run the step's tokens through the run list; float32 logits ``[M, vocab]`` at
         ``step.logit_rows``."""
         if not self._has_weights:
             raise RuntimeError("the model has no weights yet")
         step.token_side = None if self.token_side is None else self.token_side.weight
+        step.rotations = self._rotations()
         if self.embed_place is not None:
             stream = ResidualStream(self.embedding.forward(step.token_ids, step, slots[len(self.spec.run)]))
         else:

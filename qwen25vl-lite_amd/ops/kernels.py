@@ -106,9 +106,14 @@ def int32_to_device(host, device) -> torch.Tensor:
 
 
 # --------------------------------------------------------------------------------------------
-def embed_gather(ids: torch.Tensor, table: torch.Tensor, out: Optional[torch.Tensor] = None,
-                 scale: float = 1.0) -> torch.Tensor:
-    """``out[n] = scale * float32(table[ids[n]])`` — the residual stream starts in float32."""
+EMBED_TABLES = 4     # as in csrc/elementwise.hip
+
+
+def embed_gather(ids: torch.Tensor, table: torch.Tensor, out: Optional[torch.Tensor] = None, scale: float = 1.0,
+                 positions: Optional[torch.Tensor] = None, rotations: Sequence[Tuple] = ()):
+    """``out[n] = scale * float32(table[ids[n]])`` — the residual stream starts in float32.  With ``rotations``, up to
+    ``EMBED_TABLES`` tuples ``(inv_freq, freq_row, amplitude)``, also each one's :func:`rope_table` of ``positions``, in the same launch:
+    ``(out, [tables])``."""
     _dev(ids, table, out)
     _need(ids.dtype == torch.int32 and ids.dim() == 1 and ids.is_contiguous(), "ids must be contiguous int32 [N]")
     _need(table.dim() == 2 and table.is_contiguous(), "table must be contiguous [V, H]")
@@ -116,10 +121,21 @@ def embed_gather(ids: torch.Tensor, table: torch.Tensor, out: Optional[torch.Ten
     if out is None:
         out = torch.empty((n, h), dtype=torch.float32, device=table.device)
     _need(out.dtype == torch.float32 and out.shape == (n, h) and out.is_contiguous(), "out must be float32 [N, H]")
-    fn = _fn("elementwise", "qvl_embed_gather", [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_float, _c_ptr])
-    _check(fn(_ptr(ids), _ptr(table), _ptr(out), n, h, v, dtype_code(table.dtype), float(scale), _stream()),
-           "embed_gather")
-    return out
+    count = len(rotations)
+    _need(count <= EMBED_TABLES and (count == 0 or positions is not None), f"at most {EMBED_TABLES} rotations, with the positions")
+    made, arrays = [], [None] * 5
+    if count:
+        for inv_freq, freq_row, _ in rotations:
+            _check_rotation(positions, inv_freq, freq_row, n)
+            made.append(torch.empty((n, inv_freq.shape[0], 2), dtype=torch.float32, device=table.device))
+        arrays = [(_c_ptr * count)(*(_ptr(r[0]) for r in rotations)), (_c_ptr * count)(*(_ptr(r[1]) for r in rotations)),
+                  (_c_ptr * count)(*(_ptr(t) for t in made)), (_c_int * count)(*(t.shape[1] for t in made)),
+                  (_c_float * count)(*(float(r[2]) for r in rotations))]
+    fn = _fn("elementwise", "qvl_embed_gather", [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_float, _c_ptr, _c_int, _c_int]
+             + [_c_ptr] * 6)
+    _check(fn(_ptr(ids), _ptr(table), _ptr(out), n, h, v, dtype_code(table.dtype), float(scale), _ptr(positions) if count else None,
+              positions.stride(0) if count else 0, count, *arrays, _stream()), "embed_gather")
+    return (out, made) if count else out
 
 
 def add_rmsnorm(h: torch.Tensor, delta: Optional[torch.Tensor], weight: torch.Tensor, eps: float,
@@ -227,10 +243,7 @@ def rope_kv_write(x: torch.Tensor, bias: Optional[torch.Tensor], positions: torc
     return q_out
 
 
-def rope_table(positions: torch.Tensor, inv_freq: torch.Tensor, freq_row: torch.Tensor, n: int,
-               amplitude: float = 1.0) -> torch.Tensor:
-    """Cosine and sine of every token's rotation angle: float32 ``[n, rot/2, 2]`` with
-    ``amplitude * (cos, sin)(positions[freq_row[f], i] * inv_freq[f])``, or ``(1, 0)`` where ``freq_row[f] < 0``."""
+def _check_rotation(positions: torch.Tensor, inv_freq: torch.Tensor, freq_row: torch.Tensor, n: int) -> None:
     _dev(positions, inv_freq, freq_row)
     rot_half = inv_freq.shape[0]
     _need(inv_freq.dtype == torch.float32 and inv_freq.is_contiguous(), "inv_freq must be float32 [rot/2]")
@@ -238,6 +251,14 @@ def rope_table(positions: torch.Tensor, inv_freq: torch.Tensor, freq_row: torch.
           "freq_row must be int32 [rot/2]")
     _need(positions.dtype == torch.int32 and positions.dim() == 2 and positions.shape[1] >= n
           and positions.stride(1) == 1, "positions must be int32 [rows, N]")
+
+
+def rope_table(positions: torch.Tensor, inv_freq: torch.Tensor, freq_row: torch.Tensor, n: int,
+               amplitude: float = 1.0) -> torch.Tensor:
+    """Cosine and sine of every token's rotation angle: float32 ``[n, rot/2, 2]`` with
+    ``amplitude * (cos, sin)(positions[freq_row[f], i] * inv_freq[f])``, or ``(1, 0)`` where ``freq_row[f] < 0``."""
+    _check_rotation(positions, inv_freq, freq_row, n)
+    rot_half = inv_freq.shape[0]
     out = torch.empty((n, rot_half, 2), dtype=torch.float32, device=positions.device)
     fn = _fn("elementwise", "qvl_rope_table", [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_float, _c_ptr])
     _check(fn(_ptr(positions), positions.stride(0), _ptr(inv_freq), _ptr(freq_row), _ptr(out), int(n), rot_half,

@@ -15,7 +15,7 @@ import torch
 from ..ops import kernels, skinny, tile
 from ..ops.attention import paged_attention
 from ..ops.linear import NormedRows, linear, linear_into
-from .base import (CacheNeed, LayerSlot, Mixer, ParamSpec, PartSpec, StateNeed, StepContext, build_part,
+from .base import (CacheNeed, LayerSlot, Mixer, ParamSpec, PartSpec, StateNeed, StepContext, build_part, rotation_key,
                    register_part)
 
 # 17 to 64 rows that neither csrc/gemm_slice.hip takes (an inner size beyond 4,096, or more than 32 weight rows a compute unit) nor the fused kernel:
@@ -156,6 +156,9 @@ class PagedAttention(Mixer):
         self.b_out: Optional[torch.Tensor] = None
         self.w_conv: Optional[torch.Tensor] = None      # float32 [taps, convolved channels]
         self.sink: Optional[torch.Tensor] = None
+
+    def rotations(self) -> list:
+        return [(self.position, self.hd)] + ([(self.value_position, self.vd)] if self.value_position is not None else [])
 
     def cache_need(self) -> CacheNeed:
         return CacheNeed(self.nkv, self.hd, self.retain, self.keep_first, None if self.vd == self.hd else self.vd, self.chunk)
@@ -353,7 +356,7 @@ class PagedAttention(Mixer):
         """Cosines and sines of the step's angles: computed once per pass and position encoding,
         by the first layer that needs them, and read by every head of every layer."""
         position = self.position if position is None else position
-        key = ("rope_cs", position.table_key(self.hd if width is None else width))
+        key = rotation_key(position, self.hd if width is None else width)
         cs = step.per_pass.get(key)
         if cs is None:
             cs = step.per_pass[key] = kernels.rope_table(step.positions, inv_freq, freq_row, n,

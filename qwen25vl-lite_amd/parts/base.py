@@ -160,6 +160,8 @@ class StepContext:
     max_q_len: int = 0
     max_ctx_len: int = 0
     dtype: torch.dtype = torch.float32
+    # (key, position encoding, head width) of the rotation tables that the pass's mixers will look for
+    rotations: Sequence[Any] = ()
     residual: Optional[torch.Tensor] = None   # set by a block while a part may add its result in place
     # the model's second table of token rows [vocab, columns], where it has one: layers read columns of their own
     token_side: Optional[torch.Tensor] = None
@@ -279,10 +281,20 @@ class Norm(Part):
         raise NotImplementedError
 
 
+def rotation_key(position, width: int):
+    """Where a pass keeps the table of cosines and sines of its positions."""
+    return "rope_cs", position.table_key(width)
+
+
 class Mixer(Part):
     # a mixer that reads several mixes of a token's input with the one's before it names the sub-part that
     # holds their weights (a TokenMixes part): a block may then hand it the mixes instead of the input
     token_mixes: Optional[Part] = None
+
+    def rotations(self) -> list:
+        """``(position encoding, head width)`` of the tables of cosines and sines that :meth:`forward` looks for in
+        ``step.per_pass`` (:func:`rotation_key`)."""
+        return []
 
     def forward(self, x: torch.Tensor, step: StepContext, slot: LayerSlot) -> torch.Tensor:
         raise NotImplementedError

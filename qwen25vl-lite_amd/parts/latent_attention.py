@@ -21,7 +21,7 @@ import torch
 from ..ops import kernels, latent, moe as moe_ops
 from ..ops.attention import paged_attention
 from ..ops.linear import linear, linear_into
-from .base import CacheNeed, LayerSlot, Mixer, ParamSpec, PartSpec, StepContext, build_part, register_part
+from .base import CacheNeed, LayerSlot, Mixer, ParamSpec, PartSpec, StepContext, build_part, register_part, rotation_key
 
 __all__ = ["LatentAttention"]
 
@@ -137,11 +137,14 @@ class LatentAttention(Mixer):
             out[f"{n['sink']}.weight"] = self.sink
         return out
 
+    def rotations(self) -> list:
+        return [] if self.position is None else [(self.position, self.rot_dim)]
+
     def _rotation_table(self, step: StepContext, n: int) -> Optional[torch.Tensor]:
         """Cosines and sines of the step's angles, shared by the layers whose rotations agree."""
         if self.position is None:
             return None
-        key = ("rope_cs", self.position.table_key(self.rot_dim))
+        key = rotation_key(self.position, self.rot_dim)
         cs = step.per_pass.get(key)
         if cs is None:
             inv_freq, freq_row = self.position.rotary_tables(self.rot_dim)

@@ -35,7 +35,15 @@ class TokenTable(Embedding):
         self.table = tensors["weight"]
 
     def forward(self, token_ids, step):
-        return kernels.embed_gather(token_ids, self.table, scale=self.scale)
+        wanted = list(getattr(step, "rotations", ()))[:kernels.EMBED_TABLES]
+        if not wanted:
+            return kernels.embed_gather(token_ids, self.table, scale=self.scale)
+        # the pass's rotation tables come in the same launch
+        rows, tables = kernels.embed_gather(
+            token_ids, self.table, scale=self.scale, positions=step.positions,
+            rotations=[(*position.rotary_tables(width), getattr(position, "amplitude", 1.0)) for _, position, width in wanted])
+        step.per_pass.update((key, table) for (key, _, _), table in zip(wanted, tables))
+        return rows
 
 
 class NormedTokenTable(TokenTable):

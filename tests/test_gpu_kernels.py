@@ -26,6 +26,29 @@ def test_embed_gather(dtype):
     assert out.dtype == torch.float32 and torch.equal(out, table[ids.long()].float())
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width, n", [(3584, 1), (8, 300), (2052, 19), (100, 3), (8192, 2)])
+def test_embed_gather_with_rotation_tables(width, n, dtype):
+    """Rows by 16 bytes and one by one, ids beyond the table's ends, scaled; beside them up to four rotation tables, the bits of a launch of
+    their own."""
+    from qwen25vl_lite_amd.ops import kernels
+    torch.manual_seed(width)
+    table = torch.randn(40, width).to(dtype).cuda()
+    ids = torch.randint(-1, 41, (n,), dtype=torch.int32).cuda()
+    positions = torch.randint(0, 5000, (3, n + 5), dtype=torch.int32).cuda()
+    rotations = [(torch.rand(half).cuda(), torch.randint(-1, 3, (half,), dtype=torch.int32).cuda(), amplitude)
+                 for half, amplitude in ((64, 1.0), (1, 0.5), (300, 1.25), (16, 1.0))]
+    want = table[ids.long().clamp(0, 39)].float() * 1.5
+    assert torch.equal(kernels.embed_gather(ids, table, scale=1.5), want)
+    for count in (1, 3, 4):
+        rows, tables = kernels.embed_gather(ids, table, scale=1.5, positions=positions, rotations=rotations[:count])
+        assert torch.equal(rows, want) and len(tables) == count
+        for got, (inv_freq, freq_row, amplitude) in zip(tables, rotations):
+            assert torch.equal(got, kernels.rope_table(positions, inv_freq, freq_row, n, amplitude=amplitude))
+    with pytest.raises(kernels.KernelError):
+        kernels.embed_gather(ids, table, positions=positions, rotations=rotations + rotations[:1])
+
+
 @pytest.mark.parametrize("width", [97, 3584, 8200])
 @pytest.mark.parametrize("delta_dtype, out_dtype", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16),
                                                     (torch.bfloat16, torch.bfloat16), (None, torch.bfloat16)])
