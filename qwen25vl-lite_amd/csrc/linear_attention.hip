@@ -32,7 +32,6 @@
 #define LA_THREADS (64 * LA_WAVES)
 #define LA_TB (LA_DIM > 256 ? 4 : (LA_DIM > 128 ? 8 : 16))
 
-
 __device__ __forceinline__ float la_act(float z, int act) { return act ? z / (1.0f + expf(-z)) : z; }
 
 // how the decay is given: a constant per head; sigmoid(z)^(1/tau); a floored forget gate whose complement is the key
@@ -44,39 +43,46 @@ __device__ __forceinline__ float la_act(float z, int act) { return act ? z / (1.
 // and the decay is 1 minus it
 __device__ __forceinline__ float la_forget_key(float z, float lower) { return (1.0f - lower) / (1.0f + expf(z)); }
 
-// log(sigmoid(z)) = min(z, 0) - log1p(exp(-|z|))
-__device__ __forceinline__ float la_decay(float z, float inv_tau) {
-  return expf((fminf(z, 0.f) - log1pf(expf(-fabsf(z)))) * inv_tau);
-}
+// log(sigmoid(z)) = min(z, 0) - log1p(exp(-|z|)); times 1/tau: the decay's logarithm
+__device__ __forceinline__ float la_log_decay(float z, float inv_tau) { return (fminf(z, 0.f) - log1pf(expf(-fabsf(z)))) * inv_tau; }
 
-template <typename TP, int MODE, int G, bool BONUS>
+// COLS: value channels of a lane (64 apart).  What bounds a long run is LDS and the vector unit: every value of q, k and the decays
+// that a wave reads serves 64 channels with one of a lane, 128 with two, and staging is shared likewise (29 chunks of 64 tokens, 28
+// heads: of 64 x 128 with a decay for each channel 117 us and 88, of 128 x 128 with one for each head 159 and 135).  Fewer tokens at a
+// time and a bound on registers, for a fourth block a compute unit: 89 and 146.
+// CHUNK: the runs are chunks of a request's (see below): each starts from zero, its state is row `run` of `state`, and
+// `last` gets the product of its decays.
+template <typename TP, int MODE, int G, bool BONUS, int COLS, bool CHUNK>
 __global__ __launch_bounds__(LA_THREADS) void la_scan_kernel(
     const TP* __restrict__ proj, long long proj_stride, long long q_off, long long k_off, long long v_off,
     const float* __restrict__ head_decay, const float* __restrict__ z, long long z_stride, float inv_tau,
     const float* __restrict__ lower, const float* __restrict__ zbias, const float* __restrict__ bonus,
     float* __restrict__ state, const int* __restrict__ cu_q, const int* __restrict__ req_slots,
-    float* __restrict__ out, long long out_slab, int H, int vdim, int act, float q_scale) {
+    float* __restrict__ out, long long out_slab, float* __restrict__ last, int H, int vdim, int act, float q_scale) {
+  constexpr int TB = COLS > 1 && LA_DIM > 64 ? 8 : LA_TB;      // tokens staged at a time
   // key channels of this block's group (a G that does not divide the rows among the waves is never launched)
   constexpr int DG = LA_DIM % (LA_WAVES * G) == 0 ? LA_DIM / G : LA_DIM;
   constexpr int LA_ROWS = DG / LA_WAVES;    // rows of S a wave keeps
-  __shared__ float qs[LA_TB][DG];
-  __shared__ float ks[LA_TB][DG];
+  __shared__ float qs[TB][DG];
+  __shared__ float ks[TB][DG];
   constexpr bool CHANNEL_DECAY = MODE != LA_HEAD;
-  __shared__ float as[CHANNEL_DECAY ? LA_TB : 1][DG];
-  __shared__ float po[LA_TB][LA_WAVES][64];
+  __shared__ float as[CHANNEL_DECAY ? TB : 1][DG];
+  __shared__ float logs[CHUNK && CHANNEL_DECAY ? TB : 1][CHUNK ? DG : 1], log_sums[CHUNK && CHANNEL_DECAY ? DG : 1];
+  __shared__ float po[TB][LA_WAVES][64 * COLS];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int head = blockIdx.y, req = blockIdx.z;
   const int vtile = blockIdx.x / G, group = blockIdx.x % G;
   const int d0 = group * DG;
-  const int vcol = vtile * 64 + lane;
-  const bool live = vcol < vdim;
+  const int vcol = vtile * 64 * COLS + lane;      // and 64 further on
   const int begin = cu_q[req], end = cu_q[req + 1];
   if (begin >= end) return;
   out += (size_t)group * out_slab;
-  float* srow = state + (((size_t)req_slots[req] * H + head) * LA_DIM + d0 + (size_t)wave * LA_ROWS) * vdim + vcol;
-  float S[LA_ROWS];
+  float* srow = state + (((size_t)(CHUNK ? req : req_slots[req]) * H + head) * LA_DIM + d0 + (size_t)wave * LA_ROWS) * vdim + vcol;
+  float S[COLS][LA_ROWS];
 #pragma unroll
-  for (int i = 0; i < LA_ROWS; ++i) S[i] = live ? srow[(size_t)i * vdim] : 0.f;
+  for (int c = 0; c < COLS; ++c)
+#pragma unroll
+    for (int i = 0; i < LA_ROWS; ++i) S[c][i] = !CHUNK && vcol + 64 * c < vdim ? srow[(size_t)i * vdim + 64 * c] : 0.f;
   const float fixed = CHANNEL_DECAY ? 1.f : head_decay[head];
   float U[BONUS ? LA_ROWS : 1];
   if (BONUS) {
@@ -84,8 +90,10 @@ __global__ __launch_bounds__(LA_THREADS) void la_scan_kernel(
     for (int i = 0; i < LA_ROWS; ++i) U[BONUS ? i : 0] = bonus[head * LA_DIM + d0 + wave * LA_ROWS + i];
   }
 
-  for (int t0 = begin; t0 < end; t0 += LA_TB) {
-    const int nt = end - t0 < LA_TB ? end - t0 : LA_TB;
+  if (CHUNK && CHANNEL_DECAY && vtile == 0)      // (a channel's sum is one thread's all the way)
+    for (int d = tid; d < DG; d += LA_THREADS) log_sums[d] = 0.f;
+  for (int t0 = begin; t0 < end; t0 += TB) {
+    const int nt = end - t0 < TB ? end - t0 : TB;
     for (int idx = tid; idx < nt * DG; idx += LA_THREADS) {
       const int t = idx / DG, d = idx % DG;
       const TP* row = proj + (size_t)(t0 + t) * proj_stride + (size_t)head * LA_DIM + d0 + d;
@@ -96,47 +104,62 @@ __global__ __launch_bounds__(LA_THREADS) void la_scan_kernel(
         const float key = la_forget_key(zz, lower[hd]);
         ks[t][d] = key;
         as[t][d] = 1.0f - key;
+        if (CHUNK) logs[t][d] = log1pf(-key);
       } else {
         ks[t][d] = la_act(ldf<TP>(row + k_off), act & 2);
-        if (MODE == LA_CHANNEL)
-          as[t][d] = la_decay(z[(size_t)(t0 + t) * z_stride + (size_t)head * LA_DIM + d0 + d], inv_tau);
-        if (MODE == LA_EXP) {
+        if (MODE == LA_CHANNEL || MODE == LA_EXP) {
           const int hd = head * LA_DIM + d0 + d;
-          as[t][d] = expf(-expf(z[(size_t)(t0 + t) * z_stride + hd] + (zbias ? zbias[hd] : 0.f)));
+          const float zz = z[(size_t)(t0 + t) * z_stride + hd];
+          const float lg = MODE == LA_EXP ? -expf(zz + (zbias ? zbias[hd] : 0.f)) : la_log_decay(zz, inv_tau);
+          as[t][d] = expf(lg);
+          if (CHUNK) logs[t][d] = lg;
         }
       }
     }
-    float vt[LA_TB];
+    float vt[TB][COLS];
 #pragma unroll
-    for (int t = 0; t < LA_TB; ++t)
-      vt[t] = (live && t < nt)
-                  ? la_act(ldf<TP>(proj + (size_t)(t0 + t) * proj_stride + v_off + (size_t)head * vdim + vcol), act & 4)
-                  : 0.f;
+    for (int t = 0; t < TB; ++t)
+#pragma unroll
+      for (int c = 0; c < COLS; ++c)
+        vt[t][c] = (vcol + 64 * c < vdim && t < nt)
+                       ? la_act(ldf<TP>(proj + (size_t)(t0 + t) * proj_stride + v_off + (size_t)head * vdim + vcol + 64 * c), act & 4)
+                       : 0.f;
     __syncthreads();
+    if (CHUNK && CHANNEL_DECAY && vtile == 0)
+      for (int d = tid; d < DG; d += LA_THREADS) {
+        float sum = log_sums[d];
+        for (int t = 0; t < nt; ++t) sum += logs[t][d];
+        log_sums[d] = sum;
+      }
 #pragma unroll
-    for (int t = 0; t < LA_TB; ++t) {
+    for (int t = 0; t < TB; ++t) {
       if (t < nt) {
-        float acc = 0.f;
+        float acc[COLS] = {};
 #pragma unroll
         for (int i = 0; i < LA_ROWS; ++i) {
           const int d = wave * LA_ROWS + i;
-          const float a = CHANNEL_DECAY ? as[t][d] : fixed;
-          if (BONUS) {
-            const float kv = ks[t][d] * vt[t];
-            acc += (S[i] + U[BONUS ? i : 0] * kv) * qs[t][d];
-            S[i] = a * S[i] + kv;
-          } else {
-            S[i] = a * S[i] + ks[t][d] * vt[t];
-            acc += S[i] * qs[t][d];
+          const float a = CHANNEL_DECAY ? as[t][d] : fixed, k = ks[t][d], q = qs[t][d];
+#pragma unroll
+          for (int c = 0; c < COLS; ++c) {
+            float& St = S[c][i];
+            if (BONUS) {
+              const float kv = k * vt[t][c];
+              acc[c] += (St + U[BONUS ? i : 0] * kv) * q;
+              St = a * St + kv;
+            } else {
+              St = a * St + k * vt[t][c];
+              acc[c] += St * q;
+            }
           }
         }
-        po[t][wave][lane] = acc;
+#pragma unroll
+        for (int c = 0; c < COLS; ++c) po[t][wave][64 * c + lane] = acc[c];
       }
     }
     __syncthreads();
-    for (int idx = tid; idx < nt * 64; idx += LA_THREADS) {
-      const int t = idx >> 6, l = idx & 63;
-      const int c = vtile * 64 + l;
+    for (int idx = tid; idx < nt * 64 * COLS; idx += LA_THREADS) {
+      const int t = idx / (64 * COLS), l = idx % (64 * COLS);
+      const int c = vtile * 64 * COLS + l;
       if (c < vdim) {
         float sum = po[t][0][l];
 #pragma unroll
@@ -146,10 +169,15 @@ __global__ __launch_bounds__(LA_THREADS) void la_scan_kernel(
     }
     __syncthreads();
   }
-  if (live) {
+  if (CHUNK && vtile == 0)
+    for (int d = tid; d < DG; d += LA_THREADS)
+      last[((size_t)req * H + head) * LA_DIM + d0 + d] = expf(CHANNEL_DECAY ? log_sums[CHANNEL_DECAY ? d : 0] : logf(fixed) * (float)(end - begin));
 #pragma unroll
-    for (int i = 0; i < LA_ROWS; ++i) srow[(size_t)i * vdim] = S[i];
-  }
+  for (int c = 0; c < COLS; ++c)
+    if (vcol + 64 * c < vdim) {
+#pragma unroll
+      for (int i = 0; i < LA_ROWS; ++i) srow[(size_t)i * vdim + 64 * c] = S[c][i];
+    }
 }
 
 // ---------------------------------------------------------------------------------------
@@ -158,54 +186,140 @@ __global__ __launch_bounds__(LA_THREADS) void la_scan_kernel(
 //   o_t = (scan from a zero state)_t + S'^T (q_t * P_t),      S_end = diag(P_last) S' + U
 // where U is the state the scan from zero ends with; with a bonus, whose outputs are formed before the state moves
 // on, P_(t-1) stands in the first line (1 for the chunk's first token).  The scan above runs every chunk as if it were a
-// request (from zeroed rows of a scratch tensor); the kernels below form q_t * P_t and P_last, carry
-// the state from chunk to chunk, and put the second term, a plain float32 matrix product per (chunk,
-// head) done by the caller, back into token order.
+// request of its own; la_carry_kernel carries the state from chunk to chunk, and la_join_kernel forms q_t * P_t and its product with
+// the state before the chunk, on the float32 matrix instruction.
+//
+// 1,608 tokens of eight requests, 28 heads: of 64 x 128 with a decay for each channel 140 us (scan 88, carry 16, join 36), of 128 x 128
+// with one for each head 206 (135, 29, 40).  With a scan from cleared rows, q_t * P_t and the products through memory, and these put
+// back into token order by a kernel of their own, they were 208 and 263.
 // ---------------------------------------------------------------------------------------
 
-// grid (chunks, H), LA_DIM * LA_PARTS threads: qp [chunks, H, chunk_len, LA_DIM] (rows past the chunk's end
-// stay as they are), last [chunks, H, LA_DIM].  The chunk's tokens are cut into LA_PARTS ranges; a thread
-// sums the logarithms of its channel's decays over its range, learns through LDS what the ranges before
-// it add up to, and walks its range again to write q_t * P_t.
-#define LA_PARTS (LA_DIM <= 64 ? 8 : (LA_DIM <= 128 ? 4 : (LA_DIM <= 256 ? 2 : 1)))
+// grid (chunks, H), 256 threads: rows begin .. end - 1 of `out` [N, H * vdim] = (q_t * P_t)^T S', S' the chunk's row of `states`.
+// A thread sums the logarithms of its channel's decays over a part of the chunk's tokens, learns through LDS what the parts before
+// it add up to, and walks its tokens again to leave q_t * P_t in LDS; then a wave takes 32 value channels at a time.  What bounds it is
+// latency: eight tokens' loads are asked for at once (44 us one by one, 36 so), and registers kept to four blocks a compute unit.
+// (Chunks of more tokens than LDS holds are taken LA_JOIN at a time.)
+#define LA_JOIN 64
+#define LA_SPAN (LA_DIM <= 256 ? LA_DIM : 256)       // channels that threads stand side by side for
+#define LA_PARTS (256 / LA_SPAN < 16 ? 256 / LA_SPAN : 16)
+#define LA_WIDE ((LA_DIM + 15) / 16 * 16)
+
+typedef float la_f32x4 __attribute__((ext_vector_type(4)));
 
 template <typename TP, int MODE>
-__global__ void la_prefix_kernel(const TP* __restrict__ proj, long long proj_stride, long long q_off,
-                                 const float* __restrict__ head_decay, const float* __restrict__ z,
-                                 long long z_stride, float inv_tau, const float* __restrict__ lower,
-                                 const float* __restrict__ zbias, const int* __restrict__ chunk_cu,
-                                 float* __restrict__ qp, float* __restrict__ last, int H, int chunk_len, int act,
-                                 float q_scale, int before) {
-  __shared__ float part_sum[LA_PARTS][LA_DIM];
-  const int c = blockIdx.x, head = blockIdx.y, d = threadIdx.x % LA_DIM, part = threadIdx.x / LA_DIM;
-  const int begin = chunk_cu[c], end = chunk_cu[c + 1];
-  const int per = (end - begin + LA_PARTS - 1) / LA_PARTS;
-  const int lo = begin + part * per < end ? begin + part * per : end;
-  const int hi = lo + per < end ? lo + per : end;
-  const float fixed_log = MODE != LA_HEAD ? 0.f : logf(head_decay[head]);
-  const float my_lower = MODE == LA_FORGET ? lower[head * LA_DIM + d] : 0.f;
-  const float my_bias = ((MODE == LA_FORGET || MODE == LA_EXP) && zbias) ? zbias[head * LA_DIM + d] : 0.f;
-  auto log_decay = [&](int t) {
-    if (MODE == LA_HEAD) return fixed_log;
-    const float zz = z[(size_t)t * z_stride + (size_t)head * LA_DIM + d];
-    if (MODE == LA_EXP) return -expf(zz + my_bias);
-    if (MODE == LA_FORGET) return log1pf(-la_forget_key(zz + my_bias, my_lower));
-    return (fminf(zz, 0.f) - log1pf(expf(-fabsf(zz)))) * inv_tau;
-  };
-  float mine = 0.f;
-  for (int t = lo; t < hi; ++t) mine += log_decay(t);
-  part_sum[part][d] = mine;
-  __syncthreads();
-  float acc = 0.f;     // log of the running product, from the chunk's first token on
-  for (int p = 0; p < part; ++p) acc += part_sum[p][d];
-  float* row = qp + ((size_t)c * H + head) * chunk_len * LA_DIM + d;
-  for (int t = lo; t < hi; ++t) {
-    const float up_to = acc;        // the decays before t
-    acc += log_decay(t);
-    const float q = la_act(ldf<TP>(proj + (size_t)t * proj_stride + q_off + (size_t)head * LA_DIM + d), act & 1) * q_scale;
-    row[(size_t)(t - begin) * LA_DIM] = q * expf(before ? up_to : acc);
+__global__ __launch_bounds__(256) void la_join_kernel(const TP* __restrict__ proj, long long proj_stride, long long q_off,
+                                                      const float* __restrict__ head_decay, const float* __restrict__ z, long long z_stride,
+                                                      float inv_tau, const float* __restrict__ lower, const float* __restrict__ zbias,
+                                                      const int* __restrict__ chunk_cu, const float* __restrict__ states,
+                                                      float* __restrict__ out, int H, int vdim, int act, float q_scale, int before) {
+  __shared__ float part_sum[LA_PARTS][LA_SPAN], upto[LA_DIM];      // upto: logarithms of all decays so far
+  // four values of padding: the 16 rows of an operand read lie in different banks
+  __shared__ __attribute__((aligned(16))) float qp[LA_JOIN][LA_WIDE + 4];
+  const int chunk = blockIdx.x, head = blockIdx.y, part = threadIdx.x / LA_SPAN;
+  const bool works = part < LA_PARTS;      // (a few threads are left over where LA_SPAN does not divide 256)
+  if (LA_WIDE > LA_DIM)
+    for (int i = threadIdx.x; i < LA_JOIN * 16; i += 256)
+      if (LA_WIDE - 16 + i % 16 >= LA_DIM) qp[i / 16][LA_WIDE - 16 + i % 16] = 0.f;
+  for (int i = threadIdx.x; i < LA_DIM; i += 256) upto[i] = 0.f;
+  const int chunk_end = chunk_cu[chunk + 1];
+  for (int begin = chunk_cu[chunk]; begin < chunk_end; begin += LA_JOIN) {
+    const int end = min(begin + LA_JOIN, chunk_end);
+    const int per = (end - begin + LA_PARTS - 1) / LA_PARTS;
+    const int lo = works ? min(begin + part * per, end) : end, hi = min(lo + per, end);
+    for (int d0 = 0; d0 < LA_DIM; d0 += LA_SPAN) {
+      const int d = d0 + (int)threadIdx.x % LA_SPAN;
+      const bool exists = d < LA_DIM;
+      const float fixed_log = MODE != LA_HEAD ? 0.f : logf(head_decay[head]);
+      const float my_lower = MODE == LA_FORGET && exists ? lower[head * LA_DIM + d] : 0.f;
+      const float my_bias = ((MODE == LA_FORGET || MODE == LA_EXP) && zbias && exists) ? zbias[head * LA_DIM + d] : 0.f;
+      auto log_decay = [&](float zz) {
+        if (MODE == LA_HEAD) return fixed_log;
+        if (MODE == LA_EXP) return -expf(zz + my_bias);
+        if (MODE == LA_FORGET) return log1pf(-la_forget_key(zz + my_bias, my_lower));
+        return la_log_decay(zz, inv_tau);
+      };
+      __syncthreads();      // the part sums and the rows before have been read
+      float mine = 0.f;
+      if (exists)
+        for (int t0 = lo; t0 < hi; t0 += 8) {
+          float zz[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) zz[i] = MODE == LA_HEAD ? 0.f : z[(size_t)min(t0 + i, hi - 1) * z_stride + (size_t)head * LA_DIM + d];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            if (t0 + i >= hi) break;
+            const float lg = log_decay(zz[i]);
+            mine += lg;
+            qp[t0 + i - begin][d] = lg;
+          }
+        }
+      if (works) part_sum[part][d - d0] = mine;
+      __syncthreads();
+      float acc = exists ? upto[d] : 0.f;     // log of the running product, from the chunk's first token on
+      if (works && exists) {
+        for (int p = 0; p < part; ++p) acc += part_sum[p][d - d0];
+        for (int t0 = lo; t0 < hi; t0 += 8) {
+          float qq[8];
+#pragma unroll
+          for (int i = 0; i < 8; ++i) qq[i] = ldf<TP>(proj + (size_t)min(t0 + i, hi - 1) * proj_stride + q_off + (size_t)head * LA_DIM + d);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) {
+            if (t0 + i >= hi) break;
+            const float earlier = acc;        // the decays before the token
+            acc += qp[t0 + i - begin][d];
+            qp[t0 + i - begin][d] = la_act(qq[i], act & 1) * q_scale * expf(before ? earlier : acc);
+          }
+        }
+      }
+      __syncthreads();
+      if (exists && part == LA_PARTS - 1) upto[d] = acc;
+    }
+    __syncthreads();
+    // v_mfma_f32_16x16x4_f32: A 16 tokens x 4 channels, B 4 channels x 16 values.  Lane group g holds channels 4 g .. 4 g + 3 of 16 and
+    // gives one of them to each of four instructions.
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15, tiles = (end - begin + 15) / 16;
+    const float* S = states + ((size_t)chunk * H + head) * LA_DIM * vdim;
+    for (int c0 = wave * 32; c0 < vdim; c0 += 128) {
+      la_f32x4 sum[4][2];
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) sum[t][c] = la_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+      for (int k = 0; k < LA_WIDE; k += 16) {
+        float b[4][2];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int c = 0; c < 2; ++c) {
+            const int row = k + 4 * g + j, col = c0 + 16 * c + r;
+            b[j][c] = row < LA_DIM && col < vdim ? S[(size_t)row * vdim + col] : 0.f;
+          }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          if (t >= tiles) break;
+          const float4 a = *reinterpret_cast<const float4*>(&qp[16 * t + r][k + 4 * g]);
+          const float av[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) sum[t][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j], b[j][c], sum[t][c], 0, 0, 0);
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          const int col = c0 + 16 * c + r;
+          if (col >= vdim) continue;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int tok = begin + 16 * t + 4 * g + j;
+            if (tok < end) out[((size_t)tok * H + head) * vdim + col] = sum[t][c][j];
+          }
+        }
+    }
   }
-  if (part == LA_PARTS - 1) last[((size_t)c * H + head) * LA_DIM + d] = expf(acc);
 }
 
 // One thread per element of a head's state: for the request's chunks in order, scratch[c] (the chunk's
@@ -228,34 +342,20 @@ __global__ void la_carry_kernel(float* __restrict__ scratch, const float* __rest
   *mine = S;
 }
 
-// corr [chunks, H, chunk_len, vdim] -> out [N, H * vdim]
-__global__ void la_gather_kernel(const float* __restrict__ corr, const int* __restrict__ chunk_cu,
-                                 float* __restrict__ out, int H, int chunk_len, int vdim) {
-  const int c = blockIdx.x, head = blockIdx.y;
-  const int begin = chunk_cu[c], n = chunk_cu[c + 1] - begin;
-  const float* src = corr + ((size_t)c * H + head) * chunk_len * vdim;
-  for (int i = threadIdx.x; i < n * vdim; i += blockDim.x) {
-    const int t = i / vdim, v = i % vdim;
-    out[((size_t)(begin + t) * H + head) * vdim + v] = src[i];
-  }
-}
-
-// before != 0: q_t meets the decays of the tokens before it only (outputs formed before the state moves on).
-extern "C" int qvl_la_prefix(const void* proj, long long proj_stride, long long q_off, int proj_dtype, const void* head_decay,
-                             const void* z, long long z_stride, float inv_tau, const void* lower, const void* zbias,
-                             int exp_decay, int before, const void* chunk_cu, void* qp,
-                             void* last, int chunks, int H, int dim, int chunk_len, int act, float q_scale,
-                             hipStream_t stream) {
+// The last of the kernels for chunks (see above); before != 0: q_t meets the decays of the tokens before it only (outputs formed before the
+// state moves on).
+extern "C" int qvl_la_join(const void* proj, long long proj_stride, long long q_off, int proj_dtype, const void* head_decay, const void* z,
+                           long long z_stride, float inv_tau, const void* lower, const void* zbias, int exp_decay, int before,
+                           const void* chunk_cu, const void* states, void* out, int chunks, int H, int dim, int vdim, int act,
+                           float q_scale, hipStream_t stream) {
   if (chunks <= 0) return QVL_OK;
-  if (dim != LA_DIM || H <= 0 || chunk_len <= 0 || (!head_decay && !z) || (lower && !z) ||
-      (exp_decay && (lower || !z)))
+  if (dim != LA_DIM || H <= 0 || vdim <= 0 || (!head_decay && !z) || (lower && !z) || (exp_decay && (lower || !z)))
     return QVL_ERR_SHAPE;
-  if (H > 65535 || LA_DIM * LA_PARTS > 1024) return QVL_ERR_LIMIT;
-#define LAUNCH(TP, MODE)                                                                                            \
-  hipLaunchKernelGGL((la_prefix_kernel<TP, MODE>), dim3(chunks, H), dim3(LA_DIM * LA_PARTS), 0, stream, (const TP*)proj, \
-                     proj_stride, q_off, (const float*)head_decay, (const float*)z, z_stride, inv_tau,               \
-                     (const float*)lower, (const float*)zbias, (const int*)chunk_cu, (float*)qp, (float*)last, H,    \
-                     chunk_len, act, q_scale, before)
+  if (H > 65535) return QVL_ERR_LIMIT;
+#define LAUNCH(TP, MODE)                                                                                                     \
+  hipLaunchKernelGGL((la_join_kernel<TP, MODE>), dim3(chunks, H), dim3(256), 0, stream, (const TP*)proj, proj_stride, q_off,  \
+                     (const float*)head_decay, (const float*)z, z_stride, inv_tau, (const float*)lower, (const float*)zbias,  \
+                     (const int*)chunk_cu, (const float*)states, (float*)out, H, vdim, act, q_scale, before)
 #define BY_MODE(TP) { if (exp_decay) LAUNCH(TP, LA_EXP); else if (lower) LAUNCH(TP, LA_FORGET); else if (z) LAUNCH(TP, LA_CHANNEL); else LAUNCH(TP, LA_HEAD); }
   if (proj_dtype == 0) BY_MODE(float)
   else if (proj_dtype == 1) BY_MODE(bf16_t)
@@ -276,15 +376,6 @@ extern "C" int qvl_la_carry(void* scratch, const void* last, void* state, const 
   return qvl_launch_status();
 }
 
-extern "C" int qvl_la_gather(const void* corr, const void* chunk_cu, void* out, int chunks, int H, int chunk_len,
-                             int vdim, hipStream_t stream) {
-  if (chunks <= 0) return QVL_OK;
-  if (H <= 0 || H > 65535 || chunk_len <= 0 || vdim <= 0) return QVL_ERR_SHAPE;
-  hipLaunchKernelGGL(la_gather_kernel, dim3(chunks, H), dim3(256), 0, stream, (const float*)corr, (const int*)chunk_cu,
-                     (float*)out, H, chunk_len, vdim);
-  return qvl_launch_status();
-}
-
 extern "C" int qvl_la_key_size() { return LA_DIM; }
 
 // proj: rows of `proj_stride` values holding q (H * LA_DIM columns from q_off), k (from k_off) and v
@@ -295,7 +386,7 @@ extern "C" int qvl_la_key_size() { return LA_DIM; }
 // [groups, N, H * vdim] (groups 1, 2, 4 or 8 with LA_DIM a multiple of 4 * groups), slabs `out_slab` apart.
 extern "C" int qvl_la_scan(const void* proj, long long proj_stride, long long q_off, long long k_off, long long v_off,
                            int proj_dtype, const void* head_decay, const void* z, long long z_stride, float inv_tau,
-                           const void* lower, const void* zbias, int exp_decay, const void* bonus, void* state, const void* cu_q, const void* req_slots, void* out, long long out_slab, int groups, int R,
+                           const void* lower, const void* zbias, int exp_decay, const void* bonus, void* state, const void* cu_q, const void* req_slots, void* out, long long out_slab, int groups, void* last, int R,
                            int H, int dim, int vdim, int act, float q_scale, hipStream_t stream) {
   if (R <= 0) return QVL_OK;
   if (dim != LA_DIM || H <= 0 || vdim <= 0 || (!head_decay && !z) || (lower && !z) ||
@@ -305,11 +396,20 @@ extern "C" int qvl_la_scan(const void* proj, long long proj_stride, long long q_
   if (groups != 1 && groups != 2 && groups != 4 && groups != 8) return QVL_ERR_SHAPE;
   if (LA_DIM % (LA_WAVES * groups)) return QVL_ERR_SHAPE;
   if (H > 65535 || R > 65535) return QVL_ERR_LIMIT;
-  const dim3 grid(((vdim + 63) / 64) * groups, H, R);
-#define LAUNCH(TP, CH, G, BONUS)                                                                                           \
-  hipLaunchKernelGGL((la_scan_kernel<TP, CH, G, BONUS>), grid, dim3(LA_THREADS), 0, stream, (const TP*)proj, proj_stride, q_off,   \
-                     k_off, v_off, (const float*)head_decay, (const float*)z, z_stride, inv_tau,                    \
-                     (const float*)lower, (const float*)zbias, (const float*)bonus, (float*)state, (const int*)cu_q, (const int*)req_slots, (float*)out, out_slab, H, vdim, act, q_scale)
+  // two value channels a lane for chunks of more than 64 (their state fits the registers)
+  const bool two = last && vdim > 64 && LA_DIM <= 256;
+  const dim3 grid((two ? (vdim + 127) / 128 : (vdim + 63) / 64) * groups, H, R);
+#define RUN(TP, CH, G, BONUS, COLS, CHUNK)                                                                                    \
+  hipLaunchKernelGGL((la_scan_kernel<TP, CH, G, BONUS, COLS, CHUNK>), grid, dim3(LA_THREADS), 0, stream, (const TP*)proj,     \
+                     proj_stride, q_off, k_off, v_off, (const float*)head_decay, (const float*)z, z_stride, inv_tau,          \
+                     (const float*)lower, (const float*)zbias, (const float*)bonus, (float*)state, (const int*)cu_q,          \
+                     (const int*)req_slots, (float*)out, out_slab, (float*)last, H, vdim, act, q_scale)
+#define LAUNCH(TP, CH, G, BONUS)                          \
+  do {                                                    \
+    if (two) RUN(TP, CH, G, BONUS, (LA_DIM <= 256 ? 2 : 1), true); \
+    else if (last) RUN(TP, CH, G, BONUS, 1, true);        \
+    else RUN(TP, CH, G, BONUS, 1, false);                 \
+  } while (0)
 #define BY_GROUPS(TP, CH, BONUS)                                                                                           \
   switch (groups) {                                                                                                 \
     case 1: LAUNCH(TP, CH, 1, BONUS); break;                                                                               \
@@ -331,5 +431,6 @@ extern "C" int qvl_la_scan(const void* proj, long long proj_stride, long long q_
 #undef BY_MODE
 #undef BY_GROUPS
 #undef LAUNCH
+#undef RUN
   return qvl_launch_status();
 }

@@ -32,7 +32,8 @@ def decayed_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, num_hea
                  head_decay: Optional[torch.Tensor] = None, z: Optional[torch.Tensor] = None, tau: float = 1.0,
                  silu=False, q_scale: float = 1.0, groups: int = 1, out: Optional[torch.Tensor] = None,
                  lower: Optional[torch.Tensor] = None, z_bias: Optional[torch.Tensor] = None,
-                 exp_decay: bool = False, bonus: Optional[torch.Tensor] = None) -> torch.Tensor:
+                 exp_decay: bool = False, bonus: Optional[torch.Tensor] = None,
+                 last: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Run every request's tokens of the step through the recurrence, from and into ``state``.
 
     ``proj [N, cols]`` or ``[parts, N, cols]`` (float32 or bfloat16; an offset then counts through the parts,
@@ -50,7 +51,8 @@ def decayed_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, num_hea
     request's run of tokens, ``req_slots [R]`` names its row of ``state``.  Returns float32
     ``[groups, N, heads * vdim]``: with ``groups`` above 1 (2, 4 or 8; the key size must be a multiple
     of four times it) the key channels are cut into that many groups with blocks of their own, and the
-    output is the sum of the slabs (see :func:`scan_groups`)."""
+    output is the sum of the slabs (see :func:`scan_groups`).  With ``last`` (float32 ``[R, heads, dim]``) every run starts from
+    zero, run r leaves its state in row r of ``state``, and ``last`` gets the product of its decays."""
     _dev(proj, state, cu_q, req_slots, head_decay, z, lower, z_bias, bonus)
     h, d, v = int(num_heads), int(dim), int(vdim)
     n = proj.shape[-2]
@@ -80,13 +82,17 @@ def decayed_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, num_hea
         out = torch.empty((groups, n, h * v), dtype=torch.float32, device=proj.device)
     _need(out.dtype == torch.float32 and out.shape == (groups, n, h * v) and out.is_contiguous() and out.is_cuda,
           "out must be contiguous float32 [groups, N, heads vdim]")
+    if last is not None:
+        _need(last.dtype == torch.float32 and last.shape == (r, h, d) and last.is_contiguous() and last.is_cuda
+              and state.shape[0] >= r, "last must be contiguous float32 [runs, heads, dim], with a row of state for each run")
     fn = _fn("linear_attention", "qvl_la_scan",
              [_c_ptr, _c_ll, _c_ll, _c_ll, _c_ll, _c_int, _c_ptr, _c_ptr, _c_ll, _c_float, _c_ptr, _c_ptr, _c_int, _c_ptr,
-              _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ll, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_ptr],
+              _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ll, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_ptr],
              {"LA_DIM": d})
     _check(fn(_ptr(proj), proj.stride(-2), *offs, dtype_code(proj.dtype),
               _ptr(head_decay), _ptr(z), zstride, 1.0 / float(tau), _ptr(lower), _ptr(z_bias), int(bool(exp_decay)),
-              _ptr(bonus), _ptr(state), _ptr(cu_q), _ptr(req_slots), _ptr(out), out.stride(0), int(groups), r, h, d, v, silu_mask(silu), float(q_scale),
+              _ptr(bonus), _ptr(state), _ptr(cu_q), _ptr(req_slots), _ptr(out), out.stride(0), int(groups), _ptr(last), r, h, d, v,
+              silu_mask(silu), float(q_scale),
               _stream()), "decayed_scan")
     return out
 
@@ -175,38 +181,33 @@ def chunked_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, num_hea
                  bonus: Optional[torch.Tensor] = None) -> torch.Tensor:
     """:func:`decayed_scan` for steps with long runs: the chunks of ``plan`` are scanned side by side
     from zero states, the states are carried from chunk to chunk, and what the state before a chunk
-    adds to the chunk's outputs is one float32 matrix product per (chunk, head), ``(q_t P_t) S``
+    adds to the chunk's outputs is a float32 product per (chunk, head), ``(q_t P_t) S``
     with ``P_t`` the product of the decays from the chunk's first token to ``t`` (with a bonus: to the token before).  Returns float32
     ``[slabs, N, heads * vdim]`` whose sum over the slabs is the output (the last slab holds the
     second term)."""
     h, d, v = int(num_heads), int(dim), int(vdim)
     n = proj.shape[-2]
     nch, clen = plan.chunks, plan.chunk_len
-    scratch = torch.zeros((nch, h, d, v), dtype=torch.float32, device=proj.device)
-    groups = scan_groups(nch, clen, h, d, v, proj.device)
+    r = req_slots.shape[0]
+    _need(plan.req_first.shape[0] == r + 1, "the chunk plan belongs to another step")
+    scratch = torch.empty((nch, h, d, v), dtype=torch.float32, device=proj.device)
+    last = torch.empty((nch, h, d), dtype=torch.float32, device=proj.device)
+    # (a block of a chunk's scan owns twice the value channels where there are more than 64)
+    groups = scan_groups(nch, clen, h, d, (v + 1) // 2 if v > 64 and d <= 256 else v, proj.device)
     out = torch.empty((groups + 1, n, h * v), dtype=torch.float32, device=proj.device)
     decayed_scan(proj, q_off, k_off, v_off, h, d, v, scratch, plan.chunk_cu, plan.chunk_rows, head_decay=head_decay,
                  z=z, tau=tau, silu=silu, q_scale=q_scale, groups=groups, out=out[:groups], lower=lower, z_bias=z_bias,
-                 exp_decay=exp_decay, bonus=bonus)
-    qp = torch.zeros((nch, h, clen, d), dtype=torch.float32, device=proj.device)
-    last = torch.empty((nch, h, d), dtype=torch.float32, device=proj.device)
+                 exp_decay=exp_decay, bonus=bonus, last=last)
     defines = {"LA_DIM": d}
-    fn = _fn("linear_attention", "qvl_la_prefix",
-             [_c_ptr, _c_ll, _c_ll, _c_int, _c_ptr, _c_ptr, _c_ll, _c_float, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr,
-              _c_ptr, _c_ptr,
-              _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_ptr], defines)
-    _check(fn(_ptr(proj), proj.stride(-2), _place(proj, q_off, h * d), dtype_code(proj.dtype), _ptr(head_decay), _ptr(z),
-              z.stride(0) if z is not None else 0, 1.0 / float(tau), _ptr(lower), _ptr(z_bias), int(bool(exp_decay)),
-              int(bonus is not None), _ptr(plan.chunk_cu),
-              _ptr(qp), _ptr(last), nch, h, d, clen, silu_mask(silu), float(q_scale), _stream()), "chunk prefix")
-    r = req_slots.shape[0]
-    _need(plan.req_first.shape[0] == r + 1, "the chunk plan belongs to another step")
     fn = _fn("linear_attention", "qvl_la_carry", [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int,
                                                    _c_ptr], defines)
     _check(fn(_ptr(scratch), _ptr(last), _ptr(state), _ptr(plan.req_first), _ptr(req_slots), r, h, d, v, _stream()),
            "chunk carry")
-    corr = torch.matmul(qp, scratch)          # [chunks, heads, chunk_len, vdim], true float32
-    fn = _fn("linear_attention", "qvl_la_gather", [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_ptr],
-             defines)
-    _check(fn(_ptr(corr), _ptr(plan.chunk_cu), _ptr(out[groups]), nch, h, clen, v, _stream()), "chunk gather")
+    fn = _fn("linear_attention", "qvl_la_join",
+             [_c_ptr, _c_ll, _c_ll, _c_int, _c_ptr, _c_ptr, _c_ll, _c_float, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr,
+              _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_ptr], defines)
+    _check(fn(_ptr(proj), proj.stride(-2), _place(proj, q_off, h * d), dtype_code(proj.dtype), _ptr(head_decay), _ptr(z),
+              z.stride(0) if z is not None else 0, 1.0 / float(tau), _ptr(lower), _ptr(z_bias), int(bool(exp_decay)),
+              int(bonus is not None), _ptr(plan.chunk_cu), _ptr(scratch), _ptr(out[groups]), nch, h, d, v, silu_mask(silu),
+              float(q_scale), _stream()), "chunk join")
     return out

@@ -380,6 +380,41 @@ def test_long_runs_scanned_in_chunks(channel):
     assert torch.allclose(s2, s1, atol=2e-5 * s1.abs().max().item()) and torch.equal(s2[4], start[4])
 
 
+@pytest.mark.parametrize("decay", ["head", "channel", "forget", "exp", "bonus"])
+@pytest.mark.parametrize("d, v, runs, chunk", [(64, 128, [129, 1, 63, 17], 64), (128, 200, [64, 65, 2], 64), (5, 65, [16, 33], 16),
+                                               (320, 130, [131], 100), (16, 257, [150], 64)])
+def test_chunks_joined_at_edges(d, v, runs, chunk, decay):
+    """One or two value channels a lane, value sizes off the tiles', key sizes off the matrix instruction's, chunks that one pass
+    of the join does not hold.  The bound: both sides add up to d float32 products and a run's decays, whose logarithms' rounding is
+    64 eps at most: 2e-5 of the largest value, as for a single scan."""
+    from qwen25vl_lite_amd.ops.linear_attention import chunked_scan, decayed_scan, plan_chunks
+    torch.manual_seed(d + v)
+    n, h = sum(runs), 2
+    dtype = torch.float32 if d == 5 else torch.bfloat16
+    proj = torch.randn(n, 2 * h * d + h * v + 8).to(dtype).cuda()
+    z = (1 + torch.randn(n, h * d + 3)).cuda()[:, :h * d] if decay != "head" else None
+    how = dict(z=z, silu="qk", q_scale=0.3)
+    if decay == "head":
+        how["head_decay"] = torch.tensor([0.5, 1.0]).cuda()
+    elif decay == "forget":
+        how.update(lower=torch.rand(h * d).cuda(), z_bias=torch.randn(h * d).cuda())
+    elif decay in ("exp", "bonus"):
+        how.update(exp_decay=True, z_bias=(torch.randn(h * d) - 3).cuda())
+        how["bonus"] = torch.randn(h * d).cuda() if decay == "bonus" else None
+    bounds = [0]
+    for r in runs:
+        bounds.append(bounds[-1] + r)
+    cu = torch.tensor(bounds, dtype=torch.int32).cuda()
+    slots = torch.arange(len(runs), 0, -1, dtype=torch.int32).cuda()
+    start = torch.randn(len(runs) + 2, h, d, v).cuda()
+    s1, s2 = start.clone(), start.clone()
+    want = decayed_scan(proj, 0, h * d, 2 * h * d, h, d, v, s1, cu, slots, **how).sum(0)
+    got = chunked_scan(proj, 0, h * d, 2 * h * d, h, d, v, s2, plan_chunks(bounds, "cuda:0", chunk), slots, **how).sum(0)
+    assert torch.allclose(got, want, atol=2e-5 * want.abs().max().item()), (got - want).abs().max() / want.abs().max()
+    assert torch.allclose(s2, s1, atol=2e-5 * s1.abs().max().item())
+    assert torch.equal(s2[0], start[0]) and torch.equal(s2[-1], start[-1])
+
+
 @pytest.mark.parametrize("span, groups", [(7, 3), (24, 5), (128, 2), (1024, 1), (1500, 2), (4100, 1)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_group_norm_with_gate_at_any_width(span, groups, dtype):
