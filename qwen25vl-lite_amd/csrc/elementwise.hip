@@ -101,8 +101,8 @@ extern "C" int qvl_embed_gather(const void* ids, const void* table, void* out, i
 //                                       along its inner size, which are added in slab order)
 //   h[row] = v                         (unless `rows` selects rows: then h is left alone)
 //   out[m] = v * (1/sqrt(mean(v^2) + eps)) * w
-// One block per row; the reduction order depends on H only, so a row's result does not
-// depend on what else is in the batch.
+// One block per row; the reduction order depends on H only (and the two kernels for widths that 4 divides have the same),
+// so a row's result does not depend on what else is in the batch.
 // ---------------------------------------------------------------------------------------
 template <typename TD, typename TO>
 __global__ void add_rmsnorm_kernel(float* __restrict__ h, const TD* __restrict__ delta, const float* __restrict__ w,
@@ -139,13 +139,7 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ h, const TD* __restrict__
 // multiple of 4 and at most NORM_VEC_MAX * 4 * 256, read and written 4 values at a time.
 #define NORM_VEC_MAX 8
 
-template <typename T> __device__ __forceinline__ float4 ld4(const T* p);
-template <> __device__ __forceinline__ float4 ld4<float>(const float* p) { return *reinterpret_cast<const float4*>(p); }
-template <> __device__ __forceinline__ float4 ld4<bf16_t>(const bf16_t* p) {
-  const uint2 v = *reinterpret_cast<const uint2*>(p);
-  return float4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
-                __uint_as_float(v.y & 0xffff0000u)};
-}
+__device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 template <typename T> __device__ __forceinline__ void st4(T* p, float4 v);
 template <> __device__ __forceinline__ void st4<float>(float* p, float4 v) { *reinterpret_cast<float4*>(p) = v; }
 template <> __device__ __forceinline__ void st4<bf16_t>(bf16_t* p, float4 v) {
@@ -155,94 +149,160 @@ template <> __device__ __forceinline__ void st4<bf16_t>(bf16_t* p, float4 v) {
   *reinterpret_cast<uint2*>(p) = o;
 }
 
-template <typename TD, typename TO>
+// The sum of squares of these kernels and of the one for slabs below has one order, that of 16 waves of 64 lanes with one or two
+// pieces each, whatever the number of threads: here a wave stands for up to four.
+__device__ __forceinline__ float add_squares(float ss, float4 x) { 
+  return ss + fmaf(x.w, x.w, fmaf(x.z, x.z, fmaf(x.y, x.y, x.x * x.x)));
+}
+template <int N>
+__device__ __forceinline__ float norm_total(const float* sums) {
+  float t = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) t += sums[i];
+  return t;
+}
+
+// VEC: 4-value pieces of a thread.  Everything it needs is asked for before anything is waited for, converted or stored (a store to h
+// would hold up the loads of h behind it, a branch around a load the next load): pieces past the row's end read its last one.  Of an
+// addend in slabs (float32), one slab at a time, in order.
+// Bytes bound it from about a thousand rows on: 4,096 rows of 3,584 with a bfloat16 addend 28.5 -> 26.9 us, 6.6 TB/s; below, latency: 64
+// rows of 8,192 7.4 -> 5.4, when the loads waited for each other's stores and the weights for the sum.
+template <typename T> struct norm_raw;
+template <> struct norm_raw<float> { typedef float4 type; };
+template <> struct norm_raw<bf16_t> { typedef uint2 type; };
+__device__ __forceinline__ float4 norm_value(float4 v) { return v; }
+__device__ __forceinline__ float4 norm_value(uint2 v) {
+  return float4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
+                __uint_as_float(v.y & 0xffff0000u)};
+}
+
+template <typename TD, typename TO, int VEC>
 __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict__ h, const TD* __restrict__ delta,
                                                               const float* __restrict__ w, TO* __restrict__ out,
-                                                              const int* __restrict__ rows, int H, float eps) {
-  __shared__ float red[17];
+                                                              const int* __restrict__ rows, int H, float eps, int nslabs,
+                                                              long long slab_stride) {
+  constexpr int PART = VEC < 4 ? VEC : 4;
+  typedef typename norm_raw<TD>::type Raw;
+  __shared__ __attribute__((aligned(16))) float sums[4 * PART];
   const int m = blockIdx.x;
   const int row = rows ? rows[m] : m;
   float* hr = h + (size_t)row * H;
-  const TD* dr = delta ? delta + (size_t)row * H : nullptr;
   const int nvec = H >> 2;
-  float4 v[NORM_VEC_MAX];
-  float ss = 0.f;
+  int at[VEC];
+  float4 v[VEC], g[VEC];
 #pragma unroll
-  for (int j = 0; j < NORM_VEC_MAX; ++j) {
-    const int i = threadIdx.x + 256 * j;
-    if (i < nvec) {
-      float4 x = ld4<float>(hr + 4 * i);
-      if (dr) {
-        const float4 d = ld4<TD>(dr + 4 * i);
-        x.x += d.x; x.y += d.y; x.z += d.z; x.w += d.w;
-        if (!rows) st4<float>(hr + 4 * i, x);
-      }
-      v[j] = x;
-      ss += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
-    }
+  for (int j = 0; j < VEC; ++j) {
+    at[j] = 4 * min((int)threadIdx.x + 256 * j, nvec - 1);
+    v[j] = ld4(hr + at[j]);
   }
-  const float rs = 1.0f / sqrtf(block_sum(ss, red) / (float)H + eps);
+  if (delta) {
+    const TD* dr = delta + (size_t)row * H;
+    Raw d[VEC];
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) d[j] = *reinterpret_cast<const Raw*>(dr + at[j]);
+    float4 sum[VEC];
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) g[j] = ld4(w + at[j]);
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) sum[j] = norm_value(d[j]);
+    for (int c = 1; c < nslabs; ++c) {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) d[j] = *reinterpret_cast<const Raw*>(dr + (size_t)c * slab_stride + at[j]);
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        const float4 e = norm_value(d[j]);
+        sum[j].x += e.x; sum[j].y += e.y; sum[j].z += e.z; sum[j].w += e.w;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      v[j].x += sum[j].x; v[j].y += sum[j].y; v[j].z += sum[j].z; v[j].w += sum[j].w;
+      if (!rows && (int)threadIdx.x + 256 * j < nvec) st4<float>(hr + at[j], v[j]);
+    }
+  } else {
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) g[j] = ld4(w + at[j]);
+  }
+  float ss[PART] = {};
+#pragma unroll
+  for (int j = 0; j < VEC; ++j)
+    if ((int)threadIdx.x + 256 * j < nvec) ss[j % PART] = add_squares(ss[j % PART], v[j]);
+#pragma unroll
+  for (int j = 0; j < PART; ++j) {
+    ss[j] = wave_sum(ss[j]);
+    if ((threadIdx.x & 63) == 0) sums[4 * j + (threadIdx.x >> 6)] = ss[j];
+  }
+  __syncthreads();
+  const float rs = 1.0f / sqrtf(norm_total<4 * PART>(sums) / (float)H + eps);
   TO* o = out + (size_t)m * H;
 #pragma unroll
-  for (int j = 0; j < NORM_VEC_MAX; ++j) {
-    const int i = threadIdx.x + 256 * j;
-    if (i < nvec) {
-      const float4 g = ld4<float>(w + 4 * i);
-      st4<TO>(o + 4 * i, float4{(v[j].x * rs) * g.x, (v[j].y * rs) * g.y, (v[j].z * rs) * g.z, (v[j].w * rs) * g.w});
-    }
+  for (int j = 0; j < VEC; ++j) {
+    if ((int)threadIdx.x + 256 * j < nvec)
+      st4<TO>(o + at[j], float4{(v[j].x * rs) * g[j].x, (v[j].y * rs) * g[j].y, (v[j].z * rs) * g[j].z, (v[j].w * rs) * g[j].w});
   }
 }
 
-// The addend as slabs of partial sums (float32 [slab][row][H], H a multiple of 4 and at most
-// SLAB_VEC_MAX * 4096): a block of 1024 threads per row, a thread per 4 neighbouring values, the
-// slabs' loads asked for sixteen at a time (they do not depend on each other, only the sum has an
-// order: slab 0, 1, 2, ...).
-#define SLAB_VEC_MAX 2
-template <typename TO>
+// The addend as slabs of partial sums (float32 [slab][row][H]) for fewer than NORM_ROWS rows: a block of 1024 threads per row, a thread
+// per 4 or 8 values, the loads of up to sixteen slabs asked for at a time (they do not depend on each other, only the sum has an
+// order: slab 0, 1, 2, ...).  Latency bounds it: fewer rows than fill the chip wait for memory once here and once a slab in the kernel
+// above (3,584 values, eight slabs: 64 rows 4.1 us and 5.0, 256 rows 5.3 and 7.0), and rows of 8,192 once, when their second half was
+// asked for behind the store of the first 6.9 us of 64 rows and four slabs, now 5.1.  Many rows are bound by bytes: blocks of 1024 threads
+// that are all at the same point leave the memory idle (of two slabs 512 rows 7.4 and 6.0, 2,048 rows 26.5 and 20.8).
+#define NORM_ROWS 512
+template <typename TO, int VEC>
 __global__ __launch_bounds__(1024) void add_rmsnorm_slabs_kernel(float* __restrict__ h, const float* __restrict__ delta,
                                                                  const float* __restrict__ w, TO* __restrict__ out,
                                                                  const int* __restrict__ rows, int H, float eps,
                                                                  int nslabs, long long slab_stride) {
-  __shared__ float red[17];
+  constexpr int ONCE = VEC == 1 ? 16 : 4;      // slabs asked for at once (eight of two pieces: 8,192 values, one row 6.4 us for 5.4)
+  __shared__ __attribute__((aligned(16))) float sums[16];
   const int m = blockIdx.x;
   const int row = rows ? rows[m] : m;
   float* hr = h + (size_t)row * H;
   const float* dr = delta + (size_t)row * H;
-  const int nvec = H >> 2;
-  float4 v[SLAB_VEC_MAX], g[SLAB_VEC_MAX];
+  const float4 zero = {0.f, 0.f, 0.f, 0.f};
+  int at[VEC];
+  float4 v[VEC], g[VEC], d[VEC];
+  // everything the thread needs is asked for before anything is waited for: the row of h, the
+  // norm's weights and up to 16 pieces of slabs
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) {
+    at[j] = 4 * ((int)threadIdx.x + 1024 * j);
+    v[j] = at[j] < H ? ld4(hr + at[j]) : zero;
+    g[j] = at[j] < H ? ld4(w + at[j]) : zero;
+    d[j] = zero;
+  }
+  for (int c0 = 0; c0 < nslabs; c0 += ONCE) {
+    float4 e[ONCE][VEC];
+#pragma unroll
+    for (int c = 0; c < ONCE; ++c)
+#pragma unroll
+      for (int j = 0; j < VEC; ++j)
+        e[c][j] = c0 + c < nslabs && at[j] < H ? ld4(dr + (size_t)(c0 + c) * slab_stride + at[j]) : zero;
+#pragma unroll
+    for (int c = 0; c < ONCE; ++c)
+#pragma unroll
+      for (int j = 0; j < VEC; ++j)
+        if (c0 + c < nslabs) { d[j].x += e[c][j].x; d[j].y += e[c][j].y; d[j].z += e[c][j].z; d[j].w += e[c][j].w; }
+  }
   float ss = 0.f;
 #pragma unroll
-  for (int j = 0; j < SLAB_VEC_MAX; ++j) {
-    const int i = threadIdx.x + 1024 * j;
-    if (i < nvec) {
-      // everything the thread needs is asked for before anything is waited for: the row of h, the
-      // norm's weights and up to 16 slabs
-      float4 x = ld4<float>(hr + 4 * i);
-      g[j] = ld4<float>(w + 4 * i);
-      float4 d = {0.f, 0.f, 0.f, 0.f};
-      for (int c0 = 0; c0 < nslabs; c0 += 16) {
-        float4 e[16];
-#pragma unroll
-        for (int c = 0; c < 16; ++c)
-          e[c] = c0 + c < nslabs ? ld4<float>(dr + (size_t)(c0 + c) * slab_stride + 4 * i) : float4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int c = 0; c < 16; ++c) {
-          if (c0 + c < nslabs) { d.x += e[c].x; d.y += e[c].y; d.z += e[c].z; d.w += e[c].w; }
-        }
-      }
-      x.x += d.x; x.y += d.y; x.z += d.z; x.w += d.w;
-      if (!rows) st4<float>(hr + 4 * i, x);
-      v[j] = x;
-      ss += x.x * x.x + x.y * x.y + x.z * x.z + x.w * x.w;
+  for (int j = 0; j < VEC; ++j) {
+    v[j].x += d[j].x; v[j].y += d[j].y; v[j].z += d[j].z; v[j].w += d[j].w;
+    if (at[j] < H) {
+      if (!rows) st4<float>(hr + at[j], v[j]);
+      ss = add_squares(ss, v[j]);
     }
   }
-  const float rs = 1.0f / sqrtf(block_sum(ss, red) / (float)H + eps);
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  const float rs = 1.0f / sqrtf(norm_total<16>(sums) / (float)H + eps);
   TO* o = out + (size_t)m * H;
 #pragma unroll
-  for (int j = 0; j < SLAB_VEC_MAX; ++j) {
-    const int i = threadIdx.x + 1024 * j;
-    if (i < nvec)
-      st4<TO>(o + 4 * i, float4{(v[j].x * rs) * g[j].x, (v[j].y * rs) * g[j].y, (v[j].z * rs) * g[j].z, (v[j].w * rs) * g[j].w});
+  for (int j = 0; j < VEC; ++j) {
+    if (at[j] < H)
+      st4<TO>(o + at[j], float4{(v[j].x * rs) * g[j].x, (v[j].y * rs) * g[j].y, (v[j].z * rs) * g[j].z, (v[j].w * rs) * g[j].w});
   }
 }
 
@@ -253,23 +313,29 @@ extern "C" int qvl_add_rmsnorm(void* h, const void* delta, const void* w, void* 
   if (M <= 0) return QVL_OK;
   if (H <= 0 || nslabs < 1 || (nslabs > 1 && slab_stride < H)) return QVL_ERR_SHAPE;
   const int threads = H >= 2048 ? 512 : 256;
-  const bool vec = H % 4 == 0 && H <= NORM_VEC_MAX * 4 * 256 && nslabs == 1;
-  if (nslabs > 1 && delta && delta_dtype == 0 && H % 4 == 0 && slab_stride % 4 == 0 && H <= SLAB_VEC_MAX * 4096) {
-    if (out_dtype == 0)
-      hipLaunchKernelGGL((add_rmsnorm_slabs_kernel<float>), dim3(M), dim3(1024), 0, stream, (float*)h, (const float*)delta,
-                         (const float*)w, (float*)out, (const int*)rows, H, eps, nslabs, slab_stride);
-    else if (out_dtype == 1)
-      hipLaunchKernelGGL((add_rmsnorm_slabs_kernel<bf16_t>), dim3(M), dim3(1024), 0, stream, (float*)h, (const float*)delta,
-                         (const float*)w, (bf16_t*)out, (const int*)rows, H, eps, nslabs, slab_stride);
-    else
-      return QVL_ERR_DTYPE;
+  const bool wide = H % 4 == 0 && H <= NORM_VEC_MAX * 4 * 256, slabs = nslabs > 1 && delta;
+  const bool vec = wide && (!slabs || (delta_dtype == 0 && slab_stride % 4 == 0));
+  if (vec && slabs && M < NORM_ROWS) {
+#define QVL_NORM_SLABS(TO, VEC)                                                                                    \
+  hipLaunchKernelGGL((add_rmsnorm_slabs_kernel<TO, VEC>), dim3(M), dim3(1024), 0, stream, (float*)h,               \
+                     (const float*)delta, (const float*)w, (TO*)out, (const int*)rows, H, eps, nslabs, slab_stride)
+    if (out_dtype == 0 && H <= 4096) QVL_NORM_SLABS(float, 1);
+    else if (out_dtype == 0) QVL_NORM_SLABS(float, 2);
+    else if (out_dtype == 1 && H <= 4096) QVL_NORM_SLABS(bf16_t, 1);
+    else if (out_dtype == 1) QVL_NORM_SLABS(bf16_t, 2);
+    else return QVL_ERR_DTYPE;
+#undef QVL_NORM_SLABS
     return qvl_launch_status();
   }
+#define QVL_NORM_VEC(TD, TO, VEC)                                                                                  \
+  hipLaunchKernelGGL((add_rmsnorm_vec_kernel<TD, TO, VEC>), dim3(M), dim3(256), 0, stream, (float*)h,              \
+                     (const TD*)delta, (const float*)w, (TO*)out, (const int*)rows, H, eps, nslabs, slab_stride)
 #define QVL_NORM_CASE(DD, OD, TD, TO)                                                                              \
   if (delta_dtype == DD && out_dtype == OD) {                                                                      \
-    if (vec)                                                                                                       \
-      hipLaunchKernelGGL((add_rmsnorm_vec_kernel<TD, TO>), dim3(M), dim3(256), 0, stream, (float*)h,               \
-                         (const TD*)delta, (const float*)w, (TO*)out, (const int*)rows, H, eps);                   \
+    if (vec && H <= 1024) QVL_NORM_VEC(TD, TO, 1);                                                                 \
+    else if (vec && H <= 2048) QVL_NORM_VEC(TD, TO, 2);                                                            \
+    else if (vec && H <= 4096) QVL_NORM_VEC(TD, TO, 4);                                                            \
+    else if (vec) QVL_NORM_VEC(TD, TO, NORM_VEC_MAX);                                                              \
     else                                                                                                           \
       hipLaunchKernelGGL((add_rmsnorm_kernel<TD, TO>), dim3(M), dim3(threads), 0, stream, (float*)h,               \
                          (const TD*)delta, (const float*)w, (TO*)out, (const int*)rows, H, eps, nslabs,            \
@@ -281,6 +347,7 @@ extern "C" int qvl_add_rmsnorm(void* h, const void* delta, const void* w, void* 
   QVL_NORM_CASE(1, 1, bf16_t, bf16_t)
   QVL_NORM_CASE(1, 0, bf16_t, float)
 #undef QVL_NORM_CASE
+#undef QVL_NORM_VEC
   return QVL_ERR_DTYPE;
 }
 

@@ -49,6 +49,29 @@ def test_embed_gather_with_rotation_tables(width, n, dtype):
         kernels.embed_gather(ids, table, positions=positions, rotations=rotations + rotations[:1])
 
 
+@pytest.mark.parametrize("width, slabs", [(4, 2), (1028, 1), (2048, 5), (3584, 17), (4096, 2), (4100, 9), (8192, 4)])
+def test_add_rmsnorm_of_few_and_many_rows(width, slabs):
+    """Both sides of the line between the kernels: the same bits for the same rows, and what float64 gives within the rounding of
+    the slabs' sum (slabs + 1 additions) and of width squares, half an eps each at most, of which the root takes half."""
+    from qwen25vl_lite_amd.ops import kernels
+    torch.manual_seed(width)
+    rows, eps = 513, 1e-6
+    h, w = torch.randn(rows, width), torch.randn(width)
+    delta = torch.randn(slabs, rows, width) if slabs > 1 else torch.randn(rows, width)
+    total = h.double() + (delta.double().sum(0) if slabs > 1 else delta.double())
+    want = total / torch.sqrt(total.pow(2).mean(1, keepdim=True) + eps) * w.double()
+    hd = h.cuda()
+    out = kernels.add_rmsnorm(hd, delta.cuda(), w.cuda(), eps, torch.float32)
+    few_h, few_d = h[:40].contiguous().cuda(), (delta[:, :40] if slabs > 1 else delta[:40]).contiguous().cuda()
+    few = kernels.add_rmsnorm(few_h, few_d, w.cuda(), eps, torch.float32)
+    assert torch.equal(few, out[:40]) and torch.equal(few_h, hd[:40])
+    eps32, size = 2.0 ** -23, (h.abs().double() + (delta.abs().double().sum(0) if slabs > 1 else delta.abs().double()))
+    bound = (slabs + 1) * eps32 * size
+    assert ((hd.cpu().double() - total).abs() <= bound).all()
+    rel = bound.max() / total.pow(2).mean(1).sqrt().min() + (0.25 * width + 4) * eps32
+    assert ((out.cpu().double() - want).abs() <= (bound + rel * total.abs()) / torch.sqrt(total.pow(2).mean(1, keepdim=True)) * w.abs().double()).all()
+
+
 @pytest.mark.parametrize("width", [97, 3584, 8200])
 @pytest.mark.parametrize("delta_dtype, out_dtype", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16),
                                                     (torch.bfloat16, torch.bfloat16), (None, torch.bfloat16)])
