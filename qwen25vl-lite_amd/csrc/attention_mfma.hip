@@ -1421,17 +1421,29 @@ extern "C" int qvl_attn_mfma_block_plan(const int* cu_q, const int* ctx, const u
     std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
       return walks[a].kb_last - walks[a].kb_first > walks[b].kb_last - walks[b].kb_first;
     });
-    std::vector<std::vector<PlanPart>> placed(places);
     int T = (int)std::min<long long>(total / places + 1, 0x3fffffff);
-    while (!plan_at(walks, order, places, groups, T, most_cut, placed, parts_of)) T += T / 32 + 1;
+    // No time below the longest walk's allows a plan unless it allows a part of LEAST_PART.  Short prompts, whose walks then have a place
+    // each and stay whole, are done here: nothing else is between them and the device (100 tokens: 26 us of the host, 2 so).
+    const int longest = n ? (walks[order[0]].kb_last - walks[order[0]].kb_first + groups) / groups + ITEM_COST : 0;
+    while (T < std::min(longest, ITEM_COST + PART_COST + 2 * MERGE_COST + LEAST_PART)) T += T / 32 + 1;
     struct Listed {
       int blocks;
       PlanPart part;
     };
     std::vector<Listed> list;
-    for (const auto& parts : placed)
-      for (const PlanPart& part : parts) list.push_back(Listed{part.kb_last - part.kb_first + 1, part});
-    std::sort(list.begin(), list.end(), [](const Listed& a, const Listed& b) {
+    const bool whole = n <= places && T >= longest;
+    if (whole) {
+      for (int i : order) {
+        list.push_back(Listed{walks[i].kb_last - walks[i].kb_first + 1, PlanPart{i, walks[i].kb_first, walks[i].kb_last, 0}});
+        parts_of[i] = 1;
+      }
+    } else {
+      std::vector<std::vector<PlanPart>> placed(places);
+      while (!plan_at(walks, order, places, groups, T, most_cut, placed, parts_of)) T += T / 32 + 1;
+      for (const auto& parts : placed)
+        for (const PlanPart& part : parts) list.push_back(Listed{part.kb_last - part.kb_first + 1, part});
+    }
+    if (!whole) std::sort(list.begin(), list.end(), [](const Listed& a, const Listed& b) {
       return a.blocks != b.blocks ? a.blocks > b.blocks : a.part.walk != b.part.walk ? a.part.walk < b.part.walk : a.part.part < b.part.part;
     });
     if ((long long)list.size() > room) return QVL_ERR_LIMIT;

@@ -156,8 +156,8 @@ def plan_walks(cu_q, ctx_len, group: int, nkv: int, window: int, places: int, gr
     ctx = np.ascontiguousarray(ctx_len, dtype=np.int32)
     keep = None if only is None else np.ascontiguousarray(only, dtype=np.uint8)
     cols = 16 * int(_fn("attention_mfma", "qvl_attn_mfma_block_tiles", [], defines)())
-    runs = int(((np.diff(cu.astype(np.int64)) * group + cols - 1) // cols).sum())
-    room = runs * nkv + places       # a part that is cut off fills its place or ends its walk
+    # walks at most, and a part that is cut off fills its place or ends its walk
+    room = (int(cu[-1]) * group // cols + len(ctx)) * nkv + places
     out, head = np.empty((room, 8), dtype=np.int32), np.zeros(6, dtype=np.int32)
     fn = _fn("attention_mfma", "qvl_attn_mfma_block_plan", [_c_ptr] * 3 + [_c_int] * 7 + [_c_ptr, _c_ll, _c_ptr], defines)
     _check(fn(cu.ctypes.data, ctx.ctypes.data, None if keep is None else keep.ctypes.data, len(ctx), group, nkv, window, places,
@@ -184,21 +184,23 @@ def _count_tiles(step, group: int, tile_ct: int, only=None) -> int:
     """Entries of ``tile_ct`` column tiles that the step's requests make."""
     key = ("count of tiles", group, tile_ct, only)       # the same for every layer of the step
     if key not in step.derived:
-        q = np.diff(np.asarray(step.cu_q_host, dtype=np.int64))
-        if only is not None:
-            q = q * np.asarray(only, dtype=np.int64)
-        step.derived[key] = int(((q * group + 16 * tile_ct - 1) // (16 * tile_ct)).sum())
+        step.derived[key] = sum(e for e, _ in _entries(step, group, tile_ct, only))
     return step.derived[key]
+
+
+def _entries(step, group: int, tile_ct: int, only=None):
+    """Per request: ``(entries of tile_ct column tiles, tokens)``.  (Plain integers: a step of few requests waits for nothing but the host,
+    and an array of one takes 8 us for 1.)"""
+    cu, cols = step.cu_q_host, 16 * tile_ct
+    for r in range(len(cu) - 1):
+        q = int(cu[r + 1]) - int(cu[r]) if only is None or only[r] else 0
+        yield (q * group + cols - 1) // cols, q
 
 
 def _walk_blocks(step, group: int, tile_ct: int, only=None) -> int:
     """About how many 32-key blocks the step's entries of ``tile_ct`` column tiles walk, for one key/value head."""
-    q = np.diff(np.asarray(step.cu_q_host, dtype=np.int64))
-    ctx = np.asarray(step.ctx_len_host, dtype=np.int64)
-    if only is not None:
-        q = q * np.asarray(only, dtype=np.int64)
-    entries = (q * group + 16 * tile_ct - 1) // (16 * tile_ct)
-    return int((entries * np.maximum(1, (ctx - q // 2 + 31) // 32)).sum())
+    return sum(e * max(1, (int(ctx) - q // 2 + 31) // 32)
+               for (e, q), ctx in zip(_entries(step, group, tile_ct, only), step.ctx_len_host))
 
 
 def _step_walks(step, group: int, nkv: int, hd: int, window: int, device, only=None, force_wide=None, force_groups=None):

@@ -104,7 +104,8 @@ def test_a_steps_lists_are_not_made_inside_a_graph(monkeypatch):
 
 @pytest.mark.parametrize("qlens, lens, group, nkv, window", [([2048], [2048], 7, 4, 0), ([512], [8192], 7, 4, 0), ([1], [40000], 8, 1, 0),
                                                              ([700, 1, 33], [3000, 9000, 33], 1, 6, 0), ([300, 0, 90], [5000, 7, 90], 5, 8, 1000),
-                                                             ([1], [1], 1, 16, 0), ([20000], [30000], 16, 2, 0)])
+                                                             ([1], [1], 1, 16, 0), ([20000], [30000], 16, 2, 0),
+                                                             ([300, 5, 0, 129], [300, 400, 9, 200], 7, 3, 0)])
 @pytest.mark.parametrize("places, groups, wide", [(512, 1, False), (256, 2, False), (512, 1, True), (13, 1, False)])
 def test_walks_of_prompt_portions(qlens, lens, group, nkv, window, places, groups, wide):
     """Every run of column tiles of every head has its key blocks once, in parts that follow each other, longest first; the parts of
