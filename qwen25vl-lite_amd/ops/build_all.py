@@ -3,6 +3,7 @@
 from __future__ import annotations
 
 import os
+from concurrent.futures import ThreadPoolExecutor
 from typing import List
 
 from .library import build_library, python_headers
@@ -75,8 +76,10 @@ LIBRARIES = [
 
 def build_everything(force: bool = False, quiet: bool = False) -> List[str]:
     # (without the interpreter's headers the sampler's settings are gathered in Python)
-    built = [build_library(stem, defines, force=force, quiet=quiet) for stem, defines in LIBRARIES
-             if stem != "sample_gather" or python_headers()]
+    wanted = [(stem, defines) for stem, defines in LIBRARIES if stem != "sample_gather" or python_headers()]
+    # eight compilers side by side: one after another the chunks' scans alone, 120 kinds for each key size, take six minutes
+    with ThreadPoolExecutor(min(8, os.cpu_count() or 1)) as pool:
+        built = list(pool.map(lambda one: build_library(*one, force=force, quiet=quiet), wanted))
     # libraries of sources that have changed since are of no use to anyone
     keep = {os.path.basename(p) for p in built}
     for directory in {os.path.dirname(p) for p in built}:

@@ -57,7 +57,7 @@ def build_dir() -> str:
     path = os.path.join(csrc_dir(), "_build")
     try:
         os.makedirs(path, exist_ok=True)
-        probe = os.path.join(path, f".write-{os.getpid()}")
+        probe = os.path.join(path, f".write-{os.getpid()}-{threading.get_ident()}")
         with open(probe, "w"):
             pass
         os.remove(probe)
