@@ -422,9 +422,10 @@ __global__ __launch_bounds__(64 * RW) void gemm_resident_kernel(ResidentArgs p) 
         const float other = __shfl_xor(sum, 8, QVL_WAVE);   // the channel this one is rotated with
         const int head = n / p.hd, d = n - head * p.hd;
         if (m < p.M && nl < tile_rows(tile) && n < p.N) {
-          // (cos, sin) is (1, 0) for value heads; rows 0..7 of a rotated tile are the first halves
-          const float val = (nl < 8 || head >= p.nq + p.nkv) ? sum * epi[i].cs.x - other * epi[i].cs.y
-                                                              : sum * epi[i].cs.x + other * epi[i].cs.y;
+          // values are stored as they are (turned by (1, 0), one that is not finite would take its neighbour along); rows 0..7 of
+          // a rotated tile are the first halves
+          const float val = head >= p.nq + p.nkv ? sum
+                            : nl < 8 ? sum * epi[i].cs.x - other * epi[i].cs.y : sum * epi[i].cs.x + other * epi[i].cs.y;
           if (head < p.nq) {
             p.q_out[((size_t)m * p.nq + head) * p.hd + d] = f32_to_bf16(val);
           } else if (epi[i].slot >= 0) {

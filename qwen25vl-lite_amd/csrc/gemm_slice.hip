@@ -114,7 +114,7 @@ __global__ __launch_bounds__(64 * SLICE_WAVES) void gemm_slice_kernel(SliceArgs 
     for (int t = 0; t < 2; ++t) w[u][t] = load16(w_buf, u < inside ? w_at[t] : PAST_END, u * 64);
   // what the results need beside the sums; result e of the block: row e / 16 of X, pair e mod 16
   float b0[ENDS], b1[ENDS];
-  float2 turn[ENDS];
+  float2 turn[ENDS];     // (of queries and keys)
   int slot[ENDS];
 #pragma unroll
   for (int i = 0; i < ENDS; ++i) {
@@ -194,8 +194,10 @@ __global__ __launch_bounds__(64 * SLICE_WAVES) void gemm_slice_kernel(SliceArgs 
       to = key ? p.kc + (of * p.ps + place) * p.hd + f : p.vc + (of * p.hd + f) * p.ps + place;
       if (!key) apart = half * p.ps;
     }
-    to[0] = f32_to_bf16(a * turn[i].x - b * turn[i].y);
-    to[apart] = f32_to_bf16(b * turn[i].x + a * turn[i].y);
+    // (values are stored as they are: turned by (1, 0), one that is not finite would take the other along)
+    const bool turns = head < p.nq + p.nkv;
+    to[0] = f32_to_bf16(turns ? a * turn[i].x - b * turn[i].y : a);
+    to[apart] = f32_to_bf16(turns ? b * turn[i].x + a * turn[i].y : b);
   }
 }
 

@@ -203,6 +203,39 @@ def test_projection_of_few_rows_in_slices(k, nq, nkv, hd, ps, bias):
     assert not skinny.takes_slice(8, 4096, w[:, :4096], 32, 8, None) and skinny.takes_slice(8, 4096, w[:, :4096], 32, 16, None)
 
 
+@pytest.mark.parametrize("way", ["slices", "resident", "tiles"])
+def test_values_that_are_not_finite_stay_by_themselves(way):
+    """One infinite and one undefined value channel: every other channel of every head has the bits it has beside two channels of zeros."""
+    from qwen25vl_lite_amd.ops import skinny, tile
+    k, nq, nkv, hd, ps = 256, 2, 2, 128, 16
+    n = (nq + 2 * nkv) * hd
+    for m in (1, 17, 64) if way != "tiles" else (65,):
+        torch.manual_seed(m)
+        x, w = torch.randn(m, k, device="cuda").bfloat16(), (torch.randn(n, k, device="cuda") / 16).bfloat16()
+        cs = torch.rand(m, hd // 2, 2, device="cuda")
+        slots = torch.arange(m, device="cuda", dtype=torch.int32)
+        bad = [(nq + nkv) * hd + 3, (nq + nkv + 1) * hd + hd // 2 + 9]
+        results = []
+        for fill in ((0.0, 0.0), (math.inf, math.nan)):
+            w[bad[0]], w[bad[1]] = fill
+            kc = torch.zeros(m // ps + 1, nkv, ps, hd, dtype=torch.bfloat16, device="cuda")
+            vc = torch.zeros(m // ps + 1, nkv, hd, ps, dtype=torch.bfloat16, device="cuda")
+            if way == "slices":
+                q = skinny.slice_qkv_rope(w, cs, x, None, slots, kc, vc, nq, nkv, hd, ps)
+            elif way == "tiles":
+                q = tile.tile_heads(x, w, None, cs, slots, kc, vc, nq, nkv, ps)
+            else:
+                q = skinny.qkv_rope_product(w, cs, x=x, slots=slots, k_cache=kc, v_cache=vc, num_q_heads=nq, num_kv_heads=nkv,
+                                            head_dim=hd, page_size=ps)
+            v = vc.permute(0, 3, 1, 2).reshape(-1, nkv * hd)[:m]
+            results.append((q, kc, v))
+        (q0, k0, v0), (q1, k1, v1) = results
+        rest = torch.ones(nkv * hd, dtype=torch.bool, device="cuda")
+        rest[[3, hd + hd // 2 + 9]] = False
+        assert torch.equal(q0, q1) and torch.equal(k0, k1) and torch.equal(v0[:, rest], v1[:, rest]), m
+        assert not torch.isfinite(v1[:, ~rest]).any()
+
+
 def test_which_projections_take_the_rotation_with_them():
     from qwen25vl_lite_amd.ops import kernels, tile
     w = torch.empty(4608, 3584, dtype=torch.bfloat16, device="cuda")
