@@ -94,13 +94,13 @@ def tile_slabs(x: torch.Tensor, weight: torch.Tensor, ranges: Optional[int] = No
 
 def prefers_heads(x: torch.Tensor, weight: torch.Tensor, ranges: int, head_dim: int, rot_half: int, *rest: Optional[torch.Tensor]) -> bool:
     """Whether the stacked projection goes through :func:`tile_heads`: heads of 128 channels rotated whole, ``rest`` (bias, cache) on
-    16-byte boundaries, and a product that is not cut along the inner size (``ranges``: :func:`slab_ranges`), or into three ranges at most of an inner
-    size up to 2,048.
+    16-byte boundaries, and a product that is not cut along the inner size (``ranges``: :func:`slab_ranges`).
 
-    Measured, the product (the library's, or slabs) and the rotation's kernel in brackets: 16 + 2 x 2 heads, inner size 2,048, 512 rows 23 us (26, three
-    slabs), 375 rows 23 (23), 256 rows 23 (21, four slabs), 2,048 rows 31 (39); 28 + 2 x 4 heads, 3,584, 512 rows 38 (41), 2,048 rows 70 (82), 4,096 rows 135
-    (162), 375 rows 37 (32, two slabs); 64 + 2 x 8 heads, 8,192, 2,048 rows 303 (326), 512 rows 96 (96, three slabs)."""
-    return ((ranges == 1 or (1 < ranges <= 3 and x.shape[1] <= 2048)) and head_dim == 128 and rot_half == 64
+    Measured, the product (the library's, or slabs) and the rotation's kernel in brackets: 16 + 2 x 2 heads, inner size 2,048, 1,024 rows 23 us (27),
+    2,048 rows 29 (37); 28 + 2 x 4 heads, 3,584, 512 rows 35 (34), 2,048 rows 67 (77), 4,096 rows 127 (151); 32 + 2 x 8 heads, 2,048, 300 rows
+    23.1 (22.2); 64 + 2 x 8 heads, 8,192, 2,048 rows 282 (308).  Products that are cut stay so: in one chain of sums they would take 23 us (25, three
+    slabs; 16 + 2 x 2 heads, 2,048, 512 rows), with an error of 2.7e-7 of the result against 1.5e-7."""
+    return (ranges == 1 and head_dim == 128 and rot_half == 64
             and all(t is None or t.data_ptr() % 16 == 0 for t in rest))
 
 

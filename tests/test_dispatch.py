@@ -155,6 +155,15 @@ def test_walks_that_cannot_be_listed(bad):
         attn.plan_walks([0, 4], kw["lens"], 2, kw["nkv"], 0, kw["places"], kw["groups"], {"HD": 128})
 
 
+@pytest.mark.parametrize("ranges", range(5))
+@pytest.mark.parametrize("k", [512, 2048, 3584, 8192])
+def test_products_that_are_cut_stay_cut(k, ranges):
+    """The projection with the rotation inside sums in one chain: it takes only what has one chain anyway."""
+    from qwen25vl_lite_amd.ops import tile
+    x, w = torch.empty(300, k, dtype=torch.bfloat16), torch.empty(6 * 128, k, dtype=torch.bfloat16)
+    assert tile.prefers_heads(x, w, ranges, 128, 64) == (ranges == 1)
+
+
 def test_which_rows_of_the_stacked_projection_are_cut():
     """17 to 48 rows at any size, up to 64 of large weights beyond the inner size that the kernel with the rotation inside keeps in one
     pass."""
