@@ -209,6 +209,8 @@ extern "C" int qvl_gemm_slice_takes(int M, int N, int K, int cus) {
   return M > 0 && M <= 64 && K > 0 && K % 8 == 0 && K <= SLICE_K(16) && N > 0 && N % 2 == 0 && cus > 0 && N <= 32ll * cus;
 }
 
+extern "C" int qvl_gemm_slice_most_k() { return SLICE_K(16); }
+
 // The stacked projection of nq query, nkv key and nkv value heads of hd channels (hd even) with bias (float32 or null), rotation and cache write:
 // q_out bfloat16 [M, nq hd]; keys and values into their pages, kc [page][nkv][ps][hd], vc [page][nkv][hd][ps] (slot[m] = page * ps
 // + place, or -1).  cs: float32 [M, hd / 2, 2].

@@ -214,13 +214,30 @@ def qkv_rope_product(weight: torch.Tensor, cs: torch.Tensor, *, x: Optional[torc
     return q_out
 
 
+_slice_k = None
+
+
+def _slice_fits(m: int, k: int, n: int, cus: int) -> bool:
+    """The kernel's own rule of sizes (qvl_gemm_slice_takes), which every layer of a step asks: in plain integers, a call of the library takes
+    longer."""
+    global _slice_k
+    if _slice_k is None:
+        _slice_k = int(_fn("gemm_slice", "qvl_gemm_slice_most_k", [])())
+    return 0 < m <= RESIDENT_ROWS and 0 < k <= _slice_k and k % 8 == 0 and 0 < n <= 32 * cus and n % 2 == 0
+
+
 def takes_slice(m: int, k: int, weight: torch.Tensor, head_dim: int, rot_half: int, cache_dtype) -> bool:
     """Whether :func:`slice_qkv_rope` takes the stacked projection of ``m`` rows: bfloat16, a rotation over the whole head, inner sizes up to
-    4,096 and 32 weight rows a compute unit (csrc/gemm_slice.hip).  There it is the fastest way at every number of rows."""
-    if (weight.dtype != torch.bfloat16 or 2 * rot_half != head_dim or cache_dtype not in (None, torch.bfloat16)
-            or not _rows_aligned(weight, 8) or weight.shape[0] * weight.stride(0) * 2 >= 0x7fffff00):
-        return False
-    return bool(_fn("gemm_slice", "qvl_gemm_slice_takes", [_c_int] * 4)(m, weight.shape[0], k, _compute_units(weight.device)))
+    4,096 and 32 weight rows a compute unit (csrc/gemm_slice.hip).  There it is the fastest way at every number of rows (but for 49 rows and more of
+    inner sizes up to 128: 64 rows of 256 x 128 5.6 us, by the resident kernel 4.9)."""
+    return (2 * rot_half == head_dim and cache_dtype in (None, torch.bfloat16)
+            and _slice_fits(m, k, weight.shape[0], _compute_units(weight.device)) and _slice_weight(weight))
+
+
+def _slice_weight(weight: torch.Tensor) -> bool:
+    n, stride = weight.shape[0], weight.stride()
+    return (weight.dtype == torch.bfloat16 and stride[1] == 1 and stride[0] % 8 == 0 and n * stride[0] * 2 < 0x7fffff00
+            and weight.data_ptr() % 16 == 0)
 
 
 def slice_qkv_rope(weight: torch.Tensor, cs: torch.Tensor, x: torch.Tensor, bias: Optional[torch.Tensor], slots: Optional[torch.Tensor],
@@ -229,25 +246,31 @@ def slice_qkv_rope(weight: torch.Tensor, cs: torch.Tensor, x: torch.Tensor, bias
     """As :func:`qkv_rope_product`, where :func:`takes_slice` says so."""
     m, k = x.shape
     nq, nkv, hd = int(num_q_heads), int(num_kv_heads), int(head_dim)
-    if (weight.shape != ((nq + 2 * nkv) * hd, k) or not takes_slice(m, k, weight, hd, cs.shape[1], None) or x.dtype != torch.bfloat16
-            or not _rows_aligned(x, 8) or m * x.stride(0) * 2 >= 0x7fffff00):
+    n, cus, stride = (nq + 2 * nkv) * hd, _compute_units(x.device), x.stride()
+    if (weight.shape != (n, k) or not _slice_fits(m, k, n, cus) or not _slice_weight(weight) or x.dtype != torch.bfloat16
+            or stride[1] != 1 or stride[0] % 8 or m * stride[0] * 2 >= 0x7fffff00 or x.data_ptr() % 16):
         raise ValueError("the kernel does not take this projection")
-    if bias is not None and (bias.dtype != torch.float32 or not bias.is_contiguous() or bias.shape != (weight.shape[0],)):
+    if bias is not None and (bias.dtype != torch.float32 or not bias.is_contiguous() or bias.shape != (n,)):
         raise ValueError("bias must be float32 [(nq + 2 nkv) hd]")
-    if cs.dtype != torch.float32 or cs.dim() != 3 or cs.shape[0] < m or tuple(cs.shape[1:]) != (hd // 2, 2) or not cs.is_contiguous():
+    if cs.dtype != torch.float32 or cs.dim() != 3 or cs.shape[0] < m or cs.shape[1:] != (hd // 2, 2) or not cs.is_contiguous():
         raise ValueError("cs must be float32 [M, hd/2, 2]")
-    if nkv and (slots is None or slots.dtype != torch.int32 or slots.shape != (m,) or not slots.is_contiguous()
+    slots_at = k_at = v_at = None
+    if nkv:
+        if (slots is None or slots.dtype != torch.int32 or slots.shape != (m,) or not slots.is_contiguous()
                 or k_cache is None or v_cache is None or k_cache.dtype != torch.bfloat16 or v_cache.dtype != torch.bfloat16
                 or not k_cache.is_contiguous() or not v_cache.is_contiguous()
-                or tuple(k_cache.shape[1:]) != (nkv, page_size, hd) or tuple(v_cache.shape[1:]) != (nkv, hd, page_size)
+                or k_cache.shape[1:] != (nkv, page_size, hd) or v_cache.shape[1:] != (nkv, hd, page_size)
                 or v_cache.shape[0] != k_cache.shape[0]):
-        raise ValueError("slots int32 [M] and bfloat16 caches [pages, nkv, ps, hd] / [pages, nkv, hd, ps] are needed")
+            raise ValueError("slots int32 [M] and bfloat16 caches [pages, nkv, ps, hd] / [pages, nkv, hd, ps] are needed")
+        slots_at, k_at, v_at = slots.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr()
     q_out = torch.empty((m, nq * hd), dtype=torch.bfloat16, device=x.device)
-    fn = _fn("gemm_slice", "qvl_gemm_slice_rope", [_c_ptr, _c_int, _c_ptr, _c_int] + [_c_ptr] * 6 + [_c_int] * 7 + [_c_ptr])
-    _check(fn(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), _ptr(cs), _ptr(slots if nkv else None), _ptr(q_out),
-              _ptr(k_cache if nkv else None), _ptr(v_cache if nkv else None), m, k, nq, nkv, hd, int(page_size),
-              _compute_units(x.device), _stream()), "linear (slices, rotation and cache write)")
+    fn = _fn("gemm_slice", "qvl_gemm_slice_rope", _SLICE_ARGS)
+    _check(fn(x.data_ptr(), stride[0], weight.data_ptr(), weight.stride(0), _ptr(bias), cs.data_ptr(), slots_at, q_out.data_ptr(), k_at, v_at,
+              m, k, nq, nkv, hd, int(page_size), cus, _stream()), "linear (slices, rotation and cache write)")
     return q_out
+
+
+_SLICE_ARGS = [_c_ptr, _c_int, _c_ptr, _c_int] + [_c_ptr] * 6 + [_c_int] * 7 + [_c_ptr]
 
 
 SPLIT_ROWS = 64   # the most rows that are cut along the inner size

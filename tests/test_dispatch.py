@@ -164,6 +164,26 @@ def test_products_that_are_cut_stay_cut(k, ranges):
     assert tile.prefers_heads(x, w, ranges, 128, 64) == (ranges == 1)
 
 
+def test_slices_are_asked_for_without_the_library(monkeypatch):
+    """Every layer of a step asks: by the kernel's own rule, but in plain integers."""
+    import ctypes
+    from qwen25vl_lite_amd.ops import kernels, skinny
+    rule = kernels._fn("gemm_slice", "qvl_gemm_slice_takes", [ctypes.c_int] * 4)
+    for m in (0, 1, 64, 65):
+        for k in (0, 8, 12, 4088, 4096, 4104):
+            for n in (0, 2, 3, 8190, 8192, 8194, 9728):
+                for cus in (1, 256, 304):
+                    assert skinny._slice_fits(m, k, n, cus) == bool(rule(m, n, k, cus)), (m, k, n, cus)
+    asked = []
+    monkeypatch.setattr(skinny, "_fn", lambda *a, **kw: asked.append(a))
+    monkeypatch.setattr(skinny, "_compute_units", lambda device: 256)
+    w = torch.empty(256, 512, dtype=torch.bfloat16)
+    for weight, head, half, cache, want in ((w, 64, 32, torch.bfloat16, True), (w, 64, 32, None, True), (w, 64, 16, None, False), (w.float(), 64, 32, None, False),
+                                            (w, 64, 32, torch.float32, False), (w[:, 1:], 64, 32, None, False), (w.t(), 64, 32, None, False)):
+        assert skinny.takes_slice(5, weight.shape[1], weight, head, half, cache) == want
+    assert not asked
+
+
 def test_which_rows_of_the_stacked_projection_are_cut():
     """17 to 48 rows at any size, up to 64 of large weights beyond the inner size that the kernel with the rotation inside keeps in one
     pass."""
