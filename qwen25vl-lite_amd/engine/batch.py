@@ -42,6 +42,11 @@ def _align(n: int, a: int = 4) -> int:
     return (n + a - 1) // a * a
 
 
+# A run's page slots are worked out by arrays from this many tokens on, one by one below (eight runs of 5 tokens 176 us of the host so, by arrays 214; one of
+# 16 79 and 84, of 32 84 and 86, of 48 88 and 87, of 128 101 and 90).
+ARRAY_RUN = 40
+
+
 def build_step(entries: Sequence[StepEntry], cache: CacheManager, position_rows: int, dtype: torch.dtype,
                device: torch.device, vocab_size: Optional[int] = None) -> StepContext:
     """Lay out the batch (pages must have been reserved) and copy it to the device."""
@@ -78,7 +83,8 @@ def build_step(entries: Sequence[StepEntry], cache: CacheManager, position_rows:
             raise ValueError(f"request {e.req_id!r}: the cache holds {rp.num_tokens} tokens, "
                              f"the step continues from {e.start}")
         if n == 1 and e.positions is None and vocab_size is not None and type(e.tokens[0]) is int:
-            # a decoded token beside prompt portions, one of many: a store each instead of arrays of one (24 beside a portion of 232, with the portion's slots worked out by arrays, too: 0.4 of the time)
+            # a decoded token beside prompt portions, one of many: a store each instead of arrays of one (24 beside a portion of 232, with the
+            # portion's slots by arrays, too: 208 us of the host for 410)
             start, token = e.start, e.tokens[0]
             if not 0 <= token < vocab_size:
                 raise ValueError(f"request {e.req_id!r}: token id outside [0, {vocab_size})")
@@ -117,10 +123,16 @@ def build_step(entries: Sequence[StepEntry], cache: CacheManager, position_rows:
         ctx_len[i] = e.start + n
         req_slots[i] = rp.slot
         for g, t in enumerate(rp.tables):
-            pages = np.asarray(t, np.int32)
-            tables[g][i, :len(t)] = pages
-            pages = pages[seq // ps]
-            slot_maps[g][at:at + n] = pages * ps + seq % ps if pages.min() >= 0 else cache.slot_mapping(e.req_id, g, e.start, e.start + n)
+            slots = None
+            if n < ARRAY_RUN:
+                tables[g][i, :len(t)] = t
+            else:
+                pages = np.asarray(t, np.int32)
+                tables[g][i, :len(t)] = pages
+                pages = pages[seq // ps]
+                if pages.min() >= 0:
+                    slots = pages * ps + seq % ps
+            slot_maps[g][at:at + n] = cache.slot_mapping(e.req_id, g, e.start, e.start + n) if slots is None else slots
         for w in e.want:
             if not 0 <= int(w) < n:
                 raise ValueError(f"request {e.req_id!r}: wanted place {w} is outside its {n} tokens")

@@ -341,3 +341,24 @@ def test_a_steps_single_tokens_are_laid_out_as_runs_are():
     for kind in (int, np.int64):
         with pytest.raises(RuntimeError, match="given back"):
             step(kind)
+
+
+@pytest.mark.parametrize("n", [2, 39, 40, 41, 130])
+def test_a_runs_slots_one_by_one_and_by_arrays(n):
+    """Runs on both sides of the length from which their slots are worked out by arrays, from the middle of a page."""
+    import torch
+    from qwen25vl_lite_amd.engine import batch
+    assert 39 < batch.ARRAY_RUN <= 41
+    cm = CacheManager([CacheGroupSpec(CacheNeed(1, 8), 1), CacheGroupSpec(CacheNeed(1, 8, 20), 1)], 64, 16, 8, enable_prefix_cache=False)
+    for r in (5, 6):
+        cm.admit(r)
+        cm.reserve(r, 200)
+    cm.commit(6, 21)
+    entries = [batch.StepEntry(5, list(range(n)), 0, [n - 1]), batch.StepEntry(6, list(range(n)), 21)]
+    step = batch.build_step(entries, cm, 1, torch.float32, torch.device("cpu"), 1000)
+    for g in range(2):
+        assert step.groups[g].slot_mapping.tolist() == cm.slot_mapping(5, g, 0, n) + cm.slot_mapping(6, g, 21, 21 + n)
+        assert step.groups[g].block_table.tolist() == [cm.table(5, g), cm.table(6, g)]
+    cm.requests[6].tables[1][(20 + n) // 16] = -1
+    with pytest.raises(RuntimeError, match="given back"):
+        batch.build_step(entries, cm, 1, torch.float32, torch.device("cpu"), 1000)
