@@ -2,6 +2,7 @@
 // rotation + cache write, SwiGLU.  Each works for float32 and bfloat16 storage and any
 // row width; all arithmetic is float32.
 #include "common.h"
+#include <cstring>
 
 // ---------------------------------------------------------------------------------------
 // Embedding gather: out[n, :] = scale * float32(table[ids[n], :])       (reference text.py:213)
@@ -67,21 +68,20 @@ __global__ __launch_bounds__(256) void embed_kernel(EmbedArgs p) {
   }
 }
 
-// inv_freq, freq_row, rotated, rot_half, amplitude: arrays (on the host) of `tables` at most EMBED_TABLES; pos as in qvl_rope_table.
+// rotations: `tables` RotationTable records (host memory, of any alignment), at most EMBED_TABLES; pos as in qvl_rope_table.
 extern "C" int qvl_embed_gather(const void* ids, const void* table, void* out, int N, int H, int V, int dtype, float scale,
-                                const void* pos, int pos_stride, int tables, const void* const* inv_freq, const void* const* freq_row,
-                                void* const* rotated, const int* rot_half, const float* amplitude, hipStream_t stream) {
+                                const void* pos, int pos_stride, int tables, const void* rotations, hipStream_t stream) {
   if (N <= 0) return QVL_OK;
-  if (H <= 0 || V <= 0 || tables < 0 || tables > EMBED_TABLES || (tables && (!pos || pos_stride < N || !inv_freq || !freq_row || !rotated || !rot_half || !amplitude)))
-    return QVL_ERR_SHAPE;
+  if (H <= 0 || V <= 0 || tables < 0 || tables > EMBED_TABLES || (tables && (!pos || pos_stride < N || !rotations))) return QVL_ERR_SHAPE;
   EmbedArgs p;
   p.ids = (const int*)ids; p.table = table; p.out = (float*)out; p.H = H; p.V = V; p.scale = scale; p.pos = (const int*)pos; p.pos_stride = pos_stride;
   for (int t = 0; t < tables; ++t) {
-    if (rot_half[t] < 0) return QVL_ERR_SHAPE;
-    p.tables[t] = RotationTable{(const float*)inv_freq[t], (const int*)freq_row[t], (float2*)rotated[t], rot_half[t], amplitude[t]};
+    memcpy(&p.tables[t], (const char*)rotations + t * sizeof(RotationTable), sizeof(RotationTable));
+    if (p.tables[t].rot_half < 0) return QVL_ERR_SHAPE;
   }
   const dim3 grid(N, 1 + tables);
   const bool aligned = (((uintptr_t)table | (uintptr_t)out) & 15) == 0;
+  static_assert(sizeof(RotationTable) == 32, "three pointers, a count and a factor, as the caller packs them");
   if (dtype == 0) {
     if (aligned && H % 4 == 0) hipLaunchKernelGGL((embed_kernel<float, true>), grid, dim3(256), 0, stream, p);
     else hipLaunchKernelGGL((embed_kernel<float, false>), grid, dim3(256), 0, stream, p);

@@ -8,6 +8,7 @@ There is no CPU path and no library stand-in: a tensor that is not on the GPU is
 from __future__ import annotations
 
 import ctypes
+import struct
 from typing import Dict, Optional, Sequence, Tuple
 
 import torch
@@ -107,6 +108,7 @@ def int32_to_device(host, device) -> torch.Tensor:
 
 # --------------------------------------------------------------------------------------------
 EMBED_TABLES = 4     # as in csrc/elementwise.hip
+_EMBED_ARGS = [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_float, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr]
 
 
 def embed_gather(ids: torch.Tensor, table: torch.Tensor, out: Optional[torch.Tensor] = None, scale: float = 1.0,
@@ -123,18 +125,17 @@ def embed_gather(ids: torch.Tensor, table: torch.Tensor, out: Optional[torch.Ten
     _need(out.dtype == torch.float32 and out.shape == (n, h) and out.is_contiguous(), "out must be float32 [N, H]")
     count = len(rotations)
     _need(count <= EMBED_TABLES and (count == 0 or positions is not None), f"at most {EMBED_TABLES} rotations, with the positions")
-    made, arrays = [], [None] * 5
+    made, records = [], None
     if count:
-        for inv_freq, freq_row, _ in rotations:
+        values = []
+        for inv_freq, freq_row, amplitude in rotations:
             _check_rotation(positions, inv_freq, freq_row, n)
             made.append(torch.empty((n, inv_freq.shape[0], 2), dtype=torch.float32, device=table.device))
-        arrays = [(_c_ptr * count)(*(_ptr(r[0]) for r in rotations)), (_c_ptr * count)(*(_ptr(r[1]) for r in rotations)),
-                  (_c_ptr * count)(*(_ptr(t) for t in made)), (_c_int * count)(*(t.shape[1] for t in made)),
-                  (_c_float * count)(*(float(r[2]) for r in rotations))]
-    fn = _fn("elementwise", "qvl_embed_gather", [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_float, _c_ptr, _c_int, _c_int]
-             + [_c_ptr] * 6)
+            values += (inv_freq.data_ptr(), freq_row.data_ptr(), made[-1].data_ptr(), inv_freq.shape[0], amplitude)
+        records = struct.pack("=" + "QQQif" * count, *values)      # RotationTable of the source
+    fn = _fn("elementwise", "qvl_embed_gather", _EMBED_ARGS)
     _check(fn(_ptr(ids), _ptr(table), _ptr(out), n, h, v, dtype_code(table.dtype), float(scale), _ptr(positions) if count else None,
-              positions.stride(0) if count else 0, count, *arrays, _stream()), "embed_gather")
+              positions.stride(0) if count else 0, count, records, _stream()), "embed_gather")
     return (out, made) if count else out
 
 
