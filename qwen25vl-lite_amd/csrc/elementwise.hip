@@ -41,8 +41,13 @@ __device__ __forceinline__ void rotation_row(const RotationTable& t, const int* 
   }
 }
 
-// grid (N, 1 + tables).  WIDE: 16 bytes of a row at a time (rows and their number of values allow it).
-template <typename T, bool WIDE>
+template <typename T> struct norm_raw;      // four values as they lie
+template <> struct norm_raw<float> { typedef float4 type; };
+template <> struct norm_raw<bf16_t> { typedef uint2 type; };
+
+// grid (N, 1 + tables).  E: values of a row that a thread takes at a time.  Eight of bfloat16 wait for memory half as often, four let a wave's
+// stores fill whole lines: of 3,584 values 64 rows 2.43 us and 2.52, 512 rows 3.84 and 3.49, 2,048 rows 9.2 and 7.6 (9.0 one by one).
+template <typename T, int E>
 __global__ __launch_bounds__(256) void embed_kernel(EmbedArgs p) {
   const int n = blockIdx.x;
   if (blockIdx.y > 0) {
@@ -53,20 +58,21 @@ __global__ __launch_bounds__(256) void embed_kernel(EmbedArgs p) {
   id = id < 0 ? 0 : (id >= p.V ? p.V - 1 : id);  // ids are validated on the host; never read outside the table
   const T* row = reinterpret_cast<const T*>(p.table) + (size_t)id * p.H;
   float* o = p.out + (size_t)n * p.H;
-  if constexpr (WIDE) {
-    constexpr int E = 16 / sizeof(T);
+  if constexpr (E > 1) {
+#pragma unroll 4
     for (int i = threadIdx.x * E; i < p.H; i += 256 * E) {
-      const uint4 v = *reinterpret_cast<const uint4*>(row + i);
-      const T* e = reinterpret_cast<const T*>(&v);
+      struct __attribute__((aligned(E * sizeof(T)))) Values { T v[E]; };
+      const Values e = *reinterpret_cast<const Values*>(row + i);
 #pragma unroll
       for (int k = 0; k < E; k += 4)
-        *reinterpret_cast<float4*>(o + i + k) = float4{ldf<T>(e + k) * p.scale, ldf<T>(e + k + 1) * p.scale, ldf<T>(e + k + 2) * p.scale,
-                                                       ldf<T>(e + k + 3) * p.scale};
+        *reinterpret_cast<float4*>(o + i + k) = float4{ldf<T>(e.v + k) * p.scale, ldf<T>(e.v + k + 1) * p.scale, ldf<T>(e.v + k + 2) * p.scale,
+                                                       ldf<T>(e.v + k + 3) * p.scale};
     }
   } else {
     for (int i = threadIdx.x; i < p.H; i += 256) o[i] = ldf<T>(row + i) * p.scale;
   }
 }
+#define EMBED_MANY 256      // rows from which four values at a time are faster
 
 // rotations: `tables` RotationTable records (host memory, of any alignment), at most EMBED_TABLES; pos as in qvl_rope_table.
 extern "C" int qvl_embed_gather(const void* ids, const void* table, void* out, int N, int H, int V, int dtype, float scale,
@@ -75,22 +81,25 @@ extern "C" int qvl_embed_gather(const void* ids, const void* table, void* out, i
   if (H <= 0 || V <= 0 || tables < 0 || tables > EMBED_TABLES || (tables && (!pos || pos_stride < N || !rotations))) return QVL_ERR_SHAPE;
   EmbedArgs p;
   p.ids = (const int*)ids; p.table = table; p.out = (float*)out; p.H = H; p.V = V; p.scale = scale; p.pos = (const int*)pos; p.pos_stride = pos_stride;
+  static_assert(sizeof(RotationTable) == 32, "three pointers, a count and a factor, as the caller packs them");
   for (int t = 0; t < tables; ++t) {
     memcpy(&p.tables[t], (const char*)rotations + t * sizeof(RotationTable), sizeof(RotationTable));
     if (p.tables[t].rot_half < 0) return QVL_ERR_SHAPE;
   }
   const dim3 grid(N, 1 + tables);
   const bool aligned = (((uintptr_t)table | (uintptr_t)out) & 15) == 0;
-  static_assert(sizeof(RotationTable) == 32, "three pointers, a count and a factor, as the caller packs them");
+#define GO(T, E) hipLaunchKernelGGL((embed_kernel<T, E>), grid, dim3(256), 0, stream, p)
   if (dtype == 0) {
-    if (aligned && H % 4 == 0) hipLaunchKernelGGL((embed_kernel<float, true>), grid, dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL((embed_kernel<float, false>), grid, dim3(256), 0, stream, p);
+    if (aligned && H % 4 == 0) GO(float, 4);
+    else GO(float, 1);
   } else if (dtype == 1) {
-    if (aligned && H % 8 == 0) hipLaunchKernelGGL((embed_kernel<bf16_t, true>), grid, dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL((embed_kernel<bf16_t, false>), grid, dim3(256), 0, stream, p);
+    if (aligned && H % 8 == 0 && N < EMBED_MANY) GO(bf16_t, 8);
+    else if (aligned && H % 4 == 0) GO(bf16_t, 4);
+    else GO(bf16_t, 1);
   } else {
     return QVL_ERR_DTYPE;
   }
+#undef GO
   return qvl_launch_status();
 }
 
@@ -167,9 +176,6 @@ __device__ __forceinline__ float norm_total(const float* sums) {
 // addend in slabs (float32), one slab at a time, in order.
 // Bytes bound it from about a thousand rows on: 4,096 rows of 3,584 with a bfloat16 addend 28.5 -> 26.9 us, 6.6 TB/s; below, latency: 64
 // rows of 8,192 7.4 -> 5.4, when the loads waited for each other's stores and the weights for the sum.
-template <typename T> struct norm_raw;
-template <> struct norm_raw<float> { typedef float4 type; };
-template <> struct norm_raw<bf16_t> { typedef uint2 type; };
 __device__ __forceinline__ float4 norm_value(float4 v) { return v; }
 __device__ __forceinline__ float4 norm_value(uint2 v) {
   return float4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),

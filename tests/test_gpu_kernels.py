@@ -72,6 +72,17 @@ def test_add_rmsnorm_of_few_and_many_rows(width, slabs):
     assert ((out.cpu().double() - want).abs() <= (bound + rel * total.abs()) / torch.sqrt(total.pow(2).mean(1, keepdim=True)) * w.abs().double()).all()
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width", [16, 2052, 3584])
+def test_embed_gather_on_both_sides_of_many_rows(width, dtype):
+    from qwen25vl_lite_amd.ops import kernels
+    torch.manual_seed(width)
+    table = torch.randn(30, width).to(dtype).cuda()
+    for n in (255, 256):
+        ids = torch.randint(0, 30, (n,), dtype=torch.int32).cuda()
+        assert torch.equal(kernels.embed_gather(ids, table, scale=0.5), table[ids.long()].float() * 0.5)
+
+
 @pytest.mark.parametrize("width", [97, 3584, 8200])
 @pytest.mark.parametrize("delta_dtype, out_dtype", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16),
                                                     (torch.bfloat16, torch.bfloat16), (None, torch.bfloat16)])
