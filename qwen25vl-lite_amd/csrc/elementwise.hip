@@ -147,6 +147,7 @@ __global__ void add_rmsnorm_kernel(float* __restrict__ h, const TD* __restrict__
 // The same with every value held in registers between the two passes: rows whose width is a
 // multiple of 4 and at most NORM_VEC_MAX * 4 * 256, read and written 4 values at a time.
 #define NORM_VEC_MAX 8
+#define NORM_ROWS 512      // many rows, for which the kernels below are made differently
 
 __device__ __forceinline__ float4 ld4(const float* p) { return *reinterpret_cast<const float4*>(p); }
 template <typename T> __device__ __forceinline__ void st4(T* p, float4 v);
@@ -176,13 +177,16 @@ __device__ __forceinline__ float norm_total(const float* sums) {
 // addend in slabs (float32), one slab at a time, in order.
 // Bytes bound it from about a thousand rows on: 4,096 rows of 3,584 with a bfloat16 addend 28.5 -> 26.9 us, 6.6 TB/s; below, latency: 64
 // rows of 8,192 7.4 -> 5.4, when the loads waited for each other's stores and the weights for the sum.
+// LATE, for NORM_ROWS rows or more of more than 4,096 values: four pieces at a time and the weights behind the sum.  Asked for at once, eight
+// pieces take 145 registers, three waves a SIMD, and the memory idles (with a bfloat16 addend 1,024 x 5,120 13.8 us, 10.0 so; 1,024 x 8,192 19.9
+// and 17.2; without one 4,096 x 8,192 40.0 and 33.1).
 __device__ __forceinline__ float4 norm_value(float4 v) { return v; }
 __device__ __forceinline__ float4 norm_value(uint2 v) {
   return float4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
                 __uint_as_float(v.y & 0xffff0000u)};
 }
 
-template <typename TD, typename TO, int VEC>
+template <typename TD, typename TO, int VEC, bool LATE>
 __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict__ h, const TD* __restrict__ delta,
                                                               const float* __restrict__ w, TO* __restrict__ out,
                                                               const int* __restrict__ rows, int H, float eps, int nslabs,
@@ -194,38 +198,44 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict_
   const int row = rows ? rows[m] : m;
   float* hr = h + (size_t)row * H;
   const int nvec = H >> 2;
+  constexpr int STEP = LATE ? 4 : VEC;      // pieces asked for at once
   int at[VEC];
   float4 v[VEC], g[VEC];
 #pragma unroll
-  for (int j = 0; j < VEC; ++j) {
-    at[j] = 4 * min((int)threadIdx.x + 256 * j, nvec - 1);
-    v[j] = ld4(hr + at[j]);
-  }
-  if (delta) {
+  for (int j = 0; j < VEC; ++j) at[j] = 4 * min((int)threadIdx.x + 256 * j, nvec - 1);
+#pragma unroll
+  for (int j0 = 0; j0 < VEC; j0 += STEP) {
+    const int j1 = j0 + STEP < VEC ? j0 + STEP : VEC;
+#pragma unroll
+    for (int j = j0; j < j1; ++j) v[j] = ld4(hr + at[j]);
+    if (!delta) continue;
     const TD* dr = delta + (size_t)row * H;
     Raw d[VEC];
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) d[j] = *reinterpret_cast<const Raw*>(dr + at[j]);
+    for (int j = j0; j < j1; ++j) d[j] = *reinterpret_cast<const Raw*>(dr + at[j]);
     float4 sum[VEC];
+    if (!LATE) {
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) g[j] = ld4(w + at[j]);
+      for (int j = j0; j < j1; ++j) g[j] = ld4(w + at[j]);
+    }
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) sum[j] = norm_value(d[j]);
+    for (int j = j0; j < j1; ++j) sum[j] = norm_value(d[j]);
     for (int c = 1; c < nslabs; ++c) {
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) d[j] = *reinterpret_cast<const Raw*>(dr + (size_t)c * slab_stride + at[j]);
+      for (int j = j0; j < j1; ++j) d[j] = *reinterpret_cast<const Raw*>(dr + (size_t)c * slab_stride + at[j]);
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) {
+      for (int j = j0; j < j1; ++j) {
         const float4 e = norm_value(d[j]);
         sum[j].x += e.x; sum[j].y += e.y; sum[j].z += e.z; sum[j].w += e.w;
       }
     }
 #pragma unroll
-    for (int j = 0; j < VEC; ++j) {
+    for (int j = j0; j < j1; ++j) {
       v[j].x += sum[j].x; v[j].y += sum[j].y; v[j].z += sum[j].z; v[j].w += sum[j].w;
       if (!rows && (int)threadIdx.x + 256 * j < nvec) st4<float>(hr + at[j], v[j]);
     }
-  } else {
+  }
+  if (!delta && !LATE) {
 #pragma unroll
     for (int j = 0; j < VEC; ++j) g[j] = ld4(w + at[j]);
   }
@@ -242,9 +252,17 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict_
   const float rs = 1.0f / sqrtf(norm_total<4 * PART>(sums) / (float)H + eps);
   TO* o = out + (size_t)m * H;
 #pragma unroll
-  for (int j = 0; j < VEC; ++j) {
-    if ((int)threadIdx.x + 256 * j < nvec)
-      st4<TO>(o + at[j], float4{(v[j].x * rs) * g[j].x, (v[j].y * rs) * g[j].y, (v[j].z * rs) * g[j].z, (v[j].w * rs) * g[j].w});
+  for (int j0 = 0; j0 < VEC; j0 += STEP) {
+    const int j1 = j0 + STEP < VEC ? j0 + STEP : VEC;
+    if (LATE) {
+#pragma unroll
+      for (int j = j0; j < j1; ++j) g[j] = ld4(w + at[j]);
+    }
+#pragma unroll
+    for (int j = j0; j < j1; ++j) {
+      if ((int)threadIdx.x + 256 * j < nvec)
+        st4<TO>(o + at[j], float4{(v[j].x * rs) * g[j].x, (v[j].y * rs) * g[j].y, (v[j].z * rs) * g[j].z, (v[j].w * rs) * g[j].w});
+    }
   }
 }
 
@@ -254,7 +272,6 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict_
 // above (3,584 values, eight slabs: 64 rows 4.1 us and 5.0, 256 rows 5.3 and 7.0), and rows of 8,192 once, when their second half was
 // asked for behind the store of the first 6.9 us of 64 rows and four slabs, now 5.1.  Many rows are bound by bytes: blocks of 1024 threads
 // that are all at the same point leave the memory idle (of two slabs 512 rows 7.4 and 6.0, 2,048 rows 26.5 and 20.8).
-#define NORM_ROWS 512
 template <typename TO, int VEC>
 __global__ __launch_bounds__(1024) void add_rmsnorm_slabs_kernel(float* __restrict__ h, const float* __restrict__ delta,
                                                                  const float* __restrict__ w, TO* __restrict__ out,
@@ -333,15 +350,19 @@ extern "C" int qvl_add_rmsnorm(void* h, const void* delta, const void* w, void* 
 #undef QVL_NORM_SLABS
     return qvl_launch_status();
   }
-#define QVL_NORM_VEC(TD, TO, VEC)                                                                                  \
-  hipLaunchKernelGGL((add_rmsnorm_vec_kernel<TD, TO, VEC>), dim3(M), dim3(256), 0, stream, (float*)h,              \
+#define QVL_NORM_VEC(TD, TO, VEC, LATE)                                                                            \
+  hipLaunchKernelGGL((add_rmsnorm_vec_kernel<TD, TO, VEC, LATE>), dim3(M), dim3(256), 0, stream, (float*)h,        \
                      (const TD*)delta, (const float*)w, (TO*)out, (const int*)rows, H, eps, nslabs, slab_stride)
 #define QVL_NORM_CASE(DD, OD, TD, TO)                                                                              \
   if (delta_dtype == DD && out_dtype == OD) {                                                                      \
-    if (vec && H <= 1024) QVL_NORM_VEC(TD, TO, 1);                                                                 \
-    else if (vec && H <= 2048) QVL_NORM_VEC(TD, TO, 2);                                                            \
-    else if (vec && H <= 4096) QVL_NORM_VEC(TD, TO, 4);                                                            \
-    else if (vec) QVL_NORM_VEC(TD, TO, NORM_VEC_MAX);                                                              \
+    if (vec && H <= 1024) QVL_NORM_VEC(TD, TO, 1, false);                                                          \
+    else if (vec && H <= 2048) QVL_NORM_VEC(TD, TO, 2, false);                                                     \
+    else if (vec && H <= 4096) QVL_NORM_VEC(TD, TO, 4, false);                                                     \
+    else if (vec && M < NORM_ROWS) QVL_NORM_VEC(TD, TO, 8, false);                                                 \
+    else if (vec && H <= 5120) QVL_NORM_VEC(TD, TO, 5, true);                                                      \
+    else if (vec && H <= 6144) QVL_NORM_VEC(TD, TO, 6, true);                                                      \
+    else if (vec && H <= 7168) QVL_NORM_VEC(TD, TO, 7, true);                                                      \
+    else if (vec) QVL_NORM_VEC(TD, TO, 8, true);                                                                   \
     else                                                                                                           \
       hipLaunchKernelGGL((add_rmsnorm_kernel<TD, TO>), dim3(M), dim3(threads), 0, stream, (float*)h,               \
                          (const TD*)delta, (const float*)w, (TO*)out, (const int*)rows, H, eps, nslabs,            \

@@ -72,6 +72,12 @@ def test_add_rmsnorm_of_few_and_many_rows(width, slabs):
     assert ((out.cpu().double() - want).abs() <= (bound + rel * total.abs()) / torch.sqrt(total.pow(2).mean(1, keepdim=True)) * w.abs().double()).all()
 
 
+@pytest.mark.parametrize("width, slabs", [(256, 17), (1024, 16), (5120, 3), (5124, 1), (6144, 2), (6148, 1), (7168, 5), (7172, 1)])
+def test_add_rmsnorm_of_few_and_many_rows_of_other_widths(width, slabs):
+    """Rows that leave waves of the slabs' kernel without a piece, and all numbers of pieces of many wide rows."""
+    test_add_rmsnorm_of_few_and_many_rows(width, slabs)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("width", [16, 2052, 3584])
 def test_embed_gather_on_both_sides_of_many_rows(width, dtype):
