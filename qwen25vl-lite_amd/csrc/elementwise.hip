@@ -267,54 +267,58 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict_
 }
 
 // The addend as slabs of partial sums (float32 [slab][row][H]) for fewer than NORM_ROWS rows: a block of 1024 threads per row, a thread
-// per 4 or 8 values, the loads of up to sixteen slabs asked for at a time (they do not depend on each other, only the sum has an
-// order: slab 0, 1, 2, ...).  Latency bounds it: fewer rows than fill the chip wait for memory once here and once a slab in the kernel
-// above (3,584 values, eight slabs: 64 rows 4.1 us and 5.0, 256 rows 5.3 and 7.0), and rows of 8,192 once, when their second half was
-// asked for behind the store of the first 6.9 us of 64 rows and four slabs, now 5.1.  Many rows are bound by bytes: blocks of 1024 threads
-// that are all at the same point leave the memory idle (of two slabs 512 rows 7.4 and 6.0, 2,048 rows 26.5 and 20.8).
+// per 4 values (rows of up to 4,096) or 8.  The loads of ONCE slabs are asked for at a time, sixteen of one piece, four of two (they do not
+// depend on each other, only the sum has an order: slab 0, 1, 2, ...), with the first of them the rows of h and w.  Latency bounds it:
+// fewer rows than fill the chip wait for memory once for every ONCE slabs here and once a slab in the kernel above (3,584 values, eight slabs:
+// 64 rows 4.1 us and 5.0, 256 rows 5.6 and 7.0).  Threads past a row of up to 4,096 leave as waves: a condition at every load took 0.5 us (1,024
+// values, 64 rows 4.2 us, 3.0 so).  Sixteen loads of two pieces, eight slabs, do not fit the registers (rows of 8,192, four slabs, 64 of them
+// 5.8 us and 5.0; of 5,120, eight slabs, 6.5 and 5.4).
+// Many rows are bound by bytes: blocks of 1024 threads that are all at the same point leave the memory idle (of two slabs 512 rows 7.4
+// and 6.0, 2,048 rows 26.5 and 20.8).
 template <typename TO, int VEC>
 __global__ __launch_bounds__(1024) void add_rmsnorm_slabs_kernel(float* __restrict__ h, const float* __restrict__ delta,
                                                                  const float* __restrict__ w, TO* __restrict__ out,
                                                                  const int* __restrict__ rows, int H, float eps,
                                                                  int nslabs, long long slab_stride) {
-  constexpr int ONCE = VEC == 1 ? 16 : 4;      // slabs asked for at once (eight of two pieces: 8,192 values, one row 6.4 us for 5.4)
+  constexpr int ONCE = VEC == 1 ? 16 : 4;
   __shared__ __attribute__((aligned(16))) float sums[16];
   const int m = blockIdx.x;
   const int row = rows ? rows[m] : m;
   float* hr = h + (size_t)row * H;
   const float* dr = delta + (size_t)row * H;
-  const float4 zero = {0.f, 0.f, 0.f, 0.f};
   int at[VEC];
-  float4 v[VEC], g[VEC], d[VEC];
-  // everything the thread needs is asked for before anything is waited for: the row of h, the
-  // norm's weights and up to 16 pieces of slabs
-#pragma unroll
-  for (int j = 0; j < VEC; ++j) {
-    at[j] = 4 * ((int)threadIdx.x + 1024 * j);
-    v[j] = at[j] < H ? ld4(hr + at[j]) : zero;
-    g[j] = at[j] < H ? ld4(w + at[j]) : zero;
-    d[j] = zero;
-  }
-  for (int c0 = 0; c0 < nslabs; c0 += ONCE) {
-    float4 e[ONCE][VEC];
-#pragma unroll
-    for (int c = 0; c < ONCE; ++c)
-#pragma unroll
-      for (int j = 0; j < VEC; ++j)
-        e[c][j] = c0 + c < nslabs && at[j] < H ? ld4(dr + (size_t)(c0 + c) * slab_stride + at[j]) : zero;
-#pragma unroll
-    for (int c = 0; c < ONCE; ++c)
-#pragma unroll
-      for (int j = 0; j < VEC; ++j)
-        if (c0 + c < nslabs) { d[j].x += e[c][j].x; d[j].y += e[c][j].y; d[j].z += e[c][j].z; d[j].w += e[c][j].w; }
-  }
+  float4 v[VEC], g[VEC];
   float ss = 0.f;
+  if (VEC > 1 || 4 * (int)threadIdx.x < H) {      // (pieces past the end of a row of more than 4,096 read its last one)
 #pragma unroll
-  for (int j = 0; j < VEC; ++j) {
-    v[j].x += d[j].x; v[j].y += d[j].y; v[j].z += d[j].z; v[j].w += d[j].w;
-    if (at[j] < H) {
-      if (!rows) st4<float>(hr + at[j], v[j]);
-      ss = add_squares(ss, v[j]);
+    for (int j = 0; j < VEC; ++j) {
+      at[j] = min(4 * ((int)threadIdx.x + 1024 * j), H - 4);
+      v[j] = ld4(hr + at[j]);
+      g[j] = ld4(w + at[j]);
+    }
+    float4 d[VEC];
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) d[j] = float4{0.f, 0.f, 0.f, 0.f};
+    for (int c0 = 0; c0 < nslabs; c0 += ONCE) {
+      float4 e[ONCE][VEC];
+#pragma unroll
+      for (int c = 0; c < ONCE; ++c)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j)
+          e[c][j] = c0 + c < nslabs ? ld4(dr + (size_t)(c0 + c) * slab_stride + at[j]) : float4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < ONCE; ++c)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j)
+          if (c0 + c < nslabs) { d[j].x += e[c][j].x; d[j].y += e[c][j].y; d[j].z += e[c][j].z; d[j].w += e[c][j].w; }
+    }
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      v[j].x += d[j].x; v[j].y += d[j].y; v[j].z += d[j].z; v[j].w += d[j].w;
+      if (4 * ((int)threadIdx.x + 1024 * j) < H) {
+        if (!rows) st4<float>(hr + at[j], v[j]);
+        ss = add_squares(ss, v[j]);
+      }
     }
   }
   ss = wave_sum(ss);
@@ -324,7 +328,7 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_slabs_kernel(float* __restri
   TO* o = out + (size_t)m * H;
 #pragma unroll
   for (int j = 0; j < VEC; ++j) {
-    if (at[j] < H)
+    if (4 * ((int)threadIdx.x + 1024 * j) < H)
       st4<TO>(o + at[j], float4{(v[j].x * rs) * g[j].x, (v[j].y * rs) * g[j].y, (v[j].z * rs) * g[j].z, (v[j].w * rs) * g[j].w});
   }
 }
