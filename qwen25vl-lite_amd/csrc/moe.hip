@@ -103,7 +103,6 @@ __device__ __forceinline__ void route_token(const RouteArgs& p, int n, float* s,
       allowed_group = ahead < p.keep;
     }
     allowed = __ballot(allowed_group);
-    __builtin_amdgcn_wave_barrier();      // (the next token's scores go to the same place)
   }
   // a score of -1 can never be chosen before an allowed one
 #pragma unroll
@@ -197,14 +196,16 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(const int* __restrict__ 
   sort_block(sh, ids, sorted, offsets, P, E);
 }
 
-// Both for the few tokens of a decode step, one block: 8 tokens of 32 experts, six of them, 9.9 us and 4.8 in two launches as they were.
-#define ROUTE_SORT_TOKENS 64
+// Both for a few tokens, one block, which saves a launch: 8 tokens of 32 experts, six of them, 5.6 us and 5.8 in two.  Up to eight, two of the block's
+// waves a SIMD: more share a SIMD, or come one after another, where routing by itself has a block for every four (16 tokens 6.8 us and 5.8, 64
+// 16.9 and 6.0; of 256 experts in 8 groups 8 tokens 10.7 and 10.8, 16 12.5 and 11.0, 64 35.6 and 11.3).
+#define ROUTE_SORT_TOKENS 8
 __global__ __launch_bounds__(1024) void moe_route_sort_kernel(RouteArgs p, int* __restrict__ sorted, int* __restrict__ offsets) {
-  __shared__ float s_all[16][MOE_MAX_E];
-  __shared__ float g_all[16][64];
+  __shared__ float s_all[ROUTE_SORT_TOKENS][MOE_MAX_E];
+  __shared__ float g_all[ROUTE_SORT_TOKENS][64];
   __shared__ SortSpace sh;
   const int wave = threadIdx.x >> 6;
-  for (int n = wave; n < p.N; n += 16) route_token(p, n, s_all[wave], g_all[wave]);
+  if (wave < ROUTE_SORT_TOKENS && wave < p.N) route_token(p, wave, s_all[wave], g_all[wave]);
   __syncthreads();      // (a block's stores are seen by all of it)
   sort_block(sh, p.ids, sorted, offsets, p.N * p.top, p.E);
 }
@@ -214,6 +215,9 @@ static int route_check(const RouteArgs& p) {
     return QVL_ERR_SHAPE;
   return p.E > MOE_MAX_E || p.groups > 64 || p.top > 64 ? QVL_ERR_LIMIT : QVL_OK;
 }
+
+// Tokens that are routed and listed in one launch.
+extern "C" int qvl_moe_route_rows() { return ROUTE_SORT_TOKENS; }
 
 // sorted, offsets: null, or also the pairs by expert as qvl_moe_sort gives them.
 extern "C" int qvl_moe_route(const void* z, void* ids, void* wts, void* sorted, void* offsets, int N, int E, int top, int groups, int keep,

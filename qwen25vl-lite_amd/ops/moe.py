@@ -37,7 +37,7 @@ def route(logits: torch.Tensor, top: int, groups: int = 1, keep: int = 1, scale:
 
 def route_sorted(logits: torch.Tensor, top: int, groups: int = 1, keep: int = 1, scale: float = 1.0, score: str = "sigmoid",
                  normalize: bool = True, floor: float = 1e-20) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
-    """``(chosen, weights, order, offsets)``: :func:`route` and :func:`sort_pairs` of what it chose, in one launch up to 64 rows."""
+    """``(chosen, weights, order, offsets)``: :func:`route` and :func:`sort_pairs` of what it chose, in one launch up to 8 rows."""
     return _route(logits, top, groups, keep, scale, score, normalize, floor, True)
 
 

@@ -184,6 +184,12 @@ def test_slices_are_asked_for_without_the_library(monkeypatch):
     assert not asked
 
 
+def test_no_wave_routes_two_tokens_in_one_launch():
+    """Routing and listing in one block of sixteen waves: a token for each of half of them at most."""
+    from qwen25vl_lite_amd.ops import kernels
+    assert 1 <= kernels._fn("moe", "qvl_moe_route_rows", [])() <= 8
+
+
 def test_which_rows_of_the_stacked_projection_are_cut():
     """17 to 48 rows at any size, up to 64 of large weights beyond the inner size that the kernel with the rotation inside keeps in one
     pass."""

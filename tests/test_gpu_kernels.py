@@ -1005,6 +1005,20 @@ def test_routes_listed_by_expert(e, top, groups, keep, score):
         assert torch.equal(again[0], ids) and torch.equal(again[1], wts)
 
 
+@pytest.mark.parametrize("e, top, groups, keep", [(1, 1, 1, 1), (70, 64, 1, 1), (512, 8, 8, 4)])
+def test_routes_listed_on_both_sides_of_one_launch(e, top, groups, keep):
+    from qwen25vl_lite_amd.ops import moe
+    for n in (1, 7, 8, 9, 16):
+        torch.manual_seed(n)
+        z = torch.randn(n, e, device="cuda")
+        ids, wts, order, offsets = moe.route_sorted(z, top, groups, keep, 1.5)
+        again = moe.route(z, top, groups, keep, 1.5)
+        assert torch.equal(again[0], ids) and torch.equal(again[1], wts)
+        flat = ids.view(-1).long()
+        assert torch.equal(offsets.long(), torch.cat([torch.zeros(1, device="cuda").long(), torch.bincount(flat, minlength=e).cumsum(0)]))
+        assert torch.equal(order.long().sort().values, torch.arange(n * top, device="cuda")) and torch.equal(flat[order.long()], flat.sort().values)
+
+
 @pytest.mark.parametrize("e, r, k, pairs", [(3, 40, 72, "one"), (8, 300, 200, "uneven"), (70, 129, 64, "uneven"), (4, 2368, 136, "all on one"),
                                             (200, 1, 8, "uneven"), (32, 520, 2056, "few")])
 def test_experts_with_few_pairs(e, r, k, pairs):
