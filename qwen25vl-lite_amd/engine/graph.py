@@ -99,7 +99,7 @@ class _Graph:
             req_slots=d("req_slots"),
             groups=[GroupStep(d(f"slots{g}"), d(f"table{g}", (b, w)), self.ps) for g in range(self.ngroups)],
             logit_rows=d("logit_rows"), cu_q_host=list(range(b + 1)), ctx_len_host=[ctx_bucket] * b,
-            req_slots_host=[0] * b, max_q_len=1, max_ctx_len=ctx_bucket, dtype=parts.dtype)
+            req_slots_host=[0] * b, max_q_len=1, max_ctx_len=ctx_bucket, lengths_known=False, dtype=parts.dtype)
         self.graph = None
         self.logits = None
 

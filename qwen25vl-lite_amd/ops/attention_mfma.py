@@ -150,8 +150,10 @@ class BlockPlan(NamedTuple):
     head_walks: int
 
 
-def plan_walks(cu_q, ctx_len, group: int, nkv: int, window: int, places: int, groups: int, defines: dict, only=None) -> BlockPlan:
-    """The walks of a step's runs of column tiles, cut where that keeps more of ``places`` workgroups of ``groups`` wave groups busy."""
+def plan_walks(cu_q, ctx_len, group: int, nkv: int, window: int, places: int, groups: int, defines: dict, only=None,
+               cut: bool = True) -> BlockPlan:
+    """The walks of a step's runs of column tiles, cut where that keeps more of ``places`` workgroups of ``groups`` wave groups busy
+    (``cut``: whether any may be)."""
     cu = np.ascontiguousarray(cu_q, dtype=np.int32)
     ctx = np.ascontiguousarray(ctx_len, dtype=np.int32)
     keep = None if only is None else np.ascontiguousarray(only, dtype=np.uint8)
@@ -161,7 +163,7 @@ def plan_walks(cu_q, ctx_len, group: int, nkv: int, window: int, places: int, gr
     out, head = np.empty((room, 8), dtype=np.int32), np.zeros(6, dtype=np.int32)
     fn = _fn("attention_mfma", "qvl_attn_mfma_block_plan", [_c_ptr] * 3 + [_c_int] * 7 + [_c_ptr, _c_ll, _c_ptr], defines)
     _check(fn(cu.ctypes.data, ctx.ctypes.data, None if keep is None else keep.ctypes.data, len(ctx), group, nkv, window, places,
-              groups, CUT_WALKS, out.ctypes.data, room, head.ctypes.data), "paged_attention (plan of the walks)")
+              groups, CUT_WALKS if cut else 0, out.ctypes.data, room, head.ctypes.data), "paged_attention (plan of the walks)")
     grid, count, taken_places, partials, head_slots, head_walks = (int(x) for x in head)
     return BlockPlan(out[:count], grid, taken_places, partials, head_slots, head_walks)
 
@@ -205,7 +207,11 @@ def _walk_blocks(step, group: int, tile_ct: int, only=None) -> int:
 
 def _step_walks(step, group: int, nkv: int, hd: int, window: int, device, only=None, force_wide=None, force_groups=None):
     """``(wide, wave groups, defines, plan, its items on the device)`` of the step's prompt portions, the same for every layer with
-    these heads."""
+    these heads.
+
+    A step that is captured for contexts of up to some length has walks of lengths that nobody knows yet.  They stay whole and are taken by
+    tickets: cut as if all were as long as they may become, most parts would be empty (28 + 2 x 4 heads of 128, 200 decoded tokens at 275 to
+    1,100 keys, captured for 2,048: 78 us, whole 57; at 450 to 1,800 116 and 103; 160 with 16 + 2 x 4 heads of 256 at 70 to 280, for 512: 42 and 33)."""
     key = ("walks", group, nkv, hd, window, only, force_wide, force_groups)
     if key in step.derived:
         return step.derived[key]
@@ -218,10 +224,12 @@ def _step_walks(step, group: int, nkv: int, hd: int, window: int, device, only=N
                 and _walk_blocks(step, group, block_tiles(hd, True), only) * WIDE_CT <= 1.04 * 2 * blocks)
     defines = block_defines(hd, wide)
     per_cu = int(_fn("attention_mfma", "qvl_attn_mfma_block_per_cu", [], defines)())
+    known = getattr(step, "lengths_known", True)
     groups = force_groups
     if groups is None:
-        groups = block_groups(num_tiles * nkv, cus * per_cu, hd) if not wide and blocks >= GROUPS_WALK_BLOCKS * num_tiles else 1
-    plan = plan_walks(step.cu_q_host, step.ctx_len_host, group, nkv, window, cus * (per_cu if groups == 1 else 1), groups, defines, only)
+        groups = 1 if wide or known and blocks < GROUPS_WALK_BLOCKS * num_tiles else block_groups(num_tiles * nkv, cus * per_cu, hd, known)
+    plan = plan_walks(step.cu_q_host, step.ctx_len_host, group, nkv, window, cus * (per_cu if groups == 1 else 1), groups, defines, only,
+                      cut=known)
     step.derived[key] = (wide, groups, defines, plan, int32_to_device(plan.items.reshape(-1), device))
     return step.derived[key]
 
@@ -251,14 +259,14 @@ def _long_single_tiles(step, group: int, nkv: int, device):
     return tuple(int(x) for x in single)
 
 
-def block_groups(walks: int, places: int, head_dim: int) -> int:
+def block_groups(walks: int, places: int, head_dim: int, cut: bool = True) -> int:
     """Wave groups per workgroup for a step of ``walks`` (entry, head) pairs on a device that holds
     ``places`` plain workgroups at a time.  Two groups (head sizes up to 128) halve a walk's time at
     a tenth less throughput: they pay where walks are so few that they are cut into many parts, of which one then adds up
     half as many (on 512 places, 68 walks of 124 key blocks 43 us for 50, of 247 62 for 71; 112 of 120 and 128 of 240 the same within 5
-    per cent; 224 of 240 149 for 146)."""
+    per cent; 224 of 240 149 for 146).  Where none is cut, they pay as long as every walk has a place from the start, and the longest decides."""
     most = int(_fn("attention_mfma", "qvl_attn_mfma_block_max_groups", [], {"HD": head_dim})())
-    return 2 if most >= 2 and 4 * walks <= places else 1
+    return 2 if most >= 2 and walks * (4 if cut else 1) <= places else 1
 
 
 def try_attention(q, k_cache, v_cache, block_table, step, num_q_heads: int, window: Optional[int],

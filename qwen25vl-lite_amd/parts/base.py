@@ -160,6 +160,7 @@ class StepContext:
     max_q_len: int = 0
     max_ctx_len: int = 0
     dtype: torch.dtype = torch.float32
+    lengths_known: bool = True   # False: ctx_len_host says how long the contexts may become (a captured step)
     # (key, position encoding, head width) of the rotation tables that the pass's mixers will look for
     rotations: Sequence[Any] = ()
     residual: Optional[torch.Tensor] = None   # set by a block while a part may add its result in place

@@ -155,6 +155,23 @@ def test_walks_that_cannot_be_listed(bad):
         attn.plan_walks([0, 4], kw["lens"], 2, kw["nkv"], 0, kw["places"], kw["groups"], {"HD": 128})
 
 
+@pytest.mark.parametrize("nq, nkv, hd, rows, keys", [(28, 4, 128, 200, 2048), (16, 4, 256, 160, 512), (64, 8, 128, 96, 1024), (9, 3, 96, 256, 512),
+                                                     (64, 1, 64, 200, 2048), (64, 1, 64, 600, 2048)])
+def test_walks_of_lengths_that_nobody_knows_stay_whole(nq, nkv, hd, rows, keys, monkeypatch):
+    """A step captured for contexts of up to some length: its walks, where known ones would be cut, by two wave groups only where each has a
+    workgroup to itself."""
+    from types import SimpleNamespace
+    from qwen25vl_lite_amd.ops import attention_mfma as attn
+    monkeypatch.setattr(attn, "_work_queue", lambda device: (None, 256))
+    step = SimpleNamespace(cu_q_host=list(range(rows + 1)), ctx_len_host=[keys] * rows, lengths_known=False, derived={})
+    wide, groups, _, plan, _ = attn._step_walks(step, nq // nkv, nkv, hd, 0, "cpu")
+    assert plan.partials == 0 and len(plan.items) == rows * (1 if 8 % nkv == 0 else nkv)
+    assert groups == (2 if not wide and hd <= 128 and rows * nkv <= 512 else 1)
+    if rows * nkv in (800, 640, 768):
+        known = SimpleNamespace(**{**vars(step), "lengths_known": True, "derived": {}})
+        assert attn._step_walks(known, nq // nkv, nkv, hd, 0, "cpu")[3].partials > 0
+
+
 @pytest.mark.parametrize("ranges", range(5))
 @pytest.mark.parametrize("k", [512, 2048, 3584, 8192])
 def test_products_that_are_cut_stay_cut(k, ranges):

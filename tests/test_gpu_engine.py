@@ -140,6 +140,14 @@ def test_decode_from_hip_graphs_gives_the_same_tokens(model_dirs, name, dtype, b
             assert out.output_token_ids == _plain_greedy(d, prompt, p.max_tokens)
 
 
+def test_captured_steps_say_that_their_lengths_are_not_known(model_dirs):
+    from qwen25vl_lite_amd import LLM, SamplingParams
+    llm = LLM(model_dirs["C_sharp"], dtype="bfloat16", num_blocks=64, block_size=16, max_num_seqs=3, hip_graph=True)
+    llm.generate([random_tokens(9, 300, 3)], [SamplingParams(temperature=0.0, max_tokens=3, ignore_eos=True)])
+    graphs = list(llm.runner.graphs.graphs.values())
+    assert graphs and not any(g.step.lengths_known for g in graphs)
+
+
 @pytest.mark.parametrize("name, dtype", [("B_sharp", "float32"), ("C_sharp", "bfloat16")])
 def test_decode_graphs_with_padding_rows(model_dirs, name, dtype):
     """Batch sizes between the captured ones (7 and 5 requests run in graphs of 8 and 6 rows): the

@@ -547,6 +547,31 @@ def test_paged_attention_walks_in_parts(nq, nkv, hd, window, ps, kind):
         assert torch.allclose(out.float().cpu(), c["want"], atol=1.5e-2, rtol=2e-2), (out.float().cpu() - c["want"]).abs().max()
 
 
+@pytest.mark.parametrize("known", [True, False])
+@pytest.mark.parametrize("nq, nkv, hd, window, ps", [(14, 2, 128, None, 16), (3, 3, 128, 700, 32), (6, 6, 48, 700, 16)])
+def test_paged_attention_of_longer_contexts_than_planned(nq, nkv, hd, window, ps, known):
+    """Walks cut for shorter contexts than they meet: the last part goes on to the end, and a window that has moved on leaves the first ones
+    without a key; and walks that are whole because nobody knows their lengths."""
+    from types import SimpleNamespace
+    import unittest.mock as mock
+    from qwen25vl_lite_amd.ops import attention_mfma
+    lens, qlens, planned = (1501, 64, 1030), (37, 20, 1), [1024, 40, 700]
+    c = _attention_case(torch.bfloat16, nq, nkv, hd, window, lens, qlens, ps=ps)
+    cu = [0, 37, 57, 58]
+    cu_q, ctx_len = (torch.tensor(x, dtype=torch.int32).cuda() for x in (cu, lens))
+    step = SimpleNamespace(num_reqs=3, cu_q=cu_q, cu_q_host=cu, ctx_len=ctx_len, ctx_len_host=planned, max_q_len=37,
+                           max_ctx_len=max(planned), lengths_known=known, derived={})
+    with mock.patch.object(attention_mfma, "plan_splits", lambda t, n, m, d=None: ("tile", 1, 0)):
+        out = attention_mfma.try_attention(c["q"], c["kc"], c["vc"], c["table"], step, nq, window, c["scale"],
+                                           force_groups=1 if known else None)
+    plan = next(v for k, v in step.derived.items() if k[0] == "walks")[3]
+    assert plan.partials >= 2 if known else plan.partials == 0
+    if known and window:
+        first = plan.items[(plan.items[:, 0] == 0) & (plan.items[:, 5] >> 16 > 1) & (plan.items[:, 5] & 0xffff == 0)]
+        assert len(first) and (first[:, 4] < (lens[0] - qlens[0] - window + 1) >> 5).any()     # a part 0 that has no key any more
+    assert torch.allclose(out.float().cpu(), c["want"], atol=1.5e-2, rtol=2e-2), (out.float().cpu() - c["want"]).abs().max()
+
+
 @pytest.mark.parametrize("nq, nkv, hd, window, ps", [(28, 4, 128, None, 16), (6, 2, 48, 100, 16), (4, 4, 256, 257, 16),
                                                      (5, 1, 16, None, 16), (28, 4, 128, None, 48), (6, 2, 48, 100, 32),
                                                      (4, 4, 256, 257, 64), (4, 2, 32, None, 16), (8, 2, 64, 70, 32),
