@@ -67,7 +67,11 @@ __global__ __launch_bounds__(LA_THREADS) void la_scan_kernel(
   __shared__ float ks[TB][DG];
   constexpr bool CHANNEL_DECAY = MODE != LA_HEAD;
   __shared__ float as[CHANNEL_DECAY ? TB : 1][DG];
-  __shared__ float logs[CHUNK && CHANNEL_DECAY ? TB : 1][CHUNK ? DG : 1], log_sums[CHUNK && CHANNEL_DECAY ? DG : 1];
+  // The logarithms of a channel's decays are summed by the threads that stage them where these are the same all the way.  (By way of LDS
+  // they cost the fourth block of a compute unit: 63 chunks, 16 heads of 128 x 64 with a decay for each channel 271 us, so
+  // 187.)
+  constexpr bool OWN = LA_THREADS % DG == 0, LISTED = CHUNK && CHANNEL_DECAY && !OWN;
+  __shared__ float logs[LISTED ? TB : 1][LISTED ? DG : 1], log_sums[LISTED ? DG : 1];
   __shared__ float po[TB][LA_WAVES][64 * COLS];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int head = blockIdx.y, req = blockIdx.z;
@@ -90,8 +94,9 @@ __global__ __launch_bounds__(LA_THREADS) void la_scan_kernel(
     for (int i = 0; i < LA_ROWS; ++i) U[BONUS ? i : 0] = bonus[head * LA_DIM + d0 + wave * LA_ROWS + i];
   }
 
-  if (CHUNK && CHANNEL_DECAY && vtile == 0)      // (a channel's sum is one thread's all the way)
-    for (int d = tid; d < DG; d += LA_THREADS) log_sums[d] = 0.f;
+  float log_sum = 0.f;
+  if (LISTED && vtile == 0)      // (a channel's sum is one thread's all the way)
+    for (int d = tid; d < DG; d += LA_THREADS) log_sums[LISTED ? d : 0] = 0.f;
   for (int t0 = begin; t0 < end; t0 += TB) {
     const int nt = end - t0 < TB ? end - t0 : TB;
     for (int idx = tid; idx < nt * DG; idx += LA_THREADS) {
@@ -104,7 +109,11 @@ __global__ __launch_bounds__(LA_THREADS) void la_scan_kernel(
         const float key = la_forget_key(zz, lower[hd]);
         ks[t][d] = key;
         as[t][d] = 1.0f - key;
-        if (CHUNK) logs[t][d] = log1pf(-key);
+        if (CHUNK) {
+          const float lg = log1pf(-key);
+          if (OWN) log_sum += lg;
+          else logs[LISTED ? t : 0][LISTED ? d : 0] = lg;
+        }
       } else {
         ks[t][d] = la_act(ldf<TP>(row + k_off), act & 2);
         if (MODE == LA_CHANNEL || MODE == LA_EXP) {
@@ -112,7 +121,8 @@ __global__ __launch_bounds__(LA_THREADS) void la_scan_kernel(
           const float zz = z[(size_t)(t0 + t) * z_stride + hd];
           const float lg = MODE == LA_EXP ? -expf(zz + (zbias ? zbias[hd] : 0.f)) : la_log_decay(zz, inv_tau);
           as[t][d] = expf(lg);
-          if (CHUNK) logs[t][d] = lg;
+          if (CHUNK && OWN) log_sum += lg;
+          if (LISTED) logs[LISTED ? t : 0][LISTED ? d : 0] = lg;
         }
       }
     }
@@ -125,11 +135,11 @@ __global__ __launch_bounds__(LA_THREADS) void la_scan_kernel(
                        ? la_act(ldf<TP>(proj + (size_t)(t0 + t) * proj_stride + v_off + (size_t)head * vdim + vcol + 64 * c), act & 4)
                        : 0.f;
     __syncthreads();
-    if (CHUNK && CHANNEL_DECAY && vtile == 0)
+    if (LISTED && vtile == 0)
       for (int d = tid; d < DG; d += LA_THREADS) {
-        float sum = log_sums[d];
-        for (int t = 0; t < nt; ++t) sum += logs[t][d];
-        log_sums[d] = sum;
+        float sum = log_sums[LISTED ? d : 0];
+        for (int t = 0; t < nt; ++t) sum += logs[LISTED ? t : 0][LISTED ? d : 0];
+        log_sums[LISTED ? d : 0] = sum;
       }
 #pragma unroll
     for (int t = 0; t < TB; ++t) {
@@ -169,9 +179,22 @@ __global__ __launch_bounds__(LA_THREADS) void la_scan_kernel(
     }
     __syncthreads();
   }
-  if (CHUNK && vtile == 0)
-    for (int d = tid; d < DG; d += LA_THREADS)
-      last[((size_t)req * H + head) * LA_DIM + d0 + d] = expf(CHANNEL_DECAY ? log_sums[CHANNEL_DECAY ? d : 0] : logf(fixed) * (float)(end - begin));
+  if (CHUNK && vtile == 0) {
+    float* parts = &po[0][0][0];      // (read by all behind the last barrier)
+    if (CHANNEL_DECAY && OWN) {
+      parts[tid] = log_sum;
+      __syncthreads();
+    }
+    for (int d = tid; d < DG; d += LA_THREADS) {
+      float sum = CHANNEL_DECAY ? log_sums[LISTED ? d : 0] : logf(fixed) * (float)(end - begin);
+      if (CHANNEL_DECAY && OWN) {
+        sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < LA_THREADS / DG; ++i) sum += parts[i * DG + d];
+      }
+      last[((size_t)req * H + head) * LA_DIM + d0 + d] = expf(sum);
+    }
+  }
 #pragma unroll
   for (int c = 0; c < COLS; ++c)
     if (vcol + 64 * c < vdim) {
