@@ -971,8 +971,9 @@ __device__ __forceinline__ void attend_block(BlockShared<GROUPS>& sh, const Bloc
   };
   int i = 0;
   for (; i < nblk - (BLK_STAGES - 1); ++i) round(i, std::true_type{});
-  // The ticket for the workgroup's next item is on its way during the last rounds.  (It stands behind loads that these wait for
-  // with the counts of loads alone: they wait for one load more.)
+  // The ticket for the workgroup's next item is asked for before the last rounds, which wait with it for all loads: the compiler, ready for
+  // several lanes that add, wants the old value at once.  The other workgroup of the compute unit covers that: told that one lane adds, so
+  // that the ticket is on its way during the rounds, every time stays as it is (4,096 tokens at 12,288 keys 571 us and 572).
   if (tickets && threadIdx.x == 0) ticket = __hip_atomic_fetch_add(tickets, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   for (; i < rounds; ++i) round(i, std::false_type{});
   // The sums stay where they are up to here: what follows is told of new values, or the compiler, with two ways to store them,

@@ -178,8 +178,8 @@ __device__ __forceinline__ float norm_total(const float* sums) {
 // Bytes bound it from about a thousand rows on: 4,096 rows of 3,584 with a bfloat16 addend 28.5 -> 26.9 us, 6.6 TB/s; below, latency: 64
 // rows of 8,192 7.4 -> 5.4, when the loads waited for each other's stores and the weights for the sum.
 // LATE, for NORM_ROWS rows or more of more than 4,096 values: four pieces at a time and the weights behind the sum.  Asked for at once, eight
-// pieces take 145 registers, three waves a SIMD, and the memory idles (with a bfloat16 addend 1,024 x 5,120 13.8 us, 10.0 so; 1,024 x 8,192 19.9
-// and 17.2; without one 4,096 x 8,192 40.0 and 33.1).
+// pieces take 145 registers, three waves a SIMD, and the memory idles (with a bfloat16 addend 1,024 x 5,120 13.8 us, 10.4 so; 1,024 x 8,192 19.9
+// and 17.7; without one 4,096 x 8,192 40.0 and 33.7).
 __device__ __forceinline__ float4 norm_value(float4 v) { return v; }
 __device__ __forceinline__ float4 norm_value(uint2 v) {
   return float4{__uint_as_float(v.x << 16), __uint_as_float(v.x & 0xffff0000u), __uint_as_float(v.y << 16),
@@ -270,8 +270,8 @@ __global__ __launch_bounds__(256) void add_rmsnorm_vec_kernel(float* __restrict_
 // per 4 values (rows of up to 4,096) or 8.  The loads of ONCE slabs are asked for at a time, sixteen of one piece, four of two (they do not
 // depend on each other, only the sum has an order: slab 0, 1, 2, ...), with the first of them the rows of h and w.  Latency bounds it:
 // fewer rows than fill the chip wait for memory once for every ONCE slabs here and once a slab in the kernel above (3,584 values, eight slabs:
-// 64 rows 4.1 us and 5.0, 256 rows 5.6 and 7.0).  Threads past a row of up to 4,096 leave as waves: a condition at every load took 0.5 us (1,024
-// values, 64 rows 4.2 us, 3.0 so).  Sixteen loads of two pieces, eight slabs, do not fit the registers (rows of 8,192, four slabs, 64 of them
+// 64 rows 4.1 us and 5.0, 256 rows 5.6 and 7.0).  Threads past a row of up to 4,096 leave as waves: a condition at every load took most of a microsecond (1,024
+// values, 64 rows 4.2 us, 3.4 so).  Sixteen loads of two pieces, eight slabs, do not fit the registers (rows of 8,192, four slabs, 64 of them
 // 5.8 us and 5.0; of 5,120, eight slabs, 6.5 and 5.4).
 // Many rows are bound by bytes: blocks of 1024 threads that are all at the same point leave the memory idle (of two slabs 512 rows 7.4
 // and 6.0, 2,048 rows 26.5 and 20.8).

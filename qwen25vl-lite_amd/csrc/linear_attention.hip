@@ -220,7 +220,8 @@ __global__ __launch_bounds__(LA_THREADS) void la_scan_kernel(
 // grid (chunks, H), 256 threads: rows begin .. end - 1 of `out` [N, H * vdim] = (q_t * P_t)^T S', S' the chunk's row of `states`.
 // A thread sums the logarithms of its channel's decays over a part of the chunk's tokens, learns through LDS what the parts before
 // it add up to, and walks its tokens again to leave q_t * P_t in LDS; then a wave takes 32 value channels at a time.  What bounds it is
-// latency: eight tokens' loads are asked for at once (44 us one by one, 36 so), and registers kept to four blocks a compute unit.
+// latency: eight tokens' loads are asked for at once (44 us one by one, 36 so).  Registers leave three blocks a compute unit up to 128 key
+// channels (122 to 128, and 32 of the sums; for a fourth block the compiler spills), beyond it is LDS: two blocks of 256 channels, one of 512.
 // (Chunks of more tokens than LDS holds are taken LA_JOIN at a time.)
 #define LA_JOIN 64
 #define LA_SPAN (LA_DIM <= 256 ? LA_DIM : 256)       // channels that threads stand side by side for
