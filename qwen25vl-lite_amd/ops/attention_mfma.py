@@ -78,21 +78,14 @@ def block_defines(head_dim: int, wide: bool) -> dict:
     return {"HD": head_dim, "BLK_CT": WIDE_CT} if wide and head_dim <= 128 else {"HD": head_dim}
 
 
-def tiles_for(cu_q, group: int, tile_ct: int = 1, ctx_len=None) -> Tuple[np.ndarray, np.ndarray]:
-    """``(tile_req, tile_ct)``: for request r with q tokens, ceil(q * group / (16 * tile_ct)) entries.
-    With ``ctx_len`` the entries are listed by the last key they see, latest first: the longest
-    walks start first and the short ones fill the compute units as they become free."""
+def tiles_for(cu_q, group: int, tile_ct: int = 1) -> Tuple[np.ndarray, np.ndarray]:
+    """``(tile_req, tile_ct)``: for request r with q tokens, ceil(q * group / (16 * tile_ct)) entries."""
     q = np.diff(np.asarray(cu_q, dtype=np.int64))
     cols = 16 * tile_ct
     counts = (q * group + cols - 1) // cols
     req = np.repeat(np.arange(len(q), dtype=np.int32), counts)
     starts = np.cumsum(counts) - counts
     ct = (np.arange(int(counts.sum()), dtype=np.int64) - np.repeat(starts, counts)).astype(np.int32)
-    if ctx_len is not None and len(req):
-        last_token = np.minimum(((ct.astype(np.int64) + 1) * cols - 1) // group, q[req] - 1)
-        last_key = np.asarray(ctx_len, dtype=np.int64)[req] - q[req] + last_token
-        order = np.argsort(-last_key, kind="stable")
-        req, ct = req[order], ct[order]
     return req, ct
 
 

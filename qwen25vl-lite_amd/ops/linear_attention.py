@@ -28,7 +28,7 @@ CHUNKED_FROM = 128    # a step whose longest run has this many tokens or more is
 
 
 def decayed_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, num_heads: int, dim: int, vdim: int,
-                 state: torch.Tensor, cu_q: torch.Tensor, req_slots: torch.Tensor, *,
+                 state: torch.Tensor, cu_q: torch.Tensor, req_slots: Optional[torch.Tensor], *,
                  head_decay: Optional[torch.Tensor] = None, z: Optional[torch.Tensor] = None, tau: float = 1.0,
                  silu=False, q_scale: float = 1.0, groups: int = 1, out: Optional[torch.Tensor] = None,
                  lower: Optional[torch.Tensor] = None, z_bias: Optional[torch.Tensor] = None,
@@ -52,7 +52,7 @@ def decayed_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, num_hea
     ``[groups, N, heads * vdim]``: with ``groups`` above 1 (2, 4 or 8; the key size must be a multiple
     of four times it) the key channels are cut into that many groups with blocks of their own, and the
     output is the sum of the slabs (see :func:`scan_groups`).  With ``last`` (float32 ``[R, heads, dim]``) every run starts from
-    zero, run r leaves its state in row r of ``state``, and ``last`` gets the product of its decays."""
+    zero, run r leaves its state in row r of ``state`` (``req_slots`` is not read and may be None), and ``last`` gets the product of its decays."""
     _dev(proj, state, cu_q, req_slots, head_decay, z, lower, z_bias, bonus)
     h, d, v = int(num_heads), int(dim), int(vdim)
     n = proj.shape[-2]
@@ -63,9 +63,10 @@ def decayed_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, num_hea
             ((q_off, h * d), (q_off if lower is not None else k_off, h * d), (v_off, h * v))]
     _need(state.dtype == torch.float32 and state.dim() == 4 and tuple(state.shape[1:]) == (h, d, v)
           and state.is_contiguous(), "state must be contiguous float32 [slots, heads, dim, vdim]")
-    for t in (cu_q, req_slots):
+    _need(req_slots is not None or last is not None, "runs find their states by req_slots, or start from zero (last)")
+    for t in (cu_q,) if req_slots is None else (cu_q, req_slots):
         _need(t.dtype == torch.int32 and t.dim() == 1 and t.is_contiguous(), "cu_q and req_slots must be int32")
-    r = req_slots.shape[0]
+    r = cu_q.shape[0] - 1 if req_slots is None else req_slots.shape[0]
     _need(cu_q.shape[0] == r + 1, "cu_q must have one more entry than there are requests")
     _need((head_decay is None) != (z is None), "exactly one of head_decay and z is needed")
     zstride = 0
@@ -149,13 +150,12 @@ def scan_groups(num_reqs: int, max_run: int, num_heads: int, dim: int, vdim: int
 @dataclass
 class ChunkPlan:
     """A step's runs cut into chunks: ``chunk_cu [chunks + 1]`` (token bounds, chunks follow one another
-    as the runs do), ``chunk_rows [chunks]`` (0, 1, ...: a chunk's row of the scratch state),
+    as the runs do),
     ``req_first [R + 1]`` (the first chunk of each request), all int32 on the device."""
 
     chunks: int
     chunk_len: int
     chunk_cu: torch.Tensor
-    chunk_rows: torch.Tensor
     req_first: torch.Tensor
 
 
@@ -168,9 +168,8 @@ def plan_chunks(cu_q_host: Sequence[int], device, chunk_len: int = CHUNK) -> Chu
             bounds.append(at)
         first.append(len(bounds) - 1)
     n = len(bounds) - 1
-    host = np.concatenate([np.asarray(bounds, np.int32), np.arange(n, dtype=np.int32), np.asarray(first, np.int32)])
-    dev = int32_to_device(host, device)
-    return ChunkPlan(n, chunk_len, dev[:n + 1], dev[n + 1:2 * n + 1], dev[2 * n + 1:])
+    dev = int32_to_device(np.asarray(bounds + first, np.int32), device)
+    return ChunkPlan(n, chunk_len, dev[:n + 1], dev[n + 1:])
 
 
 def chunked_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, num_heads: int, dim: int, vdim: int,
@@ -195,7 +194,7 @@ def chunked_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, num_hea
     # (a block of a chunk's scan owns twice the value channels where there are more than 64)
     groups = scan_groups(nch, clen, h, d, (v + 1) // 2 if v > 64 and d <= 256 else v, proj.device)
     out = torch.empty((groups + 1, n, h * v), dtype=torch.float32, device=proj.device)
-    decayed_scan(proj, q_off, k_off, v_off, h, d, v, scratch, plan.chunk_cu, plan.chunk_rows, head_decay=head_decay,
+    decayed_scan(proj, q_off, k_off, v_off, h, d, v, scratch, plan.chunk_cu, None, head_decay=head_decay,
                  z=z, tau=tau, silu=silu, q_scale=q_scale, groups=groups, out=out[:groups], lower=lower, z_bias=z_bias,
                  exp_decay=exp_decay, bonus=bonus, last=last)
     defines = {"LA_DIM": d}
