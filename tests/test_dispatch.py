@@ -147,6 +147,39 @@ def test_walks_of_prompt_portions(qlens, lens, group, nkv, window, places, group
         assert counters
 
 
+@pytest.mark.parametrize("requests", [1, 63, 64, 150])
+def test_runs_of_column_tiles_counted_by_integers_and_by_arrays(requests):
+    from types import SimpleNamespace
+    from qwen25vl_lite_amd.ops import attention_mfma as attn
+    assert 63 < attn.MANY_REQUESTS <= 64
+    rng = np.random.default_rng(requests)
+    q = rng.integers(0, 300, requests)
+    ctx = q + rng.integers(0, 4000, requests)
+    cu = np.concatenate([[0], np.cumsum(q)]).tolist()
+    for only in (None, tuple(int(x) for x in rng.integers(0, 2, requests))):
+        step = SimpleNamespace(cu_q_host=cu, ctx_len_host=ctx.tolist(), derived={})
+        for group, tile_ct in ((1, 1), (7, 8), (3, 12)):
+            entries = [-(-int(n) * group // (16 * tile_ct)) * (only is None or only[i]) for i, n in enumerate(q)]
+            assert attn._count_tiles(step, group, tile_ct, only) == sum(entries)
+            assert attn._walk_blocks(step, group, tile_ct, only) == sum(
+                e * max(1, (int(c) - int(n) // 2 + 31) // 32) for e, n, c in zip(entries, q, ctx))
+
+
+def test_whole_walks_are_listed_longest_first():
+    """The lists are made by counting; here once more by comparing: those of one length stay as they come."""
+    from qwen25vl_lite_amd.ops import attention_mfma as attn
+    rng = np.random.default_rng(5)
+    for _ in range(20):
+        q = rng.integers(1, 400, rng.integers(1, 40))
+        ctx = q + rng.integers(0, 6000, len(q))
+        group, nkv, places = int(rng.integers(1, 9)), int(rng.choice([2, 3, 8])), int(rng.choice([16, 100, 512]))
+        plan = attn.plan_walks(np.concatenate([[0], np.cumsum(q)]), ctx, group, nkv, 0, places, 1, {"HD": 128}, cut=False)
+        heads = 1 if 8 % nkv == 0 else nkv
+        walks = [(r, cb, h, 0, (int(ctx[r]) - int(q[r]) + min((128 * cb + 127) // group, int(q[r]) - 1)) >> 5)
+                 for r in range(len(q)) for cb in range(-(-int(q[r]) * group // 128)) for h in range(heads)]
+        assert [tuple(i[:5]) for i in plan.items.tolist()] == sorted(walks, key=lambda w: -w[4]) and plan.partials == 0
+
+
 @pytest.mark.parametrize("bad", [dict(lens=[3]), dict(groups=3), dict(nkv=0), dict(places=0)])
 def test_walks_that_cannot_be_listed(bad):
     from qwen25vl_lite_amd.ops import attention_mfma as attn, kernels
