@@ -23,6 +23,7 @@
 // o go to its own slab of the output, [G, N, heads * vdim], and whoever reads the output adds the
 // slabs in order (the norm that follows does).
 #include "common.h"
+#include <atomic>
 
 #ifndef LA_DIM
 #define LA_DIM 64
@@ -49,7 +50,7 @@ __device__ __forceinline__ float la_log_decay(float z, float inv_tau) { return (
 // COLS: value channels of a lane (64 apart).  What bounds a long run is LDS and the vector unit: every value of q, k and the decays
 // that a wave reads serves 64 channels with one of a lane, 128 with two, and staging is shared likewise (29 chunks of 64 tokens, 28
 // heads: of 64 x 128 with a decay for each channel 117 us and 88, of 128 x 128 with one for each head 159 and 135).  Fewer tokens at a
-// time and a bound on registers, for a fourth block a compute unit: 89 and 146.
+// time and a bound on registers, for a fourth block a compute unit: 89 and 146.  (When two are taken: qvl_la_chunk_columns.)
 // CHUNK: the runs are chunks of a request's (see below): each starts from zero, its state is row `run` of `state`, and
 // `last` gets the product of its decays.
 template <typename TP, int MODE, int G, bool BONUS, int COLS, bool CHUNK>
@@ -402,6 +403,42 @@ extern "C" int qvl_la_carry(void* scratch, const void* last, void* state, const 
 
 extern "C" int qvl_la_key_size() { return LA_DIM; }
 
+// Value channels of a lane in the scan of chunks, for `pairs` of (full) chunks and heads.  Two where one would take the blocks in more than one round
+// and two in one: what a round takes is a block's way through its 64 tokens, longer with two channels.  16 heads, two and one: of 64 x 128
+// with a decay for each channel 512 pairs 114 us and 96, 640 121 and 139, 1,504 239 and 243; of 128 x 128 with one for each head 512 135 and 115, 640
+// 147 and 174, 1,504 320 and 304; of 256 x 256, 8 heads, 256 pairs 290 and 366 (one decay for each head 221 and 181), 320 480 and 407.
+#define LA_TWO_DIM 256      // beyond, the state of two channels does not fit the registers
+#define LA_TWO (LA_DIM <= LA_TWO_DIM ? 2 : 1)
+template <typename TP, int MODE, bool BONUS, int COLS>
+static int la_blocks_a_unit() {
+  static std::atomic<int> known{0};
+  int n = known.load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, la_scan_kernel<TP, MODE, 1, BONUS, COLS, true>, LA_THREADS, 0) != hipSuccess || n < 1) {
+      (void)hipGetLastError();
+      n = 1;
+    }
+    known.store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
+extern "C" int qvl_la_chunk_columns(int proj_dtype, int has_z, int has_lower, int exp_decay, int has_bonus, long long pairs, int vdim, int cus) {
+  if (vdim <= 64 || LA_DIM > LA_TWO_DIM || pairs <= 0) return 1;
+  const long long one = pairs * ((vdim + 63) / 64), two = pairs * ((vdim + 127) / 128);
+#define TWO_PAYS(TP, MODE, BONUS) \
+  (one > (long long)cus * la_blocks_a_unit<TP, MODE, BONUS, 1>() && two <= (long long)cus * la_blocks_a_unit<TP, MODE, BONUS, LA_TWO>())
+#define BY_MODE(TP)                                          \
+  (exp_decay && has_bonus ? TWO_PAYS(TP, LA_EXP, true)       \
+   : exp_decay            ? TWO_PAYS(TP, LA_EXP, false)      \
+   : has_lower            ? TWO_PAYS(TP, LA_FORGET, false)   \
+   : has_z                ? TWO_PAYS(TP, LA_CHANNEL, false)  \
+                          : TWO_PAYS(TP, LA_HEAD, false))
+  return (proj_dtype == 1 ? BY_MODE(bf16_t) : BY_MODE(float)) ? 2 : 1;
+#undef BY_MODE
+#undef TWO_PAYS
+}
+
 // proj: rows of `proj_stride` values holding q (H * LA_DIM columns from q_off), k (from k_off) and v
 // (H * vdim columns from v_off).  head_decay [H] float32, or z float32 rows (H * LA_DIM columns) with
 // inv_tau, or z with lower (and zbias, which may be null) float32 [H * LA_DIM]: the floored forget gate, whose
@@ -410,7 +447,7 @@ extern "C" int qvl_la_key_size() { return LA_DIM; }
 // [groups, N, H * vdim] (groups 1, 2, 4 or 8 with LA_DIM a multiple of 4 * groups), slabs `out_slab` apart.
 extern "C" int qvl_la_scan(const void* proj, long long proj_stride, long long q_off, long long k_off, long long v_off,
                            int proj_dtype, const void* head_decay, const void* z, long long z_stride, float inv_tau,
-                           const void* lower, const void* zbias, int exp_decay, const void* bonus, void* state, const void* cu_q, const void* req_slots, void* out, long long out_slab, int groups, void* last, int R,
+                           const void* lower, const void* zbias, int exp_decay, const void* bonus, void* state, const void* cu_q, const void* req_slots, void* out, long long out_slab, int groups, int columns, void* last, int R,
                            int H, int dim, int vdim, int act, float q_scale, hipStream_t stream) {
   if (R <= 0) return QVL_OK;
   if (dim != LA_DIM || H <= 0 || vdim <= 0 || (!head_decay && !z) || (lower && !z) ||
@@ -420,9 +457,8 @@ extern "C" int qvl_la_scan(const void* proj, long long proj_stride, long long q_
   if (groups != 1 && groups != 2 && groups != 4 && groups != 8) return QVL_ERR_SHAPE;
   if (LA_DIM % (LA_WAVES * groups)) return QVL_ERR_SHAPE;
   if (H > 65535 || R > 65535) return QVL_ERR_LIMIT;
-  // two value channels a lane for chunks of more than 64 (their state fits the registers)
-  const bool two = last && vdim > 64 && LA_DIM <= 256;
-  const dim3 grid((two ? (vdim + 127) / 128 : (vdim + 63) / 64) * groups, H, R);
+  if (columns != 1 && (columns != 2 || !last || groups != 1 || LA_DIM > LA_TWO_DIM)) return QVL_ERR_SHAPE;
+  const dim3 grid((vdim + 64 * columns - 1) / (64 * columns) * groups, H, R);
 #define RUN(TP, CH, G, BONUS, COLS, CHUNK)                                                                                    \
   hipLaunchKernelGGL((la_scan_kernel<TP, CH, G, BONUS, COLS, CHUNK>), grid, dim3(LA_THREADS), 0, stream, (const TP*)proj,     \
                      proj_stride, q_off, k_off, v_off, (const float*)head_decay, (const float*)z, z_stride, inv_tau,          \
@@ -430,7 +466,7 @@ extern "C" int qvl_la_scan(const void* proj, long long proj_stride, long long q_
                      (const int*)req_slots, (float*)out, out_slab, (float*)last, H, vdim, act, q_scale)
 #define LAUNCH(TP, CH, G, BONUS)                          \
   do {                                                    \
-    if (two) RUN(TP, CH, G, BONUS, (LA_DIM <= 256 ? 2 : 1), true); \
+    if (columns == 2) RUN(TP, CH, 1, BONUS, LA_TWO, true); \
     else if (last) RUN(TP, CH, G, BONUS, 1, true);        \
     else RUN(TP, CH, G, BONUS, 1, false);                 \
   } while (0)

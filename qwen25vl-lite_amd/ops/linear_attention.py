@@ -14,7 +14,7 @@ import numpy as np
 
 import torch
 
-from .kernels import _check, _dev, _fn, _need, _ptr, _stream, dtype_code, int32_to_device
+from .kernels import _check, _dev, _fn, _need, _ptr, _stream, compute_units, dtype_code, int32_to_device
 
 __all__ = ["decayed_scan", "scan_groups", "chunked_scan", "plan_chunks", "ChunkPlan", "MAX_KEY_SIZE", "CHUNK"]
 
@@ -33,7 +33,7 @@ def decayed_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, num_hea
                  silu=False, q_scale: float = 1.0, groups: int = 1, out: Optional[torch.Tensor] = None,
                  lower: Optional[torch.Tensor] = None, z_bias: Optional[torch.Tensor] = None,
                  exp_decay: bool = False, bonus: Optional[torch.Tensor] = None,
-                 last: Optional[torch.Tensor] = None) -> torch.Tensor:
+                 last: Optional[torch.Tensor] = None, columns: int = 1) -> torch.Tensor:
     """Run every request's tokens of the step through the recurrence, from and into ``state``.
 
     ``proj [N, cols]`` or ``[parts, N, cols]`` (float32 or bfloat16; an offset then counts through the parts,
@@ -52,7 +52,8 @@ def decayed_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, num_hea
     ``[groups, N, heads * vdim]``: with ``groups`` above 1 (2, 4 or 8; the key size must be a multiple
     of four times it) the key channels are cut into that many groups with blocks of their own, and the
     output is the sum of the slabs (see :func:`scan_groups`).  With ``last`` (float32 ``[R, heads, dim]``) every run starts from
-    zero, run r leaves its state in row r of ``state`` (``req_slots`` is not read and may be None), and ``last`` gets the product of its decays."""
+    zero, run r leaves its state in row r of ``state`` (``req_slots`` is not read and may be None), and ``last`` gets the product of its decays;
+    ``columns`` 2 (key sizes up to 256, ``groups`` 1): a lane has two value channels, the same sums."""
     _dev(proj, state, cu_q, req_slots, head_decay, z, lower, z_bias, bonus)
     h, d, v = int(num_heads), int(dim), int(vdim)
     n = proj.shape[-2]
@@ -88,11 +89,11 @@ def decayed_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, num_hea
               and state.shape[0] >= r, "last must be contiguous float32 [runs, heads, dim], with a row of state for each run")
     fn = _fn("linear_attention", "qvl_la_scan",
              [_c_ptr, _c_ll, _c_ll, _c_ll, _c_ll, _c_int, _c_ptr, _c_ptr, _c_ll, _c_float, _c_ptr, _c_ptr, _c_int, _c_ptr,
-              _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ll, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_ptr],
+              _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ll, _c_int, _c_int, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_ptr],
              {"LA_DIM": d})
     _check(fn(_ptr(proj), proj.stride(-2), *offs, dtype_code(proj.dtype),
               _ptr(head_decay), _ptr(z), zstride, 1.0 / float(tau), _ptr(lower), _ptr(z_bias), int(bool(exp_decay)),
-              _ptr(bonus), _ptr(state), _ptr(cu_q), _ptr(req_slots), _ptr(out), out.stride(0), int(groups), _ptr(last), r, h, d, v,
+              _ptr(bonus), _ptr(state), _ptr(cu_q), _ptr(req_slots), _ptr(out), out.stride(0), int(groups), int(columns), _ptr(last), r, h, d, v,
               silu_mask(silu), float(q_scale),
               _stream()), "decayed_scan")
     return out
@@ -191,12 +192,15 @@ def chunked_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, num_hea
     _need(plan.req_first.shape[0] == r + 1, "the chunk plan belongs to another step")
     scratch = torch.empty((nch, h, d, v), dtype=torch.float32, device=proj.device)
     last = torch.empty((nch, h, d), dtype=torch.float32, device=proj.device)
-    # (a block of a chunk's scan owns twice the value channels where there are more than 64)
-    groups = scan_groups(nch, clen, h, d, (v + 1) // 2 if v > 64 and d <= 256 else v, proj.device)
+    cus = compute_units(proj.device)
+    columns = _fn("linear_attention", "qvl_la_chunk_columns", [_c_int] * 5 + [_c_ll, _c_int, _c_int], {"LA_DIM": d})(
+        dtype_code(proj.dtype), int(z is not None), int(lower is not None), int(bool(exp_decay)), int(bonus is not None),
+        (n + clen - 1) // clen * h, v, cus)      # (as if all chunks were full: short ones leave their places early)
+    groups = 1 if columns == 2 else scan_groups(nch, clen, h, d, v, proj.device)
     out = torch.empty((groups + 1, n, h * v), dtype=torch.float32, device=proj.device)
     decayed_scan(proj, q_off, k_off, v_off, h, d, v, scratch, plan.chunk_cu, None, head_decay=head_decay,
                  z=z, tau=tau, silu=silu, q_scale=q_scale, groups=groups, out=out[:groups], lower=lower, z_bias=z_bias,
-                 exp_decay=exp_decay, bonus=bonus, last=last)
+                 exp_decay=exp_decay, bonus=bonus, last=last, columns=columns)
     defines = {"LA_DIM": d}
     fn = _fn("linear_attention", "qvl_la_carry", [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int,
                                                    _c_ptr], defines)

@@ -415,6 +415,34 @@ def test_chunks_joined_at_edges(d, v, runs, chunk, decay):
     assert torch.equal(s2[0], start[0]) and torch.equal(s2[-1], start[-1])
 
 
+@pytest.mark.parametrize("decay", ["head", "channel", "forget", "exp", "bonus"])
+@pytest.mark.parametrize("d, v", [(64, 128), (128, 200), (20, 65), (6, 130)])
+def test_one_and_two_value_channels_a_lane(d, v, decay):
+    """The same sums in the same order, a product and a sum rounded once or twice as the compiler takes them: outputs and states of runs from zero
+    within 64 tokens' roundings of a state, an eps each at most, and of an output's d of them (2e-5 of the largest value, as for chunks)."""
+    from qwen25vl_lite_amd.ops.linear_attention import decayed_scan
+    from qwen25vl_lite_amd.ops.kernels import KernelError
+    torch.manual_seed(d)
+    runs, h = [64, 1, 33, 50], 3
+    n = sum(runs)
+    proj = torch.randn(n, 2 * h * d + h * v).bfloat16().cuda()
+    how = dict(head_decay=torch.tensor([0.5, 0.9, 1.0]).cuda()) if decay == "head" else dict(z=torch.randn(n, h * d).cuda() - 1)
+    if decay == "forget":
+        how.update(lower=torch.rand(h * d).cuda(), z_bias=torch.randn(h * d).cuda())
+    elif decay in ("exp", "bonus"):
+        how.update(exp_decay=True, bonus=torch.randn(h * d).cuda() if decay == "bonus" else None)
+    cu = torch.tensor([0, 64, 65, 98, 148], dtype=torch.int32).cuda()
+    results = []
+    for columns in (1, 2):
+        state, last = torch.zeros(4, h, d, v, device="cuda"), torch.zeros(4, h, d, device="cuda")
+        out = decayed_scan(proj, 0, h * d, 2 * h * d, h, d, v, state, cu, None, last=last, columns=columns, **how)
+        results.append((out, state, last))
+    for one, two in zip(*results):
+        assert torch.allclose(one, two, atol=2e-5 * one.abs().max().item()), (one - two).abs().max() / one.abs().max()
+    with pytest.raises(KernelError):
+        decayed_scan(proj, 0, h * d, 2 * h * d, h, d, v, state, cu, torch.arange(4, dtype=torch.int32).cuda(), columns=2, **how)
+
+
 @pytest.mark.parametrize("span, groups", [(7, 3), (24, 5), (128, 2), (1024, 1), (1500, 2), (4100, 1)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_group_norm_with_gate_at_any_width(span, groups, dtype):
