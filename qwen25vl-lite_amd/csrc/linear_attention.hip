@@ -218,12 +218,14 @@ __global__ __launch_bounds__(LA_THREADS) void la_scan_kernel(
 // back into token order by a kernel of their own, they were 208 and 263.
 // ---------------------------------------------------------------------------------------
 
-// grid (chunks, H), 256 threads: rows begin .. end - 1 of `out` [N, H * vdim] = (q_t * P_t)^T S', S' the chunk's row of `states`.
+// grid (chunks, H, parts of the value channels), 256 threads: rows begin .. end - 1 of `out` [N, H * vdim] = (q_t * P_t)^T S', S' the chunk's row of `states`.
 // A thread sums the logarithms of its channel's decays over a part of the chunk's tokens, learns through LDS what the parts before
 // it add up to, and walks its tokens again to leave q_t * P_t in LDS; then a wave takes 32 value channels at a time.  What bounds it is
 // latency: eight tokens' loads are asked for at once (44 us one by one, 36 so).  Registers leave three blocks a compute unit up to 128 key
 // channels (122 to 128, and 32 of the sums; for a fourth block the compiler spills), beyond it is LDS: two blocks of 256 channels, one of 512.
-// (Chunks of more tokens than LDS holds are taken LA_JOIN at a time.)
+// (Chunks of more tokens than LDS holds are taken LA_JOIN at a time.)  Where chunks and heads are few, up to 128 value channels go to a block
+// of their own each, which forms q_t * P_t anew (4 chunks, 4 heads of 256 x 512, one decay for each head: 70 us of the
+// whole scan, by one block 118).
 #define LA_JOIN 64
 #define LA_SPAN (LA_DIM <= 256 ? LA_DIM : 256)       // channels that threads stand side by side for
 #define LA_PARTS (256 / LA_SPAN < 16 ? 256 / LA_SPAN : 16)
@@ -304,7 +306,7 @@ __global__ __launch_bounds__(256) void la_join_kernel(const TP* __restrict__ pro
     // gives one of them to each of four instructions.
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15, tiles = (end - begin + 15) / 16;
     const float* S = states + ((size_t)chunk * H + head) * LA_DIM * vdim;
-    for (int c0 = wave * 32; c0 < vdim; c0 += 128) {
+    for (int c0 = (blockIdx.z * 4 + wave) * 32; c0 < vdim; c0 += 128 * gridDim.z) {
       la_f32x4 sum[4][2];
 #pragma unroll
       for (int t = 0; t < 4; ++t)
@@ -372,13 +374,15 @@ __global__ void la_carry_kernel(float* __restrict__ scratch, const float* __rest
 extern "C" int qvl_la_join(const void* proj, long long proj_stride, long long q_off, int proj_dtype, const void* head_decay, const void* z,
                            long long z_stride, float inv_tau, const void* lower, const void* zbias, int exp_decay, int before,
                            const void* chunk_cu, const void* states, void* out, int chunks, int H, int dim, int vdim, int act,
-                           float q_scale, hipStream_t stream) {
+                           float q_scale, int cus, hipStream_t stream) {
   if (chunks <= 0) return QVL_OK;
   if (dim != LA_DIM || H <= 0 || vdim <= 0 || (!head_decay && !z) || (lower && !z) || (exp_decay && (lower || !z)))
     return QVL_ERR_SHAPE;
   if (H > 65535) return QVL_ERR_LIMIT;
+  const long long room = 2ll * cus / ((long long)chunks * H), all = (vdim + 127) / 128;
+  const int parts = (int)(room < 1 ? 1 : room < all ? room : all);
 #define LAUNCH(TP, MODE)                                                                                                     \
-  hipLaunchKernelGGL((la_join_kernel<TP, MODE>), dim3(chunks, H), dim3(256), 0, stream, (const TP*)proj, proj_stride, q_off,  \
+  hipLaunchKernelGGL((la_join_kernel<TP, MODE>), dim3(chunks, H, parts), dim3(256), 0, stream, (const TP*)proj, proj_stride, q_off,  \
                      (const float*)head_decay, (const float*)z, z_stride, inv_tau, (const float*)lower, (const float*)zbias,  \
                      (const int*)chunk_cu, (const float*)states, (float*)out, H, vdim, act, q_scale, before)
 #define BY_MODE(TP) { if (exp_decay) LAUNCH(TP, LA_EXP); else if (lower) LAUNCH(TP, LA_FORGET); else if (z) LAUNCH(TP, LA_CHANNEL); else LAUNCH(TP, LA_HEAD); }

@@ -208,9 +208,9 @@ def chunked_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, num_hea
            "chunk carry")
     fn = _fn("linear_attention", "qvl_la_join",
              [_c_ptr, _c_ll, _c_ll, _c_int, _c_ptr, _c_ptr, _c_ll, _c_float, _c_ptr, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr,
-              _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_ptr], defines)
+              _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_ptr], defines)
     _check(fn(_ptr(proj), proj.stride(-2), _place(proj, q_off, h * d), dtype_code(proj.dtype), _ptr(head_decay), _ptr(z),
               z.stride(0) if z is not None else 0, 1.0 / float(tau), _ptr(lower), _ptr(z_bias), int(bool(exp_decay)),
               int(bonus is not None), _ptr(plan.chunk_cu), _ptr(scratch), _ptr(out[groups]), nch, h, d, v, silu_mask(silu),
-              float(q_scale), _stream()), "chunk join")
+              float(q_scale), cus, _stream()), "chunk join")
     return out
