@@ -35,6 +35,11 @@ struct SliceArgs {
   bf16_t* kc;           // [page][nkv][ps][hd]
   bf16_t* vc;           // [page][nkv][hd][ps]
   int nq, nkv, hd, ps;
+  // The rows of X are rows of the sum times a norm's gain, not yet divided by their root mean square: row m's squares add up to
+  // those of squares[256 m ...], `parts` of them (up to 16 rows; null: X is as it is)
+  const float* squares;
+  int parts;
+  float eps;
 };
 
 #define PAST_END 0x80000000u      // no buffer reaches it (the host checks): a lane that asks there, or a little beyond, gets zeros without traffic
@@ -74,6 +79,7 @@ __global__ __launch_bounds__(64 * SLICE_WAVES) void gemm_slice_kernel(SliceArgs 
   constexpr int STAGE = CT * 16 * 128;                                              // two steps of a wave's rows of X in LDS
   constexpr int DEEP = CT <= 2 ? 8 / CT : 2;                                        // stages of a wave that LDS holds
   static_assert(CT > 1 || DEEP >= S / 2, "fetch_x leaves out loads");
+  __shared__ float scale[16];
   constexpr int SUMS = SLICE_WAVES * 2 * CT * 256 * 4, RING = SLICE_WAVES * DEEP * STAGE;
   __shared__ __attribute__((aligned(16))) char lds[SUMS > RING ? SUMS : RING];
   float (*sums)[2][CT * 256] = reinterpret_cast<float (*)[2][CT * 256]>(lds);
@@ -112,6 +118,13 @@ __global__ __launch_bounds__(64 * SLICE_WAVES) void gemm_slice_kernel(SliceArgs 
   for (int u = 0; u < S; ++u)
 #pragma unroll
     for (int t = 0; t < 2; ++t) w[u][t] = load16(w_buf, u < inside ? w_at[t] : PAST_END, u * 64);
+  float4 square[2];       // of rows wave and wave + 8
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    square[i] = float4{0.f, 0.f, 0.f, 0.f};
+    if (CT == 1 && p.squares && wave + 8 * i < p.M && 4 * lane < p.parts)
+      square[i] = *reinterpret_cast<const float4*>(p.squares + (wave + 8 * i) * 256 + 4 * lane);
+  }
   // what the results need beside the sums; result e of the block: row e / 16 of X, pair e mod 16
   float b0[ENDS], b1[ENDS];
   float2 turn[ENDS];     // (of queries and keys)
@@ -166,6 +179,15 @@ __global__ __launch_bounds__(64 * SLICE_WAVES) void gemm_slice_kernel(SliceArgs 
         for (int c = 0; c < CT; ++c)
           acc[2 * s >= S / 2][t][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[2 * s + h][t], x[h][c], acc[2 * s >= S / 2][t][c], 0, 0, 0);
   }
+  if (CT == 1 && p.squares) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int m = wave + 8 * i, have = p.parts - 4 * lane;
+      if (m >= p.M) break;
+      const float s = wave_sum((square[i].x + (have > 1 ? square[i].y : 0.f)) + ((have > 2 ? square[i].z : 0.f) + (have > 3 ? square[i].w : 0.f)));
+      if (lane == 0) scale[m] = 1.0f / sqrtf(s / (float)p.K + p.eps);
+    }
+  }
   __syncthreads();      // the sums' place is the stages'
 #pragma unroll
   for (int t = 0; t < 2; ++t)
@@ -180,6 +202,7 @@ __global__ __launch_bounds__(64 * SLICE_WAVES) void gemm_slice_kernel(SliceArgs 
 #pragma unroll
     for (int s = 0; s < SLICE_WAVES; ++s) a += sums[s][0][e], b += sums[s][1][e];
     const int head = pair / half, f = pair % half;
+    if (CT == 1 && p.squares) a *= scale[m], b *= scale[m];
     a += b0[i];
     b += b1[i];
     bf16_t* to;
@@ -213,10 +236,11 @@ extern "C" int qvl_gemm_slice_most_k() { return SLICE_K(16); }
 
 // The stacked projection of nq query, nkv key and nkv value heads of hd channels (hd even) with bias (float32 or null), rotation and cache write:
 // q_out bfloat16 [M, nq hd]; keys and values into their pages, kc [page][nkv][ps][hd], vc [page][nkv][hd][ps] (slot[m] = page * ps
-// + place, or -1).  cs: float32 [M, hd / 2, 2].
+// + place, or -1).  cs: float32 [M, hd / 2, 2].  squares (float32 [M, 256], on a 16-byte boundary), parts, eps: x is rows of a sum times a norm's gain as
+// qvl_gemm_stream_into leaves them (up to 16 rows); null: x as it is.
 extern "C" int qvl_gemm_slice_rope(const void* x, int ldx, const void* w, int ldw, const void* bias, const void* cs, const void* slot,
                                    void* q_out, void* kc, void* vc, int M, int K, int nq, int nkv, int hd, int ps, int cus,
-                                   hipStream_t stream) {
+                                   const void* squares, int parts, float eps, hipStream_t stream) {
   if (M <= 0) return QVL_OK;
   if (nq <= 0 || nkv < 0 || hd <= 0 || hd % 2 || !cs || ((uintptr_t)cs % 8) || !q_out || (nkv && (ps <= 0 || !slot || !kc || !vc)) ||
       (long long)(nq + 2ll * nkv) * hd > 0x7fffffffll)
@@ -226,6 +250,8 @@ extern "C" int qvl_gemm_slice_rope(const void* x, int ldx, const void* w, int ld
   p.M = M; p.N = (nq + 2 * nkv) * hd; p.K = K; p.pairs = p.N / 2;
   p.cs = (const float2*)cs; p.slot = (const int*)slot; p.q_out = (bf16_t*)q_out; p.kc = (bf16_t*)kc; p.vc = (bf16_t*)vc;
   p.nq = nq; p.nkv = nkv; p.hd = hd; p.ps = ps;
+  p.squares = (const float*)squares; p.parts = parts; p.eps = eps;
+  if (squares && (M > 16 || parts <= 0 || parts > 256 || ((uintptr_t)squares % 16))) return QVL_ERR_SHAPE;
   if (!qvl_gemm_slice_takes(M, p.N, K, cus)) return QVL_ERR_LIMIT;
   if (ldx < K || ldw < K || ldx % 8 || ldw % 8 || !x || !w || (((uintptr_t)x | (uintptr_t)w) % 16)) return QVL_ERR_SHAPE;
   // byte offsets are 32-bit, and PAST_END lies behind them

@@ -10,6 +10,7 @@ from typing import Dict, List, Optional, Tuple
 import torch
 
 from ..cache.manager import CacheGroupSpec
+from ..ops.stream import MOST_ROWS
 from ..parts.base import (Block, CacheNeed, LayerSlot, Mixer, ParamSpec, Part, PartSpec, ResidualStream, StateNeed, rotation_key,
                           StepContext, build_part)
 from .spec import ModelSpec
@@ -332,7 +333,9 @@ class DecoderModel:
         first_share = None
         if self.pass_mix is not None and any(e.mix_input for e in self.spec.run):
             first_share = self.pass_mix.from_first(stream.h)     # before any layer changes the sum in place
-        for entry, slot in zip(self.spec.run, slots):
+        run = self.spec.run
+        few = stream.h.shape[0] <= MOST_ROWS
+        for i, (entry, slot) in enumerate(zip(run, slots)):
             if entry.mix_input:
                 stream = self.pass_mix.forward(stream, first_share)
             if entry.add_vector is not None:
@@ -340,6 +343,10 @@ class DecoderModel:
                     raise RuntimeError("a block left a pass vector unadded: its first norm must fold the stream")
                 stream.row_addend = self.pass_vectors.weight[entry.add_vector]   # the layer's first norm adds it
             block = self.blocks[entry.layer]
+            if few:
+                follows = run[i + 1] if i + 1 < len(run) else None
+                step.next_norm = (self.blocks[follows.layer].norm_ahead(stream.h.shape[0])
+                                  if follows is not None and not follows.mix_input and follows.add_vector is None else None)
             stream = block.forward(stream, step, slot)
             if not block.leaves_rounded:
                 stream.rounded = None

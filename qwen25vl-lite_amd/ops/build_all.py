@@ -22,6 +22,7 @@ LIBRARIES = [
     ("gemm_tile", {}),
     ("gemm_rows", {}),
     ("gemm_slice", {}),
+    ("gemm_stream", {}),
     ("peaks", {}),
     ("gated", {}),
     ("moe", {}),

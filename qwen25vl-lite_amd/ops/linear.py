@@ -17,9 +17,9 @@ from typing import Optional, Union
 
 import torch
 
-from . import kernels, rows, skinny, tile
+from . import kernels, rows, skinny, stream, tile
 
-__all__ = ["NormedRows", "linear", "linear_into", "linear_stack", "linear_relu2", "gate_up_swiglu", "tune_library_products"]
+__all__ = ["NormedRows", "ScaledRows", "NormAhead", "linear", "linear_into", "linear_stack", "linear_relu2", "gate_up_swiglu", "tune_library_products"]
 
 
 class NormedRows:
@@ -32,6 +32,28 @@ class NormedRows:
 
     def materialize(self) -> torch.Tensor:
         return kernels.add_rmsnorm(self.h, None, self.weight, self.eps, self.dtype)
+
+
+class ScaledRows(NormedRows):
+    """The same, with what the kernel that wrote ``h`` last left of it: ``rows`` (bfloat16) are ``h * weight``, and the first ``parts`` numbers of
+    a row of ``squares`` add up to its sum of squares (:func:`stream.stream_into`).  Good until ``h`` changes."""
+
+    def __init__(self, h, weight, eps, dtype, rows: torch.Tensor, squares: torch.Tensor, parts: int):
+        super().__init__(h, weight, eps, dtype)
+        self.rows, self.squares, self.parts = rows, squares, parts
+
+    @property
+    def scaled(self):
+        return self.squares, self.parts, self.eps
+
+
+class NormAhead:
+    """The norm behind a product that is added to the residual, where what reads the norm takes :class:`ScaledRows`: the
+    product's kernel leaves them in ``left`` if it can."""
+
+    def __init__(self, weight: torch.Tensor, eps: float, dtype: torch.dtype):
+        self.weight, self.eps, self.dtype = weight, eps, dtype
+        self.left: Optional[ScaledRows] = None
 
 
 def _many_rows(x: torch.Tensor, weight: torch.Tensor, bias, out_dtype, out: Optional[torch.Tensor] = None) -> torch.Tensor:
@@ -120,13 +142,28 @@ def _aligned(x: torch.Tensor) -> bool:
     return x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
 
 
-def linear_into(residual: Optional[torch.Tensor], x: torch.Tensor, weight: torch.Tensor) -> Optional[torch.Tensor]:
+# Long inner sizes (``skinny.prefers_split``) are added in place where a norm waits for the rows that are left then; without one, up to here: the product
+# and the norm behind it, in place and in slabs, 8 rows of 3,584 x 18,944 27.1 us and 28.9, 2,048 x 11,008 13.1 and 14.0, 4,096 x 14,336 24.8 and
+# 24.8, 8,192 x 29,568 81.4 and 83.1; 16 rows 31.5 and 29.5, 15.1 and 15.2, 27.1 and 26.6, 85.0 and 81.8 (left for the norm: 28.3, 13.0, 23.9, 81.0).
+IN_PLACE_ROWS = 8
+
+
+def linear_into(residual: Optional[torch.Tensor], x: torch.Tensor, weight: torch.Tensor,
+                ahead: Optional[NormAhead] = None, in_place: bool = False) -> Optional[torch.Tensor]:
     """``residual += x @ weight.T`` inside the product's kernel where that exists (few bfloat16
-    rows): then None is returned.  Otherwise what is to be added is returned and the caller hands
+    rows): then None is returned (and the rows that the norm ``ahead`` asks for may be left in it); ``in_place``: the caller is no better off
+    with slabs.  Otherwise what is to be added is returned and the caller hands
     it on to whoever adds it (the next norm's kernel): the product ``[M, N]``, or float32
     ``[slabs, M, N]`` whose slabs are added in order (the split kernel; the tiled one over ranges of the inner size)."""
     m, k = x.shape
     fast = x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and _aligned(x)
+    if (fast and m <= stream.MOST_ROWS and residual is not None and residual.dtype == torch.float32 and residual.shape == (m, weight.shape[0]) and residual.stride(1) == 1
+            and residual.stride(0) >= residual.shape[1] and stream.takes_into(m, k, weight)
+            and (ahead is not None or (in_place and m <= IN_PLACE_ROWS) or not skinny.prefers_split(m, k, weight))):
+        left = stream.stream_into(residual, x, weight, None if ahead is None else ahead.weight)
+        if left is not None:
+            ahead.left = ScaledRows(residual, ahead.weight, ahead.eps, ahead.dtype, *left)
+        return None
     if fast and skinny.prefers_split(m, k, weight):
         return skinny.split_product(weight, x)
     if (fast and m <= skinny.ONE_BLOCK_ROWS and residual is not None and skinny.takes_resident(m, k, weight)
@@ -163,6 +200,8 @@ def gate_up_swiglu(x: Union[torch.Tensor, NormedRows], weight: torch.Tensor, gro
     rows) or ``grouped`` (alternating groups of 8 gate rows and 8 up rows).  With few bfloat16 rows
     and grouped rows the activation is applied inside the product's kernel."""
     m, k = x.shape
+    if grouped and isinstance(x, ScaledRows) and stream.takes_gated(m, k, weight):
+        return stream.stream_gated(x.rows, weight, act, x.scaled)
     if (grouped and weight.dtype == torch.bfloat16 and weight.is_cuda and weight.shape[0] % 16 == 0
             and m <= skinny.ONE_BLOCK_ROWS and not rows.wide(m, weight)):
         lazy = isinstance(x, NormedRows)

@@ -242,9 +242,13 @@ def _slice_weight(weight: torch.Tensor) -> bool:
 
 def slice_qkv_rope(weight: torch.Tensor, cs: torch.Tensor, x: torch.Tensor, bias: Optional[torch.Tensor], slots: Optional[torch.Tensor],
                    k_cache: Optional[torch.Tensor], v_cache: Optional[torch.Tensor], num_q_heads: int, num_kv_heads: int, head_dim: int,
-                   page_size: int) -> torch.Tensor:
-    """As :func:`qkv_rope_product`, where :func:`takes_slice` says so."""
+                   page_size: int, scaled=None) -> torch.Tensor:
+    """As :func:`qkv_rope_product`, where :func:`takes_slice` says so.  ``scaled``: ``(squares, parts, eps)`` of rows that
+    ``stream.stream_into`` left (up to 16)."""
     m, k = x.shape
+    squares, parts, eps = scaled if scaled is not None else (None, 0, 0.0)
+    if squares is not None and (m > ONE_TILE_ROWS or squares.dtype != torch.float32 or squares.shape != (m, 256) or not squares.is_contiguous()):
+        raise ValueError("squares must be float32 [M, 256] of at most 16 rows")
     nq, nkv, hd = int(num_q_heads), int(num_kv_heads), int(head_dim)
     n, cus, stride = (nq + 2 * nkv) * hd, _compute_units(x.device), x.stride()
     if (weight.shape != (n, k) or not _slice_fits(m, k, n, cus) or not _slice_weight(weight) or x.dtype != torch.bfloat16
@@ -266,11 +270,11 @@ def slice_qkv_rope(weight: torch.Tensor, cs: torch.Tensor, x: torch.Tensor, bias
     q_out = torch.empty((m, nq * hd), dtype=torch.bfloat16, device=x.device)
     fn = _fn("gemm_slice", "qvl_gemm_slice_rope", _SLICE_ARGS)
     _check(fn(x.data_ptr(), stride[0], weight.data_ptr(), weight.stride(0), _ptr(bias), cs.data_ptr(), slots_at, q_out.data_ptr(), k_at, v_at,
-              m, k, nq, nkv, hd, int(page_size), cus, _stream()), "linear (slices, rotation and cache write)")
+              m, k, nq, nkv, hd, int(page_size), cus, _ptr(squares), parts, eps, _stream()), "linear (slices, rotation and cache write)")
     return q_out
 
 
-_SLICE_ARGS = [_c_ptr, _c_int, _c_ptr, _c_int] + [_c_ptr] * 6 + [_c_int] * 7 + [_c_ptr]
+_SLICE_ARGS = [_c_ptr, _c_int, _c_ptr, _c_int] + [_c_ptr] * 6 + [_c_int] * 7 + [_c_ptr, _c_int, _c_float, _c_ptr]
 
 
 SPLIT_ROWS = 64   # the most rows that are cut along the inner size

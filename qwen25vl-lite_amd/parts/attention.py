@@ -12,9 +12,9 @@ from typing import Dict, Optional
 
 import torch
 
-from ..ops import kernels, skinny, tile
+from ..ops import kernels, skinny, stream, tile
 from ..ops.attention import paged_attention
-from ..ops.linear import NormedRows, linear, linear_into
+from ..ops.linear import NormedRows, ScaledRows, linear, linear_into
 from .base import (CacheNeed, LayerSlot, Mixer, ParamSpec, PartSpec, StateNeed, StepContext, build_part, rotation_key,
                    register_part)
 
@@ -78,6 +78,7 @@ class PagedAttention(Mixer):
 
     graph_safe = True
     takes_lazy_norm = True
+    leaves_ahead = True
 
     def __init__(self, params, dtype, device):
         super().__init__(dtype, device)
@@ -281,10 +282,15 @@ class PagedAttention(Mixer):
                             keep_first=self.keep_first, sinks=self.sink, chunk=self.chunk)
         return self._output(o, step)
 
+    def takes_scaled(self, rows: int) -> bool:
+        # (csrc/gemm_slice.hip divides the sums by the rows' root mean squares)
+        return (not self.normed_path and self.dtype == torch.bfloat16 and rows <= stream.MOST_ROWS
+                and skinny.takes_slice(rows, self.hidden, self.w_in, self.hd, self.position.rotary_tables(self.hd)[0].shape[0], None))
+
     def _output(self, o: torch.Tensor, step: StepContext):
         """The output projection: into the residual where the block offers it and there is no bias."""
         if self.b_out is None:
-            return linear_into(step.residual, o, self.w_out)
+            return linear_into(step.residual, o, self.w_out, getattr(step, "ahead", None))
         return linear(o, self.w_out, self.b_out,
                       out_dtype=torch.float32 if o.shape[0] <= skinny.ONE_BLOCK_ROWS else None)
 
@@ -366,16 +372,16 @@ class PagedAttention(Mixer):
     def _project_few_rows(self, x, step, group, slot, write, inv_freq, freq_row) -> Optional[torch.Tensor]:
         """A decode step's few bfloat16 rows: projection, bias, rotation and cache write in one
         kernel (the float32 sums never leave it)."""
-        lazy = isinstance(x, NormedRows)
+        lazy, scaled = isinstance(x, NormedRows), isinstance(x, ScaledRows)
         m, k = x.shape
-        if self.dtype == torch.bfloat16 and m <= skinny.RESIDENT_ROWS and (not lazy or m > LAZY_ROWS or k > skinny.NARROW_K) and skinny.takes_slice(
+        if self.dtype == torch.bfloat16 and m <= skinny.RESIDENT_ROWS and (not lazy or scaled or m > LAZY_ROWS or k > skinny.NARROW_K) and skinny.takes_slice(
                 m, k, self.w_in, self.hd, inv_freq.shape[0], slot.k_cache.dtype if write else None):
-            rows = x.materialize() if lazy else x
+            rows = x.rows if scaled else x.materialize() if lazy else x
             if rows.dtype == torch.bfloat16 and rows.stride(1) == 1 and rows.stride(0) % 8 == 0 and rows.data_ptr() % 16 == 0:
                 return skinny.slice_qkv_rope(
                     self.w_in, self._rotation_table(step, inv_freq, freq_row, m), rows, self.b_in, group.slot_mapping if write else None,
                     slot.k_cache if write else None, slot.v_cache if write else None, self.nq, self.nkv if write else 0, self.hd,
-                    group.page_size)
+                    group.page_size, x.scaled if scaled else None)
         if not lazy and m > FUSED_ROWS and _splits(m, self.w_in.shape[0], k):
             return None
         if self.dtype != torch.bfloat16 or not skinny.takes_qkv_rope(

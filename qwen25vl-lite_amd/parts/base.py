@@ -164,6 +164,10 @@ class StepContext:
     # (key, position encoding, head width) of the rotation tables that the pass's mixers will look for
     rotations: Sequence[Any] = ()
     residual: Optional[torch.Tensor] = None   # set by a block while a part may add its result in place
+    # set with it: the norm that stands behind that part (ops.linear.NormAhead), whose rows the product that adds may leave
+    ahead: Any = None
+    # set by the model: the first norm of the block that comes next, where that block takes such rows
+    next_norm: Any = None
     # the model's second table of token rows [vocab, columns], where it has one: layers read columns of their own
     token_side: Optional[torch.Tensor] = None
     derived: Dict[Any, Any] = field(default_factory=dict)   # per-step arrays kernels derive once (tile lists)
@@ -189,6 +193,9 @@ class ResidualStream:
     copies: Optional[torch.Tensor] = None
     # (mix [copies, copies], out [copies]) float32: how the pending addend joins the copies
     pending_join: Optional[Tuple[torch.Tensor, torch.Tensor]] = None
+    # what the last product left of ``h`` for the norm that comes next (ops.linear.ScaledRows): set by a block for the one right
+    # behind it, which asked for it
+    scaled: Any = None
     # ``h`` rounded to the run dtype, where the kernel that wrote ``h`` last wrote that too (a block that leaves it
     # says so: ``Block.leaves_rounded``)
     rounded: Optional[torch.Tensor] = None
@@ -251,6 +258,8 @@ class Part:
 
     graph_safe: bool = False
     takes_lazy_norm: bool = False   # forward accepts NormedRows in place of the normalised tensor
+    # what forward adds to ``step.residual`` is one product, the last thing it does, which leaves rows for the norm in ``step.ahead``
+    leaves_ahead: bool = False
 
     def __init__(self, dtype: torch.dtype, device: torch.device):
         self.dtype = dtype
@@ -264,6 +273,10 @@ class Part:
 
     def sub_parts(self) -> Dict[str, "Part"]:
         return {}
+
+    def takes_scaled(self, rows: int) -> bool:
+        """Whether :meth:`forward` makes use of ScaledRows of so many rows."""
+        return False
 
     def cache_need(self) -> Optional[CacheNeed]:
         """Keys and values this part keeps per token in pages, or None."""
@@ -280,6 +293,10 @@ class Norm(Part):
         """Fold ``stream.pending`` into ``stream.h`` and return the normalised rows; with ``lazy`` it
         may return :class:`~qwen25vl_lite_amd.ops.linear.NormedRows` instead of computing them."""
         raise NotImplementedError
+
+    def ahead(self):
+        """This norm as an ops.linear.NormAhead, or None where no product can leave its rows."""
+        return None
 
 
 def rotation_key(position, width: int):
@@ -330,6 +347,10 @@ class PositionEncoding(Part):
 
 class Block(Part):
     leaves_rounded: bool = False    # forward leaves ``stream.rounded`` equal to the ``stream.h`` it leaves
+
+    def norm_ahead(self, rows: int):
+        """The block's first norm as a NormAhead, where the block takes ScaledRows in ``stream.scaled``; else None."""
+        return None
 
     def forward(self, stream: ResidualStream, step: StepContext, slot: LayerSlot) -> ResidualStream:
         raise NotImplementedError

@@ -6,6 +6,7 @@ from typing import Dict, Optional
 
 import torch
 
+from ..ops.stream import MOST_ROWS
 from .base import Block, LayerSlot, Part, PartSpec, ResidualStream, StepContext, SumTerm, build_part, register_part
 
 __all__ = ["PreNormBlock", "ParallelBlock", "SandwichBlock", "PostNormBlock", "SumNormBlock"]
@@ -34,14 +35,29 @@ class PreNormBlock(Block):
         return {self.names["norm1"]: self.norm1, self.names["mixer"]: self.mixer,
                 self.names["norm2"]: self.norm2, self.names["ffn"]: self.ffn}
 
+    def norm_ahead(self, rows: int):
+        return self.norm1.ahead() if self.mixer.takes_scaled(rows) else None
+
     def forward(self, stream: ResidualStream, step: StepContext, slot: LayerSlot) -> ResidualStream:
-        x = self.norm1.forward(stream, lazy=self.mixer.takes_lazy_norm)
+        x, stream.scaled = stream.scaled, None
+        if x is None:
+            x = self.norm1.forward(stream, lazy=self.mixer.takes_lazy_norm)
         step.residual = stream.h            # the mixer may add its result in place and return None
+        rows = stream.h.shape[0]
+        ahead = None
+        if rows <= MOST_ROWS and self.mixer.leaves_ahead and self.ffn.takes_scaled(rows):
+            ahead = step.ahead = self.norm2.ahead()
         stream.pending = self.mixer.forward(x, step, slot.of(self.names["mixer"]))
-        y = self.norm2.forward(stream, lazy=self.ffn.takes_lazy_norm)
+        if ahead is not None and ahead.left is not None:
+            y = ahead.left                  # the kernel that added the mixer's result has left the norm's rows
+        else:
+            y = self.norm2.forward(stream, lazy=self.ffn.takes_lazy_norm)
         step.residual = stream.h
+        ahead = step.ahead = getattr(step, "next_norm", None) if self.ffn.leaves_ahead else None
         stream.pending = self.ffn.forward(y, step)
-        step.residual = None
+        if ahead is not None:
+            stream.scaled = ahead.left
+        step.residual = step.ahead = None
         return stream
 
 

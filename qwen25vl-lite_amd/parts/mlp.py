@@ -6,6 +6,7 @@ from typing import Dict, Optional
 
 import torch
 
+from ..ops import stream
 from ..ops.linear import gate_up_swiglu, linear_into
 from .base import FeedForward, ParamSpec, StepContext, register_part
 
@@ -22,6 +23,7 @@ class SwiGLU(FeedForward):
 
     graph_safe = True
     takes_lazy_norm = True
+    leaves_ahead = True
 
     def __init__(self, params, dtype, device):
         super().__init__(dtype, device)
@@ -64,9 +66,14 @@ class SwiGLU(FeedForward):
         return {f"{self.names['gate']}.weight": gate, f"{self.names['up']}.weight": up,
                 f"{self.names['down']}.weight": self.w_down}
 
+    def takes_scaled(self, rows: int) -> bool:
+        return self.grouped and self.dtype == torch.bfloat16 and stream.takes_gated(rows, self.hidden, self.w_gate_up)
+
     def forward(self, x, step: StepContext):
         act = gate_up_swiglu(x, self.w_gate_up, self.grouped, self.activation)
-        return linear_into(step.residual if step is not None else None, act, self.w_down)
+        if step is None:
+            return linear_into(None, act, self.w_down)
+        return linear_into(step.residual, act, self.w_down, getattr(step, "ahead", None), in_place=True)
 
 
 class ClampedGatedFF(FeedForward):
@@ -121,13 +128,13 @@ class ClampedGatedFF(FeedForward):
         # (37,888 x 3,584, 8 rows: 44 us; the resident kernel's product 45 and the activation's kernel 5)
         if x.is_cuda and self.w_gate_up.is_cuda and rows.takes_rows(x, self.w_gate_up) and rows.many_outputs(self.w_gate_up):
             act = rows.rows_gated(x, self.w_gate_up, self.alpha, self.limit, self.shift)
-            return linear_into(step.residual if step is not None else None, act, self.w_down)
+            return linear_into(step.residual if step is not None else None, act, self.w_down, in_place=True)
         if x.is_cuda and tile.prefers_tile(x, self.w_gate_up, halves=True):
             act = tile.tile_gated(x, self.w_gate_up, self.alpha, self.limit, self.shift)
-            return linear_into(step.residual if step is not None else None, act, self.w_down)
+            return linear_into(step.residual if step is not None else None, act, self.w_down, in_place=True)
         both = linear(x, self.w_gate_up)
         act = gated_act(both if both.is_contiguous() else both.contiguous(), self.alpha, self.limit, self.shift)
-        return linear_into(step.residual if step is not None else None, act, self.w_down)
+        return linear_into(step.residual if step is not None else None, act, self.w_down, in_place=True)
 
 
 class PlainFF(FeedForward):
@@ -184,7 +191,7 @@ class PlainFF(FeedForward):
             z = linear(x, self.w_up)
             z = z if z.is_contiguous() else z.contiguous()
             act = rownorm.normed_powers(z, self.coeff, self.eps, self.dtype)
-        return linear_into(step.residual if step is not None else None, act, self.w_down)
+        return linear_into(step.residual if step is not None else None, act, self.w_down, in_place=True)
 
 
 register_part("ffn", "swiglu", SwiGLU)

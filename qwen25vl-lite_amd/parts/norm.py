@@ -7,7 +7,7 @@ from typing import Dict, Optional
 import torch
 
 from ..ops import kernels, skinny
-from ..ops.linear import NormedRows
+from ..ops.linear import NormAhead, NormedRows
 from .base import Norm, ParamSpec, ResidualStream, SumTerm, register_part
 
 __all__ = ["RMSNorm", "LayerNorm"]
@@ -57,6 +57,10 @@ class RMSNorm(Norm):
             stream.pending = None  # folded into h
         return out
 
+
+    def ahead(self) -> Optional[NormAhead]:
+        """This norm for the product in front of it, which may leave its rows."""
+        return NormAhead(self.weight, self.eps, self.dtype) if self.dtype == torch.bfloat16 else None
 
     def forward_pair(self, stream: ResidualStream, other: "RMSNorm"):
         """Fold what is pending into the sum and return its rows normed under this norm's gain and under
