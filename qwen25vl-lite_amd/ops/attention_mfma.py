@@ -277,6 +277,18 @@ def block_groups(walks: int, places: int, head_dim: int, cut: bool = True) -> in
     return 2 if most >= 2 and walks * (4 if cut else 1) <= places else 1
 
 
+_COOP_ARGS = [_c_ptr] * 4 + [_c_int] + [_c_ptr] * 4 + [_c_int, _c_ptr, _c_ptr] + [_c_int] * 4 + [_c_float, _c_int, _c_int, _c_ptr]
+_MERGED_ARGS = [_c_ptr] * 4 + [_c_int] + [_c_ptr] * 4 + [_c_int] + [_c_ptr] * 5 + [_c_ll] + [_c_int] * 4 + [_c_float, _c_int, _c_int, _c_ptr]
+
+
+def _step_splits(step, group: int, nkv: int, device):
+    """:func:`plan_splits` of all of the step's tokens, the same for every layer with these heads (and for as long as what it goes by)."""
+    key = ("splits", group, nkv, TARGET_BLOCKS, FILL_BLOCKS, MIN_KEYS_PER_SPLIT, SPLIT_FROM_KEYS)
+    if key not in step.derived:
+        step.derived[key] = plan_splits(_count_tiles(step, group, 1), nkv, step.max_ctx_len, device)
+    return step.derived[key]
+
+
 def try_attention(q, k_cache, v_cache, block_table, step, num_q_heads: int, window: Optional[int],
                   scale: float, force_groups: Optional[int] = None, force_wide: Optional[bool] = None,
                   sinks: Optional[torch.Tensor] = None,
@@ -305,7 +317,7 @@ def try_attention(q, k_cache, v_cache, block_table, step, num_q_heads: int, wind
     gate_args = (_ptr(gate), 0 if gate is None else gate.stride(0))
     out = torch.empty_like(q)
     defines = {"HD": hd}
-    kind, nsplit, per = plan_splits(_count_tiles(step, nq // nkv, 1), nkv, step.max_ctx_len, q.device)
+    kind, nsplit, per = _step_splits(step, nq // nkv, nkv, q.device)
 
     def many_tiles(only):
         wide, groups, defines, plan, items = _step_walks(step, nq // nkv, nkv, hd, int(window or 0), q.device, only, force_wide, force_groups)
@@ -344,9 +356,7 @@ def try_attention(q, k_cache, v_cache, block_table, step, num_q_heads: int, wind
         if merged or sinks is not None or gate is not None:
             # the block of each (tile, head) that finishes last merges the splits: one launch
             counters = _counters(q.device) if merged else None
-            fn = _fn("attention_mfma", "qvl_attn_mfma_coop_merged",
-                     [_c_ptr] * 4 + [_c_int] + [_c_ptr] * 4 + [_c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ll] + [_c_int] * 4
-                     + [_c_float, _c_int, _c_int, _c_ptr], defines)
+            fn = _fn("attention_mfma", "qvl_attn_mfma_coop_merged", _MERGED_ARGS, defines)
             code = fn(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), block_table.shape[1], _ptr(cu_q),
                       _ptr(step.ctx_len), _ptr(tile_req), _ptr(tile_ct), num_tiles, _ptr(out), _ptr(scratch),
                       _ptr(counters), _ptr(sinks), *gate_args, nq, nkv, ps, int(window or 0), float(scale), nsplit, per, _stream())
@@ -356,9 +366,7 @@ def try_attention(q, k_cache, v_cache, block_table, step, num_q_heads: int, wind
             taken["shared tiles, keys split among blocks, merged in the launch" if merged else "shared tiles"
                   + (", keys split among blocks, merged by a second launch" if nsplit > 1 else "")] += 1
             return
-        fn = _fn("attention_mfma", "qvl_attn_mfma_coop",
-                 [_c_ptr] * 4 + [_c_int] + [_c_ptr] * 4 + [_c_int, _c_ptr, _c_ptr] + [_c_int] * 4
-                 + [_c_float, _c_int, _c_int, _c_ptr], defines)
+        fn = _fn("attention_mfma", "qvl_attn_mfma_coop", _COOP_ARGS, defines)
         _check(fn(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), block_table.shape[1], _ptr(cu_q),
                   _ptr(step.ctx_len), _ptr(tile_req), _ptr(tile_ct), num_tiles, _ptr(out), _ptr(scratch), nq, nkv, ps,
                   int(window or 0), float(scale), nsplit, per, _stream()),

@@ -34,7 +34,7 @@ _functions: Dict[Tuple[str, str, Tuple], ctypes._CFuncPtr] = {}
 
 
 def _fn(stem: str, name: str, argtypes, defines=None, restype=_c_int):
-    key = (stem, name, tuple(sorted(defines.items())) if defines else ())
+    key = (stem, name, tuple(sorted(defines.items()))) if defines else (stem, name)
     fn = _functions.get(key)
     if fn is None:
         fn = getattr(load_library(stem, defines), name)
@@ -148,32 +148,40 @@ def add_rmsnorm(h: torch.Tensor, delta: Optional[torch.Tensor], weight: torch.Te
     ``delta`` may be float32 ``[slabs, N, H]``: partial sums of a product that was cut along its
     inner size, added in slab order.
     """
-    _dev(h, delta, weight, rows, out)
+    if not (h.is_cuda and weight.is_cuda):
+        _dev(h, weight)
     _need(h.dtype == torch.float32 and h.dim() == 2 and h.is_contiguous(), "h must be contiguous float32 [N, H]")
     n, width = h.shape
     _need(weight.dtype == torch.float32 and weight.shape == (width,) and weight.is_contiguous(),
           "norm weight must be float32 [H]")
-    nslabs, slab_stride = 1, 0
-    if delta is not None and delta.dim() == 3:
-        _need(delta.dtype == torch.float32 and tuple(delta.shape[1:]) == tuple(h.shape) and delta.is_contiguous(),
-              "slabs of delta must be contiguous float32 [slabs, N, H]")
-        nslabs, slab_stride = delta.shape[0], n * width
-    elif delta is not None:
-        _need(delta.shape == h.shape and delta.is_contiguous(), "delta must match h's shape")
+    nslabs, slab_stride, delta_at, delta_dtype = 1, 0, None, out_dtype
+    if delta is not None:
+        if not delta.is_cuda:
+            _dev(delta)
+        delta_at, delta_dtype = delta.data_ptr(), delta.dtype
+        if delta.dim() == 3:
+            _need(delta_dtype == torch.float32 and delta.shape[1:] == h.shape and delta.is_contiguous(),
+                  "slabs of delta must be contiguous float32 [slabs, N, H]")
+            nslabs, slab_stride = delta.shape[0], n * width
+        else:
+            _need(delta.shape == h.shape and delta.is_contiguous(), "delta must match h's shape")
     m = n
     if rows is not None:
+        _dev(rows)
         _need(rows.dtype == torch.int32 and rows.dim() == 1 and rows.is_contiguous(), "rows must be int32 [M]")
         m = rows.shape[0]
     if out is None:
         out = torch.empty((m, width), dtype=out_dtype, device=h.device)
-    _need(out.shape == (m, width) and out.dtype == out_dtype and out.is_contiguous(), "out must be [M, H]")
-    fn = _fn("elementwise", "qvl_add_rmsnorm",
-             [_c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_float, _c_int, _c_int, _c_int,
-              ctypes.c_longlong, _c_ptr])
-    _check(fn(_ptr(h), _ptr(delta), _ptr(weight), _ptr(out), _ptr(rows), m, width, float(eps),
-              dtype_code(delta.dtype if delta is not None else out_dtype), dtype_code(out_dtype), nslabs, slab_stride,
-              _stream()), "add_rmsnorm")
+    else:
+        _dev(out)
+        _need(out.shape == (m, width) and out.dtype == out_dtype and out.is_contiguous(), "out must be [M, H]")
+    fn = _fn("elementwise", "qvl_add_rmsnorm", _ADD_RMSNORM_ARGS)
+    _check(fn(h.data_ptr(), delta_at, weight.data_ptr(), out.data_ptr(), _ptr(rows), m, width, eps, dtype_code(delta_dtype),
+              dtype_code(out_dtype), nslabs, slab_stride, _stream()), "add_rmsnorm")
     return out
+
+
+_ADD_RMSNORM_ARGS = [_c_ptr] * 5 + [_c_int, _c_int, _c_float, _c_int, _c_int, _c_int, ctypes.c_longlong, _c_ptr]
 
 
 def rope_kv_write(x: torch.Tensor, bias: Optional[torch.Tensor], positions: torch.Tensor, inv_freq: torch.Tensor,
@@ -199,14 +207,13 @@ def rope_kv_write(x: torch.Tensor, bias: Optional[torch.Tensor], positions: torc
     _dev(x, bias, positions, inv_freq, freq_row, slots, k_cache, v_cache, q_out)
     nq, nkv, hd = int(num_q_heads), int(num_kv_heads), int(head_dim)
     cols = (nq + 2 * nkv) * hd
-    nslabs, slab_stride = 1, 0
-    if x.dim() == 3:
-        _need(x.dtype == torch.float32 and x.is_contiguous() and cs is not None,
+    nslabs, slab_stride, stride, shape = 1, 0, x.stride(), x.shape
+    if len(shape) == 3:
+        _need(x.dtype == torch.float32 and x.is_contiguous() and cs is not None and shape[0] > 0,
               "slabs of x must be contiguous float32 and come with the table of cosines and sines")
-        nslabs, slab_stride = x.shape[0], x.stride(0)
-        x = x[0]
-    n = x.shape[0]
-    _need(x.dim() == 2 and x.shape[1] == cols and x.stride(1) == 1, "x must be [N, (nq + 2 nkv) hd]")
+        nslabs, slab_stride, stride, shape = shape[0], stride[0], stride[1:], shape[1:]
+    n = shape[0]
+    _need(len(shape) == 2 and shape[1] == cols and stride[1] == 1, "x must be [N, (nq + 2 nkv) hd]")
     odt = out_dtype or x.dtype
     rot_half = inv_freq.shape[0]
     _need(inv_freq.dtype == torch.float32 and inv_freq.is_contiguous() and 2 * rot_half <= hd,
@@ -223,10 +230,11 @@ def rope_kv_write(x: torch.Tensor, bias: Optional[torch.Tensor], positions: torc
               "slots must be int32 [N]")
         _need(k_cache is not None and v_cache is not None and k_cache.dtype == odt and v_cache.dtype == odt,
               "the cache must have the activation dtype")
-        _need(k_cache.is_contiguous() and k_cache.dim() == 4 and tuple(k_cache.shape[1:]) == (nkv, page_size, hd),
+        kshape, vshape = k_cache.shape, v_cache.shape
+        _need(k_cache.is_contiguous() and len(kshape) == 4 and kshape[1:] == (nkv, page_size, hd),
               "k_cache must be [pages, nkv, page_size, hd]")
-        _need(v_cache.is_contiguous() and v_cache.dim() == 4 and tuple(v_cache.shape[1:]) == (nkv, hd, page_size)
-              and v_cache.shape[0] == k_cache.shape[0], "v_cache must be [pages, nkv, hd, page_size]")
+        _need(v_cache.is_contiguous() and len(vshape) == 4 and vshape[1:] == (nkv, hd, page_size)
+              and vshape[0] == kshape[0], "v_cache must be [pages, nkv, hd, page_size]")
     if q_out is None:
         q_out = torch.empty((n, nq * hd), dtype=odt, device=x.device)
     _need(q_out.shape == (n, nq * hd) and q_out.dtype == odt and q_out.is_contiguous(), "q_out must be [N, nq hd]")
@@ -234,14 +242,15 @@ def rope_kv_write(x: torch.Tensor, bias: Optional[torch.Tensor], positions: torc
         _dev(cs)
         _need(cs.dtype == torch.float32 and cs.is_contiguous() and cs.dim() == 3 and cs.shape[0] >= n
               and tuple(cs.shape[1:]) == (rot_half, 2), "cs must be float32 [N, rot/2, 2]")
-    fn = _fn("elementwise", "qvl_rope_kv_write",
-             [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_int, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr, _c_ptr,
-              _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, ctypes.c_longlong, _c_ptr])
-    _check(fn(_ptr(x), x.stride(0), _ptr(bias), _ptr(positions), positions.stride(0), _ptr(inv_freq),
+    fn = _fn("elementwise", "qvl_rope_kv_write", _ROPE_ARGS)
+    _check(fn(_ptr(x), stride[0], _ptr(bias), _ptr(positions), positions.stride(0), _ptr(inv_freq),
               _ptr(freq_row), _ptr(cs), _ptr(slots), _ptr(q_out), _ptr(k_cache), _ptr(v_cache), n, nq, nkv, hd, rot_half,
               int(page_size), dtype_code(x.dtype), dtype_code(odt), int(nslabs), int(slab_stride), _stream()),
            "rope_kv_write")
     return q_out
+
+
+_ROPE_ARGS = [_c_ptr, _c_int, _c_ptr, _c_ptr, _c_int] + [_c_ptr] * 7 + [_c_int] * 9 + [ctypes.c_longlong, _c_ptr]
 
 
 def _check_rotation(positions: torch.Tensor, inv_freq: torch.Tensor, freq_row: torch.Tensor, n: int) -> None:

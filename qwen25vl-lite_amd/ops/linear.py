@@ -215,5 +215,5 @@ def gate_up_swiglu(x: Union[torch.Tensor, NormedRows], weight: torch.Tensor, gro
         if rows.prefers_rows(x, weight):
             return rows.rows_swiglu(x, weight, act)
         if x.is_cuda and tile.prefers_tile(x, weight, gated=True):
-            return tile.tile_swiglu(x, weight, act)
+            return tile.tile_swiglu(x, weight, act, taken=True)
     return kernels.swiglu(linear(x, weight), grouped=grouped, act=act)

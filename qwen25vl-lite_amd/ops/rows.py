@@ -25,7 +25,7 @@ def _aligned(t: torch.Tensor) -> bool:
 def takes_rows(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """Whether the kernel takes ``x [M, K] @ weight[N, K].T``: up to 64 bfloat16 rows on 16-byte boundaries, an inner size in
     steps of 8, operands within 32-bit byte offsets."""
-    return (x.is_cuda and weight.is_cuda and x.dtype == weight.dtype == torch.bfloat16 and x.dim() == 2 and weight.dim() == 2
+    return (x.dim() == 2 and x.shape[0] <= MOST_ROWS and x.is_cuda and weight.is_cuda and x.dtype == weight.dtype == torch.bfloat16 and weight.dim() == 2
             and x.shape[1] == weight.shape[1] and 0 < x.shape[0] <= MOST_ROWS and x.shape[1] > 0 and x.shape[1] % 8 == 0
             and _aligned(x) and _aligned(weight) and ((weight.shape[0] - 1) * weight.stride(0) + x.shape[1]) * 2 < _REACH
             and ((x.shape[0] - 1) * x.stride(0) + x.shape[1]) * 2 < _REACH)

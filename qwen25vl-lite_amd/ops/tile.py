@@ -3,6 +3,7 @@
 from __future__ import annotations
 
 import ctypes
+from functools import lru_cache
 from typing import Optional
 
 import torch
@@ -17,19 +18,32 @@ _STORE, _SLABS, _GROUPED, _HALVES = range(4)
 _REACH = 0xffff0000      # bytes that a tile's rows may span from its first
 
 
-def _rows_aligned(t: torch.Tensor) -> bool:
-    return t.stride(1) == 1 and t.stride(0) % 8 == 0 and t.stride(0) >= t.shape[1] and t.data_ptr() % 16 == 0
+def _entry(name: str, argtypes):
+    """A function of the library, looked up at its first call (a step of many layers makes several calls a layer and waits for the host)."""
+    found = []
+
+    def call(*args):
+        if not found:
+            found.append(_fn("gemm_tile", name, argtypes))
+        return found[0](*args)
+    return call
+
+
+_blocks_of = lru_cache(maxsize=4096)(_entry("qvl_gemm_tile_blocks", [_c_int] * 4))      # (numbers of the sizes alone)
+_splits_of = lru_cache(maxsize=4096)(_entry("qvl_gemm_tile_splits", [_c_int] * 4))
+_tile = _entry("qvl_gemm_tile", [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ll] + [_c_int] * 7 + [_c_float] * 3 + [_c_int, _c_int, _c_ptr])
+_heads = _entry("qvl_gemm_tile_heads", [_c_ptr, _c_ll, _c_ptr, _c_ll] + [_c_ptr] * 6 + [_c_int] * 7 + [_c_ptr])
 
 
 def takes_tile(x: torch.Tensor, weight: torch.Tensor, halves: bool = False) -> bool:
     """Whether the kernel takes ``x [M, K] @ weight[N, K].T``: bfloat16 rows on 16-byte boundaries, an inner size in steps
     of 32, and rows that lie within 32-bit offsets of a tile's first (``halves``: the up rows, N / 2 further on, too)."""
-    if not (x.is_cuda and weight.is_cuda and x.dtype == weight.dtype == torch.bfloat16 and x.dim() == 2 and weight.dim() == 2
-            and x.shape[1] == weight.shape[1] and x.shape[0] > 0 and x.shape[1] > 0 and x.shape[1] % 32 == 0
-            and _rows_aligned(x) and _rows_aligned(weight)):
+    if not (x.is_cuda and weight.is_cuda and x.dtype == weight.dtype == torch.bfloat16 and x.dim() == 2 and weight.dim() == 2):
         return False
-    span = 256 + (weight.shape[0] // 2 if halves else 0)
-    return span * weight.stride(0) * 2 < _REACH and 256 * x.stride(0) * 2 < _REACH
+    (m, k), (n, wk) = x.shape, weight.shape
+    (ldx, sx), (ldw, sw) = x.stride(), weight.stride()
+    return (k == wk and m > 0 and k > 0 and k % 32 == 0 and sx == 1 and sw == 1 and ldx % 8 == 0 and ldw % 8 == 0 and ldx >= k and ldw >= k
+            and (x.data_ptr() | weight.data_ptr()) % 16 == 0 and (256 + (n // 2 if halves else 0)) * ldw * 2 < _REACH and 256 * ldx * 2 < _REACH)
 
 
 MANY_ROWS = 64           # up to here the decode kernels and the library run
@@ -44,16 +58,14 @@ def prefers_tile(x: torch.Tensor, weight: torch.Tensor, halves: bool = False, ga
     if x.shape[0] <= MANY_ROWS or not takes_tile(x, weight, halves):
         return False
     cus = compute_units(x.device)
-    blocks = int(_fn("gemm_tile", "qvl_gemm_tile_blocks", [_c_int] * 4)(x.shape[0], weight.shape[0], x.shape[1], cus))
+    blocks = _blocks_of(x.shape[0], weight.shape[0], x.shape[1], cus)
     return 2 * blocks >= cus if gated or halves else 4 * blocks >= 3 * cus
 
 
 def _launch(x, weight, out, ldo, mode, splits=1, relu2=0, gelu=0, alpha=1.0, limit=0.0, shift=0.0, shape=-1):
-    fn = _fn("gemm_tile", "qvl_gemm_tile", [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ll, _c_int, _c_int, _c_int, _c_int, _c_int,
-                                            _c_int, _c_int, _c_float, _c_float, _c_float, _c_int, _c_int, _c_ptr])
     m, k = x.shape
-    _check(fn(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(out), ldo, m, weight.shape[0], k, mode, splits, relu2,
-              gelu, alpha, limit, shift, shape, compute_units(x.device), _stream()), "linear (tiles)")
+    _check(_tile(x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), out.data_ptr(), ldo, m, weight.shape[0], k, mode, splits, relu2,
+                 gelu, alpha, limit, shift, shape, compute_units(x.device), _stream()), "linear (tiles)")
     return out
 
 
@@ -75,7 +87,7 @@ def slab_ranges(x: torch.Tensor, weight: torch.Tensor) -> int:
     not take the product or has few rows."""
     if x.shape[0] <= MANY_ROWS or not takes_tile(x, weight):
         return 0
-    return int(_fn("gemm_tile", "qvl_gemm_tile_splits", [_c_int] * 4)(x.shape[0], weight.shape[0], x.shape[1], compute_units(x.device)))
+    return _splits_of(x.shape[0], weight.shape[0], x.shape[1], compute_units(x.device))
 
 
 def tile_slabs(x: torch.Tensor, weight: torch.Tensor, ranges: Optional[int] = None) -> Optional[torch.Tensor]:
@@ -126,16 +138,16 @@ def tile_heads(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tenso
               and tuple(k_cache.shape[1:]) == (nkv, page_size, 128) and tuple(v_cache.shape[1:]) == (nkv, 128, page_size)
               and v_cache.shape[0] == k_cache.shape[0], "caches must be bfloat16 [pages, nkv, ps, 128] / [pages, nkv, 128, ps]")
     q_out = torch.empty((m, nq * 128), dtype=torch.bfloat16, device=x.device)
-    fn = _fn("gemm_tile", "qvl_gemm_tile_heads", [_c_ptr, _c_ll, _c_ptr, _c_ll] + [_c_ptr] * 6 + [_c_int] * 7 + [_c_ptr])
-    _check(fn(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), _ptr(cs), _ptr(slots if nkv else None), _ptr(q_out),
+    _check(_heads(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), _ptr(cs), _ptr(slots if nkv else None), _ptr(q_out),
               _ptr(k_cache if nkv else None), _ptr(v_cache if nkv else None), m, k, nq, nkv, int(page_size), shape,
               compute_units(x.device), _stream()), "linear (tiles, rotation and cache write)")
     return q_out
 
 
-def tile_swiglu(x: torch.Tensor, weight: torch.Tensor, act: str = "silu", shape: int = -1) -> torch.Tensor:
-    """``act(gate) * up`` for a weight whose rows come in groups of 8 gate and 8 up rows: bfloat16 ``[M, N / 2]``."""
-    _need(takes_tile(x, weight) and weight.shape[0] % 16 == 0, "the tiled kernel does not take this product")
+def tile_swiglu(x: torch.Tensor, weight: torch.Tensor, act: str = "silu", shape: int = -1, taken: bool = False) -> torch.Tensor:
+    """``act(gate) * up`` for a weight whose rows come in groups of 8 gate and 8 up rows: bfloat16 ``[M, N / 2]``.  ``taken``: :func:`takes_tile`
+    has just said so."""
+    _need((taken or takes_tile(x, weight)) and weight.shape[0] % 16 == 0, "the tiled kernel does not take this product")
     _need(act in ("silu", "gelu_tanh"), "the activation is silu or gelu_tanh")
     half = weight.shape[0] // 2
     out = torch.empty((x.shape[0], half), dtype=torch.bfloat16, device=x.device)

@@ -372,9 +372,11 @@ class PagedAttention(Mixer):
     def _project_few_rows(self, x, step, group, slot, write, inv_freq, freq_row) -> Optional[torch.Tensor]:
         """A decode step's few bfloat16 rows: projection, bias, rotation and cache write in one
         kernel (the float32 sums never leave it)."""
-        lazy, scaled = isinstance(x, NormedRows), isinstance(x, ScaledRows)
         m, k = x.shape
-        if self.dtype == torch.bfloat16 and m <= skinny.RESIDENT_ROWS and (not lazy or scaled or m > LAZY_ROWS or k > skinny.NARROW_K) and skinny.takes_slice(
+        if m > skinny.RESIDENT_ROWS:
+            return None
+        lazy, scaled = isinstance(x, NormedRows), isinstance(x, ScaledRows)
+        if self.dtype == torch.bfloat16 and (not lazy or scaled or m > LAZY_ROWS or k > skinny.NARROW_K) and skinny.takes_slice(
                 m, k, self.w_in, self.hd, inv_freq.shape[0], slot.k_cache.dtype if write else None):
             rows = x.rows if scaled else x.materialize() if lazy else x
             if rows.dtype == torch.bfloat16 and rows.stride(1) == 1 and rows.stride(0) % 8 == 0 and rows.data_ptr() % 16 == 0:
