@@ -157,10 +157,10 @@ def linear_into(residual: Optional[torch.Tensor], x: torch.Tensor, weight: torch
     ``[slabs, M, N]`` whose slabs are added in order (the split kernel; the tiled one over ranges of the inner size)."""
     m, k = x.shape
     fast = x.is_cuda and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and _aligned(x)
-    if (fast and m <= stream.MOST_ROWS and residual is not None and residual.dtype == torch.float32 and residual.shape == (m, weight.shape[0]) and residual.stride(1) == 1
-            and residual.stride(0) >= residual.shape[1] and stream.takes_into(m, k, weight)
-            and (ahead is not None or (in_place and m <= IN_PLACE_ROWS) or not skinny.prefers_split(m, k, weight))):
-        left = stream.stream_into(residual, x, weight, None if ahead is None else ahead.weight)
+    if (fast and m <= stream.MOST_ROWS and residual is not None and residual.dtype == torch.float32 and residual.stride(1) == 1
+            and (ahead is not None or (in_place and m <= IN_PLACE_ROWS) or not skinny.prefers_split(m, k, weight))
+            and residual.shape == (m, weight.shape[0]) and residual.stride(0) >= residual.shape[1] and stream.takes_into(m, k, weight)):
+        left = stream.stream_into(residual, x, weight, None if ahead is None else ahead.weight, taken=True)
         if left is not None:
             ahead.left = ScaledRows(residual, ahead.weight, ahead.eps, ahead.dtype, *left)
         return None

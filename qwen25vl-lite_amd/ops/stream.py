@@ -26,14 +26,11 @@ MOST_TILES = 4         # tiles of 16 rows of W a block takes where the product i
 MOST_GATED_TILES = 16  # tiles of 8 channels (STREAM_MOST_GATED)
 
 
-def _aligned(t: torch.Tensor) -> bool:
-    stride = t.stride()
-    return stride[1] == 1 and stride[0] % 8 == 0 and stride[0] >= t.shape[1] and t.data_ptr() % 16 == 0
-
-
 def _fits(m: int, k: int, weight: torch.Tensor) -> bool:
-    return (0 < m <= MOST_ROWS and k > 0 and k % 8 == 0 and weight.dtype == torch.bfloat16 and weight.dim() == 2 and weight.shape[1] == k
-            and weight.is_cuda and _aligned(weight) and ((weight.shape[0] - 1) * weight.stride(0) + k) * 2 < _REACH)
+    if not (0 < m <= MOST_ROWS and k > 0 and k % 8 == 0 and weight.dtype == torch.bfloat16 and weight.dim() == 2 and weight.is_cuda):
+        return False
+    (n, width), (ld, apart) = weight.shape, weight.stride()
+    return width == k and apart == 1 and ld % 8 == 0 and ld >= k and ((n - 1) * ld + k) * 2 < _REACH and weight.data_ptr() % 16 == 0
 
 
 def _blocks(n: int, cus: int) -> int:
@@ -55,27 +52,34 @@ def takes_gated(m: int, k: int, weight: torch.Tensor) -> bool:
     return -(-(-(-(n // 2) // blocks)) // 8) <= MOST_GATED_TILES
 
 
-def _check_x(x: torch.Tensor, weight: torch.Tensor, taken: bool) -> None:
-    _need(taken and x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and _aligned(x)
-          and ((x.shape[0] - 1) * x.stride(0) + x.shape[1]) * 2 < _REACH, "the kernel does not take this product")
+def _check_x(x: torch.Tensor, taken: bool):
+    """``(m, k, rows' distance)`` of an operand that a kernel takes."""
+    (m, k), (ld, apart) = x.shape, x.stride()
+    _need(taken and x.is_cuda and x.dtype == torch.bfloat16 and apart == 1 and ld % 8 == 0 and ld >= k and ((m - 1) * ld + k) * 2 < _REACH
+          and x.data_ptr() % 16 == 0, "the kernel does not take this product")
+    return m, k, ld
 
 
-def stream_into(residual: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, gain: Optional[torch.Tensor] = None):
-    """``residual += x @ weight.T`` (float32, in place).  With ``gain`` (float32 ``[N]``): returns ``(rows, squares, parts)``, the new
+_INTO_ARGS = [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ll] + [_c_ptr] * 3 + [_c_int] * 4 + [_c_ptr]
+_GATED_ARGS = [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_int, _c_float] + [_c_int] * 5 + [_c_ptr]
+
+
+def stream_into(residual: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, gain: Optional[torch.Tensor] = None, taken: bool = False):
+    """``residual += x @ weight.T`` (float32, in place).  ``taken``: :func:`takes_into` has just said so.  With ``gain`` (float32 ``[N]``): returns ``(rows, squares, parts)``, the new
     residual times the gain in bfloat16 and float32 ``[M, PARTS]`` whose first ``parts`` numbers of a row add up to the residual row's sum of squares."""
-    m, n = x.shape[0], weight.shape[0]
-    _check_x(x, weight, takes_into(m, x.shape[1], weight))
-    _need(residual.is_cuda and residual.dtype == torch.float32 and residual.shape == (m, n) and residual.stride(1) == 1
-          and residual.stride(0) >= n, "the residual must be float32 [M, N] on the GPU")
+    m, k, ldx = _check_x(x, taken or takes_into(x.shape[0], x.shape[1], weight))
+    n, (ldh, apart) = weight.shape[0], residual.stride()
+    _need(residual.is_cuda and residual.dtype == torch.float32 and residual.shape == (m, n) and apart == 1 and ldh >= n,
+          "the residual must be float32 [M, N] on the GPU")
     rows = squares = None
     cus = compute_units(x.device)
     if gain is not None:
         _need(gain.is_cuda and gain.dtype == torch.float32 and gain.shape == (n,) and gain.is_contiguous(), "gain must be float32 [N] on the GPU")
         rows = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
         squares = torch.empty((m, PARTS), dtype=torch.float32, device=x.device)
-    fn = _fn("gemm_stream", "qvl_gemm_stream_into", [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ll] + [_c_ptr] * 3 + [_c_int] * 4 + [_c_ptr])
-    _check(fn(x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), residual.data_ptr(), residual.stride(0), _ptr(gain), _ptr(rows),
-              _ptr(squares), m, n, x.shape[1], cus, _stream()), "linear (stream, into the residual)")
+    fn = _fn("gemm_stream", "qvl_gemm_stream_into", _INTO_ARGS)
+    _check(fn(x.data_ptr(), ldx, weight.data_ptr(), weight.stride(0), residual.data_ptr(), ldh, _ptr(gain), _ptr(rows),
+              _ptr(squares), m, n, k, cus, _stream()), "linear (stream, into the residual)")
     return None if gain is None else (rows, squares, _blocks(n, cus))
 
 
@@ -83,13 +87,12 @@ def stream_gated(x: torch.Tensor, weight: torch.Tensor, act: str = "silu", scale
     """``act(gate) * up`` for a weight whose rows come in groups of 8 gate and 8 up rows: bfloat16 ``[M, N / 2]``.  ``scaled``: ``(squares, parts,
     eps)`` of rows that :func:`stream_into` left."""
     _need(act in ("silu", "gelu_tanh"), "the activation is silu or gelu_tanh")
-    m, n = x.shape[0], weight.shape[0]
-    _check_x(x, weight, takes_gated(m, x.shape[1], weight))
+    m, k, ldx = _check_x(x, takes_gated(x.shape[0], x.shape[1], weight))
+    n = weight.shape[0]
     out = torch.empty((m, n // 2), dtype=torch.bfloat16, device=x.device)
     squares, parts, eps = scaled if scaled is not None else (None, 0, 0.0)
     _need(squares is None or (squares.is_cuda and squares.dtype == torch.float32 and squares.shape == (m, PARTS) and squares.is_contiguous()),
           "squares must be float32 [M, PARTS] on the GPU")
-    fn = _fn("gemm_stream", "qvl_gemm_stream_gated", [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_int, _c_float] + [_c_int] * 5 + [_c_ptr])
-    _check(fn(x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), out.data_ptr(), out.stride(0), _ptr(squares), parts, eps, m, n,
-              x.shape[1], int(act == "gelu_tanh"), compute_units(x.device), _stream()), "linear (stream, gated)")
+    fn = _fn("gemm_stream", "qvl_gemm_stream_gated", _GATED_ARGS)
+    _check(fn(x.data_ptr(), ldx, weight.data_ptr(), weight.stride(0), out.data_ptr(), n // 2, _ptr(squares), parts, eps, m, n, k, int(act == "gelu_tanh"), compute_units(x.device), _stream()), "linear (stream, gated)")
     return out
