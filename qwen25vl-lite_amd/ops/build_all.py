@@ -23,6 +23,7 @@ LIBRARIES = [
     ("gemm_rows", {}),
     ("gemm_slice", {}),
     ("gemm_stream", {}),
+    ("gemm_mid", {}),
     ("peaks", {}),
     ("gated", {}),
     ("moe", {}),

@@ -17,7 +17,7 @@ from typing import Optional, Union
 
 import torch
 
-from . import kernels, rows, skinny, stream, tile
+from . import kernels, mid, rows, skinny, stream, tile
 
 __all__ = ["NormedRows", "ScaledRows", "NormAhead", "linear", "linear_into", "linear_stack", "linear_relu2", "gate_up_swiglu", "tune_library_products"]
 
@@ -169,6 +169,10 @@ def linear_into(residual: Optional[torch.Tensor], x: torch.Tensor, weight: torch
     if (fast and m <= skinny.ONE_BLOCK_ROWS and residual is not None and skinny.takes_resident(m, k, weight)
             and residual.dtype == torch.float32 and residual.shape == (m, weight.shape[0]) and residual.stride(1) == 1):
         skinny.resident_product(weight, x=x, epilogue=skinny.RESIDUAL, out=residual)
+        return None
+    if (fast and in_place and residual is not None and residual.dtype == torch.float32 and mid.prefers_into(m, k, weight) and residual.stride(1) == 1
+            and residual.shape == (m, weight.shape[0]) and residual.stride(0) >= residual.shape[1] and mid.takes_mid(x, weight)):
+        mid.mid_into(residual, x, weight)
         return None
     if fast:
         slabs = tile.tile_slabs(x, weight)

@@ -116,6 +116,21 @@ def prefers_heads(x: torch.Tensor, weight: torch.Tensor, ranges: int, head_dim: 
             and all(t is None or t.data_ptr() % 16 == 0 for t in rest))
 
 
+def check_heads(m: int, n: int, nkv: int, page_size: int, bias, cs, slots, k_cache, v_cache) -> None:
+    """Refuses what a projection with rotation and cache write of heads of 128 channels reads and writes beside its operands, where it does not fit."""
+    _need(bias is None or (bias.dtype == torch.float32 and bias.shape == (n,) and bias.is_contiguous() and bias.is_cuda),
+          "bias must be float32 [(nq + 2 nkv) 128]")
+    _need(cs.is_cuda and cs.dtype == torch.float32 and cs.dim() == 3 and cs.shape[0] >= m and cs.shape[1:] == (64, 2)
+          and cs.is_contiguous(), "cs must be float32 [M, 64, 2]")
+    if nkv:
+        _need(slots is not None and slots.is_cuda and slots.dtype == torch.int32 and slots.shape == (m,) and slots.is_contiguous(),
+              "slots must be int32 [M]")
+        _need(k_cache is not None and v_cache is not None and k_cache.is_cuda and v_cache.is_cuda
+              and k_cache.dtype == v_cache.dtype == torch.bfloat16 and k_cache.is_contiguous() and v_cache.is_contiguous()
+              and k_cache.shape[1:] == (nkv, page_size, 128) and v_cache.shape[1:] == (nkv, 128, page_size)
+              and v_cache.shape[0] == k_cache.shape[0], "caches must be bfloat16 [pages, nkv, ps, 128] / [pages, nkv, 128, ps]")
+
+
 def tile_heads(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor], cs: torch.Tensor, slots: Optional[torch.Tensor],
                k_cache: Optional[torch.Tensor], v_cache: Optional[torch.Tensor], num_q_heads: int, num_kv_heads: int, page_size: int,
                shape: int = -1) -> torch.Tensor:
@@ -126,17 +141,7 @@ def tile_heads(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tenso
     nq, nkv = int(num_q_heads), int(num_kv_heads)
     n = (nq + 2 * nkv) * 128
     _need(takes_tile(x, weight) and weight.shape[0] == n, "the tiled kernel does not take this projection")
-    _need(bias is None or (bias.dtype == torch.float32 and bias.shape == (n,) and bias.is_contiguous() and bias.is_cuda),
-          "bias must be float32 [(nq + 2 nkv) 128]")
-    _need(cs.is_cuda and cs.dtype == torch.float32 and cs.dim() == 3 and cs.shape[0] >= m and tuple(cs.shape[1:]) == (64, 2)
-          and cs.is_contiguous(), "cs must be float32 [M, 64, 2]")
-    if nkv:
-        _need(slots is not None and slots.is_cuda and slots.dtype == torch.int32 and slots.shape == (m,) and slots.is_contiguous(),
-              "slots must be int32 [M]")
-        _need(k_cache is not None and v_cache is not None and k_cache.is_cuda and v_cache.is_cuda
-              and k_cache.dtype == v_cache.dtype == torch.bfloat16 and k_cache.is_contiguous() and v_cache.is_contiguous()
-              and tuple(k_cache.shape[1:]) == (nkv, page_size, 128) and tuple(v_cache.shape[1:]) == (nkv, 128, page_size)
-              and v_cache.shape[0] == k_cache.shape[0], "caches must be bfloat16 [pages, nkv, ps, 128] / [pages, nkv, 128, ps]")
+    check_heads(m, n, nkv, page_size, bias, cs, slots, k_cache, v_cache)
     q_out = torch.empty((m, nq * 128), dtype=torch.bfloat16, device=x.device)
     _check(_heads(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), _ptr(cs), _ptr(slots if nkv else None), _ptr(q_out),
               _ptr(k_cache if nkv else None), _ptr(v_cache if nkv else None), m, k, nq, nkv, int(page_size), shape,

@@ -12,7 +12,7 @@ from typing import Dict, Optional
 
 import torch
 
-from ..ops import kernels, skinny, stream, tile
+from ..ops import kernels, mid, skinny, stream, tile
 from ..ops.attention import paged_attention
 from ..ops.linear import NormedRows, ScaledRows, linear, linear_into
 from .base import (CacheNeed, LayerSlot, Mixer, ParamSpec, PartSpec, StateNeed, StepContext, build_part, rotation_key,
@@ -290,7 +290,7 @@ class PagedAttention(Mixer):
     def _output(self, o: torch.Tensor, step: StepContext):
         """The output projection: into the residual where the block offers it and there is no bias."""
         if self.b_out is None:
-            return linear_into(step.residual, o, self.w_out, getattr(step, "ahead", None))
+            return linear_into(step.residual, o, self.w_out, getattr(step, "ahead", None), in_place=True)
         return linear(o, self.w_out, self.b_out,
                       out_dtype=torch.float32 if o.shape[0] <= skinny.ONE_BLOCK_ROWS else None)
 
@@ -334,6 +334,11 @@ class PagedAttention(Mixer):
         m, k = x.shape
         nkv = self.nkv if write else 0
         many = self.dtype == torch.bfloat16 and isinstance(x, torch.Tensor)
+        if many and m > tile.MANY_ROWS and self.w_in.shape[0] == (self.nq + 2 * nkv) * self.hd and mid.prefers_heads(
+                x, self.w_in, self.hd, inv_freq.shape[0], self.b_in, slot.k_cache if write else None, slot.v_cache if write else None):
+            return mid.mid_heads(x, self.w_in, self.b_in, self._rotation_table(step, inv_freq, freq_row, m),
+                                 group.slot_mapping if write else None, slot.k_cache if write else None,
+                                 slot.v_cache if write else None, self.nq, nkv, group.page_size)
         ranges = tile.slab_ranges(x, self.w_in) if many else 0
         if many and self.w_in.shape[0] == (self.nq + 2 * nkv) * self.hd and tile.prefers_heads(
                 x, self.w_in, ranges, self.hd, inv_freq.shape[0], self.b_in, slot.k_cache if write else None,
