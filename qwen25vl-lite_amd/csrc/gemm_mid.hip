@@ -12,6 +12,10 @@
 // 16 + 2 x 2 heads of 2,048, 280 rows 13.5 (20.8), 420 16.7 (22.9).  Three, four or five steps on their way, and blocks that begin at one or at
 // different places of K, the same within 2 per cent; steps of 64 columns 12.5 us for 11.2 (2,048 x 2,048, 420 rows).  Error of the sums against 64
 // bits 0.86e-7 of the result (tiles in slabs 1.2 to 1.5e-7).  420 prompt tokens, 8 layers of 3B sizes: 1,245 us to 1,109.
+//
+// Where a norm waits behind the sum, whose reader takes rows that are not yet divided by their root mean square, the blocks leave the new rows times the
+// norm's gain and their sums of squares (1.2 us), and the norm's kernel (4.0 us, and a launch of a host that is hardly ahead) falls away: the pass above
+// 2 per cent, one that mixes prompts and decoding 0.6.
 #include "tile_product.h"
 
 #include <type_traits>
@@ -19,6 +23,7 @@
 #define MID_WAVES 8
 #define MID_N 64
 #define MID_LDS 163840
+#define MID_PARTS 256                            // places of a row's sums of squares
 
 enum { MID_INTO = 0, MID_HEADS = 1 };
 
@@ -31,6 +36,9 @@ struct MidArgs {
   float* h;              // MID_INTO: [M, N] += product, rows ldh apart
   long long ldh;
   int wide;              // four results may be read and written at once
+  const float* gain;     // [N], of the norm behind the sum, or null: then nothing is left for it
+  bf16_t* left;          // [M, N]: the new h times gain
+  float* left_squares;   // [M, MID_PARTS]: of a row of the new h the sum of squares of every block's outputs
   // MID_HEADS: W's rows are nq query, nkv key and nkv value heads of 128 channels
   const float* bias;     // [N] or null
   const float2* cs;      // [M, 64]: cosine and sine
@@ -150,6 +158,19 @@ __global__ __launch_bounds__(64 * MID_WAVES) void gemm_mid_kernel(MidArgs p) {
     step(s, even, odd);
     if (s < steps) step(s + 1, odd, even);
   }
+  // MID_INTO: what the sums are added to, and the gain, are on their way while the quarters meet
+  constexpr int ENDS = (16 * 16 * MT + 64 * MID_WAVES - 1) / (64 * MID_WAVES);
+  const int mine = MID_N * block + 4 * (threadIdx.x & 15);      // the first of this lane's four outputs
+  const bool four = OUT == MID_INTO && p.wide && mine + 3 < p.N;
+  tp_f32x4 h4[ENDS], g4 = {0.f, 0.f, 0.f, 0.f};
+  if (four) {
+    if (p.gain) g4 = *reinterpret_cast<const tp_f32x4*>(p.gain + mine);
+#pragma unroll
+    for (int t = 0; t < ENDS; ++t) {
+      const int m = m0 + ((threadIdx.x + 64 * MID_WAVES * t) >> 4);
+      h4[t] = *reinterpret_cast<const tp_f32x4*>(p.h + min(m, p.M - 1) * p.ldh + mine);
+    }
+  }
   tp_wait_fetches<0>();
   tp_wait_lds();
   __syncthreads();                            // the stages have been read: their place is the quarters'
@@ -170,17 +191,36 @@ __global__ __launch_bounds__(64 * MID_WAVES) void gemm_mid_kernel(MidArgs p) {
     return v;
   };
   if constexpr (OUT == MID_INTO) {
-    for (int e = threadIdx.x; e < 16 * 16 * MT; e += 64 * MID_WAVES) {
-      const int i = e & 15, m = e >> 4, n = MID_N * block + 4 * i;
-      if (m0 + m >= p.M || n >= p.N) continue;
+#pragma unroll
+    for (int t = 0; t < ENDS; ++t) {
+      const int e = threadIdx.x + 64 * MID_WAVES * t, i = e & 15, m = e >> 4, n = mine;      // (a row's sixteen lanes stay together)
+      if (m >= 16 * MT || m0 + m >= p.M) break;
       float* h = p.h + (m0 + m) * p.ldh + n;
-      const tp_f32x4 v = total(i, m);
-      if (p.wide && n + 3 < p.N) {
-        *reinterpret_cast<tp_f32x4*>(h) += v;
+      bf16_t* left = p.left + (size_t)(m0 + m) * p.N + n;
+      tp_f32x4 v = total(i, m);
+      if (four) {
+        v += h4[t];
+        *reinterpret_cast<tp_f32x4*>(h) = v;
+        if (p.gain) {                 // (N is a multiple of 4 there, gain and left lie on 16-byte boundaries)
+          const uint32_t a = f32_to_bf16(v[0] * g4[0]), b = f32_to_bf16(v[1] * g4[1]), c = f32_to_bf16(v[2] * g4[2]), d = f32_to_bf16(v[3] * g4[3]);
+          *reinterpret_cast<uint2*>(left) = uint2{a | b << 16, c | d << 16};
+        }
       } else {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (n + j < p.N) h[j] += v[j];
+        for (int j = 0; j < 4; ++j) {
+          if (n + j < p.N) {
+            h[j] = v[j] = h[j] + v[j];
+            if (p.gain) left[j] = f32_to_bf16(v[j] * p.gain[n + j]);
+          } else {
+            v[j] = 0.f;
+          }
+        }
+      }
+      if (p.gain) {
+        float square = (v[0] * v[0] + v[1] * v[1]) + (v[2] * v[2] + v[3] * v[3]);
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) square += __shfl_xor(square, o, QVL_WAVE);
+        if (i == 0) p.left_squares[(size_t)(m0 + m) * MID_PARTS + block] = square;
       }
     }
   } else {
@@ -251,14 +291,16 @@ static int mid_launch(MidArgs& p, int cus, hipStream_t stream) {
 }
 
 // h (float32 [M, N], rows ldh apart) += x . w^T; x: bfloat16 [M, K], rows ldx apart; w: bfloat16 [N, K], rows ldw apart; both on 16-byte boundaries, K a
-// multiple of 8.
-extern "C" int qvl_gemm_mid_into(const void* x, long long ldx, const void* w, long long ldw, void* h, long long ldh, int M, int N, int K, int cus,
-                                 hipStream_t stream) {
+// multiple of 8.  gain (float32 [N], or null), for the norm behind the sum: left (bfloat16 [M, N]) = the new h times gain, left_squares (float32 [M, 256]): the
+// sums of squares of 64 values each of a row of the new h, one after the other.
+extern "C" int qvl_gemm_mid_into(const void* x, long long ldx, const void* w, long long ldw, void* h, long long ldh, const void* gain, void* left,
+                                 void* left_squares, int M, int N, int K, int cus, hipStream_t stream) {
   if (M <= 0 || N <= 0) return QVL_OK;
-  if (!h || ldh < N) return QVL_ERR_SHAPE;
+  if (!h || ldh < N || (gain && (!left || !left_squares || N > MID_N * MID_PARTS))) return QVL_ERR_SHAPE;
   MidArgs p{};
   p.x = (const bf16_t*)x; p.ldx = ldx; p.w = (const bf16_t*)w; p.ldw = ldw; p.M = M; p.N = N; p.K = K;
-  p.h = (float*)h; p.ldh = ldh; p.wide = ldh % 4 == 0 && (uintptr_t)h % 16 == 0;
+  p.gain = (const float*)gain; p.left = (bf16_t*)left; p.left_squares = (float*)left_squares;
+  p.h = (float*)h; p.ldh = ldh; p.wide = ldh % 4 == 0 && (uintptr_t)h % 16 == 0 && (!gain || (N % 4 == 0 && ((uintptr_t)gain | (uintptr_t)left) % 16 == 0));
   return mid_launch<MID_INTO>(p, cus, stream);
 }
 

@@ -14,7 +14,7 @@
 
 #include <cmath>
 
-enum { OUT_BF16 = 0, OUT_F32 = 1, OUT_GROUPED = 2, OUT_HALVES = 3, OUT_HEADS = 4 };
+enum { OUT_BF16 = 0, OUT_F32 = 1, OUT_GROUPED = 2, OUT_HALVES = 3, OUT_HEADS = 4, OUT_SCALED = 5 };     // (scaled: grouped, of such rows)
 
 struct TileArgs {
   const bf16_t* x;
@@ -28,6 +28,11 @@ struct TileArgs {
   int tiles_m, tiles_n, splits;
   int relu2, gelu;
   float alpha, limit, shift;
+  // OUT_SCALED: X's rows are rows of a sum times a norm's gain, not yet divided by their root mean square: row m's squares add up to the first `parts`
+  // numbers from squares[TILE_PARTS m] on
+  const float* squares;
+  int parts;
+  float eps;
   // OUT_HEADS: W holds nq query, nkv key and nkv value heads of HEAD rows; out takes the rotated queries [M, nq, HEAD]
   const float* bias;     // [N] or null
   const float4* cs;      // [M, HEAD / 2]: cosine and sine, two frequencies a value
@@ -37,6 +42,7 @@ struct TileArgs {
   int nq, nkv, ps;
 };
 #define HEAD 128
+#define TILE_PARTS 256     // places of a row's sums of squares
 
 __device__ __forceinline__ uint32_t two_bf16(float a, float b) {
   typedef __bf16 pair_t __attribute__((ext_vector_type(2)));
@@ -133,6 +139,45 @@ __device__ __forceinline__ void store_heads(const T& t, const TileArgs& p, int n
   }
 }
 
+// One over the root mean square of each row of X that this lane has results of.  A row's four lanes (g) take four of its numbers at a time; those of
+// the first 32 are asked for in front of the first fetches of W and X and added up behind them, on their way (22,016 x 2,048, 420 rows 47.2 us, waited for
+// in front of them 49.6, of rows that need no scale 44.8; the norm's kernel that falls away takes 4.0 and 10 us of the host).
+template <typename T>
+struct RowScales {
+  float4 first[T::MT][2];
+  float scale[T::MT];
+
+  __device__ __forceinline__ const float* at(const T& t, const TileArgs& p, int m0, int m) const {
+    const int gm = m0 + (t.wm * T::MT + m) * 16 + t.r;
+    return p.squares + (size_t)(gm < p.M ? gm : 0) * TILE_PARTS;
+  }
+  __device__ __forceinline__ void ask(const T& t, const TileArgs& p, int m0) {
+#pragma unroll
+    for (int m = 0; m < T::MT; ++m)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) first[m][i] = *reinterpret_cast<const float4*>(at(t, p, m0, m) + 16 * i + 4 * t.g);
+  }
+  __device__ static __forceinline__ float some(const float4& v, int have) {      // the first `have`: those behind the last part hold anything
+    return ((have > 0 ? v.x : 0.f) + (have > 1 ? v.y : 0.f)) + ((have > 2 ? v.z : 0.f) + (have > 3 ? v.w : 0.f));
+  }
+  __device__ __forceinline__ void finish(const T& t, const TileArgs& p, int m0) {
+    const int have = p.parts - 4 * t.g;
+#pragma unroll
+    for (int m = 0; m < T::MT; ++m) scale[m] = some(first[m][0], have) + some(first[m][1], have - 16);
+    for (int k = 32; k < p.parts; k += 16) {
+#pragma unroll
+      for (int m = 0; m < T::MT; ++m) scale[m] += some(*reinterpret_cast<const float4*>(at(t, p, m0, m) + min(k + 4 * t.g, TILE_PARTS - 4)), have - k);
+    }
+#pragma unroll
+    for (int m = 0; m < T::MT; ++m) {
+      float s = scale[m];
+      s += __shfl_xor(s, 16, QVL_WAVE);
+      s += __shfl_xor(s, 32, QVL_WAVE);
+      scale[m] = 1.0f / sqrtf(s / (float)p.K + p.eps);
+    }
+  }
+};
+
 template <typename T, int OUT>
 __global__ __launch_bounds__(512) void gemm_tile_kernel(TileArgs p) {
   __shared__ __attribute__((aligned(16))) char lds[T::LDS];
@@ -152,6 +197,8 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(TileArgs p) {
   const int s0 = (int)((long long)steps_all * split / p.splits), s1 = (int)((long long)steps_all * (split + 1) / p.splits);
   const bf16_t* w = p.w + (size_t)n0 * p.ldw + (size_t)s0 * 64;
   const bf16_t* x = p.x + (size_t)m0 * p.ldx + (size_t)s0 * 64;
+  RowScales<T> rows;
+  if (OUT == OUT_SCALED) rows.ask(t, p, m0);
   // rows that do not exist are read from one that does; their sums are not stored
   t.set_rows(
       [&](int h, int rho) {
@@ -166,7 +213,9 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(TileArgs p) {
         const int m = T::x_row(h, rho);
         return (uint32_t)((size_t)(m0 + m < p.M ? m : 0) * p.ldx * 2);
       });
-  t.multiply(lds, w, x, s1 - s0, p.K % 64 != 0 && s1 == steps_all);
+  t.multiply(lds, w, x, s1 - s0, p.K % 64 != 0 && s1 == steps_all, [&]() __attribute__((always_inline)) {
+    if (OUT == OUT_SCALED) rows.finish(t, p, m0);
+  });
   // a lane holds, of tile (n, m): X's row 16 m + r, W's rows 16 n + 4 g ... + 3
   if constexpr (OUT == OUT_HEADS) {
     store_heads(t, p, n0, m0);
@@ -217,7 +266,8 @@ __global__ __launch_bounds__(512) void gemm_tile_kernel(TileArgs p) {
         for (int i = 0; i < 4; ++i) {
           const float one = t.acc[n][m][i], next = t.acc[n + 1][m][i];
           const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(one), __float_as_uint(next), false, false);
-          v[i] = gate_act(__uint_as_float((uint32_t)both[0]), p.gelu) * __uint_as_float((uint32_t)both[1]);
+          const float scale = OUT == OUT_SCALED ? rows.scale[m] : 1.f;
+          v[i] = gate_act(__uint_as_float((uint32_t)both[0]) * scale, p.gelu) * (__uint_as_float((uint32_t)both[1]) * scale);
         }
         const int first = n0 + (t.wn * T::NT + n + (t.g >> 1)) * 16;      // the lane's tile's first row of W
         if (gm < p.M && first < p.N)
@@ -318,9 +368,9 @@ extern "C" int qvl_gemm_tile_blocks(int M, int N, int K, int cus) {
 // 2: N in groups of 8 gate + 8 up rows, out bfloat16 [M, N / 2] = act(gate) up (gelu: gelu's tanh form, else silu);
 // 3: N / 2 gate rows, then the up rows: out = g sigmoid(alpha g) (u + shift), g capped at limit, u clamped to +-limit.
 // tile: -1, or the shape to take (0 .. 9).
-extern "C" int qvl_gemm_tile(const void* x, long long ldx, const void* w, long long ldw, void* out, long long ldo, int M, int N,
-                             int K, int mode, int splits, int relu2, int gelu, float alpha, float limit, float shift, int tile,
-                             int cus, hipStream_t stream) {
+static int tile_launch(const void* x, long long ldx, const void* w, long long ldw, void* out, long long ldo, int M, int N,
+                       int K, int mode, int splits, int relu2, int gelu, float alpha, float limit, float shift, int tile,
+                       int cus, const void* squares, int parts, float eps, hipStream_t stream) {
   if (M <= 0 || N <= 0) return QVL_OK;
   if (K <= 0 || K % 32 || ldx < K || ldw < K || ldx % 8 || ldw % 8 || !x || !w || !out || cus <= 0 || splits < 1 ||
       ((uintptr_t)x % 16) || ((uintptr_t)w % 16) || ((uintptr_t)out % 16) || splits > (K + 63) / 64 || (mode != 1 && splits != 1))
@@ -334,6 +384,7 @@ extern "C" int qvl_gemm_tile(const void* x, long long ldx, const void* w, long l
   p.x = (const bf16_t*)x; p.ldx = ldx; p.w = (const bf16_t*)w; p.ldw = ldw; p.out = out; p.ldo = ldo;
   p.M = M; p.N = N; p.K = K; p.rows = mode == 3 ? N / 2 : N; p.splits = splits; p.relu2 = relu2; p.gelu = gelu;
   p.alpha = alpha; p.limit = limit; p.shift = shift;
+  p.squares = (const float*)squares; p.parts = parts; p.eps = eps;
   int shape = tile >= 0 ? tile : shape_for(M, N, K, splits, cus);
   if ((unsigned long long)SHAPES[shape].bm * ldx * 2 >= 0xffff0000ull) shape = 0;
   const TileShape& s = SHAPES[shape];
@@ -359,11 +410,24 @@ extern "C" int qvl_gemm_tile(const void* x, long long ldx, const void* w, long l
   } while (0)
   if (mode == 0) SHAPE(OUT_BF16);
   else if (mode == 1) SHAPE(OUT_F32);
+  else if (mode == 2 && squares) SHAPE(OUT_SCALED);
   else if (mode == 2) SHAPE(OUT_GROUPED);
   else SHAPE(OUT_HALVES);
 #undef SHAPE
 #undef GO
   return qvl_launch_status();
+}
+extern "C" int qvl_gemm_tile(const void* x, long long ldx, const void* w, long long ldw, void* out, long long ldo, int M, int N,
+                             int K, int mode, int splits, int relu2, int gelu, float alpha, float limit, float shift, int tile,
+                             int cus, hipStream_t stream) {
+  return tile_launch(x, ldx, w, ldw, out, ldo, M, N, K, mode, splits, relu2, gelu, alpha, limit, shift, tile, cus, nullptr, 0, 0.f, stream);
+}
+// Mode 2 for rows x of a sum times a norm's gain that are still to be divided by their root mean square: row m's squares add up to squares[256 m ...],
+// `parts` numbers (float32 [M, 256] on a 16-byte boundary).
+extern "C" int qvl_gemm_tile_scaled(const void* x, long long ldx, const void* w, long long ldw, void* out, long long ldo, const void* squares, int parts,
+                                    float eps, int M, int N, int K, int gelu, int tile, int cus, hipStream_t stream) {
+  if (!squares || parts <= 0 || parts > TILE_PARTS || (uintptr_t)squares % 16) return QVL_ERR_SHAPE;
+  return tile_launch(x, ldx, w, ldw, out, ldo, M, N, K, 2, 1, 0, gelu, 1.f, 0.f, 0.f, tile, cus, squares, parts, eps, stream);
 }
 
 // Shapes whose waves hold both halves of a head (8 or 4 tiles of W's rows).
@@ -388,6 +452,7 @@ extern "C" int qvl_gemm_tile_heads(const void* x, long long ldx, const void* w, 
   TileArgs p;
   p.x = (const bf16_t*)x; p.ldx = ldx; p.w = (const bf16_t*)w; p.ldw = ldw; p.out = q_out; p.ldo = 0;
   p.M = M; p.N = N; p.K = K; p.rows = N; p.splits = 1; p.relu2 = p.gelu = 0; p.alpha = p.limit = p.shift = 0.f;
+  p.squares = nullptr; p.parts = 0; p.eps = 0.f;
   p.bias = (const float*)bias; p.cs = (const float4*)cs; p.slot = (const int*)slot; p.kc = (bf16_t*)kc; p.vc = (bf16_t*)vc;
   p.nq = nq; p.nkv = nkv; p.ps = ps;
   int shape = tile >= 0 ? tile : shape_for(M, N, K, 1, cus, HEAD_SHAPES);

@@ -134,8 +134,12 @@ struct Tile {
   }
 
   // acc = the tile's products over `steps` steps of 64 values from w and x on.  half_last: the last step has 32
-  // values only.
-  __device__ __forceinline__ void multiply(char* lds, const void* w, const void* x, int steps, bool half_last) {
+  // values only.  meanwhile(): what is done while the first values are on their way.
+  struct Nothing {
+    __device__ __forceinline__ void operator()() const {}
+  };
+  template <typename Meanwhile = Nothing>
+  __device__ __forceinline__ void multiply(char* lds, const void* w, const void* x, int steps, bool half_last, Meanwhile meanwhile = Meanwhile()) {
     constexpr std::integral_constant<int, 0> I{};
     constexpr std::integral_constant<int, 1> II{};
     w = tp_uniform(w);
@@ -237,6 +241,11 @@ struct Tile {
       tp_barrier();
     };
     issue_w(I, 0, 0); issue_x(I, 0, 0); issue_x(II, 0, 0); issue_w(II, 0, 0); issue_w(I, 1, BUF); issue_x(I, 1, BUF); issue_x(II, 1, BUF);
+    if constexpr (!std::is_same<Meanwhile, Nothing>::value) {
+      __builtin_amdgcn_sched_barrier(0);
+      meanwhile();
+      __builtin_amdgcn_sched_barrier(0);
+    }
     tp_wait_fetches<LX1 + LW1 + LW0 + LX0 + LX1>();     // the first halves of step 0
     tp_barrier();
     if (wave >= 4) tp_barrier();            // the second group, a phase behind

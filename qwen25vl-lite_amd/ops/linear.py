@@ -172,7 +172,9 @@ def linear_into(residual: Optional[torch.Tensor], x: torch.Tensor, weight: torch
         return None
     if (fast and in_place and residual is not None and residual.dtype == torch.float32 and mid.prefers_into(m, k, weight) and residual.stride(1) == 1
             and residual.shape == (m, weight.shape[0]) and residual.stride(0) >= residual.shape[1] and mid.takes_mid(x, weight)):
-        mid.mid_into(residual, x, weight)
+        left = mid.mid_into(residual, x, weight, ahead.weight if ahead is not None and mid.leaves(weight.shape[0]) else None)
+        if left is not None:
+            ahead.left = ScaledRows(residual, ahead.weight, ahead.eps, ahead.dtype, *left)
         return None
     if fast:
         slabs = tile.tile_slabs(x, weight)
@@ -206,6 +208,8 @@ def gate_up_swiglu(x: Union[torch.Tensor, NormedRows], weight: torch.Tensor, gro
     m, k = x.shape
     if grouped and isinstance(x, ScaledRows) and stream.takes_gated(m, k, weight):
         return stream.stream_gated(x.rows, weight, act, x.scaled)
+    if grouped and isinstance(x, ScaledRows) and tile.MANY_ROWS < m and tile.prefers_tile(x.rows, weight, gated=True):
+        return tile.tile_swiglu(x.rows, weight, act, taken=True, scaled=x.scaled)
     if (grouped and weight.dtype == torch.bfloat16 and weight.is_cuda and weight.shape[0] % 16 == 0
             and m <= skinny.ONE_BLOCK_ROWS and not rows.wide(m, weight)):
         lazy = isinstance(x, NormedRows)

@@ -11,11 +11,12 @@ import torch
 from . import tile
 from .kernels import _check, _fn, _need, _ptr, _stream, compute_units
 
-__all__ = ["takes_mid", "prefers_into", "mid_into", "prefers_heads", "mid_heads"]
+__all__ = ["takes_mid", "prefers_into", "leaves", "mid_into", "prefers_heads", "mid_heads"]
 
 _c_int, _c_ptr, _c_ll = ctypes.c_int, ctypes.c_void_p, ctypes.c_longlong
 _REACH = 0xffffff00
 _OUTPUTS = 64            # of a block (MID_N in the source)
+PARTS = 256              # places of a row's sums of squares (MID_PARTS)
 # Inner sizes up to here, and one block a compute unit at most.  A projection with rotation and cache write, for the product in slabs and the rotation's
 # kernel, at 65, 160, 320 and (16 + 2 x 2 heads) 400 rows: 8 + 2 x 2 heads, inner size 1,024 8.3, 8.3, 8.5 us for 11.9, 14.2, 16.6; 16 + 2 x 2, 2,048
 # 12.3, 12.8, 13.5, 15.7 for 14.3, 17.9, 21.9, 22.4; 28 + 2 x 4, 2,048 12.6, 13.3 for 15.7, 19.9; 3,072 16.3, 17.6 for 16.7, 21.8; but 3,584 20.3 (100
@@ -45,19 +46,32 @@ def prefers_into(m: int, k: int, weight: torch.Tensor) -> bool:
     return tile.MANY_ROWS < m and k <= LONGEST_INTO and 8 * m >= k and _one_round(m, weight.shape[0], compute_units(weight.device))
 
 
-def mid_into(residual: torch.Tensor, x: torch.Tensor, weight: torch.Tensor) -> None:
-    """``residual += x @ weight.T`` (float32, in place)."""
+def leaves(n: int) -> bool:
+    """Whether a row of ``n`` outputs has a place for every block's sum of squares."""
+    return n <= _OUTPUTS * PARTS
+
+
+def mid_into(residual: torch.Tensor, x: torch.Tensor, weight: torch.Tensor, gain: Optional[torch.Tensor] = None):
+    """``residual += x @ weight.T`` (float32, in place).  With ``gain`` (float32 ``[N]``): returns ``(rows, squares, parts)``, as
+    :func:`stream.stream_into`."""
     m, n = x.shape[0], weight.shape[0]
     _need(takes_mid(x, weight), "the kernel does not take this product")
     ldh, apart = residual.stride()
     _need(residual.is_cuda and residual.dtype == torch.float32 and residual.shape == (m, n) and apart == 1 and ldh >= n,
           "the residual must be float32 [M, N] on the GPU")
+    rows = squares = None
+    if gain is not None:
+        _need(gain.is_cuda and gain.dtype == torch.float32 and gain.shape == (n,) and gain.is_contiguous() and leaves(n),
+              "gain must be float32 [N] on the GPU")
+        rows = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+        squares = torch.empty((m, PARTS), dtype=torch.float32, device=x.device)
     fn = _fn("gemm_mid", "qvl_gemm_mid_into", _INTO_ARGS)
-    _check(fn(x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), residual.data_ptr(), ldh, m, n, x.shape[1], compute_units(x.device),
-              _stream()), "linear (small tiles, into the residual)")
+    _check(fn(x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), residual.data_ptr(), ldh, _ptr(gain), _ptr(rows), _ptr(squares), m, n,
+              x.shape[1], compute_units(x.device), _stream()), "linear (small tiles, into the residual)")
+    return None if gain is None else (rows, squares, -(-n // _OUTPUTS))
 
 
-_INTO_ARGS = [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ll] + [_c_int] * 4 + [_c_ptr]
+_INTO_ARGS = [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ll] + [_c_ptr] * 3 + [_c_int] * 4 + [_c_ptr]
 _HEADS_ARGS = [_c_ptr, _c_ll, _c_ptr, _c_ll] + [_c_ptr] * 6 + [_c_int] * 6 + [_c_ptr]
 
 

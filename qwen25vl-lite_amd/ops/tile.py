@@ -10,11 +10,12 @@ import torch
 
 from .kernels import _check, _fn, _need, _ptr, _stream, compute_units
 
-__all__ = ["MANY_ROWS", "takes_tile", "prefers_tile", "tile_product", "slab_ranges", "tile_slabs", "prefers_heads", "tile_heads", "tile_swiglu",
+__all__ = ["MANY_ROWS", "takes_tile", "prefers_tile", "enough_gated", "tile_product", "slab_ranges", "tile_slabs", "prefers_heads", "tile_heads", "tile_swiglu",
            "tile_gated"]
 
 _c_int, _c_ptr, _c_ll, _c_float = ctypes.c_int, ctypes.c_void_p, ctypes.c_longlong, ctypes.c_float
 _STORE, _SLABS, _GROUPED, _HALVES = range(4)
+PARTS = 256              # places of a row's sums of squares (TILE_PARTS in the source)
 _REACH = 0xffff0000      # bytes that a tile's rows may span from its first
 
 
@@ -32,6 +33,7 @@ def _entry(name: str, argtypes):
 _blocks_of = lru_cache(maxsize=4096)(_entry("qvl_gemm_tile_blocks", [_c_int] * 4))      # (numbers of the sizes alone)
 _splits_of = lru_cache(maxsize=4096)(_entry("qvl_gemm_tile_splits", [_c_int] * 4))
 _tile = _entry("qvl_gemm_tile", [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ll] + [_c_int] * 7 + [_c_float] * 3 + [_c_int, _c_int, _c_ptr])
+_scaled = _entry("qvl_gemm_tile_scaled", [_c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_ll, _c_ptr, _c_int, _c_float] + [_c_int] * 6 + [_c_ptr])
 _heads = _entry("qvl_gemm_tile_heads", [_c_ptr, _c_ll, _c_ptr, _c_ll] + [_c_ptr] * 6 + [_c_int] * 7 + [_c_ptr])
 
 
@@ -60,6 +62,15 @@ def prefers_tile(x: torch.Tensor, weight: torch.Tensor, halves: bool = False, ga
     cus = compute_units(x.device)
     blocks = _blocks_of(x.shape[0], weight.shape[0], x.shape[1], cus)
     return 2 * blocks >= cus if gated or halves else 4 * blocks >= 3 * cus
+
+
+def enough_gated(m: int, weight: torch.Tensor) -> bool:
+    """The sizes' part of ``prefers_tile(gated=True)`` for ``m`` rows that are yet to be made."""
+    n, k = weight.shape
+    if m <= MANY_ROWS or k % 32:
+        return False
+    cus = compute_units(weight.device)
+    return 2 * _blocks_of(m, n, k, cus) >= cus
 
 
 def _launch(x, weight, out, ldo, mode, splits=1, relu2=0, gelu=0, alpha=1.0, limit=0.0, shift=0.0, shape=-1):
@@ -149,14 +160,21 @@ def tile_heads(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tenso
     return q_out
 
 
-def tile_swiglu(x: torch.Tensor, weight: torch.Tensor, act: str = "silu", shape: int = -1, taken: bool = False) -> torch.Tensor:
+def tile_swiglu(x: torch.Tensor, weight: torch.Tensor, act: str = "silu", shape: int = -1, taken: bool = False, scaled=None) -> torch.Tensor:
     """``act(gate) * up`` for a weight whose rows come in groups of 8 gate and 8 up rows: bfloat16 ``[M, N / 2]``.  ``taken``: :func:`takes_tile`
-    has just said so."""
+    has just said so.  ``scaled``: ``(squares, parts, eps)`` of rows that a product into the sum left (:func:`mid.mid_into`)."""
     _need((taken or takes_tile(x, weight)) and weight.shape[0] % 16 == 0, "the tiled kernel does not take this product")
     _need(act in ("silu", "gelu_tanh"), "the activation is silu or gelu_tanh")
-    half = weight.shape[0] // 2
-    out = torch.empty((x.shape[0], half), dtype=torch.bfloat16, device=x.device)
-    return _launch(x, weight, out, half, _GROUPED, gelu=int(act == "gelu_tanh"), shape=shape)
+    m, half = x.shape[0], weight.shape[0] // 2
+    out = torch.empty((m, half), dtype=torch.bfloat16, device=x.device)
+    if scaled is None:
+        return _launch(x, weight, out, half, _GROUPED, gelu=int(act == "gelu_tanh"), shape=shape)
+    squares, parts, eps = scaled
+    _need(squares.is_cuda and squares.dtype == torch.float32 and squares.shape == (m, PARTS) and squares.is_contiguous(),
+          "squares must be float32 [M, PARTS] on the GPU")
+    _check(_scaled(x.data_ptr(), x.stride(0), weight.data_ptr(), weight.stride(0), out.data_ptr(), half, squares.data_ptr(), parts, eps, m,
+                   weight.shape[0], x.shape[1], int(act == "gelu_tanh"), shape, compute_units(x.device), _stream()), "linear (tiles, scaled rows)")
+    return out
 
 
 def tile_gated(x: torch.Tensor, weight: torch.Tensor, alpha: float, limit: Optional[float], shift: float,

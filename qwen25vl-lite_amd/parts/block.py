@@ -6,7 +6,6 @@ from typing import Dict, Optional
 
 import torch
 
-from ..ops.stream import MOST_ROWS
 from .base import Block, LayerSlot, Part, PartSpec, ResidualStream, StepContext, SumTerm, build_part, register_part
 
 __all__ = ["PreNormBlock", "ParallelBlock", "SandwichBlock", "PostNormBlock", "SumNormBlock"]
@@ -45,7 +44,7 @@ class PreNormBlock(Block):
         step.residual = stream.h            # the mixer may add its result in place and return None
         rows = stream.h.shape[0]
         ahead = None
-        if rows <= MOST_ROWS and self.mixer.leaves_ahead and self.ffn.takes_scaled(rows):
+        if self.mixer.leaves_ahead and self.ffn.takes_scaled(rows):
             ahead = step.ahead = self.norm2.ahead()
         stream.pending = self.mixer.forward(x, step, slot.of(self.names["mixer"]))
         if ahead is not None and ahead.left is not None:

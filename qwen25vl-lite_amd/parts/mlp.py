@@ -6,7 +6,7 @@ from typing import Dict, Optional
 
 import torch
 
-from ..ops import stream
+from ..ops import stream, tile
 from ..ops.linear import gate_up_swiglu, linear_into
 from .base import FeedForward, ParamSpec, StepContext, register_part
 
@@ -67,7 +67,8 @@ class SwiGLU(FeedForward):
                 f"{self.names['down']}.weight": self.w_down}
 
     def takes_scaled(self, rows: int) -> bool:
-        return self.grouped and self.dtype == torch.bfloat16 and stream.takes_gated(rows, self.hidden, self.w_gate_up)
+        return self.grouped and self.dtype == torch.bfloat16 and (stream.takes_gated(rows, self.hidden, self.w_gate_up)
+                                                                  or tile.enough_gated(rows, self.w_gate_up))
 
     def forward(self, x, step: StepContext):
         act = gate_up_swiglu(x, self.w_gate_up, self.grouped, self.activation)
