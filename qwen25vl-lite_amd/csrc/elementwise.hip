@@ -104,6 +104,31 @@ extern "C" int qvl_embed_gather(const void* ids, const void* table, void* out, i
 }
 
 // ---------------------------------------------------------------------------------------
+// A replayed step's integers (15 to 270 KB at batch 8 to 64) from pinned host memory, read where they lie.  The runtime's copy of more than 16 KB runs on
+// a copy engine, and the step's graph waits for its signal: 20 to 23 us from the last kernel in front of the copy to the first behind it, with this
+// kernel 10.  A pass of 16 steps at batch 8 of 7B sizes 15,530 us to 15,330, of 8 steps at batch 64 10,360 to 10,240; smaller transfers, which the runtime
+// makes with a kernel of its own, take as long as they did.  The loads go to the host's memory whatever the caches hold of it.
+// ---------------------------------------------------------------------------------------
+__global__ __launch_bounds__(256) void from_host_kernel(const unsigned long long* __restrict__ from, unsigned long long* __restrict__ to, int n) {
+  const int i = blockIdx.x * 512 + threadIdx.x, j = i + 256;
+  unsigned long long a = 0, b = 0;
+  if (i < n) a = __hip_atomic_load(from + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (j < n) b = __hip_atomic_load(from + j, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  if (i < n) to[i] = a;
+  if (j < n) to[j] = b;
+}
+
+// from: pinned host memory, to: device memory, `pairs` pairs of 4-byte words, both on 8-byte boundaries.
+extern "C" int qvl_from_host(const void* from, void* to, long long pairs, hipStream_t stream) {
+  if (pairs <= 0) return QVL_OK;
+  if (!from || !to || (((uintptr_t)from | (uintptr_t)to) & 7)) return QVL_ERR_SHAPE;
+  if (pairs > 0x7ffffc00ll) return QVL_ERR_LIMIT;
+  hipLaunchKernelGGL(from_host_kernel, dim3((unsigned)((pairs + 511) / 512)), dim3(256), 0, stream, (const unsigned long long*)from,
+                     (unsigned long long*)to, (int)pairs);
+  return qvl_launch_status();
+}
+
+// ---------------------------------------------------------------------------------------
 // Residual add + RMSNorm  (reference layers.py:27-31, text.py:196-205)
 //   v = h[row] + delta[row]            (delta optional; the sum is float32; delta may come as
 //                                       several slabs [slab][row], partial sums of a product cut

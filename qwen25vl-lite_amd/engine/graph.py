@@ -36,6 +36,7 @@ import numpy as np
 import torch
 
 from ..parts.base import GroupStep, StepContext
+from ..ops.kernels import int32_from_pinned
 from .batch import StepEntry
 
 __all__ = ["DecodeGraphs"]
@@ -103,6 +104,11 @@ class _Graph:
         self.graph = None
         self.logits = None
 
+    def __del__(self):
+        copied = getattr(self, "copied", None)
+        if copied is not None:
+            copied.synchronize()           # the pinned buffer goes back to its pool: nothing may still read it
+
     def h(self, name, shape=None):
         """The named array of the pinned host buffer."""
         o, n = self.offsets[name]
@@ -161,7 +167,7 @@ class _Graph:
     def run(self, entries: Sequence[StepEntry], device_tokens: Optional[torch.Tensor] = None) -> torch.Tensor:
         parts = self.parts
         self.fill(entries)
-        self.dev.copy_(self.host, non_blocking=True)
+        int32_from_pinned(self.host, self.dev)
         self.copied.record()
         if device_tokens is not None:
             # the entries' token ids are still on the device (sampled by the step before, whose ids

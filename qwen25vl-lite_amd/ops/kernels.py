@@ -106,6 +106,15 @@ def int32_to_device(host, device) -> torch.Tensor:
     return staged.to(device, non_blocking=True)
 
 
+def int32_from_pinned(host: torch.Tensor, out: torch.Tensor) -> None:
+    """``out`` (on the device) = ``host`` (pinned, int32, an even number) by a kernel that reads the host's memory: the caller keeps ``host`` as it is, and
+    alive, until an event recorded behind the call has come."""
+    _need(host.dtype == out.dtype == torch.int32 and host.is_contiguous() and out.is_contiguous() and host.numel() == out.numel()
+          and host.numel() % 2 == 0 and out.is_cuda and host.is_pinned(), "a pinned and a device int32 tensor of one even size")
+    fn = _fn("elementwise", "qvl_from_host", [_c_ptr, _c_ptr, ctypes.c_longlong, _c_ptr])
+    _check(fn(host.data_ptr(), out.data_ptr(), host.numel() // 2, _stream()), "int32_from_pinned")
+
+
 # --------------------------------------------------------------------------------------------
 EMBED_TABLES = 4     # as in csrc/elementwise.hip
 _EMBED_ARGS = [_c_ptr, _c_ptr, _c_ptr, _c_int, _c_int, _c_int, _c_int, _c_float, _c_ptr, _c_int, _c_int, _c_ptr, _c_ptr]
