@@ -781,12 +781,6 @@ static_assert(BLK_MAX_GROUPS == 1 || BLK_CT * MERGE_REGS * BLK_WAVES * 64 * 4 <=
               "the second group's sums do not fit its stages");
 
 // Device-scope ("agent") stores and loads: visible across the XCDs' L2 caches.
-__device__ __forceinline__ void store_device_scope(float* p, float v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float load_device_scope(const float* p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 __device__ __forceinline__ void store_device_scope(unsigned long long* p, float a, float b) {
   __hip_atomic_store(p, (unsigned long long)__float_as_uint(a) | (unsigned long long)__float_as_uint(b) << 32, __ATOMIC_RELAXED,
                      __HIP_MEMORY_SCOPE_AGENT);
@@ -1103,8 +1097,11 @@ __global__ __launch_bounds__(64 * BLK_WAVES * GROUPS, GROUPS == 1 ? BLK_PER_CU :
 // ---- few tiles (decode): the waves of a block share one tile ---------------------------------
 // The COOP_WAVES waves of a block take the tile's 32-key blocks in turn (wave w the blocks
 // w, w + COOP_WAVES, ...), then merge their sums and statistics through LDS in wave order.  With
-// nsplit > 1 the key range is further cut among blocks (grid.z); each block then writes its
-// merged partial to scratch.  The splits are merged by the block that finishes last (one counter
+// nsplit > 1 the keys that the tile sees are further cut among blocks (grid.z), evenly, but into splits of
+// keys_per_split at least: a captured step has blocks for the longest contexts of its bucket, and what a tile's blocks
+// share is what is there now.  Blocks that then have no keys end at once, and one that has all of them writes the result.  (28 + 2 x 4
+// heads, 8 tokens at 177 to 513 keys, captured for 1,024: cut as for the longest context, and merged float by float, 10.3 us, now 7.8; 64 + 2 x 8, 19 at 300 to
+// 1,025, captured for 2,048, 22.3 and 15.9; one token at 12,290, 25.3 and 17.6.)  Each block writes its merged partial to scratch.  The splits are merged by the block that finishes last (one counter
 // per (tile, kv head) tells a block whether it is that one), or, for callers without counters, by
 // a second kernel.
 // Blocks of one tile may run on different XCDs, whose L2 caches do not see each other's lines: the
@@ -1125,10 +1122,14 @@ __global__ __launch_bounds__(64 * BLK_WAVES * GROUPS, GROUPS == 1 ? BLK_PER_CU :
 // Merge the nsplit partial results of one (tile, kv head) and write the tile's rows of the output:
 // thread -> (column, 4 channels); splits are summed in order.  ACROSS: the partial results were
 // written by other blocks of the running kernel (device-scope loads); otherwise by a kernel before.
-template <bool ACROSS>
-__device__ __forceinline__ void merge_splits(const float* __restrict__ base, int nsplit, int r, int ct, int kvh, int g,
-                                             const int* __restrict__ cu_q, bf16_t* __restrict__ out, int nq,
-                                             const HeadEnd& end) {
+// AT_ONCE splits at a time: their values are asked for together (one trip to memory, not one per split, as pairs of floats), then
+// folded into the running sums against the running maximum, in split order.  As many as there are, up to eight, and by pairs: what is asked for in
+// vain, or float by float, is waited for too (sixteen at a time 26.8 us and eight 25.3 as single floats, eight 17.6 as pairs, sixteen 19.1: one token at 12,290
+// keys, 28 + 2 x 4 heads).
+template <bool ACROSS, int AT_ONCE>
+__device__ __forceinline__ void merge_splits_by(const float* __restrict__ base, int nsplit, int r, int ct, int kvh, int g,
+                                                const int* __restrict__ cu_q, bf16_t* __restrict__ out, int nq,
+                                                const HeadEnd& end) {
   const Run run = run_of(cu_q, r);
   const int q0 = run.q0, qlen = run.qlen;
   for (int idx = threadIdx.x; idx < 16 * (HD / 4); idx += blockDim.x) {
@@ -1136,36 +1137,34 @@ __device__ __forceinline__ void merge_splits(const float* __restrict__ base, int
     const int colg = ct * 16 + col;
     const int i = colg / g, gh = colg - i * g;
     if (i >= qlen) continue;
-    auto ld = [&](const float* p) { return ACROSS ? load_device_scope(p) : *p; };
-    // Eight splits at a time: their 48 values are asked for together (one trip to memory, not one
-    // per split), then folded into the running sums against the running maximum, in split order.
-    constexpr int AT_ONCE = 8;
+    auto ld = [&](const float* p) {
+      return ACROSS ? load_device_scope(reinterpret_cast<const unsigned long long*>(p)) : *reinterpret_cast<const float2*>(p);
+    };
     float m = -INFINITY, den = 0.f;
     float4 num = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = 0; s0 < nsplit; s0 += AT_ONCE) {
-      float pm[AT_ONCE], pl[AT_ONCE];
-      float4 pn[AT_ONCE];
+      float2 ml[AT_ONCE], pn[AT_ONCE][2];
 #pragma unroll
       for (int j = 0; j < AT_ONCE; ++j) {
         const int s = s0 + j < nsplit ? s0 + j : nsplit - 1;   // beyond the last: read it again, weight 0 below
         const float* p = base + (size_t)s * PART_STRIDE + col * PART_COLS;
-        pm[j] = ld(p + HD);
-        pl[j] = ld(p + HD + 1);
-        pn[j] = float4{ld(p + d), ld(p + d + 1), ld(p + d + 2), ld(p + d + 3)};
+        ml[j] = ld(p + HD);
+        pn[j][0] = ld(p + d);
+        pn[j][1] = ld(p + d + 2);
       }
       float m_new = m;
 #pragma unroll
       for (int j = 0; j < AT_ONCE; ++j)
-        if (s0 + j < nsplit) m_new = fmaxf(m_new, pm[j]);
+        if (s0 + j < nsplit) m_new = fmaxf(m_new, ml[j].x);
       const float keep = (m == -INFINITY) ? 0.f : exp2f(m - m_new);
       num.x *= keep; num.y *= keep; num.z *= keep; num.w *= keep;
       den *= keep;
       m = m_new;
 #pragma unroll
       for (int j = 0; j < AT_ONCE; ++j) {
-        const float wgt = (s0 + j < nsplit && pm[j] != -INFINITY) ? exp2f(pm[j] - m) : 0.f;
-        num.x += wgt * pn[j].x; num.y += wgt * pn[j].y; num.z += wgt * pn[j].z; num.w += wgt * pn[j].w;
-        den += wgt * pl[j];
+        const float wgt = (s0 + j < nsplit && ml[j].x != -INFINITY) ? exp2f(ml[j].x - m) : 0.f;
+        num.x += wgt * pn[j][0].x; num.y += wgt * pn[j][0].y; num.z += wgt * pn[j][1].x; num.w += wgt * pn[j][1].y;
+        den += wgt * ml[j].y;
       }
     }
     const float inv = head_end(end, q0 + i, kvh * g + gh, den, m);
@@ -1174,6 +1173,14 @@ __device__ __forceinline__ void merge_splits(const float* __restrict__ base, int
     wv.y = pack2(num.z * inv, num.w * inv);
     *reinterpret_cast<uint2*>(out + ((size_t)(q0 + i) * nq + kvh * g + gh) * HD + d) = wv;
   }
+}
+template <bool ACROSS>
+__device__ __forceinline__ void merge_splits(const float* __restrict__ base, int nsplit, int r, int ct, int kvh, int g,
+                                             const int* __restrict__ cu_q, bf16_t* __restrict__ out, int nq,
+                                             const HeadEnd& end) {
+  if (nsplit <= 2) merge_splits_by<ACROSS, 2>(base, nsplit, r, ct, kvh, g, cu_q, out, nq, end);
+  else if (nsplit <= 4) merge_splits_by<ACROSS, 4>(base, nsplit, r, ct, kvh, g, cu_q, out, nq, end);
+  else merge_splits_by<ACROSS, 8>(base, nsplit, r, ct, kvh, g, cu_q, out, nq, end);
 }
 
 __global__ __launch_bounds__(64 * COOP_WAVES) void attn_mfma_coop_kernel(
@@ -1192,12 +1199,18 @@ __global__ __launch_bounds__(64 * COOP_WAVES) void attn_mfma_coop_kernel(
   const int r = tile_req ? tile_req[tile] : tile, ct = tile_req ? tile_ct[tile] : 0;
   const TileInfo t = tile_info(cu_q, ctx_len, r, ct, g, kvh, window);
   int first = t.lo_tile, last = t.hi_tile;
-  if (nsplit > 1) {  // splits are cut by absolute key index, in multiples of 32
-    first = (t.lo_tile >> 5 << 5) + split * keys_per_split;
-    last = first + keys_per_split - 1;
+  int live = 1;         // splits that have keys
+  if (nsplit > 1) {     // splits are cut by absolute key index, in multiples of 32
+    const int base = t.lo_tile >> 5 << 5, span = t.hi_tile + 1 - base;
+    const int even = ((span + nsplit - 1) / nsplit + 31) >> 5 << 5, per = even > keys_per_split ? even : keys_per_split;
+    live = (span + per - 1) / per;
+    if (counters && split >= live) return;
+    first = base + split * per;
+    last = first + per - 1;
     last = last < t.hi_tile ? last : t.hi_tile;
     first = first > t.lo_tile ? first : t.lo_tile;
   }
+  const bool alone = nsplit == 1 || (counters && live == 1);
   TileState st;
   init_state(st);
   if (first <= last) {
@@ -1245,21 +1258,17 @@ __global__ __launch_bounds__(64 * COOP_WAVES) void attn_mfma_coop_kernel(
     const int i = colg / g, gh = colg - i * g;
     const Run run = run_of(cu_q, r);
     const int q0 = run.q0, qlen = run.qlen;
-    if (nsplit > 1) {
+    if (!alone) {
       float* part = scratch + (((size_t)tile * nkv + kvh) * nsplit + split) * PART_STRIDE + (size_t)col * PART_COLS;
+      if (i >= qlen) continue;
       if (counters) {   // read by another block of this launch
-        store_device_scope(part + d, num.x); store_device_scope(part + d + 1, num.y);
-        store_device_scope(part + d + 2, num.z); store_device_scope(part + d + 3, num.w);
-        if (d == 0) {
-          store_device_scope(part + HD, m);
-          store_device_scope(part + HD + 1, den);
-        }
+        unsigned long long* pairs = reinterpret_cast<unsigned long long*>(part + d);
+        store_device_scope(pairs, num.x, num.y);
+        store_device_scope(pairs + 1, num.z, num.w);
+        if (d == 0) store_device_scope(reinterpret_cast<unsigned long long*>(part + HD), m, den);
       } else {
         *reinterpret_cast<float4*>(part + d) = num;
-        if (d == 0) {
-          part[HD] = m;
-          part[HD + 1] = den;
-        }
+        if (d == 0) *reinterpret_cast<float2*>(part + HD) = float2{m, den};
       }
     } else if (i < qlen) {
       const float inv = head_end(end, q0 + i, kvh * g + gh, den, m);
@@ -1269,19 +1278,19 @@ __global__ __launch_bounds__(64 * COOP_WAVES) void attn_mfma_coop_kernel(
       *reinterpret_cast<uint2*>(out + ((size_t)(q0 + i) * nq + kvh * g + gh) * HD + d) = wv;
     }
   }
-  if (nsplit > 1 && counters) {
+  if (!alone && counters) {
     // every thread's stores have arrived before anyone counts this block in
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0) {
       int* count = counters + tile * nkv + kvh;
       const int before = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      is_last = before == nsplit - 1;
+      is_last = before == live - 1;
       if (is_last) __hip_atomic_store(count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
     if (is_last)
-      merge_splits<true>(scratch + ((size_t)tile * nkv + kvh) * nsplit * PART_STRIDE, nsplit, r, ct, kvh, g, cu_q, out, nq, end);
+      merge_splits<true>(scratch + ((size_t)tile * nkv + kvh) * nsplit * PART_STRIDE, live, r, ct, kvh, g, cu_q, out, nq, end);
   }
 }
 
@@ -1617,7 +1626,7 @@ extern "C" int qvl_attn_mfma_coop_static(const void* q, const void* kc, const vo
   int err = QVL_OK;
   float* ptr = static_scratch(&err);
   if (!ptr) return err;
-  // Every (tile, head, split) block writes all of its part before the merge kernel reads it, so
+  // Every (tile, head, split) block writes what the merge kernel reads of its part before that does, so
   // nothing of the array has to start at zero, whatever the call before left there.
   return launch_coop(q, kc, vc, bt, table_width, cu_q, ctx_len, tile_req, tile_ct, num_tiles, out, ptr, nullptr, HeadEnd{nullptr, nullptr, 0}, nq, nkv,
                      ps, window, scale, nsplit, keys_per_split, stream);

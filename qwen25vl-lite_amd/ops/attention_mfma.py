@@ -33,9 +33,9 @@ TARGET_BLOCKS = None
 FILL_BLOCKS = None
 MIN_KEYS_PER_SPLIT = 256   # keys a split has at least
 SPLIT_FROM_KEYS = 768      # shorter contexts are walked by one block: merging splits (stores, a counter and loads that go
-                           # through to memory) costs a decode step about 4.5 us, a block's walk 12.7 us per 1,000 keys
-                           # (one compute unit by itself fetches its keys and values at about 40 GB/s); measured at batch 1 and 8:
-                           # 527 keys 11.5 us whole, 11.9 in two splits; 1,024 keys 17.8 whole, 12.0 in four
+                           # through to memory) costs a decode step 2 to 2.5 us, a block's walk some 10 us per 1,000 keys (one compute unit by
+                           # itself fetches its keys and values at about 40 GB/s); whole and in two splits, 8 tokens with 28 + 2 x 4 heads: 300 keys
+                           # 6.3 us and 7.6, 400 6.9 and 7.6, 512 8.6 and 8.6; one token at 500 7.1 and 7.4
 MERGE_COUNTERS = 1 << 16   # (tile, kv head) pairs whose splits one launch can merge by itself
 TICKET_COUNTERS = 8 * 64   # WALK_COUNTERS_AT in the source
 CUT_WALKS = 1 << 13        # walks of one launch that may be cut into parts
@@ -90,7 +90,7 @@ def tiles_for(cu_q, group: int, tile_ct: int = 1) -> Tuple[np.ndarray, np.ndarra
 
 
 def plan_splits(num_tiles: int, nkv: int, max_ctx: int, device=None) -> Tuple[str, int, int]:
-    """``(kernel, nsplit, keys_per_split)``.  ``"tile"``: many tiles, as in prefill: a block owns
+    """``(kernel, nsplit, least keys of a split)``.  ``"tile"``: many tiles, as in prefill: a block owns
     several tiles per wave and shares the keys through LDS.  ``"coop"``: the waves of a block share a tile (few tiles, as in decode); its keys are
     split among ``nsplit`` blocks when the context is long and the blocks are few."""
     blocks = num_tiles * nkv
@@ -102,7 +102,10 @@ def plan_splits(num_tiles: int, nkv: int, max_ctx: int, device=None) -> Tuple[st
         return "coop", 1, 0
     # splits begin at a multiple of 32 at or below the first key a tile sees: up to 31 keys more
     per = ((max_ctx + 31 + nsplit - 1) // nsplit + 31) // 32 * 32
-    return "coop", (max_ctx + 31 + per - 1) // per, per
+    nsplit = (max_ctx + 31 + per - 1) // per
+    # the kernel cuts what keys a tile has evenly; where not all blocks run at once, those of shorter contexts have fewer splits instead
+    # (24 tiles of 1,040 keys at most, 8 heads, captured for 2,048: two even splits 22.5 us, one of them empty 15.9)
+    return "coop", nsplit, MIN_KEYS_PER_SPLIT if blocks * nsplit <= _fill_blocks(device) else per
 
 
 _queues = {}
