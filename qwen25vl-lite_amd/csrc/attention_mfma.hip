@@ -1113,6 +1113,9 @@ __global__ __launch_bounds__(64 * BLK_WAVES * GROUPS, GROUPS == 1 ? BLK_PER_CU :
 // padding that keeps every column 16-byte aligned).
 #define PART_COLS (HD + 4)
 #define PART_STRIDE (16 * PART_COLS)
+// With eight waves of staged keys (head size 128) a block has 133 KB of LDS, and a compute unit one block.  More blocks than compute units whose walks are
+// short run in half the waves, two blocks a unit: 420 tiles of prompts of up to 120 tokens 6.9 us for 10.2, 320 of 80 tokens at 120, 250, 400 keys 8.6, 12.8,
+// 17.9 for 11.1, 15.6, 20.4; beside a few long ones (24 of 177 to 769 keys, 128 of a prompt of 256) 12.0 for 11.2.
 #if HD <= 128
 #define COOP_WAVES 8
 #else
@@ -1183,14 +1186,15 @@ __device__ __forceinline__ void merge_splits(const float* __restrict__ base, int
   else merge_splits_by<ACROSS, 8>(base, nsplit, r, ct, kvh, g, cu_q, out, nq, end);
 }
 
-__global__ __launch_bounds__(64 * COOP_WAVES) void attn_mfma_coop_kernel(
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES, WAVES < COOP_WAVES ? 2 : 1) void attn_mfma_coop_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
     const int* __restrict__ bt, int table_width, const int* __restrict__ cu_q, const int* __restrict__ ctx_len,
     const int* __restrict__ tile_req, const int* __restrict__ tile_ct, bf16_t* __restrict__ out,
     float* __restrict__ scratch, int* __restrict__ counters, int nq, int nkv, int ps, int window, float scale,
     int nsplit, int keys_per_split, HeadEnd end) {
-  __shared__ __attribute__((aligned(16))) float sm[COOP_WAVES][PART_STRIDE];
-  __shared__ __attribute__((aligned(16))) char second_place[K_VIA_LDS ? COOP_WAVES : 1][K_VIA_LDS ? 32 * HD * 2 : 16];   // of staged keys
+  __shared__ __attribute__((aligned(16))) float sm[WAVES][PART_STRIDE];
+  __shared__ __attribute__((aligned(16))) char second_place[K_VIA_LDS ? WAVES : 1][K_VIA_LDS ? 32 * HD * 2 : 16];   // of staged keys
   __shared__ int is_last;
   const int tile = blockIdx.x, kvh = blockIdx.y, split = blockIdx.z;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lg = lane >> 4, c = lane & 15;
@@ -1223,7 +1227,7 @@ __global__ __launch_bounds__(64 * COOP_WAVES) void attn_mfma_coop_kernel(
     const uint32_t k_stage2 = __builtin_amdgcn_readfirstlane(
         (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)&second_place[K_VIA_LDS ? wave : 0][0]);
     attend<1>(kc, vc, bt + (size_t)r * table_width, table_width, nkv, kvh, ps, qb, &t.my_lo, &t.my_p, scale * LOG2E,
-              first, last, wave, COOP_WAVES, &st, k_stage, K_VIA_LDS ? reinterpret_cast<const char*>(&sm[wave][0]) : nullptr,
+              first, last, wave, WAVES, &st, k_stage, K_VIA_LDS ? reinterpret_cast<const char*>(&sm[wave][0]) : nullptr,
               k_stage2, &second_place[K_VIA_LDS ? wave : 0][0]);
   }
   // every wave leaves its column sums in LDS: column c, channels dt*16 + 4*lg .. +3, then m and l
@@ -1243,11 +1247,11 @@ __global__ __launch_bounds__(64 * COOP_WAVES) void attn_mfma_coop_kernel(
     const int col = idx / (HD / 4), d = (idx - col * (HD / 4)) * 4;
     float m = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < COOP_WAVES; ++w) m = fmaxf(m, sm[w][col * PART_COLS + HD]);
+    for (int w = 0; w < WAVES; ++w) m = fmaxf(m, sm[w][col * PART_COLS + HD]);
     float4 num = {0.f, 0.f, 0.f, 0.f};
     float den = 0.f;
 #pragma unroll
-    for (int w = 0; w < COOP_WAVES; ++w) {
+    for (int w = 0; w < WAVES; ++w) {
       const float* p = &sm[w][col * PART_COLS];
       const float wgt = (p[HD] == -INFINITY) ? 0.f : exp2f(p[HD] - m);
       const float4 a = *reinterpret_cast<const float4*>(p + d);
@@ -1535,17 +1539,24 @@ extern "C" long long qvl_attn_mfma_scratch_floats(int num_tiles, int nkv, int ns
 static int launch_coop(const void* q, const void* kc, const void* vc, const void* bt, int table_width,
                        const void* cu_q, const void* ctx_len, const void* tile_req, const void* tile_ct,
                        int num_tiles, void* out, void* scratch, void* counters, const HeadEnd& end, int nq, int nkv,
-                       int ps, int window, float scale, int nsplit, int keys_per_split, hipStream_t stream) {
+                       int ps, int window, float scale, int nsplit, int keys_per_split, hipStream_t stream, bool halved = false) {
   const int c = check_common(num_tiles, nq, nkv, ps, table_width);
   if (c >= 0) return c;
   if (nsplit <= 0 || nsplit > 65535 || (nsplit > 1 && (keys_per_split <= 0 || keys_per_split % 32 || !scratch)))
     return QVL_ERR_SHAPE;
   if (!(scale > 0.f)) return QVL_ERR_SHAPE;
-  hipLaunchKernelGGL(attn_mfma_coop_kernel, dim3(num_tiles, nkv, nsplit), dim3(64 * COOP_WAVES), 0, stream,
-                     (const bf16_t*)q, (const bf16_t*)kc, (const bf16_t*)vc, (const int*)bt, table_width,
-                     (const int*)cu_q, (const int*)ctx_len, (const int*)tile_req, (const int*)tile_ct, (bf16_t*)out,
-                     (float*)scratch, nsplit > 1 ? (int*)counters : nullptr, nq, nkv, ps, window, scale, nsplit,
-                     keys_per_split, end);
+  const auto go = [&](auto kernel, int waves) {
+    hipLaunchKernelGGL(kernel, dim3(num_tiles, nkv, nsplit), dim3(64 * waves), 0, stream,
+                       (const bf16_t*)q, (const bf16_t*)kc, (const bf16_t*)vc, (const int*)bt, table_width,
+                       (const int*)cu_q, (const int*)ctx_len, (const int*)tile_req, (const int*)tile_ct, (bf16_t*)out,
+                       (float*)scratch, nsplit > 1 ? (int*)counters : nullptr, nq, nkv, ps, window, scale, nsplit,
+                       keys_per_split, end);
+  };
+#if K_VIA_LDS
+  if (halved) go(attn_mfma_coop_kernel<COOP_WAVES / 2>, COOP_WAVES / 2);
+  else
+#endif
+    go(attn_mfma_coop_kernel<COOP_WAVES>, COOP_WAVES);
   if (hipGetLastError() != hipSuccess) return QVL_ERR_LAUNCH;
   if (nsplit > 1 && !counters)
     hipLaunchKernelGGL(attn_mfma_merge_kernel, dim3(num_tiles, nkv), dim3(256), 0, stream, (const float*)scratch,
@@ -1572,6 +1583,15 @@ extern "C" int qvl_attn_mfma_coop_merged(const void* q, const void* kc, const vo
                                          int keys_per_split, hipStream_t stream) {
   return launch_coop(q, kc, vc, bt, table_width, cu_q, ctx_len, tile_req, tile_ct, num_tiles, out, scratch, counters,
                      HeadEnd{(const float*)sinks, (const float*)gates, gate_stride}, nq, nkv, ps, window, scale, nsplit, keys_per_split, stream);
+}
+
+// The same without splits, in blocks of half the waves where staged keys fill a compute unit's LDS (head size 128): for more blocks than compute units.
+extern "C" int qvl_attn_mfma_coop_halved(const void* q, const void* kc, const void* vc, const void* bt, int table_width, const void* cu_q,
+                                         const void* ctx_len, const void* tile_req, const void* tile_ct, int num_tiles, void* out,
+                                         const void* sinks, const void* gates, long long gate_stride, int nq, int nkv, int ps, int window,
+                                         float scale, hipStream_t stream) {
+  return launch_coop(q, kc, vc, bt, table_width, cu_q, ctx_len, tile_req, tile_ct, num_tiles, out, nullptr, nullptr,
+                     HeadEnd{(const float*)sinks, (const float*)gates, gate_stride}, nq, nkv, ps, window, scale, 1, 0, stream, true);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -36,6 +36,7 @@ SPLIT_FROM_KEYS = 768      # shorter contexts are walked by one block: merging s
                            # through to memory) costs a decode step 2 to 2.5 us, a block's walk some 10 us per 1,000 keys (one compute unit by
                            # itself fetches its keys and values at about 40 GB/s); whole and in two splits, 8 tokens with 28 + 2 x 4 heads: 300 keys
                            # 6.3 us and 7.6, 400 6.9 and 7.6, 512 8.6 and 8.6; one token at 500 7.1 and 7.4
+HALVED_KEYS = 512          # more blocks than compute units, whose contexts are no longer, run in half the waves (COOP_WAVES in the source has both sides)
 MERGE_COUNTERS = 1 << 16   # (tile, kv head) pairs whose splits one launch can merge by itself
 TICKET_COUNTERS = 8 * 64   # WALK_COUNTERS_AT in the source
 CUT_WALKS = 1 << 13        # walks of one launch that may be cut into parts
@@ -281,6 +282,7 @@ def block_groups(walks: int, places: int, head_dim: int, cut: bool = True) -> in
 
 
 _COOP_ARGS = [_c_ptr] * 4 + [_c_int] + [_c_ptr] * 4 + [_c_int, _c_ptr, _c_ptr] + [_c_int] * 4 + [_c_float, _c_int, _c_int, _c_ptr]
+_HALVED_ARGS = [_c_ptr] * 4 + [_c_int] + [_c_ptr] * 4 + [_c_int] + [_c_ptr] * 3 + [_c_ll] + [_c_int] * 4 + [_c_float, _c_ptr]
 _MERGED_ARGS = [_c_ptr] * 4 + [_c_int] + [_c_ptr] * 4 + [_c_int] + [_c_ptr] * 5 + [_c_ll] + [_c_int] * 4 + [_c_float, _c_int, _c_int, _c_ptr]
 
 
@@ -355,6 +357,13 @@ def try_attention(q, k_cache, v_cache, block_table, step, num_q_heads: int, wind
             floats = _fn("attention_mfma", "qvl_attn_mfma_scratch_floats", [_c_int] * 3, defines)
             floats.restype = ctypes.c_longlong
             scratch = torch.empty(int(floats(num_tiles, nkv, nsplit)), dtype=torch.float32, device=q.device)
+        if nsplit == 1 and hd == 128 and step.max_ctx_len <= HALVED_KEYS and num_tiles * nkv > _fill_blocks(q.device):
+            fn = _fn("attention_mfma", "qvl_attn_mfma_coop_halved", _HALVED_ARGS, defines)
+            _check(fn(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), block_table.shape[1], _ptr(cu_q),
+                      _ptr(step.ctx_len), _ptr(tile_req), _ptr(tile_ct), num_tiles, _ptr(out), _ptr(sinks), *gate_args, nq, nkv, ps,
+                      int(window or 0), float(scale), _stream()), "paged_attention (matrix cores, shared tiles)")
+            taken["shared tiles"] += 1
+            return
         merged = nsplit > 1 and num_tiles * nkv <= MERGE_COUNTERS
         if merged or sinks is not None or gate is not None:
             # the block of each (tile, head) that finishes last merges the splits: one launch
