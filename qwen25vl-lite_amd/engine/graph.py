@@ -5,8 +5,8 @@ the host, not the GPU, sets the step time (the reference measured the same on it
 reference src/qwen25vl_lite/graphs.py:3-7, and also answers with graph capture).  A step in
 which every request brings exactly one token has a fixed shape, so it is captured once per
 (batch bucket, context bucket) and replayed: per step the host fills one pinned buffer with the
-step's integers (token ids, positions, page slots, block tables, context lengths), copies it to
-a fixed device buffer in one transfer, and launches the graph.
+step's integers (token ids, positions, page slots, block tables, context lengths), has a kernel
+bring it to a fixed device buffer, and launches the graph.
 
 Batch sizes are rounded up to 1, 2, 3, 4, 6, 8, 12, 16, ... so that a server whose batch shrinks
 and grows request by request captures a dozen graphs, not one per size.  The rows added are
