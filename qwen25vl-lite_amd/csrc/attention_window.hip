@@ -17,8 +17,8 @@
 //   O^T += V^T P^T   per 16 value channels one product; V^T rows are 8 consecutive keys of a channel,
 //                 one 16-byte load from the transposed value pages.
 // Many tiles: a wave per entry of two neighbouring tiles (every fetched key and value fragment is used
-// for both), four entries a block.  Few tiles (decoded tokens): the four waves of a block share a tile,
-// wave w taking blocks w, w + 4, ..., and merge through LDS.
+// for both), four entries a block.  Few tiles (decoded tokens): the four or, for long walks, eight waves of a
+// block share a tile, wave w taking blocks w, w + 4 (8), ..., and merge through LDS.
 #include "common.h"
 
 #ifndef HD
@@ -67,16 +67,17 @@ struct WindowArgs {
   }
 };
 
-// W: waves that share an entry's key blocks (1 or 4).  CT: column tiles of an entry, all carried by the
+// W: waves that share an entry's key blocks (1, 4 or 8).  CT: column tiles of an entry, all carried by the
 // same wave: a key or value fragment that has been fetched is multiplied with each of them, and what a
 // kernel of this kind waits for is its fetches (its keys and values come from L2 for every entry anew).
 // TURN: values lie turned in the cache.  Two waves a SIMD is what the registers of a walk allow; told so, the compiler
 // keeps all of a block's key fetches in flight instead of saving registers for waves that cannot come (a walk with the
 // turn behind it: 161 us a 2,048-token prompt without, 106 with).
 template <int W, int CT, bool TURN>
-__attribute__((amdgpu_waves_per_eu(2, 2))) __global__ __launch_bounds__(256) void attn_window_kernel(WindowArgs a) {
-  __shared__ float s_m[3][CT][16], s_l[3][CT][16];
-  __shared__ __attribute__((aligned(16))) float s_acc[W > 1 ? 3 : 1][W > 1 ? CT * NT : 1][64][4];
+__attribute__((amdgpu_waves_per_eu(2, 2))) __global__ __launch_bounds__(W > 4 ? 64 * W : 256) void attn_window_kernel(WindowArgs a) {
+  constexpr int OTHERS = W > 1 ? W - 1 : 1;
+  __shared__ float s_m[OTHERS][CT][16], s_l[OTHERS][CT][16];
+  __shared__ __attribute__((aligned(16))) float s_acc[OTHERS][W > 1 ? CT * NT : 1][64][4];
   __shared__ float s_out[TURN && TURN_BY_LDS ? (W > 1 ? 1 : 4) : 1][TURN && TURN_BY_LDS ? 16 : 1][TURN && TURN_BY_LDS ? VD + 1 : 1];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lg = lane >> 4, r = lane & 15;
   const int entry = W == 1 ? blockIdx.x * 4 + wave : blockIdx.x;
@@ -207,7 +208,7 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) __global__ __launch_bounds__(256) voi
   }
 
   if (W > 1) {
-    // waves 1 .. 3 hand their maxima, sums and sums of values to wave 0
+    // the other waves hand their maxima, sums and sums of values to wave 0
     if (wave > 0) {
 #pragma unroll
       for (int c = 0; c < CT; ++c) {
@@ -224,13 +225,13 @@ __attribute__((amdgpu_waves_per_eu(2, 2))) __global__ __launch_bounds__(256) voi
 #pragma unroll
     for (int c = 0; c < CT; ++c) {
       float m_all = m[c];
-      for (int w = 0; w < 3; ++w) m_all = fmaxf(m_all, s_m[w][c][r]);
+      for (int w = 0; w < OTHERS; ++w) m_all = fmaxf(m_all, s_m[w][c][r]);
       const float m_safe = m_all == -INFINITY ? 0.f : m_all;
       float f = expf(m[c] - m_safe);
       l[c] *= f;
 #pragma unroll
       for (int dt = 0; dt < NT; ++dt) acc[c][dt] *= f;
-      for (int w = 0; w < 3; ++w) {
+      for (int w = 0; w < OTHERS; ++w) {
         f = expf(s_m[w][c][r] - m_safe);
         l[c] += s_l[w][c][r] * f;
 #pragma unroll
@@ -329,7 +330,7 @@ extern "C" int qvl_attn_window_sizes(int* hd, int* vd) {
   return QVL_OK;
 }
 
-// share != 0: the four waves of a block share an entry of one column tile (few tiles); else a wave per
+// share 1: the four waves of a block share an entry of one column tile (few tiles); 2: its eight waves; 0: a wave per
 // entry of qvl_attn_window_entry_tiles() column tiles (tile_ct counts in such entries).
 extern "C" int qvl_attn_window(const void* q, const void* kc, const void* vc, const void* bt, int table_width,
                                const void* cu_q, const void* ctx_len, const void* tile_req, const void* tile_ct,
@@ -350,7 +351,8 @@ extern "C" int qvl_attn_window(const void* q, const void* kc, const void* vc, co
   a.sinks = (const float*)sinks;
   a.chunk = chunk; a.turn = (const float2*)turn; a.turn_pairs = turn_pairs;
 #define LAUNCH(TURN)                                                                                                   \
-  if (share) hipLaunchKernelGGL((attn_window_kernel<4, 1, TURN>), dim3(num_tiles, nkv), dim3(256), 0, stream, a);      \
+  if (share == 2) hipLaunchKernelGGL((attn_window_kernel<8, 1, TURN>), dim3(num_tiles, nkv), dim3(512), 0, stream, a); \
+  else if (share) hipLaunchKernelGGL((attn_window_kernel<4, 1, TURN>), dim3(num_tiles, nkv), dim3(256), 0, stream, a);      \
   else hipLaunchKernelGGL((attn_window_kernel<1, WIDE_CT, TURN>), dim3((num_tiles + 3) / 4, nkv), dim3(256), 0, stream, a)
   if (turn) { LAUNCH(true); }
   else { LAUNCH(false); }

@@ -24,6 +24,11 @@ _c_int, _c_float, _c_ptr = ctypes.c_int, ctypes.c_float, ctypes.c_void_p
 # or chunks of 1,024 97 / 62, 2,048 pairs 101 / 86; 3,584 pairs 124 / 141 in windows, 106 / 112 in chunks; 7,168 pairs
 # 238 / 297)
 SHARE_BELOW_PER_CU = 9
+# With a block a compute unit or fewer, walks of more keys than this are shared by eight waves: the walk is halved, and one wave adds up seven others'
+# sums instead of three (1.7 us more with values of 192).  Decoded tokens, four and eight waves, us at 129, 300, 600, 1,500 keys: heads of 256 and values of
+# 192, 28 of one group, 8 tokens 11.1, 15.4, 22.4, 48.2 and 11.1, 15.3, 20.2, 36.9; heads of 128, 28 + 4, 8 tokens 8.4, 11.4, 18.9, 42.8 and 8.2, 10.1, 14.9,
+# 29.1, 64 tokens 10.1, 15.8, 23.4, 51.0 and 9.9, 14.2, 19.7, 39.8; 64 and 32, 16 + 2, 1 token 5.1, 6.6, 12.2, 25.6 and 4.8, 5.8, 9.3, 16.8; at 16 and 64 keys 0.2 to 1.8 slower
+EIGHT_WAVES_FROM = 256
 
 
 def supports(head_dim: int, value_dim: int, page_size: int, dtype: torch.dtype) -> bool:
@@ -32,11 +37,11 @@ def supports(head_dim: int, value_dim: int, page_size: int, dtype: torch.dtype) 
 
 
 def try_attention(q, k_cache, v_cache, block_table, step, num_q_heads: int, window: Optional[int], keep_first: int,
-                  scale: float, share: Optional[bool] = None, sinks: Optional[torch.Tensor] = None,
+                  scale: float, share: Optional[int] = None, sinks: Optional[torch.Tensor] = None,
                   chunk: Optional[int] = None, turn: Optional[torch.Tensor] = None, turn_pairs: bool = False
                   ) -> Optional[torch.Tensor]:
     """The attention through this kernel, or None if it does not take the shape.  ``share`` (tests):
-    whether the waves of a block share a tile, else chosen by the number of tiles."""
+    whether the waves of a block share a tile, 2 that there are eight of them, else chosen by the number of tiles and the longest walk."""
     pages, nkv, ps, hd = k_cache.shape
     vd = v_cache.shape[2]
     if not supports(hd, vd, ps, q.dtype):
@@ -58,7 +63,9 @@ def try_attention(q, k_cache, v_cache, block_table, step, num_q_heads: int, wind
     defines = {"HD": hd, "VD": vd}
     tile_req, tile_ct, num_tiles = _step_tiles(step, group, 1, q.device)
     if share is None:
-        share = num_tiles * nkv < SHARE_BELOW_PER_CU * _compute_units(q.device)
+        pairs, cus = num_tiles * nkv, _compute_units(q.device)
+        longest = min(getattr(step, "max_ctx_len", 0), int(window) + int(keep_first) if window else 1 << 30, int(chunk or 1 << 30))
+        share = 2 if pairs <= cus and longest > EIGHT_WAVES_FROM else int(pairs < SHARE_BELOW_PER_CU * cus)
     cu_q = step.cu_q
     if share and step.max_q_len == 1 and num_tiles == step.num_reqs == len(step.cu_q_host) - 1 == step.cu_q_host[-1]:
         tile_req = tile_ct = cu_q = None     # decoded tokens only: request i brings token i and has tile i
@@ -74,7 +81,7 @@ def try_attention(q, k_cache, v_cache, block_table, step, num_q_heads: int, wind
     _check(fn(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), block_table.shape[1], _ptr(cu_q),
               _ptr(step.ctx_len), _ptr(tile_req), _ptr(tile_ct), num_tiles, _ptr(out), nq, nkv, ps, int(window or 0),
               int(keep_first) if window else 0, int(chunk or 0), float(scale), _ptr(sinks), _ptr(turn), int(turn_pairs),
-              int(bool(share)), _stream()),
+              int(share), _stream()),
            "paged_attention (matrix cores, window with kept keys)")
     taken["window with kept keys, " + ("shared tiles" if share else "a wave per tile")] += 1
     return out
