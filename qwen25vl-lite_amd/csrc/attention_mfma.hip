@@ -1207,7 +1207,7 @@ __global__ __launch_bounds__(64 * WAVES, WAVES < COOP_WAVES ? 2 : 1) void attn_m
   if (nsplit > 1) {     // splits are cut by absolute key index, in multiples of 32
     const int base = t.lo_tile >> 5 << 5, span = t.hi_tile + 1 - base;
     const int even = ((span + nsplit - 1) / nsplit + 31) >> 5 << 5, per = even > keys_per_split ? even : keys_per_split;
-    live = (span + per - 1) / per;
+    live = span > 0 ? (span + per - 1) / per : 1;      // (a tile that sees no key has one, which writes its rows)
     if (counters && split >= live) return;
     first = base + split * per;
     last = first + per - 1;

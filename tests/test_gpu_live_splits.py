@@ -48,3 +48,32 @@ def test_splits_of_the_keys_that_are_there(nsplit, least, nq, nkv, hd, window, c
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])      # the counters are at zero each time
     if counted:
         assert int(attention_mfma._counters(rows.device).abs().sum()) == 0
+
+
+@pytest.mark.parametrize("counted", [True, False])
+@pytest.mark.parametrize("window", [None, 7])
+def test_a_row_without_keys_is_written(counted, window, monkeypatch):
+    """A request whose context is empty, between others: with sinks every probability goes there and its row is zeros, whatever the memory held."""
+    from qwen25vl_lite_amd.ops import attention_mfma
+    from qwen25vl_lite_amd.parts import StepContext
+    lens, ps, nq, nkv, hd = [40, 0, 100], 16, 4, 2, 128
+    if not counted:
+        monkeypatch.setattr(attention_mfma, "MERGE_COUNTERS", 0)
+    monkeypatch.setattr(attention_mfma, "plan_splits", lambda t, n, m, d=None: ("coop", 4, 32))
+    g = torch.Generator(device="cuda").manual_seed(5)
+    kc, vc, rows = (torch.randn(*s, device="cuda", generator=g).bfloat16() for s in ((8, nkv, ps, hd), (8, nkv, hd, ps), (3, nq * hd)))
+    table = torch.arange(24, device="cuda", dtype=torch.int32).view(3, 8) % 8
+    cu, none = [0, 1, 2, 3], torch.zeros(0, dtype=torch.int32).cuda()
+    step = StepContext(num_tokens=3, num_reqs=3, token_ids=none, positions=none, token_req=none, token_seqpos=none,
+                       cu_q=torch.tensor(cu, dtype=torch.int32).cuda(), ctx_len=torch.tensor(lens, dtype=torch.int32).cuda(), req_slots=none, groups=[],
+                       logit_rows=none, cu_q_host=cu, ctx_len_host=[1024] * 3, max_q_len=1, max_ctx_len=1024, lengths_known=False, dtype=torch.bfloat16)
+    made, sinks = [], torch.linspace(-1, 2, nq).cuda()
+
+    def filled(like):
+        made.append(torch.full_like(like, 7.0))
+        return made[-1]
+    monkeypatch.setattr(attention_mfma.torch, "empty_like", filled)
+    out = attention_mfma.try_attention(rows, kc, vc, table, step, nq, window, hd ** -0.5, sinks=sinks)
+    assert out is made[-1] and bool((out[1] == 0).all()) and bool((out[[0, 2]] != 7.0).any(1).all())
+    if counted:
+        assert int(attention_mfma._counters(rows.device).abs().sum()) == 0
