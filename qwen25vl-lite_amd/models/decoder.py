@@ -343,10 +343,11 @@ class DecoderModel:
                     raise RuntimeError("a block left a pass vector unadded: its first norm must fold the stream")
                 stream.row_addend = self.pass_vectors.weight[entry.add_vector]   # the layer's first norm adds it
             block = self.blocks[entry.layer]
-            if few:
-                follows = run[i + 1] if i + 1 < len(run) else None
-                step.next_norm = (self.blocks[follows.layer].norm_ahead(stream.h.shape[0])
-                                  if follows is not None and not follows.mix_input and follows.add_vector is None else None)
+            step.next_norm = None
+            if few and block.leaves_ahead and i + 1 < len(run):
+                follows = run[i + 1]
+                if not follows.mix_input and follows.add_vector is None:
+                    step.next_norm = self.blocks[follows.layer].norm_ahead(stream.h.shape[0])
             stream = block.forward(stream, step, slot)
             if not block.leaves_rounded:
                 stream.rounded = None

@@ -166,7 +166,7 @@ class StepContext:
     residual: Optional[torch.Tensor] = None   # set by a block while a part may add its result in place
     # set with it: the norm that stands behind that part (ops.linear.NormAhead), whose rows the product that adds may leave
     ahead: Any = None
-    # set by the model: the first norm of the block that comes next, where that block takes such rows
+    # set by the model for a block that leaves such rows: the first norm of the block that comes next, where that one takes them
     next_norm: Any = None
     # the model's second table of token rows [vocab, columns], where it has one: layers read columns of their own
     token_side: Optional[torch.Tensor] = None
@@ -347,6 +347,8 @@ class PositionEncoding(Part):
 
 class Block(Part):
     leaves_rounded: bool = False    # forward leaves ``stream.rounded`` equal to the ``stream.h`` it leaves
+    # leaves_ahead of a block: the last product of its forward leaves rows for the norm in ``step.next_norm``, which is set for such a block only (what
+    # a block of blocks has inside would leave them too early)
 
     def norm_ahead(self, rows: int):
         """The block's first norm as a NormAhead, where the block takes ScaledRows in ``stream.scaled``; else None."""

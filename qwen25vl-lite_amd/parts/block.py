@@ -21,6 +21,7 @@ class PreNormBlock(Block):
     """
 
     graph_safe = True
+    leaves_ahead = True
 
     def __init__(self, params, dtype, device):
         super().__init__(dtype, device)
