@@ -12,7 +12,7 @@ import torch
 from ..cache.manager import CacheGroupSpec
 from ..ops.stream import MOST_ROWS
 from ..parts.base import (Block, CacheNeed, LayerSlot, Mixer, ParamSpec, Part, PartSpec, ResidualStream, StateNeed, rotation_key,
-                          StepContext, build_part)
+                          StepContext, build_part, says)
 from .spec import ModelSpec
 
 __all__ = ["DecoderModel"]
@@ -344,10 +344,11 @@ class DecoderModel:
                 stream.row_addend = self.pass_vectors.weight[entry.add_vector]   # the layer's first norm adds it
             block = self.blocks[entry.layer]
             step.next_norm = None
-            if few and block.leaves_ahead and i + 1 < len(run):
+            if few and block.leaves_ahead and says(block, "leaves_ahead") and i + 1 < len(run):
                 follows = run[i + 1]
-                if not follows.mix_input and follows.add_vector is None:
-                    step.next_norm = self.blocks[follows.layer].norm_ahead(stream.h.shape[0])
+                taker = self.blocks[follows.layer]
+                if not follows.mix_input and follows.add_vector is None and says(taker, "norm_ahead"):
+                    step.next_norm = taker.norm_ahead(stream.h.shape[0])
             stream = block.forward(stream, step, slot)
             if not block.leaves_rounded:
                 stream.rounded = None

@@ -30,6 +30,7 @@ New kinds are added with :func:`register_part` and named in a model's layer spec
 from __future__ import annotations
 
 from dataclasses import dataclass, field
+from functools import lru_cache
 from typing import Any, Callable, Dict, List, Optional, Sequence, Tuple
 
 import torch
@@ -38,7 +39,7 @@ __all__ = [
     "ParamSpec", "PartSpec", "CacheNeed", "StateNeed", "LayerSlot", "GroupStep", "StepContext", "ResidualStream",
     "NormedMean", "SumTerm", "ScaledSum",
     "Part", "Norm", "Mixer", "FeedForward", "Filter", "PositionEncoding", "Block", "register_part", "build_part",
-    "known_parts", "Embedding", "Head",
+    "known_parts", "says", "Embedding", "Head",
 ]
 
 
@@ -247,6 +248,22 @@ class SumTerm:
         return [SumTerm(result)]
 
 
+@lru_cache(maxsize=1024)
+def _said_with_forward(cls: type, name: str) -> bool:
+    for c in cls.__mro__:
+        if name in vars(c):
+            return True
+        if "forward" in vars(c):
+            return False
+    return False
+
+
+def says(part: "Part", name: str) -> bool:
+    """Whether ``name`` is said of the forward that ``part`` runs: what ``leaves_ahead``, ``takes_scaled``, ``ahead`` and ``norm_ahead`` say of a class's forward
+    does not hold for that of a subclass, which says it anew or hands on nothing."""
+    return _said_with_forward(type(part), name)
+
+
 class Part:
     """Base of all parts.  ``graph_safe`` says that ``forward`` only launches device work whose
     shape depends on the step's shape alone (no host reads of device data, no host loops over
@@ -258,7 +275,7 @@ class Part:
 
     graph_safe: bool = False
     takes_lazy_norm: bool = False   # forward accepts NormedRows in place of the normalised tensor
-    # what forward adds to ``step.residual`` is one product, the last thing it does, which leaves rows for the norm in ``step.ahead``
+    # what forward adds to ``step.residual`` is one product, the last thing it does, which leaves rows for the norm in ``step.ahead`` (see :func:`says`)
     leaves_ahead: bool = False
 
     def __init__(self, dtype: torch.dtype, device: torch.device):

@@ -6,7 +6,7 @@ from typing import Dict, Optional
 
 import torch
 
-from .base import Block, LayerSlot, Part, PartSpec, ResidualStream, StepContext, SumTerm, build_part, register_part
+from .base import Block, LayerSlot, Part, PartSpec, ResidualStream, StepContext, SumTerm, build_part, register_part, says
 
 __all__ = ["PreNormBlock", "ParallelBlock", "SandwichBlock", "PostNormBlock", "SumNormBlock"]
 
@@ -36,7 +36,9 @@ class PreNormBlock(Block):
                 self.names["norm2"]: self.norm2, self.names["ffn"]: self.ffn}
 
     def norm_ahead(self, rows: int):
-        return self.norm1.ahead() if self.mixer.takes_scaled(rows) else None
+        if not (says(self.mixer, "takes_scaled") and self.mixer.takes_scaled(rows) and says(self.norm1, "ahead")):
+            return None
+        return self.norm1.ahead()
 
     def forward(self, stream: ResidualStream, step: StepContext, slot: LayerSlot) -> ResidualStream:
         x, stream.scaled = stream.scaled, None
@@ -45,7 +47,8 @@ class PreNormBlock(Block):
         step.residual = stream.h            # the mixer may add its result in place and return None
         rows = stream.h.shape[0]
         ahead = None
-        if self.mixer.leaves_ahead and self.ffn.takes_scaled(rows):
+        if (self.mixer.leaves_ahead and says(self.mixer, "leaves_ahead") and says(self.ffn, "takes_scaled") and self.ffn.takes_scaled(rows)
+                and says(self.norm2, "ahead")):
             ahead = step.ahead = self.norm2.ahead()
         stream.pending = self.mixer.forward(x, step, slot.of(self.names["mixer"]))
         if ahead is not None and ahead.left is not None:
@@ -53,7 +56,7 @@ class PreNormBlock(Block):
         else:
             y = self.norm2.forward(stream, lazy=self.ffn.takes_lazy_norm)
         step.residual = stream.h
-        ahead = step.ahead = getattr(step, "next_norm", None) if self.ffn.leaves_ahead else None
+        ahead = step.ahead = getattr(step, "next_norm", None) if self.ffn.leaves_ahead and says(self.ffn, "leaves_ahead") else None
         stream.pending = self.ffn.forward(y, step)
         if ahead is not None:
             stream.scaled = ahead.left

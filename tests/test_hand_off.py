@@ -11,6 +11,7 @@ import torch
 
 from qwen25vl_lite_amd.models import DecoderModel, LayerSpec, ModelSpec, RunEntry
 from qwen25vl_lite_amd.parts import (Block, Embedding, FeedForward, Head, Mixer, Norm, ParamSpec, PartSpec, build_part, known_parts, register_part)
+from qwen25vl_lite_amd.parts.block import PreNormBlock
 
 HIDDEN, VOCAB = 12, 20
 calls = []                       # what ran, in order: "norm <name>" and "taken <name>" (rows that were left, in place of a norm)
@@ -109,8 +110,43 @@ class ToyHead(Head):
         return x @ self.weight.T
 
 
+class OtherNorm(ToyNorm):
+    """A norm with a forward of its own that says nothing about rows left for it."""
+
+    def forward(self, stream, rows=None, lazy=False):
+        return 0.5 * super().forward(stream, rows, lazy) + 0.25
+
+
+class OtherMixer(ToyMixer):
+    """Adds something else behind the product, to a sum that it may change in place."""
+
+    def forward(self, x, step, slot=None):
+        y = super().forward(x, step, slot)
+        step.residual += 0.125
+        return y
+
+
+class OtherFeedForward(ToyFeedForward):
+    """Reads normed rows as a tensor."""
+
+    def forward(self, x, step, slot=None):
+        return super().forward(x * 1.5, step, slot)
+
+
 class BiasedMixer(ToyMixer):
     bias = True
+
+
+class OtherBlock(PreNormBlock):
+    """An arrangement of its own, by what a block was asked for before rows could be left."""
+
+    def forward(self, stream, step, slot):
+        x = self.norm1.forward(stream)
+        step.residual = None
+        stream.pending = self.mixer.forward(x, step, slot)
+        y = self.norm2.forward(stream)
+        stream.pending = self.ffn.forward(y, step)
+        return stream
 
 
 class Twice(Block):
@@ -127,9 +163,10 @@ class Twice(Block):
         return self.b.forward(self.a.forward(stream, step, slot), step, slot)
 
 
-for _category, _kind, _part in (("norm", "cpu_norm", ToyNorm), ("mixer", "cpu_mixer", ToyMixer),
-                                ("mixer", "cpu_mixer_biased", BiasedMixer), ("ffn", "cpu_ffn", ToyFeedForward),
-                                ("embedding", "cpu_embedding", ToyEmbedding), ("head", "cpu_head", ToyHead), ("block", "cpu_twice", Twice)):
+for _category, _kind, _part in (("norm", "cpu_norm", ToyNorm), ("norm", "cpu_norm_other", OtherNorm), ("mixer", "cpu_mixer", ToyMixer),
+                                ("mixer", "cpu_mixer_other", OtherMixer), ("mixer", "cpu_mixer_biased", BiasedMixer), ("ffn", "cpu_ffn", ToyFeedForward),
+                                ("ffn", "cpu_ffn_other", OtherFeedForward), ("embedding", "cpu_embedding", ToyEmbedding), ("head", "cpu_head", ToyHead),
+                                ("block", "cpu_block_other", OtherBlock), ("block", "cpu_twice", Twice)):
     if _kind not in known_parts(_category):
         register_part(_category, _kind, _part)
 
@@ -202,6 +239,17 @@ def test_the_embedding_mixed_in(monkeypatch):
 def test_a_product_that_is_handed_back():
     """An output projection with a bias does not add in place and leaves nothing: the norm behind it runs."""
     assert _run([_layer("a", mixer="cpu_mixer_biased"), _layer("b")]) == ["norm a1", "norm a2", "taken b1", "taken b2", "norm end"]
+
+
+@pytest.mark.parametrize("what, ran", [
+    (dict(norm1="cpu_norm_other"), ["norm a1", "taken a2", "norm b1", "taken b2", "taken c1", "taken c2", "norm end"]),
+    (dict(norm2="cpu_norm_other"), ["norm a1", "taken a2", "taken b1", "norm b2", "taken c1", "taken c2", "norm end"]),
+    (dict(mixer="cpu_mixer_other"), ["norm a1", "taken a2", "norm b1", "norm b2", "taken c1", "taken c2", "norm end"]),
+    (dict(ffn="cpu_ffn_other"), ["norm a1", "taken a2", "taken b1", "norm b2", "norm c1", "taken c2", "norm end"]),
+    (dict(block="cpu_block_other"), ["norm a1", "taken a2", "norm b1", "norm b2", "norm c1", "taken c2", "norm end"])])
+def test_a_subclass_with_a_forward_of_its_own(what, ran):
+    """What a class says about its forward does not hold for a subclass's."""
+    assert _run([_layer("a"), _layer("b", **what), _layer("c")]) == ran
 
 
 def test_layers_within_a_layer():
