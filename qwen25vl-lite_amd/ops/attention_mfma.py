@@ -361,8 +361,8 @@ def try_attention(q, k_cache, v_cache, block_table, step, num_q_heads: int, wind
             fn = _fn("attention_mfma", "qvl_attn_mfma_coop_halved", _HALVED_ARGS, defines)
             _check(fn(_ptr(q), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), block_table.shape[1], _ptr(cu_q),
                       _ptr(step.ctx_len), _ptr(tile_req), _ptr(tile_ct), num_tiles, _ptr(out), _ptr(sinks), *gate_args, nq, nkv, ps,
-                      int(window or 0), float(scale), _stream()), "paged_attention (matrix cores, shared tiles)")
-            taken["shared tiles"] += 1
+                      int(window or 0), float(scale), _stream()), "paged_attention (matrix cores, shared tiles, half the waves)")
+            taken["shared tiles, half the waves"] += 1
             return
         merged = nsplit > 1 and num_tiles * nkv <= MERGE_COUNTERS
         if merged or sinks is not None or gate is not None:
