@@ -275,7 +275,7 @@ __global__ __launch_bounds__(64 * ROWS_WAVES) void gemm_halves_kernel(RowsArgs p
   constexpr bool GATED = OUT == ROWS_GATED || OUT == ROWS_HALVES;
   constexpr int NT = (RG + 1) / 2, W_BYTES = 4 * RG * 1024, STAGE = W_BYTES + MT * 2048;
   constexpr int ALL = 4 * RG + 2 * MT, EACH = ALL / 8, FEW = ALL % 8, F = EACH + (FEW > 0);      // fetches of 8 rows a step: the first FEW waves one more
-    constexpr int STAGES = 4, MERGE = 4 * NT * MT * 1024;            // (five steps on their way instead of four are no faster, three slower)
+  constexpr int STAGES = 4, MERGE = 4 * NT * MT * 1024;            // (five steps on their way instead of four are no faster, three slower)
   static_assert(STAGES * STAGE <= ROWS_LDS && MERGE <= STAGES * STAGE, "the halves' sums lie where the steps were");
   __shared__ __attribute__((aligned(16))) char lds[STAGES * STAGE];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
@@ -449,23 +449,24 @@ static int rows_launch(RowsArgs& p, int mode, hipStream_t stream) {
   const int rows = mode >= ROWS_GATED ? 2 * p.per : p.per, fetches = rows <= 16 ? 2 : (rows + 7) / 8;
   const dim3 grid((unsigned)p.blocks), block(64 * ROWS_WAVES);
 #define GO(MT, F, OUT) hipLaunchKernelGGL((gemm_rows_kernel<MT, F, OUT>), grid, block, 0, stream, p)
-#define MODE(MT, F)                               \
-  do {                                            \
-    if (mode == ROWS_BF16) GO(MT, F, ROWS_BF16);  \
-    else if (mode == ROWS_F32) GO(MT, F, ROWS_F32); \
-    else if (mode == ROWS_GATED) GO(MT, F, ROWS_GATED); \
-    else GO(MT, F, ROWS_HALVES);                  \
-  } while (0)
-#define FETCHES(MT)                     \
-  do {                                  \
-    if (fetches == 2) MODE(MT, 2);      \
-    else if (fetches == 3) MODE(MT, 3); \
-    else MODE(MT, 4);                   \
-  } while (0)
-  if (p.M <= 32) FETCHES(1);
-  else FETCHES(2);
-#undef FETCHES
+#define PLAIN(MT, F)                            \
+  if (mode == ROWS_BF16) GO(MT, F, ROWS_BF16);  \
+  else if (mode == ROWS_F32) GO(MT, F, ROWS_F32)
+#define MODE(MT, F)                                   \
+  PLAIN(MT, F);                                       \
+  else if (mode == ROWS_GATED) GO(MT, F, ROWS_GATED); \
+  else GO(MT, F, ROWS_HALVES)
+  if (p.M <= 32) {
+    if (fetches == 2) { MODE(1, 2); }
+    else if (fetches == 3) { MODE(1, 3); }
+    else { MODE(1, 4); }
+  } else {
+    if (fetches == 2) { PLAIN(2, 2); else return QVL_ERR_LIMIT; }      // (gated ones of so few rows a wave run in halves)
+    else if (fetches == 3) { MODE(2, 3); }
+    else { MODE(2, 4); }
+  }
 #undef MODE
+#undef PLAIN
 #undef GO
   return qvl_launch_status();
 }
