@@ -1,5 +1,6 @@
 // Products with up to 64 rows: out = X[M, K] . W[N, K]^T, bfloat16 operands, float32 sums, stored as they are, as bfloat16, through
-// the gated activation of W's rows (groups of 8 gate and 8 up rows, or all gate rows first), or as one slab of sums for each range of K.
+// the gated activation of W's rows (groups of 8 gate and 8 up rows, or all gate rows first), or as one slab of sums for each range of K (those, and
+// gated ones of 17 to 64 rows with few rows of W a wave, by a second kernel, whose waves share a step's columns by halves).
 //
 // What bounds it is reading W once.  A wave owns up to 32 rows of W and all rows of X (operands of
 // v_mfma_f32_32x32x16_bf16), eight waves are a block and a block has a compute unit to itself; the rows a wave takes at a time

@@ -7,8 +7,10 @@
 // through its columns 64 at a time.  Operands come through a ring of LDS places of 2 KB (whole lines) that belongs to the
 // wave: it waits for its own fetches only and asks for the next as soon as a place has been read, so nothing is waited for from the
 // first fetch to the last and the waves meet once, when their sums are added in wave order.  X's columns come through the same ring,
-// once for all of the block's rows.  Few places are better than many: with four a wave
-// 2,048 x 11,008, 1 row, 10.0 us, nine 11.0; 3,584 x 3,584 6.9 and 7.4; 22,016 x 2,048 17.6 and 18.3.
+// once for all of the block's rows.  Few places do. Two, three and four a wave where it has one tile of
+// outputs: 3,584 x 18,944, 8 rows 26.0 us, 23.9, 24.8, 16 rows 30.9, 28.0, 28.7; 2,048 x 11,008, 8 rows 11.6, 11.1, 11.4, 16 rows 16.9, 13.2, 13.6; 3,584 x
+// 3,584, 1 row 7.3, 7.0, 7.0: there it has three. With more tiles three and four are the same within 2 per cent either way (22,016 x 2,048 gated, 1 row 17.6
+// and 17.9, 59,136 x 8,192, 16 rows 147.3 and 146.4), and it has four.
 //
 // The norm between two products of a layer has no kernel of its own.  Where the residual is formed here its new rows are left times the next
 // norm's gain, with each block's sums of their squares; the product behind the norm takes these rows and divides its sums by

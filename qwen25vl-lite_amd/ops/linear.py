@@ -2,10 +2,13 @@
 
 float32 runs through hand-written kernels on the matrix cores' float32 instruction (true 32-bit, fixed summation order; plain
 multiply-adds where strides or sizes do not suit it).
-bfloat16 with up to 32 rows (a decode step) runs through the hand-written matrix-core kernel that keeps the rows
+bfloat16 with up to 16 rows (a decode step) that is added to the residual, or gated behind such a sum, runs through the kernel whose waves share the inner
+size (:mod:`~qwen25vl_lite_amd.ops.stream`): the sum leaves its new rows for the norm behind it (:class:`ScaledRows`), which then has no kernel.  What else
+has up to 32 rows runs through the one that keeps the rows
 (:mod:`~qwen25vl_lite_amd.ops.skinny`), which also folds the norm before a product, the residual add after it and the SwiGLU
 activation into itself; up to 64 rows with many outputs through one that needs not keep them (:mod:`~qwen25vl_lite_amd.ops.rows`);
-with more rows the tiled kernel runs (:mod:`~qwen25vl_lite_amd.ops.tile`), with the activation on its sums.  Where the result
+with more rows the tiled kernel runs (:mod:`~qwen25vl_lite_amd.ops.tile`), with the activation on its sums, or at some hundred rows of narrow models small
+tiles over all of the inner size (:mod:`~qwen25vl_lite_amd.ops.mid`), which leave rows for a norm too.  Where the result
 joins a sum anyway products may be cut along the inner size.  The vendor library's product, which the
 reference's engine uses for its projections (reference src/qwen25vl_lite/text.py:61-66, 80-90), is left
 for what neither takes or does as fast.
@@ -143,8 +146,8 @@ def _aligned(x: torch.Tensor) -> bool:
 
 
 # Long inner sizes (``skinny.prefers_split``) are added in place where a norm waits for the rows that are left then; without one, up to here: the product
-# and the norm behind it, in place and in slabs, 8 rows of 3,584 x 18,944 27.1 us and 28.9, 2,048 x 11,008 13.1 and 14.0, 4,096 x 14,336 24.8 and
-# 24.8, 8,192 x 29,568 81.4 and 83.1; 16 rows 31.5 and 29.5, 15.1 and 15.2, 27.1 and 26.6, 85.0 and 81.8 (left for the norm: 28.3, 13.0, 23.9, 81.0).
+# and the norm behind it, in place and in slabs, 8 rows of 3,584 x 18,944 27.2 us and 29.1, 2,048 x 11,008 13.5 and 14.3, 4,096 x 14,336 25.0 and
+# 25.0, 8,192 x 29,568 79.8 and 81.6; 16 rows 31.5 and 28.3, 15.3 and 15.4, 27.2 and 24.9, 83.3 and 78.3 (left for the norm: 28.4, 13.2, 24.1, 79.0).
 IN_PLACE_ROWS = 8
 
 

@@ -41,12 +41,11 @@ def wide(m: int, weight: torch.Tensor) -> bool:
     """Whether the kernel is the fastest way to ``m`` rows: many outputs, and an inner size beyond the resident kernel's
     narrow build (a norm formed in each of its blocks takes longer than a kernel of its own), or more rows than that
     carries in one column tile.  Against
-    the resident kernel at 32 rows: 22,016 x 2,048 gated 22 us for 27, with the norm in front 27 for 32; 37,888 x 3,584 45
-    for 54, 50 for 65; 152,064 x 3,584 186 for 200; with 9 rows and the norm
-    37,888 x 3,584 49.7 us for 52.5, with 16 50.1 for 55.6 (22,016 x 2,048 26.3 for 25.5); a pass of 8 decode steps, 7B sizes, 8
-    layers, 1 row 8,291 us for 8,347, 4 rows 8,498 for 8,727, 8 rows 8,757 for 9,006, 16 rows 9,150 for 9,651; 3B sizes, 16
-    rows, 5,730 for 5,723.  Against the library at 64 rows: 37,888 x 3,584 gated 49 us for 69 with the
-    activation's kernel, 59,136 x 8,192 151 for 199; heads of 152,064 x 3,584 194 for 219, x 8,192 438 for 500."""
+    the resident kernel at 32 rows: 22,016 x 2,048 gated 18 us for 24, with the norm in front 21 for 29; 37,888 x 3,584 45
+    for 53, 49 for 64; 152,064 x 3,584 187 for 197; with 9 rows and the norm
+    37,888 x 3,584 46.6 us for 50.7, with 16 47.1 for 53.9 (22,016 x 2,048 22.6 for 22.0, 23.0 for 23.5); with 1 row 48.7 for 49.7 (23.6 for
+    20.9).  Against the library at 64 rows: 37,888 x 3,584 gated 51 us for 65 with the
+    activation's kernel, 59,136 x 8,192 143 for 195; heads of 152,064 x 3,584 198 for 218, x 8,192 421 for 493."""
     k = weight.shape[1]
     return (m <= MOST_ROWS and many_outputs(weight)
             and (k > skinny.NARROW_K or m > skinny.ONE_TILE_ROWS or not skinny.takes_resident(m, k, weight)))

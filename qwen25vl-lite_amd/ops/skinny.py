@@ -280,14 +280,13 @@ _SLICE_ARGS = [_c_ptr, _c_int, _c_ptr, _c_int] + [_c_ptr] * 6 + [_c_int] * 7 + [
 SPLIT_ROWS = 64   # the most rows that are cut along the inner size
 SPLIT_K = 2048    # the longest inner size, for each compute unit: with more of it a block of the few rows' kernel could not keep its range
 # Up to here a block keeps its range of the rows and walks several tiles (csrc/gemm_resident.hip: few ranges, so few slabs for the
-# norm behind to add), with more rows csrc/gemm_rows.hip cuts (3,584 x 18,944 alone: 8 rows 25.4 us for 26.9, 16 rows 25.4 for 28.3, 64
-# rows 28.3 for 36.7).  A pass of 8 decode steps with the norms, cut by gemm_rows.hip for this kernel: 3B sizes, 8 layers, 1 row 4,698
-# us for 4,579, 8 rows 5,207 for 5,095; 7B, 8 layers, 1 row 8,248 for 8,298, 4 rows 8,420 for 8,432, 8 rows 8,701 for 8,678; 72B, 2
-# layers, 1 row 8,686 for 8,637, 8 rows 8,958 for 9,010: within 0.6 per cent at the long inner sizes, 2 per cent slower at 11,008.
+# norm behind to add), with more rows csrc/gemm_rows.hip cuts.  The line is older than the latter's halves; with the norm that adds the slabs, kept and cut
+# by gemm_rows.hip, 1 and 8 rows of 2,048 x 11,008 13.4 us and 13.6, 14.3 and 14.0; 4,096 x 14,336 24.6 and 24.3, 25.0 and 24.6; 3,584 x 18,944 29.6 and 28.3, 29.1 and 27.8;
+# 8,192 x 29,568 79.8 and 81.4, 81.6 and 77.9.  It decides little: so few rows that join a sum hardly come here (linear_into adds them in place).
 KEPT_SPLIT_ROWS = 8
-# Up to 16 rows likewise where the weight has no more values than this: its few slabs then count for more than the pace of the stream.  A pass of
-# 6 decode steps, 3B sizes, 6 layers (2,048 x 11,008), kept for cut by gemm_rows.hip: 9 rows 3,136 us for 3,180, 12 rows 3,163 for 3,211,
-# 16 rows 3,299 for 3,340; 7B, 4 layers (3,584 x 18,944), 16 rows 4,232 for 4,213; 72B, 2 layers (8,192 x 29,568), 16 rows 6,956 for 6,848
+# Up to 16 rows likewise where the weight has no more values than this, its few slabs counting for more than the pace of the stream; older than the halves
+# too, now kept and cut, 9, 12 and 16 rows of 2,048 x 11,008 14.3 us and 14.2, 14.8 and 14.2, 15.4 and 14.3; with more values, 16 rows, 4,096 x 14,336 26.1 and
+# 24.9, 3,584 x 18,944 31.9 and 28.3, 8,192 x 29,568 86.0 and 78.3
 KEPT_WEIGHTS = 1 << 25
 
 
@@ -311,17 +310,14 @@ def takes_split(m: int, k: int, weight: torch.Tensor) -> bool:
 
 
 def prefers_split(m: int, k: int, weight: torch.Tensor) -> bool:
-    """Where the split kernel is the fastest way to a product that is added to the residual
-    (measured on MI355X at the 3B, 7B and 72B decoders' output and down projections): up to 16 rows
+    """Where ranges of the inner size, whose slabs the norm behind adds, are the fastest way to a product that is added to the residual
+    but for :mod:`stream`, which ``linear_into`` asks first (up to 16 rows in place: where a norm waits for the rows it leaves, up to 8 also without): up to 16 rows
     when the inner size is too long for a block of the resident kernel to keep its rows for one
-    pass over the weight (the down projection at 8 rows: 26.9 us against 37.3).  A shorter one adds into the sum in place: the
-    next product may form the norm itself, and where it does not (many outputs, an inner size beyond 2,048) a norm
-    without slabs stands in front of it (the output projection in slabs for in place, a pass of 8 decode steps: 3B sizes, 1 row 4,703 us for
-    4,579, 8 rows 5,255 for 5,095; 7B, 1 row 8,318 for 8,298, 8 rows 8,699 for 8,678, 16 rows 9,023 for 9,095; 72B, 1 row 8,654 for 8,637,
-    8 rows 8,923 for 9,010).  With more rows always (the output projection at 32 rows:
-    10.3 us and a norm kernel of 6 against 14.2 in place and 11 more for the norm inside the gate | up
-    product; at 64 rows 12.3 us against the library's 13.9 to 17.6, the down projection 28.3
-    against 46.6)."""
+    pass over the weight (with the norm behind it, 8 rows of 3,584 x 18,944 29.1 us, by the resident kernel in place 33.6; 16 rows of 2,048 x 11,008
+    15.4 and 23.0; left for the norm by ``stream`` 24.1, 13.2).  A shorter one adds into the sum in place: the next product may form the norm itself, or has its rows left
+    (3,584 x 3,584, 8 rows, 7.1 us, in slabs with the norm 11.2).  With more rows always (with the norm behind it, in slabs, in place by the resident kernel, by the
+    library, 32 rows of 3,584 x 3,584 12.7 us, 16.0, 16.0, 3,584 x 18,944 28.9, 53.6, 113, 2,048 x 2,048 8.9, 9.8, 14.4; 64 rows, slabs and library, 15.4
+    and 17.9, 31.7 and 94, 11.1 and 15.0)."""
     if not takes_split(m, k, weight):
         return False
     return m > ONE_TILE_ROWS or (k > NARROW_K and k > resident_norm_k())
